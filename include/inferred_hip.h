@@ -280,6 +280,10 @@ uint32_t it_hip_argmax(it_hip*, const float* buf, uint64_t len);
  * logits have no device copy. */
 int it_hip_embed_argmax(it_hip*, const it_weights* table, const float* logits, uint64_t logits_len, float* x,
                         uint64_t x_len, uint64_t ring_index);
+/* x = the rows ids[0..n) of `table`, dequantized on the device (Model::embed, src/model/qwen35.rs:855-873, which does it on
+ * the host and leaves the backend a copy to make: 8 KB a token).  Called inside a pass in place of the host embedding and
+ * host_wrote.  Returns 0 without doing anything when the table type is not handled or an id is outside the table. */
+int it_hip_embed_rows(it_hip*, const it_weights* table, const uint32_t* ids, uint64_t n, float* x, uint64_t x_len);
 /* ids filed by it_hip_embed_argmax at ring indices first_index .. first_index + n (waits for the device) */
 void it_hip_read_tokens(it_hip*, uint64_t first_index, uint64_t n, uint32_t* out);
 void it_hip_sync(it_hip*);

@@ -76,32 +76,64 @@ void it_hip::dyn_rotate() {
     dyn_host = dyn_hosts[dyn_cur];
     dyn_count = 0;
 }
+// What a recorded pass reads that its launches do not carry: host copies, positions, the token's embedding row.
+void it_hip::issue_inputs() {
+    for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
+    precopies.clear();
+    dyn_upload();
+    if (pre_embed.x) (void)itk::poke(nullptr, dyn_host, 0, &pre_embed.table, pre_embed.token, pre_embed.x, stream);
+    pre_embed.x = nullptr;
+}
 void it_hip::dyn_upload() {
     if (!dyn_count) return;
     // a token's pass has a few dozen: they go with a small kernel's arguments (between two replayed passes a
     // host-to-device copy is a transfer the stream waits for); a long pass's thousands are copied
-    if (itk::poke_ints(dyn_dev, dyn_host, (int)dyn_count, stream)) return;
+    if (itk::poke(dyn_dev, dyn_host, (int)dyn_count, pre_embed.x ? &pre_embed.table : nullptr, pre_embed.token, pre_embed.x, stream)) {
+        pre_embed.x = nullptr;
+        return;
+    }
     check(hipMemcpyAsync(dyn_dev, dyn_host, dyn_count * sizeof(int), hipMemcpyHostToDevice, stream), "upload positions");
     if (hipEventRecord(dyn_evt[dyn_cur], stream) == hipSuccess) dyn_evt_used[dyn_cur] = true;
 }
 
+void it_hip::drop_one(Graph& g) {
+    if (g.valid && !g.replays) graph_unused++;
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    if (g.graph) (void)hipGraphDestroy(g.graph);
+    g = Graph{};
+}
 void it_hip::drop_graph() {
-    if (graph.exec) (void)hipGraphExecDestroy(graph.exec);
-    if (graph.graph) (void)hipGraphDestroy(graph.graph);
-    graph.exec = nullptr;
-    graph.graph = nullptr;
-    graph.valid = false;
-    graph.signature.clear();
-    graph.attn_slots.clear();
+    for (Graph& g : graphs) drop_one(g);
     stable_passes = 0;
+}
+// The first op of a single-token pass says which kind of pass it is (fed an id by the host, or by the arg-max of the last
+// logits): it is replayed from the graph of that kind, recorded, or issued op by op.  A backend that holds one graph has
+// its weights resident and its buffers sized, so a pass of a kind not seen before is recorded at once, without the two
+// op-by-op passes that the first graph waits for (ten milliseconds each on 48 layers); not so once graphs have been recorded
+// in vain, by a caller whose passes keep changing.
+void it_hip::open_pass(uint64_t sig) {
+    bool any = false;
+    for (Graph& g : graphs) {
+        any |= g.valid;
+        if (!g.valid || g.signature.empty() || g.signature[0] != sig) continue;
+        graph = &g;
+        mode = Mode::Replay;
+        profile_pass = prof_on;   // the fused launches one by one between timing events instead of the graph
+        return;
+    }
+    const bool stable = stable_passes >= 1 && !prev_signature.empty() && prev_signature[0] == sig;
+    if (!prof_on && (stable || (any && graph_unused < 4))) {
+        mode = Mode::Capture;
+        return;
+    }
+    mode = Mode::Eager;
+    issue_inputs();
 }
 
 // what a deferred pass has recorded so far goes to the stream, fused; the pass stays deferred
 void it_hip::flush_deferred() {
     if (chain_enabled && fuse_enabled && !exact && !expert_cold_entries && (!itk::layer_chain_fits() || !chain_acquire())) chain_enabled = false;
-    for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
-    precopies.clear();
-    dyn_upload();
+    issue_inputs();
     if (pending.empty()) return;
     auto todo = std::move(pending);
     pending.clear();
@@ -119,12 +151,13 @@ void it_hip::need_eager(const char* why) {
         flush_deferred();
         return;
     }
-    drop_graph();
-    graph_aborts++;
+    if (mode != Mode::Open) {
+        if (mode == Mode::Replay) drop_one(*graph);
+        stable_passes = 0;
+        graph_aborts++;
+    }
     mode = Mode::Eager;
-    for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
-    precopies.clear();
-    dyn_upload();
+    issue_inputs();
     auto todo = std::move(pending);
     pending.clear();
     for (auto& op : todo) op.run(stream);
@@ -139,6 +172,10 @@ void it_hip::finish_pass() {
         stable_passes = 0;
         return;
     }
+    if (mode == Mode::Open) {   // no op came
+        mode = Mode::Eager;
+        issue_inputs();
+    }
     if (mode == Mode::Eager) {
         if (pass_tokens == 1 && allow_graph && !mid_pass_read && !prof_on) {
             stable_passes = (pass_signature == prev_signature && !pass_signature.empty()) ? stable_passes + 1 : 0;
@@ -149,9 +186,7 @@ void it_hip::finish_pass() {
         return;
     }
     if (mode == Mode::Capture) {
-        // inputs first (they are not part of the graph), then record the fused pass
-        for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
-        precopies.clear();
+        // record the fused pass; its inputs are not part of the graph
         hipGraph_t g = nullptr;
         // a chain's hand-off space is allocated and cleared here: neither is allowed while the stream is capturing
         if (chain_enabled && fuse_enabled && !exact && (!itk::layer_chain_fits() || !chain_acquire())) chain_enabled = false;
@@ -163,56 +198,60 @@ void it_hip::finish_pass() {
             if (le != hipSuccess) e = le;
         }
         mode = Mode::Eager;
+        graph = nullptr;
         if (e == hipSuccess && g) {
             hipGraphExec_t ex = nullptr;
             e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
             if (e == hipSuccess && ex) {
-                drop_graph();
-                graph.graph = g;
-                graph.exec = ex;
-                graph.signature = pass_signature;
-                graph.attn_slots = fused_attn_slots;
-                graph.elided = fused_elided;
-                graph.has_chain = chain_launches > 0;
-                graph.valid = true;
-                graph_captures++;
+                // a free slot, else the oldest graph's
+                graph = &graphs[0];
+                for (Graph& c : graphs)
+                    if (!c.valid || (graph->valid && c.born < graph->born)) graph = &c;
+                drop_one(*graph);
+                graph->born = ++graph_captures;
+                graph->graph = g;
+                graph->exec = ex;
+                graph->signature = pass_signature;
+                graph->attn_slots = fused_attn_slots;
+                graph->elided = fused_elided;
+                graph->has_chain = chain_launches > 0;
+                graph->valid = true;
                 stable_passes = 1;
             } else if (g) {
                 (void)hipGraphDestroy(g);
             }
         }
         (void)hipGetLastError();
-        if (!graph.valid) {  // could not build a graph: run the pass eagerly
-            mode = Mode::Replay;  // reuse the fallback path
+        if (!graph) {  // could not build a graph: run the pass eagerly
+            mode = Mode::Capture;  // reuse the fallback path
             need_eager("graph instantiation failed");
             allow_graph = false;
             return;
         }
     } else {  // Replay
         mode = Mode::Eager;
-        if (replay_cursor != graph.signature.size()) {
+        graph->replays++;
+        if (replay_cursor != graph->signature.size()) {
             mode = Mode::Replay;
             need_eager("the pass ended early");
             return;
         }
-        if (!attn_positions_agree(graph.attn_slots)) {
+        if (!attn_positions_agree(graph->attn_slots)) {
             mode = Mode::Replay;
             need_eager("a fused attention block's rope, cache-write and context positions do not agree");
             return;
         }
     }
-    for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
-    precopies.clear();
-    dyn_upload();
+    issue_inputs();
     if (profile_pass) {
         run_fused(pending);  // the launches the graph holds, each between two events
         check(hipGetLastError(), "kernel launch");
     } else {
-        check(hipGraphLaunch(graph.exec, stream), "hipGraphLaunch");
+        check(hipGraphLaunch(graph->exec, stream), "hipGraphLaunch");
         graph_launches++;
     }
-    mark_elided(graph.elided);
-    if (graph.has_chain) chain_ran = true;
+    mark_elided(graph->elided);
+    if (graph->has_chain) chain_ran = true;
     pending.clear();
 }
 
@@ -1126,6 +1165,10 @@ it_hip::~it_hip() {
     if (argmax_val) (void)hipFree(argmax_val);
     if (argmax_out) (void)hipFree(argmax_out);
     if (argmax_host) (void)hipHostFree(argmax_host);
+    for (auto& st : id_stage) {
+        if (st.host) (void)hipHostFree(st.host);
+        if (st.evt) (void)hipEventDestroy(st.evt);
+    }
     for (auto e : prof_pool) (void)hipEventDestroy(e);
     if (dyn_dev) (void)hipFree(dyn_dev);
     if (route_counter) (void)hipFree(route_counter);
@@ -1263,6 +1306,10 @@ it_hip* it_hip_create(uint32_t flags, int device, char* err, size_t err_len) {
     if (it_hip_noalloc_setup() != 0) {
         delete be;
         return bad("cannot resolve the fixed attention scratch on this device");
+    }
+    if (!be->argmax_ready()) {
+        delete be;
+        return bad("cannot allocate the arg-max scratch");
     }
     if (hipMalloc((void**)&be->route_counter, sizeof(unsigned)) != hipSuccess ||
         hipMemset(be->route_counter, 0, sizeof(unsigned)) != hipSuccess) {
@@ -2091,20 +2138,14 @@ void it_hip_begin_pass(it_hip* be, uint64_t n_tokens) {
     be->pass_signature.clear();
     be->pending.clear();
     be->precopies.clear();
+    be->pre_embed.x = nullptr;
     be->dyn_rotate();
     be->replay_cursor = 0;
     be->mode = it_hip::Mode::Eager;
     be->profile_pass = false;
     // cold experts are resolved from the picks inside the pass, which a graph cannot replay (experts.rs:91-93)
     if (n_tokens == 1 && be->allow_graph && !be->mid_pass_read && !be->has_error && !be->expert_cold_entries) {
-        if (be->graph.valid) {
-            // while profiling, the pass is recorded like a replay and its fused launches are
-            // then issued one by one between timing events instead of as the graph
-            be->mode = it_hip::Mode::Replay;
-            be->profile_pass = be->prof_on;
-        } else if (be->stable_passes >= 1 && !be->prof_on) {
-            be->mode = it_hip::Mode::Capture;
-        }
+        be->mode = it_hip::Mode::Open;   // replayed, recorded or issued op by op: the first op decides
     } else if (n_tokens == 1 && be->expert_cold_entries && be->fuse_enabled && !be->has_error) {
         be->mode = it_hip::Mode::Deferred;   // picks are read back inside the pass: fused launches, no graph
     } else if (n_tokens == 1 && be->eager_fused && !be->allow_graph && be->fuse_enabled && !be->has_error && !be->prof_on) {
@@ -2343,6 +2384,27 @@ int64_t it_hip_clock_pick(uint8_t* heat, const uint8_t* leased, uint64_t n, uint
 // ------------------------------------------------------------------ extensions
 }  // extern "C"
 
+// Page-locked copies of a batch's token ids, two in turn: a pass may be issued while the one before it still runs.
+const int32_t* it_hip::stage_ids(const uint32_t* ids, uint64_t n) {
+    IdStage& st = id_stage[id_cur ^= 1];
+    if (st.used) check(hipEventSynchronize(st.evt), "wait for the token id staging buffer");
+    st.used = false;
+    if (st.cap < n) {
+        if (st.host) (void)hipHostFree(st.host);
+        st.host = nullptr;
+        st.cap = 0;
+        if (!st.evt && !check(hipEventCreateWithFlags(&st.evt, hipEventDisableTiming), "hipEventCreate(token ids)")) return nullptr;
+        if (!check(hipHostMalloc((void**)&st.host, n * 4, hipHostMallocDefault), "hipHostMalloc(token ids)")) return nullptr;
+        st.cap = n;
+    }
+    memcpy(st.host, ids, n * 4);
+    return st.host;
+}
+void it_hip::staged_ids() {
+    IdStage& st = id_stage[id_cur];
+    st.used = check(hipEventRecord(st.evt, stream), "record the token id staging event");
+}
+
 bool it_hip::argmax_ready() {
     if (argmax_idx) return true;
     need_eager("argmax scratch is allocated");
@@ -2368,6 +2430,36 @@ uint32_t it_hip_argmax(it_hip* be, const float* buf, uint64_t len) {
     be->d2h++;
     be->d2h_bytes += 4;
     return (uint32_t)*be->argmax_host;
+}
+
+int it_hip_embed_rows(it_hip* be, const it_weights* table, const uint32_t* ids, uint64_t n, float* x, uint64_t x_len) {
+    if (!table || !ids || !x || n == 0 || n >= (1ull << 31) || table->n_in == 0 || x_len != n * table->n_in) return 0;
+    if (table->ty != IT_Q8_0 && table->ty != IT_F16 && table->ty != IT_BF16 && table->ty != IT_F32) return 0;
+    if (be->has_error) return 0;
+    for (uint64_t i = 0; i < n; i++)
+        if (ids[i] >= table->n_out) return 0;
+    itk::WView w;
+    if (!be->weights_view(table, "embed_rows", &w)) return 0;
+    float* dx = be->act_out(x, x_len);
+    if (!dx) return 0;
+    if (n == 1 && be->mode != it_hip::Mode::Eager) {
+        // a recorded pass: the row is made by the small kernel that carries the pass's positions
+        be->pre_embed = {w, (int)ids[0], dx};
+        return 1;
+    }
+    be->launches++;
+    if (!be->held.empty()) be->release_held();
+    it_hip::Span sp(be, it_hip::FAM_OTHER, x_len * 5);
+    if (n == 1) {
+        (void)itk::poke(nullptr, nullptr, 0, &w, (int)ids[0], dx, be->stream);
+    } else {
+        const int32_t* staged = be->stage_ids(ids, n);
+        if (!staged) return 0;
+        itk::embed_rows(w, staged, (int)n, dx, be->stream);
+        be->staged_ids();
+    }
+    be->check(hipGetLastError(), "kernel launch");
+    return 1;
 }
 
 int it_hip_embed_argmax(it_hip* be, const it_weights* table, const float* logits, uint64_t logits_len, float* x,

@@ -213,6 +213,7 @@ struct it_hip {
         hipGraphExec_t exec = nullptr;
         std::vector<uint64_t> signature;  // hash of each seam call's static arguments
         bool valid = false;
+        uint64_t born = 0, replays = 0;
         // position slots of every fused attention block: {rope, key write, value write, attend}.  The fused kernel
         // takes ONE position for all four, so a replay is only valid while write row == rope position and the
         // context length == position + 1 (the seam does not tie them together; the model loop does)
@@ -220,11 +221,18 @@ struct it_hip {
         std::vector<const void*> elided;   // device buffers whose ops the graph's fused kernels skip
         bool has_chain = false;
     };
-    Graph graph;
+    // One graph for each kind of single-token pass (fed by the host, fed by the arg-max, ...): a request that takes its
+    // prompt's last token one way and goes on the other replays both.  `graph`: the one this pass replays or has recorded.
+    std::array<Graph, 4> graphs;
+    Graph* graph = nullptr;
+    uint64_t graph_unused = 0;   // graphs dropped without a replay
+    void drop_one(Graph& g);
+    void open_pass(uint64_t sig);
     // Deferred: a single-token pass whose ops are recorded like a captured pass's and issued as fused launches whenever
     // something needs them on the stream (a cold expert's resolve reads the picks back, a host read, the pass's end):
     // the fusion of the decode path without its graph, for passes a graph cannot hold.
-    enum class Mode { Eager, Capture, Replay, Deferred } mode = Mode::Eager;
+    // Open: a single-token pass whose first op has not come yet (open_pass).
+    enum class Mode { Eager, Open, Capture, Replay, Deferred } mode = Mode::Eager;
     void flush_deferred();
     std::vector<uint64_t> pass_signature, prev_signature;
     int stable_passes = 0;      // consecutive eager decode passes with the same op sequence
@@ -284,6 +292,24 @@ struct it_hip {
     bool small_ffn(const std::vector<OpRec>& run);   // the routed FFN of a short batch as two launches
     bool small_ffn_enabled = true;           // INFERRED_HIP_NO_SMALL_FFN=1 issues it op by op (a measurement switch)
     std::vector<PreCopy> precopies;  // host -> device inputs of a graphed pass, issued before the graph
+    // the embedding row of a recorded single-token pass, made by the kernel that carries its positions (x: not yet issued)
+    struct PreEmbed {
+        itk::WView table;
+        int token;
+        float* x;
+    };
+    PreEmbed pre_embed{};
+    void issue_inputs();
+    struct IdStage {
+        int32_t* host = nullptr;   // page-locked
+        uint64_t cap = 0;
+        hipEvent_t evt = nullptr;
+        bool used = false;
+    };
+    IdStage id_stage[2];
+    int id_cur = 0;
+    const int32_t* stage_ids(const uint32_t* ids, uint64_t n);
+    void staged_ids();
     int* dyn_dev = nullptr;    // device ints read by position-dependent kernels
     // pinned staging, double-buffered: a pass may fill one while the previous pass's async
     // copy of the other has not run yet
@@ -307,6 +333,7 @@ struct it_hip {
     template <class F>
     void submit(int fam, uint64_t bytes, uint64_t sig, OpRec rec, F&& f) {
         launches++;
+        if (mode == Mode::Open) open_pass(sig);
         if (mode == Mode::Eager) {
             if (in_pass && pass_tokens == 1) pass_signature.push_back(sig);
             if (in_pass && pass_tokens > 1 && !exact && fuse_enabled) {
@@ -339,7 +366,7 @@ struct it_hip {
         if (mode == Mode::Deferred) return;
         if (mode == Mode::Capture) {
             // queued: the whole pass is fused and captured at end_pass
-        } else if (replay_cursor >= graph.signature.size() || graph.signature[replay_cursor] != sig) {
+        } else if (replay_cursor >= graph->signature.size() || graph->signature[replay_cursor] != sig) {
             need_eager("the op sequence changed");
         } else {
             replay_cursor++;

@@ -159,18 +159,18 @@ void scatter_chunks(const float* src, int64_t src_len, int64_t chunk, int64_t st
 void kv_write(uint16_t* slab, int64_t offset, const int* offset_dyn, int64_t offset_mul, const float* src,
               int64_t n, hipStream_t s);
 void fill_zero(void* p, int64_t bytes, hipStream_t s);
-// n <= POKE_MAX host ints to device memory as one small kernel whose argument block carries them (the host array may be
-// reused as soon as the call returns); false: too many, nothing was launched
+// n <= POKE_MAX host ints to device memory, and (x non-null) the dequantized row `tok` of an embedding table to x, as one
+// small kernel whose argument block carries them (the host array may be reused as soon as the call returns); false: too
+// many, nothing was launched.
 constexpr int POKE_MAX = 256;
-bool poke_ints(int* dst, const int* host_values, int n, hipStream_t s);
+bool poke(int* dst, const int* host_values, int n, const WView* table, int tok, float* x, hipStream_t s);
+// x = the dequantized rows ids[0..n) (a page-locked host array) of an embedding table (Q8_0 repacked, F16, BF16 or F32)
+void embed_rows(const WView& w, const int32_t* ids, int n, float* x, hipStream_t s);
 void argmax(const float* x, int64_t n, int32_t* out, int32_t* scratch_idx, float* scratch_val, hipStream_t s);
-// x = dequantized row `*token` of an embedding table (Q8_0 repacked, F16, BF16 or F32); the id goes to
+// arg-max of the logits and the dequantized embedding row of the winner, in two launches; the id goes to
 // ring[ring_dyn ? *ring_dyn : ring_idx] when ring is non-null
-// arg-max of the logits and the embedding row of the winner (the two above) in two launches instead of three
 void argmax_embed(const float* logits, int64_t n, int32_t* out, int32_t* scratch_idx, float* scratch_val, const WView& w,
                   float* x, int32_t* ring, int ring_idx, const int* ring_dyn, hipStream_t s);
-void embed_row(const WView& w, const int32_t* token, float* x, int32_t* ring, int ring_idx, const int* ring_dyn,
-               hipStream_t s);
 
 // ---- gated delta net ---------------------------------------------------------------
 void ssm_conv(float* state, const float* x, const float* w, int kernel, int nc, int n_tok, float* out, int exact,
