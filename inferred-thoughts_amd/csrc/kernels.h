@@ -28,8 +28,15 @@ bool conv_split_l2(float* state, const float* x, const float* w, int kernel, int
                    float* v_out, int kdim, float eps, hipStream_t s);
 bool gated_norm_silu_q8(const float* core, const float* w, float* z, float* scales, int8_t* quants, int64_t n_heads, float eps,
                         hipStream_t s);
-// two unquantized matrices of one element type over the same batch of activations, one launch (fast mode, > 16 tokens)
-bool float_matmul_pair(const WView& a, const WView& b, const float* x, int n_tok, float* out_a, float* out_b, hipStream_t s);
+// Unquantized matrices: one, or two of one element type read with the same activations (router + shared-gate logit, ssm
+// alpha + beta) as one launch: rows 0 .. n0 are matrix 0's, the next n1 matrix 1's, each with its own output.
+struct FloatMats {
+    const uint8_t *w0, *w1;
+    float *out0, *out1;
+    int n0, n1;
+};
+void float_matmul(const FloatMats& m, int fmt, const float* x, int n_in, int n_tok, float out_scale, int exact, hipStream_t s);
+bool float_matmul_pair(const WView& a, const WView& b, const float* x, int n_tok, float* out_a, float* out_b, int exact, hipStream_t s);
 void repack_q8_0(const uint8_t* raw, int8_t* q, uint16_t* scales, int64_t n_rows, int n_in, hipStream_t s);
 void repack_nvfp4(const uint8_t* raw, uint8_t* nib, uint8_t* scales, int64_t n_rows, int n_in, hipStream_t s);
 
