@@ -284,6 +284,13 @@ int it_hip_embed_argmax(it_hip*, const it_weights* table, const float* logits, u
  * the host and leaves the backend a copy to make: 8 KB a token).  Called inside a pass in place of the host embedding and
  * host_wrote.  Returns 0 without doing anything when the table type is not handled or an id is outside the table. */
 int it_hip_embed_rows(it_hip*, const it_weights* table, const uint32_t* ids, uint64_t n, float* x, uint64_t x_len);
+/* A caller whose single-token passes differ only in position and token says so with a tag of its own (any address; one per
+ * kind of pass), inside the pass, between begin_pass and the first op.  replay_pass then issues a whole pass of that tag at
+ * `pos` (*id: its token, embedded as by it_hip_embed_rows; id NULL: the arg-max, as by it_hip_embed_argmax at ring_index) from
+ * what earlier passes of the tag recorded, in place of begin_pass, the ops and end_pass.  Returns 0, with nothing done, while
+ * it cannot (the tag is new, buffers moved, graphs are off): the caller issues the pass as usual. */
+void it_hip_tag_pass(it_hip*, const void* tag, uint64_t pos);
+int it_hip_replay_pass(it_hip*, const void* tag, uint64_t pos, const uint32_t* id, uint64_t ring_index);
 /* ids filed by it_hip_embed_argmax at ring indices first_index .. first_index + n (waits for the device) */
 void it_hip_read_tokens(it_hip*, uint64_t first_index, uint64_t n, uint32_t* out);
 void it_hip_sync(it_hip*);

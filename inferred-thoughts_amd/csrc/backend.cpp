@@ -6,6 +6,7 @@
 // (/root/reference src/ops/cuda/ops/mod.rs:91-110).
 #include "backend.h"
 
+#include <atomic>
 #include <mutex>
 
 #include <chrono>
@@ -62,7 +63,7 @@ static uint64_t sig_of(const A&... a) {
 const int* it_hip::dyn_slot(int value) {
     if (mode == Mode::Eager) return nullptr;
     if (dyn_count >= DYN_CAP) {
-        need_eager("too many position-dependent launches in one pass");
+        need_eager("too many position-dependent launches in one pass", false);
         return nullptr;
     }
     dyn_host[dyn_count] = value;
@@ -143,7 +144,8 @@ void it_hip::flush_deferred() {
     if (chain_launches) chain_ran = true;
 }
 
-void it_hip::need_eager(const char* why) {
+void it_hip::need_eager(const char* why, bool moved) {
+    res_epoch += moved;
     if (!held.empty()) release_held();   // whatever follows (a copy, a free, a wait) must find the stream complete
     if (mode == Mode::Eager) return;
     (void)why;
@@ -215,6 +217,8 @@ void it_hip::finish_pass() {
                 graph->attn_slots = fused_attn_slots;
                 graph->elided = fused_elided;
                 graph->has_chain = chain_launches > 0;
+                graph->launches = std::move(fused_runs);
+                graph->direct = graph->launches.size() <= 4 && chain_layers <= 4;
                 graph->valid = true;
                 stable_passes = 1;
             } else if (g) {
@@ -233,12 +237,12 @@ void it_hip::finish_pass() {
         graph->replays++;
         if (replay_cursor != graph->signature.size()) {
             mode = Mode::Replay;
-            need_eager("the pass ended early");
+            need_eager("the pass ended early", false);
             return;
         }
         if (!attn_positions_agree(graph->attn_slots)) {
             mode = Mode::Replay;
-            need_eager("a fused attention block's rope, cache-write and context positions do not agree");
+            need_eager("a fused attention block's rope, cache-write and context positions do not agree", false);
             return;
         }
     }
@@ -247,12 +251,89 @@ void it_hip::finish_pass() {
         run_fused(pending);  // the launches the graph holds, each between two events
         check(hipGetLastError(), "kernel launch");
     } else {
-        check(hipGraphLaunch(graph->exec, stream), "hipGraphLaunch");
-        graph_launches++;
+        launch(*graph);
     }
     mark_elided(graph->elided);
     if (graph->has_chain) chain_ran = true;
+    if (!profile_pass) learn(*graph);
     pending.clear();
+}
+
+void it_hip::launch(Graph& g) {
+    // Up to four launches with small argument blocks go out one by one, 7 us a token sooner on two layers (70.6 against 77.7 us
+    // back to back).  A chain of more than four layers has a 30 KB block, which the graph holds and a launch copies (48
+    // layers: 1.419 ms a token so, 1.407 as a graph), and long lists cost the host more than the graph does.
+    if (g.direct) {
+        for (auto& f : g.launches) f(stream);
+        check(hipGetLastError(), "kernel launch");
+        graph_launches++;
+        return;
+    }
+    check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
+    graph_launches++;
+}
+
+// After a recorded pass was launched: what a later one of the same tag needs to be launched without being recorded again.
+// The scalars of two passes at different positions tell which follow the position (they move with it, one for one) and
+// which are fixed; anything else keeps the tag's passes recorded.
+void it_hip::learn(Graph& g) {
+    if (!pass_tag || (g.known && g.epoch == res_epoch)) return;
+    const bool second = g.tag == pass_tag && g.pos != pass_pos && g.dyn.size() == dyn_count && g.ring_slot == pass_ring_slot;
+    g.known = second;
+    if (second) {
+        const int64_t step = (int64_t)pass_pos - (int64_t)g.pos;
+        g.moves.assign(dyn_count, 0);
+        for (size_t i = 0; i < dyn_count; i++) {
+            const int64_t d = (int64_t)dyn_host[i] - g.dyn[i];
+            g.moves[i] = d != 0;
+            if ((int)i != g.ring_slot && d != 0 && d != step) g.known = false;
+        }
+        g.epoch = res_epoch;
+        g.pos_cap = ~0ull;
+        for (auto& r : ropes) g.pos_cap = std::min<uint64_t>(g.pos_cap, r.second.cap_pos);
+        g.left.clear();
+        for (auto& kv : acts)
+            if (kv.second.dev_current) g.left.push_back({&kv.second, kv.second.elided, kv.second.q_valid, kv.second.q_len});
+    }
+    g.tag = pass_tag;
+    g.pos = pass_pos;
+    g.ring_slot = pass_ring_slot;
+    g.table = pass_embed.table;
+    g.x = pass_embed.x;
+    g.dyn.assign(dyn_host, dyn_host + dyn_count);
+}
+
+// A whole single-token pass whose kind is known, launched from its graph: the 35 ops of a layer are not issued, hashed and
+// compared again (35 us of host time for two layers, in front of 75 us on the device).
+bool it_hip::replay_pass(const void* tag, uint64_t pos, const uint32_t* id, uint64_t ring_index) {
+    if (in_pass || !allow_graph || mid_pass_read || has_error || prof_on || expert_cold_entries || pool_tabled || !held.empty()) return false;
+    Graph* g = nullptr;
+    for (Graph& c : graphs)
+        if (c.valid && c.known && c.tag == tag && c.epoch == res_epoch && pos < c.pos_cap && (c.ring_slot >= 0) == (id == nullptr)) g = &c;
+    if (!g || (id && (!g->x || *id >= (uint32_t)g->table.n_out))) return false;
+    dyn_rotate();
+    dyn_count = g->dyn.size();
+    for (size_t i = 0; i < dyn_count; i++) dyn_host[i] = g->dyn[i] + (g->moves[i] ? (int)((int64_t)pos - (int64_t)g->pos) : 0);
+    if (id) pre_embed = {g->table, (int)*id, g->x};
+    else dyn_host[g->ring_slot] = (int)(ring_index % TOK_RING_CAP);
+    issue_inputs();
+    launch(*g);
+    g->replays++;
+    launches += g->signature.size();
+    for (auto& kv : acts) {
+        kv.second.dev_current = false;
+        kv.second.elided = false;
+        kv.second.q_valid = false;
+    }
+    for (const Graph::Left& l : g->left) {
+        l.a->dev_current = true;
+        l.a->elided = l.elided;
+        l.a->q_valid = l.q_valid;
+        l.a->q_len = l.q_len;
+    }
+    route_gen++;
+    if (g->has_chain) chain_ran = true;
+    return true;
 }
 
 bool it_hip::attn_positions_agree(const std::vector<std::array<int, 4>>& slots) const {
@@ -1165,6 +1246,9 @@ it_hip::~it_hip() {
     if (argmax_val) (void)hipFree(argmax_val);
     if (argmax_out) (void)hipFree(argmax_out);
     if (argmax_host) (void)hipHostFree(argmax_host);
+    if (home.cells) (void)hipHostFree(home.cells);
+    if (home.arrived) (void)hipFree(home.arrived);
+    if (home.stage) (void)hipHostFree(home.stage);
     for (auto& st : id_stage) {
         if (st.host) (void)hipHostFree(st.host);
         if (st.evt) (void)hipEventDestroy(st.evt);
@@ -1237,7 +1321,9 @@ void it_hip::chain_check() {
         (void)hipGetLastError();
         return;
     }
-    if (!flag) return;
+    if (flag) chain_gave_up();
+}
+void it_hip::chain_gave_up() {
     // a wait inside a chain ran out of tries: what the pass computed is void.  The chains are switched off for this
     // backend, the graph that holds them is dropped and the hand-off space starts from zero again.
     chain_enabled = false;
@@ -2064,8 +2150,8 @@ void it_hip_kv_write(it_hip* be, uint16_t* slab, uint64_t slab_len, uint64_t off
             mul = n;
             off = 0;
         }
-    } else {
-        be->need_eager("a kv_write offset is not a whole row");
+    } else if (be->mode != it_hip::Mode::Eager) {
+        be->need_eager("a kv_write offset is not a whole row", false);
     }
     it_hip::OpRec rec;
     rec.id = OP_KVWRITE; rec.p[0] = dslab; rec.p[1] = dyn; rec.p[2] = ds; rec.i[0] = mul; rec.i[1] = off; rec.i[2] = n;
@@ -2114,12 +2200,14 @@ void it_hip_host_needs(it_hip* be, float* buf, uint64_t len) {
         // a read inside a pass cannot be served from a graph that has not run yet:
         // graphs are latched off for this backend (src/ops/cuda/ops/mod.rs:565-582)
         be->mid_pass_read = true;
-        be->need_eager("the host read a device buffer inside a pass");
+        be->need_eager("the host read a device buffer inside a pass", false);
     }
     size_t n = len < it->second.cap ? len : it->second.cap;
-    if (!be->check(hipMemcpyAsync(buf, it->second.dev, n * sizeof(float), hipMemcpyDeviceToHost, be->stream), "download activation")) return;
-    be->check(hipStreamSynchronize(be->stream), "download activation");
-    be->chain_check();
+    if (!be->fetch(it->second, buf, n)) {
+        if (!be->check(hipMemcpyAsync(buf, it->second.dev, n * sizeof(float), hipMemcpyDeviceToHost, be->stream), "download activation")) return;
+        be->check(hipStreamSynchronize(be->stream), "download activation");
+        be->chain_check();
+    }
     be->d2h++;
     be->d2h_bytes += n * 4;
 }
@@ -2137,6 +2225,9 @@ void it_hip_begin_pass(it_hip* be, uint64_t n_tokens) {
     be->pending.clear();
     be->precopies.clear();
     be->pre_embed.x = nullptr;
+    be->pass_tag = nullptr;
+    be->pass_embed.x = nullptr;
+    be->pass_ring_slot = -1;
     be->dyn_rotate();
     be->replay_cursor = 0;
     be->mode = it_hip::Mode::Eager;
@@ -2157,6 +2248,16 @@ void it_hip_begin_pass(it_hip* be, uint64_t n_tokens) {
     }
 }
 
+void it_hip_tag_pass(it_hip* be, const void* tag, uint64_t pos) {
+    if (!be->in_pass || be->pass_tokens != 1) return;
+    be->pass_tag = tag;
+    be->pass_pos = pos;
+}
+
+int it_hip_replay_pass(it_hip* be, const void* tag, uint64_t pos, const uint32_t* id, uint64_t ring_index) {
+    return tag && be->replay_pass(tag, pos, id, ring_index) ? 1 : 0;
+}
+
 void it_hip_end_pass(it_hip* be) {
     if (!be->in_pass) return;
     be->finish_pass();
@@ -2164,25 +2265,29 @@ void it_hip_end_pass(it_hip* be) {
 }
 
 void it_hip_forget_state(it_hip* be) {
+    be->res_epoch++;
     for (auto& kv : be->slabs)
         if (kv.second.is_state) kv.second.dev_owned = false;
 }
 
 void it_hip_zero_state(it_hip* be) {
     // the host copies were just zeroed: zero the device copies in place instead of uploading zeros at the next use
+    std::vector<itk::ZeroSpan> spans;
     for (auto& kv : be->slabs) {
         if (!kv.second.is_state) continue;
         if (kv.second.dev) {
-            fill_zero(kv.second.dev, (int64_t)kv.second.bytes, be->stream);
+            spans.push_back({(uint32_t*)kv.second.dev, (int64_t)kv.second.bytes / 4});
+            if (!kv.second.dev_owned) be->res_epoch++;
             kv.second.dev_owned = true;
         } else {
             kv.second.dev_owned = false;
         }
     }
+    zero_spans(spans.data(), (int)spans.size(), be->stream);
 }
 
 void it_hip_read_state(it_hip* be, float* host, uint64_t len) {
-    be->need_eager("a state slab is read");
+    be->need_eager("a state slab is read", false);
     auto it = be->slabs.find(host);
     if (it == be->slabs.end() || !it->second.dev_owned) return;
     size_t bytes = len * 4 < it->second.bytes ? len * 4 : it->second.bytes;
@@ -2193,7 +2298,7 @@ void it_hip_read_state(it_hip* be, float* host, uint64_t len) {
 }
 
 void it_hip_read_kv(it_hip* be, uint16_t* slab, uint64_t len) {
-    be->need_eager("a kv slab is read");
+    be->need_eager("a kv slab is read", false);
     auto it = be->slabs.find(slab);
     if (it == be->slabs.end() || !it->second.dev_owned) return;
     size_t bytes = len * 2 < it->second.bytes ? len * 2 : it->second.bytes;
@@ -2382,6 +2487,55 @@ int64_t it_hip_clock_pick(uint8_t* heat, const uint8_t* leased, uint64_t n, uint
 // ------------------------------------------------------------------ extensions
 }  // extern "C"
 
+// A read by the host: a kernel behind the pass writes the floats, the chains' abort word and then a sequence number into
+// page-locked memory, and the host watches that number.  Against a copy, a stream synchronisation and a second copy for the
+// abort word (32 KB: 45 us after the pass's last kernel) the host has the values a few microseconds after it.
+bool it_hip::fetch(Act& a, float* buf, size_t n) {
+    constexpr size_t MAX = 1 << 18;   // floats
+    if (!n || n > MAX) return false;
+    if (!home.cells) {
+        unsigned* p = nullptr;
+        if (hipHostMalloc((void**)&p, 256, hipHostMallocDefault) != hipSuccess || hipMalloc((void**)&home.arrived, 4) != hipSuccess ||
+            hipHostMalloc((void**)&home.stage, MAX * 4, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        memset(p, 0, 256);
+        fill_zero(home.arrived, 4, stream);
+        home.cells = p;
+    }
+    if (a.host_locked < 0) {
+        hipPointerAttribute_t at;
+        a.host_locked = hipPointerGetAttributes(&at, buf) == hipSuccess && at.type == hipMemoryTypeHost && (((uintptr_t)buf) & 15) == 0;
+        (void)hipGetLastError();
+    }
+    float* to = a.host_locked ? buf : home.stage;
+    const unsigned seq = ++home.seq;
+    itk::fetch(a.dev, to, (int64_t)n, chain_ran ? chain.abort_flag : nullptr, home.cells + 16, home.arrived, home.cells, seq, stream);
+    if (!check(hipGetLastError(), "download activation")) return true;
+    volatile unsigned* flag = home.cells;
+    const uint64_t t0 = now_us();
+    for (uint64_t i = 1; *flag != seq; i++) {
+        __builtin_ia32_pause();
+        // a long wait (a prompt's passes): let the runtime do the waiting, and report a fault if there is one
+        if ((i & 1023) == 0 && now_us() - t0 > 2000) {
+            if (!check(hipStreamSynchronize(stream), "download activation")) return true;
+            break;
+        }
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    if (*flag != seq) {
+        fail("download activation: the device did not report the end of the pass");
+        return true;
+    }
+    if (!a.host_locked) memcpy(buf, to, n * sizeof(float));
+    if (chain_ran) {
+        chain_ran = false;
+        if (home.cells[16]) chain_gave_up();
+    }
+    return true;
+}
+
 // Page-locked copies of a batch's token ids, two in turn: a pass may be issued while the one before it still runs.
 const int32_t* it_hip::stage_ids(const uint32_t* ids, uint64_t n) {
     IdStage& st = id_stage[id_cur ^= 1];
@@ -2420,7 +2574,7 @@ uint32_t it_hip_argmax(it_hip* be, const float* buf, uint64_t len) {
     float* d = be->act_in(buf, len);
     if (!d) return 0;
     if (!be->argmax_ready()) return 0;
-    be->need_eager("argmax");
+    be->need_eager("argmax", false);
     argmax(d, (int64_t)len, be->argmax_out, be->argmax_idx, be->argmax_val, be->stream);
     be->launches += 2;
     if (!be->check(hipMemcpyAsync(be->argmax_host, be->argmax_out, 4, hipMemcpyDeviceToHost, be->stream), "download argmax")) return 0;
@@ -2443,6 +2597,7 @@ int it_hip_embed_rows(it_hip* be, const it_weights* table, const uint32_t* ids, 
     if (n == 1 && be->mode != it_hip::Mode::Eager) {
         // a recorded pass: the row is made by the small kernel that carries the pass's positions
         be->pre_embed = {w, (int)ids[0], dx};
+        be->pass_embed = be->pre_embed;
         return 1;
     }
     be->launches++;
@@ -2478,6 +2633,7 @@ int it_hip_embed_argmax(it_hip* be, const it_weights* table, const float* logits
     if (!dx || !be->argmax_ready()) return 0;
     const int slot = (int)(ring_index % it_hip::TOK_RING_CAP);
     const int* dyn = be->dyn_slot(slot);
+    if (dyn) be->pass_ring_slot = (int)(dyn - be->dyn_dev);
     int32_t *out = be->argmax_out, *idx = be->argmax_idx, *ring = be->tok_ring;
     float* val = be->argmax_val;
     int64_t n = (int64_t)logits_len;
@@ -2553,7 +2709,7 @@ void it_hip_chain_stats(it_hip* be, uint64_t out[4]) {
 }
 
 void it_hip_profile_begin(it_hip* be) {
-    be->need_eager("profiling");
+    be->need_eager("profiling", false);
     be->check(hipStreamSynchronize(be->stream), "sync");
     be->prof_spans.clear();
     be->prof_pool_next = 0;

@@ -71,7 +71,16 @@ struct it_hip {
         size_t q_cap = 0;  // floats covered
         size_t q_len = 0;
         bool q_valid = false;
+        int host_locked = -1;  // the host buffer is page-locked (fetch): not asked yet, no, yes
     };
+    struct Home {
+        unsigned* cells = nullptr;     // page-locked: [0] sequence number, [16] abort word
+        unsigned* arrived = nullptr;   // device: blocks of a fetch that are done
+        float* stage = nullptr;        // page-locked, for host buffers that are not
+        unsigned seq = 0;
+    };
+    Home home;
+    bool fetch(Act& a, float* buf, size_t n);
     std::unordered_map<const void*, Act> acts;
     Act* act_slot(const float* host, size_t len);
     float* act_in(const float* host, size_t len);     // device copy current for reading
@@ -214,6 +223,24 @@ struct it_hip {
         std::vector<uint64_t> signature;  // hash of each seam call's static arguments
         bool valid = false;
         uint64_t born = 0, replays = 0;
+        std::vector<std::function<void(hipStream_t)>> launches;   // what the graph holds
+        bool direct = false;         // launched one by one (launch)
+        // replay_pass: the caller's tag of this kind of pass, a pass it recorded (position, position scalars) and, once a
+        // second pass has shown which scalars follow the position, what a pass leaves behind (the mirrors that are current)
+        const void* tag = nullptr;
+        uint64_t pos = 0, pos_cap = 0, epoch = 0;
+        std::vector<int> dyn;
+        std::vector<uint8_t> moves;
+        int ring_slot = -1;          // the scalar that is the token ring's index (a pass fed by the arg-max), or -1
+        itk::WView table{};          // the embedding table and row of a pass fed by the host
+        float* x = nullptr;
+        bool known = false;
+        struct Left {
+            Act* a;
+            bool elided, q_valid;
+            size_t q_len;
+        };
+        std::vector<Left> left;
         // position slots of every fused attention block: {rope, key write, value write, attend}.  The fused kernel
         // takes ONE position for all four, so a replay is only valid while write row == rope position and the
         // context length == position + 1 (the seam does not tie them together; the model loop does)
@@ -226,6 +253,12 @@ struct it_hip {
     std::array<Graph, 4> graphs;
     Graph* graph = nullptr;
     uint64_t graph_unused = 0;   // graphs dropped without a replay
+    const void* pass_tag = nullptr;
+    uint64_t pass_pos = 0;
+    int pass_ring_slot = -1;
+    void learn(Graph& g);
+    void launch(Graph& g);
+    bool replay_pass(const void* tag, uint64_t pos, const uint32_t* id, uint64_t ring_index);
     void drop_one(Graph& g);
     void open_pass(uint64_t sig);
     // Deferred: a single-token pass whose ops are recorded like a captured pass's and issued as fused launches whenever
@@ -254,6 +287,7 @@ struct it_hip {
     bool fuse_enabled = true;
     unsigned* route_counter = nullptr;  // device word used by the fused router (zero between launches)
     uint64_t fused_launches = 0;  // launches in the captured graph after fusion
+    std::vector<std::function<void(hipStream_t)>> fused_runs;   // those launches
     void run_fused(std::vector<OpRec>& ops);
     std::vector<std::array<int, 4>> fused_attn_slots;  // filled by run_fused for the pass being captured
     // ---- layer chains (k_chain.hip): runs of decode layers as one persistent kernel each
@@ -276,6 +310,7 @@ struct it_hip {
     uint64_t chain_launches = 0, chain_layers = 0;   // per fused pass, for the statistics
     bool chain_acquire();
     void chain_release();
+    void chain_gave_up();
     void chain_check();                // after a stream synchronisation: raises the sticky error if a chain gave up
     std::vector<const void*> fused_elided;   // device buffers the pass being fused no longer writes (filled by run_fused)
     bool attn_positions_agree(const std::vector<std::array<int, 4>>& slots) const;
@@ -298,7 +333,7 @@ struct it_hip {
         int token;
         float* x;
     };
-    PreEmbed pre_embed{};
+    PreEmbed pre_embed{}, pass_embed{};   // pass_embed: kept to the end of the pass
     void issue_inputs();
     struct IdStage {
         int32_t* host = nullptr;   // page-locked
@@ -323,7 +358,10 @@ struct it_hip {
     size_t dyn_count = 0;
     static constexpr size_t DYN_CAP = 4096;
     const int* dyn_slot(int value);   // null in eager mode: the kernel takes the scalar by value
-    void need_eager(const char* why); // leave capture/replay: run what the pass queued so far eagerly
+    // leave capture/replay: run what the pass queued so far eagerly.  `moved`: a buffer is about to be allocated, moved or
+    // filled anew, so that what earlier passes found in place has to be looked at again (replay_pass)
+    void need_eager(const char* why, bool moved = true);
+    uint64_t res_epoch = 0;
     void finish_pass();
     bool mid_pass_read = false;
     bool profile_pass = false;  // a replay-shaped pass whose fused launches run one by one between timing events
@@ -367,7 +405,7 @@ struct it_hip {
         if (mode == Mode::Capture) {
             // queued: the whole pass is fused and captured at end_pass
         } else if (replay_cursor >= graph->signature.size() || graph->signature[replay_cursor] != sig) {
-            need_eager("the op sequence changed");
+            need_eager("the op sequence changed", false);
         } else {
             replay_cursor++;
         }

@@ -1222,18 +1222,18 @@ void it_hip::run_fused(std::vector<OpRec>& ops) {
         }
     }
     if (fuse_enabled && !expert_cold_entries) build_chains(pl, expert_tally);
-    uint64_t n = 0;
+    fused_runs.clear();
     for (size_t i = 0; i < ops.size(); i++) {
         for (auto& l : pl.at[i]) {
             Span sp(this, l.fam, l.bytes);
             l.fn(stream);
-            n++;
+            fused_runs.push_back(l.fn);
         }
         if (!pl.consumed[i]) {
             Span sp(this, FAM_OTHER, 0);
             ops[i].run(stream);
-            n++;
+            fused_runs.push_back(ops[i].run);
         }
     }
-    fused_launches = n;
+    fused_launches = fused_runs.size();
 }

@@ -330,6 +330,33 @@ __global__ void kv_write_k(uint16_t* __restrict__ slab, int64_t offset, const in
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         slab[off + i] = it_f32_to_f16(src[i]);
 }
+// several buffers in one launch (a sequence reset: two state slabs a recurrent layer), a grid row each
+constexpr int ZERO_SPANS = 64;
+struct ZeroSpans {
+    ZeroSpan s[ZERO_SPANS];
+};
+__global__ __launch_bounds__(256) void zero_spans_k(ZeroSpans z) {
+    const ZeroSpan sp = z.s[blockIdx.y];
+    const int64_t quads = sp.words / 4;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) ((uint4*)sp.p)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (blockIdx.x == 0 && threadIdx.x < (sp.words & 3)) sp.p[quads * 4 + threadIdx.x] = 0u;
+}
+// Floats into page-locked host memory, then (with everything of every block there) the abort word and the sequence number
+// that the host waits for.  `arrived` is zero between launches.
+__global__ __launch_bounds__(256) void fetch_k(const float* __restrict__ src, float* __restrict__ dst, int64_t n, const unsigned* abort_word,
+                                               unsigned* abort_to, unsigned* arrived, unsigned* flag, unsigned seq) {
+    const int64_t quads = n / 4;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) ((float4*)dst)[i] = ((const float4*)src)[i];
+    if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dst[quads * 4 + threadIdx.x] = src[quads * 4 + threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0 && atomicAdd(arrived, 1u) == gridDim.x - 1) {
+        *arrived = 0u;
+        if (abort_word) *(volatile unsigned*)abort_to = *(const volatile unsigned*)abort_word;
+        __threadfence_system();
+        __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
 __global__ void fill_zero_k(uint32_t* p, int64_t n_words) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words;
          i += (int64_t)gridDim.x * blockDim.x)
@@ -431,6 +458,23 @@ void scatter_chunks(const float* src, int64_t src_len, int64_t chunk, int64_t st
 void kv_write(uint16_t* slab, int64_t offset, const int* offset_dyn, int64_t offset_mul, const float* src,
               int64_t n, hipStream_t s) {
     EW_LAUNCH(kv_write_k, n, slab, offset, offset_dyn, offset_mul, src, n);
+}
+void fetch(const float* src, float* dst, int64_t n, const unsigned* abort_word, unsigned* abort_to, unsigned* arrived, unsigned* flag, unsigned seq,
+           hipStream_t s) {
+    hipLaunchKernelGGL(fetch_k, dim3((unsigned)std::min<int64_t>((n + 2047) / 2048, 64)), dim3(256), 0, s, src, dst, n, abort_word, abort_to, arrived,
+                       flag, seq);
+}
+void zero_spans(const ZeroSpan* spans, int n, hipStream_t s) {
+    for (int at = 0; at < n; at += ZERO_SPANS) {
+        ZeroSpans z;
+        const int take = std::min(n - at, ZERO_SPANS);
+        int64_t most = 1;
+        for (int i = 0; i < take; i++) {
+            z.s[i] = spans[at + i];
+            most = std::max(most, z.s[i].words);
+        }
+        hipLaunchKernelGGL(zero_spans_k, dim3((unsigned)std::min<int64_t>((most + 4095) / 4096, 256), take), dim3(256), 0, s, z);
+    }
 }
 void fill_zero(void* p, int64_t bytes, hipStream_t s) {
     int64_t words = bytes / 4;

@@ -166,6 +166,15 @@ void scatter_chunks(const float* src, int64_t src_len, int64_t chunk, int64_t st
 void kv_write(uint16_t* slab, int64_t offset, const int* offset_dyn, int64_t offset_mul, const float* src,
               int64_t n, hipStream_t s);
 void fill_zero(void* p, int64_t bytes, hipStream_t s);
+struct ZeroSpan {
+    uint32_t* p;   // 16-byte aligned
+    int64_t words;
+};
+void zero_spans(const ZeroSpan* spans, int n, hipStream_t s);
+// n floats to page-locked host memory (16-byte aligned), *abort_word (may be null) to *abort_to, then `seq` to *flag, all
+// visible to the host in that order; *arrived is zero before and after
+void fetch(const float* src, float* dst, int64_t n, const unsigned* abort_word, unsigned* abort_to, unsigned* arrived, unsigned* flag, unsigned seq,
+           hipStream_t s);
 // n <= POKE_MAX host ints to device memory, and (x non-null) the dequantized row `tok` of an embedding table to x, as one
 // small kernel whose argument block carries them (the host array may be reused as soon as the call returns); false: too
 // many, nothing was launched.

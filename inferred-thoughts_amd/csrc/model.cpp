@@ -291,6 +291,7 @@ struct it_engine {
     uint64_t ring_next = 0;  // next slot of the backend's device token ring this engine files into
     std::vector<uint16_t> k_slabs, v_slabs;
     std::vector<float> conv, ssm;
+    bool host_state = false;   // a state was written to the host copies (read home, or restored) since they were zeros
     it_trace_fn trace = nullptr;
     void* trace_user = nullptr;
     std::string err;
@@ -424,6 +425,20 @@ void gated_delta(it_engine* e, const Block& b, uint64_t il, uint64_t n) {
     e->tr("linear_attn_out", il, e->mixed, n * nd);
 }
 
+// The end of a pass: the logits come home if they are wanted.  A pass whose logits stay on the device does not wait for it
+// (the host goes on to issue the next one), and one whose logits have come home is over: only an error already recorded is
+// looked at, and the caller polls, with a wait, after its last pass.
+int finish(it_engine* e, bool want_logits, bool host_fed) {
+    const uint64_t nv = e->m->d.n_vocab;
+    if (want_logits) it_hip_host_needs(e->be, e->logits.p(), nv);
+    if (e->trace) e->tr("result_output", 0, e->logits, nv);
+    if (!host_fed && !it_hip_has_error(e->be)) return 0;
+    char msg[512];
+    if (!it_hip_take_error(e->be, msg, sizeof msg)) return 0;
+    e->err = msg;
+    return -10;
+}
+
 // Runs one pass; logits stay on the device unless `want_logits`.
 // `tokens == nullptr` is the greedy feedback pass: one token, chosen on the device as the arg-max
 // of the previous pass's logits and embedded there (its id lands at `ring_index` of the device ring).
@@ -437,7 +452,14 @@ int forward(it_engine* e, const uint32_t* tokens, uint64_t n, uint64_t start, bo
     for (uint64_t t = 0; tokens && t < n; t++)
         if (tokens[t] >= d.n_vocab) { e->err = "token id " + std::to_string(tokens[t]) + " outside the vocabulary"; return -3; }
     uint64_t nd = d.n_embd;
+    // two kinds of single-token pass: fed by the caller, and by the arg-max
+    const void* tag = n == 1 && !e->trace ? (tokens ? (const void*)e : (const void*)&e->len) : nullptr;
+    if (tag && it_hip_replay_pass(be, tag, start, tokens, ring_index)) {
+        e->len = start + n;
+        return finish(e, want_logits, false);
+    }
     it_hip_begin_pass(be, n);
+    if (tag) it_hip_tag_pass(be, tag, start);
     if (!fit(e, n)) {
         it_hip_end_pass(be);
         e->err = "cannot allocate the page-locked logits buffer";
@@ -484,17 +506,7 @@ int forward(it_engine* e, const uint32_t* tokens, uint64_t n, uint64_t start, bo
     it_hip_matmul(be, &m->output, e->final_norm.p(), nd, e->logits.p(), d.n_vocab);
     if (m->has_output_scale) it_hip_scale(be, e->logits.p(), d.n_vocab, m->output_scale);
     it_hip_end_pass(be);
-    if (want_logits) it_hip_host_needs(be, e->logits.p(), d.n_vocab);
-    if (e->trace) e->tr("result_output", 0, e->logits, d.n_vocab);
-    // a pass whose logits stay on the device does not wait for it (the host goes on to issue the next one): only an
-    // error already recorded is looked at, and the caller polls, with a wait, after its last pass
-    if (!want_logits && !host_fed && !it_hip_has_error(be)) return 0;
-    char msg[512];
-    if (it_hip_take_error(be, msg, sizeof msg)) {
-        e->err = msg;
-        return -10;
-    }
-    return 0;
+    return finish(e, want_logits, host_fed);
 }
 
 uint32_t host_argmax(const float* l, uint64_t n) {  // src/profile.rs:192-213
@@ -631,8 +643,11 @@ void it_engine_free(it_engine* e) {
 // Engine::reset, src/engine/mod.rs:296-306
 void it_engine_reset(it_engine* e) {
     e->len = 0;
-    std::fill(e->conv.begin(), e->conv.end(), 0.0f);
-    std::fill(e->ssm.begin(), e->ssm.end(), 0.0f);
+    if (e->host_state) {   // else the host copies are the zeros they were made as
+        std::fill(e->conv.begin(), e->conv.end(), 0.0f);
+        std::fill(e->ssm.begin(), e->ssm.end(), 0.0f);
+        e->host_state = false;
+    }
     it_hip_zero_state(e->be);
 }
 // Engine::checkpoint / restore / rewind, src/engine/mod.rs:223-294.  The device owns the recurrent state once it has
@@ -645,6 +660,7 @@ void it_engine_state_sizes(const it_engine* e, uint64_t out[2]) {
 }
 uint64_t it_engine_checkpoint(it_engine* e, float* conv_out, float* ssm_out) {
     const Dims& d = e->m->d;
+    e->host_state = true;
     for (uint64_t il = 0; il < d.layers(); il++) {
         if (!d.recurrent(il)) continue;
         it_hip_read_state(e->be, e->conv_of(il), d.conv_len());
@@ -664,6 +680,7 @@ int it_engine_restore(it_engine* e, uint64_t pos, const float* conv_in, const fl
         return -2;
     }
     e->len = pos;
+    e->host_state = true;
     memcpy(e->conv.data(), conv_in, e->conv.size() * sizeof(float));
     memcpy(e->ssm.data(), ssm_in, e->ssm.size() * sizeof(float));
     it_hip_forget_state(e->be);  // after both halves
@@ -768,11 +785,13 @@ int64_t it_engine_decode_greedy(it_engine* e, uint64_t n, uint32_t* out_ids) {
 
 const float* it_engine_ssm_state(it_engine* e, uint64_t layer, uint64_t* len) {
     *len = e->m->d.ssm_len();
+    e->host_state = true;
     it_hip_read_state(e->be, e->ssm_of(layer), *len);
     return e->ssm_of(layer);
 }
 const float* it_engine_conv_state(it_engine* e, uint64_t layer, uint64_t* len) {
     *len = e->m->d.conv_len();
+    e->host_state = true;
     it_hip_read_state(e->be, e->conv_of(layer), *len);
     return e->conv_of(layer);
 }
