@@ -209,13 +209,16 @@ __global__ __launch_bounds__(256) void attend_split_k(AttnArgs a, int n_split, f
 constexpr int TILE = 64;
 
 // ------------------------------------------------------------------ split-K for a few queries on the f16 matrix cores
-// One block per (query, kv head, key range): the live context is cut into n_split equal ranges (a multiple
+// One block per (query, kv head, key range), or (TWO) per pair of queries: the live context is cut into n_split equal ranges (a multiple
 // of 16 keys), so every block has work whatever the position.  A range is walked in tiles of 64 keys; a tile's K
-// (as stored, [key][dim]) and V (transposed on the way in, [dim][key]) are staged in LDS with coalesced 16-byte
-// loads, the next tile's loads in flight while the current one is used.
+// (as stored, [key][dim]) and V (transposed on the way in, [dim][key]) are staged in LDS with coalesced 16-byte loads, the next tile's loads in flight while the current one is used.  Bound by latency, a chain of load, two LDS
+// round trips and two short products, until the range streams.  16 query heads of 256, 2 KV heads: 10 us with the merge at
+// 1,024 positions, 21 us (3.1 TB/s) at 32,000; five queries at 5,431: 16.6 us (21.4 with a block per query).
 //     S^T = K Q^T   (32 keys x 32 columns per MFMA tile): the G query heads sit in columns 0..G-1 as the high
 //                   f16 halves of the scaled query and in columns 8..8+G-1 as the low halves, so one
-//                   product carries both and a lane move within its row of 16 lanes adds them;
+//                   product carries both and a lane move within its row of 16 lanes adds them; with TWO, columns 16..31
+//                   hold the next query's heads the same way: a verify batch reads K and V half as often (V then takes K's
+//                   place in LDS, so that two blocks still share a CU);
 //     O^T = V^T P^T (32 dims x 32 columns per MFMA tile).
 // All four waves form the same scores (they run on different SIMDs, so the repetition costs no time and
 // saves every exchange: each wave has the whole P^T in registers and the same running maximum and sum);
@@ -236,8 +239,14 @@ IT_DEV float row_ror8(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));
 }
 
-template <int HD, int G, bool PREP>
-__global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr, int n_split, float* __restrict__ part) {
+template <int HD, bool TWO> constexpr int decode_vt_at() { return TWO ? 0 : TILE * (HD + 8); }
+template <int HD, bool TWO> constexpr int decode_q_at() {
+    return TWO && TILE * (HD + 8) > HD * DVS ? TILE * (HD + 8) : decode_vt_at<HD, TWO>() + HD * DVS;
+}
+template <bool TWO> constexpr int decode_q_rows() { return TWO ? 32 : 17; }
+
+template <int HD, int G, bool PREP, bool TWO>
+__global__ __launch_bounds__(256, 2) void attend_decode_k(AttnArgs a, TilePrepP pr, int n_split, float* __restrict__ part) {
     constexpr int KS = HD + 8;                  // row stride of K and of the query rows in LDS, in f16
     constexpr int NS = HD / 16;                 // k steps of a score tile
     constexpr int ND = HD / 32;                 // output tiles along the head dimension
@@ -245,35 +254,31 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
     constexpr int KSEG = TILE * HD / 8 / 256;   // 16-byte pieces of K per thread
     constexpr int UNITS = (TILE / 4) * (HD / 8);  // 4-key x 8-dim pieces of V per tile
     constexpr int VU = (UNITS + 255) / 256;     // per thread
-    constexpr int QROWS = 17;                   // high halves of 8 heads, low halves of 8 heads, a row of zeros
-    static_assert(G <= 8, "hi and lo halves of the query heads share the 32 columns in two groups of 8");
+    constexpr int QROWS = decode_q_rows<TWO>(); // high halves of 8 heads, low halves of 8 heads; the next query's, or a row of zeros
+    static_assert(G <= 8, "hi and lo halves of the query heads share 16 columns in two groups of 8");
     extern __shared__ __align__(16) uint16_t dlds[];
     uint16_t* Ks = dlds;                      // [64][KS]
-    uint16_t* Vt = dlds + TILE * KS;          // [HD][DVS]
-    uint16_t* Qs = Vt + HD * DVS;             // [17][KS]
+    uint16_t* Vt = dlds + decode_vt_at<HD, TWO>();   // [HD][DVS] (TWO: in K's place, once the scores are formed)
+    uint16_t* Qs = dlds + decode_q_at<HD, TWO>();    // [QROWS][KS]
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 31, g = lane >> 5;
-    const int t = blockIdx.x / a.n_head_kv, kvh = blockIdx.x % a.n_head_kv;
+    const int t = (TWO ? 2 : 1) * (blockIdx.x / a.n_head_kv), kvh = blockIdx.x % a.n_head_kv;
+    const bool two = TWO && t + 1 < a.n_q;                          // queries t and t + 1
     const int split = blockIdx.y;
     ATTN_STAMP(0);
     const int n_pos_last = a.n_pos_dyn ? *a.n_pos_dyn : a.n_pos;
-    const int n_pos = n_pos_last - a.n_q + 1 + t;
+    const int n_pos = n_pos_last - a.n_q + 1 + t + (two ? 1 : 0);   // of the later query
+    const int my_pos = two && c < 16 ? n_pos - 1 : n_pos;           // of this lane's column
     const int h0 = kvh * G;
+    const int64_t part_query_stride = (int64_t)a.n_head * n_split * (HD + 2);
     float* my_part = part + (((int64_t)t * a.n_head + h0) * n_split + split) * (HD + 2);
     const int64_t part_head_stride = (int64_t)n_split * (HD + 2);
     // keys per block: the live context over the blocks, in whole groups of 16
     const int kpb = max(16, ((n_pos + n_split - 1) / n_split + 15) & ~15);
     const int k0 = split * kpb, k1 = min(n_pos, k0 + kpb);
-    if (k0 >= k1) {
-        if (tid < G) {
-            float* p = my_part + tid * part_head_stride;
-            p[HD] = -INFINITY;
-            p[HD + 1] = 0.0f;
-        }
-        return;
-    }
+    // (a range without keys leaves its marks at the end, like every other)
     ATTN_STAMP(1);
-    const int n_kt = (k1 - k0 + TILE - 1) / TILE;
+    const int n_kt = max(0, k1 - k0 + TILE - 1) / TILE;
     const uint16_t* kbase = a.k + kvh * HD;
     const uint16_t* vbase = a.v + kvh * HD;
 
@@ -336,7 +341,7 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
     };
 
     // The query heads as rows of Q^T's columns in LDS: row h = high f16 halves of head h (scaled), row 8 + h = the
-    // low halves, row 16 = zeros (what the columns without a head read).  Their loads go out ahead of the tile's.
+    // low halves, rows 16 .. 31 the next query's (one query: row 16 zeros); zeros where there is no head.  Their loads go out ahead of the tile's.
     const float qsc = a.scale * 1.4426950408889634f;
     auto put_q = [&](int head, int d4, float4 v) __attribute__((always_inline)) {
         const float x[4] = {v.x * qsc, v.y * qsc, v.z * qsc, v.w * qsc};
@@ -353,25 +358,32 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
     // rows no head fills
     for (int i = tid; i < QROWS * (HD / 4); i += 256) {
         const int row = i / (HD / 4), d4 = i % (HD / 4);
-        if (row == 16 || (row & 7) >= G) *(uint2*)(Qs + row * KS + 4 * d4) = make_uint2(0, 0);
+        if ((row & 7) >= G || (TWO ? row >= 16 && !two : row == 16)) *(uint2*)(Qs + row * KS + 4 * d4) = make_uint2(0, 0);
     }
-    float4 qv[(G * HD / 4 + 255) / 256];
+    constexpr int QV = (G * HD / 4 + 255) / 256;
+    constexpr int NQ = TWO ? 2 : 1;
+    float4 qv[NQ][QV];
     if (!PREP) {
 #pragma unroll
-        for (int j = 0; j < (G * HD / 4 + 255) / 256; j++) {
-            const int i = tid + j * 256;
-            qv[j] = i < G * HD / 4 ? ((const float4*)(a.q + ((int64_t)t * a.n_head + h0) * HD))[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
+        for (int z = 0; z < NQ; z++)
+#pragma unroll
+            for (int j = 0; j < QV; j++) {
+                const int i = tid + j * 256;
+                qv[z][j] = i < G * HD / 4 && (z == 0 || two) ? ((const float4*)(a.q + ((int64_t)(t + z) * a.n_head + h0) * HD))[i]
+                                                             : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
     }
     fetch_k(0);
     fetch_v(0);
     ATTN_STAMP(2);
     if (!PREP) {
 #pragma unroll
-        for (int j = 0; j < (G * HD / 4 + 255) / 256; j++) {
-            const int i = tid + j * 256;
-            if (i < G * HD / 4) put_q(i / (HD / 4), i % (HD / 4), qv[j]);
-        }
+        for (int z = 0; z < NQ; z++)
+#pragma unroll
+            for (int j = 0; j < QV; j++) {
+                const int i = tid + j * 256;
+                if (i < G * HD / 4 && (z == 0 || two)) put_q(16 * z + i / (HD / 4), i % (HD / 4), qv[z][j]);
+            }
     } else {
         constexpr int LPH = HD / 4, HPP = 64 / LPH;  // lanes per head, heads per wave pass
         const int li = lane % LPH;
@@ -393,7 +405,7 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
 #pragma unroll
         for (int i = 0; i < 16; i++) o[dw][i] = 0.0f;
     float m = -INFINITY, l = 0.0f;
-    const uint16_t* qcol = Qs + (c < 16 ? c : 16) * KS + 8 * g;  // this lane's column of Q^T
+    const uint16_t* qcol = Qs + (TWO || c < 16 ? c : 16) * KS + 8 * g;  // this lane's column of Q^T
 
     ATTN_STAMP(3);
     for (int kt = 0; kt < n_kt; kt++) {
@@ -434,7 +446,7 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
         }
         ATTN_STAMP(7);
         // high + low halves (columns c and c + 8 of the same row of 16 lanes), then the keys past the range
-        const int left = k1 - (k0 + kt * TILE);  // live keys of this tile
+        const int left = min(k1, my_pos) - (k0 + kt * TILE);  // live keys of this tile for this column
 #pragma unroll
         for (int kk = 0; kk < 2; kk++)
 #pragma unroll
@@ -450,15 +462,16 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
 #pragma unroll
             for (int i = 0; i < 16; i++) mt = fmaxf(mt, sc[kk][i]);
         mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-        const float m_new = fmaxf(m, mt);  // finite: the first key of a tile is live
-        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+        const float m_new = fmaxf(m, mt);
+        const float m_sub = m_new != -INFINITY ? m_new : 0.0f;   // (the earlier query of a pair may have no key in the range)
+        const float alpha = __builtin_amdgcn_exp2f(m - m_sub);
         float psum = 0.0f;
         h8 pf[4];
 #pragma unroll
         for (int kk = 0; kk < 2; kk++)
 #pragma unroll
             for (int i = 0; i < 16; i++) {
-                const float p = __builtin_amdgcn_exp2f(sc[kk][i] - m_new);
+                const float p = __builtin_amdgcn_exp2f(sc[kk][i] - m_sub);
                 psum += p;
                 pf[2 * kk + (i >> 3)][i & 7] = (_Float16)p;
             }
@@ -472,6 +485,7 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
         }
         ATTN_STAMP(8);
         // the values arrive while the scores are formed
+        if (TWO) __syncthreads();
         stash_v();
         if (fresh) {
             __syncthreads();  // the stale row of the tile is written before the new one
@@ -511,22 +525,24 @@ __global__ __launch_bounds__(256) void attend_decode_k(AttnArgs a, TilePrepP pr,
     }
 
     l += __shfl_xor(l, 32, 64);
-    if (c < G) {
-        float* p = my_part + c * part_head_stride;
+    if ((c & 15) < G && (c < 16 || two)) {
+        float* p = my_part + (c & 15) * part_head_stride + (c >> 4) * part_query_stride;
+        if (n_kt > 0) {
 #pragma unroll
-        for (int dw = 0; dw < NDW; dw++) {
-            const int dt = w + 4 * dw;
-            if (dt < ND) {
+            for (int dw = 0; dw < NDW; dw++) {
+                const int dt = w + 4 * dw;
+                if (dt < ND) {
 #pragma unroll
-                for (int i4 = 0; i4 < 4; i4++) {
-                    float* q = p + 32 * dt + 8 * i4 + 4 * g;  // 8-byte aligned: the partial stride is even
-                    *(float2*)q = make_float2(o[dw][4 * i4], o[dw][4 * i4 + 1]);
-                    *(float2*)(q + 2) = make_float2(o[dw][4 * i4 + 2], o[dw][4 * i4 + 3]);
+                    for (int i4 = 0; i4 < 4; i4++) {
+                        float* q = p + 32 * dt + 8 * i4 + 4 * g;  // 8-byte aligned: the partial stride is even
+                        *(float2*)q = make_float2(o[dw][4 * i4], o[dw][4 * i4 + 1]);
+                        *(float2*)(q + 2) = make_float2(o[dw][4 * i4 + 2], o[dw][4 * i4 + 3]);
+                    }
                 }
             }
         }
-        if (w == 0 && g == 0) {
-            p[HD] = m * 0.6931471805599453f;  // the maximum in the natural-log domain, as the merge expects
+        if (w == 0 && g == 0) {   // the maximum in the natural-log domain, as the merge expects
+            p[HD] = m * 0.6931471805599453f;
             p[HD + 1] = l;
         }
     }
@@ -686,23 +702,28 @@ static bool attend_split_impl(const AttnArgs& a, const TilePrepP* prep, int n_sp
                               const float* gate, int gate_stride, hipStream_t s) {
     if (a.n_q <= 0) return true;
     const int G = a.n_head / a.n_head_kv;
-    dim3 grid(a.n_q * a.n_head_kv, n_split), block(256);
     const bool tile = tile_path(a.n_q, a.head_dim, G);
+    const bool two = tile && a.n_q > 1;
+    dim3 grid((two ? (a.n_q + 1) / 2 : a.n_q) * a.n_head_kv, n_split), block(256);
     if (tile) {
-#define IT_TILE(HD, GG)                                                                                          \
+#define IT_TILE_LAUNCH(HD, K, PR, TWO)                                                                           \
     do {                                                                                                         \
-        constexpr size_t lds = ((size_t)(TILE + 17) * (HD + 8) + (size_t)HD * DVS) * sizeof(uint16_t); \
-        static bool sized[2] = {false, false};                                                                   \
-        if (!sized[prep ? 1 : 0]) {                                                                              \
-            const void* fn = prep ? (const void*)attend_decode_k<HD, GG, true> : (const void*)attend_decode_k<HD, GG, false>; \
-            if (lds > 64 * 1024 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
+        constexpr size_t lds = ((size_t)decode_q_at<HD, TWO>() + (size_t)decode_q_rows<TWO>() * (HD + 8)) * sizeof(uint16_t); \
+        static bool sized = false;                                                                               \
+        if (!sized) {                                                                                            \
+            if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)K, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) { \
                 (void)hipGetLastError();                                                                         \
                 return false;                                                                                    \
             }                                                                                                    \
-            sized[prep ? 1 : 0] = true;                                                                          \
+            sized = true;                                                                                        \
         }                                                                                                        \
-        if (prep) hipLaunchKernelGGL((attend_decode_k<HD, GG, true>), grid, block, lds, s, a, *prep, n_split, scratch); \
-        else hipLaunchKernelGGL((attend_decode_k<HD, GG, false>), grid, block, lds, s, a, TilePrepP{}, n_split, scratch); \
+        hipLaunchKernelGGL(K, grid, block, lds, s, a, PR, n_split, scratch);                                     \
+    } while (0)
+#define IT_TILE(HD, GG)                                                                                          \
+    do {                                                                                                         \
+        if (prep) IT_TILE_LAUNCH(HD, (attend_decode_k<HD, GG, true, false>), *prep, false);                      \
+        else if (two) IT_TILE_LAUNCH(HD, (attend_decode_k<HD, GG, false, true>), TilePrepP{}, true);             \
+        else IT_TILE_LAUNCH(HD, (attend_decode_k<HD, GG, false, false>), TilePrepP{}, false);                               \
     } while (0)
 #define IT_TILE_G(HD)                  \
     switch (G) {                       \
@@ -717,6 +738,7 @@ static bool attend_split_impl(const AttnArgs& a, const TilePrepP* prep, int n_sp
         else { IT_TILE_G(256) }
 #undef IT_TILE_G
 #undef IT_TILE
+#undef IT_TILE_LAUNCH
     } else {
         size_t lds = ((size_t)G * a.head_dim + (size_t)CHUNK * G) * sizeof(float);
         switch (G) {

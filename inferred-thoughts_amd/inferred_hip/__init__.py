@@ -9,6 +9,8 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -268,6 +270,9 @@ class HipError(RuntimeError):
 
 
 NOALLOC_SCRATCH_BYTES = 8 << 20
+_noalloc = threading.local()
+_ATTN_PACK = struct.Struct("@10Qf").pack_into   # the members of Attn
+_NOALLOC_OK = (0, "")
 
 
 def attend_noalloc(q_ptr: int, q_len: int, k_ptr: int, v_ptr: int, kv_len: int, kv_dim: int, n_pos: int,
@@ -275,10 +280,17 @@ def attend_noalloc(q_ptr: int, q_len: int, k_ptr: int, v_ptr: int, kv_len: int, 
                    stream: int = 0):
     """it_hip_attend_noalloc over DEVICE addresses (q, out: f32; k, v: f16 bits).  Returns (code, message):
     0 = enqueued on `stream`, 1 = bad argument, 2 = too large for the fixed scratch, 3 = device error."""
-    a = Attn(q_ptr, q_len, k_ptr, v_ptr, kv_len, kv_dim, n_pos, head_dim, n_head, n_head_kv, scale)
-    err = C.create_string_buffer(512)
-    rc = lib().it_hip_attend_noalloc(C.addressof(a), out_ptr, out_len, stream, err, 512)
-    return int(rc), err.value.decode()
+    # one packed argument block and message buffer per thread: building ctypes objects anew cost more than the launch
+    try:
+        args, at, err, fn = _noalloc.held
+    except AttributeError:
+        args, err = bytearray(C.sizeof(Attn)), C.create_string_buffer(512)
+        at = C.addressof(C.c_char.from_buffer(args))
+        fn = lib().it_hip_attend_noalloc
+        _noalloc.held = args, at, err, fn
+    _ATTN_PACK(args, 0, q_ptr, q_len, k_ptr, v_ptr, kv_len, kv_dim, n_pos, head_dim, n_head, n_head_kv, scale)
+    rc = fn(at, out_ptr, out_len, stream, err, 512)
+    return (rc, err.value.decode()) if rc else _NOALLOC_OK
 
 
 class Hip:
