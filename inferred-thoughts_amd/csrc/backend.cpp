@@ -1685,7 +1685,7 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
         it_hip::OpRec rec;
         rec.id = OP_ATTEND; rec.p[0] = dq; rec.p[1] = dk; rec.p[2] = dv; rec.p[3] = dyn; rec.p[4] = sc; rec.p[5] = dout;
         rec.i[0] = args.n_q; rec.i[1] = args.kv_dim; rec.i[2] = args.head_dim; rec.i[3] = args.n_head;
-        rec.i[4] = args.n_head_kv; rec.i[6] = 1; rec.i[8] = (int64_t)a->n_pos; rec.f[0] = args.scale;  // exact form: launched as is
+        rec.i[4] = args.n_head_kv; rec.i[6] = 1; rec.i[8] = (int64_t)a->n_pos; rec.i[9] = args.n_pos; rec.f[0] = args.scale;
         be->submit(it_hip::FAM_ATTEND, bytes,
                    sig_of(OP_ATTEND, 0, sg.q, sg.k, sg.v, sg.n_q, sg.kv_dim, dyn ? sg.n_pos : 0, sg.head_dim, sg.n_head,
                           sg.n_head_kv, sg.scale, dyn, sc, dout), rec,

@@ -39,7 +39,7 @@
 //   FINISH     p: out, rows, weights, shared, logit   i: at, n, n_tok, n_used, logit_at
 //   ROPE       p: x, table, dyn             i: half, n_tok, head_dim, n_rot, n_heads, pos
 //   KVWRITE    p: slab, dyn, src            i: mul, offset, n
-//   ATTEND     p: q, k, v, dyn, scratch, out   i: n_q, kv_dim, head_dim, n_head, n_head_kv, n_split, exact, n_pos  f: scale
+//   ATTEND     p: q, k, v, dyn, scratch, out   i: n_q, kv_dim, head_dim, n_head, n_head_kv, n_split, exact, n_pos (live: [8], exact form, sized for: [9])  f: scale
 enum OpId : int {
     OP_RMS = 1, OP_RMS_HEADS, OP_L2, OP_MATMUL, OP_ROPE, OP_SOFTMAX, OP_ATTEND, OP_EW, OP_SCALE, OP_CONV, OP_GATHER,
     OP_SCATTER, OP_DELTA, OP_ROUTE, OP_EXPERTS, OP_GLU, OP_FINISH, OP_ROWS, OP_SIGADD, OP_KVWRITE, OP_EMBED,

@@ -94,9 +94,9 @@ bool mm_reads(const Op& m, const void* x, const Op& q) {
 }
 
 // MATMUL `m` with unquantized weights (the router and ssm alpha / beta of real files are F32) reads the f32
-// activation `x` itself, one token.  Only the fast kernels take such a matrix into a fused launch.
-bool mm_reads_f32(const Op& m, const void* x, int64_t n_in, int exact) {
-    return !exact && m.id == OP_MATMUL && m.p[2] == x && m.i[3] == 1 && float_fmt(m.i[0]) && m.i[1] == n_in;
+// activation `x` itself, one token.
+bool mm_reads_f32(const Op& m, const void* x, int64_t n_in) {
+    return m.id == OP_MATMUL && m.p[2] == x && m.i[3] == 1 && float_fmt(m.i[0]) && m.i[1] == n_in;
 }
 
 FusedMat mat_of(const Op& m, int epi, float* out_override = nullptr) {
@@ -122,8 +122,8 @@ bool match_gdn(Plan& pl, size_t i, int exact) {
     const void* normed = rms.p[2];
     if (rms.i[0] != 1 || q1.p[0] != normed || q1.i[0] != rms.i[1]) return false;
     if (!mm_reads(mqkv, normed, q1) || !mm_reads(mz, normed, q1)) return false;
-    if (!mm_reads(ma, normed, q1) && !mm_reads_f32(ma, normed, rms.i[1], exact)) return false;
-    if (!mm_reads(mb, normed, q1) && !mm_reads_f32(mb, normed, rms.i[1], exact)) return false;
+    if (!mm_reads(ma, normed, q1) && !mm_reads_f32(ma, normed, rms.i[1])) return false;
+    if (!mm_reads(mb, normed, q1) && !mm_reads_f32(mb, normed, rms.i[1])) return false;
     int64_t dk = dl.i[1], dv = dl.i[2], nk = dl.i[3], nv = dl.i[4];
     int64_t kdim = nk * dk, vdim = nv * dv, cdim = 2 * kdim + vdim;
     if (dl.i[0] != 1 || dk != dv || (dk != 64 && dk != 128)) return false;
@@ -158,7 +158,7 @@ bool match_gdn(Plan& pl, size_t i, int exact) {
     a.m[3] = mat_of(mb, 0);
     a.conv_state = (float*)conv.p[0];
     a.conv_w = (const float*)conv.p[2];
-    if ((float_fmt(ma.i[0]) || float_fmt(mb.i[0])) && !fused_gemv_fast_takes(a)) return false;
+    if ((float_fmt(ma.i[0]) || float_fmt(mb.i[0])) && !(exact ? fused_gemv_exact_takes(a) : fused_gemv_fast_takes(a))) return false;
 
     GdnCoreP c{};
     c.conv = (const float*)cv;
@@ -415,11 +415,9 @@ bool match_attn(Plan& pl, size_t i, int exact) {
         });
     } else {
         pl.add(i, it_hip::FAM_ATTN_PREP, (uint64_t)(2 * hd * nh + 2 * kvd) * 4 + kvd * 4, [=](hipStream_t s) { attn_prep(pp, s); });
-        // the exact attention kernel and its gate stay as they are
-        auto run_attend = at.run, run_gate = sg.run, run_gather_gate = gg.run;
-        pl.add(i, it_hip::FAM_OTHER, 0, run_gather_gate);
-        pl.add(i, it_hip::FAM_ATTEND, kv_bytes, run_attend);
-        pl.add(i, it_hip::FAM_OTHER, 0, run_gate);
+        AttnArgs ax = aa;
+        ax.n_pos = (int)at.i[9];   // what the scratch rows are sized for
+        pl.add(i, it_hip::FAM_ATTEND, kv_bytes, [=](hipStream_t s) { attend_exact(ax, scratch, attn_out, s, gate, gate_stride); });
     }
     Plan::Launch& l_out = pl.add(i, it_hip::FAM_FUSED_GEMV, gemv_bytes(b), [=](hipStream_t s) { fused_gemv(b, s); });
     if (three) {   // the form whose in- and out-projection a layer chain may take over
@@ -446,7 +444,6 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
     if (!rms_p || !ga_p) return false;
     const Op* q1_p = take(OP_QUANT);
     const bool q_first = q1_p != nullptr;
-    if (!q_first && exact) return false;
     const Op *mr_p = take(OP_MATMUL), *ml_p = take(OP_MATMUL), *sm_p = take(OP_SOFTMAX), *rt_p = take(OP_ROUTE);
     if (!mr_p || !ml_p || !sm_p || !rt_p) return false;
     if (!q_first && !(q1_p = take(OP_QUANT))) return false;
@@ -488,8 +485,8 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
     if (ga.p[0] != rms.p[2] || ga.i[0] != nd || ga.i[2] != 0 || ga.i[3] != nd) return false;
     const void* x = ga.p[1];
     if (q1.p[0] != x || q1.i[0] != nd || ml.i[2] != 1) return false;
-    if (q_first ? !mm_reads(mr, x, q1) : !mm_reads_f32(mr, x, nd, exact)) return false;
-    if (!mm_reads(ml, x, q1) && !mm_reads_f32(ml, x, nd, exact)) return false;
+    if (q_first ? !mm_reads(mr, x, q1) : !mm_reads_f32(mr, x, nd)) return false;
+    if (!mm_reads(ml, x, q1) && !mm_reads_f32(ml, x, nd)) return false;
     int64_t ne = mr.i[2];
     const void* router = mr.p[5];
     if (sm.p[0] != router || sm.i[0] != 1 || sm.i[1] != ne) return false;
@@ -533,7 +530,7 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
     a.n_used = (int)nu;
     a.route_ids = (int32_t*)rt.p[1];
     a.route_w = (float*)rt.p[2];
-    if ((float_fmt(mr.i[0]) || float_fmt(ml.i[0])) && !fused_gemv_fast_takes(a)) return false;
+    if ((float_fmt(mr.i[0]) || float_fmt(ml.i[0])) && !(exact ? fused_gemv_exact_takes(a) : fused_gemv_fast_takes(a))) return false;
 
     MoeGluP g{};
     g.x = (const float*)x;

@@ -4,34 +4,39 @@
 
 namespace itk {
 
-// ------------------------------------------------------------------ sum of squares
-// Serial f64 accumulation of f32 squares (naive.rs:633-640) by one lane, or a tree.
-// `buf` holds the row in LDS.  Returns the sum to every thread of the block.
+// ------------------------------------------------------------------ mean of squares
+// (float)(sum / div), the sum being the f64 sum of f32 squares over `buf` (LDS): all that the norms use of it.
+//
+// The CPU path adds the squares one by one (naive.rs:633-640).  Any other order of n such additions of non-negative terms
+// differs from that sum by less than n * 2^-52 of it, and division and rounding to f32 are monotonic: where both ends of
+// that interval give the same f32, so does the serial sum, and only where they do not (n = 2,048: one row in 10^5) is it
+// formed, by one lane (2,048 dependent f64 additions: 20 us, the tree 1).  Exact mode therefore has the CPU's bits.
+IT_DEV bool mean_is_certain(double sum, int n, double div, float* mean) {
+    const double off = sum * ((double)(n + 16) * 0x1p-52);
+    *mean = (float)((sum - off) / div);
+    return *mean == (float)((sum + off) / div);
+}
 template <int THREADS>
-__device__ double block_sumsq(const float* buf, int n, int exact, double* red) {
-    if (exact) {
-        if (threadIdx.x == 0) {
-            double sum = 0.0;
-            for (int i = 0; i < n; i++) sum += (double)(buf[i] * buf[i]);
-            red[0] = sum;
-        }
-        __syncthreads();
-        return red[0];
-    }
+__device__ float block_meansq(const float* buf, int n, double div, int exact, double* red) {
     double part = 0.0;
     for (int i = threadIdx.x; i < n; i += THREADS) part += (double)(buf[i] * buf[i]);
     for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
     __syncthreads();
+    double sum = 0.0;
+    for (int w = 0; w < THREADS / 64; w++) sum += red[w];
+    if (!exact) return (float)(sum / div);
+    float mean;
+    if (mean_is_certain(sum, n, div, &mean)) return mean;   // (the same answer in every thread)
+    __syncthreads();
     if (threadIdx.x == 0) {
-        double sum = 0.0;
-        for (int w = 0; w < THREADS / 64; w++) sum += red[w];
+        sum = 0.0;
+        for (int i = 0; i < n; i++) sum += (double)(buf[i] * buf[i]);
         red[0] = sum;
     }
     __syncthreads();
-    return red[0];
+    return (float)(red[0] / div);
 }
-
 
 // ------------------------------------------------------------------ lane exchanges without LDS
 // DPP moves reach the lanes of a row of 16: neighbour (quad_perm 1,0,3,2), pair (quad_perm

@@ -34,66 +34,116 @@ __device__ int it_attn_stamp_split;
 namespace itk {
 
 // ------------------------------------------------------------------ exact
-__global__ __launch_bounds__(256) void attend_exact_k(AttnArgs a, float* __restrict__ scratch,
-                                                      float* __restrict__ out) {
-    extern __shared__ float qs[];  // head_dim
+// One block per (query, head).  Scores and weights sit in LDS up to EXACT_LDS positions (beyond, in `scratch`).  What has an
+// order is a chain: a position's dot in its thread, the weights' sum in one lane, a dim's weighted sum in its thread, each
+// with its loads several steps ahead.  333 positions, 16 heads of 256: TIMES
+constexpr int EXACT_LDS = 4096;
+__global__ __launch_bounds__(256) void attend_exact_k(AttnArgs a, float* __restrict__ scratch, float* __restrict__ out,
+                                                      const float* __restrict__ gate, int gate_stride, int lds_pos) {
+    extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each)
     __shared__ float red[8];
-    const int hd = a.head_dim;
+    const int hd = a.head_dim, tid = threadIdx.x;
     const int n_pos_last = a.n_pos_dyn ? *a.n_pos_dyn : a.n_pos;
     const int t = blockIdx.x / a.n_head, h = blockIdx.x % a.n_head;
     const int group = a.n_head / a.n_head_kv;
     const int h_kv = h / group;
-    const int n_pos = n_pos_last - a.n_q + 1 + t;
+    const int n_pos = n_pos_last - a.n_q + 1 + t, n_lds = min(n_pos, lds_pos);
     const int off = h_kv * hd;
     const float* q = a.q + ((int64_t)t * a.n_head + h) * hd;
-    float* sc = scratch + (int64_t)blockIdx.x * n_pos_last;
-    for (int i = threadIdx.x; i < hd; i += 256) qs[i] = q[i];
+    float* near = qs + ((hd + 3) & ~3);
+    float* far = scratch + (int64_t)blockIdx.x * n_pos_last;
+    auto score = [&](int s) -> float& { return s < lds_pos ? near[s] : far[s]; };
+    for (int i = tid; i < hd; i += 256) qs[i] = q[i];
     __syncthreads();
     float m = -INFINITY;
-    for (int s = threadIdx.x; s < n_pos; s += 256) {
+    for (int s = tid; s < n_pos; s += 256) {
         const uint16_t* key = a.k + (int64_t)s * a.kv_dim + off;
         float dot = 0.0f;
-        for (int i = 0; i < hd; i += 8) {
-            uint4 kk = *(const uint4*)(key + i);
-            uint32_t w[4] = {kk.x, kk.y, kk.z, kk.w};
+        auto add8 = [&](int i, uint4 kk) {
+            const uint32_t w[4] = {kk.x, kk.y, kk.z, kk.w};
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 dot += qs[i + 2 * c] * it_f16_to_f32((uint16_t)(w[c] & 0xffff));
                 dot += qs[i + 2 * c + 1] * it_f16_to_f32((uint16_t)(w[c] >> 16));
             }
+        };
+        int i = 0;
+        if (hd >= 64) {   // 64 dims at a time, the next 64 on their way
+            uint4 nx[8];
+#pragma unroll
+            for (int p = 0; p < 8; p++) nx[p] = *(const uint4*)(key + 8 * p);
+            for (; i + 64 <= hd; i += 64) {
+                uint4 cur[8];
+#pragma unroll
+                for (int p = 0; p < 8; p++) cur[p] = nx[p];
+                const int n = i + 128 <= hd ? i + 64 : i;
+#pragma unroll
+                for (int p = 0; p < 8; p++) nx[p] = *(const uint4*)(key + n + 8 * p);
+#pragma unroll
+                for (int p = 0; p < 8; p++) add8(i + 8 * p, cur[p]);
+            }
         }
-        float v = dot * a.scale;
-        sc[s] = v;
+        for (; i < hd; i += 8) add8(i, *(const uint4*)(key + i));
+        const float v = dot * a.scale;
+        score(s) = v;
         m = fmaxf(m, v);
     }
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_down(m, o, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    if ((tid & 63) == 0) red[tid >> 6] = m;
     __syncthreads();
     m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    for (int s = threadIdx.x; s < n_pos; s += 256) sc[s] = it_expf(sc[s] - m);
+    for (int s = tid; s < n_pos; s += 256) score(s) = it_expf(score(s) - m);
     __threadfence_block();
     __syncthreads();
-    if (threadIdx.x == 0) {
+    if (tid == 0) {
         float sum = 0.0f;
-        for (int s = 0; s < n_pos; s++) sum += sc[s];
+        int s = 0;
+        for (; s + 16 <= n_lds; s += 16) {
+            float4 v[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = *(const float4*)(near + s + 4 * c);
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                sum += v[c].x;
+                sum += v[c].y;
+                sum += v[c].z;
+                sum += v[c].w;
+            }
+        }
+        for (; s < n_lds; s++) sum += near[s];
+#pragma unroll 16
+        for (s = lds_pos; s < n_pos; s++) sum += far[s];
         red[4] = sum;
     }
     __syncthreads();
-    float sum = red[4];
-    for (int i = threadIdx.x; i < hd; i += 256) {
+    const float sum = red[4];
+    for (int s = tid; s < n_pos; s += 256) score(s) = score(s) / sum;
+    __threadfence_block();
+    __syncthreads();
+    for (int i = tid; i < hd; i += 256) {
+        const uint16_t* v = a.v + off + i;
         float acc = 0.0f;
-        for (int s = 0; s < n_pos; s++) {
-            float w = sc[s] / sum;
-            acc += w * it_f16_to_f32(a.v[(int64_t)s * a.kv_dim + off + i]);
+        int s = 0;
+        for (; s + 16 <= n_lds; s += 16) {
+            uint16_t x[16];
+#pragma unroll
+            for (int c = 0; c < 16; c++) x[c] = v[(int64_t)(s + c) * a.kv_dim];
+#pragma unroll
+            for (int c = 0; c < 16; c++) acc += near[s + c] * it_f16_to_f32(x[c]);
         }
+        for (; s < n_lds; s++) acc += near[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
+#pragma unroll 8
+        for (s = lds_pos; s < n_pos; s++) acc += far[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
+        if (gate) acc *= it_sigmoid(gate[(int64_t)h * gate_stride + i]);   // (n_q == 1: sigmoid_mul of the gated block)
         out[((int64_t)t * a.n_head + h) * hd + i] = acc;
     }
 }
 
-void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s) {
+void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate, int gate_stride) {
     if (a.n_q <= 0) return;
-    hipLaunchKernelGGL(attend_exact_k, dim3(a.n_q * a.n_head), dim3(256), a.head_dim * sizeof(float), s, a,
-                       scratch, out);
+    const int lds_pos = std::min((a.n_pos + 3) & ~3, EXACT_LDS);
+    hipLaunchKernelGGL(attend_exact_k, dim3(a.n_q * a.n_head), dim3(256), ((size_t)((a.head_dim + 3) & ~3) + lds_pos) * sizeof(float), s, a,
+                       scratch, out, gate, gate_stride, lds_pos);
 }
 
 // ------------------------------------------------------------------ split-K

@@ -13,6 +13,7 @@
 //   moe_down_fused  quantize + expert down + shared down + moe_finish + add_assign
 //   attn_prep       gather q/gate + rms_norm_heads(q,k) + rope(q,k) + kv_write(k,v)
 //   attn_merge_gate split-K merge + sigmoid_mul
+#include <algorithm>
 #include "it_device.h"
 #include "it_dot.h"
 #include "it_reduce.h"
@@ -203,7 +204,7 @@ __device__ void wave_route(float* probs, int n_expert, int n_used, int exact, in
     wave_lds_sync();
 }
 
-constexpr int FG_THREADS = 512;
+constexpr int FG_THREADS = 512, FG_LDS_MAX = 128 * 1024;
 
 IT_DEV int mat_index(const FusedGemvP& p, int g) {
     int mi = 0;
@@ -213,6 +214,11 @@ IT_DEV int mat_index(const FusedGemvP& p, int g) {
     return mi;
 }
 
+// A router's logits are read by another block of the same launch: they go past the caches that the XCDs do not share.
+IT_DEV void put_out(const FusedGemvP& p, const FusedMat& m, int j, float v) {
+    if (p.route_counter) __hip_atomic_store(m.out + j, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else m.out[j] = v;
+}
 // fold each row's terms in order and apply the matrix's epilogue
 IT_DEV void finish_rows(const FusedGemvP& p, const FusedMat& m, int row0, int nrows, const float* terms, int tstride,
                         int nb, int lane) {
@@ -221,7 +227,7 @@ IT_DEV void finish_rows(const FusedGemvP& p, const FusedMat& m, int row0, int nr
     float acc = fold_terms(terms + lane * tstride, T);
     const int j = row0 + lane;
     if (m.epi == 0) {
-        m.out[j] = acc;
+        put_out(p, m, j, acc);
     } else if (m.epi == 2) {
         m.out[j] += acc;
     } else if (m.epi == 3) {
@@ -258,7 +264,7 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
     constexpr int W = FG_THREADS / 64;
     const int R = p.rows_per_wave;
     const int tstride = nb * 2 + 4;
-    float* terms = terms_all + (size_t)wave * R * tstride;
+    float* terms = terms_all + (size_t)wave * p.terms_stride;
     const int g0 = blockIdx.x * W + wave;
     const bool has0 = g0 < p.total_groups;
     const FusedMat& m0 = p.m[has0 ? mat_index(p, g0) : 0];
@@ -273,30 +279,34 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
     for (int i = tid; i < n_in; i += FG_THREADS) xf[i] = p.x[i];
     __syncthreads();
     if (p.mode == 1) {
-        double sum = block_sumsq<FG_THREADS>(xf, n_in, p.exact, red);
-        float mean = (float)(sum / (double)n_in);
+        float mean = block_meansq<FG_THREADS>(xf, n_in, (double)n_in, p.exact, red);
         float scale = 1.0f / sqrtf(mean + p.eps);
         for (int i = tid; i < n_in; i += FG_THREADS) xf[i] = xf[i] * scale * p.norm_w[i];
         __syncthreads();
     } else if (p.mode == 2 || p.mode == 3) {
         const int hd = p.head_dim, nh = n_in / hd;  // nh <= 64 (checked on the host)
-        if (p.exact) {
-            if (tid < nh) {
-                double sum = 0.0;
-                const float* h = xf + tid * hd;
-                for (int i = 0; i < hd; i++) sum += (double)(h[i] * h[i]);
-                hscale[tid] = 1.0f / sqrtf((float)(sum / (double)hd) + p.eps);
-            }
-        } else {
-            // 4 lanes per head
-            for (int h0 = 0; h0 < nh; h0 += FG_THREADS / 4) {
-                int h = h0 + (tid >> 2), sub = tid & 3;
-                double part = 0.0;
-                if (h < nh)
-                    for (int i = sub; i < hd; i += 4) part += (double)(xf[h * hd + i] * xf[h * hd + i]);
-                part += __shfl_xor(part, 1, 64);
-                part += __shfl_xor(part, 2, 64);
-                if (h < nh && sub == 0) hscale[h] = 1.0f / sqrtf((float)(part / (double)hd) + p.eps);
+        // 8 lanes per head; a head's walk starts at its own place, so that the heads of a wave read different banks
+        for (int h0 = 0; h0 < nh; h0 += FG_THREADS / 8) {
+            const int h = h0 + (tid >> 3), sub = tid & 7, steps = hd / 8;
+            double part = 0.0;
+            if (h < nh)
+                for (int k = 0; k < steps; k++) {
+                    const float v = xf[h * hd + sub + 8 * ((k + h) % steps)];
+                    part += (double)(v * v);
+                }
+            part += dpp_f64(part, 0);
+            part += dpp_f64(part, 1);
+            part += dpp_f64(part, 2);
+            if (h < nh && sub == 0) {
+                float mean;
+                if (!p.exact) {
+                    mean = (float)(part / (double)hd);
+                } else if (!mean_is_certain(part, hd, (double)hd, &mean)) {
+                    part = 0.0;
+                    for (int i = 0; i < hd; i++) part += (double)(xf[h * hd + i] * xf[h * hd + i]);
+                    mean = (float)(part / (double)hd);
+                }
+                hscale[h] = 1.0f / sqrtf(mean + p.eps);
             }
         }
         __syncthreads();
@@ -312,8 +322,10 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         if (p.x_copy2)
             for (int i = tid; i < n_in; i += FG_THREADS) p.x_copy2[i] = xf[i];
     }
-    lds_quantize_q8_0(xf, n_in, xs, xq);
-    __syncthreads();
+    if (p.n_mats) {
+        lds_quantize_q8_0(xf, n_in, xs, xq);
+        __syncthreads();
+    }
 
     if (has0) {
         if (m0.fmt == W_NVFP4) compute_items<W_NVFP4, 8>(rr, n_in, nrows0, xq, xs, terms, tstride, lane);
@@ -332,22 +344,37 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         finish_rows(p, m, row0, nrows, terms, tstride, nb, lane);
         wave_lds_sync();
     }
+    // Unquantized rows: the wave forms a row's products, one lane folds them in order (naive.rs:843-861).  Dealt out over
+    // the blocks first: the fold is a chain of n_in additions.
+    for (int fr = wave * gridDim.x + blockIdx.x; fr < p.total_frows; fr += W * gridDim.x) {
+        int k = p.n_mats, j = fr;
+        while (j >= p.m[k].n_out) j -= p.m[k++].n_out;
+        const FusedMat& m = p.m[k];
+        const float* row = (const float*)m.q + (int64_t)j * n_in;
+#pragma unroll 8
+        for (int i = lane * 4; i < n_in; i += 256) {
+            const float4 w = *(const float4*)(row + i), x = *(const float4*)(xf + i);
+            *(float4*)(terms + i) = make_float4(w.x * x.x, w.y * x.y, w.z * x.z, w.w * x.w);
+        }
+        wave_lds_sync();
+        if (lane == 0) put_out(p, m, j, fold_terms(terms, n_in));
+        wave_lds_sync();
+    }
     if (p.route_counter) {
         // The block that finishes last turns the router logits (matrix 0's output) into the
         // token's expert choice, so the next kernel starts with the ids in hand.
         __shared__ int is_last;
-        __threadfence();
+        __builtin_amdgcn_s_waitcnt(0);   // the logits went past the caches (put_out): they are there, no fence needed
         __syncthreads();
         if (tid == 0) {
-            unsigned prev = atomicAdd(p.route_counter, 1u);
+            unsigned prev = __hip_atomic_fetch_add(p.route_counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             is_last = prev == gridDim.x - 1;
         }
         __syncthreads();
         if (is_last) {
-            __threadfence();
             float* probs = xf;  // n_expert <= n_in (checked on the host)
             for (int i = tid; i < p.n_expert; i += FG_THREADS)
-                probs[i] = __hip_atomic_load(p.m[0].out + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                probs[i] = __hip_atomic_load(p.route_logits + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __syncthreads();
             if (wave == 0) {
                 __shared__ int rids[64];
@@ -366,8 +393,22 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
 void fused_gemv(FusedGemvP p, hipStream_t s) {
     if (fused_gemv_fast(p, s)) return;
     constexpr int W = FG_THREADS / 64;
-    int total_rows = 0;
-    for (int i = 0; i < p.n_mats; i++) total_rows += p.m[i].n_out;
+    // unquantized matrices behind the quantized ones
+    p.route_logits = p.m[0].out;
+    FusedMat all[4];
+    int nq = 0, nf = 0, total_rows = 0;
+    for (int i = 0; i < p.n_mats; i++)
+        if (p.m[i].fmt != W_F32) all[nq++] = p.m[i];
+    for (int i = 0; i < p.n_mats; i++)
+        if (p.m[i].fmt == W_F32) all[nq + nf++] = p.m[i];
+    p.total_frows = 0;
+    for (int i = 0; i < nq + nf; i++) {
+        p.m[i] = all[i];
+        if (i < nq) total_rows += all[i].n_out;
+        else p.total_frows += all[i].n_out;
+    }
+    p.n_mats = nq;
+    p.n_fmats = nf;
     const int nb = p.n_in / 32;
     // enough waves to cover HBM latency: aim for ~4096 row groups, at most 512 items per wave pass
     // fewest passes per wave over 256 blocks of W waves, then the fewest rows per pass
@@ -382,22 +423,45 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
             }
         }
     }
+    // a router whose rows one block can take in one pass: nothing has to be handed from block to block
+    if (p.route_counter && !nf)
+        for (int r = 1; r <= 16 && r * nb <= 512; r *= 2)
+            if ((total_rows + r - 1) / r <= W) {
+                R = r;
+                break;
+            }
+    auto stride_for = [&](int r) { return std::max(r * (nb * 2 + 4), nf ? p.n_in : 0); };
     auto lds_for = [&](int r) {
-        return (size_t)p.n_in * 4 + (size_t)((nb + 3) & ~3) * 4 + p.n_in + (size_t)W * r * (nb * 2 + 4) * 4;
+        return (size_t)p.n_in * 4 + (size_t)((nb + 3) & ~3) * 4 + p.n_in + (size_t)W * stride_for(r) * 4;
     };
     while (R > 1 && lds_for(R) > 60 * 1024) R /= 2;
     p.rows_per_wave = R;
+    p.terms_stride = stride_for(R);
     int g = 0;
-    for (int i = 0; i < p.n_mats; i++) {
+    for (int i = 0; i < nq; i++) {
         p.m[i].group0 = g;
         g += (p.m[i].n_out + R - 1) / R;
     }
     p.total_groups = g;
-    int blocks = (g + W - 1) / W;
+    int blocks = std::max((g + W - 1) / W, p.total_frows);
     // one block per CU: every block pays the activation prologue, so more blocks than CUs
     // only repeats it (measured: 256 blocks 12 us, 772 blocks 22 us for norm + 12k rows of 2048)
     if (blocks > 256) blocks = 256;
-    hipLaunchKernelGGL(fused_gemv_k, dim3(blocks), dim3(FG_THREADS), lds_for(R), s, p);
+    const size_t lds = lds_for(R);
+    if (lds > 64 * 1024) {
+        static const bool sized = hipFuncSetAttribute((const void*)fused_gemv_k, hipFuncAttributeMaxDynamicSharedMemorySize, FG_LDS_MAX) == hipSuccess;
+        if (!sized) (void)hipGetLastError();
+    }
+    hipLaunchKernelGGL(fused_gemv_k, dim3(blocks), dim3(FG_THREADS), lds, s, p);
+}
+// F32 rows beside (or in place of) quantized ones, in the kernel that keeps the CPU path's order
+bool fused_gemv_exact_takes(const FusedGemvP& p) {
+    for (int i = 0; i < p.n_mats; i++) {
+        if (p.m[i].fmt == W_Q8_0 || p.m[i].fmt == W_NVFP4) continue;
+        if (p.m[i].fmt != W_F32 || p.m[i].epi != 0 || (reinterpret_cast<uintptr_t>(p.m[i].q) & 15)) return false;
+    }
+    const int nb = p.n_in / 32;
+    return p.n_in % 256 == 0 && (size_t)p.n_in * 5 + (size_t)((nb + 3) & ~3) * 4 + (size_t)(FG_THREADS / 64) * std::max(p.n_in, 2 * nb + 4) * 4 <= FG_LDS_MAX;
 }
 
 // ------------------------------------------------------------------ gdn rows
@@ -413,8 +477,8 @@ __device__ void load_kq_l2(const float* conv, int key_dim, int kh, float eps, in
     __syncthreads();
     for (int which = 0; which < 2; which++) {
         float* dst = kq + which * DK;
-        double sum = block_sumsq<THREADS>(dst, DK, exact, red);
-        float scale = 1.0f / fmaxf(sqrtf((float)sum), eps);
+        float sum = block_meansq<THREADS>(dst, DK, 1.0, exact, red);
+        float scale = 1.0f / fmaxf(sqrtf(sum), eps);
         __syncthreads();
         for (int i = tid; i < DK; i += THREADS) dst[i] = dst[i] * scale;
         __syncthreads();
@@ -809,8 +873,7 @@ __global__ __launch_bounds__(64) void attn_prep_k(AttnPrepP p) {
     const float* w = is_q ? p.q_norm : p.k_norm;
     for (int i = tid; i < hd; i += 64) hbuf[i] = src[i];
     __syncthreads();
-    double sum = block_sumsq<64>(hbuf, hd, p.exact, red);
-    float scale = 1.0f / sqrtf((float)(sum / (double)hd) + p.eps);
+    float scale = 1.0f / sqrtf(block_meansq<64>(hbuf, hd, (double)hd, p.exact, red) + p.eps);
     __syncthreads();
     for (int i = tid; i < hd; i += 64) hbuf[i] = hbuf[i] * scale * w[i];
     __syncthreads();

@@ -4,106 +4,134 @@
 // batch; head grouping is modulo (src/ops/mod.rs:404-413).  State is
 // [value head][value row][key] f32, key contiguous.
 //
-// One lane owns one value row: the row's dk floats stay in registers for the
-// whole batch, so the three sweeps (decay+predict, correct, read out) run in the
-// reference's order with no cross-lane reduction and the result is bit-identical
-// to the CPU path.  The 64-row tile moves between HBM and registers through a
-// padded LDS tile so both the load and the store are fully coalesced.
+// Exact mode: four lanes own one value row, a quarter of its dk floats each, in registers for the whole batch.  Decay,
+// correction and products are the lane's own; a sum over the row runs through the four in turn, each adding its quarter to
+// what the one before it hands over, so that every addition is the reference's, in its order.
 #include "it_device.h"
 #include "it_reduce.h"
 #include "kernels.h"
 
 namespace itk {
 
+// A block is one wave: 16 rows of one head (256 blocks for 32 heads of 128).  Tokens go in chunks of 16: a chunk's k, q
+// (scaled), v and gates are staged in LDS, the next chunk's loads in flight meanwhile.  Bound by the two chains of dk dependent
+// additions a token (128: TIMES a token; one lane per row, with every token's loads waited for, took 4.1 us).
+constexpr int DX_TCH = 16, DX_ROWS = 16;
+IT_DEV float quad_lane(float v, int which) {   // lane `which` of each aligned group of four, to all of it
+    const int u = __builtin_bit_cast(int, v);
+    const int r = which == 0   ? __builtin_amdgcn_update_dpp(0, u, 0x00, 0xf, 0xf, true)
+                  : which == 1 ? __builtin_amdgcn_update_dpp(0, u, 0x55, 0xf, 0xf, true)
+                  : which == 2 ? __builtin_amdgcn_update_dpp(0, u, 0xAA, 0xf, 0xf, true)
+                               : __builtin_amdgcn_update_dpp(0, u, 0xFF, 0xf, 0xf, true);
+    return __builtin_bit_cast(float, r);
+}
+template <int SEG>
+IT_DEV float quad_chain(const float (&p)[SEG]) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        float a = acc;
+#pragma unroll
+        for (int e = 0; e < SEG; e++) a += p[e];
+        acc = quad_lane(a, s);
+    }
+    return acc;
+}
 template <int DK>
-__global__ __launch_bounds__(64) void delta_rule_k(DeltaArgs d, float* __restrict__ state,
-                                                   float* __restrict__ out, float q_scale) {
-    __shared__ float tile[64 * (DK + 1)];
-    __shared__ __align__(16) float kq[2 * DK];
-    const int lane = threadIdx.x;
+__global__ __launch_bounds__(64) void delta_rule_k(DeltaArgs d, float* __restrict__ state, float* __restrict__ out, float q_scale) {
+    constexpr int SEG = DK / 4, SS = SEG + 4;             // + 4: the four quarters' 16-byte reads fall on different banks
+    constexpr int L4 = DX_TCH * DK / 4 / 64;              // float4 of k (and of q) per lane and chunk
+    __shared__ __align__(16) float kb[2][DX_TCH][4 * SS], qb[2][DX_TCH][4 * SS];
+    __shared__ float vb[2][DX_TCH][DX_ROWS], gb[2][DX_TCH][2];
+    const int lane = threadIdx.x, r = lane >> 2, seg = lane & 3;
     const int dv = d.head_v_dim;
-    const int blocks_per_head = (dv + 63) / 64;
-    const int h = blockIdx.x / blocks_per_head, jb = blockIdx.x % blocks_per_head;
+    const int bph = (dv + DX_ROWS - 1) / DX_ROWS;
+    const int h = blockIdx.x / bph, jb = blockIdx.x % bph;
     const int kh = h % d.n_k_heads;
-    const int j = jb * 64 + lane;
-    const bool live = j < dv;
-    const int rows_here = min(64, dv - jb * 64);
-    float* S = state + ((int64_t)h * dv + (int64_t)jb * 64) * DK;
+    const int j = jb * DX_ROWS + r, jc = min(j, dv - 1);   // rows past the head repeat its last one and are not stored
+    float* S = state + ((int64_t)h * dv + jc) * DK + seg * SEG;
+    const int kper = d.n_k_heads * DK, vper = d.n_v_heads * dv, n = d.n_tokens;
 
-    // 64 rows x DK floats = 16*DK float4; every load is issued before the first LDS write
-    {
-        constexpr int V = DK / 4;  // float4 per row
-        const float4* S4 = (const float4*)S;
-        float4 stage[V];
+    float row[SEG];
 #pragma unroll
-        for (int it = 0; it < V; it++) {
-            int idx4 = it * 64 + lane;
-            stage[it] = (idx4 < rows_here * V) ? S4[idx4] : make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < SEG / 4; i++) {
+        const float4 t = ((const float4*)S)[i];
+        row[4 * i] = t.x; row[4 * i + 1] = t.y; row[4 * i + 2] = t.z; row[4 * i + 3] = t.w;
+    }
+    float4 rk[L4], rq[L4];
+    float rv[DX_TCH * DX_ROWS / 64], ra = 0.0f, rb = 0.0f;
+    auto load = [&](int t0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < L4; p++) {
+            const int idx = p * 64 + lane, t = min(t0 + idx / (DK / 4), n - 1), c = idx % (DK / 4);
+            rk[p] = ((const float4*)(d.k + (int64_t)t * kper + kh * DK))[c];
+            rq[p] = ((const float4*)(d.q + (int64_t)t * kper + kh * DK))[c];
         }
 #pragma unroll
-        for (int it = 0; it < V; it++) {
-            int idx4 = it * 64 + lane;
-            int r = idx4 / V, c = (idx4 - r * V) * 4;
-            float* t = tile + r * (DK + 1) + c;
-            t[0] = stage[it].x; t[1] = stage[it].y; t[2] = stage[it].z; t[3] = stage[it].w;
+        for (int p = 0; p < DX_TCH * DX_ROWS / 64; p++) {
+            const int idx = p * 64 + lane, t = min(t0 + idx / DX_ROWS, n - 1);
+            rv[p] = d.v[(int64_t)t * vper + h * dv + min(jb * DX_ROWS + idx % DX_ROWS, dv - 1)];
+        }
+        const int t = min(t0 + (lane & (DX_TCH - 1)), n - 1);
+        ra = d.alpha[(int64_t)t * d.n_v_heads + h] + d.dt_bias[h];
+        rb = d.beta[(int64_t)t * d.n_v_heads + h];
+    };
+    auto stash = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < L4; p++) {
+            const int idx = p * 64 + lane, t = idx / (DK / 4), i = 4 * (idx % (DK / 4));
+            const int at = i / SEG * SS + i % SEG;
+            *(float4*)&kb[b][t][at] = rk[p];
+            *(float4*)&qb[b][t][at] = make_float4(rq[p].x * q_scale, rq[p].y * q_scale, rq[p].z * q_scale, rq[p].w * q_scale);
+        }
+#pragma unroll
+        for (int p = 0; p < DX_TCH * DX_ROWS / 64; p++) vb[b][(p * 64 + lane) / DX_ROWS][(p * 64 + lane) % DX_ROWS] = rv[p];
+        const float softplus = ra > 20.0f ? ra : it_logf(1.0f + it_expf(ra));
+        const float g = it_expf(softplus * d.ssm_a[h]), beta = 1.0f / (1.0f + it_expf(-rb));
+        if (lane < DX_TCH) {
+            gb[b][lane][0] = g;
+            gb[b][lane][1] = beta;
+        }
+    };
+    load(0);
+    for (int t0 = 0, b = 0; t0 < n; t0 += DX_TCH, b ^= 1) {
+        stash(b);
+        __syncthreads();   // (one wave: an LDS wait)
+        if (t0 + DX_TCH < n) load(t0 + DX_TCH);
+        const int live = min(DX_TCH, n - t0);
+        for (int t = 0; t < live; t++) {
+            const float g = gb[b][t][0], beta = gb[b][t][1], v = vb[b][t][r];
+            const float4* k4 = (const float4*)&kb[b][t][seg * SS];
+            const float4* q4 = (const float4*)&qb[b][t][seg * SS];
+            float kk[SEG], p[SEG];
+#pragma unroll
+            for (int i = 0; i < SEG / 4; i++) {
+                const float4 x = k4[i];
+                kk[4 * i] = x.x; kk[4 * i + 1] = x.y; kk[4 * i + 2] = x.z; kk[4 * i + 3] = x.w;
+            }
+#pragma unroll
+            for (int i = 0; i < SEG; i++) {
+                row[i] *= g;
+                p[i] = row[i] * kk[i];
+            }
+            const float delta = beta * (v - quad_chain<SEG>(p));
+#pragma unroll
+            for (int i = 0; i < SEG / 4; i++) {
+                const float4 x = q4[i];
+                const float qq[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    row[4 * i + e] += kk[4 * i + e] * delta;
+                    p[4 * i + e] = row[4 * i + e] * qq[e];
+                }
+            }
+            const float o = quad_chain<SEG>(p);
+            if (seg == 0 && j < dv) out[(int64_t)(t0 + t) * vper + h * dv + j] = o;
         }
     }
-    __syncthreads();
-    float row[DK];
+    if (j < dv) {
 #pragma unroll
-    for (int i = 0; i < DK; i++) row[i] = live ? tile[lane * (DK + 1) + i] : 0.0f;
-
-    const int kper = d.n_k_heads * DK, vper = d.n_v_heads * dv;
-    for (int t = 0; t < d.n_tokens; t++) {
-        __syncthreads();
-        for (int i = lane; i < DK; i += 64) {
-            kq[i] = d.k[(int64_t)t * kper + kh * DK + i];
-            kq[DK + i] = d.q[(int64_t)t * kper + kh * DK + i];
-        }
-        __syncthreads();
-        float a = d.alpha[(int64_t)t * d.n_v_heads + h] + d.dt_bias[h];
-        float softplus = a > 20.0f ? a : it_logf(1.0f + it_expf(a));
-        float g = it_expf(softplus * d.ssm_a[h]);
-        float beta = 1.0f / (1.0f + it_expf(-d.beta[(int64_t)t * d.n_v_heads + h]));
-        float v = live ? d.v[(int64_t)t * vper + h * dv + j] : 0.0f;
-        float pred = 0.0f;
-        const float4* k4 = (const float4*)kq;
-        const float4* q4 = (const float4*)(kq + DK);
-#pragma unroll
-        for (int i = 0; i < DK; i += 4) {
-            float4 kk = k4[i / 4];
-            row[i] *= g;     pred += row[i] * kk.x;
-            row[i + 1] *= g; pred += row[i + 1] * kk.y;
-            row[i + 2] *= g; pred += row[i + 2] * kk.z;
-            row[i + 3] *= g; pred += row[i + 3] * kk.w;
-        }
-        float delta = beta * (v - pred);
-        float o = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DK; i += 4) {
-            float4 kk = k4[i / 4], qq = q4[i / 4];
-            row[i] += kk.x * delta;     o += row[i] * (qq.x * q_scale);
-            row[i + 1] += kk.y * delta; o += row[i + 1] * (qq.y * q_scale);
-            row[i + 2] += kk.z * delta; o += row[i + 2] * (qq.z * q_scale);
-            row[i + 3] += kk.w * delta; o += row[i + 3] * (qq.w * q_scale);
-        }
-        if (live) out[(int64_t)t * vper + h * dv + j] = o;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < DK; i++)
-        if (live) tile[lane * (DK + 1) + i] = row[i];
-    __syncthreads();
-    {
-        constexpr int V = DK / 4;
-        float4* S4 = (float4*)S;
-#pragma unroll
-        for (int it = 0; it < V; it++) {
-            int idx4 = it * 64 + lane;
-            int r = idx4 / V, c = (idx4 - r * V) * 4;
-            const float* t = tile + r * (DK + 1) + c;
-            if (idx4 < rows_here * V) S4[idx4] = make_float4(t[0], t[1], t[2], t[3]);
-        }
+        for (int i = 0; i < SEG / 4; i++) ((float4*)S)[i] = make_float4(row[4 * i], row[4 * i + 1], row[4 * i + 2], row[4 * i + 3]);
     }
 }
 
@@ -230,7 +258,7 @@ void delta_rule(const DeltaArgs& d, float* state, float* out, int exact, float* 
         else hipLaunchKernelGGL(delta_rule_fast_k<128>, dim3(blocks), dim3(256), gate_lds, s, d, state, out, q_scale);
         return;
     }
-    int blocks = d.n_v_heads * ((d.head_v_dim + 63) / 64);
+    int blocks = d.n_v_heads * ((d.head_v_dim + DX_ROWS - 1) / DX_ROWS);
     switch (d.head_k_dim) {
         case 32: hipLaunchKernelGGL(delta_rule_k<32>, dim3(blocks), dim3(64), 0, s, d, state, out, q_scale); break;
         case 64: hipLaunchKernelGGL(delta_rule_k<64>, dim3(blocks), dim3(64), 0, s, d, state, out, q_scale); break;

@@ -209,8 +209,8 @@ struct AttnArgs {
     const int* n_pos_dyn;  // overrides n_pos when non-null (decode graphs)
 };
 // exact: the oracle's order (scores, serial softmax sum, positions outermost).
-// scratch: n_q * n_head * n_pos floats.
-void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s);
+// scratch: n_q * n_head * n_pos floats.  gate (n_q == 1; may be null): out *= sigmoid(gate[head * gate_stride + i])
+void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate = nullptr, int gate_stride = 0);
 // split-K flash decoding; scratch: n_q*n_head*n_split*(head_dim+2) floats.
 int attend_split_count(int n_pos_max, int n_q, int head_dim, int group);
 bool attend_split(const AttnArgs& a, int n_split_max, float* scratch, float* out, hipStream_t s);  // false: not launched

@@ -22,7 +22,7 @@ struct FusedGemvP {
     float eps;
     int n_in, mode, head_dim, exact, n_mats, rows_per_wave, total_groups;
     FusedMat m[4];
-    // fast kernels only: the launcher moves unquantized (F32 / F16 / BF16) matrices behind the quantized ones;
+    // the launcher moves unquantized (F32 / F16 / BF16; exact kernel: F32) matrices behind the quantized ones;
     // m[n_mats .. n_mats + n_fmats) are those, total_frows rows in all (epi 0 only)
     int n_fmats, total_frows;
     int fsplit;   // waves that share one unquantized row (1 or 2; the kernel also takes 4): a launch of few such rows and nothing else spreads over more CUs
@@ -30,13 +30,16 @@ struct FusedGemvP {
     const float* conv_w;
     // optional: matrix 0 is the router; the last block to finish picks the experts
     unsigned* route_counter;  // zero between launches
+    const float* route_logits;   // filled by the launcher
+    int terms_stride;            // filled by the launcher: floats of LDS per wave
     int n_expert, n_used;
     int32_t* route_ids;
     float* route_w;
 };
 void fused_gemv(FusedGemvP p, hipStream_t s);
-// whether the fast kernel takes p (formats, shapes, alignment); unquantized matrices are taken by the fast kernel only
+// whether the fast (exact) kernel takes p with unquantized matrices in it (formats, shapes, alignment)
 bool fused_gemv_fast_takes(const FusedGemvP& p);
+bool fused_gemv_exact_takes(const FusedGemvP& p);
 
 struct GdnCoreP {
     const float* conv;  // [q | k | v] after conv + silu
