@@ -140,58 +140,61 @@ __device__ void wave_row_terms(const uint8_t* wq, const uint8_t* ws, int n_in, i
 // ------------------------------------------------------------------ router in one wave
 // softmax over all experts, then n_used rounds of arg-max with ties to the lower id, the
 // picked probabilities summed in pick order (src/ops/mod.rs:1191-1216, naive.rs:362-376).
-// Called by one wave; probs (LDS, n_expert floats) holds the logits on entry.
-__device__ void wave_route(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane) {
+// Called by one wave; probs (LDS, n_expert floats) holds the logits on entry.  A lane keeps its NE probabilities (experts
+// lane + 64 i) in registers; a round is two reductions over the wave, the value and then the lowest id that has it.
+template <int NE>
+__device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane) {
+    float v[NE];
     float m = -INFINITY;
-    for (int e = lane; e < n_expert; e += 64) m = fmaxf(m, probs[e]);
-    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        const int e = lane + 64 * i;
+        v[i] = e < n_expert ? probs[e] : -INFINITY;
+        m = fmaxf(m, v[i]);
+    }
+    m = group_max<64>(m);
     float part = 0.0f;
-    for (int e = lane; e < n_expert; e += 64) {
-        float v = it_expf(probs[e] - m);
-        probs[e] = v;
-        part += v;
+#pragma unroll
+    for (int i = 0; i < NE; i++) {
+        const int e = lane + 64 * i;
+        v[i] = e < n_expert ? it_expf(v[i] - m) : -1.0f;
+        if (e < n_expert) {
+            probs[e] = v[i];
+            part += v[i];
+        }
     }
     wave_lds_sync();
     float sum;
     if (exact) {
-        float acc = 0.0f;
-        if (lane == 0)
-            for (int e = 0; e < n_expert; e++) acc += probs[e];
-        sum = __shfl(acc, 0, 64);
+        sum = __shfl(lane == 0 ? fold_terms(probs, n_expert) : 0.0f, 0, 64);
     } else {
         for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
         sum = part;
     }
-    for (int e = lane; e < n_expert; e += 64) probs[e] = probs[e] / sum;
-    wave_lds_sync();
+#pragma unroll
+    for (int i = 0; i < NE; i++)
+        if (lane + 64 * i < n_expert) v[i] = v[i] / sum;
+    constexpr float TOP = (float)(1 << 20);
     float picked_p = 0.0f;  // lane r keeps pick r's probability
     int picked_id = -1;
     for (int r = 0; r < n_used; r++) {
-        float bv = 0.0f;
-        int bi = -1;
-        for (int e = lane; e < n_expert; e += 64) {
-            float v = probs[e];
-            if (v < 0.0f) continue;  // taken (probabilities are never negative)
-            if (bi < 0 || v > bv) {
-                bv = v;
-                bi = e;
-            }
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-            float ov = __shfl_xor(bv, o, 64);
-            int oi = __shfl_xor(bi, o, 64);
-            bool take = oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi < bi));
-            if (take) {
-                bv = ov;
-                bi = oi;
-            }
-        }
+        float best = v[0];
+#pragma unroll
+        for (int i = 1; i < NE; i++) best = fmaxf(best, v[i]);
+        best = group_max<64>(best);
+        float at = 0.0f;   // TOP - the lowest id of this lane with that probability (taken and absent ones hold -1)
+#pragma unroll
+        for (int i = NE - 1; i >= 0; i--)
+            if (v[i] == best && best >= 0.0f) at = TOP - (float)(lane + 64 * i);
+        at = group_max<64>(at);
+        const int id = at > 0.0f ? (int)(TOP - at) : r;   // (probabilities that are not numbers: some expert)
         if (lane == r) {
-            picked_p = bv;
-            picked_id = bi;
+            picked_p = best;
+            picked_id = id;
         }
-        if (lane == 0 && bi >= 0) probs[bi] = -1.0f;
-        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < NE; i++)
+            if (lane + 64 * i == id) v[i] = -1.0f;
     }
     // sum in pick order, serial f32
     float s = 0.0f;
@@ -202,6 +205,12 @@ __device__ void wave_route(float* probs, int n_expert, int n_used, int exact, in
         weights[lane] = picked_p / denom;
     }
     wave_lds_sync();
+}
+constexpr int ROUTE_MAX_EXPERTS = 2048;
+__device__ void wave_route(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane) {
+    if (n_expert <= 64) wave_route_n<1>(probs, n_expert, n_used, exact, ids, weights, lane);
+    else if (n_expert <= 512) wave_route_n<8>(probs, n_expert, n_used, exact, ids, weights, lane);
+    else wave_route_n<32>(probs, n_expert, n_used, exact, ids, weights, lane);   // up to ROUTE_MAX_EXPERTS (match_ffn)
 }
 
 constexpr int FG_THREADS = 512, FG_LDS_MAX = 128 * 1024;
@@ -366,7 +375,9 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         __shared__ int is_last;
         __builtin_amdgcn_s_waitcnt(0);   // the logits went past the caches (put_out): they are there, no fence needed
         __syncthreads();
-        if (tid == 0) {
+        if (tid == 0 && gridDim.x == 1) {
+            is_last = 1;
+        } else if (tid == 0) {
             unsigned prev = __hip_atomic_fetch_add(p.route_counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             is_last = prev == gridDim.x - 1;
         }
@@ -762,11 +773,12 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     float* terms = terms_all + (size_t)wave * (NU + 1) * R * tstride;
     const int groups = (p.n_out + R - 1) / R;
     RowRegs<1> rr[MAXU], rsh;
-    auto load_all = [&](int row0, int nrows) {
+    const int my_id = p.route_ids[lane < NU ? lane : 0];   // every pick in one load
+    auto load_all = [&](int row0, int nrows) __attribute__((always_inline)) {
 #pragma unroll
         for (int y = 0; y < MAXU; y++) {
             if (y < NU) {
-                const int64_t e = p.route_ids[y];
+                const int64_t e = __builtin_amdgcn_readlane(my_id, y);
                 if (p.fmt == W_NVFP4) load_items<W_NVFP4, 1>(rr[y], p.q + e * p.q_stride, p.s + e * p.s_stride, n_in, row0, nrows, lane);
                 else load_items<W_Q8_0, 1>(rr[y], p.q + e * p.q_stride, p.s + e * p.s_stride, n_in, row0, nrows, lane);
             }
