@@ -565,6 +565,8 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
         g.route_w_out = (float*)rt.p[2];
     }
 
+    if (exact && sff > 2048) return false;   // a row of the shared down product is one pass of a wave
+
     MoeDownP d{};
     d.g_all = (const float*)g_all;
     d.g_shared = (const float*)e_gate;

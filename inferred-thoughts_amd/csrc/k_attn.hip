@@ -13,6 +13,7 @@
 // path at 1e-3.
 #include <algorithm>
 #include "it_device.h"
+#include "it_dot.h"
 #include "it_reduce.h"
 #include "kernels.h"
 
@@ -36,13 +37,14 @@ namespace itk {
 // ------------------------------------------------------------------ exact
 // One block per (query, head).  Scores and weights sit in LDS up to EXACT_LDS positions (beyond, in `scratch`).  What has an
 // order is a chain: a position's dot in its thread, the weights' sum in one lane, a dim's weighted sum in its thread, each
-// with its loads several steps ahead.  333 positions, 16 heads of 256: TIMES
+// with its loads several steps ahead.  333 positions, 16 heads of 256: 28 us (115 with every read waited for
+// and the weight divided anew for every dim).
 constexpr int EXACT_LDS = 4096;
-__global__ __launch_bounds__(256) void attend_exact_k(AttnArgs a, float* __restrict__ scratch, float* __restrict__ out,
+__global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __restrict__ scratch, float* __restrict__ out,
                                                       const float* __restrict__ gate, int gate_stride, int lds_pos) {
     extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each)
-    __shared__ float red[8];
-    const int hd = a.head_dim, tid = threadIdx.x;
+    __shared__ float red[17];
+    const int hd = a.head_dim, tid = threadIdx.x, nt = blockDim.x;
     const int n_pos_last = a.n_pos_dyn ? *a.n_pos_dyn : a.n_pos;
     const int t = blockIdx.x / a.n_head, h = blockIdx.x % a.n_head;
     const int group = a.n_head / a.n_head_kv;
@@ -53,10 +55,10 @@ __global__ __launch_bounds__(256) void attend_exact_k(AttnArgs a, float* __restr
     float* near = qs + ((hd + 3) & ~3);
     float* far = scratch + (int64_t)blockIdx.x * n_pos_last;
     auto score = [&](int s) -> float& { return s < lds_pos ? near[s] : far[s]; };
-    for (int i = tid; i < hd; i += 256) qs[i] = q[i];
+    for (int i = tid; i < hd; i += nt) qs[i] = q[i];
     __syncthreads();
     float m = -INFINITY;
-    for (int s = tid; s < n_pos; s += 256) {
+    for (int s = tid; s < n_pos; s += nt) {
         const uint16_t* key = a.k + (int64_t)s * a.kv_dim + off;
         float dot = 0.0f;
         auto add8 = [&](int i, uint4 kk) {
@@ -91,45 +93,46 @@ __global__ __launch_bounds__(256) void attend_exact_k(AttnArgs a, float* __restr
     for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_down(m, o, 64));
     if ((tid & 63) == 0) red[tid >> 6] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    for (int s = tid; s < n_pos; s += 256) score(s) = it_expf(score(s) - m);
+    m = red[0];
+    for (int w = 1; w < nt / 64; w++) m = fmaxf(m, red[w]);
+    for (int s = tid; s < n_pos; s += nt) score(s) = it_expf(score(s) - m);
     __threadfence_block();
     __syncthreads();
     if (tid == 0) {
-        float sum = 0.0f;
-        int s = 0;
-        for (; s + 16 <= n_lds; s += 16) {
-            float4 v[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) v[c] = *(const float4*)(near + s + 4 * c);
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                sum += v[c].x;
-                sum += v[c].y;
-                sum += v[c].z;
-                sum += v[c].w;
-            }
-        }
-        for (; s < n_lds; s++) sum += near[s];
+        float sum = fold_terms(near, n_lds);
 #pragma unroll 16
-        for (s = lds_pos; s < n_pos; s++) sum += far[s];
-        red[4] = sum;
+        for (int s = lds_pos; s < n_pos; s++) sum += far[s];
+        red[16] = sum;
     }
     __syncthreads();
-    const float sum = red[4];
-    for (int s = tid; s < n_pos; s += 256) score(s) = score(s) / sum;
+    const float sum = red[16];
+    for (int s = tid; s < n_pos; s += nt) score(s) = score(s) / sum;
     __threadfence_block();
     __syncthreads();
-    for (int i = tid; i < hd; i += 256) {
+    for (int i = tid; i < hd; i += nt) {
         const uint16_t* v = a.v + off + i;
         float acc = 0.0f;
         int s = 0;
-        for (; s + 16 <= n_lds; s += 16) {
-            uint16_t x[16];
+        constexpr int AHEAD = 32;   // positions whose values are on their way while as many are added
+        uint16_t x0[AHEAD], x1[AHEAD];
+        auto ask = [&](uint16_t (&x)[AHEAD], int from) __attribute__((always_inline)) {
 #pragma unroll
-            for (int c = 0; c < 16; c++) x[c] = v[(int64_t)(s + c) * a.kv_dim];
+            for (int c = 0; c < AHEAD; c++) x[c] = v[(int64_t)min(from + c, n_pos - 1) * a.kv_dim];
+        };
+        auto add = [&](const uint16_t (&x)[AHEAD], int from) __attribute__((always_inline)) {
 #pragma unroll
-            for (int c = 0; c < 16; c++) acc += near[s + c] * it_f16_to_f32(x[c]);
+            for (int c = 0; c < AHEAD; c++) acc += near[from + c] * it_f16_to_f32(x[c]);
+        };
+        if (n_lds >= AHEAD) ask(x0, 0);
+        for (; s + 2 * AHEAD <= n_lds; s += 2 * AHEAD) {
+            ask(x1, s + AHEAD);
+            add(x0, s);
+            ask(x0, s + 2 * AHEAD);
+            add(x1, s + AHEAD);
+        }
+        if (s + AHEAD <= n_lds) {
+            add(x0, s);
+            s += AHEAD;
         }
         for (; s < n_lds; s++) acc += near[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
 #pragma unroll 8
@@ -142,7 +145,9 @@ __global__ __launch_bounds__(256) void attend_exact_k(AttnArgs a, float* __restr
 void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate, int gate_stride) {
     if (a.n_q <= 0) return;
     const int lds_pos = std::min((a.n_pos + 3) & ~3, EXACT_LDS);
-    hipLaunchKernelGGL(attend_exact_k, dim3(a.n_q * a.n_head), dim3(256), ((size_t)((a.head_dim + 3) & ~3) + lds_pos) * sizeof(float), s, a,
+    // few blocks: a thread per position while the score phase has that many; many: blocks that share a CU
+    const int threads = a.n_q * a.n_head < 512 && a.n_pos > 256 ? 1024 : 256;
+    hipLaunchKernelGGL(attend_exact_k, dim3(a.n_q * a.n_head), dim3(threads), ((size_t)((a.head_dim + 3) & ~3) + lds_pos) * sizeof(float), s, a,
                        scratch, out, gate, gate_stride, lds_pos);
 }
 

@@ -4,6 +4,7 @@
 // same products summed by the f32 matrix instruction, whose inputs, products and sums are f32 as well.
 #include "it_device.h"
 #include "kernels.h"
+#include "it_dot.h"
 
 namespace itk {
 namespace {
@@ -45,32 +46,26 @@ __global__ __launch_bounds__(256) void float_fold_exact_k(FloatMats m, const flo
     __shared__ __align__(16) float prod[EX_ROWS][EX_K + 4];   // + 4: the rows' 16-byte reads fall on different banks
     const int row0 = blockIdx.x * EX_ROWS, t = blockIdx.y, tid = threadIdx.x;
     const float* xt = x + (int64_t)t * n_in;
+    const uint8_t* rows[EX_ROWS];
+#pragma unroll
+    for (int r = 0; r < EX_ROWS; r++) rows[r] = float_row<FMT>(m, row0 + r, n_in);
     float sum = 0.0f;
     for (int k0 = 0; k0 < n_in; k0 += EX_K) {
         const int kn = min(EX_K, n_in - k0);
         if (k0) __syncthreads();
-        for (int r = 0; r < EX_ROWS; r++) {
-            const uint8_t* row = float_row<FMT>(m, row0 + r, n_in);
-#pragma unroll 8
-            for (int i = tid; i < kn; i += 256) prod[r][i] = load_w1<FMT>(row, k0 + i) * xt[k0 + i];
+        // (the activation once, every row's loads of a step together)
+#pragma unroll 2
+        for (int i = tid; i < kn; i += 256) {
+            const float xv = xt[k0 + i];
+            float wv[EX_ROWS];
+#pragma unroll
+            for (int r = 0; r < EX_ROWS; r++) wv[r] = load_w1<FMT>(rows[r], k0 + i);
+#pragma unroll
+            for (int r = 0; r < EX_ROWS; r++) prod[r][i] = wv[r] * xv;
         }
         __syncthreads();
         if (tid < EX_ROWS) {
-            const float* p = prod[tid];
-            int i = 0;
-            for (; i + 16 <= kn; i += 16) {
-                float4 v[4];
-#pragma unroll
-                for (int c = 0; c < 4; c++) v[c] = *(const float4*)(p + i + 4 * c);
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    sum += v[c].x;
-                    sum += v[c].y;
-                    sum += v[c].z;
-                    sum += v[c].w;
-                }
-            }
-            for (; i < kn; i++) sum += p[i];
+            sum = fold_terms_from(sum, prod[tid], kn);
         }
     }
     if (tid < EX_ROWS) float_store(m, t, row0 + tid, out_scale != 1.0f ? sum * out_scale : sum);

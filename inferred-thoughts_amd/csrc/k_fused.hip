@@ -141,7 +141,7 @@ __device__ void wave_row_terms(const uint8_t* wq, const uint8_t* ws, int n_in, i
 // softmax over all experts, then n_used rounds of arg-max with ties to the lower id, the
 // picked probabilities summed in pick order (src/ops/mod.rs:1191-1216, naive.rs:362-376).
 // Called by one wave; probs (LDS, n_expert floats) holds the logits on entry.  A lane keeps its NE probabilities (experts
-// lane + 64 i) in registers; a round is two reductions over the wave, the value and then the lowest id that has it.
+// lane + 64 i) in registers; a round is one reduction over the wave for the value and a ballot per register for the lowest id that has it.
 template <int NE>
 __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane) {
     float v[NE];
@@ -174,20 +174,19 @@ __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, 
 #pragma unroll
     for (int i = 0; i < NE; i++)
         if (lane + 64 * i < n_expert) v[i] = v[i] / sum;
-    constexpr float TOP = (float)(1 << 20);
     float picked_p = 0.0f;  // lane r keeps pick r's probability
     int picked_id = -1;
     for (int r = 0; r < n_used; r++) {
         float best = v[0];
 #pragma unroll
         for (int i = 1; i < NE; i++) best = fmaxf(best, v[i]);
-        best = group_max<64>(best);
-        float at = 0.0f;   // TOP - the lowest id of this lane with that probability (taken and absent ones hold -1)
+        best = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, group_max_tail<64>(best)), 63));
+        int id = best >= 0.0f ? -1 : r;   // (probabilities that are not numbers: some expert)
 #pragma unroll
-        for (int i = NE - 1; i >= 0; i--)
-            if (v[i] == best && best >= 0.0f) at = TOP - (float)(lane + 64 * i);
-        at = group_max<64>(at);
-        const int id = at > 0.0f ? (int)(TOP - at) : r;   // (probabilities that are not numbers: some expert)
+        for (int i = 0; i < NE; i++) {    // taken and absent experts hold -1
+            const unsigned long long has = __ballot(v[i] == best);
+            if (id < 0 && has) id = 64 * i + __builtin_ctzll(has);
+        }
         if (lane == r) {
             picked_p = best;
             picked_id = id;
@@ -752,6 +751,7 @@ void moe_glu_fused(MoeGluP p, hipStream_t s) {
 // ------------------------------------------------------------------ moe_down_fused
 // x[j] += sum_e w_e * (down_e[j] . g_e * scale2_e) + (shared_down[j] . g_sh) * sigmoid(logit)
 // (src/ops/mod.rs:1134-1171 then add_assign), experts ascending, shared last.
+constexpr int DOWN_ITEMS = 8;
 __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int n_in = p.n_in, nb = n_in >> 5;       // expert down: n_in = expert_ff
@@ -763,8 +763,7 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     float* terms_all = (float*)(xq + ((NU * n_in + sh_in + 15) & ~15));
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     it_count_expert_reads(p.route_ids, NU, p.counts_gate, p.counts_up, p.counts_down, p.tally);
-    constexpr int MAXU = 16;  // n_used <= 16 (checked on the host)
-    const int R = p.rows_per_wave;  // R * (n_in / 32) <= 64: one item per lane per expert
+    const int R = p.rows_per_wave;
     const int T = p.fmt == W_NVFP4 ? nb * 2 : nb;
     const int shT = p.sh_fmt == W_NVFP4 ? sh_nb * 2 : sh_nb;
     const int Tmax = (T > shT ? T : shT);
@@ -772,22 +771,38 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     // terms[(y * R + r) * tstride + k]
     float* terms = terms_all + (size_t)wave * (NU + 1) * R * tstride;
     const int groups = (p.n_out + R - 1) / R;
-    RowRegs<1> rr[MAXU], rsh;
+    // A wave's (pick, row, 32-element unit) items are dealt out over its lanes without a gap, 64 * DOWN_ITEMS of them (all of
+    // a group's, for what the launcher sizes it for) in flight at once.
+    RowRegs<DOWN_ITEMS> rr;
+    RowRegs<1> rsh;
     const int my_id = p.route_ids[lane < NU ? lane : 0];   // every pick in one load
-    auto load_all = [&](int row0, int nrows) __attribute__((always_inline)) {
+    auto load_all = [&](int row0, int nrows, int i0) __attribute__((always_inline)) {
+        const int per = nrows * nb;
 #pragma unroll
-        for (int y = 0; y < MAXU; y++) {
-            if (y < NU) {
-                const int64_t e = __builtin_amdgcn_readlane(my_id, y);
-                if (p.fmt == W_NVFP4) load_items<W_NVFP4, 1>(rr[y], p.q + e * p.q_stride, p.s + e * p.s_stride, n_in, row0, nrows, lane);
-                else load_items<W_Q8_0, 1>(rr[y], p.q + e * p.q_stride, p.s + e * p.s_stride, n_in, row0, nrows, lane);
+        for (int k = 0; k < DOWN_ITEMS; k++) {
+            const int it = min(i0 + k * 64 + lane, NU * per - 1), y = it / per, ru = it - y * per, r = ru / nb, u = ru - r * nb;
+            const int64_t e = __shfl(my_id, y, 64);
+            const int64_t row = row0 + r;
+            const uint8_t *q = p.q + e * p.q_stride, *sc = p.s + e * p.s_stride;
+            if (p.fmt == W_NVFP4) {
+                rr.wa[k] = *(const uint4*)(q + row * (n_in >> 1) + u * 16);
+            } else {
+                const uint4* wp = (const uint4*)(q + row * n_in + u * 32);
+                rr.wa[k] = wp[0];
+                rr.wb[k] = wp[1];
             }
+            rr.sc[k] = ((const uint16_t*)sc)[row * nb + u];
         }
+    };
+    auto load_shared = [&](int row0, int nrows) __attribute__((always_inline)) {
         if (p.sh_fmt == W_NVFP4) load_items<W_NVFP4, 1>(rsh, p.sh_q, p.sh_s, sh_in, row0, nrows, lane);
         else load_items<W_Q8_0, 1>(rsh, p.sh_q, p.sh_s, sh_in, row0, nrows, lane);
     };
     const int g0 = blockIdx.x * 4 + wave;
-    if (g0 < groups) load_all(g0 * R, min(R, p.n_out - g0 * R));
+    if (g0 < groups) {
+        load_all(g0 * R, min(R, p.n_out - g0 * R), 0);
+        load_shared(g0 * R, min(R, p.n_out - g0 * R));
+    }
     const float gate = it_sigmoid(p.logit[0]);
     // stage all NU + 1 intermediates as f32 (the term region is free until the main loop)
     {
@@ -801,13 +816,26 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     }
     for (int g = g0; g < groups; g += gridDim.x * 4) {
         const int row0 = g * R, nrows = min(R, p.n_out - row0);
-        if (g != g0) load_all(row0, nrows);
+        if (g != g0) load_shared(row0, nrows);
+        const int per = nrows * nb;
+        for (int i0 = 0; i0 < NU * per; i0 += 64 * DOWN_ITEMS) {
+            if (g != g0 || i0) load_all(row0, nrows, i0);
 #pragma unroll
-        for (int y = 0; y < MAXU; y++) {
-            if (y < NU) {
-                float* t = terms + (size_t)y * R * tstride;
-                if (p.fmt == W_NVFP4) compute_items<W_NVFP4, 1>(rr[y], n_in, nrows, xq + y * n_in, xs + y * nb, t, tstride, lane);
-                else compute_items<W_Q8_0, 1>(rr[y], n_in, nrows, xq + y * n_in, xs + y * nb, t, tstride, lane);
+            for (int k = 0; k < DOWN_ITEMS; k++) {
+                const int it = i0 + k * 64 + lane, y = it / per, ru = it - y * per, r = ru / nb, u = ru - r * nb;
+                if (it >= NU * per) continue;
+                const uint4* ap = (const uint4*)(xq + y * n_in + u * 32);
+                const uint4 a0 = ap[0], a1 = ap[1];
+                const float dx = xs[y * nb + u];
+                float* t = terms + ((size_t)y * R + r) * tstride;
+                if (p.fmt == W_Q8_0) {
+                    t[u] = unit_q8_0(rr.wa[k], rr.wb[k], (uint16_t)rr.sc[k], a0, a1, dx);
+                } else {
+                    float tA, tB;
+                    unit_nvfp4(rr.wa[k], rr.sc[k], a0, a1, dx, &tA, &tB);
+                    t[2 * u] = tA;
+                    t[2 * u + 1] = tB;
+                }
             }
         }
         {
@@ -846,9 +874,9 @@ void moe_down_fused(MoeDownP p, hipStream_t s) {
     const int nb = p.n_in / 32, sh_nb = p.sh_n_in / 32;
     const int T = (p.fmt == W_NVFP4 ? nb * 2 : nb), shT = (p.sh_fmt == W_NVFP4 ? sh_nb * 2 : sh_nb);
     const int Tmax = T > shT ? T : shT;
+    // a row group per wave over the whole chip (256 blocks of four waves), and what the kernel's registers hold
     int R = 4;
-    while (R > 1 && (p.n_used + 1) * R > 64) R /= 2;
-    while (R > 1 && (R * nb > 64 || R * sh_nb > 64)) R /= 2;
+    while (R > 1 && ((p.n_used + 1) * R > 64 || R * sh_nb > 64 || p.n_used * R * nb > 64 * DOWN_ITEMS || (p.n_out + R - 1) / R < 1024)) R /= 2;
     auto lds_for = [&](int r) {
         size_t terms = (size_t)4 * (p.n_used + 1) * r * (Tmax + 4) * 4;
         size_t stage = (size_t)(p.n_used * p.n_in + p.sh_n_in) * 4;  // f32 staging shares the term region
