@@ -167,7 +167,7 @@ void it_hip::need_eager(const char* why, bool moved) {
 }
 
 void it_hip::finish_pass() {
-    if (!held.empty()) release_held();
+    if (!held.empty()) flush_held(nullptr);
     if (mode == Mode::Deferred) {
         flush_deferred();
         mode = Mode::Eager;
@@ -323,7 +323,7 @@ bool it_hip::replay_pass(const void* tag, uint64_t pos, const uint32_t* id, uint
     for (auto& kv : acts) {
         kv.second.dev_current = false;
         kv.second.elided = false;
-        kv.second.q_valid = false;
+        kv.second.stale();
     }
     for (const Graph::Left& l : g->left) {
         l.a->dev_current = true;
@@ -399,7 +399,7 @@ float* it_hip::act_in(const float* host, size_t len) {
         h2d++;
         h2d_bytes += len * sizeof(float);
         a->dev_current = true;
-        a->q_valid = false;
+        a->stale();
     }
     return a->dev;
 }
@@ -408,7 +408,7 @@ float* it_hip::act_out(const float* host, size_t len) {
     if (!a) return nullptr;
     a->dev_current = true;
     a->elided = false;
-    a->q_valid = false;
+    a->stale();
     return a->dev;
 }
 bool it_hip::held_touches(const void* dev, size_t bytes) const {
@@ -431,7 +431,7 @@ void it_hip::mark_elided(const std::vector<const void*>& devs) {
 }
 float* it_hip::act_inout(const float* host, size_t len) {
     float* d = act_in(host, len);
-    if (d) acts[host].q_valid = false;
+    if (d) acts[host].stale();
     return d;
 }
 
@@ -452,7 +452,7 @@ bool it_hip::act_q_reserve(Act& a, size_t len) {
         return false;
     a.q_cap = len;
     quant_bytes += len / 32 * 4 + len;
-    a.q_valid = false;
+    a.stale();
     return true;
 }
 
@@ -476,6 +476,43 @@ bool it_hip::act_quantized(const float* host, size_t len, const float** scales, 
     *scales = a.q_scales;
     *quants = a.q_quants;
     if (dev_x) *dev_x = x;
+    return true;
+}
+
+bool it_hip::act_split(const float* host, size_t len, int row, SplitOut* out) {
+    const float* as;
+    const int8_t* aq;
+    if (!act_quantized(host, len, &as, &aq, nullptr)) return false;
+    Act& a = acts[host];
+    if (a.s_cap < len) {
+        need_eager("a split-activation buffer has to grow");
+        if (a.split.h) {
+            check(hipStreamSynchronize(stream), "sync before split free");
+            quant_bytes -= a.s_cap * 4 + a.s_cap / 32 * 4;
+            (void)hipFree(a.split.h);
+            a.split = SplitOut{};
+            a.s_cap = 0;
+        }
+        const size_t cap = (len + 255) / 256 * 256;
+        if (!check(hipMalloc((void**)&a.split.h, cap * 4 + cap / 32 * 4), "hipMalloc(split activations)")) return false;
+        a.split.l = a.split.h + cap;
+        a.split.scale = (float*)(a.split.l + cap);
+        a.s_cap = cap;
+        quant_bytes += cap * 4 + cap / 32 * 4;
+        a.s_valid = false;
+    }
+    if (!a.s_valid || a.s_len != len || a.s_row != row) {
+        const SplitOut sp = a.split;
+        OpRec rec;
+        rec.id = OP_SPLIT;
+        rec.p[0] = aq; rec.p[1] = as; rec.p[2] = sp.h; rec.p[3] = sp.l; rec.p[4] = sp.scale; rec.i[0] = (int64_t)len; rec.i[1] = row;
+        submit(FAM_OTHER, len * 5, sig_of(OP_SPLIT, aq, as, sp.h, len, row), rec,
+               [=](hipStream_t s) { split_rows(aq, as, (int64_t)len / row, row, sp, s); });
+        a.s_valid = true;
+        a.s_len = len;
+        a.s_row = row;
+    }
+    *out = a.split;
     return true;
 }
 
@@ -1065,22 +1102,6 @@ const float2* it_hip::rope_table(float theta, uint64_t n_rot, uint64_t need_pos)
     return r.dev;
 }
 
-void* it_hip::moe_f16_for(size_t bytes) {
-    if (moe_f16_bytes < bytes) {
-        need_eager("expert activation scratch has to grow");
-        if (moe_f16) {
-            check(hipStreamSynchronize(stream), "sync before scratch free");
-            (void)hipFree(moe_f16);
-            moe_f16 = nullptr;
-            moe_f16_bytes = 0;
-        }
-        const size_t want = bytes + bytes / 4;
-        if (!check(hipMalloc(&moe_f16, want), "hipMalloc(expert activation scratch)")) return nullptr;
-        moe_f16_bytes = want;
-    }
-    return moe_f16;
-}
-
 const int32_t* it_hip::zero_ids_for(size_t n) {
     if (zero_ids_n < n) {
         need_eager("the one-expert id list has to grow");
@@ -1195,6 +1216,7 @@ void it_hip::drop_all() {
     if (stream) (void)hipStreamSynchronize(stream);
     for (auto& kv : acts) {
         if (kv.second.dev) (void)hipFree(kv.second.dev);
+        if (kv.second.split.h) (void)hipFree(kv.second.split.h);
         if (kv.second.q_scales) (void)hipFree(kv.second.q_scales);
         if (kv.second.q_quants) (void)hipFree(kv.second.q_quants);
     }
@@ -1239,7 +1261,6 @@ it_hip::~it_hip() {
     if (route_w) (void)hipFree(route_w);
     if (attn_scratch) (void)hipFree(attn_scratch);
     if (gdn_work) (void)hipFree(gdn_work);
-    if (moe_f16) (void)hipFree(moe_f16);
     if (zero_ids) (void)hipFree(zero_ids);
     if (moe_work) (void)hipFree(moe_work);
     if (argmax_idx) (void)hipFree(argmax_idx);
@@ -1452,26 +1473,26 @@ void it_hip_rms_norm(it_hip* be, const float* x, uint64_t x_len, const float* w,
     float* dx = be->act_in(x, x_len);
     float* dout = (out == x) ? dx : be->act_out(out, out_len);
     if (!dw || !dx || !dout) return;
-    if (out == x) be->acts[x].q_valid = false;
+    if (out == x) be->acts[x].stale();
     int64_t rows = (int64_t)(x_len / w_len);
     int nd = (int)w_len, exact = be->exact;
     // A batch's normed rows go to products with quantized weights next (qwen35.rs:1006-1093): their Q8_0 form is
     // written by the same launch.  Single-token passes keep the two ops apart for the pass fuser.
-    float* qs = nullptr;
-    int8_t* qq = nullptr;
+    QuantOut qo;
     if (rows > 1 && be->mode == it_hip::Mode::Eager && rms_norm_writes_q8(dx, dw, dout, nd)) {
         it_hip::Act& a = be->acts[out];
         if (be->act_q_reserve(a, out_len)) {
-            qs = a.q_scales;
-            qq = a.q_quants;
+            qo.scales = a.q_scales;
+            qo.quants = a.q_quants;
             a.q_valid = true;
             a.q_len = out_len;
         }
     }
     it_hip::OpRec rec;
-    rec.id = OP_RMS; rec.p[0] = dx; rec.p[1] = dw; rec.p[2] = dout; rec.i[0] = rows; rec.i[1] = nd; rec.f[0] = eps;
+    rec.id = OP_RMS; rec.p[0] = dx; rec.p[1] = dw; rec.p[2] = dout; rec.p[3] = qo.scales; rec.p[4] = qo.quants;
+    rec.i[0] = rows; rec.i[1] = nd; rec.f[0] = eps;
     be->submit(it_hip::FAM_NORM, x_len * 8, sig_of(OP_RMS, dx, dw, eps, dout, rows, nd), rec,
-               [=](hipStream_t s) { rms_norm(dx, dw, eps, dout, rows, nd, exact, s, qs, qq); });
+               [=](hipStream_t s) { rms_norm(dx, dw, eps, dout, rows, nd, exact, s, qo.scales, qo.quants); });
 }
 
 void it_hip_rms_norm_heads(it_hip* be, float* x, uint64_t x_len, const float* w, uint64_t w_len,
@@ -1487,7 +1508,7 @@ void it_hip_rms_norm_heads(it_hip* be, float* x, uint64_t x_len, const float* w,
     it_hip::OpRec rec;
     rec.id = OP_RMS_HEADS; rec.p[0] = dx; rec.p[1] = dw; rec.i[0] = hd; rec.i[1] = heads; rec.f[0] = eps;
     be->submit(it_hip::FAM_NORM, x_len * 8, sig_of(OP_RMS_HEADS, dx, dw, hd, eps, heads), rec,
-               [=](hipStream_t s) { rms_norm_heads(dx, dw, hd, eps, heads, exact, s); });
+               [=, batch = be->in_pass && be->pass_tokens > 1](hipStream_t s) { rms_norm_heads(dx, dw, hd, eps, heads, exact, s, batch); });
 }
 
 void it_hip_l2_norm_heads(it_hip* be, float* x, uint64_t x_len, uint64_t head_dim, float eps) {
@@ -1501,7 +1522,7 @@ void it_hip_l2_norm_heads(it_hip* be, float* x, uint64_t x_len, uint64_t head_di
     it_hip::OpRec rec;
     rec.id = OP_L2; rec.p[0] = dx; rec.i[0] = hd; rec.i[1] = heads; rec.f[0] = eps;
     be->submit(it_hip::FAM_NORM, x_len * 8, sig_of(OP_L2, dx, hd, eps, heads), rec,
-               [=](hipStream_t s) { l2_norm_heads(dx, hd, eps, heads, exact, s); });
+               [=, batch = be->in_pass && be->pass_tokens > 1](hipStream_t s) { l2_norm_heads(dx, hd, eps, heads, exact, s, batch); });
 }
 
 static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_t x_len, float* out,
@@ -1531,51 +1552,30 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     if (!dout) return;
     int nt = (int)n;
     const int exact = be->exact;
-    // A dense NVFP4 matrix over a batch (the shared expert of an NVFP4 file during prefill) has no int8 tile kernel
-    // of its own; in fast mode it runs as a batch of one expert on the f16 tile kernel instead of one GEMV per token.
+    // A dense NVFP4 matrix over a batch (the shared expert of an NVFP4 file) has no int8 tile kernel of its own; in fast mode
+    // it runs on the f16 tile kernels of the experts, as one of them:
+    //   128 .. 1,024 tokens: tiles of 16 (2048 x 512 over 1,024 tokens: 34 against 68 us on the 128-wide tiles, whose handful
+    //     of blocks is latency-bound there; 16 against 19 us of GEMVs at 128 tokens)
+    //   above: tiles of 128 (82 against 736 us of GEMVs at 5,700 tokens)
+    //   128 .. 512 tokens of a shape that the tiles do not take: eight or sixteen tokens per pass over the rows
+    //     (k_moe_rows.hip; 32 against 70 us for 2048 x 512 at 512 tokens)
     ExpertsView ev{};
+    ev.q = v.q; ev.scales = v.scales; ev.fmt = v.fmt; ev.n_in = v.n_in; ev.n_out = v.n_out; ev.n_expert = 1;
     const int32_t* zids = nullptr;
     int32_t* work = nullptr;
-    void* fwork = nullptr;
-    size_t work_ints = 0, fwork_bytes = 0;
-    bool one_expert = false, grouped = false;
-    // (from 513 tokens on: a call costs 55-80 us for the grouping, the f16 split and a latency-bound handful of
-    // tiles, which the GEMVs reach at about 512 tokens)
-    // A dense NVFP4 matrix over 128 .. 512 tokens whose shape the 16-pair tiles do not take: eight or sixteen tokens per
-    // pass over the rows (k_moe_rows.hip) instead of one GEMV per token (32 against 70 us for 2048 x 512 at 512 tokens;
-    // below 128 tokens the GEMVs, which fill the chip with one block row per token, are as fast).
-    ExpertsView rv{};
-    rv.q = v.q; rv.scales = v.scales; rv.q_stride = 0; rv.s_stride = 0; rv.fmt = v.fmt; rv.n_in = v.n_in; rv.n_out = v.n_out;
-    rv.n_expert = 1; rv.scale2 = nullptr; rv.counts = nullptr;
-    // 128 .. 1,024 tokens: as a batch of ONE expert on the 16-pair tiles (2048 x 512 over 1,024 tokens: 34 against 68 us
-    // on the 128-pair tiles, whose handful of blocks is latency-bound there; 16 against 19 us of GEMVs at 128 tokens)
-    bool skinny_dense = false;
-    if (!exact && v.fmt == W_NVFP4 && n >= 128 && n <= 1024) {
-        ev.q = v.q; ev.scales = v.scales; ev.q_stride = 0; ev.s_stride = 0;
-        ev.fmt = v.fmt; ev.n_in = v.n_in; ev.n_out = v.n_out; ev.n_expert = 1; ev.scale2 = nullptr; ev.counts = nullptr;
-        zids = be->zero_ids_for(n);
-        work = be->moe_work_for(n, 1, &work_ints);
-        fwork_bytes = itk::experts_f16_work_bytes(nt, v.n_in);
-        fwork = be->moe_f16_for(fwork_bytes);
-        skinny_dense = zids && work && fwork && itk::experts_f16s_takes(ev, nullptr, nt, aq, dout);
-        if (skinny_dense) grouped = be->group_cached(nt, 1, 16);
+    size_t work_ints = 0;
+    bool grouped = false;
+    int tiles = 0;   // 1: tiles of 16, 2: tiles of 128
+    SplitOut sp;
+    if (!exact && v.fmt == W_NVFP4 && n >= 128) {
+        tiles = n <= 1024 ? (itk::experts_f16s_takes(ev, nullptr, nt, dout) ? 1 : 0) : (itk::experts_f16_takes(ev, nullptr, nt, dout) ? 2 : 0);
+        if (tiles && !be->act_split(x, x_len, v.n_in, &sp)) return;
     }
-    const bool rows_dense = !skinny_dense && !exact && v.fmt == W_NVFP4 && n >= 128 && n <= 512 && itk::expert_rows_takes(rv, nullptr, aq);
-    if (!skinny_dense && !exact && v.fmt == W_NVFP4 && n > 512) {   // the 128-pair tiles (82 against 736 us at 5,700 tokens)
-        ev.q = v.q; ev.scales = v.scales; ev.q_stride = 0; ev.s_stride = 0;
-        ev.fmt = v.fmt; ev.n_in = v.n_in; ev.n_out = v.n_out; ev.n_expert = 1; ev.scale2 = nullptr; ev.counts = nullptr;
-        zids = be->zero_ids_for(n);
-        work = be->moe_work_for(n, 1, &work_ints);
-        fwork_bytes = itk::experts_f16_work_bytes(nt, v.n_in);
-        fwork = be->moe_f16_for(fwork_bytes);
-        one_expert = zids && work && fwork && itk::experts_f16_takes(ev, nullptr, nt, aq, dout);
-        if (one_expert) grouped = be->group_cached(nt, 1, 128);
-    }
+    const bool rows_dense = !tiles && !exact && v.fmt == W_NVFP4 && n >= 128 && n <= 512 && itk::expert_rows_takes(ev, nullptr, aq);
     // Exact mode: the int8 tiles of the expert products, which keep the GEMV's bits, from 64 tokens on (2,048 x 512 over 333
     // tokens: 20 us, 47 as a GEMV per token)
     bool int8_tiles = false;
     if (exact && v.fmt == W_NVFP4 && n >= 64) {
-        ev = rv;
         zids = be->zero_ids_for(n);
         work = be->moe_work_for(n, 1, &work_ints);
         int8_tiles = zids && work;
@@ -1583,19 +1583,18 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     }
     it_hip::OpRec rec;
     rec.id = OP_MATMUL; rec.p[0] = v.q; rec.p[1] = v.scales; rec.p[2] = dx; rec.p[3] = as; rec.p[4] = aq; rec.p[5] = dout;
-    rec.i[0] = v.fmt; rec.i[1] = v.n_in; rec.i[2] = v.n_out; rec.i[3] = nt;
+    rec.p[6] = sp.h; rec.p[7] = sp.l; rec.p[8] = sp.scale;
+    rec.i[0] = v.fmt; rec.i[1] = v.n_in; rec.i[2] = v.n_out; rec.i[3] = nt; rec.i[4] = tiles;
+    auto run = [=](hipStream_t s, float scale_by) {
+        if (tiles == 1 && experts_gemm_f16s(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
+        if (tiles == 2 && experts_gemm_f16(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
+        if (int8_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, grouped, s)) return;
+        if (rows_dense && expert_rows(ev, nullptr, nullptr, nt, 1, 0, as, aq, dout, scale_by, nullptr, 0, false, s)) return;
+        matmul(v, dx, as, aq, nt, dout, scale_by, exact, s);
+    };
+    if (n > 1 && !exact) rec.scaled = run;
     be->submit(it_hip::FAM_MATMUL, w->len + n * w->n_in + n * w->n_out * 4,
-               sig_of(OP_MATMUL, v.q, v.scales, v.fmt, v.n_in, v.n_out, dx, as, aq, nt, dout), rec,
-               [=](hipStream_t s) {
-                   if (skinny_dense && experts_gemm_f16s(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, fwork, fwork_bytes, grouped, s))
-                       return;
-                   if (int8_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, grouped, s)) return;
-                   if (rows_dense && expert_rows(rv, nullptr, nullptr, nt, 1, 0, as, aq, dout, 1.0f, nullptr, 0, false, s)) return;
-                   if (one_expert && experts_gemm_f16(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, fwork,
-                                                      fwork_bytes, grouped, s))
-                       return;
-                   matmul(v, dx, as, aq, nt, dout, 1.0f, exact, s);
-               });
+               sig_of(OP_MATMUL, v.q, v.scales, v.fmt, v.n_in, v.n_out, dx, as, aq, nt, dout), rec, [=](hipStream_t s) { run(s, 1.0f); });
 }
 
 void it_hip_matmul(it_hip* be, const it_weights* w, const float* x, uint64_t x_len, float* out,
@@ -1618,7 +1617,8 @@ void it_hip_matmul_pair(it_hip* be, const it_weights* a, const it_weights* b, co
         if (!dx || !da || !db) return;
         const int nt = (int)(x_len / a->n_in);
         it_hip::OpRec rec;
-        rec.id = OP_MATMUL;
+        rec.id = OP_MATMUL; rec.p[0] = va.q; rec.p[1] = vb.q; rec.p[2] = dx; rec.p[5] = da; rec.p[6] = db;
+        rec.i[0] = va.fmt; rec.i[1] = va.n_in; rec.i[2] = va.n_out; rec.i[3] = nt;
         be->submit(it_hip::FAM_MATMUL, a->len + b->len + x_len * 4 + (out_a_len + out_b_len) * 4,
                    sig_of(OP_MATMUL, va.q, vb.q, va.fmt, va.n_in, va.n_out, vb.n_out, dx, nt, da, db), rec,
                    [=](hipStream_t s) { float_matmul_pair(va, vb, dx, nt, da, db, be->exact, s); });
@@ -1683,8 +1683,9 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
     uint64_t group = a->n_head / a->n_head_kv;
     bool split_ok = (group == 1 || group == 2 || group == 4 || group == 8) && a->head_dim <= 256;
     bool graphed = be->mode != it_hip::Mode::Eager;
-    // a graphed pass keeps one launch shape while the context grows: size for the whole slab
-    uint64_t n_pos_cap = graphed ? a->kv_len / a->kv_dim : a->n_pos;
+    // a graphed pass keeps one launch shape while the context grows: size for the whole slab (any single-token pass, so that
+    // one issued op by op adds the splits up in the same order)
+    uint64_t n_pos_cap = graphed || n_q == 1 ? a->kv_len / a->kv_dim : a->n_pos;
     uint64_t bytes = a->n_pos * a->n_head_kv * a->head_dim * 4 + a->q_len * 8;
     if (be->exact || !split_ok) {
         float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap));
@@ -1969,16 +1970,13 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
     const bool rows_pay = !skinny_pay && expert_rows_pay(be, picks, w->n_expert);
     int32_t* work = skinny_pay || rows_pay || expert_tiles_pay(picks, w->n_expert) ? be->moe_work_for(picks, w->n_expert, &work_ints) : nullptr;
     const bool rows_shape = rows_pay && work && itk::expert_rows_takes(v, nullptr, aq);
-    void* fwork = nullptr;
-    size_t fwork_bytes = 0;
-    if (!be->exact && work && !rows_shape && v.fmt == itk::W_NVFP4) {
-        fwork_bytes = itk::experts_f16_work_bytes((int)rows, (int)w->n_in);
-        fwork = be->moe_f16_for(fwork_bytes);
-    }
-    const bool skinny_shape = skinny_pay && fwork && itk::experts_f16s_takes(v, nullptr, np, aq, dout);
+    const bool f16_pay = !be->exact && work && !rows_shape && v.fmt == itk::W_NVFP4;
+    const bool skinny_shape = skinny_pay && f16_pay && itk::experts_f16s_takes(v, nullptr, np, dout);
     // the tile size the launch below will group for: 8 or 16 pairs for the row kernel, 128 for the wide f16 kernel,
     // 16 for the skinny f16 kernel and the int8 one
-    const bool f16_shape = !skinny_shape && fwork && itk::experts_f16_takes(v, nullptr, np, aq, dout);
+    const bool f16_shape = !skinny_shape && f16_pay && itk::experts_f16_takes(v, nullptr, np, dout);
+    SplitOut sp;
+    if ((skinny_shape || f16_shape) && !be->act_split(x, x_len, (int)w->n_in, &sp)) return;
     const bool grouped = work && be->group_cached(np, (int)w->n_expert, rows_shape ? itk::expert_rows_tile(np, (int)w->n_expert, v.n_in) : f16_shape ? 128 : 16);
     it_hip::OpRec rec;
     rec.id = OP_EXPERTS; rec.p[0] = v.q; rec.p[1] = v.scales; rec.p[2] = v.scale2; rec.p[3] = ids; rec.p[4] = as; rec.p[5] = aq;
@@ -1989,12 +1987,11 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
     be->submit(it_hip::FAM_MOE_DOWN, picks * (w->len / w->n_expert) + x_len + out_len * 4,
                sig_of(OP_EXPERTS, v.q, v.scales, (const void*)v.q_tab, v.fmt, v.n_in, v.n_out, v.scale2, ids, np, nu, xm, as, aq, dout), rec,
                [=](hipStream_t s) {
+                   const TileCount tc{counts, nullptr, tally, v.tier, nullptr};
+                   if (skinny_shape && experts_gemm_f16s(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
+                   if (f16_shape && experts_gemm_f16(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
                    expert_count(ids, np, v.n_expert, counts, nullptr, tally, s, v.tier, nullptr);
-                   if (skinny_shape && experts_gemm_f16s(v, nullptr, ids, np, nu, xm, as, aq, dout, work, work_ints, fwork, fwork_bytes, grouped, s))
-                       return;
                    if (rows_shape && expert_rows(v, nullptr, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, grouped, s)) return;
-                   if (f16_shape && experts_gemm_f16(v, nullptr, ids, np, nu, xm, as, aq, dout, work, work_ints, fwork, fwork_bytes, grouped, s))
-                       return;
                    if (!experts_gemm(v, nullptr, ids, np, nu, xm, as, aq, dout, work, work_ints, grouped && !f16_shape, s))
                        matmul_experts(v, ids, np, nu, xm, as, aq, dout, s);
                });
@@ -2037,14 +2034,11 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
     const bool rows_pay = !skinny_pay && expert_rows_pay(be, picks, gate->n_expert);
     int32_t* work = skinny_pay || rows_pay || expert_tiles_pay(picks, gate->n_expert) ? be->moe_work_for(picks, gate->n_expert, &work_ints) : nullptr;
     const bool rows_shape = rows_pay && work && itk::expert_rows_takes(g, &u, aq);
-    void* fwork = nullptr;
-    size_t fwork_bytes = 0;
-    if (!be->exact && work && !rows_shape && g.fmt == itk::W_NVFP4) {
-        fwork_bytes = itk::experts_f16_work_bytes((int)rows, (int)gate->n_in);
-        fwork = be->moe_f16_for(fwork_bytes);
-    }
-    const bool skinny_shape = skinny_pay && fwork && itk::experts_f16s_takes(g, &u, np, aq, dout);
-    const bool f16_shape = !skinny_shape && fwork && itk::experts_f16_takes(g, &u, np, aq, dout);
+    const bool f16_pay = !be->exact && work && !rows_shape && g.fmt == itk::W_NVFP4;
+    const bool skinny_shape = skinny_pay && f16_pay && itk::experts_f16s_takes(g, &u, np, dout);
+    const bool f16_shape = !skinny_shape && f16_pay && itk::experts_f16_takes(g, &u, np, dout);
+    SplitOut sp;
+    if ((skinny_shape || f16_shape) && !be->act_split(x, x_len, (int)gate->n_in, &sp)) return;
     const bool grouped = work && be->group_cached(np, (int)gate->n_expert, rows_shape ? itk::expert_rows_tile(np, (int)gate->n_expert, g.n_in) : f16_shape ? 128 : 16);
     it_hip::OpRec rec;
     rec.id = OP_GLU; rec.p[0] = g.q; rec.p[1] = g.scales; rec.p[2] = u.q; rec.p[3] = u.scales; rec.p[4] = g.scale2;
@@ -2057,12 +2051,11 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
                sig_of(OP_GLU, g.q, g.scales, u.q, u.scales, (const void*)g.q_tab, (const void*)u.q_tab, g.fmt, g.n_in, g.n_out, g.scale2, u.scale2, ids, np, nu, xm,
                       as, aq, dout), rec,
                [=](hipStream_t s) {
+                   const TileCount tc{cg, cu, tally, g.tier, u.tier};
+                   if (skinny_shape && experts_gemm_f16s(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
+                   if (f16_shape && experts_gemm_f16(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
                    expert_count(ids, np, g.n_expert, cg, cu, tally, s, g.tier, u.tier);
-                   if (skinny_shape && experts_gemm_f16s(g, &u, ids, np, nu, xm, as, aq, dout, work, work_ints, fwork, fwork_bytes, grouped, s))
-                       return;
                    if (rows_shape && expert_rows(g, &u, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, grouped, s)) return;
-                   if (f16_shape && experts_gemm_f16(g, &u, ids, np, nu, xm, as, aq, dout, work, work_ints, fwork, fwork_bytes, grouped, s))
-                       return;
                    if (!experts_gemm(g, &u, ids, np, nu, xm, as, aq, dout, work, work_ints, grouped && !f16_shape, s))
                        moe_glu(g, u, ids, np, nu, xm, as, aq, dout, s);
                });
@@ -2195,7 +2188,7 @@ void it_hip_host_wrote(it_hip* be, const float* buf, uint64_t len) {
     auto it = be->acts.find(buf);
     if (it != be->acts.end()) {
         it->second.dev_current = false;
-        it->second.q_valid = false;
+        it->second.stale();
     }
 }
 
@@ -2255,7 +2248,7 @@ void it_hip_begin_pass(it_hip* be, uint64_t n_tokens) {
     for (auto& kv : be->acts) {
         kv.second.dev_current = false;
         kv.second.elided = false;
-        kv.second.q_valid = false;
+        kv.second.stale();
     }
 }
 
@@ -2283,6 +2276,7 @@ void it_hip_forget_state(it_hip* be) {
 
 void it_hip_zero_state(it_hip* be) {
     // the host copies were just zeroed: zero the device copies in place instead of uploading zeros at the next use
+    if (!be->held.empty()) be->release_held();
     std::vector<itk::ZeroSpan> spans;
     for (auto& kv : be->slabs) {
         if (!kv.second.is_state) continue;
@@ -2688,6 +2682,8 @@ void it_hip_release(it_hip* be, const void* host) {
     if (a != be->acts.end()) {
         be->mirror_bytes -= a->second.cap * sizeof(float);
         if (a->second.q_scales) be->quant_bytes -= a->second.q_cap / 32 * 4 + a->second.q_cap;
+        if (a->second.split.h) be->quant_bytes -= a->second.s_cap * 4 + a->second.s_cap / 32 * 4;
+        if (a->second.split.h) (void)hipFree(a->second.split.h);
         if (a->second.dev) (void)hipFree(a->second.dev);
         if (a->second.q_scales) (void)hipFree(a->second.q_scales);
         if (a->second.q_quants) (void)hipFree(a->second.q_quants);

@@ -43,7 +43,7 @@
 enum OpId : int {
     OP_RMS = 1, OP_RMS_HEADS, OP_L2, OP_MATMUL, OP_ROPE, OP_SOFTMAX, OP_ATTEND, OP_EW, OP_SCALE, OP_CONV, OP_GATHER,
     OP_SCATTER, OP_DELTA, OP_ROUTE, OP_EXPERTS, OP_GLU, OP_FINISH, OP_ROWS, OP_SIGADD, OP_KVWRITE, OP_EMBED,
-    OP_QUANT = 101
+    OP_QUANT = 101, OP_SPLIT = 102
 };
 
 struct it_hip {
@@ -71,6 +71,12 @@ struct it_hip {
         size_t q_cap = 0;  // floats covered
         size_t q_len = 0;
         bool q_valid = false;
+        // the split form (f16 hi / lo, the rows' powers of two) of the Q8_0 form, for rows of s_row floats
+        itk::SplitOut split;
+        size_t s_cap = 0, s_len = 0;
+        int s_row = 0;
+        bool s_valid = false;
+        void stale() { q_valid = s_valid = false; }
         int host_locked = -1;  // the host buffer is page-locked (fetch): not asked yet, no, yes
     };
     struct Home {
@@ -88,6 +94,8 @@ struct it_hip {
     float* act_inout(const float* host, size_t len);  // read then written in place
     bool act_quantized(const float* host, size_t len, const float** scales, const int8_t** quants,
                        float** dev_x);
+    // the split form of a batch's rows of `row` floats (made from the Q8_0 form, which it makes too)
+    bool act_split(const float* host, size_t len, int row, itk::SplitOut* out);
     bool act_q_reserve(Act& a, size_t len);  // room for the Q8_0 form of `len` floats
     Act* act_by_dev(const void* dev);        // the mirror whose device buffer holds `dev`, or null
     bool held_touches(const void* dev, size_t bytes) const;   // an op held back reads or writes inside [dev, dev + bytes)
@@ -181,12 +189,9 @@ struct it_hip {
     int32_t* moe_work = nullptr;
     size_t moe_work_ints = 0;
     int32_t* moe_work_for(size_t picks, size_t n_expert, size_t* ints);
-    void* moe_f16 = nullptr;     // f16 hi / lo copies of the expert GEMM's activations
     int32_t* zero_ids = nullptr;  // expert id 0 for every token: a dense NVFP4 matrix run as a one-expert batch
     size_t zero_ids_n = 0;
     const int32_t* zero_ids_for(size_t n);
-    size_t moe_f16_bytes = 0;
-    void* moe_f16_for(size_t bytes);
     float* gdn_work = nullptr;   // T and P matrices of the chunked delta rule
     size_t gdn_work_floats = 0;
     float* gdn_work_for(size_t floats);
@@ -282,6 +287,7 @@ struct it_hip {
         int64_t i[10] = {};
         float f[2] = {};
         std::function<void(hipStream_t)> run;
+        std::function<void(hipStream_t, float)> scaled;   // a product with a factor on its results, where one can be applied
     };
     std::vector<OpRec> pending;
     bool fuse_enabled = true;
@@ -319,11 +325,12 @@ struct it_hip {
         const void* host;
         size_t bytes;
     };
-    // ops of a batch pass held back because they begin a run that has a one-kernel form (fuser.cpp)
+    // ops of a batch pass held back because they may belong to a run that has a one-kernel form (fuser.cpp)
     std::vector<OpRec> held;
-    int hold_step(const OpRec& rec) const;   // 0: not part of a run, 1: continues it, 2: completes it
-    void release_held();                     // the run broke off: issue what is held op by op, in order
-    void finish_held();                      // the run is complete: one kernel (or op by op when its shape is not taken)
+    bool hold(const OpRec& rec);             // whether the op waits (what is held may be issued first)
+    void release_held();                     // issue what is held op by op, in order
+    void flush_held(const OpRec* next);      // issue what is held, its known runs as one launch each; next: the op that follows, or null
+    size_t fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next);   // ops of the run issued from h[i] on, 0: none begins there
     bool small_ffn(const std::vector<OpRec>& run);   // the routed FFN of a short batch as two launches
     bool small_ffn_enabled = true;           // INFERRED_HIP_NO_SMALL_FFN=1 issues it op by op (a measurement switch)
     std::vector<PreCopy> precopies;  // host -> device inputs of a graphed pass, issued before the graph
@@ -375,19 +382,13 @@ struct it_hip {
         if (mode == Mode::Eager) {
             if (in_pass && pass_tokens == 1) pass_signature.push_back(sig);
             if (in_pass && pass_tokens > 1 && !exact && fuse_enabled) {
-                // a batch pass in fast mode holds back the ops of two known elementwise runs and issues each run as
-                // one kernel once it is complete (hold_step, fuser.cpp); anything else releases what is held first
-                int st = hold_step(rec);
-                if (!st && !held.empty()) {
-                    release_held();
-                    st = hold_step(rec);
-                }
-                if (st) {
+                // a batch pass in fast mode holds the row-wise ops between two products back and issues the known runs
+                // among them as one kernel each (fuser.cpp)
+                if (hold(rec)) {
                     rec.run = f;
                     rec.fam = fam;
                     rec.bytes = bytes;
                     held.push_back(std::move(rec));
-                    if (st == 2) finish_held();
                     return;
                 }
             } else if (!held.empty()) {

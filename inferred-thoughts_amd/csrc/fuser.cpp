@@ -947,88 +947,102 @@ bool references(const Op& op, const void* a, const void* b) {
 }  // namespace
 
 // ---------------------------------------------------------------------------------- batch passes
-// Two runs of elementwise ops of a Gated DeltaNet layer over a batch (src/model/qwen35.rs:1255-1315) have a one-kernel
-// form in fast mode:
+// Between two products of a batch pass stand short row-wise ops.  In fast mode they are held back as they arrive, until an op
+// comes that is none of them (a product, attention, the delta rule, the pass's end); then the runs among them that have a
+// one-kernel form are issued as that kernel, the rest op by op, in order (flush_held).  The known runs:
+//   [FINISH,] EW x += y [, RMS x [, GATHER: a copy of the normed rows [, QUANT of it]]]      -> residual_row
+//   [EW silu / sigmoid mul,] QUANT [, SPLIT]                                                 -> mul_forms
+//   SOFTMAX, ROUTE                                                                           -> softmax_route
+//   GATHER q, GATHER gate, RMS_HEADS q, k, ROPE q, k, KVWRITE k, v                           -> attn_rows
 //   CONV, GATHER q, GATHER k, GATHER v, L2 q, L2 k      -> conv_split_l2 (the conv output and the unnormed q, k are
 //                                                          not written: nothing else in the loop reads them)
 //   RMS_HEADS core, EW silu_mul(z, core), QUANT z        -> gated_norm_silu_q8 (core is left unnormed)
-// The ops are held back as they arrive and checked link by link (an op's input must be the run's own buffer).
-// The routed FFN of a short batch (2..32 tokens; src/model/qwen35.rs:1630-1700) as a run:
+//   MATMUL, SCALE of its result                          -> the product with the factor in its epilogue
+//   MATMUL gate, MATMUL up, [SCALE up,] [SCALE gate,] EW silu_mul(gate, up), both NVFP4   -> one gate / up product
+// and the routed FFN of a short batch (2..32 tokens; src/model/qwen35.rs:1630-1700), whose products are held back too:
 //   SOFTMAX, ROUTE, [QUANT x], GLU, QUANT g, EXPERTS, MATMUL shared gate, MATMUL shared up, [SCALE]*, EW silu_mul,
-//   QUANT, MATMUL shared down, [SCALE], FINISH
-// Where the run stands follows from what is held; an op is accepted by its kind here, and the links between the ops
-// (whose output feeds whom, the shapes) are checked once the run is complete: a run that fails there is issued op by op.
+//   QUANT, MATMUL shared down, [SCALE], FINISH                                               -> small_ffn
+// Every link (whose output feeds whom, the shapes) is checked; a buffer that a run does not write is marked, and the run is
+// only taken if no op behind it reads that buffer.
 namespace {
 constexpr int SMALL_FFN_MAX = 32;   // tokens (measured on the 512-expert top-10 layer: 176 against 232 us at 32, 271 against 298 at 48, behind from about 56 on)
-enum FfnAt { F_ROUTE = 1, F_QX_OR_GLU, F_GLU, F_QG, F_EXPERTS, F_SG, F_SU, F_SCALE_OR_SILU, F_QS, F_SD, F_SCALE_OR_FINISH, F_FINISH };
-int ffn_at(const std::vector<it_hip::OpRec>& held) {   // what may come next
-    int at = F_ROUTE;
-    for (size_t k = 1; k < held.size(); k++) {
-        const int id = held[k].id;
-        switch (at) {
-            case F_ROUTE: at = F_QX_OR_GLU; break;
-            case F_QX_OR_GLU: at = id == OP_QUANT ? F_GLU : F_QG; break;
-            case F_GLU: at = F_QG; break;
-            case F_QG: at = F_EXPERTS; break;
-            case F_EXPERTS: at = F_SG; break;
-            case F_SG: at = F_SU; break;
-            case F_SU: at = F_SCALE_OR_SILU; break;
-            case F_SCALE_OR_SILU: at = id == OP_SCALE ? F_SCALE_OR_SILU : F_QS; break;
-            case F_QS: at = F_SD; break;
-            case F_SD: at = F_SCALE_OR_FINISH; break;
-            case F_SCALE_OR_FINISH: at = F_FINISH; break;
-            default: break;
-        }
+constexpr size_t HELD_MAX = 48;
+
+bool row_wise(int id) {
+    switch (id) {
+        case OP_RMS: case OP_RMS_HEADS: case OP_L2: case OP_ROPE: case OP_SOFTMAX: case OP_ROUTE: case OP_EW: case OP_SCALE:
+        case OP_CONV: case OP_GATHER: case OP_FINISH: case OP_KVWRITE: case OP_QUANT: case OP_SPLIT: return true;
+        default: return false;
     }
-    return at;
+}
+bool reads_or_writes(const it_hip::OpRec& r, const void* dev) {
+    if (!dev) return false;
+    for (const void* p : r.p)
+        if (p == dev) return true;
+    return false;
+}
+// some op of h[from..], or the op behind them, has to do with the buffer
+bool used_later(const std::vector<it_hip::OpRec>& h, size_t from, const it_hip::OpRec* next, const void* dev) {
+    for (size_t k = from; k < h.size(); k++)
+        if (reads_or_writes(h[k], dev)) return true;
+    return next && reads_or_writes(*next, dev);
+}
+// ... other than making the forms of it
+bool changed_later(const std::vector<it_hip::OpRec>& h, size_t from, const void* dev) {
+    for (size_t k = from; k < h.size(); k++)
+        if (h[k].id != OP_QUANT && h[k].id != OP_SPLIT && reads_or_writes(h[k], dev)) return true;
+    return false;
+}
+// the small FFN's products, while its run is being held: which may come next
+bool small_ffn_next(const std::vector<it_hip::OpRec>& held, const it_hip::OpRec& r) {
+    if (held.empty() || held[0].id != OP_SOFTMAX || r.i[8]) return false;
+    const it_hip::OpRec& h0 = held[0];
+    if (h0.i[0] < 2 || h0.i[0] > SMALL_FFN_MAX || h0.i[1] < 16 || h0.i[1] > 2048) return false;
+    if (held.size() < 2 || held[1].id != OP_ROUTE || held[1].p[0] != h0.p[0] || held[1].i[2] > 16) return false;
+    int glu = 0, experts = 0, mats = 0, finish = 0;
+    for (const auto& o : held) {
+        glu += o.id == OP_GLU;
+        experts += o.id == OP_EXPERTS;
+        mats += o.id == OP_MATMUL;
+        finish += o.id == OP_FINISH;
+    }
+    if (finish) return false;
+    if (r.id == OP_GLU) return !glu && !mats;
+    if (r.id == OP_EXPERTS) return glu && !experts && !mats;
+    return r.id == OP_MATMUL && experts && mats < 3;
 }
 }  // namespace
 
-int it_hip::hold_step(const OpRec& r) const {
-    const size_t n = held.size();
-    if (n == 0) {
-        if (r.id == OP_CONV && r.i[2] >= 64 && r.i[1] % 128 == 0) return 1;
-        if (r.id == OP_RMS_HEADS && r.i[0] == 128 && r.i[1] >= 256) return 1;
-        if (r.id == OP_SOFTMAX && r.i[0] >= 2 && r.i[0] <= SMALL_FFN_MAX && r.i[1] >= 16 && r.i[1] <= 2048 && !expert_cold_entries && small_ffn_enabled) return 1;
-        return 0;
+bool it_hip::hold(const OpRec& r) {
+    if (row_wise(r.id)) {
+        if (held.size() >= HELD_MAX) flush_held(&r);
+        return true;
     }
-    const OpRec& h0 = held[0];
-    if (h0.id == OP_SOFTMAX) {
-        switch (ffn_at(held)) {
-            case F_ROUTE: return r.id == OP_ROUTE && r.p[0] == h0.p[0] && r.i[0] == h0.i[0] && r.i[1] == h0.i[1] && r.i[2] <= 16 ? 1 : 0;
-            case F_QX_OR_GLU: return r.id == OP_QUANT || (r.id == OP_GLU && !r.i[8]) ? 1 : 0;
-            case F_GLU: return r.id == OP_GLU && !r.i[8] ? 1 : 0;
-            case F_QG: return r.id == OP_QUANT ? 1 : 0;
-            case F_EXPERTS: return r.id == OP_EXPERTS && !r.i[8] ? 1 : 0;
-            case F_SG:
-            case F_SU:
-            case F_SD: return r.id == OP_MATMUL ? 1 : 0;
-            case F_SCALE_OR_SILU: return r.id == OP_SCALE || (r.id == OP_EW && r.i[0] == 0) ? 1 : 0;
-            case F_QS: return r.id == OP_QUANT ? 1 : 0;
-            case F_SCALE_OR_FINISH: return r.id == OP_SCALE ? 1 : r.id == OP_FINISH ? 2 : 0;
-            case F_FINISH: return r.id == OP_FINISH ? 2 : 0;
+    if (held.size() < HELD_MAX) {
+        if (small_ffn_enabled && !expert_cold_entries && small_ffn_next(held, r)) return true;
+        if (r.id == OP_MATMUL && r.i[4]) {   // a dense matrix on the expert tiles: the shared expert's
+            // (behind ops that are not its own it would keep the device waiting for them)
+            for (const OpRec& h : held)
+                if (h.id != OP_MATMUL && h.id != OP_SCALE && h.id != OP_EW && h.id != OP_QUANT && h.id != OP_SPLIT) {
+                    flush_held(&r);
+                    break;
+                }
+            return true;
         }
-        return 0;
     }
-    if (h0.id == OP_CONV) {
-        const int64_t nc = h0.i[1], nt = h0.i[2];
-        if (n <= 3) {
-            if (r.id != OP_GATHER || r.p[0] != h0.p[3] || r.i[1] != nc) return 0;
-            const int64_t kdim = n == 1 ? r.i[0] : held[1].i[0];
-            if (kdim <= 0 || kdim % 128 || 2 * kdim >= nc) return 0;
-            const int64_t chunk = n == 3 ? nc - 2 * kdim : kdim, off = (int64_t)(n - 1) * kdim;
-            return r.i[0] == chunk && r.i[2] == off && r.i[3] == nt * chunk ? 1 : 0;
+    if (held.empty()) return false;
+    // a product that has nothing to do with what is held goes ahead of it (the key and value projections, behind the
+    // split of the query projection's rows)
+    if (r.id == OP_MATMUL) {
+        bool apart = true;
+        for (const OpRec& h : held) {
+            apart &= h.id == OP_GATHER;
+            for (const void* p : h.p) apart &= !p || (p != r.p[5] && p != r.p[6] && (p != r.p[2] || p == h.p[0]));
         }
-        const OpRec& g = held[n - 3];   // n = 4: the q part, n = 5: the k part
-        if (r.id != OP_L2 || r.p[0] != g.p[1] || r.i[0] != 128 || r.i[1] * 128 != nt * held[1].i[0]) return 0;
-        if (n == 5 && r.f[0] != held[4].f[0]) return 0;
-        return n == 5 ? 2 : 1;
+        if (apart) return false;
     }
-    if (h0.id == OP_RMS_HEADS) {
-        if (n == 1) return r.id == OP_EW && r.i[0] == 0 && r.p[1] == h0.p[0] && r.i[1] == h0.i[1] * 128 ? 1 : 0;
-        if (n == 2) return r.id == OP_QUANT && r.p[0] == held[1].p[0] && r.i[0] == held[1].i[1] ? 2 : 0;
-    }
-    return 0;
+    flush_held(&r);
+    return false;
 }
 
 void it_hip::release_held() {
@@ -1044,7 +1058,10 @@ void it_hip::release_held() {
 // The complete FFN run of a short batch as two launches: gate / up with the route inside (every block ranks its
 // token's logits; grid row = token), then down + combine.  False, with nothing launched, when a link or a shape is not
 // what the kernels take.
-bool it_hip::small_ffn(const std::vector<OpRec>& h) {
+bool it_hip::small_ffn(const std::vector<OpRec>& run) {
+    std::vector<OpRec> h;   // (the split forms are made for kernels that this run does not use)
+    for (const OpRec& o : run)
+        if (o.id != OP_SPLIT) h.push_back(o);
     size_t k = 0;
     auto take = [&](int id) -> const OpRec* { return k < h.size() && h[k].id == id ? &h[k++] : nullptr; };
     const OpRec *sm = take(OP_SOFTMAX), *rt = take(OP_ROUTE), *q1 = take(OP_QUANT), *glu = take(OP_GLU), *q2 = take(OP_QUANT);
@@ -1135,6 +1152,9 @@ bool it_hip::small_ffn(const std::vector<OpRec>& h) {
         d.tally = expert_tally;
     }
     if (!moe_glu_fast(g, stream, true) || !moe_down_fast(d, stream, true)) return false;
+    uint64_t bytes = 0;
+    for (const OpRec& o : run) bytes += o.bytes;
+    Span sp(this, FAM_MOE_GLU, bytes);
     moe_glu_fast(g, stream);
     moe_down_fast(d, stream);
     // what the two launches do not write: the probabilities (the router buffer keeps its logits), the shared expert's
@@ -1142,48 +1162,239 @@ bool it_hip::small_ffn(const std::vector<OpRec>& h) {
     mark_elided({router, sum_->p[5], ex->p[6], sdm->p[5]});
     for (const OpRec* q : {q1, q2, q3})
         if (q)
-            if (Act* a = act_by_dev(q->p[0])) a->q_valid = false;
+            if (Act* a = act_by_dev(q->p[0])) a->stale();
     return true;
 }
 
-void it_hip::finish_held() {
-    bool done = false;
-    uint64_t bytes = 0;
-    for (auto& op : held) bytes += op.bytes;
-    if (held[0].id == OP_SOFTMAX) {
-        {
-            Span sp(this, FAM_MOE_GLU, bytes);
-            done = small_ffn(held);
+void it_hip::flush_held(const OpRec* next) {
+    const auto ops = std::move(held);
+    held.clear();
+    for (size_t i = 0; i < ops.size();) {
+        const size_t k = fuse_at(ops, i, next);
+        if (!k) {
+            Span sp(this, ops[i].fam, ops[i].bytes);
+            ops[i].run(stream);
         }
-        if (done) {
-            held.clear();
-            check(hipGetLastError(), "kernel launch");
-        } else {
-            release_held();
-        }
-        return;
+        i += k ? k : 1;
     }
+    check(hipGetLastError(), "kernel launch");
+}
+
+size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next) {
+    const size_t n = h.size();
+    auto id = [&](size_t k) { return k < n ? h[k].id : 0; };
+    auto span_of = [&](size_t len) {
+        uint64_t bytes = 0;
+        for (size_t k = i; k < i + len; k++) bytes += h[k].bytes;
+        return bytes;
+    };
+    const OpRec& a = h[i];
+    if (a.id == OP_SOFTMAX && id(i + 1) == OP_ROUTE) {
+        if (a.i[0] >= 2 && a.i[0] <= SMALL_FFN_MAX && i == 0 && small_ffn_enabled && !expert_cold_entries) {
+            size_t end = i;
+            while (end < n && h[end].id != OP_FINISH) end++;
+            if (end < n) {
+                if (small_ffn(std::vector<OpRec>(h.begin() + i, h.begin() + end + 1))) return end + 1 - i;
+            }
+        }
+        const OpRec& r = h[i + 1];
+        if (r.p[0] == a.p[0] && r.i[0] == a.i[0] && r.i[1] == a.i[1]) {
+            Span sp(this, a.fam, span_of(2));
+            if (softmax_route((float*)a.p[0], (int)a.i[0], (int)a.i[1], (int)r.i[2], (int32_t*)r.p[1], (float*)r.p[2], stream)) return 2;
+        }
+        return 0;
+    }
+    // ---- the residual row
     {
-        Span sp(this, held[0].fam, bytes);
-        if (held[0].id == OP_CONV && held.size() == 6) {
-            const OpRec &c = held[0], &gq = held[1], &gk = held[2], &gv = held[3], &l = held[4];
-            done = conv_split_l2((float*)c.p[0], (const float*)c.p[1], (const float*)c.p[2], (int)c.i[0], (int)c.i[1], (int)c.i[2],
-                                 (float*)gq.p[1], (float*)gk.p[1], (float*)gv.p[1], (int)gq.i[0], l.f[0], stream);
-        } else if (held[0].id == OP_RMS_HEADS && held.size() == 3) {
-            const OpRec &n = held[0], &e = held[1], &q = held[2];
-            done = gated_norm_silu_q8((const float*)n.p[0], (const float*)n.p[1], (float*)e.p[0], (float*)q.p[1], (int8_t*)q.p[2],
-                                      n.i[1], n.f[0], stream);
+        const bool fin = a.id == OP_FINISH && a.i[0] == 0;
+        const size_t k = i + fin;
+        if (id(k) == OP_EW && h[k].i[0] == 2) {
+            const OpRec& e = h[k];
+            size_t len = k + 1 - i;
+            ResidualP p{};
+            p.x = (float*)e.p[0];
+            p.y = (float*)e.p[1];
+            bool ok = p.x != p.y;
+            int64_t rows = 0, width = 0;
+            if (fin) {
+                rows = a.i[2];
+                width = a.i[1];
+                p.rows = (const float*)a.p[1]; p.rw = (const float*)a.p[2]; p.shared = (const float*)a.p[3];
+                p.logit = (const float*)a.p[4] + a.i[4];
+                p.n_used = (int)a.i[3];
+                ok &= a.p[0] == e.p[1] && a.p[0] != e.p[0];
+            }
+            Act *out_act = nullptr, *copy_act = nullptr;
+            if (ok && id(k + 1) == OP_RMS && h[k + 1].p[0] == p.x && h[k + 1].p[2] != p.x && h[k + 1].p[2] != p.y &&
+                (!fin || (h[k + 1].i[0] == rows && h[k + 1].i[1] == width))) {
+                const OpRec& m = h[k + 1];
+                rows = m.i[0];
+                width = m.i[1];
+                len++;
+                p.w = (const float*)m.p[1]; p.eps = m.f[0]; p.out = (float*)m.p[2];
+                const int64_t all = rows * width;
+                if (id(k + 2) == OP_GATHER && h[k + 2].p[0] == m.p[2] && h[k + 2].i[2] == 0 && h[k + 2].i[0] == all && h[k + 2].i[3] == all &&
+                    h[k + 2].p[1] != p.x && h[k + 2].p[1] != p.y) {
+                    // the copy is what the products read: its forms are made instead of the normed rows'
+                    p.copy = (float*)h[k + 2].p[1];
+                    len++;
+                    const OpRec* q = id(k + 3) == OP_QUANT && h[k + 3].p[0] == p.copy && h[k + 3].i[0] == all ? &h[k + 3] : nullptr;
+                    if (q) len++;
+                    copy_act = changed_later(h, i + len, p.copy) ? nullptr : act_by_dev(p.copy);
+                    if (q) {
+                        p.q.scales = (float*)q->p[1]; p.q.quants = (int8_t*)q->p[2];
+                    } else if (m.p[3] && copy_act && copy_act->cap >= (size_t)all && act_q_reserve(*copy_act, (size_t)all)) {
+                        p.q.scales = copy_act->q_scales; p.q.quants = copy_act->q_quants;
+                    }
+                    if (p.q.quants && m.p[3]) {
+                        if (Act* o = act_by_dev(p.out)) o->stale();
+                    } else if (m.p[3]) {
+                        ok = false;
+                    }
+                } else if (m.p[3]) {
+                    p.q.scales = (float*)m.p[3]; p.q.quants = (int8_t*)m.p[4];
+                    out_act = changed_later(h, i + len, p.out) ? nullptr : act_by_dev(p.out);
+                }
+            }
+            if (!width) {
+                width = 1024;
+                while (width > 32 && e.i[1] % width) width >>= 1;
+                rows = e.i[1] / width;
+            }
+            Act* formed = copy_act ? copy_act : out_act;
+            // the split form too, once something has asked for it for rows of this length
+            if (p.q.quants && formed && formed->s_row == (int)width && formed->s_cap >= (size_t)(rows * width)) p.q.split = formed->split;
+            p.n_tok = (int)std::min<int64_t>(rows, INT32_MAX);
+            p.n = (int)std::min<int64_t>(width, INT32_MAX);
+            ok &= rows * width == e.i[1] && (fin || p.w);   // (x += y alone has its kernel)
+            if (ok) {
+                Span sp(this, a.fam, span_of(len));
+                if (residual_row(p, stream)) {
+                    if (formed && p.q.quants && copy_act) {
+                        copy_act->q_valid = true;
+                        copy_act->q_len = rows * width;
+                    }
+                    if (formed && p.q.split.h) {
+                        formed->s_valid = true;
+                        formed->s_len = rows * width;
+                    }
+                    return len;
+                }
+            }
+            return 0;
         }
     }
-    if (done) {
-        // the conv output (first run) and the normed read-out (second run: `core` keeps the delta rule's raw values) are
-        // not what their ops would have left there
-        mark_elided({held[0].id == OP_CONV ? held[0].p[3] : held[0].p[0]});
-        held.clear();
-        check(hipGetLastError(), "kernel launch");
-    } else {
-        release_held();
+    // ---- the forms of a row, behind the op that makes it
+    {
+        const bool ew = a.id == OP_EW && (a.i[0] == 0 || a.i[0] == 1);
+        const size_t k = i + ew;
+        if (id(k) == OP_QUANT && (!ew || (h[k].p[0] == a.p[0] && h[k].i[0] == a.i[1]))) {
+            const OpRec& q = h[k];
+            const bool split = id(k + 1) == OP_SPLIT && h[k + 1].p[0] == q.p[2] && h[k + 1].i[0] == q.i[0];
+            if (ew || split) {
+                QuantOut o;
+                o.scales = (float*)q.p[1]; o.quants = (int8_t*)q.p[2];
+                int64_t row = 1024;
+                if (split) {
+                    o.split.h = (uint16_t*)h[k + 1].p[2]; o.split.l = (uint16_t*)h[k + 1].p[3]; o.split.scale = (float*)h[k + 1].p[4];
+                    row = h[k + 1].i[1];
+                } else {
+                    while (row > 32 && q.i[0] % row) row >>= 1;
+                }
+                const size_t len = (ew ? 2 : 1) + split;
+                Span sp(this, a.fam, span_of(len));
+                if (q.i[0] % row == 0 && mul_forms((float*)q.p[0], ew ? (const float*)a.p[1] : nullptr, ew ? 1 + (int)a.i[0] : 0, q.i[0] / row, (int)row, o, stream))
+                    return len;
+            }
+            return 0;
+        }
     }
+    if (a.id == OP_CONV) {
+        const int64_t nc = a.i[1], nt = a.i[2];
+        if (nt < a.i[0] || nc % 128 || i + 6 > n || used_later(h, i + 6, next, a.p[3])) return 0;
+        const int64_t kdim = h[i + 1].i[0];
+        if (kdim <= 0 || kdim % 128 || 2 * kdim >= nc) return 0;
+        for (size_t k = 1; k <= 3; k++) {
+            const OpRec& g = h[i + k];
+            const int64_t chunk = k == 3 ? nc - 2 * kdim : kdim;
+            if (g.id != OP_GATHER || g.p[0] != a.p[3] || g.i[1] != nc || g.i[0] != chunk || g.i[2] != (int64_t)(k - 1) * kdim || g.i[3] != nt * chunk) return 0;
+        }
+        for (size_t k = 4; k <= 5; k++) {
+            const OpRec& l = h[i + k];
+            if (l.id != OP_L2 || l.p[0] != h[i + k - 3].p[1] || l.i[0] != 128 || l.i[1] * 128 != nt * kdim || l.f[0] != h[i + 4].f[0]) return 0;
+        }
+        Span sp(this, a.fam, span_of(6));
+        if (!conv_split_l2((float*)a.p[0], (const float*)a.p[1], (const float*)a.p[2], (int)a.i[0], (int)nc, (int)nt, (float*)h[i + 1].p[1],
+                           (float*)h[i + 2].p[1], (float*)h[i + 3].p[1], (int)kdim, h[i + 4].f[0], stream))
+            return 0;
+        mark_elided({a.p[3]});
+        return 6;
+    }
+    if (a.id == OP_RMS_HEADS && a.i[0] == 128 && id(i + 1) == OP_EW && h[i + 1].i[0] == 0 && h[i + 1].p[1] == a.p[0] && h[i + 1].p[0] != a.p[0] &&
+        h[i + 1].i[1] == a.i[1] * 128 && id(i + 2) == OP_QUANT && h[i + 2].p[0] == h[i + 1].p[0] && h[i + 2].i[0] == h[i + 1].i[1] &&
+        !used_later(h, i + 3, next, a.p[0])) {
+        const OpRec &e = h[i + 1], &q = h[i + 2];
+        Span sp(this, a.fam, span_of(3));
+        if (!gated_norm_silu_q8((const float*)a.p[0], (const float*)a.p[1], (float*)e.p[0], (float*)q.p[1], (int8_t*)q.p[2], a.i[1], a.f[0], stream))
+            return 0;
+        mark_elided({a.p[0]});   // (it keeps the delta rule's raw values)
+        return 3;
+    }
+    // ---- attention's rows
+    if (a.id == OP_GATHER && i + 8 <= n && id(i + 1) == OP_GATHER && id(i + 2) == OP_RMS_HEADS && id(i + 3) == OP_RMS_HEADS && id(i + 4) == OP_ROPE &&
+        id(i + 5) == OP_ROPE && id(i + 6) == OP_KVWRITE && id(i + 7) == OP_KVWRITE) {
+        const OpRec &g = h[i + 1], &nq = h[i + 2], &nk = h[i + 3], &rq = h[i + 4], &rk = h[i + 5], &wk = h[i + 6], &wv = h[i + 7];
+        const int64_t hd = a.i[0], qn = a.i[3], kn = wk.i[2], nt = rq.i[1];
+        const int64_t nh = rq.i[4], nkv = rk.i[4];
+        const bool ok = hd == nq.i[0] && hd == nk.i[0] && a.i[1] == 2 * hd && a.i[2] == 0 && g.p[0] == a.p[0] && g.i[0] == hd && g.i[1] == 2 * hd &&
+                        g.i[2] == hd && g.i[3] == qn && nq.p[0] == a.p[1] && nq.i[1] * hd == qn && rq.p[0] == a.p[1] && rk.p[0] == nk.p[0] &&
+                        nk.i[1] * hd == kn && rk.i[1] == nt && rq.i[0] == rk.i[0] && rq.p[1] == rk.p[1] && rq.i[2] == hd && rk.i[2] == hd &&
+                        rq.i[5] == rk.i[5] && !rq.p[2] && !rk.p[2] && nt * nh * hd == qn && nt * nkv * hd == kn && wk.p[2] == nk.p[0] && wv.i[2] == kn &&
+                        wv.p[2] != nk.p[0] && !wk.p[1] && !wv.p[1] && g.p[1] != a.p[1] && wk.p[0] != wv.p[0];
+        if (!ok) return 0;
+        AttnRowsP p{};
+        p.qg = (const float*)a.p[0]; p.v = (const float*)wv.p[2]; p.q_w = (const float*)nq.p[1]; p.k_w = (const float*)nk.p[1];
+        p.q = (float*)a.p[1]; p.g = (float*)g.p[1]; p.k = (float*)nk.p[0];
+        p.k_slab = (uint16_t*)wk.p[0]; p.v_slab = (uint16_t*)wv.p[0]; p.k_at = wk.i[1]; p.v_at = wv.i[1];
+        p.table = (const float2*)rq.p[1];
+        p.n_tok = (int)nt; p.n_head = (int)nh; p.n_kv = (int)nkv; p.half = (int)rq.i[0]; p.pos = (int)rq.i[5];
+        p.q_eps = nq.f[0]; p.k_eps = nk.f[0];
+        Span sp(this, FAM_ATTN_PREP, span_of(8));
+        return attn_rows(p, (int)hd, stream) ? 8 : 0;
+    }
+    // ---- dense products held back
+    if (a.id == OP_MATMUL && a.i[4] && id(i + 1) == OP_MATMUL && h[i + 1].i[4] == a.i[4]) {
+        const OpRec& u = h[i + 1];
+        size_t k = i + 2;
+        float su = 1.0f, sg = 1.0f;
+        if (id(k) == OP_SCALE && h[k].p[0] == u.p[5] && h[k].i[0] == u.i[2] * u.i[3]) su = h[k++].f[0];
+        if (id(k) == OP_SCALE && h[k].p[0] == a.p[5] && h[k].i[0] == a.i[2] * a.i[3]) sg = h[k++].f[0];
+        if (id(k) == OP_EW && h[k].i[0] == 0 && h[k].p[0] == a.p[5] && h[k].p[1] == u.p[5] && h[k].i[1] == a.i[2] * a.i[3] && a.p[5] != u.p[5] &&
+            u.p[6] == a.p[6] && u.i[0] == a.i[0] && u.i[1] == a.i[1] && u.i[2] == a.i[2] && u.i[3] == a.i[3] && !used_later(h, k + 1, next, u.p[5])) {
+            auto view = [](const OpRec& m) {
+                ExpertsView v{};
+                v.q = m.p[0]; v.scales = m.p[1]; v.fmt = (int)m.i[0]; v.n_in = (int)m.i[1]; v.n_out = (int)m.i[2]; v.n_expert = 1;
+                return v;
+            };
+            const ExpertsView vg = view(a), vu = view(u);
+            SplitOut x;
+            x.h = (uint16_t*)a.p[6]; x.l = (uint16_t*)a.p[7]; x.scale = (float*)a.p[8];
+            const int nt = (int)a.i[3];
+            Span sp(this, FAM_MATMUL, span_of(k + 1 - i));
+            const bool done = a.i[4] == 1 ? experts_gemm_f16s(vg, &vu, nullptr, nt, 1, 0, x, (float*)a.p[5], nullptr, 0, false, {}, sg, su, stream)
+                                          : experts_gemm_f16(vg, &vu, nullptr, nt, 1, 0, x, (float*)a.p[5], nullptr, 0, false, {}, sg, su, stream);
+            if (done) {
+                mark_elided({u.p[5]});
+                return k + 1 - i;
+            }
+        }
+    }
+    if (a.id == OP_MATMUL && a.scaled && id(i + 1) == OP_SCALE && h[i + 1].p[0] == a.p[5] && h[i + 1].i[0] == a.i[2] * a.i[3]) {
+        Span sp(this, a.fam, span_of(2));
+        a.scaled(stream, h[i + 1].f[0]);
+        return 2;
+    }
+    return 0;
 }
 
 void it_hip::run_fused(std::vector<OpRec>& ops) {

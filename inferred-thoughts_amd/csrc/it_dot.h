@@ -1,6 +1,7 @@
 // Per-block integer dots shared by the GEMV kernels and the fused decode kernels.
 #pragma once
 #include "it_device.h"
+#include "kernels.h"
 
 namespace itk {
 
@@ -72,9 +73,28 @@ struct ExpertsF16P {
     float* out;
     int n_in, n_out, x_mode, n_used;
     const int32_t* n_tiles;
-    const int4* tiles;
+    const int4* tiles;           // null: one matrix, tile t holds the pairs from t * (pairs a tile) on, in order
     const int32_t* order;
+    int n_pairs;
+    float scale_a, scale_b;      // factors of the two products
+    TileCount count;
 };
+IT_DEV int4 tile_of(const ExpertsF16P& p, int tile, int per_tile) {
+    return p.tiles ? p.tiles[tile] : make_int4(0, tile * per_tile, min(per_tile, p.n_pairs - tile * per_tile), 0);
+}
+IT_DEV int n_tiles_of(const ExpertsF16P& p, int per_tile) { return p.tiles ? *p.n_tiles : (p.n_pairs + per_tile - 1) / per_tile; }
+IT_DEV int pair_at(const ExpertsF16P& p, int slot) { return p.tiles ? p.order[slot] : slot; }
+// one thread per tile: the tile's reads of its expert (expert_count_k)
+IT_DEV void count_tile(const ExpertsF16P& p, int64_t e, int cnt) {
+    const TileCount& c = p.count;
+    if (!c.a || !c.tally) return;
+    atomicAdd(c.a + e, (uint32_t)cnt);
+    if (c.b) atomicAdd(c.b + e, (uint32_t)cnt);
+    const unsigned long long host = (c.tier_a && c.tier_a[e] ? cnt : 0) + (c.b && c.tier_b && c.tier_b[e] ? cnt : 0);
+    const unsigned long long all = (unsigned long long)cnt * (c.b ? 2 : 1);
+    if (host) atomicAdd(c.tally + 1, host);
+    if (all > host) atomicAdd(c.tally, all - host);
+}
 
 // Serial ascending fold of T per-block terms from a 16-byte aligned LDS row.  A group is asked for ahead of the one being
 // added, in registers of its own; 32 terms a group, whose additions outlast the reads (2,048 terms: 16 a group 10 us).

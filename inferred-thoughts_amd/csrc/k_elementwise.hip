@@ -87,6 +87,14 @@ bool rms_norm_writes_q8(const float* x, const float* w, const float* out, int nd
 void rms_norm(const float* x, const float* w, float eps, float* out, int64_t n_rows, int nd, int exact,
               hipStream_t s, float* q_scales, int8_t* q_quants) {
     if (n_rows <= 0) return;
+    if (!exact && n_rows > 1 && n_rows < (1 << 24)) {
+        ResidualP p{};
+        p.x = const_cast<float*>(x);
+        p.n_tok = (int)n_rows; p.n = nd;
+        p.w = w; p.eps = eps; p.out = out;
+        p.q.scales = q_scales; p.q.quants = q_quants;
+        if (residual_row(p, s)) return;
+    }
     if (q_scales && q_quants && rms_norm_writes_q8(x, w, out, nd)) {
         hipLaunchKernelGGL(rms_norm_q8_k<256>, dim3((unsigned)n_rows), dim3(256), nd * sizeof(float), s, x, w, eps, out, nd,
                            exact, q_scales, q_quants);
@@ -115,7 +123,7 @@ __global__ __launch_bounds__(64) void head_norm_k(float* __restrict__ x, const f
     }
 }
 
-// The same for many heads when the order of the sum is free: a wave per head, PER neighbouring elements per
+// The same when the order of the sum is free: a wave per head, PER neighbouring elements per
 // lane held in registers, the f64 partial sums added across the wave by lane moves (no LDS, no barrier).
 template <int PER>
 __global__ __launch_bounds__(256) void head_norm_wave_k(float* __restrict__ x, const float* __restrict__ w,
@@ -157,7 +165,7 @@ __global__ __launch_bounds__(256) void head_norm_wave_k(float* __restrict__ x, c
 }
 
 static bool head_norm_wave(float* x, const float* w, int head_dim, float eps, int64_t n_heads, int mode, hipStream_t s) {
-    if (n_heads < 256 || ((uintptr_t)x & 15) != 0) return false;
+    if (((uintptr_t)x & 15) != 0) return false;
     const dim3 grid((unsigned)((n_heads + 3) / 4)), block(256);
     switch (head_dim) {
         case 64: hipLaunchKernelGGL(head_norm_wave_k<1>, grid, block, 0, s, x, w, n_heads, eps, mode); return true;
@@ -168,15 +176,15 @@ static bool head_norm_wave(float* x, const float* w, int head_dim, float eps, in
 }
 
 void rms_norm_heads(float* x, const float* w, int head_dim, float eps, int64_t n_heads, int exact,
-                    hipStream_t s) {
+                    hipStream_t s, bool batch) {
     if (n_heads <= 0) return;
-    if (!exact && head_norm_wave(x, w, head_dim, eps, n_heads, 0, s)) return;
+    if (!exact && (batch || n_heads >= 256) && head_norm_wave(x, w, head_dim, eps, n_heads, 0, s)) return;
     hipLaunchKernelGGL(head_norm_k, dim3((unsigned)n_heads), dim3(64), head_dim * sizeof(float), s, x, w,
                        head_dim, eps, 0, exact);
 }
-void l2_norm_heads(float* x, int head_dim, float eps, int64_t n_heads, int exact, hipStream_t s) {
+void l2_norm_heads(float* x, int head_dim, float eps, int64_t n_heads, int exact, hipStream_t s, bool batch) {
     if (n_heads <= 0) return;
-    if (!exact && head_norm_wave(x, nullptr, head_dim, eps, n_heads, 1, s)) return;
+    if (!exact && (batch || n_heads >= 256) && head_norm_wave(x, nullptr, head_dim, eps, n_heads, 1, s)) return;
     hipLaunchKernelGGL(head_norm_k, dim3((unsigned)n_heads), dim3(64), head_dim * sizeof(float), s, x,
                        (const float*)nullptr, head_dim, eps, 1, exact);
 }
@@ -263,6 +271,7 @@ __global__ __launch_bounds__(THREADS) void softmax_k(float* __restrict__ x, int 
 
 void softmax_rows(float* x, int64_t n_rows, int row, int exact, hipStream_t s) {
     if (n_rows <= 0 || row <= 0) return;
+    if (!exact && n_rows > 1 && n_rows < (1 << 24) && softmax_route(x, (int)n_rows, row, 0, nullptr, nullptr, s)) return;
     hipLaunchKernelGGL(softmax_k<256>, dim3((unsigned)n_rows), dim3(256), row * sizeof(float), s, x, row, exact);
 }
 
@@ -680,7 +689,7 @@ __global__ __launch_bounds__(128) void conv_split_l2_k(float* __restrict__ state
 
 bool conv_split_l2(float* state, const float* x, const float* w, int kernel, int nc, int n_tok, float* q_out, float* k_out,
                    float* v_out, int kdim, float eps, hipStream_t s) {
-    if (n_tok < 64 || nc % 128 || kdim <= 0 || kdim % 128 || 2 * kdim >= nc || kernel < 2 || kernel > 5) return false;
+    if (n_tok < kernel || nc % 128 || kdim <= 0 || kdim % 128 || 2 * kdim >= nc || kernel < 2 || kernel > 5) return false;
     if (!aligned16(x) || !aligned16(q_out) || !aligned16(k_out) || !aligned16(v_out)) return false;
     dim3 grid((nc / 4 + 127) / 128, (n_tok + CONV_TOK - 1) / CONV_TOK), block(128);
     switch (kernel) {
@@ -733,7 +742,7 @@ __global__ __launch_bounds__(256) void gated_norm_silu_q8_k(const float* __restr
 
 bool gated_norm_silu_q8(const float* core, const float* w, float* z, float* scales, int8_t* quants, int64_t n_heads, float eps,
                         hipStream_t s) {
-    if (n_heads < 256 || ((uintptr_t)core & 7) || ((uintptr_t)z & 7) || ((uintptr_t)quants & 1)) return false;
+    if (n_heads <= 0 || ((uintptr_t)core & 7) || ((uintptr_t)z & 7) || ((uintptr_t)quants & 1)) return false;
     hipLaunchKernelGGL(gated_norm_silu_q8_k, dim3((unsigned)((n_heads + 3) / 4)), dim3(256), 0, s, core, w, z, scales, quants, n_heads, eps);
     return true;
 }
@@ -741,7 +750,7 @@ bool gated_norm_silu_q8(const float* core, const float* w, float* z, float* scal
 void ssm_conv(float* state, const float* x, const float* w, int kernel, int nc, int n_tok, float* out, int exact,
               hipStream_t s) {
     if (nc <= 0 || n_tok <= 0) return;
-    if (n_tok >= 64 && nc % 4 == 0 && aligned16(x) && aligned16(out) && kernel >= 2 && kernel <= 5) {
+    if (n_tok >= (exact ? 64 : kernel) && nc % 4 == 0 && aligned16(x) && aligned16(out) && kernel >= 2 && kernel <= 5) {
         dim3 grid((nc / 4 + 127) / 128, (n_tok + CONV_TOK - 1) / CONV_TOK), block(128);
 #define IT_CONV4(KEEP)                                                                                        \
     do {                                                                                                      \

@@ -52,46 +52,10 @@ namespace {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int FK = 64;          // k per slab
-constexpr int FBS = FK + 4;     // LDS row stride of a token slab, in f16 (136 bytes: no bank is hit twice by 16 lanes)
+constexpr int FBS = FK + 8;     // LDS row stride of a token slab, in f16 (144 bytes: eight lanes' 16-byte reads hit every bank once)
 constexpr int FPAIRS = 128;     // pairs per tile
 constexpr int FSUPER = 256;     // k per weight staging step (one 128-byte line of nibbles per row)
 constexpr int FWS = 128 + 16;   // LDS row stride of a weight segment, in bytes
-
-// rows of f16 hi / lo and the row's power of two, from Q8_0 quants and scales
-__global__ __launch_bounds__(256) void acts_split_f16_k(const int8_t* __restrict__ q, const float* __restrict__ sc,
-                                                         int n_in, uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
-                                                         float* __restrict__ rscale) {
-    __shared__ float part[4];
-    const int row = blockIdx.x, tid = threadIdx.x, nb = n_in >> 5;
-    float mx = 0.0f;
-    for (int b = tid; b < nb; b += 256) mx = fmaxf(mx, fabsf(sc[(int64_t)row * nb + b]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if ((tid & 63) == 0) part[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])) * 127.0f;
-    int ex = 0;
-    if (mx > 0.0f) (void)frexpf(mx, &ex);                     // mx = m * 2^ex, m in [0.5, 1)
-    ex = max(-100, min(100, ex));
-    const float down = ldexpf(1.0f, -ex);
-    if (tid == 0) rscale[row] = ldexpf(1.0f, ex);
-    for (int i = tid; i < n_in / 4; i += 256) {
-        const uint32_t qq = ((const uint32_t*)(q + (int64_t)row * n_in))[i];
-        const float d = sc[(int64_t)row * nb + (i >> 3)] * down;
-        uint16_t h[4], l[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float x = (float)(int8_t)(qq >> (8 * k)) * d;
-            const _Float16 hi = (_Float16)x;
-            const _Float16 lo = (_Float16)(x - (float)hi);
-            h[k] = __builtin_bit_cast(uint16_t, hi);
-            l[k] = __builtin_bit_cast(uint16_t, lo);
-        }
-        ((uint2*)(xh + (int64_t)row * n_in))[i] = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-        ((uint2*)(xl + (int64_t)row * n_in))[i] = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
-    }
-}
-
 
 template <bool GLU, int T>
 __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int4 td, const int row_block, uint16_t* Bh, uint16_t* Bl,
@@ -103,7 +67,7 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
     const int wave = wave8 & 3;      // which 32 (GLU) or 64 rows of the block
     const int th = wave8 >> 2;       // which half of the tile's token groups: T groups each
     const int r = lane & 31, kg = lane >> 5;
-    const int n_in = p.n_in, nslab = n_in / FK;
+    const int n_in = p.n_in;
     // the two row sets of this wave
     const int rows_per_block = GLU ? 128 : 256;
     const int rb0 = row_block * rows_per_block + (GLU ? 32 : 64) * wave;
@@ -199,10 +163,8 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
             const int idx = tid + u * 512, tok = idx >> 3, seg = idx & 7;
             uint16_t* dh = Bh + (buf * FPAIRS + tok) * FBS + seg * 8;
             uint16_t* dl = Bl + (buf * FPAIRS + tok) * FBS + seg * 8;
-            *(uint2*)dh = make_uint2(rbh[u].x, rbh[u].y);
-            *(uint2*)(dh + 4) = make_uint2(rbh[u].z, rbh[u].w);
-            *(uint2*)dl = make_uint2(rbl[u].x, rbl[u].y);
-            *(uint2*)(dl + 4) = make_uint2(rbl[u].z, rbl[u].w);
+            *(uint4*)dh = rbh[u];
+            *(uint4*)dl = rbl[u];
         }
     };
     // The same stores one at a time, to go between the MFMA groups of the slab's second half: issued together at the
@@ -217,11 +179,11 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
         const int idx = tid + u * 512;
         xdst[u] = Bh + (idx >> 3) * FBS + (idx & 7) * 8;
     }
-    auto stash_x_part = [&](int buf, int i) __attribute__((always_inline)) {   // i < 4 T
-        const int u = i >> 2, part = i & 3;
-        uint16_t* d = xdst[u] + buf * FPAIRS * FBS + (part < 2 ? 0 : 2 * FPAIRS * FBS) + 4 * (part & 1);
-        const uint4 v = part < 2 ? rbh[u] : rbl[u];
-        *(uint2*)d = (part & 1) ? make_uint2(v.z, v.w) : make_uint2(v.x, v.y);
+    auto stash_x_part = [&](int buf, int i) __attribute__((always_inline)) {   // i < 2 T
+        // (picked by conditionals, like the weights' below)
+        const uint4 v = i == 0 ? rbh[0] : i == 1 ? rbl[0] : i == 2 ? rbh[T - 1] : rbl[T - 1];
+        uint16_t* d = i < 2 ? xdst[0] : xdst[T - 1];
+        *(uint4*)(d + buf * FPAIRS * FBS + (i & 1) * 2 * FPAIRS * FBS) = v;
     };
     auto stash_w_part = [&](int b, int i) __attribute__((always_inline)) {   // i < 5
         // (the register set picked by conditionals: indexed by a value the compiler does not fold early enough, the
@@ -257,15 +219,9 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
     };
     struct Tok { h8 h, l; };
     auto read_tok = [&](int buf, int n, int tt) __attribute__((always_inline)) -> Tok {
-        // bytes 16 * kg + 4 * n .. + 3 of the row's slab: sub-block 2 * kg + n / 2, elements 4 * (n % 2) + {0..3}
-        // from the low nibbles and 8 more from the high ones
-        const int k0 = 32 * kg + 16 * (n >> 1) + 4 * (n & 1);
-        const uint16_t* bh = Bh + (buf * FPAIRS + 32 * (T * th + tt) + r) * FBS + k0;
-        const uint16_t* bl = Bl + (buf * FPAIRS + 32 * (T * th + tt) + r) * FBS + k0;
-        const uint2 h0 = *(const uint2*)bh, h1 = *(const uint2*)(bh + 8);
-        const uint2 l0 = *(const uint2*)bl, l1 = *(const uint2*)(bl + 8);
-        return Tok{__builtin_bit_cast(h8, make_uint4(h0.x, h0.y, h1.x, h1.y)),
-                   __builtin_bit_cast(h8, make_uint4(l0.x, l0.y, l1.x, l1.y))};
+        // bytes 16 * kg + 4 * n .. + 3 of the row's slab: in the split form's order one run of eight elements
+        const int at = (buf * FPAIRS + 32 * (T * th + tt) + r) * FBS + 32 * kg + 8 * n;
+        return Tok{__builtin_bit_cast(h8, *(const uint4*)(Bh + at)), __builtin_bit_cast(h8, *(const uint4*)(Bl + at))};
     };
 
     const bool live_half = __builtin_amdgcn_readfirstlane(32 * T * th < cnt ? 1 : 0) != 0;
@@ -331,10 +287,10 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
                             if (i < 5) stash_w_part(wb ^ 1, i);
                     }
                     if (more && g1 > 2 * T && g1 < 4 * T) {
-                        constexpr int PPG = (4 * T + 2 * T - 2) / (2 * T - 1);
+                        constexpr int PPG = (2 * T + 2 * T - 2) / (2 * T - 1);
 #pragma unroll
                         for (int i = (g1 - 2 * T - 1) * PPG; i < (g1 - 2 * T) * PPG; i++)
-                            if (i < 4 * T) stash_x_part(par ^ 1, i);
+                            if (i < 2 * T) stash_x_part(par ^ 1, i);
                     }
                     if (g1 == 4 * T) {
                         GEMM_STAMP(2);
@@ -360,8 +316,8 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
         }
     }
 
-    const float e2a = p.scale2 ? p.scale2[e] : 1.0f;
-    const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : 1.0f) : e2a;
+    const float e2a = p.scale2 ? p.scale2[e] : p.scale_a;
+    const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : p.scale_b) : e2a;
 #pragma unroll
     for (int tt = 0; tt < T; tt++) {
         const int slot = 32 * (T * th + tt) + r;
@@ -408,11 +364,12 @@ __global__ __launch_bounds__(512) void experts_f16_k(ExpertsF16P p) {
     const int n_rb = (p.n_out + (GLU ? 128 : 256) - 1) / (GLU ? 128 : 256);
     const int lin = blockIdx.x;
     const int tile = 8 * (lin / (8 * n_rb)) + (lin & 7), row_block = (lin >> 3) % n_rb;
-    if (tile >= *p.n_tiles) return;
-    const int4 td = p.tiles[tile];
+    if (tile >= n_tiles_of(p, FPAIRS)) return;
+    const int4 td = tile_of(p, tile, FPAIRS);
     const int cnt = td.z;
+    if (row_block == 0 && threadIdx.x == 0) count_tile(p, td.x, cnt);
     if (threadIdx.x < FPAIRS) {
-        const int pair = p.order[td.y + min((int)threadIdx.x, cnt - 1)];
+        const int pair = pair_at(p, td.y + min((int)threadIdx.x, cnt - 1));
         pair_s[threadIdx.x] = pair;
         xrow_s[threadIdx.x] = p.x_mode == 0 ? pair : (p.x_mode == 1 ? pair / p.n_used : 0);
     }
@@ -427,14 +384,11 @@ __global__ __launch_bounds__(512) void experts_f16_k(ExpertsF16P p) {
 size_t experts_f16_work_ints(int n_picks, int n_expert) {
     return 16 + (size_t)(n_expert + n_picks / FPAIRS + 2) * 4 + (size_t)n_picks;
 }
-size_t experts_f16_work_bytes(int x_rows, int n_in) {
-    return (size_t)x_rows * n_in * 4 + (((size_t)x_rows * 4 + 255) & ~(size_t)255);
-}
 
-bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const int8_t* act_quants, const float* out) {
+bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const float* out) {
     if (n_picks < 32 || w.n_expert > 1024 || w.fmt != W_NVFP4 || w.n_in % FSUPER || w.n_out % 4) return false;
     if ((reinterpret_cast<uintptr_t>(w.q) & 15) || w.q_stride % 16 || w.s_stride % 16 || (reinterpret_cast<uintptr_t>(w.scales) & 15) ||
-        (reinterpret_cast<uintptr_t>(act_quants) & 3) || (reinterpret_cast<uintptr_t>(out) & 15))
+        (reinterpret_cast<uintptr_t>(out) & 15))
         return false;
     if (up && (up->fmt != w.fmt || up->n_in != w.n_in || up->n_out != w.n_out || (reinterpret_cast<uintptr_t>(up->q) & 15) ||
                (reinterpret_cast<uintptr_t>(up->scales) & 15) || up->q_stride != w.q_stride || up->s_stride != w.s_stride))
@@ -451,22 +405,17 @@ bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks,
 }
 
 bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
-                      int x_mode, const float* act_scales, const int8_t* act_quants, float* out, int32_t* work,
-                      size_t work_ints, void* fwork, size_t fwork_bytes, bool grouped, hipStream_t s) {
-    if (!work || !fwork || !experts_f16_takes(w, up, n_picks, act_quants, out)) return false;
+                      int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
+                      const TileCount& count, float scale_a, float scale_b, hipStream_t s) {
+    if (!x.h || !experts_f16_takes(w, up, n_picks, out)) return false;
+    if (ids && (!work || work_ints < experts_f16_work_ints(n_picks, w.n_expert))) return false;
     if (n_used < 1) n_used = 1;
-    const int x_rows = x_mode == 0 ? n_picks : (x_mode == 1 ? (n_picks + n_used - 1) / n_used : 1);
-    if (work_ints < experts_f16_work_ints(n_picks, w.n_expert) || fwork_bytes < experts_f16_work_bytes(x_rows, w.n_in)) return false;
     const size_t lds = (size_t)4 * FPAIRS * FBS * sizeof(uint16_t) + (size_t)2 * 256 * (FWS + 16);
-    const int max_tiles = w.n_expert + n_picks / FPAIRS + 1;
-    int32_t* n_tiles = work;
-    int4* tiles = (int4*)(work + 16);
-    int32_t* order = work + 16 + (size_t)(max_tiles + 1) * 4;
-    if (!grouped) moe_group(ids, n_picks, w.n_expert, FPAIRS, n_tiles, tiles, order, s);
-    uint16_t* xh = (uint16_t*)fwork;
-    uint16_t* xl = xh + (size_t)x_rows * w.n_in;
-    float* rscale = (float*)(xl + (size_t)x_rows * w.n_in);
-    hipLaunchKernelGGL(acts_split_f16_k, dim3(x_rows), dim3(256), 0, s, act_quants, act_scales, w.n_in, xh, xl, rscale);
+    const int max_tiles = ids ? w.n_expert + n_picks / FPAIRS + 1 : (n_picks + FPAIRS - 1) / FPAIRS;
+    int32_t* n_tiles = ids ? work : nullptr;
+    int4* tiles = ids ? (int4*)(work + 16) : nullptr;
+    int32_t* order = ids ? work + 16 + (size_t)(max_tiles + 1) * 4 : nullptr;
+    if (ids && !grouped) moe_group(ids, n_picks, w.n_expert, FPAIRS, n_tiles, tiles, order, s);
     ExpertsF16P p{};
     p.q = (const uint8_t*)w.q;
     p.s = (const uint8_t*)w.scales;
@@ -480,9 +429,13 @@ bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t
     p.s2_tab = up ? up->s_tab : nullptr;
     p.scale2 = w.scale2;
     p.scale2_up = up ? up->scale2 : nullptr;
-    p.xh = xh;
-    p.xl = xl;
-    p.rscale = rscale;
+    p.xh = x.h;
+    p.xl = x.l;
+    p.rscale = x.scale;
+    p.n_pairs = n_picks;
+    p.scale_a = scale_a;
+    p.scale_b = scale_b;
+    p.count = count;
     p.out = out;
     p.n_in = w.n_in;
     p.n_out = w.n_out;

@@ -12,7 +12,7 @@
 //    the A operand straight from the nibble bytes it loads from global memory: two 128-bit loads per 256-wide
 //    k chunk, units kg and kg + 4, so that the four lanes of a row fetch its whole 128-byte line at once
 //    (with one load per 128-wide chunk every line was fetched in two halves, far apart in time: 10 % slower);
-//  * the activations of the 16 pairs are stored by acts_split_perm_k in the order the MFMA steps consume
+//  * the activations of the 16 pairs are stored (the split form, k_rows.hip) in the order the MFMA steps consume
 //    them, so a lane's B operands of a chunk are sixteen 128-bit loads (from L2: a batch's activations are a
 //    few MB).  They stay in registers while the wave walks its row groups, so every B load feeds
 //    `groups` MFMAs;
@@ -40,46 +40,6 @@ constexpr int SK_KC = 256;     // k per chunk: two 32-wide units per k group, 12
 constexpr int SK_G = 8;        // row groups per wave at most
 constexpr int SK_AHEAD = 1;    // steps of weights in flight per wave
 
-// Rows of f16 hi / lo in MFMA step order and the row's power of two, from Q8_0 quants and scales (the values of
-// acts_split_f16_k; inside every 32-element unit, element j moves to 8 n + 4 (j / 8 % 2) + j % 4 with
-// n = 2 (j / 16) + (j / 4) % 2).
-__global__ __launch_bounds__(256) void acts_split_perm_k(const int8_t* __restrict__ q, const float* __restrict__ sc,
-                                                          int n_in, uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
-                                                          float* __restrict__ rscale) {
-    __shared__ float part[4];
-    const int row = blockIdx.x, tid = threadIdx.x, nb = n_in >> 5;
-    float mx = 0.0f;
-    for (int b = tid; b < nb; b += 256) mx = fmaxf(mx, fabsf(sc[(int64_t)row * nb + b]));
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-    if ((tid & 63) == 0) part[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])) * 127.0f;
-    int ex = 0;
-    if (mx > 0.0f) (void)frexpf(mx, &ex);                     // mx = m * 2^ex, m in [0.5, 1)
-    ex = max(-100, min(100, ex));
-    const float down = ldexpf(1.0f, -ex);
-    if (tid == 0) rscale[row] = ldexpf(1.0f, ex);
-    for (int i = tid; i < n_in / 4; i += 256) {
-        const uint32_t qq = ((const uint32_t*)(q + (int64_t)row * n_in))[i];
-        const float d = sc[(int64_t)row * nb + (i >> 3)] * down;
-        uint16_t h[4], l[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float x = (float)(int8_t)(qq >> (8 * k)) * d;
-            const _Float16 hi = (_Float16)x;
-            const _Float16 lo = (_Float16)(x - (float)hi);
-            h[k] = __builtin_bit_cast(uint16_t, hi);
-            l[k] = __builtin_bit_cast(uint16_t, lo);
-        }
-        const int j0 = 4 * (i & 7);                            // first of this thread's four elements inside the unit
-        const int n = 2 * (j0 >> 4) + ((j0 >> 2) & 1);
-        const int64_t at = (int64_t)row * n_in + 32 * (i >> 3) + 8 * n + 4 * ((j0 >> 3) & 1);
-        *(uint2*)(xh + at) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-        *(uint2*)(xl + at) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
-    }
-}
-
 struct RawW {
     uint4 nib[2];     // units kg and kg + 4 of the chunk: a row's whole 128-byte line is read by its four lanes at once
     uint32_t sc[2];
@@ -105,10 +65,11 @@ template <bool GLU>
 __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
     __shared__ float4 handoff[GLU ? 2 * SK_G * 64 : 1];
     const int tile = blockIdx.x;
-    if (tile >= *p.n_tiles) return;
-    const int4 td = p.tiles[tile];
+    if (tile >= n_tiles_of(p, SK_PAIRS)) return;
+    const int4 td = tile_of(p, tile, SK_PAIRS);
     const int64_t e = td.x;
     const int cnt = td.z;
+    if (blockIdx.y == 0 && threadIdx.x == 0) count_tile(p, e, cnt);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kg = lane >> 4;
@@ -119,7 +80,7 @@ __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
     // this wave's row groups: rows g0 * 16 .. of the matrix, `mine` of them (none: the wave only keeps the barrier)
     const int g0 = (blockIdx.y * WPB + wslot) * gpw;
     const int mine = max(0, min(gpw, (p.n_out + 15) / 16 - g0));
-    const int pair = p.order[td.y + min(r16, cnt - 1)];
+    const int pair = pair_at(p, td.y + min(r16, cnt - 1));
     const int xrow = p.x_mode == 0 ? pair : (p.x_mode == 1 ? pair / p.n_used : 0);
     const uint16_t* bh = p.xh + (int64_t)xrow * n_in + 32 * kg;
     const uint16_t* bl = p.xl + (int64_t)xrow * n_in + 32 * kg;
@@ -200,8 +161,8 @@ __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
     }
     if (r16 >= cnt) return;
     const float rsc = p.rscale[xrow];
-    const float e2a = p.scale2 ? p.scale2[e] : 1.0f;
-    const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : 1.0f) : e2a;
+    const float e2a = p.scale2 ? p.scale2[e] : p.scale_a;
+    const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : p.scale_b) : e2a;
 #pragma unroll
     for (int g = 0; g < SK_G; g++) {
         if (g >= mine) break;
@@ -236,16 +197,17 @@ __global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches
     constexpr int RS = 8 / KW;        // row sets per block
     __shared__ float4 red[2][8][4][64];   // [buffer][wave][tile of the batch][lane]
     const int tile = blockIdx.x;
-    if (tile >= *p.n_tiles) return;
-    const int4 td = p.tiles[tile];
+    if (tile >= n_tiles_of(p, SK_PAIRS)) return;
+    const int4 td = tile_of(p, tile, SK_PAIRS);
     const int64_t e = td.x;
     const int cnt = td.z;
+    if (blockIdx.y == 0 && threadIdx.x == 0) count_tile(p, e, cnt);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kw = wave % KW, rs = wave / KW;
     const int r16 = lane & 15, kg = lane >> 4;
     const int n_in = p.n_in, n_groups = (p.n_out + 15) / 16;
-    const int pair = p.order[td.y + min(r16, cnt - 1)];
+    const int pair = pair_at(p, td.y + min(r16, cnt - 1));
     const int xrow = p.x_mode == 0 ? pair : (p.x_mode == 1 ? pair / p.n_used : 0);
     const uint8_t* wq[2] = {it_expert_at(p.q, p.q_tab, e, p.q_stride), GLU ? it_expert_at(p.q2, p.q2_tab, e, p.q_stride) : nullptr};
     const uint8_t* ws[2] = {it_expert_at(p.s, p.s_tab, e, p.s_stride), GLU ? it_expert_at(p.s2, p.s2_tab, e, p.s_stride) : nullptr};
@@ -290,8 +252,8 @@ __global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches
         }
     }
     const float rsc = p.rscale[xrow];
-    const float e2a = p.scale2 ? p.scale2[e] : 1.0f;
-    const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : 1.0f) : e2a;
+    const float e2a = p.scale2 ? p.scale2[e] : p.scale_a;
+    const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : p.scale_b) : e2a;
 
     for (int i = 0; i < batches_per_block; i++) {
         const int buf = i & 1;
@@ -341,10 +303,10 @@ __global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches
 
 }  // namespace
 
-bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const int8_t* act_quants, const float* out) {
+bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const float* out) {
     if (n_picks < 32 || w.n_expert > 1024 || w.fmt != W_NVFP4 || w.n_in % SK_KC || w.n_out % 4) return false;
     if ((reinterpret_cast<uintptr_t>(w.q) & 15) || w.q_stride % 16 || w.s_stride % 2 || (reinterpret_cast<uintptr_t>(w.scales) & 1) ||
-        (reinterpret_cast<uintptr_t>(act_quants) & 3) || (reinterpret_cast<uintptr_t>(out) & 15))
+        (reinterpret_cast<uintptr_t>(out) & 15))
         return false;
     if (up && (up->fmt != w.fmt || up->n_in != w.n_in || up->n_out != w.n_out || (reinterpret_cast<uintptr_t>(up->q) & 15) ||
                (reinterpret_cast<uintptr_t>(up->scales) & 1) || up->q_stride != w.q_stride || up->s_stride != w.s_stride))
@@ -353,22 +315,17 @@ bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks
 }
 
 bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
-                       int x_mode, const float* act_scales, const int8_t* act_quants, float* out, int32_t* work,
-                       size_t work_ints, void* fwork, size_t fwork_bytes, bool grouped, hipStream_t s) {
-    if (!work || !fwork || !experts_f16s_takes(w, up, n_picks, act_quants, out)) return false;
+                       int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
+                       const TileCount& count, float scale_a, float scale_b, hipStream_t s) {
+    if (!x.h || !experts_f16s_takes(w, up, n_picks, out)) return false;
+    if (ids && (!work || work_ints < experts_group_work_ints(n_picks, w.n_expert))) return false;
     if (n_used < 1) n_used = 1;
-    const int x_rows = x_mode == 0 ? n_picks : (x_mode == 1 ? (n_picks + n_used - 1) / n_used : 1);
-    if (work_ints < experts_group_work_ints(n_picks, w.n_expert) || fwork_bytes < experts_f16_work_bytes(x_rows, w.n_in)) return false;
     // the layout of the int8 tile kernel's grouping (tiles of 16 pairs): either may reuse the other's
-    const int max_tiles = w.n_expert + n_picks / SK_PAIRS + 1;
-    int32_t* n_tiles = work;
-    int4* tiles = (int4*)(work + 16);
-    int32_t* order = work + 16 + (size_t)(max_tiles + 1) * 4;
-    if (!grouped) moe_group(ids, n_picks, w.n_expert, SK_PAIRS, n_tiles, tiles, order, s);
-    uint16_t* xh = (uint16_t*)fwork;
-    uint16_t* xl = xh + (size_t)x_rows * w.n_in;
-    float* rscale = (float*)(xl + (size_t)x_rows * w.n_in);
-    hipLaunchKernelGGL(acts_split_perm_k, dim3(x_rows), dim3(256), 0, s, act_quants, act_scales, w.n_in, xh, xl, rscale);
+    const int max_tiles = ids ? w.n_expert + n_picks / SK_PAIRS + 1 : (n_picks + SK_PAIRS - 1) / SK_PAIRS;
+    int32_t* n_tiles = ids ? work : nullptr;
+    int4* tiles = ids ? (int4*)(work + 16) : nullptr;
+    int32_t* order = ids ? work + 16 + (size_t)(max_tiles + 1) * 4 : nullptr;
+    if (ids && !grouped) moe_group(ids, n_picks, w.n_expert, SK_PAIRS, n_tiles, tiles, order, s);
     ExpertsF16P p{};
     p.q = (const uint8_t*)w.q;
     p.s = (const uint8_t*)w.scales;
@@ -382,9 +339,13 @@ bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_
     p.s2_tab = up ? up->s_tab : nullptr;
     p.scale2 = w.scale2;
     p.scale2_up = up ? up->scale2 : nullptr;
-    p.xh = xh;
-    p.xl = xl;
-    p.rscale = rscale;
+    p.xh = x.h;
+    p.xl = x.l;
+    p.rscale = x.scale;
+    p.n_pairs = n_picks;
+    p.scale_a = scale_a;
+    p.scale_b = scale_b;
+    p.count = count;
     p.out = out;
     p.n_in = w.n_in;
     p.n_out = w.n_out;
@@ -394,7 +355,7 @@ bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_
     p.tiles = tiles;
     p.order = order;
     const int groups = (w.n_out + 15) / 16;
-    const int likely_tiles = std::min(n_picks, w.n_expert) + n_picks / SK_PAIRS;
+    const int likely_tiles = ids ? std::min(n_picks, w.n_expert) + n_picks / SK_PAIRS : max_tiles;
     const int n_chunk = w.n_in / SK_KC;
     if (n_chunk == 1 || n_chunk == 2 || n_chunk == 4 || n_chunk == 8) {
         // k split over the waves: a batch is 4 / NM row groups per row set, 8 / n_chunk row sets per block; 8 batches

@@ -43,6 +43,48 @@ void repack_nvfp4(const uint8_t* raw, uint8_t* nib, uint8_t* scales, int64_t n_r
 // ---- activation quantization --------------------------------------------------
 void quantize_q8_0(const float* x, float* scales, int8_t* quants, int64_t n, hipStream_t s);
 
+// The split form of quantized rows (k_rows.hip): q * d divided by the row's power of two as f16 hi + lo, in the operand
+// order of the f16 matrix-core kernels; scale[row] is that power of two.
+struct SplitOut {
+    uint16_t* h = nullptr;
+    uint16_t* l = nullptr;
+    float* scale = nullptr;
+};
+struct QuantOut {
+    float* scales = nullptr;
+    int8_t* quants = nullptr;
+    SplitOut split;          // split.h null: the Q8_0 form alone
+};
+void split_rows(const int8_t* quants, const float* scales, int64_t n_rows, int row, const SplitOut& o, hipStream_t s);
+
+// ---- runs of row-wise ops of a batch pass (k_rows.hip, fast mode); false: nothing launched, the shape is not taken ----
+struct ResidualP {           // [y = the picks' rows and the gated shared row summed ->] x += y [-> out = rms norm -> copy -> forms]
+    float* x;
+    float* y;                // null: no sum, x stays as it is
+    int n_tok, n;
+    const float *rows, *rw, *logit;   // rows null: y is there already
+    const float* shared;
+    int n_used;
+    const float* w;                   // null: no norm
+    float eps;
+    float *out, *copy;
+    QuantOut q;                       // of the normed rows; quants null: none
+};
+bool residual_row(const ResidualP& p, hipStream_t s);
+// op 0: the forms of a; 1: a = silu(a) * b first; 2: a *= sigmoid(b) first
+bool mul_forms(float* a, const float* b, int op, int64_t n_rows, int row, const QuantOut& o, hipStream_t s);
+struct AttnRowsP {
+    const float *qg, *v, *q_w, *k_w;
+    float *q, *g, *k;
+    uint16_t *k_slab, *v_slab;
+    int64_t k_at, v_at;
+    const float2* table;
+    int n_tok, n_head, n_kv, half, pos;
+    float q_eps, k_eps;
+};
+bool attn_rows(const AttnRowsP& p, int head_dim, hipStream_t s);
+bool softmax_route(float* x, int n_tok, int n_expert, int n_used, int32_t* ids, float* weights, hipStream_t s);
+
 // ---- matmul family -------------------------------------------------------------
 // out[t][j] = dot(w.row(j), x[t]); act is the Q8_0 form of x for quantized formats.
 void matmul(const WView& w, const float* x, const float* act_scales, const int8_t* act_quants, int n_tok,
@@ -79,24 +121,30 @@ void matmul_experts(const ExpertsView& w, const int32_t* ids, int n_picks, int n
 size_t experts_group_work_ints(int n_picks, int n_expert);
 // NVFP4 only, fast mode: the same products on the f16 matrix cores, weights expanded exactly to f16 and the
 // Q8_0 activations as an f16 hi/lo pair; results agree with the int8 kernels to ~1e-6 relative.
-// work: experts_f16_work_ints ints; fwork: experts_f16_work_bytes bytes, 16-byte aligned.
+// work: experts_f16_work_ints ints.  ids null: one dense matrix, the pairs are the n_picks rows of x in order.
 size_t experts_f16_work_ints(int n_picks, int n_expert);
 // pairs sorted into per-expert lists cut into tiles of at most tile_pairs: n_tiles[0] = tile count, tiles = {expert,
 // first slot, pairs, 0}, order[slot] = pair
 void moe_group(const int32_t* ids, int n_picks, int n_expert, int tile_pairs, int32_t* n_tiles, int4* tiles,
                int32_t* order, hipStream_t s);
-size_t experts_f16_work_bytes(int x_rows, int n_in);
-// whether experts_gemm_f16 takes these operands (shape, format, alignment), given scratch of the sizes above
-bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const int8_t* act_quants, const float* out);
+// what the tile kernels below add to the expert read counters (one launch less than expert_count)
+struct TileCount {
+    uint32_t *a = nullptr, *b = nullptr;
+    unsigned long long* tally = nullptr;
+    const uint8_t *tier_a = nullptr, *tier_b = nullptr;
+};
+// whether experts_gemm_f16 takes these operands (shape, format, alignment), given scratch of the size above
+bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const float* out);
 bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
-                      int x_mode, const float* act_scales, const int8_t* act_quants, float* out, int32_t* work,
-                      size_t work_ints, void* fwork, size_t fwork_bytes, bool grouped, hipStream_t s);
+                      int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
+                      const TileCount& count, float scale_a, float scale_b, hipStream_t s);
 // NVFP4 experts with few pairs per expert in fast mode (k_gemm_f16s.hip): tiles of 16 pairs on MFMA 16x16x32 f16, no LDS;
-// the grouping has the layout of experts_gemm's (tiles of 16 pairs).  Scratch as for experts_gemm_f16.
-bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const int8_t* act_quants, const float* out);
+// the grouping has the layout of experts_gemm's (tiles of 16 pairs).  ids as for experts_gemm_f16; scale_a, scale_b: factors
+// of the two products.
+bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const float* out);
 bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
-                       int x_mode, const float* act_scales, const int8_t* act_quants, float* out, int32_t* work,
-                       size_t work_ints, void* fwork, size_t fwork_bytes, bool grouped, hipStream_t s);
+                       int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
+                       const TileCount& count, float scale_a, float scale_b, hipStream_t s);
 // Small batches in fast mode (k_moe_rows.hip): pairs sorted by expert in tiles of 8 or 16, every weight row of a tile's
 // expert streamed once and multiplied with all its pairs by integer dots.  ids null: one dense matrix (strides
 // ignored), tile t = tokens 8 t .. 8 t + 7.  False: nothing launched (shape, alignment or scratch do not fit).
@@ -145,9 +193,10 @@ void rms_norm(const float* x, const float* w, float eps, float* out, int64_t n_r
 // whether rms_norm writes the Q8_0 form when given the buffers for it (row length and alignments): the caller marks the
 // quantized form valid only then
 bool rms_norm_writes_q8(const float* x, const float* w, const float* out, int nd);
+// batch: the rows of several tokens, whose norms do not depend on which of the kernels makes them (fast mode: a wave a head)
 void rms_norm_heads(float* x, const float* w, int head_dim, float eps, int64_t n_heads, int exact,
-                    hipStream_t s);
-void l2_norm_heads(float* x, int head_dim, float eps, int64_t n_heads, int exact, hipStream_t s);
+                    hipStream_t s, bool batch = false);
+void l2_norm_heads(float* x, int head_dim, float eps, int64_t n_heads, int exact, hipStream_t s, bool batch = false);
 void rope_neox(float* x, const float2* table, int table_half, int64_t n_tok, int pos, const int* pos_dyn,
                int head_dim, int n_rot, int n_heads, hipStream_t s);
 // exact = 0: long batches take the exponential on the transcendental unit (fast mode)
