@@ -181,6 +181,7 @@ static void launch_gemv(GemvP p, int n_y, hipStream_t s) {
 void matmul(const WView& w, const float* x, const float* act_scales, const int8_t* act_quants, int n_tok,
             float* out, float out_scale, int exact, hipStream_t s) {
     if (n_tok <= 0 || w.n_out <= 0) return;
+    if (!exact && q8_short(w, act_scales, act_quants, n_tok, out, out_scale, s)) return;
     // (fast mode adds each scaled block sum with one rounding: 4 ms of a 174 ms prefill pass)
     if (q8_gemm(w, act_scales, act_quants, n_tok, out, out_scale, s, !exact)) return;
     if (w.fmt == W_Q8_0 || w.fmt == W_NVFP4) {

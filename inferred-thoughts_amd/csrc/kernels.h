@@ -57,6 +57,9 @@ struct QuantOut {
 };
 void split_rows(const int8_t* quants, const float* scales, int64_t n_rows, int row, const SplitOut& o, hipStream_t s);
 
+// The same for a short batch, fast mode: the k range cut over a block's waves (k_q8_short.hip)
+bool q8_short(const WView& w, const float* act_scales, const int8_t* act_quants, int n_tok, float* out, float out_scale, hipStream_t s);
+
 // ---- runs of row-wise ops of a batch pass (k_rows.hip, fast mode); false: nothing launched, the shape is not taken ----
 struct ResidualP {           // [y = the picks' rows and the gated shared row summed ->] x += y [-> out = rms norm -> copy -> forms]
     float* x;

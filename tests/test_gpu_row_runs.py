@@ -79,7 +79,7 @@ def test_the_residual_row(pair, orc, n, nd):
         be.gather_chunks(b["normed"], n * nd, n * nd, 0, b["copy"])
         be.matmul(ih.weights(w, ih.Q8_0, nd, 64), b["copy"], b["out"])
         be.matmul(ih.weights(w, ih.Q8_0, nd, 64), b["normed"], b["out2"])   # the normed rows are still there for others
-    run(pair, n, b, script, ["x", "normed", "copy"], at_most=4)
+    run(pair, n, b, script, ["x", "normed", "copy"], at_most=5)
     run(pair, n, b, script, ["out", "out2"], tol=3e-2)
 
 
