@@ -49,18 +49,25 @@ IT_DEV void unit_nvfp4(const uint4 w, uint32_t sc2, const uint4 a0, const uint4 
 
 // ------------------------------------------------------------------ E2M1 nibbles -> f16
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-// four nibbles (one per byte, 0..15) -> four f16 weights (two dwords), scaled by the sub-block scale
-IT_DEV void fp4x4_to_f16x4(uint32_t v, h2 scale, h2* a, h2* b) {
-    // f16 high bytes of 128 x the doubled e2m1 magnitudes 0 1 2 3 4 6 8 12 (the low bytes are zero): the 128 pays
-    // for the 2^-8 the scale carries (see expand) and the halving that goes with the doubled magnitudes
-    const uint32_t mag = __builtin_amdgcn_perm(0x66646260u, 0x5e5c5800u, v & 0x07070707u);
-    const uint32_t hb = mag | ((v & 0x08080808u) << 4);
-    const uint32_t d0 = __builtin_amdgcn_perm(hb, hb, 0x010c000cu);   // bytes 0, hb.0, 0, hb.1
-    const uint32_t d1 = __builtin_amdgcn_perm(hb, hb, 0x030c020cu);   // bytes 0, hb.2, 0, hb.3
-    *a = __builtin_bit_cast(h2, d0) * scale;
-    *b = __builtin_bit_cast(h2, d1) * scale;
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+// a sub-block's scale for fp4x8_to_f16x8: an e4m3 code moved into an f16's exponent and mantissa fields is the scale times
+// 2^-8, subnormal codes included (4 exponent bits with bias 7 against 5 with bias 15; f16 subnormals are computed with, not
+// flushed); code 0x7f (not a number) counts as zero, as in the CPU path
+IT_DEV h2 e4m3_to_scale(uint32_t code) {
+    const uint32_t em = code & 0x7fu;
+    const _Float16 sv = __builtin_bit_cast(_Float16, (uint16_t)(em == 0x7fu ? 0u : em << 7));
+    return h2{sv, sv};
 }
-
+// the eight weights of a dword of nibbles: byte i's low nibble (element i of its sub-block's half) and high nibble (element
+// 8 + i) side by side, through the conversion of the matrix cores' own fp4 (times 2^8, which pays for the scale's 2^-8) and
+// one packed product; exact.  Half the vector operations of byte permutes and sign bits.
+IT_DEV h8v fp4x8_to_f16x8(uint32_t w, h2 scale) {
+    const h2 a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 0) * scale;
+    const h2 b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 1) * scale;
+    const h2 c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 2) * scale;
+    const h2 d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, 256.0f, 3) * scale;
+    return h8v{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+}
 
 // operands of the f16 expert tile kernels (k_gemm_f16.hip, k_gemm_f16s.hip)
 struct ExpertsF16P {

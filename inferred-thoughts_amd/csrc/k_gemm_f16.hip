@@ -16,10 +16,8 @@
 // read from LDS feeds four MFMAs (two sets, hi and lo) and the f32 sums of a wave stay within the
 // registers that two waves per SIMD leave.  Weight nibbles go through LDS as full 128-byte lines to
 // the owning lane's registers (a lane owns 16 contiguous bytes of a row per 64-wide k slab: the
-// k order inside an MFMA is free once the scales are folded in) and are expanded there: a byte
-// permute yields the f16 high bytes of four magnitudes, the sign bit is or-ed in, two more
-// permutes interleave zero low bytes, and v_pk_mul_f16 applies the sub-block scale (the scale code's bits moved
-// into an f16's fields are the scale times 2^-8; the magnitudes are stored times 2^7, which also takes the halving).
+// k order inside an MFMA is free once the scales are folded in) and are expanded there
+// (fp4x8_to_f16x8).
 //
 // MFMA operand layout (32x32x16, f16): lane l supplies 8 k values of row (l % 32), k group
 // l / 32, for both A (weight rows) and B (tokens); it receives D for token l % 32 and weight
@@ -204,18 +202,8 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
     };
     // fragment n of set z from ra / rs
     auto expand = [&](int z, int n) __attribute__((always_inline)) -> h8 {
-        // An e4m3 code shifted into an f16's exponent and mantissa fields IS the scale times 2^-8, subnormal codes
-        // included (4 exponent bits with bias 7 against 5 with bias 15; f16 subnormals are computed with, not flushed):
-        // no conversion arithmetic.  The magnitudes carry the 2^7 back; code 0x7f (not a number) counts as zero, as
-        // in the CPU path.
-        const uint32_t em = (n < 2 ? rs[z] : rs[z] >> 8) & 0x7fu;
-        const _Float16 sv = __builtin_bit_cast(_Float16, (uint16_t)(em == 0x7fu ? 0u : em << 7));
-        const h2 sc = h2{sv, sv};
         const uint32_t wd = n == 0 ? ra[z].x : n == 1 ? ra[z].y : n == 2 ? ra[z].z : ra[z].w;
-        h2 a0, a1, a2, a3;
-        fp4x4_to_f16x4(wd & 0x0f0f0f0fu, sc, &a0, &a1);          // low nibbles: elements i
-        fp4x4_to_f16x4((wd >> 4) & 0x0f0f0f0fu, sc, &a2, &a3);   // high nibbles: elements 8 + i
-        return h8{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+        return fp4x8_to_f16x8(wd, e4m3_to_scale(n < 2 ? rs[z] : rs[z] >> 8));
     };
     struct Tok { h8 h, l; };
     auto read_tok = [&](int buf, int n, int tt) __attribute__((always_inline)) -> Tok {

@@ -22,8 +22,8 @@
 //
 // MFMA 16x16x32 f16 operands: lane l holds A[l % 16][8 (l / 16) .. + 8], B[8 (l / 16) .. + 8][l % 16] and
 // receives D[4 (l / 16) + i][l % 16], i = 0..3.  The k order inside a step is free as long as A and B agree:
-// step n of a lane's 32-wide unit takes the elements the n-th dword of the 16 nibble bytes holds (low nibbles:
-// elements 16 (n / 2) + 4 (n % 2) + {0..3}; high nibbles: the same + 8).
+// step n of a lane's 32-wide unit takes the elements the n-th dword of the 16 nibble bytes holds (byte i: low nibble element
+// 16 (n / 2) + 4 (n % 2) + i, high nibble the same + 8).
 #include <algorithm>
 
 #include "it_device.h"
@@ -47,16 +47,8 @@ struct RawW {
 
 // fragment n (8 weights as f16, sub-block scale folded in) of a lane's 16 nibble bytes
 IT_DEV h8 expand_frag(const uint4 nib, const uint32_t rsc, int n) {
-    // an e4m3 code moved into an f16's exponent and mantissa fields is the scale times 2^-8 (subnormal codes included);
-    // the magnitudes carry 2^7 and the halving back; code 0x7f (not a number) counts as zero, as in the CPU path
-    const uint32_t em = (n < 2 ? rsc : rsc >> 8) & 0x7fu;
-    const _Float16 sv = __builtin_bit_cast(_Float16, (uint16_t)(em == 0x7fu ? 0u : em << 7));
-    const h2 sc = h2{sv, sv};
     const uint32_t wd = n == 0 ? nib.x : n == 1 ? nib.y : n == 2 ? nib.z : nib.w;
-    h2 a0, a1, a2, a3;
-    fp4x4_to_f16x4(wd & 0x0f0f0f0fu, sc, &a0, &a1);
-    fp4x4_to_f16x4((wd >> 4) & 0x0f0f0f0fu, sc, &a2, &a3);
-    return h8{a0[0], a0[1], a1[0], a1[1], a2[0], a2[1], a3[0], a3[1]};
+    return fp4x8_to_f16x8(wd, e4m3_to_scale(n < 2 ? rsc : rsc >> 8));
 }
 
 // GLU: waves 0 and 1 take the gate matrix, waves 2 and 3 the up matrix of the same rows (a wave streams ONE matrix, so

@@ -9,7 +9,7 @@
 //
 // The split form of a row (what the f16 matrix-core kernels multiply): the Q8_0 value q * d divided by the row's power of
 // two and written as f16 hi + lo (22 bits kept), inside every unit of 32 elements in the order in which a lane's operand of
-// those kernels takes them: element j at 8 n + 4 (j / 8 % 2) + j % 4 with n = 2 (j / 16) + (j / 4) % 2.
+// those kernels takes them: element j at 8 n + 2 (j % 4) + j / 8 % 2 with n = 2 (j / 16) + (j / 4) % 2.
 #include <algorithm>
 
 #include "it_device.h"
@@ -28,6 +28,36 @@ IT_DEV float row_reduce_max(float v, float* red, int tid, int waves) {
     v = red[0];
     for (int w = 1; w < waves; w++) v = fmaxf(v, red[w]);
     return v;
+}
+
+// The split form of four neighbouring elements: their quants times d (the block's scale over the row's power of two).  The
+// elements that lie between them in the operand order are two lanes away: of such a pair one lane writes the hi parts of all
+// eight, 16 bytes, and the other the lo parts.  i: number of the four in the row.
+IT_DEV void put_split(uint32_t quants, float d, int i, int64_t row_at, const SplitOut& o) {
+    uint32_t h[4], l[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float x = (float)(int8_t)(quants >> (8 * k)) * d;
+        const _Float16 hi = (_Float16)x;
+        const _Float16 lo = (_Float16)(x - (float)hi);
+        h[k] = __builtin_bit_cast(uint16_t, hi);
+        l[k] = __builtin_bit_cast(uint16_t, lo);
+    }
+    const bool second = (i >> 1) & 1;             // elements 8 .. 15 of their sixteen
+    uint32_t keep[4], give[2], got[2];
+#pragma unroll
+    for (int k = 0; k < 4; k++) keep[k] = second ? l[k] : h[k];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        give[k] = second ? h[2 * k] | (h[2 * k + 1] << 16) : l[2 * k] | (l[2 * k + 1] << 16);
+        got[k] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)give[k], 0x4E, 0xf, 0xf, true);   // lane ^ 2
+    }
+    const uint32_t other[4] = {got[0] & 0xffffu, got[0] >> 16, got[1] & 0xffffu, got[1] >> 16};
+    uint32_t w[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k] = second ? other[k] | (keep[k] << 16) : keep[k] | (other[k] << 16);
+    const int j0 = 4 * (i & 7), n = 2 * (j0 >> 4) + ((j0 >> 2) & 1);
+    *(uint4*)((second ? o.l : o.h) + row_at + 32 * (i >> 3) + 8 * n) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
 // The Q8_0 (and, xh given, the split) form of a row held four neighbouring elements a thread: thread `tid` of T holds
@@ -73,21 +103,7 @@ IT_DEV void put_forms(const float4 (&val)[NV], int64_t row, int n4, int tid, con
     for (int v = 0; v < NV; v++) {
         const int i = tid + T * v;
         if (i >= n4) continue;
-        const float d = dq[v] * down;
-        uint16_t h[4], l[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float x = (float)(int8_t)(qq[v] >> (8 * k)) * d;
-            const _Float16 hi = (_Float16)x;
-            const _Float16 lo = (_Float16)(x - (float)hi);
-            h[k] = __builtin_bit_cast(uint16_t, hi);
-            l[k] = __builtin_bit_cast(uint16_t, lo);
-        }
-        const int j0 = 4 * (i & 7);               // first of the four elements inside its unit of 32
-        const int n = 2 * (j0 >> 4) + ((j0 >> 2) & 1);
-        const int64_t at = base * 4 + 32 * (i >> 3) + 8 * n + 4 * ((j0 >> 3) & 1);
-        *(uint2*)(o.split.h + at) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-        *(uint2*)(o.split.l + at) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+        put_split(qq[v], dq[v] * down, i, base * 4, o.split);
     }
 }
 
@@ -217,21 +233,7 @@ __global__ __launch_bounds__(256) void split_rows_k(const int8_t* __restrict__ q
     if (tid == 0) o.scale[row] = ldexpf(1.0f, ex);
     for (int i = tid; i < n_in / 4; i += 256) {
         const uint32_t qq = ((const uint32_t*)(q + row * n_in))[i];
-        const float d = sc[row * nb + (i >> 3)] * down;
-        uint16_t h[4], l[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const float x = (float)(int8_t)(qq >> (8 * k)) * d;
-            const _Float16 hi = (_Float16)x;
-            const _Float16 lo = (_Float16)(x - (float)hi);
-            h[k] = __builtin_bit_cast(uint16_t, hi);
-            l[k] = __builtin_bit_cast(uint16_t, lo);
-        }
-        const int j0 = 4 * (i & 7);
-        const int n = 2 * (j0 >> 4) + ((j0 >> 2) & 1);
-        const int64_t at = row * n_in + 32 * (i >> 3) + 8 * n + 4 * ((j0 >> 3) & 1);
-        *(uint2*)(o.h + at) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
-        *(uint2*)(o.l + at) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+        put_split(qq, sc[row * nb + (i >> 3)] * down, i, row * n_in, o);
     }
 }
 
