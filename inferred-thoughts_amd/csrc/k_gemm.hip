@@ -10,6 +10,8 @@
 // MFMA operand layout (16x16x32, i8): lane l supplies 8 consecutive k of row (l % 16) at
 // k = 8 * (l / 16) for both A (weight rows) and B (tokens); it receives D for token l % 16
 // and weight rows 4 * (l / 16) + {0,1,2,3}.
+#include <type_traits>
+
 #include "it_device.h"
 #include "it_dot.h"
 #include "kernels.h"
@@ -138,6 +140,133 @@ __global__ __launch_bounds__(GT) void q8_gemm_k(const int8_t* __restrict__ wq, c
     }
 }
 
+// ------------------------------------------------------------------ rows of whole 256-wide slabs
+// The same products where n_in is a multiple of 256, staged by loads that go from memory straight to LDS.  A block owns 64
+// weight rows x 16 NT tokens; a stage is 256 k (eight blocks' scales are one 16-byte load), two of them in LDS.  The kernel
+// above has one slab of 128 in flight, in registers, and stores it between the products of two slabs: on a batch of some
+// dozen to some hundred tokens every slab waits out most of a trip to memory.  Here a stage is asked for as soon as its
+// buffer has been read and costs no register, no store and one barrier for 256 k.  Such a load writes its lanes' 16 bytes
+// side by side, so a row's sixteen pieces are permuted by the row's number instead of being padded apart: sixteen rows' reads
+// meet every bank once.  The arithmetic is the same, product by product, in the same order.
+// Bound by the vector ALU from some 500 tokens on (twelve operations per product of the matrix cores), below by the stages'
+// latency.  8192 x 2048 over 64 / 201 / 512 / 5,700 tokens: 18.1 -> 11.2, 33.0 -> 27.5, 55.7 -> 50.8, 618 -> 528 us; 4096 x 2048:
+// 16.0 -> 9.3, 24.9 -> 15.4, 33.7 -> 28.3, 296 -> 272; 2048 x 4096: 28.5 -> 15.8, 32.4 -> 18.7, 41.2 -> 27.4, 290 -> 276.
+// Not kept: three or four stages (0 to 50 % slower everywhere: fewer blocks fit a CU); the f16 matrix cores with the
+// activations as an f16 pair and no scale per token, 128 x 256 tiles (8192 x 2048 over 5,700: 437 us with three stages, 46 % of
+// the rate the matrix cores sustain, but 20 % behind on everything smaller).
+typedef __attribute__((address_space(3))) void* lptr;
+typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
+
+// 16 bytes a lane from memory to LDS, one lane's behind the other's from `to` on (the same in every lane).  Written out because
+// the compiler's own form makes every later read of LDS wait for all such loads; here they are waited for by count, in front
+// of the barrier of the stage that reads them.
+IT_DEV void to_lds(const void* from, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(from) : "memory");
+}
+
+template <int NT> constexpr int tile_stage_bytes() { return 64 * 256 + NT * 16 * 256 + 1024 + (NT > 2 ? 2048 : 1024); }
+
+template <int NT, bool FMA>
+__global__ __launch_bounds__(256) void q8_tile_k(const int8_t* __restrict__ wq, const uint16_t* __restrict__ ws,
+                                                 const int8_t* __restrict__ xq, const float* __restrict__ xs,
+                                                 float* __restrict__ out, int n_in, int n_out, int n_tok, float out_scale) {
+    constexpr int STAGE = tile_stage_bytes<NT>(), X_AT = 64 * 256, WS_AT = X_AT + NT * 16 * 256, XS_AT = WS_AT + 1024;
+    constexpr int XS = NT > 2 ? 2 : 1;                  // waves that bring token scales
+    extern __shared__ __align__(1024) uint8_t tlds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.x * 64, tok0 = blockIdx.y * NT * 16;
+    const int nb = n_in >> 5, n_stage = n_in >> 8;
+    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)tlds);
+
+    // what this lane fetches every stage: four weight rows, NT token rows, and for the first waves a row's scales
+    const int8_t* wp[4];
+    const int8_t* xp[NT];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int row = (wave * 4 + i) * 4 + (lane >> 4);
+        wp[i] = wq + (int64_t)min(row0 + row, n_out - 1) * n_in + (((lane & 15) ^ (row & 15)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < NT; i++) {
+        const int row = (wave * NT + i) * 4 + (lane >> 4);
+        xp[i] = xq + (int64_t)min(tok0 + row, n_tok - 1) * n_in + (((lane & 15) ^ (row & 15)) << 4);
+    }
+    const bool has_scales = wave <= XS;
+    const uint8_t* sp = wave == 0 ? (const uint8_t*)(ws + (int64_t)min(row0 + lane, n_out - 1) * nb)
+                                  : (const uint8_t*)(xs + (int64_t)min(tok0 + min((wave - 1) * 32 + (lane >> 1), NT * 16 - 1), n_tok - 1) * nb + 4 * (lane & 1));
+    const int s_step = wave == 0 ? 16 : 32;
+    auto ask = [&](int s, int buf) __attribute__((always_inline)) {
+        const uint32_t d = at + buf * STAGE;
+#pragma unroll
+        for (int i = 0; i < 4; i++) to_lds(wp[i] + s * 256, d + (wave * 4 + i) * 1024);
+#pragma unroll
+        for (int i = 0; i < NT; i++) to_lds(xp[i] + s * 256, d + X_AT + (wave * NT + i) * 1024);
+        if (has_scales) to_lds(sp + s * s_step, d + WS_AT + wave * 1024);
+    };
+    float acc[NT][4];
+#pragma unroll
+    for (int tt = 0; tt < NT; tt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[tt][i] = 0.0f;
+
+    ask(0, 0);
+    for (int s = 0; s < n_stage; s++) {
+        const int buf = s & 1;
+        __builtin_amdgcn_s_waitcnt(0x0f70);      // stage s has landed (vmcnt 0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (s + 1 < n_stage) ask(s + 1, buf ^ 1);      // (every wave has read that buffer)
+        const uint8_t* const d = tlds + buf * STAGE;
+        hv8 dw[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) dw[i] = *(const hv8*)(d + WS_AT + (wave * 16 + 4 * g + i) * 16);
+#pragma unroll
+        for (int b4 = 0; b4 < 2; b4++) {
+            float4 dx[NT];
+#pragma unroll
+            for (int tt = 0; tt < NT; tt++) dx[tt] = *(const float4*)(d + XS_AT + (tt * 16 + m) * 32 + b4 * 16);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int b = 4 * b4 + q, piece = ((2 * b + (g >> 1)) ^ m) << 4;
+                const long a = *(const long*)(d + (wave * 16 + m) * 256 + piece + 8 * (g & 1));
+                float w[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = (float)dw[i][b];
+#pragma unroll
+                for (int tt = 0; tt < NT; tt++) {
+                    const long bv = *(const long*)(d + X_AT + (tt * 16 + m) * 256 + piece + 8 * (g & 1));
+                    const float x = q == 0 ? dx[tt].x : q == 1 ? dx[tt].y : q == 2 ? dx[tt].z : dx[tt].w;
+                    const v4i z = {0, 0, 0, 0};
+                    const v4i c = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bv, z, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        if (FMA) acc[tt][i] = fmaf((float)c[i], w[i] * x, acc[tt][i]);
+                        else acc[tt][i] += (float)c[i] * (w[i] * x);
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int tt = 0; tt < NT; tt++) {
+        const int t = tok0 + tt * 16 + m, j = row0 + wave * 16 + 4 * g;
+        if (t >= n_tok) continue;
+        float* o = out + (int64_t)t * n_out + j;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (out_scale != 1.0f) acc[tt][i] *= out_scale;
+        if (j + 3 < n_out && !(n_out & 3)) {
+            *(float4*)o = make_float4(acc[tt][0], acc[tt][1], acc[tt][2], acc[tt][3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (j + i < n_out) o[i] = acc[tt][i];
+        }
+    }
+}
+
 }  // namespace
 
 bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, int n_tok, float* out, float out_scale,
@@ -155,6 +284,29 @@ bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, 
         else hipLaunchKernelGGL((q8_gemm_k<NT, false>), dim3(gx, (tiles + NT - 1) / NT), dim3(GT), 0, s, wq, ws, act_quants, act_scales, \
                                 out, w.n_in, w.n_out, n_tok, out_scale);                                            \
     } while (0)
+    const bool slabs = w.n_in % 256 == 0 && !((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(act_scales) | reinterpret_cast<uintptr_t>(out)) & 15);
+    if (slabs) {
+        // 16 tokens a block up to 640 of the smallest blocks (2.5 a CU), 32 above, 64 from 32,768 on (8192 rows over 5,700 tokens:
+        // 528 us with 64, 617 with 32; 4096 rows: 290, 272)
+        const int64_t units = (int64_t)gx * tiles;
+        auto launch = [&](auto nt, auto fm) {
+            constexpr int NT = decltype(nt)::value;
+            constexpr bool F = decltype(fm)::value;
+            constexpr size_t lds = 2 * tile_stage_bytes<NT>();
+            static const bool ok = hipFuncSetAttribute((const void*)q8_tile_k<NT, F>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
+            if (!ok) {
+                (void)hipGetLastError();
+                return false;
+            }
+            hipLaunchKernelGGL((q8_tile_k<NT, F>), dim3(gx, (tiles + NT - 1) / NT), dim3(256), lds, s, wq, ws, act_quants, act_scales, out, w.n_in,
+                               w.n_out, n_tok, out_scale);
+            return true;
+        };
+        auto by_mode = [&](auto nt) { return fma ? launch(nt, std::true_type{}) : launch(nt, std::false_type{}); };
+        using std::integral_constant;
+        if (units <= 640 ? by_mode(integral_constant<int, 1>{}) : units <= 32768 ? by_mode(integral_constant<int, 2>{}) : by_mode(integral_constant<int, 4>{}))
+            return true;
+    }
     // 64 tokens per block at most: four blocks fit a CU (38 KB of LDS, 98 VGPRs) and hide each other's LDS and
     // barrier waits; 128 tokens per block (two blocks per CU) measured 20 % slower despite reading the weights half as often
     // ... unless that leaves fewer than two blocks per CU (a short batch, few rows): then narrower blocks, which re-read

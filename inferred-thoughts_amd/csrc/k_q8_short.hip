@@ -1,8 +1,8 @@
 // Dense Q8_0 products of a short batch on the int8 matrix cores (fast mode).
 //
-// The tiles of k_gemm.hip walk the k range slab by slab, each slab a round trip through LDS: sixteen or more of them in a row,
-// 18 to 32 us for matrices whose bytes take 2 us and whose arithmetic takes one.  Here the k range is cut over the waves of a
-// block and every wave asks at once for all it will read, 16 RT weight rows and 32 tokens of its 256 (or twice 256) k, straight
+// The tiles of k_gemm.hip walk the k range slab by slab, a round trip through LDS each, for matrices whose bytes take 2 us and
+// whose arithmetic takes one.  Here the k range is cut over the waves of a
+// block and every wave asks at once for all it will read, 16 RT weight rows and up to 32 tokens of its 256 (or 512) k, straight
 // into registers: one trip to memory.  The waves' sums meet in LDS behind one barrier.
 // The products are those of k_gemm.hip (an exact int32 sum per 32 terms, scaled and added in f32 with one rounding); the f32
 // sums of the waves are added at the end instead of one running over the whole row.
@@ -32,7 +32,7 @@ __global__ __launch_bounds__(64 * KW) void q8_short_k(const int8_t* __restrict__
     const int lane = threadIdx.x & 63;
     const int kw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
-    const int row0 = blockIdx.x * 16 * RT, t0 = blockIdx.y * 32;
+    const int row0 = blockIdx.x * 16 * RT;
 
     // everything this wave reads, asked for at once: its part of the weight rows, of the tokens, and their scales (the
     // weights' for the four rows that a lane receives)
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(64 * KW) void q8_short_k(const int8_t* __restrict__
         }
 #pragma unroll
         for (int t = 0; t < 2; t++) {
-            const int64_t tok = min(t0 + 16 * t + r, n_tok - 1);
+            const int64_t tok = min(16 * t + r, n_tok - 1);
             const int8_t* p = xq + tok * n_in + k + g * 8;
 #pragma unroll
             for (int b = 0; b < 8; b++) x[u][t][b] = *(const long*)(p + b * 32);
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * KW) void q8_short_k(const int8_t* __restrict__
             const float4 v = red[k][c][lane];
             s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
         }
-        const int tok = t0 + 16 * (c / RT) + r, row = row0 + 16 * (c % RT) + 4 * g;
+        const int tok = 16 * (c / RT) + r, row = row0 + 16 * (c % RT) + 4 * g;
         if (tok >= n_tok) continue;
         s.x *= out_scale; s.y *= out_scale; s.z *= out_scale; s.w *= out_scale;
         float* o = out + (int64_t)tok * n_out + row;
@@ -114,16 +114,14 @@ bool q8_short(const WView& w, const float* act_scales, const int8_t* act_quants,
     if (w.fmt != W_Q8_0 || n_tok < 2 || w.n_out < 1 || w.n_in % 256 || (kw != 1 && kw != 2 && kw != 4 && kw != 8 && kw != 16)) return false;
     auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     if (!al16(w.q) || !al16(w.scales) || !al16(act_quants) || !al16(act_scales) || !al16(out)) return false;
-    // Up to 256 blocks of 32 rows and 32 tokens, one a CU (8192 x 2048 over 32 tokens: 15.5 against 20.3 us as tiles of k_gemm.hip,
-    // over 64: 25.5 against 22.9; 2048 x 4096 over 128: 23.9 against 32.5); half as many leave room for blocks of 16 rows.
-    const int pairs = (n_tok + 31) / 32;
-    const int64_t units = (int64_t)((w.n_out + 31) / 32) * pairs;
-    if (units > 256) return false;
+    // Up to 32 tokens and a block of 32 rows per CU; half as many leave room for blocks of 16 rows.  (The tiles of k_gemm.hip
+    // are 1 to 2 us behind at 16 tokens, level at 32 and ahead above.)
+    if (n_tok > 32 || w.n_out > 8192) return false;
+    const int rt = w.n_out > 4096 ? 2 : 1;
     // below 16 tokens against one GEMV each: from 16,384 results on (4096 rows: 9.1 against 9.7 us for 3 tokens, 9.0 against 12.6
     // for 5; 512 rows: behind, 9.0 against 7.1 for 12)
     if (n_tok < 16 && (int64_t)n_tok * w.n_out < 16384) return false;
-    const int rt = units > 128 ? 2 : 1;
-    const dim3 grid((w.n_out + 16 * rt - 1) / (16 * rt), pairs), block(64 * std::min(kw, 8));
+    const dim3 grid((w.n_out + 16 * rt - 1) / (16 * rt)), block(64 * std::min(kw, 8));
 #define IT_QS(KW, U)                                                                                                                  \
     do {                                                                                                                              \
         if (rt == 2) hipLaunchKernelGGL((q8_short_k<KW, U, 2>), grid, block, 0, s, (const int8_t*)w.q, (const uint16_t*)w.scales,     \

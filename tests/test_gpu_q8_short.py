@@ -32,3 +32,34 @@ def test_short_batches(n_in, n_out, n):
             assert np.abs(a[s] - b[s]).max() <= 1e-5 * np.abs(b[s]).max(), (t, np.abs(a[s] - b[s]).max(), np.abs(b[s]).max())
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("exact", [True, False])
+@pytest.mark.parametrize("n_in,n_out,n", [(256, 64, 33), (512, 130, 40), (2048, 8192, 70), (2048, 8192, 100), (2048, 514, 1300),
+                                          (4096, 2046, 65), (256, 8192, 4200), (2048, 66, 17)])
+def test_tiles_over_whole_slabs(exact, n_in, n_out, n):
+    """q8_tile_k (k_gemm.hip): one to sixteen stages, the three token widths of a block with ragged ends; exact mode keeps the
+    oracle's bits."""
+    import inferred_hip as ih
+    from oracle import binding as ob
+    orc = ob.Oracle(threads=8)
+    be = ih.Hip(exact=exact)
+    try:
+        r = rng(n_in + n_out + n)
+        w = q8_0_weights(orc, r, n_out, n_in, std=0.05)
+        x = (r.standard_normal(n * n_in) * np.repeat(10.0 ** r.uniform(-2, 2, n), n_in)).astype(np.float32)
+        a = np.zeros(n * n_out, np.float32)
+        be.matmul(ih.weights(w, ih.Q8_0, n_in, n_out), x, a)
+        be.host_needs(a)
+        be.raise_if_error()
+        rows = np.unique(np.r_[0:3, n // 2, n - 18:n])          # the oracle on the edges of the tiles
+        xs = np.ascontiguousarray(x.reshape(n, n_in)[rows]).reshape(-1)
+        b = np.zeros(len(rows) * n_out, np.float32)
+        orc.matmul(ob.weights(w, ih.Q8_0, n_in, n_out), xs, b)
+        got, want = a.reshape(n, n_out)[rows], b.reshape(len(rows), n_out)
+        if exact:
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        else:
+            assert (np.abs(got - want).max(1) <= 1e-5 * np.abs(want).max(1)).all()
+    finally:
+        be.close()
