@@ -69,6 +69,14 @@ IT_DEV h8v fp4x8_to_f16x8(uint32_t w, h2 scale) {
     return h8v{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
+typedef __attribute__((address_space(3))) void* lptr;
+// 16 bytes a lane from memory to LDS, one lane's behind the other's from `to` on (the same in every lane).  Written out because
+// the compiler's own form makes every later read of LDS wait for all such loads; here they are waited for by count, in front
+// of the barrier of the stage that reads them.
+IT_DEV void to_lds(const void* from, uint32_t to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(from) : "memory");
+}
+
 // operands of the f16 expert tile kernels (k_gemm_f16.hip, k_gemm_f16s.hip)
 struct ExpertsF16P {
     const uint8_t *q, *s, *q2, *s2;

@@ -154,15 +154,7 @@ __global__ __launch_bounds__(GT) void q8_gemm_k(const int8_t* __restrict__ wq, c
 // Not kept: three or four stages (0 to 50 % slower everywhere: fewer blocks fit a CU); the f16 matrix cores with the
 // activations as an f16 pair and no scale per token, 128 x 256 tiles (8192 x 2048 over 5,700: 437 us with three stages, 46 % of
 // the rate the matrix cores sustain, but 20 % behind on everything smaller).
-typedef __attribute__((address_space(3))) void* lptr;
 typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
-
-// 16 bytes a lane from memory to LDS, one lane's behind the other's from `to` on (the same in every lane).  Written out because
-// the compiler's own form makes every later read of LDS wait for all such loads; here they are waited for by count, in front
-// of the barrier of the stage that reads them.
-IT_DEV void to_lds(const void* from, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(from) : "memory");
-}
 
 template <int NT> constexpr int tile_stage_bytes() { return 64 * 256 + NT * 16 * 256 + 1024 + (NT > 2 ? 2048 : 1024); }
 

@@ -180,14 +180,23 @@ __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
 // waves of a row set take one 256-wide chunk EACH (n_in = 256 KW, KW = 1, 2, 4 or 8) and walk the same row groups
 // together: the block reads whole rows at a time, a wave's B operands are loaded once for the whole kernel, and both
 // matrices of the gate/up pair share them.  The price is a reduction of the KW partial sums of every 16 x 16 tile
-// through LDS: a batch of four tiles per wave (two row groups of gate and up, or four of one matrix), one barrier per
-// batch, two LDS buffers in turn.
+// through LDS, a batch of two tiles per wave at a time (a row group of gate and up, or two of one matrix).
+//
+// Bound by the stream of the touched experts' nibbles.  A wave brings a step (16 rows of its chunk, 2 KB; the scales of two
+// steps with every second one) straight into a ring of its own in LDS, two to three steps ahead: no register waits on
+// memory, no other wave is waited for, and a row's 128-byte line is one request.  (With one step ahead in registers, two
+// requests a line: 4.5 TB/s of the 6.7 to 8 that such reads reach.)  A load writes its lanes' 16 bytes side by side, so a
+// row's eight pieces are permuted by the row's number and sixteen rows' reads meet every bank once.
+constexpr int SK_RING = 3;
+constexpr int SK_WAVE_LDS = SK_RING * 2048 + 2 * 512;     // a wave's steps and scales
+
 template <bool GLU, int KW>
-__global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches_per_block) {
+__global__ __launch_bounds__(512, 4) void experts_f16k_k(ExpertsF16P p, int batches_per_block) {
     constexpr int NM = GLU ? 2 : 1;
-    constexpr int GB = 4 / NM;        // row groups per batch
+    constexpr int GB = 2 / NM;        // row groups per batch
     constexpr int RS = 8 / KW;        // row sets per block
-    __shared__ float4 red[2][8][4][64];   // [buffer][wave][tile of the batch][lane]
+    __shared__ float4 red[8][2][64];  // [wave][tile of the batch][lane]
+    __shared__ __align__(16) uint8_t ring[8 * SK_WAVE_LDS];
     const int tile = blockIdx.x;
     if (tile >= n_tiles_of(p, SK_PAIRS)) return;
     const int4 td = tile_of(p, tile, SK_PAIRS);
@@ -204,34 +213,24 @@ __global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches
     const uint8_t* wq[2] = {it_expert_at(p.q, p.q_tab, e, p.q_stride), GLU ? it_expert_at(p.q2, p.q2_tab, e, p.q_stride) : nullptr};
     const uint8_t* ws[2] = {it_expert_at(p.s, p.s_tab, e, p.s_stride), GLU ? it_expert_at(p.s2, p.s2_tab, e, p.s_stride) : nullptr};
 
-    // step st = batch i, group slot j, matrix z of this wave: i = st / 4, (j, z) = st % 4
-    const int n_steps = batches_per_block * 4;
-    auto group_of = [&](int st) { return ((blockIdx.y * batches_per_block + st / 4) * RS + rs) * GB + (st % 4) / NM; };
-    // (the matrix z is passed as a constant of the unrolled code: a pointer picked by a run-time index stops being a
-    // global pointer for the compiler, and its loads become flat loads that every wait has to drain)
-    auto load_step = [&](int st, int z) __attribute__((always_inline)) -> RawW {
-        RawW o;
-        const int64_t row = min(group_of(st) * 16 + r16, p.n_out - 1);
-        // units 2 kg and 2 kg + 1 of the chunk: the four lanes of a row read its 128-byte line between them, and a
-        // lane's four scale bytes are one load (two-byte loads, eight bytes per row, cost a quarter of the stream's time)
-        const int u = 8 * kw + 2 * kg;
-        o.nib[0] = *(const uint4*)(wq[z] + row * (n_in >> 1) + u * 16);
-        o.nib[1] = *(const uint4*)(wq[z] + row * (n_in >> 1) + u * 16 + 16);
-        o.sc[0] = *(const uint32_t*)(ws[z] + row * (n_in >> 4) + u * 2);   // unit 2 kg in the low half, 2 kg + 1 above
-        o.sc[1] = 0;
-        return o;
+    // step st = batch st / 2, tile st % 2 of it: a row group's gate, then up rows, or two row groups
+    const int n_steps = batches_per_block * 2;
+    auto group_of = [&](int st) { return ((blockIdx.y * batches_per_block + st / 2) * RS + rs) * GB + (GLU ? 0 : st & 1); };
+    uint8_t* const mine = ring + wave * SK_WAVE_LDS;
+    const uint32_t mine_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)mine);
+    auto ask = [&](int st, int slot, int z) __attribute__((always_inline)) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int r = 8 * h + (lane >> 3), row = min(group_of(st) * 16 + r, p.n_out - 1);
+            to_lds(wq[z] + (int64_t)row * (n_in >> 1) + kw * 128 + (((lane & 7) ^ ((r >> 1) & 7)) << 4), mine_at + slot * 2048 + h * 1024);
+        }
     };
-    // Four register sets, one per step of a batch: step t computes from set t while the load of step t + 3 goes
-    // straight into set (t + 3) % 4.  No set is ever copied (a copy of a load's destination waits for the load) and
-    // the load is unconditional (past the end it repeats the last step), so the compiler's wait before a step counts
-    // exactly the loads issued after the ones it needs.
-    constexpr int QD = GLU ? 2 : 4;
-    RawW q[QD];
-    q[0] = load_step(0, 0);
-    if (QD == 4) {
-        q[1] = load_step(1, GLU ? 1 : 0);
-        q[2] = load_step(2, 0);
-    }
+    auto ask_scales = [&](int i) __attribute__((always_inline)) {     // of batch i: lanes 0 .. 15 its first tile's rows, 16 .. 31 its second's
+        if (lane < 32) {
+            const int row = min(group_of(2 * i + (lane >> 4)) * 16 + r16, p.n_out - 1);
+            to_lds((GLU && lane >= 16 ? ws[1] : ws[0]) + (int64_t)row * (n_in >> 4) + kw * 16, mine_at + SK_RING * 2048 + (i & 1) * 512);
+        }
+    };
     // this wave's B operands: chunk kw of the tile's 16 pairs, for the whole kernel
     h8 fh[8], fl[8];
     {
@@ -246,30 +245,55 @@ __global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches
     const float rsc = p.rscale[xrow];
     const float e2a = p.scale2 ? p.scale2[e] : p.scale_a;
     const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : p.scale_b) : e2a;
+    // (in the order of their use: what a step waits for is older than the five loads that may be out behind it)
+    ask_scales(0);
+    ask(0, 0, 0);
+    ask(1, 1, NM - 1);
+    if (batches_per_block > 1) {
+        ask_scales(1);
+        ask(2, 2, 0);
+    }
 
+    int slot = 0;
     for (int i = 0; i < batches_per_block; i++) {
-        const int buf = i & 1;
+        float4 part[2];
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int st = 4 * i + t;
-            q[(t + QD - 1) % QD] = load_step(min(st + QD - 1, n_steps - 1), GLU ? (t + QD - 1) & 1 : 0);
-            __builtin_amdgcn_sched_barrier(0);   // the loads stay ahead of the step they overlap
+        for (int t = 0; t < 2; t++) {
+            const int st = 2 * i + t;
+            // the step has landed: behind it two steps of two loads and one of scales may be out
+            if (st + 3 <= n_steps) __builtin_amdgcn_s_waitcnt(0x0f75);
+            else __builtin_amdgcn_s_waitcnt(0x0f70);
+            asm volatile("" ::: "memory");
+            const uint8_t* const d = mine + slot * 2048 + r16 * 128;
+            const uint4 n0 = *(const uint4*)(d + (((2 * kg) ^ ((r16 >> 1) & 7)) << 4)), n1 = *(const uint4*)(d + (((2 * kg + 1) ^ ((r16 >> 1) & 7)) << 4));
+            const uint32_t sc = *(const uint32_t*)(mine + SK_RING * 2048 + (i & 1) * 512 + (16 * t + r16) * 16 + 4 * kg);
+            __builtin_amdgcn_s_waitcnt(0xc07f);     // (read: the slot may be filled again)
+            asm volatile("" ::: "memory");
+            if (st + 3 < n_steps) ask(st + 3, slot, GLU ? (t + 1) & 1 : 0);
+            if (t == 1 && i + 2 < batches_per_block) ask_scales(i + 2);
+            slot = slot == SK_RING - 1 ? 0 : slot + 1;
             v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int n = 0; n < 8; n++) {
-                const h8 a = expand_frag(q[t % QD].nib[n >> 2], n < 4 ? q[t % QD].sc[0] : q[t % QD].sc[0] >> 16, n & 3);
+                const h8 a = expand_frag(n < 4 ? n0 : n1, n < 4 ? sc : sc >> 16, n & 3);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, fh[n], acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, fl[n], acc, 0, 0, 0);
             }
-            red[buf][wave][t][lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            part[t] = make_float4(acc[0], acc[1], acc[2], acc[3]);
         }
-        __syncthreads();
+        if (i) __builtin_amdgcn_s_barrier();      // (the last batch's sums have been read)
+        asm volatile("" ::: "memory");
+        red[wave][0][lane] = part[0];
+        red[wave][1][lane] = part[1];
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();             // (not __syncthreads: the loads ahead stay out)
+        asm volatile("" ::: "memory");
         // group slot j of the batch is finished by the wave kw == j % KW of its row set: the KW partial sums of its
         // tile (of both tiles for the gate/up pair), the epilogue and the store
 #pragma unroll
         for (int j = 0; j < GB; j++) {
             if (j % KW != kw) continue;
-            const int g = group_of(4 * i + j * NM);
+            const int g = group_of(2 * i + j * NM);
             const int row = g * 16 + 4 * kg;
             if (g >= n_groups || row >= p.n_out || r16 >= cnt) continue;
             float sum[NM][4];
@@ -278,7 +302,7 @@ __global__ __launch_bounds__(512) void experts_f16k_k(ExpertsF16P p, int batches
                 sum[z][0] = sum[z][1] = sum[z][2] = sum[z][3] = 0.0f;
 #pragma unroll
                 for (int k = 0; k < KW; k++) {
-                    const float4 v = red[buf][rs * KW + k][j * NM + z][lane];
+                    const float4 v = red[rs * KW + k][j * NM + z][lane];
                     sum[z][0] += v.x; sum[z][1] += v.y; sum[z][2] += v.z; sum[z][3] += v.w;
                 }
             }
@@ -349,12 +373,13 @@ bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_
     const int groups = (w.n_out + 15) / 16;
     const int likely_tiles = ids ? std::min(n_picks, w.n_expert) + n_picks / SK_PAIRS : max_tiles;
     const int n_chunk = w.n_in / SK_KC;
-    if (n_chunk == 1 || n_chunk == 2 || n_chunk == 4 || n_chunk == 8) {
-        // k split over the waves: a batch is 4 / NM row groups per row set, 8 / n_chunk row sets per block; 8 batches
-        // per block while that leaves about 1,024 blocks (16 or 32 batches measured 10 % slower, 4 the same)
-        const int per_batch = (up ? 2 : 4) * (8 / n_chunk);
+    const bool scales16 = w.s_stride % 16 == 0 && !(reinterpret_cast<uintptr_t>(w.scales) & 15) && !(up && (reinterpret_cast<uintptr_t>(up->scales) & 15));
+    if (scales16 && (n_chunk == 1 || n_chunk == 2 || n_chunk == 4 || n_chunk == 8)) {
+        // k split over the waves: a batch is 2 / NM row groups per row set, 8 / n_chunk row sets per block; 16 batches
+        // per block while that leaves about 1,024 blocks
+        const int per_batch = (up ? 1 : 2) * (8 / n_chunk);
         const int batches = (groups + per_batch - 1) / per_batch;
-        int bpb = std::min(batches, 8);
+        int bpb = std::min(batches, 16);
         while (bpb > 1 && (int64_t)likely_tiles * ((batches + bpb - 1) / bpb) < 1024) bpb >>= 1;
         const dim3 grid(std::min(n_picks, max_tiles), (batches + bpb - 1) / bpb);
 #define IT_F16K(G, K) hipLaunchKernelGGL((experts_f16k_k<G, K>), grid, dim3(512), 0, s, p, bpb)
