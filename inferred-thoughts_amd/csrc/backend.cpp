@@ -1566,8 +1566,9 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     const int exact = be->exact;
     // A dense NVFP4 matrix over a batch (the shared expert of an NVFP4 file) has no int8 tile kernel of its own; in fast mode
     // it runs on the f16 tile kernels of the experts, as one of them:
-    //   128 .. 1,024 tokens: tiles of 16 (2048 x 512 over 1,024 tokens: 34 against 68 us on the 128-wide tiles, whose handful
-    //     of blocks is latency-bound there; 16 against 19 us of GEMVs at 128 tokens)
+    //   33 .. 1,024 tokens: tiles of 16 (2048 x 512 over 1,024 tokens: 34 against 68 us on the 128-wide tiles, whose handful
+    //     of blocks is latency-bound there; with a GEMV per token two layers' pass of 34 tokens takes 560 us instead of 513, of
+    //     120 tokens 827 instead of 732)
     //   above: tiles of 128 (82 against 736 us of GEMVs at 5,700 tokens)
     //   128 .. 512 tokens of a shape that the tiles do not take: eight or sixteen tokens per pass over the rows
     //     (k_moe_rows.hip; 32 against 70 us for 2048 x 512 at 512 tokens)
@@ -1579,7 +1580,7 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     bool grouped = false;
     int tiles = 0;   // 1: tiles of 16, 2: tiles of 128
     SplitOut sp;
-    if (!exact && v.fmt == W_NVFP4 && n >= 128) {
+    if (!exact && v.fmt == W_NVFP4 && n > 32) {
         tiles = n <= 1024 ? (itk::experts_f16s_takes(ev, nullptr, nt, dout) ? 1 : 0) : (itk::experts_f16_takes(ev, nullptr, nt, dout) ? 2 : 0);
         if (tiles && !be->act_split(x, x_len, v.n_in, &sp)) return;
     }
@@ -1936,15 +1937,17 @@ static bool host_ids_in_range(it_hip* be, const it_route* r, uint64_t n_expert, 
 // against 772 us tiled; at 256 tokens it is 1,180 against 848).
 static bool expert_tiles_pay(uint64_t picks, uint64_t n_expert) { return picks >= 32 && 2 * picks >= 7 * n_expert; }
 // Fast mode between the per-pair GEMVs and the wide matrix-core tiles, measured on the 512-expert top-10 FFN (hidden
-// 2048, inter 512): from 1.25 pairs per expert on, grouping the pairs by expert beats one GEMV per pair; NVFP4 then
-// runs 16-pair tiles on the f16 matrix cores (k_gemm_f16s.hip) up to 48 pairs per expert (2,048 tokens: 961 against
-// 1,017 us for the whole FFN; 4,096 tokens: 1,571 against 1,447), where the 128-pair tiles take over; what that kernel does not take (Q8_0, odd shapes) streams each expert's rows once for all its pairs
-// (k_moe_rows.hip) until the int8 tiles pay.
+// 2048, inter 512).  NVFP4 runs 16-pair tiles on the f16 matrix cores (k_gemm_f16s.hip): level with the per-pair kernels at
+// 40 pairs (four tokens: 307 against 314 us for two layers' whole pass), ahead behind (40 tokens: 574 against 699, 63: 664
+// against 893; up to 32 tokens the FFN is two launches of its own, fuser.cpp), up to 48 pairs per expert (2,048 tokens: 961
+// against 1,017 us for the whole FFN; 4,096 tokens: 1,571 against 1,447), where the 128-pair tiles take over.  What that kernel
+// does not take (Q8_0, odd shapes) streams each expert's rows once for all its pairs (k_moe_rows.hip) from 1.25 pairs per
+// expert on, until the int8 tiles pay.
 static bool expert_grouping_pays(const it_hip* be, uint64_t picks, uint64_t n_expert) {
     return !be->exact && picks >= 32 && 4 * picks >= 5 * n_expert;
 }
 static bool expert_skinny_pay(const it_hip* be, uint64_t picks, uint64_t n_expert) {
-    return expert_grouping_pays(be, picks, n_expert) && picks < 48 * n_expert;
+    return !be->exact && picks >= 32 && picks < 48 * n_expert;
 }
 static bool expert_rows_pay(const it_hip* be, uint64_t picks, uint64_t n_expert) {
     return expert_grouping_pays(be, picks, n_expert) && !expert_tiles_pay(picks, n_expert);
