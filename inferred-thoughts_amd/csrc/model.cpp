@@ -360,7 +360,9 @@ void moe_batch(it_engine* e, const Block& b, uint64_t at, uint64_t n, uint64_t t
     it_hip_silu_mul(be, e->e_gate.p(), sff, e->e_up.p(), sff);
     it_hip_matmul(be, &b.sh_down, e->e_gate.p(), sff, e->e_out.p(), n * nd);
     if (b.sh_has[2]) it_hip_scale(be, e->e_out.p(), n * nd, b.sh_scale[2]);
-    it_hip_moe_finish(be, e->ffn_out.p(), total * nd, at, nd, e->o_all.p(), pairs * nd, &route, e->e_out.p(),
+    // (the rows so far, not the whole buffer: a part of one that the device does not hold yet would bring the rest of it
+    // from the host first; 64 MiB and 2.2 ms in front of each pass of 8,192 tokens)
+    it_hip_moe_finish(be, e->ffn_out.p(), at + n * nd, at, nd, e->o_all.p(), pairs * nd, &route, e->e_out.p(),
                       n * nd, e->shexp_logit.p(), n, 0);
 }
 
