@@ -6,8 +6,8 @@
 // in the CPU path's order.
 //
 // A block owns 128 query rows of one KV head: 128 / G tokens x the G query heads that share the head.
-// It walks the keys in tiles of 64; a tile's K (as stored, f16 [key][dim]) and V (transposed on the
-// way in, [dim][key]) are staged in LDS once for all 128 rows.  Each wave owns 32 rows and forms
+// It walks the keys in tiles of 64; a tile's K and V are brought to LDS as stored ([key][dim], f16) by loads that go
+// straight there, two tiles of each, and serve all 128 rows.  Each wave owns 32 rows and forms
 //     S^T = K Q^T   (32 keys x 32 queries per MFMA tile, A = K from LDS, B = Q from registers)
 //     O^T = V^T P^T (32 dims x 32 queries per MFMA tile, A = V^T from LDS, B = P from registers)
 // so a lane holds, for ITS query (column l % 32), 16 of the 32 keys of a score tile and 16 of the 32
@@ -15,13 +15,17 @@
 // the lane (one exchange with lane l ^ 32), and the probabilities go from the score accumulators
 // to the next MFMA's B operand without leaving the registers (the k order of an MFMA is free as
 // long as both operands agree: lane group g's eight probabilities of step j are keys
-// 16 j + 4 g + {0..3} and 8 more, and V^T is read at those keys).
+// 16 j + 4 g + {0..3} and 8 more; V is read at those keys by the transposing LDS read, which gives
+// lane i of 16 four keys' value of column i).
+// The rows of 2 * HD bytes lie whole in LDS; which 16-byte piece of a row lies where is turned by the row, for K so that
+// rows read together hit different banks, for V so that eight keys' 64-byte blocks do (swap_k, swap_v).
 // The query is scaled by scale * log2(e) and split into an f16 pair (hi + lo, 22 bits kept); K, V
 // are f16 in the cache; probabilities are rounded to f16 (relative 2^-11 each, unbiased).
 //
 // MFMA operand layout (32x32x16, f16): lane l supplies 8 k values of row (l % 32), k group l / 32,
 // for A and for B; it receives D for column l % 32 and rows 8 * (i / 4) + 4 * (l / 32) + i % 4.
 #include "it_device.h"
+#include "it_dot.h"
 #include "kernels.h"
 
 namespace itk {
@@ -29,22 +33,45 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-constexpr int KT = 64;       // keys per tile
-constexpr int VS = KT + 4;   // row stride of V^T in LDS, in f16 (136 bytes)
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4 ls4;
+typedef __attribute__((address_space(3))) uint8_t* lptr;
+constexpr int KT = 64;          // keys per tile
+constexpr float GROW = 8.0f;    // the running maximum follows when the scores pass it by more than this (log2): probabilities stay below 2^8
 
+// the 16-byte piece of row `key` that lies at piece p of its row in LDS (and the other way round)
+template <int HD>
+IT_DEV int swap_k(int key) { return HD >= 128 ? key & 15 : (key >> 1) & 7; }
+template <int HD>
+IT_DEV int swap_v(int key) { return HD == 256 ? (key & 7) << 2 : HD == 128 ? (key & 3) << 2 : ((key >> 1) & 1) << 2; }
+
+// formed here, not later where it is first read
+IT_DEV void here(float& x, h8& v) {
+    uint4 t = __builtin_bit_cast(uint4, v);
+    asm volatile("" : "+v"(x), "+v"(t.x), "+v"(t.y), "+v"(t.z), "+v"(t.w));
+    v = __builtin_bit_cast(h8, t);
+}
+
+template <int V>
+struct Is { static constexpr int value = V; };
+
+// What bounds it: the matrix cores' instructions (96 per wave and tile at head_dim 256: 64 for the scores, the query being a
+// pair, 32 for the values), with one wave on each SIMD, since a row's query pair and sums take about 300 registers.  So
+// nothing else may stand between them: the softmax of a tile runs in the shadow of the next tile's scores, a tile's loads
+// are asked for one tile ahead, and there is one barrier per tile.  5,700 queries, 16 heads of 256 on 2: 0.42 ms, 960 TFLOP/s
+// as issued (0.68 ms when a tile was fetched through registers, V turned on its way into LDS, and softmax and products
+// took turns between two barriers); 30,000 in four batches: 10.3 ms (16.9).
 template <int HD, int G>
 __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __restrict__ out) {
     constexpr int QT = 128 / G;                     // tokens per block
-    constexpr int KS = HD + 8;                      // row stride of K in LDS, in f16
     constexpr int NS = HD / 16;                     // k steps of a score tile
     constexpr int ND = HD / 32;                     // output tiles along the head dimension
-    constexpr int KSEG = KT * HD / 8 / 256;         // 16-byte pieces of K per thread
-    constexpr int UNITS = (KT / 4) * (HD / 8);      // 4-key x 8-dim pieces of V per tile
-    constexpr int VU = (UNITS + 255) / 256;         // per thread
-    extern __shared__ __align__(16) uint16_t lds[];
-    uint16_t* Ks = lds;                // [64][KS]
-    uint16_t* Vt = lds + KT * KS;      // [HD][VS]
-    uint16_t* Ql = Vt + HD * VS;       // [128][KS]: the low halves of the query rows (registers are short)
+    constexpr int P = HD / 8;                       // 16-byte pieces of a row
+    constexpr int NL = HD / 32;                     // loads of a wave per tile of K, and of V (1,024 bytes each)
+    constexpr int RL = 512 / HD;                    // rows of one
+    constexpr int TILE = KT * HD * 2;               // bytes
+    constexpr int V_AT = 2 * TILE;
+    extern __shared__ __align__(1024) uint8_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 31, g = lane >> 5;
     const int n_qt = (a.n_q + QT - 1) / QT;
@@ -57,8 +84,34 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
     const int pos = valid ? base_pos + token : 0x7fffffff;
     const int qdim = a.n_head * HD;
 
+    const int first_pos = base_pos + qt * QT;                            // smallest position of the block
+    const int last_pos = base_pos + min(a.n_q, (qt + 1) * QT) - 1;       // largest
+    const int n_kt = last_pos / KT + 1;
+    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)lds);
+
+    const int lrow = w * 16 + lane / P;             // this lane's row of the wave's first load
+    auto ask_k = [&](int kt, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int key = lrow + i * RL;
+            const uint16_t* from = a.k + kvh * HD + (int64_t)min(kt * KT + key, a.n_pos - 1) * a.kv_dim + 8 * ((lane % P) ^ swap_k<HD>(key));
+            to_lds(from, at + buf * TILE + (w * NL + i) * 1024);
+        }
+    };
+    auto ask_v = [&](int kt, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NL; i++) {
+            const int key = lrow + i * RL;
+            const uint16_t* from = a.v + kvh * HD + (int64_t)min(kt * KT + key, a.n_pos - 1) * a.kv_dim + 8 * ((lane % P) ^ swap_v<HD>(key));
+            to_lds(from, at + V_AT + buf * TILE + (w * NL + i) * 1024);
+        }
+    };
+    ask_k(0, 0);
+    ask_v(0, 0);
+    ask_k(1, 1);                                    // (past the end: the last key again, never read)
+
     // this lane's query row, scaled, as an f16 pair
-    h8 qh[NS];
+    h8 qh[NS], ql[NS];
     {
         const float qs = a.scale * 1.4426950408889634f;
         const float* qrow = a.q + (int64_t)min(token, a.n_q - 1) * qdim + head * HD + 8 * g;
@@ -66,74 +119,30 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
         for (int s = 0; s < NS; s++) {
             const float4 x0 = *(const float4*)(qrow + 16 * s), x1 = *(const float4*)(qrow + 16 * s + 4);
             const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            h8 lo;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const float v = valid ? x[e] * qs : 0.0f;
                 const _Float16 hi = (_Float16)v;
                 qh[s][e] = hi;
-                lo[e] = (_Float16)(v - (float)hi);
+                ql[s][e] = (_Float16)(v - (float)hi);
             }
-            *(h8*)(Ql + row * KS + 16 * s + 8 * g) = lo;   // read back by this lane only
         }
     }
 
-    const int first_pos = base_pos + qt * QT;                            // smallest position of the block
-    const int last_pos = base_pos + min(a.n_q, (qt + 1) * QT) - 1;       // largest
-    const int n_kt = last_pos / KT + 1;
-    const uint16_t* kbase = a.k + kvh * HD;
-    const uint16_t* vbase = a.v + kvh * HD;
-
-    uint4 rk[KSEG], rv[VU][4];
-#pragma unroll
-    for (int p = 0; p < KSEG; p++) rk[p] = make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int u = 0; u < VU; u++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) rv[u][c] = make_uint4(0, 0, 0, 0);
-    auto fetch = [&](int kt) __attribute__((always_inline)) {
-#pragma unroll
-        for (int p = 0; p < KSEG; p++) {
-            const int idx = tid + p * 256, key = idx / (HD / 8), seg = idx % (HD / 8);
-            const int64_t gk = min(kt * KT + key, a.n_pos - 1);
-            rk[p] = *(const uint4*)(kbase + gk * a.kv_dim + seg * 8);
-        }
-#pragma unroll
-        for (int u = 0; u < VU; u++) {
-            const int unit = tid + u * 256, ka = unit % (KT / 4), b = unit / (KT / 4);   // 16 key groups across lanes: the transposed LDS writes of a wave hit every bank once
-            if (unit < UNITS) {
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const int64_t gk = min(kt * KT + 4 * ka + c, a.n_pos - 1);
-                    rv[u][c] = *(const uint4*)(vbase + gk * a.kv_dim + 8 * b);
-                }
-            }
-        }
+    const uint8_t* const k_row = lds + r * HD * 2;
+    const int k_swap = g ^ swap_k<HD>(r);           // piece 2 s + g of row r (and of row r + 32)
+    auto k_frag = [&](int buf, int s, int kk) __attribute__((always_inline)) {
+        return *(const h8*)(k_row + buf * TILE + kk * 32 * HD * 2 + (((2 * s) ^ k_swap) << 4));
     };
-    auto stash = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int p = 0; p < KSEG; p++) {
-            const int idx = tid + p * 256, key = idx / (HD / 8), seg = idx % (HD / 8);
-            *(uint4*)(Ks + key * KS + seg * 8) = rk[p];
-        }
-#pragma unroll
-        for (int u = 0; u < VU; u++) {
-            const int unit = tid + u * 256, ka = unit % (KT / 4), b = unit / (KT / 4);   // 16 key groups across lanes: the transposed LDS writes of a wave hit every bank once
-            if (unit >= UNITS) continue;
-            const uint32_t x[4][4] = {{rv[u][0].x, rv[u][0].y, rv[u][0].z, rv[u][0].w},
-                                      {rv[u][1].x, rv[u][1].y, rv[u][1].z, rv[u][1].w},
-                                      {rv[u][2].x, rv[u][2].y, rv[u][2].z, rv[u][2].w},
-                                      {rv[u][3].x, rv[u][3].y, rv[u][3].z, rv[u][3].w}};
-#pragma unroll
-            for (int p = 0; p < 4; p++) {   // dims 8b + 2p (low halves) and 8b + 2p + 1 (high halves) of the four keys
-                const uint32_t lo0 = __builtin_amdgcn_perm(x[1][p], x[0][p], 0x05040100u);
-                const uint32_t lo1 = __builtin_amdgcn_perm(x[3][p], x[2][p], 0x05040100u);
-                const uint32_t hi0 = __builtin_amdgcn_perm(x[1][p], x[0][p], 0x07060302u);
-                const uint32_t hi1 = __builtin_amdgcn_perm(x[3][p], x[2][p], 0x07060302u);
-                *(uint2*)(Vt + (8 * b + 2 * p) * VS + 4 * ka) = make_uint2(lo0, lo1);
-                *(uint2*)(Vt + (8 * b + 2 * p + 1) * VS + 4 * ka) = make_uint2(hi0, hi1);
-            }
-        }
+    const int v_key = 4 * g + ((lane & 15) >> 2);   // key this lane names of the eight of a transposing read
+    const uint8_t* const v_row = lds + V_AT + v_key * HD * 2 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+    const int v_swap = swap_v<HD>(v_key) << 4;
+    auto v_frag = [&](int buf, int j, int dt) __attribute__((always_inline)) {
+        const uint8_t* const p = v_row + buf * TILE + 16 * j * HD * 2 + ((64 * dt) ^ v_swap);
+        const s4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)p);
+        const s4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((ls4*)(p + 8 * HD * 2));
+        typedef short s8 __attribute__((ext_vector_type(8)));
+        return __builtin_bit_cast(h8, s8(__builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7)));
     };
 
     v16f o[ND];
@@ -143,29 +152,9 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
         for (int i = 0; i < 16; i++) o[dt][i] = 0.0f;
     float m = -INFINITY, l = 0.0f;
 
-    fetch(0);
-    for (int kt = 0; kt < n_kt; kt++) {
-        stash();
-        __syncthreads();
-        if (kt + 1 < n_kt) fetch(kt + 1);
-
-        v16f sc[2];
-#pragma unroll
-        for (int kk = 0; kk < 2; kk++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) sc[kk][i] = 0.0f;
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-            const h8 qlo = *(const h8*)(Ql + row * KS + 16 * s + 8 * g);
-#pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
-                const h8 kf = *(const h8*)(Ks + (32 * kk + r) * KS + 16 * s + 8 * g);
-                sc[kk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qh[s], sc[kk], 0, 0, 0);
-                sc[kk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qlo, sc[kk], 0, 0, 0);
-            }
-            if ((s & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // a few fragments in flight: registers are short
-        }
-        if (kt * KT + KT - 1 > first_pos) {   // some row of the block cannot see the whole tile
+    // a row sees keys up to its own position
+    auto mask = [&](v16f (&sc)[2], int kt) __attribute__((always_inline)) {
+        if (kt * KT + KT - 1 > first_pos) {         // some row of the block cannot see the whole tile
 #pragma unroll
             for (int kk = 0; kk < 2; kk++)
 #pragma unroll
@@ -174,44 +163,120 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
                     if (key > pos) sc[kk][i] = -INFINITY;
                 }
         }
-        float mt = -INFINITY;
+    };
+
+    // Tile kt, whose scores are sc: its softmax, beside it (NEXT) tile kt + 1's scores to sn, then its values.
+    // B: the half of LDS that holds tile kt.
+    auto tile = [&](auto next, auto half, int kt, v16f (&sc)[2], v16f (&sn)[2]) __attribute__((always_inline)) {
+        constexpr bool NEXT = decltype(next)::value;
+        constexpr int B = decltype(half)::value;
+        __builtin_amdgcn_s_waitcnt(0x0f70);         // tile kt's V and tile kt + 1's K have landed (vmcnt 0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (NEXT) {                                 // (every wave is past tile kt's K and tile kt - 1's V)
+            ask_v(kt + 1, B ^ 1);
+            ask_k(kt + 2, B);
+        }
+        float mt = -INFINITY, alpha = 1.0f, psum = 0.0f;
+        h8 pf[4], kf[2][2], vf[2][4];
+        if (NEXT) {
+            kf[0][0] = k_frag(B ^ 1, 0, 0);
+            kf[0][1] = k_frag(B ^ 1, 0, 1);
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++)
+            for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int i = 0; i < 16; i++) mt = fmaxf(mt, sc[kk][i]);
-        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-        const float m_new = fmaxf(m, mt);   // finite from the first tile on: key 0 is visible to every row
-        const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-        float psum = 0.0f;
-        h8 pf[4];
+                for (int i = 0; i < 16; i++) sn[kk][i] = 0.0f;
+        }
 #pragma unroll
-        for (int kk = 0; kk < 2; kk++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const float p = __builtin_amdgcn_exp2f(sc[kk][i] - m_new);
-                psum += p;
-                pf[2 * kk + (i >> 3)][i & 7] = (_Float16)p;
+        for (int s = 0; s < NS; s++) {
+            if (NEXT) {
+                if (s + 1 < NS) {
+                    kf[(s + 1) & 1][0] = k_frag(B ^ 1, s + 1, 0);
+                    kf[(s + 1) & 1][1] = k_frag(B ^ 1, s + 1, 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                sn[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s & 1][0], qh[s], sn[0], 0, 0, 0);
+                sn[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s & 1][1], qh[s], sn[1], 0, 0, 0);
+                sn[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s & 1][0], ql[s], sn[0], 0, 0, 0);
+                sn[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[s & 1][1], ql[s], sn[1], 0, 0, 0);
             }
+            constexpr int NM = NS / 4, NE = NS / 2;     // steps that take the maximum, that form the probabilities
+            if (s < NM) {
+#pragma unroll
+                for (int e = s * (32 / NM); e < (s + 1) * (32 / NM); e++) mt = fmaxf(mt, sc[e >> 4][e & 15]);
+                if (s == NM - 1) {
+                    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+                    const float m_new = mt > m + GROW ? mt : m;   // finite from the first tile on: key 0 is visible to every row
+                    alpha = __builtin_amdgcn_exp2f(m - m_new);
+                    m = m_new;
+                }
+            } else if (s < NM + NE) {
+#pragma unroll
+                for (int e = (s - NM) * (32 / NE); e < (s - NM + 1) * (32 / NE); e++) {
+                    const float p = __builtin_amdgcn_exp2f(sc[e >> 4][e & 15] - m);
+                    psum += p;
+                    pf[e >> 3][e & 7] = (_Float16)p;
+                }
+                here(psum, pf[(s - NM) * 4 / NE]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
         l = l * alpha + psum;
-        m = m_new;
         if (__any(alpha != 1.0f)) {
 #pragma unroll
             for (int dt = 0; dt < ND; dt++)
 #pragma unroll
-                for (int i = 0; i < 16; i++) o[dt][i] *= alpha;
+                for (int i = 0; i < 16; i++) {
+                    float x = o[dt][i], t;
+                    asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\tv_accvgpr_write_b32 %0, %1" : "+a"(x), "=&v"(t) : "v"(alpha));
+                    o[dt][i] = x;
+                }
+            asm volatile("s_nop 4");
         }
+        constexpr int W = ND < 4 ? ND : 4, NG = 4 * ND / W;   // output tiles of a group, groups: group q is step q % 4 of tiles W (q / 4) ...
 #pragma unroll
-        for (int dt = 0; dt < ND; dt++) {
+        for (int i = 0; i < W; i++) vf[0][i] = v_frag(B, 0, i);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const uint16_t* vp = Vt + (32 * dt + r) * VS + 16 * j + 4 * g;
-                const uint2 v0 = *(const uint2*)vp, v1 = *(const uint2*)(vp + 8);
-                const h8 vf = __builtin_bit_cast(h8, make_uint4(v0.x, v0.y, v1.x, v1.y));
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[j], o[dt], 0, 0, 0);
+        for (int q = 0; q < NG; q++) {
+            if (q + 1 < NG) {
+#pragma unroll
+                for (int i = 0; i < W; i++) vf[(q + 1) & 1][i] = v_frag(B, (q + 1) & 3, W * ((q + 1) >> 2) + i);
+                __builtin_amdgcn_sched_barrier(0);  // (ahead of the products, not between)
             }
+#pragma unroll
+            for (int i = 0; i < W; i++)
+                o[W * (q >> 2) + i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[q & 1][i], pf[q & 3], o[W * (q >> 2) + i], 0, 0, 0);
             __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
+        if (NEXT) mask(sn, kt + 1);
+    };
+
+    v16f s0[2], s1[2];
+    __builtin_amdgcn_s_waitcnt(0x0f70);             // tile 0 has landed
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int kk = 0; kk < 2; kk++) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) s0[kk][i] = 0.0f;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const h8 kf = k_frag(0, s, kk);
+            s0[kk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qh[s], s0[kk], 0, 0, 0);
+            s0[kk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, ql[s], s0[kk], 0, 0, 0);
+        }
+    }
+    mask(s0, 0);
+    int kt = 0;
+    for (; kt + 2 < n_kt; kt += 2) {
+        tile(Is<1>(), Is<0>(), kt, s0, s1);
+        tile(Is<1>(), Is<1>(), kt + 1, s1, s0);
+    }
+    if (kt + 1 < n_kt) {
+        tile(Is<1>(), Is<0>(), kt, s0, s1);
+        tile(Is<0>(), Is<1>(), kt + 1, s1, s0);
+    } else {
+        tile(Is<0>(), Is<0>(), kt, s0, s1);
     }
 
     l += __shfl_xor(l, 32, 64);
@@ -230,7 +295,7 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
 template <int HD, int G>
 bool launch_prefill(const AttnArgs& a, float* out, hipStream_t s) {
     constexpr int QT = 128 / G;
-    const size_t lds = ((size_t)(KT + 128) * (HD + 8) + (size_t)HD * VS) * sizeof(uint16_t);
+    const size_t lds = (size_t)4 * KT * HD * sizeof(uint16_t);   // two tiles of K, two of V
     static bool sized = false;
     if (!sized) {
         if (lds > 64 * 1024 &&
