@@ -1717,8 +1717,9 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
                    [=](hipStream_t s) { attend_exact(args, sc, dout, s); });
     } else {
         int n_split = attend_split_count((int)n_pos_cap, (int)n_q, (int)a->head_dim, (int)group);
-        // the one-pass kernel of a large batch (never a graphed pass) keeps no partial results: what is reserved is
-        // what the single-token passes that follow will ask for (the whole slab's splits), so that they do not grow it
+        // the one-pass kernel of a large batch (never a graphed pass) keeps partial results only of what its few blocks
+        // share; what the single-token passes that follow will ask for (the whole slab's splits) is reserved beside it, so
+        // that they do not grow it
         AttnArgs probe{dq, dk, dv, (int)n_q, (int)a->kv_dim, (int)a->n_pos, (int)a->head_dim, (int)a->n_head, (int)a->n_head_kv,
                        a->scale, nullptr};
         const bool one_pass = !graphed && attend_prefill_takes(probe, dout);
@@ -1727,7 +1728,8 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
         // a few-query call reserves the decode size too, so that the first graphed pass after it (whose split count is
         // the whole slab's) does not have to grow the scratch in the middle of a capture
         const size_t call_floats = (size_t)(n_q * a->n_head) * n_split * (a->head_dim + 2);
-        float* sc = be->scratch_f32(one_pass ? decode_floats : std::max(call_floats, decode_floats));
+        const int shares = one_pass ? attend_prefill_splits(probe) : 1;
+        float* sc = be->scratch_f32(std::max(decode_floats, one_pass ? attend_prefill_floats(probe) : call_floats));
         if (!sc) return;
         const int* dyn = be->dyn_slot((int)a->n_pos);
         AttnArgs args{dq, dk, dv, (int)n_q, (int)a->kv_dim, dyn ? 0 : (int)a->n_pos, (int)a->head_dim,
@@ -1741,10 +1743,10 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
                    sig_of(OP_ATTEND, 1, dq, dk, dv, args.n_q, args.kv_dim, args.head_dim, args.n_head, args.n_head_kv,
                           args.scale, dyn, dyn ? n_split : 0, sc, dout), rec,
                    [=](hipStream_t s) {
-                       // a one-pass prefill reserved the decode passes' scratch only: it must not fall into the split
+                       // a one-pass prefill reserved its own and the decode passes' scratch only: it must not fall into the split
                        // kernels, whose partials for the whole batch would not fit there
                        if (one_pass) {
-                           if (!attend_prefill(args, dout, s)) be->fail("attend: the one-pass prefill kernel could not be launched");
+                           if (!attend_prefill(args, shares, sc, dout, s)) be->fail("attend: the one-pass prefill kernel could not be launched");
                        } else if (!attend_split_gated(args, n_split, sc, dout, nullptr, 0, s)) {
                            be->fail("attend: the split-K kernels could not be launched");
                        }

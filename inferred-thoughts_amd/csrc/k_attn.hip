@@ -710,7 +710,7 @@ __global__ __launch_bounds__(256) void attend_merge_wide_k(const float* __restri
 }
 
 bool attend_split(const AttnArgs& a, int n_split, float* scratch, float* out, hipStream_t s) {
-    if (attend_prefill(a, out, s)) return true;
+    if (attend_prefill(a, 1, nullptr, out, s)) return true;
     return attend_split_gated(a, n_split, scratch, out, nullptr, 0, s);
 }
 

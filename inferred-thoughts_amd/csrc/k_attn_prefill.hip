@@ -28,6 +28,8 @@
 #include "it_dot.h"
 #include "kernels.h"
 
+#include <algorithm>
+
 namespace itk {
 namespace {
 
@@ -52,6 +54,11 @@ IT_DEV void here(float& x, h8& v) {
     v = __builtin_bit_cast(h8, t);
 }
 
+constexpr float NONE = -1e30f;  // the maximum of a row that has seen no key
+
+// Partial results of n_split shares: the sums [token][head][share][HD], then maximum (log2) and weight of each.
+IT_DEV float* part_stats(float* part, const AttnArgs& a, int hd) { return part + (int64_t)a.n_q * a.n_head * gridDim.z * hd; }
+
 template <int V>
 struct Is { static constexpr int value = V; };
 
@@ -62,7 +69,7 @@ struct Is { static constexpr int value = V; };
 // as issued (0.68 ms when a tile was fetched through registers, V turned on its way into LDS, and softmax and products
 // took turns between two barriers); 30,000 in four batches: 10.3 ms (16.9).
 template <int HD, int G>
-__global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __restrict__ out) {
+__global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __restrict__ out, float* __restrict__ part) {
     constexpr int QT = 128 / G;                     // tokens per block
     constexpr int NS = HD / 16;                     // k steps of a score tile
     constexpr int ND = HD / 32;                     // output tiles along the head dimension
@@ -86,7 +93,14 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
 
     const int first_pos = base_pos + qt * QT;                            // smallest position of the block
     const int last_pos = base_pos + min(a.n_q, (qt + 1) * QT) - 1;       // largest
-    const int n_kt = last_pos / KT + 1;
+    const int all_kt = last_pos / KT + 1;
+    const int kt0 = (int)((int64_t)all_kt * blockIdx.z / gridDim.z);     // this block's share of the tiles
+    const int n_kt = (int)((int64_t)all_kt * (blockIdx.z + 1) / gridDim.z);
+    const int row_at = token * a.n_head + head;
+    if (kt0 == n_kt) {                              // more shares than tiles: weight 0 for the merge
+        if (valid && g == 0) *(float2*)(part_stats(part, a, HD) + ((int64_t)row_at * gridDim.z + blockIdx.z) * 2) = make_float2(NONE, 0.0f);
+        return;
+    }
     const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)lds);
 
     const int lrow = w * 16 + lane / P;             // this lane's row of the wave's first load
@@ -106,9 +120,9 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
             to_lds(from, at + V_AT + buf * TILE + (w * NL + i) * 1024);
         }
     };
-    ask_k(0, 0);
-    ask_v(0, 0);
-    ask_k(1, 1);                                    // (past the end: the last key again, never read)
+    ask_k(kt0, 0);
+    ask_v(kt0, 0);
+    ask_k(kt0 + 1, 1);                                    // (past the end: the last key again, never read)
 
     // this lane's query row, scaled, as an f16 pair
     h8 qh[NS], ql[NS];
@@ -150,7 +164,7 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
     for (int dt = 0; dt < ND; dt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) o[dt][i] = 0.0f;
-    float m = -INFINITY, l = 0.0f;
+    float m = NONE, l = 0.0f;
 
     // a row sees keys up to its own position
     auto mask = [&](v16f (&sc)[2], int kt) __attribute__((always_inline)) {
@@ -206,7 +220,7 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
                 for (int e = s * (32 / NM); e < (s + 1) * (32 / NM); e++) mt = fmaxf(mt, sc[e >> 4][e & 15]);
                 if (s == NM - 1) {
                     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-                    const float m_new = mt > m + GROW ? mt : m;   // finite from the first tile on: key 0 is visible to every row
+                    const float m_new = mt > m + GROW ? mt : m;   // (NONE while the row has seen no key: its probabilities are 0)
                     alpha = __builtin_amdgcn_exp2f(m - m_new);
                     m = m_new;
                 }
@@ -266,8 +280,8 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
             s0[kk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, ql[s], s0[kk], 0, 0, 0);
         }
     }
-    mask(s0, 0);
-    int kt = 0;
+    mask(s0, kt0);
+    int kt = kt0;
     for (; kt + 2 < n_kt; kt += 2) {
         tile(Is<1>(), Is<0>(), kt, s0, s1);
         tile(Is<1>(), Is<1>(), kt + 1, s1, s0);
@@ -281,8 +295,10 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
 
     l += __shfl_xor(l, 32, 64);
     if (valid) {
-        const float inv = 1.0f / l;
-        float* orow = out + (int64_t)token * qdim + head * HD + 4 * g;
+        const int64_t at_part = (int64_t)row_at * gridDim.z + blockIdx.z;
+        if (part && g == 0) *(float2*)(part_stats(part, a, HD) + at_part * 2) = make_float2(m, l);
+        const float inv = part ? 1.0f : 1.0f / l;
+        float* orow = (part ? part + at_part * HD : out + (int64_t)token * qdim + head * HD) + 4 * g;
 #pragma unroll
         for (int dt = 0; dt < ND; dt++)
 #pragma unroll
@@ -292,8 +308,30 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
     }
 }
 
+// The shares' sums, weighted and divided: four dims of a row per thread.  Memory: each partial is read once.
+__global__ __launch_bounds__(256) void prefill_merge_k(const float* __restrict__ part, int64_t rows, int n_split, int hd4, float* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, row = i / hd4;
+    if (row >= rows) return;
+    const float2* const st = (const float2*)(part + rows * n_split * hd4 * 4) + row * n_split;
+    const float4* const p = (const float4*)part + row * n_split * hd4 + i % hd4;
+    float m = st[0].x;
+    for (int z = 1; z < n_split; z++) m = fmaxf(m, st[z].x);
+    float l = 0.0f;
+    float4 o = make_float4(0, 0, 0, 0);
+    for (int z = 0; z < n_split; z++) {
+        const float2 t = st[z];
+        if (t.y <= 0.0f) continue;                  // an empty share's sums were never written
+        const float w = __builtin_amdgcn_exp2f(t.x - m);
+        const float4 x = p[(int64_t)z * hd4];
+        l += w * t.y;
+        o.x += w * x.x; o.y += w * x.y; o.z += w * x.z; o.w += w * x.w;
+    }
+    const float inv = 1.0f / l;
+    ((float4*)out)[i] = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+}
+
 template <int HD, int G>
-bool launch_prefill(const AttnArgs& a, float* out, hipStream_t s) {
+bool launch_prefill(const AttnArgs& a, int n_split, float* part, float* out, hipStream_t s) {
     constexpr int QT = 128 / G;
     const size_t lds = (size_t)4 * KT * HD * sizeof(uint16_t);   // two tiles of K, two of V
     static bool sized = false;
@@ -305,18 +343,23 @@ bool launch_prefill(const AttnArgs& a, float* out, hipStream_t s) {
         }
         sized = true;
     }
-    hipLaunchKernelGGL((attend_prefill_k<HD, G>), dim3((a.n_q + QT - 1) / QT, a.n_head_kv), dim3(256), lds, s, a, out);
+    hipLaunchKernelGGL((attend_prefill_k<HD, G>), dim3((a.n_q + QT - 1) / QT, a.n_head_kv, n_split), dim3(256), lds, s, a, out,
+                       n_split > 1 ? part : nullptr);
+    if (n_split > 1) {
+        const int64_t rows = (int64_t)a.n_q * a.n_head;
+        hipLaunchKernelGGL(prefill_merge_k, dim3((unsigned)((rows * (HD / 4) + 255) / 256)), dim3(256), 0, s, part, rows, n_split, HD / 4, out);
+    }
     return true;
 }
 
 template <int HD>
-bool launch_prefill_g(const AttnArgs& a, float* out, hipStream_t s) {
+bool launch_prefill_g(const AttnArgs& a, int n_split, float* part, float* out, hipStream_t s) {
     switch (a.n_head / a.n_head_kv) {
-        case 1: return launch_prefill<HD, 1>(a, out, s);
-        case 2: return launch_prefill<HD, 2>(a, out, s);
-        case 4: return launch_prefill<HD, 4>(a, out, s);
-        case 8: return launch_prefill<HD, 8>(a, out, s);
-        case 16: return launch_prefill<HD, 16>(a, out, s);
+        case 1: return launch_prefill<HD, 1>(a, n_split, part, out, s);
+        case 2: return launch_prefill<HD, 2>(a, n_split, part, out, s);
+        case 4: return launch_prefill<HD, 4>(a, n_split, part, out, s);
+        case 8: return launch_prefill<HD, 8>(a, n_split, part, out, s);
+        case 16: return launch_prefill<HD, 16>(a, n_split, part, out, s);
         default: return false;
     }
 }
@@ -334,13 +377,30 @@ bool attend_prefill_takes(const AttnArgs& a, const float* out) {
     return a.head_dim == 64 || a.head_dim == 128 || a.head_dim == 256;
 }
 
+// Shares the keys are cut into: a batch whose blocks leave compute units idle gets as many as fill them once, as long as a
+// share keeps PREFILL_SHARE tiles (2 to 8 measure the same; a tile is 2 us, the merge's launch 5).  16,000 tokens in passes of
+// 512, two layers: 44.9 ms with whole rows on 64 of 256 compute units, 38.0 so.
+constexpr int PREFILL_SHARE = 4, CUS = 256;
+int attend_prefill_splits_max(const AttnArgs& a) {
+    const int qt = 128 / (a.n_head / a.n_head_kv);
+    return (int)std::max<int64_t>(1, CUS / ((int64_t)((a.n_q + qt - 1) / qt) * a.n_head_kv));
+}
+int attend_prefill_splits(const AttnArgs& a) {
+    return std::max(1, std::min(attend_prefill_splits_max(a), (a.n_pos + KT - 1) / KT / PREFILL_SHARE));
+}
+// floats of partial results, at any n_pos (so that a context that grows does not make them grow)
+size_t attend_prefill_floats(const AttnArgs& a) {
+    const int n = attend_prefill_splits_max(a);
+    return n > 1 ? (size_t)a.n_q * a.n_head * n * (a.head_dim + 2) : 0;
+}
+
 // false: not a shape this kernel takes (the caller uses the split kernels)
-bool attend_prefill(const AttnArgs& a, float* out, hipStream_t s) {
+bool attend_prefill(const AttnArgs& a, int n_split, float* part, float* out, hipStream_t s) {
     if (!attend_prefill_takes(a, out)) return false;
     switch (a.head_dim) {
-        case 64: return launch_prefill_g<64>(a, out, s);
-        case 128: return launch_prefill_g<128>(a, out, s);
-        case 256: return launch_prefill_g<256>(a, out, s);
+        case 64: return launch_prefill_g<64>(a, n_split, part, out, s);
+        case 128: return launch_prefill_g<128>(a, n_split, part, out, s);
+        case 256: return launch_prefill_g<256>(a, n_split, part, out, s);
         default: return false;
     }
 }

@@ -267,7 +267,9 @@ void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, 
 int attend_split_count(int n_pos_max, int n_q, int head_dim, int group);
 bool attend_split(const AttnArgs& a, int n_split_max, float* scratch, float* out, hipStream_t s);  // false: not launched
 // more than 16 queries, fast mode: one pass over the keys on the f16 matrix cores; false when the shape is not taken
-bool attend_prefill(const AttnArgs& a, float* out, hipStream_t s);
+bool attend_prefill(const AttnArgs& a, int n_split, float* part, float* out, hipStream_t s);
+int attend_prefill_splits(const AttnArgs& a);
+size_t attend_prefill_floats(const AttnArgs& a);
 bool attend_prefill_takes(const AttnArgs& a, const float* out);
 // What one decode token's attention needs before it can attend, folded into the tile kernel: the
 // query heads' norm + rotation (every block, for its own heads) and the new position's key
