@@ -176,6 +176,8 @@ __global__ __launch_bounds__(256) void float_gemv_fast_k(FloatMats m, const floa
 // v_mfma_f32_16x16x4_f32 per pair of tiles, instruction j taking element j of both (k = 4 (lane / 16) + j: the same k on
 // both sides, in whatever order).  Operands come straight from L2: no LDS, no barrier in the loop.  513 x 2,048 F32 rows
 // (router + gate logit): 10 us for 23 tokens (9 blocks of a 64 x 64 tile on the vector ALU: 100 us), 146 us for 5,700 (369).
+// (Asking for two or four steps at a time, twice buffered, is 10 to 60 % slower: not the latency of a step bounds it but the
+// rate at which loads of sixteen rows' 64 bytes are served.)
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 template <int FMT, int RT, int TT, int KW>
 __global__ __launch_bounds__(64 * KW) void float_mfma_k(FloatMats m, const float* __restrict__ x, int n_in, int n_tok, float out_scale) {
