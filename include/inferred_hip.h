@@ -330,7 +330,9 @@ int it_hip_mfma_ceiling(it_hip*, int kind, int iters, double* ops_per_s);
  * No counterpart in the reference (its device backend sizes its pools with the driver's allocator as it goes,
  * src/ops/cuda/mod.rs:1011-1158).  For callers that cannot allocate: code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc.  The computation is it_hip_attend's split-K form (fast mode) for at most 16
- * query rows: same kernels, same split count, bit-identical output.  Differences from it_hip_attend:
+ * query rows: same kernels, same split count, bit-identical output.  (A single-token pass that is tagged, or recorded as a
+ * graph, splits by the rows of its slab instead of by n_pos, so that one launch shape serves a growing context: the same
+ * values but for the order of the splits' sums.)  Differences from it_hip_attend:
  *  - every pointer in `a`, and `out`, is a DEVICE pointer the caller owns (nothing is mirrored or copied);
  *  - `stream` is a hipStream_t (NULL = the null stream); the call only enqueues work on it;
  *  - the split-K partial results live in a fixed array of IT_HIP_NOALLOC_SCRATCH_BYTES inside the library's code

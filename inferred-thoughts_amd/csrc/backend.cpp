@@ -131,6 +131,14 @@ void it_hip::open_pass(uint64_t sig) {
     issue_inputs();
 }
 
+bool it_hip::may_record() const {
+    if (mode != Mode::Open) return mode != Mode::Eager;
+    if (!prof_on && stable_passes >= 1) return true;
+    for (const Graph& g : graphs)
+        if (g.valid) return true;
+    return false;
+}
+
 // what a deferred pass has recorded so far goes to the stream, fused; the pass stays deferred
 void it_hip::flush_deferred() {
     if (chain_enabled && fuse_enabled && !exact && !expert_cold_entries && (!itk::layer_chain_fits() || !chain_acquire())) chain_enabled = false;
@@ -1695,10 +1703,13 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
     if (!dq || !dk || !dv || !dout) return;
     uint64_t group = a->n_head / a->n_head_kv;
     bool split_ok = (group == 1 || group == 2 || group == 4 || group == 8) && a->head_dim <= 256;
-    bool graphed = be->mode != it_hip::Mode::Eager;
-    // a graphed pass keeps one launch shape while the context grows: size for the whole slab (any single-token pass, so that
-    // one issued op by op adds the splits up in the same order)
-    uint64_t n_pos_cap = graphed || n_q == 1 ? a->kv_len / a->kv_dim : a->n_pos;
+    const bool graphed = be->mode != it_hip::Mode::Eager;
+    // A recorded pass keeps one launch shape while the context grows: it is sized for the whole slab, and so is a tagged pass
+    // that is issued op by op, which adds the splits up in the order of the recorded ones of its tag.  Every other call is
+    // split by its context alone (6,000 positions in a slab of 8,192 rows: 94 splits, not 128), as it_hip_attend_noalloc does.
+    const uint64_t slab_rows = a->kv_len / a->kv_dim;
+    const bool by_slab = be->may_record() || (n_q == 1 && be->in_pass && be->pass_tag);
+    const uint64_t n_pos_cap = (be->exact || !split_ok ? graphed : by_slab) ? slab_rows : a->n_pos;
     uint64_t bytes = a->n_pos * a->n_head_kv * a->head_dim * 4 + a->q_len * 8;
     if (be->exact || !split_ok) {
         float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap));
@@ -1723,8 +1734,7 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
         AttnArgs probe{dq, dk, dv, (int)n_q, (int)a->kv_dim, (int)a->n_pos, (int)a->head_dim, (int)a->n_head, (int)a->n_head_kv,
                        a->scale, nullptr};
         const bool one_pass = !graphed && attend_prefill_takes(probe, dout);
-        const size_t decode_floats = (size_t)a->n_head * attend_split_count((int)(a->kv_len / a->kv_dim), 1, (int)a->head_dim, (int)group) *
-                                     (a->head_dim + 2);
+        const size_t decode_floats = (size_t)a->n_head * attend_split_count((int)slab_rows, 1, (int)a->head_dim, (int)group) * (a->head_dim + 2);
         // a few-query call reserves the decode size too, so that the first graphed pass after it (whose split count is
         // the whole slab's) does not have to grow the scratch in the middle of a capture
         const size_t call_floats = (size_t)(n_q * a->n_head) * n_split * (a->head_dim + 2);
@@ -1741,7 +1751,7 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
         rec.f[0] = args.scale;
         be->submit(it_hip::FAM_ATTEND, bytes,
                    sig_of(OP_ATTEND, 1, dq, dk, dv, args.n_q, args.kv_dim, args.head_dim, args.n_head, args.n_head_kv,
-                          args.scale, dyn, dyn ? n_split : 0, sc, dout), rec,
+                          args.scale, dyn, dyn ? attend_split_count((int)slab_rows, (int)n_q, (int)a->head_dim, (int)group) : 0, sc, dout), rec,
                    [=](hipStream_t s) {
                        // a one-pass prefill reserved its own and the decode passes' scratch only: it must not fall into the split
                        // kernels, whose partials for the whole batch would not fit there

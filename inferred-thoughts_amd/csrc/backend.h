@@ -267,6 +267,7 @@ struct it_hip {
     bool replay_pass(const void* tag, uint64_t pos, const uint32_t* id, uint64_t ring_index);
     void drop_one(Graph& g);
     void open_pass(uint64_t sig);
+    bool may_record() const;   // the pass is recorded, deferred or replayed, or its first op may still make it so
     // Deferred: a single-token pass whose ops are recorded like a captured pass's and issued as fused launches whenever
     // something needs them on the stream (a cold expert's resolve reads the picks back, a host read, the pass's end):
     // the fusion of the decode path without its graph, for passes a graph cannot hold.

@@ -134,3 +134,33 @@ def test_the_first_call_of_a_process_needs_no_backend():
     code = _FIRST_CALL.format(tests=str(root / "tests"), pkg=str(root / "inferred-thoughts_amd"), root=str(root))
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and "FIRST CALL OK" in out.stdout, out.stdout[-2000:] + out.stderr[-2000:]
+
+
+def test_a_pass_issued_op_by_op_with_every_buffer_in_place_splits_by_its_context():
+    """The second of two such passes finds mirrors, slabs and scratch as it needs them, so nothing takes it out of the state
+    in which it could still turn out to be a recorded pass: it is not one, and gives the first pass's bits."""
+    hd, nh, nkv, n_pos, slab = 256, 16, 2, 700, 4096
+    hip = ih.Hip(exact=False)
+    rt = Hiprt()
+    try:
+        r = rng(79)
+        q = r.standard_normal(nh * hd).astype(np.float32)
+        k = f16_bits(r.standard_normal(slab * nkv * hd)); v = f16_bits(r.standard_normal(slab * nkv * hd))
+        out, got = np.zeros_like(q), []
+        for _ in range(2):
+            hip.begin_pass(1)
+            hip.host_wrote(q)
+            hip.attend(q, k, v, nkv * hd, n_pos, hd, nh, nkv, 0.0625, out)
+            hip.end_pass()
+            hip.host_needs(out)
+            got.append(out.copy())
+        hip.raise_if_error()
+        dq, dk, dv, dout = rt.upload(q), rt.upload(k), rt.upload(v), rt.filled(q.nbytes, 0xff)
+        rc, msg = ih.attend_noalloc(dq, q.size, dk, dv, k.size, nkv * hd, n_pos, hd, nh, nkv, 0.0625, dout, q.size, stream=0)
+        assert rc == 0, msg
+        other = rt.download(dout, q)
+        for i, g in enumerate(got):
+            assert_bits_equal(g, other, f"pass {i + 1}")
+    finally:
+        rt.free_all()
+        hip.close()
