@@ -1859,7 +1859,7 @@ void it_hip_scatter_chunks(it_hip* be, const float* src, uint64_t src_len, uint6
     if (!ds || !dd) return;
     int64_t sl = (int64_t)src_len, c = (int64_t)chunk, st = (int64_t)stride, off = (int64_t)offset;
     it_hip::OpRec rec;
-    rec.id = OP_SCATTER;
+    rec.id = OP_SCATTER; rec.p[0] = ds; rec.p[1] = dd;
     be->submit(it_hip::FAM_OTHER, src_len * 8, sig_of(OP_SCATTER, ds, sl, c, st, off, dd), rec,
                [=](hipStream_t s) { scatter_chunks(ds, sl, c, st, off, dd, s); });
 }
@@ -2145,7 +2145,7 @@ void it_hip_add_scaled_rows(it_hip* be, float* acc, uint64_t acc_len, const floa
     int64_t n = (int64_t)acc_len;
     int ns = (int)scales_len;
     it_hip::OpRec rec;
-    rec.id = OP_ROWS;
+    rec.id = OP_ROWS; rec.p[0] = da; rec.p[1] = dr; rec.p[2] = dsc;
     be->submit(it_hip::FAM_OTHER, rows_len * 4, sig_of(OP_ROWS, da, n, dr, dsc, ns), rec,
                [=](hipStream_t s) { add_scaled_rows(da, n, dr, dsc, ns, s); });
 }
@@ -2160,7 +2160,7 @@ void it_hip_add_scaled_sigmoid(it_hip* be, float* acc, uint64_t acc_len, const f
     if (!da || !db || !dl) return;
     int64_t n = (int64_t)acc_len;
     it_hip::OpRec rec;
-    rec.id = OP_SIGADD;
+    rec.id = OP_SIGADD; rec.p[0] = da; rec.p[1] = db; rec.p[2] = dl;
     be->submit(it_hip::FAM_OTHER, acc_len * 12, sig_of(OP_SIGADD, da, db, n, dl), rec,
                [=](hipStream_t s) { add_scaled_sigmoid(da, db, n, dl, s); });
 }

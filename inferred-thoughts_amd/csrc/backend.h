@@ -38,6 +38,7 @@
 //   EXPERTS    p: q, s, scale2, ids, act_scales, act_quants, out     i: as GLU
 //   FINISH     p: out, rows, weights, shared, logit   i: at, n, n_tok, n_used, logit_at
 //   ROPE       p: x, table, dyn             i: half, n_tok, head_dim, n_rot, n_heads, pos
+//   SCATTER    p: src, out     ROWS  p: acc, rows, scales     SIGADD  p: acc, b, logit
 //   KVWRITE    p: slab, dyn, src            i: mul, offset, n
 //   ATTEND     p: q, k, v, dyn, scratch, out   i: n_q, kv_dim, head_dim, n_head, n_head_kv, n_split, exact, n_pos (live: [8], exact form, sized for: [9])  f: scale
 enum OpId : int {

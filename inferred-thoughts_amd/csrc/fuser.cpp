@@ -1020,11 +1020,13 @@ bool used_later(const std::vector<it_hip::OpRec>& h, size_t from, const it_hip::
         if (reads_or_writes(h[k], dev)) return true;
     return next && reads_or_writes(*next, dev);
 }
-// ... other than making the forms of it
-bool changed_later(const std::vector<it_hip::OpRec>& h, size_t from, const void* dev) {
+// ... other than making the forms of it.  The op behind may be the product that reads it: its pointers were taken, and the
+// forms of what it writes marked as gone, before the run in front of it is issued.
+bool changed_later(const std::vector<it_hip::OpRec>& h, size_t from, const it_hip::OpRec* next, const void* dev) {
+    auto changes = [&](const it_hip::OpRec& r) { return r.id != OP_QUANT && r.id != OP_SPLIT && reads_or_writes(r, dev); };
     for (size_t k = from; k < h.size(); k++)
-        if (h[k].id != OP_QUANT && h[k].id != OP_SPLIT && reads_or_writes(h[k], dev)) return true;
-    return false;
+        if (changes(h[k])) return true;
+    return next && changes(*next) && !(next->id == OP_MATMUL && next->p[5] != dev && next->p[6] != dev);
 }
 // the small FFN's products, while its run is being held: which may come next
 bool small_ffn_next(const std::vector<it_hip::OpRec>& held, const it_hip::OpRec& r) {
@@ -1266,17 +1268,20 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
                 len++;
                 p.w = (const float*)m.p[1]; p.eps = m.f[0]; p.out = (float*)m.p[2];
                 const int64_t all = rows * width;
-                if (id(k + 2) == OP_GATHER && h[k + 2].p[0] == m.p[2] && h[k + 2].i[2] == 0 && h[k + 2].i[0] == all && h[k + 2].i[3] == all &&
-                    h[k + 2].p[1] != p.x && h[k + 2].p[1] != p.y) {
-                    // the copy is what the products read: its forms are made instead of the normed rows'
+                const bool copied = id(k + 2) == OP_GATHER && h[k + 2].p[0] == m.p[2] && h[k + 2].i[2] == 0 && h[k + 2].i[0] == all &&
+                                    h[k + 2].i[3] == all && h[k + 2].p[1] != p.x && h[k + 2].p[1] != p.y;
+                // The copy is what the products read: its forms are made instead of the normed rows'.  Not so where an op that has
+                // been asked for already reads the normed rows' own (the norm marked them as valid when it was asked for).
+                if (copied && !(m.p[3] && used_later(h, k + 3, next, m.p[4]))) {
                     p.copy = (float*)h[k + 2].p[1];
                     len++;
                     const OpRec* q = id(k + 3) == OP_QUANT && h[k + 3].p[0] == p.copy && h[k + 3].i[0] == all ? &h[k + 3] : nullptr;
                     if (q) len++;
-                    copy_act = changed_later(h, i + len, p.copy) ? nullptr : act_by_dev(p.copy);
+                    copy_act = changed_later(h, i + len, next, p.copy) ? nullptr : act_by_dev(p.copy);
                     if (q) {
                         p.q.scales = (float*)q->p[1]; p.q.quants = (int8_t*)q->p[2];
-                    } else if (m.p[3] && copy_act && copy_act->cap >= (size_t)all && act_q_reserve(*copy_act, (size_t)all)) {
+                    } else if (m.p[3] && copy_act && copy_act->cap >= (size_t)all && copy_act->q_cap >= (size_t)all) {
+                        // (room that is there: what is held, and the op behind, may hold the address of what there is)
                         p.q.scales = copy_act->q_scales; p.q.quants = copy_act->q_quants;
                     }
                     if (p.q.quants && m.p[3]) {
@@ -1286,7 +1291,7 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
                     }
                 } else if (m.p[3]) {
                     p.q.scales = (float*)m.p[3]; p.q.quants = (int8_t*)m.p[4];
-                    out_act = changed_later(h, i + len, p.out) ? nullptr : act_by_dev(p.out);
+                    out_act = changed_later(h, i + len, next, p.out) ? nullptr : act_by_dev(p.out);
                 }
             }
             if (!width) {

@@ -83,6 +83,40 @@ def test_the_residual_row(pair, orc, n, nd):
     run(pair, n, b, script, ["out", "out2"], tol=3e-2)
 
 
+@pytest.mark.parametrize("what", ["normed_first", "normed_first_nvfp4", "into_the_copy", "part_of_the_copy", "scatter_into_the_copy"])
+@pytest.mark.parametrize("n,nd", [(3, 1024), (40, 2048)])
+def test_the_residual_row_in_front_of_other_readers_and_writers(pair, orc, n, nd, what):
+    """The op behind the run had its pointers taken before the run was issued: one that reads the normed rows' Q8_0 form, one
+    that writes the copy, one that reads a part of the copy (whose form has less room than the whole one needs).  Every
+    product is compared with the one of the backend that issues the ops one by one."""
+    import inferred_hip as ih
+    r = rng(7)
+    w, sq = q8_0_weights(orc, r, 64, nd, std=0.05), q8_0_weights(orc, r, nd, nd, std=0.05)
+    w4 = nvfp4_weights(r, 64, nd)
+    norm = (0.5 + r.random(nd)).astype(np.float32)
+    z = lambda k: np.zeros(k, np.float32)  # noqa: E731
+    b = dict(x=f32(r, n * nd), y=f32(r, n * nd), z=f32(r, n * nd), normed=z(n * nd), copy=z(n * nd), out=z(n * 64), out2=z(n * 64))
+    w64 = ih.weights(w, ih.Q8_0, nd, 64)
+
+    def script(be, b):
+        be.add_assign(b["x"], b["y"])
+        be.rms_norm(b["x"], norm, EPS, b["normed"])
+        be.gather_chunks(b["normed"], n * nd, n * nd, 0, b["copy"])
+        if what == "normed_first":
+            be.matmul(w64, b["normed"], b["out2"])
+        elif what == "normed_first_nvfp4":
+            be.matmul(ih.weights(w4, ih.NVFP4, nd, 64), b["normed"], b["out2"])
+        elif what == "into_the_copy":
+            be.matmul(ih.weights(sq, ih.Q8_0, nd, nd), b["z"], b["copy"])
+        elif what == "part_of_the_copy":
+            be.matmul(w64, b["copy"][:nd], b["out2"][:64])
+            return   # (the form of the whole copy is never asked for)
+        else:
+            be.scatter_chunks(b["z"], n * nd, n * nd, 0, b["copy"])
+        be.matmul(w64, b["copy"], b["out"])
+    run(pair, n, b, script, ["x", "normed", "copy", "out", "out2"], tol=3e-2)
+
+
 @pytest.mark.parametrize("n,nd,nu", [(2, 1024, 4), (3, 2048, 10), (5, 1056, 3), (40, 2048, 8)])
 def test_the_routed_sum_in_front_of_the_residual(pair, n, nd, nu):
     r = rng(2)
