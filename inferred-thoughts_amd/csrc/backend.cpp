@@ -1154,19 +1154,21 @@ float* it_hip::gdn_work_for(size_t floats) {
     return gdn_work;
 }
 
-// true when moe_work already holds this grouping (the gate/up and down products of one MoE layer share it);
-// records the grouping as held otherwise.  Eager passes only: a recorded launch may run later.
-bool it_hip::group_cached(int picks, int n_expert, int tile) {
-    if (mode != Mode::Eager) {
-        group_gen = ~0ull;
-        return false;
+it_hip::Grouping it_hip::grouping(int picks, int n_expert) {
+    if (mode != Mode::Eager) grouped.gen = ~0ull;
+    Grouping g;
+    g.be = mode == Mode::Eager ? this : nullptr;
+    g.gen = route_gen;
+    g.picks = picks;
+    g.experts = n_expert;
+    return g;
+}
+bool it_hip::Grouping::made(int t) const {
+    if (be) {
+        be->grouped = *this;
+        be->grouped.tile = t;
     }
-    const bool hit = group_gen == route_gen && group_picks == picks && group_experts == n_expert && group_tile == tile;
-    group_gen = route_gen;
-    group_picks = picks;
-    group_experts = n_expert;
-    group_tile = tile;
-    return hit;
+    return true;
 }
 
 int32_t* it_hip::moe_work_for(size_t picks, size_t n_expert, size_t* ints) {
@@ -1182,7 +1184,7 @@ int32_t* it_hip::moe_work_for(size_t picks, size_t n_expert, size_t* ints) {
             moe_work_ints = 0;
         }
         const size_t want = need + need / 2;
-        group_gen = ~0ull;
+        grouped.gen = ~0ull;
         if (!check(hipMalloc((void**)&moe_work, want * sizeof(int32_t)), "hipMalloc(expert grouping scratch)")) return nullptr;
         moe_work_ints = want;
     }
@@ -1585,7 +1587,6 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     const int32_t* zids = nullptr;
     int32_t* work = nullptr;
     size_t work_ints = 0;
-    bool grouped = false;
     int tiles = 0;   // 1: tiles of 16, 2: tiles of 128
     SplitOut sp;
     if (!exact && v.fmt == W_NVFP4 && n > 32) {
@@ -1600,8 +1601,8 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
         zids = be->zero_ids_for(n);
         work = be->moe_work_for(n, 1, &work_ints);
         int8_tiles = zids && work;
-        if (int8_tiles) grouped = be->group_cached(nt, 1, 16);
     }
+    const it_hip::Grouping gr = int8_tiles ? be->grouping(nt, 1) : it_hip::Grouping{};   // (every token on the one expert)
     it_hip::OpRec rec;
     rec.id = OP_MATMUL; rec.p[0] = v.q; rec.p[1] = v.scales; rec.p[2] = dx; rec.p[3] = as; rec.p[4] = aq; rec.p[5] = dout;
     rec.p[6] = sp.h; rec.p[7] = sp.l; rec.p[8] = sp.scale;
@@ -1609,7 +1610,7 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     auto run = [=](hipStream_t s, float scale_by) {
         if (tiles == 1 && experts_gemm_f16s(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
         if (tiles == 2 && experts_gemm_f16(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
-        if (int8_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, grouped, s)) return;
+        if (int8_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;
         if (rows_dense && expert_rows(ev, nullptr, nullptr, nt, 1, 0, as, aq, dout, scale_by, nullptr, 0, false, s)) return;
         matmul(v, dx, as, aq, nt, dout, scale_by, exact, s);
     };
@@ -1999,12 +2000,13 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
     const bool rows_shape = rows_pay && work && itk::expert_rows_takes(v, nullptr, aq);
     const bool f16_pay = !be->exact && work && !rows_shape && v.fmt == itk::W_NVFP4;
     const bool skinny_shape = skinny_pay && f16_pay && itk::experts_f16s_takes(v, nullptr, np, dout);
-    // the tile size the launch below will group for: 8 or 16 pairs for the row kernel, 128 for the wide f16 kernel,
-    // 16 for the skinny f16 kernel and the int8 one
+    // the tile sizes the launch below may group for: 8 or 16 pairs for the row kernel, 128 for the wide f16 kernel, 16 for
+    // the skinny f16 kernel and the int8 one
     const bool f16_shape = !skinny_shape && f16_pay && itk::experts_f16_takes(v, nullptr, np, dout);
     SplitOut sp;
     if ((skinny_shape || f16_shape) && !be->act_split(x, x_len, (int)w->n_in, &sp)) return;
-    const bool grouped = work && be->group_cached(np, (int)w->n_expert, rows_shape ? itk::expert_rows_tile(np, (int)w->n_expert, v.n_in) : f16_shape ? 128 : 16);
+    const it_hip::Grouping gr = be->grouping(np, (int)w->n_expert);
+    const int rows_tile = itk::expert_rows_tile(np, (int)w->n_expert, v.n_in);
     it_hip::OpRec rec;
     rec.id = OP_EXPERTS; rec.p[0] = v.q; rec.p[1] = v.scales; rec.p[2] = v.scale2; rec.p[3] = ids; rec.p[4] = as; rec.p[5] = aq;
     rec.p[6] = dout; rec.i[0] = v.fmt; rec.i[1] = v.n_in; rec.i[2] = v.n_out; rec.i[3] = np; rec.i[4] = nu; rec.i[5] = xm;
@@ -2015,12 +2017,12 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
                sig_of(OP_EXPERTS, v.q, v.scales, (const void*)v.q_tab, v.fmt, v.n_in, v.n_out, v.scale2, ids, np, nu, xm, as, aq, dout), rec,
                [=](hipStream_t s) {
                    const TileCount tc{counts, nullptr, tally, v.tier, nullptr};
-                   if (skinny_shape && experts_gemm_f16s(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
-                   if (f16_shape && experts_gemm_f16(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
+                   if (skinny_shape && experts_gemm_f16s(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(16), tc, 1.0f, 1.0f, s) && gr.made(16)) return;
+                   if (f16_shape && experts_gemm_f16(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(128), tc, 1.0f, 1.0f, s) && gr.made(128)) return;
                    expert_count(ids, np, v.n_expert, counts, nullptr, tally, s, v.tier, nullptr);
-                   if (rows_shape && expert_rows(v, nullptr, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, grouped, s)) return;
-                   if (!experts_gemm(v, nullptr, ids, np, nu, xm, as, aq, dout, work, work_ints, grouped && !f16_shape, s))
-                       matmul_experts(v, ids, np, nu, xm, as, aq, dout, s);
+                   if (rows_shape && expert_rows(v, nullptr, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, gr.held(rows_tile), s) && gr.made(rows_tile)) return;
+                   if (experts_gemm(v, nullptr, ids, np, nu, xm, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;
+                   matmul_experts(v, ids, np, nu, xm, as, aq, dout, s);
                });
 }
 
@@ -2066,7 +2068,8 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
     const bool f16_shape = !skinny_shape && f16_pay && itk::experts_f16_takes(g, &u, np, dout);
     SplitOut sp;
     if ((skinny_shape || f16_shape) && !be->act_split(x, x_len, (int)gate->n_in, &sp)) return;
-    const bool grouped = work && be->group_cached(np, (int)gate->n_expert, rows_shape ? itk::expert_rows_tile(np, (int)gate->n_expert, g.n_in) : f16_shape ? 128 : 16);
+    const it_hip::Grouping gr = be->grouping(np, (int)gate->n_expert);
+    const int rows_tile = itk::expert_rows_tile(np, (int)gate->n_expert, g.n_in);
     it_hip::OpRec rec;
     rec.id = OP_GLU; rec.p[0] = g.q; rec.p[1] = g.scales; rec.p[2] = u.q; rec.p[3] = u.scales; rec.p[4] = g.scale2;
     rec.p[5] = u.scale2; rec.p[6] = ids; rec.p[7] = as; rec.p[8] = aq; rec.p[9] = dout;
@@ -2079,12 +2082,12 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
                       as, aq, dout), rec,
                [=](hipStream_t s) {
                    const TileCount tc{cg, cu, tally, g.tier, u.tier};
-                   if (skinny_shape && experts_gemm_f16s(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
-                   if (f16_shape && experts_gemm_f16(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, grouped, tc, 1.0f, 1.0f, s)) return;
+                   if (skinny_shape && experts_gemm_f16s(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(16), tc, 1.0f, 1.0f, s) && gr.made(16)) return;
+                   if (f16_shape && experts_gemm_f16(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(128), tc, 1.0f, 1.0f, s) && gr.made(128)) return;
                    expert_count(ids, np, g.n_expert, cg, cu, tally, s, g.tier, u.tier);
-                   if (rows_shape && expert_rows(g, &u, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, grouped, s)) return;
-                   if (!experts_gemm(g, &u, ids, np, nu, xm, as, aq, dout, work, work_ints, grouped && !f16_shape, s))
-                       moe_glu(g, u, ids, np, nu, xm, as, aq, dout, s);
+                   if (rows_shape && expert_rows(g, &u, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, gr.held(rows_tile), s) && gr.made(rows_tile)) return;
+                   if (experts_gemm(g, &u, ids, np, nu, xm, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;
+                   moe_glu(g, u, ids, np, nu, xm, as, aq, dout, s);
                });
 }
 

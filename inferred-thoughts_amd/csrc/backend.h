@@ -181,10 +181,18 @@ struct it_hip {
     size_t route_cap = 0;  // picks
     uint64_t route_n_used = 0, route_n_tok = 0;
     uint64_t route_gen = 0;   // bumped whenever the device route ids are rewritten
-    // the expert grouping that moe_work holds: valid for one route generation, pick count, expert count and tile size
-    uint64_t group_gen = ~0ull;
-    int group_picks = 0, group_experts = 0, group_tile = 0;
-    bool group_cached(int picks, int n_expert, int tile);
+    // The expert grouping that moe_work holds: one route generation, pick count, expert count and tile size.  A launch says
+    // what it grouped when it is issued (an op that is held back may be dropped for a run of several, and not every kernel
+    // groups), and the next one on the same route asks then.
+    struct Grouping {
+        it_hip* be = nullptr;   // null: inside a recorded pass, whose launches run again later
+        uint64_t gen = ~0ull;
+        int picks = 0, experts = 0, tile = 0;
+        bool held(int t) const { return be && be->grouped.gen == gen && be->grouped.picks == picks && be->grouped.experts == experts && be->grouped.tile == t; }
+        bool made(int t) const;   // true
+    };
+    Grouping grouped;
+    Grouping grouping(int picks, int n_expert);
     bool route_reserve(size_t picks);
     // scratch of the grouped expert matmuls (expert-sorted pair lists and their tiles)
     int32_t* moe_work = nullptr;
