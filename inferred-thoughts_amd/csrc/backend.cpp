@@ -536,6 +536,25 @@ bool it_hip::act_split(const float* host, size_t len, int row, SplitOut* out) {
     return true;
 }
 
+bool it_hip::split_at_launch(const float* scales, const int8_t* quants, size_t len, int row, SplitOut* out, hipStream_t s) {
+    if (launch_split_cap < len) {
+        if (launch_split.h) {
+            check(hipStreamSynchronize(stream), "sync before split free");
+            (void)hipFree(launch_split.h);
+            launch_split = SplitOut{};
+            launch_split_cap = 0;
+        }
+        const size_t cap = (len + 255) / 256 * 256;
+        if (!check(hipMalloc((void**)&launch_split.h, cap * 4 + cap / 32 * 4), "hipMalloc(split activations)")) return false;
+        launch_split.l = launch_split.h + cap;
+        launch_split.scale = (float*)(launch_split.l + cap);
+        launch_split_cap = cap;
+    }
+    *out = launch_split;
+    split_rows(quants, scales, (int64_t)len / row, row, *out, s);
+    return true;
+}
+
 const float* it_hip::const_in(const float* host, size_t len) {
     auto it = consts.find(host);
     const uint64_t ident = weight_ident((const uint8_t*)host, len * sizeof(float));
@@ -1285,6 +1304,7 @@ it_hip::~it_hip() {
     if (gdn_work) (void)hipFree(gdn_work);
     if (zero_ids) (void)hipFree(zero_ids);
     if (moe_work) (void)hipFree(moe_work);
+    if (launch_split.h) (void)hipFree(launch_split.h);
     if (argmax_idx) (void)hipFree(argmax_idx);
     if (argmax_val) (void)hipFree(argmax_val);
     if (argmax_out) (void)hipFree(argmax_out);
@@ -2004,7 +2024,8 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
     // the skinny f16 kernel and the int8 one
     const bool f16_shape = !skinny_shape && f16_pay && itk::experts_f16_takes(v, nullptr, np, dout);
     SplitOut sp;
-    if ((skinny_shape || f16_shape) && !be->act_split(x, x_len, (int)w->n_in, &sp)) return;
+    const bool late = be->short_ffn(n_tok);
+    if ((skinny_shape || f16_shape) && !late && !be->act_split(x, x_len, (int)w->n_in, &sp)) return;
     const it_hip::Grouping gr = be->grouping(np, (int)w->n_expert);
     const int rows_tile = itk::expert_rows_tile(np, (int)w->n_expert, v.n_in);
     it_hip::OpRec rec;
@@ -2017,8 +2038,10 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
                sig_of(OP_EXPERTS, v.q, v.scales, (const void*)v.q_tab, v.fmt, v.n_in, v.n_out, v.scale2, ids, np, nu, xm, as, aq, dout), rec,
                [=](hipStream_t s) {
                    const TileCount tc{counts, nullptr, tally, v.tier, nullptr};
-                   if (skinny_shape && experts_gemm_f16s(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(16), tc, 1.0f, 1.0f, s) && gr.made(16)) return;
-                   if (f16_shape && experts_gemm_f16(v, nullptr, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(128), tc, 1.0f, 1.0f, s) && gr.made(128)) return;
+                   SplitOut sx = sp;
+                   if ((skinny_shape || f16_shape) && late && !be->split_at_launch(as, aq, x_len, v.n_in, &sx, s)) return;
+                   if (skinny_shape && experts_gemm_f16s(v, nullptr, ids, np, nu, xm, sx, dout, work, work_ints, gr.held(16), tc, 1.0f, 1.0f, s) && gr.made(16)) return;
+                   if (f16_shape && experts_gemm_f16(v, nullptr, ids, np, nu, xm, sx, dout, work, work_ints, gr.held(128), tc, 1.0f, 1.0f, s) && gr.made(128)) return;
                    expert_count(ids, np, v.n_expert, counts, nullptr, tally, s, v.tier, nullptr);
                    if (rows_shape && expert_rows(v, nullptr, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, gr.held(rows_tile), s) && gr.made(rows_tile)) return;
                    if (experts_gemm(v, nullptr, ids, np, nu, xm, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;
@@ -2067,7 +2090,8 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
     const bool skinny_shape = skinny_pay && f16_pay && itk::experts_f16s_takes(g, &u, np, dout);
     const bool f16_shape = !skinny_shape && f16_pay && itk::experts_f16_takes(g, &u, np, dout);
     SplitOut sp;
-    if ((skinny_shape || f16_shape) && !be->act_split(x, x_len, (int)gate->n_in, &sp)) return;
+    const bool late = be->short_ffn(n_tok);
+    if ((skinny_shape || f16_shape) && !late && !be->act_split(x, x_len, (int)gate->n_in, &sp)) return;
     const it_hip::Grouping gr = be->grouping(np, (int)gate->n_expert);
     const int rows_tile = itk::expert_rows_tile(np, (int)gate->n_expert, g.n_in);
     it_hip::OpRec rec;
@@ -2082,8 +2106,10 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
                       as, aq, dout), rec,
                [=](hipStream_t s) {
                    const TileCount tc{cg, cu, tally, g.tier, u.tier};
-                   if (skinny_shape && experts_gemm_f16s(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(16), tc, 1.0f, 1.0f, s) && gr.made(16)) return;
-                   if (f16_shape && experts_gemm_f16(g, &u, ids, np, nu, xm, sp, dout, work, work_ints, gr.held(128), tc, 1.0f, 1.0f, s) && gr.made(128)) return;
+                   SplitOut sx = sp;
+                   if ((skinny_shape || f16_shape) && late && !be->split_at_launch(as, aq, x_len, g.n_in, &sx, s)) return;
+                   if (skinny_shape && experts_gemm_f16s(g, &u, ids, np, nu, xm, sx, dout, work, work_ints, gr.held(16), tc, 1.0f, 1.0f, s) && gr.made(16)) return;
+                   if (f16_shape && experts_gemm_f16(g, &u, ids, np, nu, xm, sx, dout, work, work_ints, gr.held(128), tc, 1.0f, 1.0f, s) && gr.made(128)) return;
                    expert_count(ids, np, g.n_expert, cg, cu, tally, s, g.tier, u.tier);
                    if (rows_shape && expert_rows(g, &u, ids, np, nu, xm, as, aq, dout, 1.0f, work, work_ints, gr.held(rows_tile), s) && gr.made(rows_tile)) return;
                    if (experts_gemm(g, &u, ids, np, nu, xm, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;

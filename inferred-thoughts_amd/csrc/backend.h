@@ -97,6 +97,17 @@ struct it_hip {
                        float** dev_x);
     // the split form of a batch's rows of `row` floats (made from the Q8_0 form, which it makes too)
     bool act_split(const float* host, size_t len, int row, itk::SplitOut* out);
+    // The routed FFN of a short batch is held back to become two launches that read none of these forms (fuser.cpp), so its
+    // expert products do not ask for one: a launch that turns out to need it makes it there, in room of the backend's own that
+    // the next launch reads and nothing else.
+    static constexpr int SHORT_FFN_TOKENS = 32;   // (measured on the 512-expert top-10 layer: 176 against 232 us at 32, 271 against 298 at 48, behind from about 56 on)
+    bool short_ffn(uint64_t n_tok) const {
+        return mode == Mode::Eager && in_pass && pass_tokens > 1 && n_tok >= 2 && n_tok <= SHORT_FFN_TOKENS && !exact && fuse_enabled &&
+               small_ffn_enabled && !expert_cold_entries;
+    }
+    itk::SplitOut launch_split;
+    size_t launch_split_cap = 0;   // floats covered
+    bool split_at_launch(const float* scales, const int8_t* quants, size_t len, int row, itk::SplitOut* out, hipStream_t s);
     bool act_q_reserve(Act& a, size_t len);  // room for the Q8_0 form of `len` floats
     Act* act_by_dev(const void* dev);        // the mirror whose device buffer holds `dev`, or null
     bool held_touches(const void* dev, size_t bytes) const;   // an op held back reads or writes inside [dev, dev + bytes)

@@ -998,7 +998,6 @@ bool references(const Op& op, const void* a, const void* b) {
 // Every link (whose output feeds whom, the shapes) is checked; a buffer that a run does not write is marked, and the run is
 // only taken if no op behind it reads that buffer.
 namespace {
-constexpr int SMALL_FFN_MAX = 32;   // tokens (measured on the 512-expert top-10 layer: 176 against 232 us at 32, 271 against 298 at 48, behind from about 56 on)
 constexpr size_t HELD_MAX = 48;
 
 bool row_wise(int id) {
@@ -1032,7 +1031,7 @@ bool changed_later(const std::vector<it_hip::OpRec>& h, size_t from, const it_hi
 bool small_ffn_next(const std::vector<it_hip::OpRec>& held, const it_hip::OpRec& r) {
     if (held.empty() || held[0].id != OP_SOFTMAX || r.i[8]) return false;
     const it_hip::OpRec& h0 = held[0];
-    if (h0.i[0] < 2 || h0.i[0] > SMALL_FFN_MAX || h0.i[1] < 16 || h0.i[1] > 2048) return false;
+    if (h0.i[0] < 2 || h0.i[0] > it_hip::SHORT_FFN_TOKENS || h0.i[1] < 16 || h0.i[1] > 2048) return false;
     if (held.size() < 2 || held[1].id != OP_ROUTE || held[1].p[0] != h0.p[0] || held[1].i[2] > 16) return false;
     int glu = 0, experts = 0, mats = 0, finish = 0;
     for (const auto& o : held) {
@@ -1093,10 +1092,7 @@ void it_hip::release_held() {
 // The complete FFN run of a short batch as two launches: gate / up with the route inside (every block ranks its
 // token's logits; grid row = token), then down + combine.  False, with nothing launched, when a link or a shape is not
 // what the kernels take.
-bool it_hip::small_ffn(const std::vector<OpRec>& run) {
-    std::vector<OpRec> h;   // (the split forms are made for kernels that this run does not use)
-    for (const OpRec& o : run)
-        if (o.id != OP_SPLIT) h.push_back(o);
+bool it_hip::small_ffn(const std::vector<OpRec>& h) {
     size_t k = 0;
     auto take = [&](int id) -> const OpRec* { return k < h.size() && h[k].id == id ? &h[k++] : nullptr; };
     const OpRec *sm = take(OP_SOFTMAX), *rt = take(OP_ROUTE), *q1 = take(OP_QUANT), *glu = take(OP_GLU), *q2 = take(OP_QUANT);
@@ -1132,7 +1128,7 @@ bool it_hip::small_ffn(const std::vector<OpRec>& run) {
     const int64_t nd = glu->i[1], ff = glu->i[2], sff = sgm->i[2];
     const void* router = sm->p[0];
     const void* x = sgm->p[2];   // the f32 activation: the shared expert's products read the same rows as the routed ones
-    if (nt < 2 || nt > SMALL_FFN_MAX || nu < 1 || nu > 16 || ne < nu) return false;
+    if (nt < 2 || nt > it_hip::SHORT_FFN_TOKENS || nu < 1 || nu > 16 || ne < nu) return false;
     if (q1 && (q1->p[0] != x || q1->i[0] != nt * nd)) return false;
     if (glu->p[6] != rt->p[1] || glu->p[7] != sgm->p[3] || glu->p[8] != sgm->p[4] || glu->i[3] != nt * nu || glu->i[4] != nu ||
         glu->i[5] != 1 || !quantized_fmt(glu->i[0]))
@@ -1188,7 +1184,7 @@ bool it_hip::small_ffn(const std::vector<OpRec>& run) {
     }
     if (!moe_glu_fast(g, stream, true) || !moe_down_fast(d, stream, true)) return false;
     uint64_t bytes = 0;
-    for (const OpRec& o : run) bytes += o.bytes;
+    for (const OpRec& o : h) bytes += o.bytes;
     Span sp(this, FAM_MOE_GLU, bytes);
     moe_glu_fast(g, stream);
     moe_down_fast(d, stream);
@@ -1225,7 +1221,7 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
     };
     const OpRec& a = h[i];
     if (a.id == OP_SOFTMAX && id(i + 1) == OP_ROUTE) {
-        if (a.i[0] >= 2 && a.i[0] <= SMALL_FFN_MAX && i == 0 && small_ffn_enabled && !expert_cold_entries) {
+        if (a.i[0] >= 2 && a.i[0] <= it_hip::SHORT_FFN_TOKENS && i == 0 && small_ffn_enabled && !expert_cold_entries) {
             size_t end = i;
             while (end < n && h[end].id != OP_FINISH) end++;
             if (end < n) {
