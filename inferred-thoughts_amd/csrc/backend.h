@@ -361,7 +361,7 @@ struct it_hip {
     void release_held();                     // issue what is held op by op, in order
     void flush_held(const OpRec* next);      // issue what is held, its known runs as one launch each; next: the op that follows, or null
     size_t fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next);   // ops of the run issued from h[i] on, 0: none begins there
-    bool small_ffn(const std::vector<OpRec>& run);   // the routed FFN of a short batch as two launches
+    bool small_ffn(const std::vector<OpRec>& held_ops, size_t end, const OpRec* next);   // the routed FFN of a short batch (held_ops[0 .. end)) as two launches
     bool small_ffn_enabled = true;           // INFERRED_HIP_NO_SMALL_FFN=1 issues it op by op (a measurement switch)
     std::vector<PreCopy> precopies;  // host -> device inputs of a graphed pass, issued before the graph
     // the embedding row of a recorded single-token pass, made by the kernel that carries its positions (x: not yet issued)

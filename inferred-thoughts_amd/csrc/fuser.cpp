@@ -1091,8 +1091,9 @@ void it_hip::release_held() {
 
 // The complete FFN run of a short batch as two launches: gate / up with the route inside (every block ranks its
 // token's logits; grid row = token), then down + combine.  False, with nothing launched, when a link or a shape is not
-// what the kernels take.
-bool it_hip::small_ffn(const std::vector<OpRec>& h) {
+// what the kernels take, or an op behind the run reads or writes what its kernels leave out.
+bool it_hip::small_ffn(const std::vector<OpRec>& held_ops, size_t end, const OpRec* next) {
+    const std::vector<OpRec> h(held_ops.begin(), held_ops.begin() + (long)end);
     size_t k = 0;
     auto take = [&](int id) -> const OpRec* { return k < h.size() && h[k].id == id ? &h[k++] : nullptr; };
     const OpRec *sm = take(OP_SOFTMAX), *rt = take(OP_ROUTE), *q1 = take(OP_QUANT), *glu = take(OP_GLU), *q2 = take(OP_QUANT);
@@ -1150,6 +1151,14 @@ bool it_hip::small_ffn(const std::vector<OpRec>& h) {
         return false;
     if (fin->p[1] != ex->p[6] || fin->p[2] != rt->p[2] || fin->p[3] != sdm->p[5] || fin->i[1] != nd || fin->i[2] != nt || fin->i[3] != nu)
         return false;
+    // What the two launches do not write: the probabilities (the router buffer keeps its logits), the shared expert's up
+    // product, the pairs' down products, the shared down product, and every quantized form of the run.  An op that was asked
+    // for before the run is issued may have taken the address of one.
+    const std::vector<const void*> skipped = {router, sum_->p[5], ex->p[6], sdm->p[5]};
+    for (const void* b : skipped)
+        if (used_later(held_ops, end, next, b)) return false;
+    for (const OpRec* q : {q1, q2, q3})
+        if (q && used_later(held_ops, end, next, q->p[2])) return false;
 
     MoeGluP g{};
     g.x = (const float*)x;
@@ -1188,9 +1197,7 @@ bool it_hip::small_ffn(const std::vector<OpRec>& h) {
     Span sp(this, FAM_MOE_GLU, bytes);
     moe_glu_fast(g, stream);
     moe_down_fast(d, stream);
-    // what the two launches do not write: the probabilities (the router buffer keeps its logits), the shared expert's
-    // up product, the pairs' down products, and every quantized form of the run
-    mark_elided({router, sum_->p[5], ex->p[6], sdm->p[5]});
+    mark_elided(skipped);
     for (const OpRec* q : {q1, q2, q3})
         if (q)
             if (Act* a = act_by_dev(q->p[0])) a->stale();
@@ -1225,7 +1232,7 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
             size_t end = i;
             while (end < n && h[end].id != OP_FINISH) end++;
             if (end < n) {
-                if (small_ffn(std::vector<OpRec>(h.begin() + i, h.begin() + end + 1))) return end + 1 - i;
+                if (small_ffn(h, end + 1, next)) return end + 1;
             }
         }
         const OpRec& r = h[i + 1];

@@ -96,7 +96,7 @@ def compare(pair, n, b0, script, outs, taken):
     for o in outs:
         want = got[1][o].astype(np.float64)
         assert np.isfinite(got[0][o]).all(), o
-        err = np.linalg.norm(got[0][o] - want) / np.linalg.norm(want)
+        err = np.linalg.norm(got[0][o] - want) / max(np.linalg.norm(want), 1e-30)
         print(o, err, launches, flush=True)
         assert err <= 1e-2, (o, err)
     # a run that is taken has ten ops in two launches; one that is not has softmax and route in one
@@ -119,6 +119,37 @@ def test_further_expert_products_behind_the_run(pair, orc, n, same_route):
         be.moe_glu(ffn.gate, ffn.up, route, b["x"], b["g2"], b["u"])
         be.matmul_experts(ffn.down, route, b["g2"], b["o2"])
     compare(pair, n, buffers(rng(11), n, NU, ffn), script, ["y", "g2", "o2"], True)
+
+
+BEHIND = {   # an op right behind the run, and the outputs to compare
+    "product_on_the_rows": lambda f, be, b: be.matmul(f.w64, b["x"], b["out"]),
+    "product_on_the_gated_rows": lambda f, be, b: be.matmul(f.w64_ff, b["e_gate"], b["out"]),
+    "sum_of_the_picks": lambda f, be, b: be.add_scaled_rows(b["acc"], b["o"], b["pick_w"]),
+    "probabilities": lambda f, be, b: be.gather_chunks(b["router"], NE, NE, 0, b["router2"]),
+    "probabilities_changed": lambda f, be, b: be.scale(b["router"], 2.0),
+    "up_product": lambda f, be, b: be.scatter_chunks(b["e_up"], FF, FF, 0, b["acc"]),
+    "new_probabilities": lambda f, be, b: be.matmul(f.router, b["y"], b["router"]),
+}
+
+
+@pytest.mark.parametrize("what", sorted(BEHIND))
+@pytest.mark.parametrize("n", [3, 8])
+def test_an_op_behind_that_uses_what_the_run_leaves_out(pair, orc, n, what):
+    ffn = Ffn(orc)
+    b = buffers(rng(15), n, NU, ffn)
+    if what == "product_on_the_rows":   # an F32 router: the rows are quantized for the experts, inside the run
+        for name, rows in (("router", NE), ("logit", 1)):
+            w = ffn.hold((rng(17).standard_normal(rows * ND) * 0.1).astype(np.float32))
+            setattr(ffn, name, ffn.ih.weights(w.view(np.uint8), ffn.ih.F32, ND, rows))
+    if what == "sum_of_the_picks":
+        b.update(pick_w=rng(16).standard_normal(n * NU).astype(np.float32), acc=z(ND))
+
+    def script(be, b):
+        if "pick_w" in b:
+            be.host_wrote(b["pick_w"])
+        ffn.run(be, b, NU)
+        BEHIND[what](ffn, be, b)
+    compare(pair, n, b, script, ["y", "out", "acc", "router2"] + (["router"] if "probabilities_" in what or "new" in what else []), False)
 
 
 @pytest.mark.parametrize("n", [8, 32])
