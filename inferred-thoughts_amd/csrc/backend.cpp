@@ -60,13 +60,15 @@ static uint64_t sig_of(const A&... a) {
     return h;
 }
 
-const int* it_hip::dyn_slot(int value) {
+const int* it_hip::dyn_slot(int value, DynRange range) {
     if (mode == Mode::Eager) return nullptr;
     if (dyn_count >= DYN_CAP) {
         need_eager("too many position-dependent launches in one pass", false);
         return nullptr;
     }
     dyn_host[dyn_count] = value;
+    dyn_range.resize(dyn_count);
+    dyn_range.push_back(range);
     return dyn_dev + dyn_count++;
 }
 
@@ -301,8 +303,6 @@ void it_hip::learn(Graph& g) {
             if ((int)i != g.ring_slot && d != 0 && d != step) g.known = false;
         }
         g.epoch = res_epoch;
-        g.pos_cap = ~0ull;
-        for (auto& r : ropes) g.pos_cap = std::min<uint64_t>(g.pos_cap, r.second.cap_pos);
         g.left.clear();
         for (auto& kv : acts)
             if (kv.second.dev_current) g.left.push_back({&kv.second, kv.second.elided, kv.second.q_valid, kv.second.q_len});
@@ -313,6 +313,8 @@ void it_hip::learn(Graph& g) {
     g.table = pass_embed.table;
     g.x = pass_embed.x;
     g.dyn.assign(dyn_host, dyn_host + dyn_count);
+    g.dyn_range = dyn_range;
+    g.dyn_range.resize(dyn_count);
 }
 
 // A whole single-token pass whose kind is known, launched from its graph: the 35 ops of a layer are not issued, hashed and
@@ -321,11 +323,19 @@ bool it_hip::replay_pass(const void* tag, uint64_t pos, const uint32_t* id, uint
     if (in_pass || !allow_graph || mid_pass_read || has_error || prof_on || expert_cold_entries || pool_tabled || !held.empty()) return false;
     Graph* g = nullptr;
     for (Graph& c : graphs)
-        if (c.valid && c.known && c.tag == tag && c.epoch == res_epoch && pos < c.pos_cap && (c.ring_slot >= 0) == (id == nullptr)) g = &c;
+        if (c.valid && c.known && c.tag == tag && c.epoch == res_epoch && (c.ring_slot >= 0) == (id == nullptr)) g = &c;
     if (!g || (id && (!g->x || *id >= (uint32_t)g->table.n_out))) return false;
+    // The ops are not issued, so neither are their checks: every scalar that follows the position (a rotation, a cache row, a
+    // context length) has to be one that its op would take.  The caller issues the pass, and gets the op's own error.
+    if (pos >= (1ull << 31)) return false;
+    const int64_t step = (int64_t)pos - (int64_t)g->pos;
+    for (size_t i = 0; i < g->dyn.size(); i++) {
+        const int64_t v = g->dyn[i] + (g->moves[i] ? step : 0);
+        if ((int)i != g->ring_slot && (v < g->dyn_range[i].lo || v > g->dyn_range[i].hi)) return false;
+    }
     dyn_rotate();
     dyn_count = g->dyn.size();
-    for (size_t i = 0; i < dyn_count; i++) dyn_host[i] = g->dyn[i] + (g->moves[i] ? (int)((int64_t)pos - (int64_t)g->pos) : 0);
+    for (size_t i = 0; i < dyn_count; i++) dyn_host[i] = g->dyn[i] + (g->moves[i] && (int)i != g->ring_slot ? (int)step : 0);
     const bool self_start = g->self_start && id && g->table.fmt == itk::W_Q8_0 && g->table.n_in == 2048 && attn_positions_agree(g->attn_slots);
     if (self_start) {
         chain_start.emb_q = (const uint8_t*)g->table.q + (size_t)*id * g->table.n_in;
@@ -1111,11 +1121,12 @@ bool it_hip::route_stage(const it_route* r, const int32_t** ids, const float** w
 }
 
 // ------------------------------------------------------------------ rope
-const float2* it_hip::rope_table(float theta, uint64_t n_rot, uint64_t need_pos) {
+const float2* it_hip::rope_table(float theta, uint64_t n_rot, uint64_t need_pos, uint64_t* rows) {
     uint32_t tb;
     memcpy(&tb, &theta, 4);
     uint64_t key = ((uint64_t)tb << 32) | n_rot;
     Rope& r = ropes[key];
+    *rows = r.cap_pos;
     if (r.cap_pos >= need_pos) return r.dev;
     need_eager("the rope table has to grow");
     size_t cap = r.cap_pos ? r.cap_pos : 8192;
@@ -1138,6 +1149,7 @@ const float2* it_hip::rope_table(float theta, uint64_t n_rot, uint64_t need_pos)
     if (r.dev) (void)hipFree(r.dev);
     r.dev = dev;
     r.cap_pos = cap;
+    *rows = cap;
     return r.dev;
 }
 
@@ -1678,10 +1690,11 @@ void it_hip_rope_neox(it_hip* be, float* x, uint64_t x_len, uint64_t pos, uint64
     if (x_len == 0 || n_rot == 0) return;
     uint64_t n = x_len / per_row;
     REQUIRE(pos + n < (1ull << 31), "rope_neox: position out of range");
-    const float2* tab = be->rope_table(theta, n_rot, pos + n);
+    uint64_t rows = 0;
+    const float2* tab = be->rope_table(theta, n_rot, pos + n, &rows);
     float* dx = be->act_inout(x, x_len);
     if (!tab || !dx) return;
-    const int* dyn = be->dyn_slot((int)pos);
+    const int* dyn = be->dyn_slot((int)pos, {0, (int)std::min<uint64_t>(rows - n, INT32_MAX)});
     int pv = dyn ? 0 : (int)pos, half = (int)(n_rot / 2), hd = (int)head_dim, nr = (int)n_rot, nh = (int)n_heads;
     int64_t nt = (int64_t)n;
     it_hip::OpRec rec;
@@ -1735,7 +1748,7 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
     if (be->exact || !split_ok) {
         float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap));
         if (!sc) return;
-        const int* dyn = be->dyn_slot((int)a->n_pos);
+        const int* dyn = be->dyn_slot((int)a->n_pos, {(int)n_q, (int)std::min<uint64_t>(slab_rows, INT32_MAX)});
         AttnArgs args{dq, dk, dv, (int)n_q, (int)a->kv_dim, dyn ? (int)n_pos_cap : (int)a->n_pos, (int)a->head_dim,
                       (int)a->n_head, (int)a->n_head_kv, a->scale, dyn};
         AttnArgs sg = args;
@@ -1762,7 +1775,7 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
         const int shares = one_pass ? attend_prefill_splits(probe) : 1;
         float* sc = be->scratch_f32(std::max(decode_floats, one_pass ? attend_prefill_floats(probe) : call_floats));
         if (!sc) return;
-        const int* dyn = be->dyn_slot((int)a->n_pos);
+        const int* dyn = be->dyn_slot((int)a->n_pos, {(int)n_q, (int)std::min<uint64_t>(slab_rows, INT32_MAX)});
         AttnArgs args{dq, dk, dv, (int)n_q, (int)a->kv_dim, dyn ? 0 : (int)a->n_pos, (int)a->head_dim,
                       (int)a->n_head, (int)a->n_head_kv, a->scale, dyn};
         it_hip::OpRec rec;
@@ -2205,7 +2218,7 @@ void it_hip_kv_write(it_hip* be, uint16_t* slab, uint64_t slab_len, uint64_t off
     const int* dyn = nullptr;
     int64_t mul = 0, off = (int64_t)offset, n = (int64_t)src_len;
     if (be->mode != it_hip::Mode::Eager && offset % src_len == 0 && offset / src_len < (1ull << 31)) {
-        dyn = be->dyn_slot((int)(offset / src_len));
+        dyn = be->dyn_slot((int)(offset / src_len), {0, (int)std::min<uint64_t>(slab_len / src_len - 1, INT32_MAX)});
         if (dyn) {
             mul = n;
             off = 0;
@@ -2693,7 +2706,7 @@ int it_hip_embed_argmax(it_hip* be, const it_weights* table, const float* logits
     float* dx = be->act_out(x, x_len);
     if (!dx || !be->argmax_ready()) return 0;
     const int slot = (int)(ring_index % it_hip::TOK_RING_CAP);
-    const int* dyn = be->dyn_slot(slot);
+    const int* dyn = be->dyn_slot(slot, {0, (int)it_hip::TOK_RING_CAP - 1});
     if (dyn) be->pass_ring_slot = (int)(dyn - be->dyn_dev);
     int32_t *out = be->argmax_out, *idx = be->argmax_idx, *ring = be->tok_ring;
     float* val = be->argmax_val;

@@ -223,7 +223,7 @@ struct it_hip {
         size_t cap_pos = 0;
     };
     std::unordered_map<uint64_t, Rope> ropes;
-    const float2* rope_table(float theta, uint64_t n_rot, uint64_t need_pos);
+    const float2* rope_table(float theta, uint64_t n_rot, uint64_t need_pos, uint64_t* rows);   // rows: how many the table has
 
     // ---- scratch
     float* attn_scratch = nullptr;
@@ -241,6 +241,9 @@ struct it_hip {
     // ---- pass / graph state
     bool in_pass = false;
     uint64_t pass_tokens = 0;
+    struct DynRange {
+        int lo, hi;   // both inclusive
+    };
     // decode graph (captured stream work of one n == 1 pass)
     struct Graph {
         hipGraph_t graph = nullptr;
@@ -254,8 +257,9 @@ struct it_hip {
         // replay_pass: the caller's tag of this kind of pass, a pass it recorded (position, position scalars) and, once a
         // second pass has shown which scalars follow the position, what a pass leaves behind (the mirrors that are current)
         const void* tag = nullptr;
-        uint64_t pos = 0, pos_cap = 0, epoch = 0;
+        uint64_t pos = 0, epoch = 0;
         std::vector<int> dyn;
+        std::vector<DynRange> dyn_range;   // what each scalar may be: the op's own check, which a replayed pass skips
         std::vector<uint8_t> moves;
         int ring_slot = -1;          // the scalar that is the token ring's index (a pass fed by the arg-max), or -1
         itk::WView table{};          // the embedding table and row of a pass fed by the host
@@ -394,7 +398,9 @@ struct it_hip {
     void dyn_upload();
     size_t dyn_count = 0;
     static constexpr size_t DYN_CAP = 4096;
-    const int* dyn_slot(int value);   // null in eager mode: the kernel takes the scalar by value
+    std::vector<DynRange> dyn_range;   // of the pass's scalars, in step with dyn_count
+    // null in eager mode: the kernel takes the scalar by value.  range: the values that the op would accept.
+    const int* dyn_slot(int value, DynRange range);
     // leave capture/replay: run what the pass queued so far eagerly.  `moved`: a buffer is about to be allocated, moved or
     // filled anew, so that what earlier passes found in place has to be looked at again (replay_pass)
     void need_eager(const char* why, bool moved = true);
