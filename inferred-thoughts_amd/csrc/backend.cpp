@@ -231,7 +231,7 @@ void it_hip::finish_pass() {
                 graph->direct = graph->launches.size() <= 4 && chain_layers <= 4;
                 // every position of the pass belongs to an attention layer inside the one chain (rope twice, the two cache
                 // writes and the attention of each), so nothing else waits for the kernel that carries them
-                graph->self_start = graph->direct && graph->launches.size() <= 2 && chain_launches == 1 && chain_attn == fused_attn_slots.size() &&
+                graph->self_start = graph->direct && graph->launches.size() == 2 && chain_launches == 1 && chain_attn == fused_attn_slots.size() &&
                                     dyn_count == 5 * fused_attn_slots.size() && pass_embed.x && pass_embed.x == chain_x && precopies.empty();
                 graph->valid = true;
                 stable_passes = 1;

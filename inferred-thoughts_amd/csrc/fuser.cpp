@@ -26,7 +26,7 @@ struct Plan {
     std::vector<char> consumed;
     // which stage of a layer a fused launch is (0: none of them), with its arguments: the chain pass below rebuilds
     // runs of them as one persistent kernel
-    enum Stage { ST_NONE = 0, ST_GDN_IN, ST_GDN_CORE, ST_GDN_OUT, ST_ROUTER, ST_GLU, ST_DOWN, ST_ATTN_IN, ST_ATTEND, ST_ATTN_OUT, ST_HEAD };
+    enum Stage { ST_NONE = 0, ST_GDN_IN, ST_GDN_CORE, ST_GDN_OUT, ST_ROUTER, ST_GLU, ST_DOWN, ST_ATTN_IN, ST_ATTEND, ST_ATTN_OUT };
     struct Launch {
         int fam;         // it_hip::Family, for the per-kernel timing
         uint64_t bytes;  // algorithmic bytes of the launch (weights + state it must move once)
@@ -280,9 +280,7 @@ bool match_final(Plan& pl, size_t i, int exact) {
     a.n_mats = 1;
     a.m[0] = mat_of(m, 0);
     pl.take(i, 4);
-    Plan::Launch& l = pl.add(i, it_hip::FAM_LM_HEAD, gemv_bytes(a), [=](hipStream_t s) { fused_gemv(a, s); });
-    l.stage = Plan::ST_HEAD;
-    l.gv = a;
+    pl.add(i, it_hip::FAM_LM_HEAD, gemv_bytes(a), [=](hipStream_t s) { fused_gemv(a, s); });
     return true;
 }
 
@@ -724,21 +722,6 @@ bool chain_attn_in(const FusedGemvP& a, ChainTail* t) {
     return true;
 }
 
-// the output matrix as a short chain's last stage
-bool chain_head(const FusedGemvP& a, ChainHead* h) {
-    if (a.exact || a.mode != 1 || a.n_in != 2048 || a.n_mats != 1 || a.route_counter || a.m[0].fmt != W_Q8_0 || a.m[0].epi != 0 ||
-        a.m[0].n_out < 1 || a.m[0].n_out > CHAIN_HEAD_ROWS)
-        return false;
-    if (!al16(a.m[0].q) || !al16(a.m[0].s) || !al16(a.norm_w) || !a.x_copy || !al16(a.x_copy)) return false;
-    h->norm_w = a.norm_w;
-    h->q = a.m[0].q; h->s = a.m[0].s;
-    h->out = a.m[0].out;
-    h->normed = a.x_copy;
-    h->eps = a.eps;
-    h->rows = a.m[0].n_out;
-    return true;
-}
-
 // a whole attention block as a chain layer: in-projection, attention launch and out-projection must be the shapes the
 // chain's stages are written for and hang together (the attention reads what the in-projection writes and writes what
 // the out-projection reads; the gate is the second half of every head's wq rows)
@@ -784,7 +767,6 @@ void build_chains(Plan& pl, unsigned long long* tally) {
         size_t pos;
         Kind kind;
     };
-    size_t head_pos = 0;   // position of the output matrix that is cp's head
     size_t tail_pos = 0;   // position of the attention block whose in-projection is cp's tail
     // (30 KB, nearly all of it the layer array: on the heap, and only the entries in use are cleared and copied)
     std::unique_ptr<ChainP, void (*)(void*)> cp_box((ChainP*)calloc(1, sizeof(ChainP)), free);
@@ -810,7 +792,6 @@ void build_chains(Plan& pl, unsigned long long* tally) {
             n--;
             n_units--;
             cp.has_tail = 0;
-            cp.head.rows = 0;
         }
         if (n >= 1 && be->chain_acquire()) {
             cp.n_layers = n;
@@ -848,7 +829,6 @@ void build_chains(Plan& pl, unsigned long long* tally) {
                     skips_of(units[u].kind == U_GDN ? pl.gdn_skips : pl.ffn_skips, units[u].pos, &be->fused_elided);
                 }
             }
-            if (cp.head.rows) pl.at[head_pos].clear();
             if (cp.has_tail) {
                 drop_stage(tail_pos, Plan::ST_ATTN_IN);
                 skips_of(pl.attn_skips, tail_pos, &be->fused_elided);
@@ -958,13 +938,6 @@ void build_chains(Plan& pl, unsigned long long* tally) {
             }
         }
         if (taken) continue;
-        if (ls.size() == 1 && ls[0].stage == Plan::ST_HEAD && !mixer_open && cp.n_layers >= 1 && cp.n_layers <= CHAIN_SHORT_LAYERS &&
-            cp.x == ls[0].gv.x && chain_head(ls[0].gv, &cp.head)) {
-            head_pos = i;
-            bytes += ls[0].bytes;
-            emit();
-            continue;
-        }
         // anything that runs here ends the run: other fused launches, or an op issued as it is
         if (!ls.empty() || !pl.consumed[i]) emit();
     }

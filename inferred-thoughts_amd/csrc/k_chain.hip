@@ -349,15 +349,6 @@ IT_DEV void fetch_tail(const T& t, AW& a, int b, int wave, int lane) {
     load_row<W_Q8_0, 2, 64>(a.t[4], kk ? t.k_q : t.v_q, kk ? t.k_s : t.v_s, D, b + NB * (wave & 1), lane, wave < 4);
 }
 
-// four rows a wave of the output matrix, from row 8,192 * part on
-IT_DEV void fetch_head(const ChainHead& h, int part, AW& a, int b, int wave, int lane) {
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const int row = 4 * NB * CW * part + b + NB * (wave + CW * k);
-        load_row<W_Q8_0, 2, 64>(a.t[k], h.q, h.s, D, row, lane, row < h.rows);
-    }
-}
-
 // An NVFP4 chunk against the activation through gfx950's own conversions: v_cvt_scalef32_pk_f16_fp4 turns one byte (two
 // e2m1 nibbles) into two f16 and v_dot2_f32_f16 multiplies them with two f16 activations, 2 instructions for 2 elements
 // where nibbles -> int8 through v_perm_b32 + v_dot4 takes 7 for 4.  The activations are the Q8_0 quants as f16 (exact),
@@ -1402,7 +1393,6 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
         // own wave has in flight)
         auto fetch_next = [&]() {
             if (l + 1 == p.n_layers && p.has_tail) fetch_tail(p.tail, aw, b, wave, lane);
-            if (NL == CHAIN_SHORT_LAYERS && l + 1 == p.n_layers && p.head.rows) fetch_head(p.head, 0, aw, b, wave, lane);
             if (l + 1 < p.n_layers && p.layer[l + 1].has_mixer == 3) fetch_tail(p.layer[l + 1].a, aw, b, wave, lane);
             if (next_mixer && ((IT_CHAIN_A_AT >> 4) & 15)) fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane, (IT_CHAIN_A_AT >> 4) & 15);
         };
@@ -1545,39 +1535,6 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             }
         }
     }
-    // -------------------------------------------------------------------- head: the final norm and the output matrix
-    if (NL == CHAIN_SHORT_LAYERS && p.head.rows) {
-        __syncthreads();
-        if (!dead) {
-            int tid = tid0, b = b0;
-            asm volatile("" : "+v"(tid), "+s"(b));
-            const int lane = tid & 63;
-            const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-            const ChainHead& t = p.head;
-            const unsigned e = e0 + 1u + (unsigned)p.n_layers;
-            const float4 nw = ((const float4*)t.norm_w)[tid];
-            float* const nf = (float*)route_sh.keys;
-            float4 v;
-            if (!ll_wait_quad(p.ll + RX, tid, e, ctl, &v)) dead = 1;
-            if (norm_quant(v, nw, t.eps, xq, xs, red, &dead, tid, nf)) {
-                if (b == 0) ((float4*)t.normed)[tid] = ((const float4*)nf)[tid];
-                XChunks<W_Q8_0, 2> x;
-                load_x<W_Q8_0, 2, 64>(x, xq, xs, lane);
-                for (int part = 0; part * 4 * NB * CW < t.rows; part++) {
-                    if (part) fetch_head(t, part, aw, b, wave, lane);
-                    float mine = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        const float acc = reduce_lanes<64>(dot_chunks<W_Q8_0, 2>(aw.t[k], x));
-                        const float r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 63));
-                        mine = lane == k ? r : mine;
-                    }
-                    const int row = 4 * NB * CW * part + b + NB * (wave + CW * lane);
-                    if (lane < 4 && row < t.rows) t.out[row] = mine;
-                }
-            }
-        }
-    }
     if (b0 == 0 && tid0 == 0) *p.epoch = e0 + 1u + (unsigned)p.n_layers;
 }
 
@@ -1642,8 +1599,6 @@ bool layer_chain(const ChainP& p, hipStream_t s) {
     }
     if (p.has_tail && !all({p.tail.norm_w, p.tail.q_q, p.tail.q_s, p.tail.k_q, p.tail.k_s, p.tail.v_q, p.tail.v_s, p.tail.out_q,
                             p.tail.out_k, p.tail.out_v}))
-        return false;
-    if (p.head.rows && (p.n_layers > CHAIN_SHORT_LAYERS || p.has_tail || p.head.rows > CHAIN_HEAD_ROWS || !all({p.head.norm_w, p.head.q, p.head.s, p.head.out, p.head.normed})))
         return false;
     if (!layer_chain_fits()) return false;
     const size_t lds = has_attn ? ATTN_LDS : 0;

@@ -170,15 +170,6 @@ struct ChainTail {
     it_gptr<float> out_q, out_k, out_v;
     float eps;
 };
-// The product behind a token's last layer (final norm, the rows of the output matrix, Q8_0) as a short chain's last stage:
-// its first four rows a wave are on their way before the last layer is done.
-struct ChainHead {
-    it_gptr<const float> norm_w;
-    it_gptr<const uint8_t> q, s;
-    it_gptr<float> out, normed;      // the results; the normed vector
-    float eps;
-    int rows;                        // 0: no such stage
-};
 // A whole attention mixer inside the chain (has_mixer == 3): in-projection, norm + rotation of the query heads and of
 // the new key, the cache rows of the new position, attention over the context split over the blocks, merge + sigmoid
 // gate; the out-projection's matrix is the layer's ChainMixer o_q / o_s.  16 query heads of 256 on 2 KV heads.
@@ -215,7 +206,6 @@ template <int NL> struct ChainPT {
     int n_layers;
     int has_tail;
     ChainTail tail;
-    ChainHead head;
     int sh_fmt;                  // the shared expert's format (W_Q8_0 or W_NVFP4)
     int rf;                      // 1: the router, the shared expert's gate-logit row and ssm alpha / beta are F32 matrices (as real
                                  // files keep them; their *_q pointers hold floats, their *_s are null), 0: Q8_0
@@ -237,8 +227,6 @@ typedef ChainPT<CHAIN_MAX_LAYERS> ChainP;
 // A chain of up to this many layers is launched with a small argument block: a launch queued outside a graph pays the
 // host's copy of its arguments (8-10 us for 30 KB against 2.5 us for 2 KB, measured; a replayed graph pays neither).
 constexpr int CHAIN_SHORT_LAYERS = 4;
-// ... and takes the output matrix up to this many rows (8 a wave; a larger one streams better in a launch of its own)
-constexpr int CHAIN_HEAD_ROWS = 16384;
 // whether this device can hold the chain's grid (one block per compute unit, all resident at once)
 bool layer_chain_fits();
 // false: not launched
