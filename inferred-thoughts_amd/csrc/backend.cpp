@@ -229,10 +229,6 @@ void it_hip::finish_pass() {
                 graph->has_chain = chain_launches > 0;
                 graph->launches = std::move(fused_runs);
                 graph->direct = graph->launches.size() <= 4 && chain_layers <= 4;
-                // every position of the pass belongs to an attention layer inside the one chain (rope twice, the two cache
-                // writes and the attention of each), so nothing else waits for the kernel that carries them
-                graph->self_start = graph->direct && graph->launches.size() == 2 && chain_launches == 1 && chain_attn == fused_attn_slots.size() &&
-                                    dyn_count == 5 * fused_attn_slots.size() && pass_embed.x && pass_embed.x == chain_x && precopies.empty();
                 graph->valid = true;
                 stable_passes = 1;
             } else if (g) {
@@ -336,18 +332,10 @@ bool it_hip::replay_pass(const void* tag, uint64_t pos, const uint32_t* id, uint
     dyn_rotate();
     dyn_count = g->dyn.size();
     for (size_t i = 0; i < dyn_count; i++) dyn_host[i] = g->dyn[i] + (g->moves[i] && (int)i != g->ring_slot ? (int)step : 0);
-    const bool self_start = g->self_start && id && g->table.fmt == itk::W_Q8_0 && g->table.n_in == 2048 && attn_positions_agree(g->attn_slots);
-    if (self_start) {
-        chain_start.emb_q = (const uint8_t*)g->table.q + (size_t)*id * g->table.n_in;
-        chain_start.emb_s = (const uint16_t*)g->table.scales + (size_t)*id * (g->table.n_in / 32);
-        chain_start.n_pos = g->attn_slots.empty() ? 0 : dyn_host[g->attn_slots[0][3]];
-    } else {
-        if (id) pre_embed = {g->table, (int)*id, g->x};
-        else dyn_host[g->ring_slot] = (int)(ring_index % TOK_RING_CAP);
-        issue_inputs();
-    }
+    if (id) pre_embed = {g->table, (int)*id, g->x};
+    else dyn_host[g->ring_slot] = (int)(ring_index % TOK_RING_CAP);
+    issue_inputs();
     launch(*g);
-    chain_start = ChainStart{};
     g->replays++;
     launches += g->signature.size();
     for (auto& kv : acts) {

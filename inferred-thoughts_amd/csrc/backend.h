@@ -253,7 +253,6 @@ struct it_hip {
         uint64_t born = 0, replays = 0;
         std::vector<std::function<void(hipStream_t)>> launches;   // what the graph holds
         bool direct = false;         // launched one by one (launch)
-        bool self_start = false;     // one chain and what reads its result: the chain can take the embedding row and the position itself
         // replay_pass: the caller's tag of this kind of pass, a pass it recorded (position, position scalars) and, once a
         // second pass has shown which scalars follow the position, what a pass leaves behind (the mirrors that are current)
         const void* tag = nullptr;
@@ -339,15 +338,7 @@ struct it_hip {
     bool eager_fused = false;          // single-token passes without a graph still go through the fuser (measurement switch)
     bool chain_ran = false;            // a chain has been issued since the abort word was last looked at
     int chain_spin_limit = 1 << 21;
-    uint64_t chain_launches = 0, chain_layers = 0, chain_attn = 0;   // per fused pass (chain_attn: attention layers inside its chains)
-    const float* chain_x = nullptr;                  // the residual stream of the pass's last chain
-    // what the chain about to be launched takes from its arguments (null, 0: nothing)
-    struct ChainStart {
-        const uint8_t* emb_q = nullptr;
-        const uint16_t* emb_s = nullptr;
-        int n_pos = 0;
-    };
-    ChainStart chain_start;
+    uint64_t chain_launches = 0, chain_layers = 0;   // per fused pass, for the statistics
     bool chain_acquire();
     void chain_release();
     void chain_gave_up();

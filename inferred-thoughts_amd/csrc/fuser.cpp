@@ -834,15 +834,9 @@ void build_chains(Plan& pl, unsigned long long* tally) {
                 skips_of(pl.attn_skips, tail_pos, &be->fused_elided);
             }
             pl.add(units[0].pos, it_hip::FAM_CHAIN, bytes, [=](hipStream_t s) {
-                // (a pass launched from its own arguments: replay_pass)
-                launch->emb_q = be->chain_start.emb_q;
-                launch->emb_s = be->chain_start.emb_s;
-                launch->n_pos = be->chain_start.n_pos;
                 if (!layer_chain(*launch, s)) be->fail("layer chain: the persistent kernel could not be launched");
             });
             be->chain_launches++;
-            be->chain_x = launch->x;
-            for (int l = 0; l < n; l++) be->chain_attn += launch->layer[l].has_mixer == 3;
             be->chain_layers += (uint64_t)n;
         }
         memset((void*)&cp, 0, cp_head + (size_t)cp_touched * sizeof(ChainLayer));
@@ -1415,8 +1409,7 @@ void it_hip::run_fused(std::vector<OpRec>& ops) {
     Plan pl(this, ops);
     fused_attn_slots.clear();
     fused_elided.clear();
-    chain_launches = chain_layers = chain_attn = 0;
-    chain_x = nullptr;
+    chain_launches = chain_layers = 0;
     if (fuse_enabled) {
         for (size_t i = 0; i < ops.size(); i++) {
             if (pl.consumed[i]) continue;

@@ -44,7 +44,6 @@
 // grid drains.  The grid must be resident at once (one block per compute unit), which the launcher checks.
 #include <cstddef>
 #include <cstring>
-#include <type_traits>
 #define IT_CHAIN_DEVICE_POINTERS
 #include "it_fast.h"
 #include "kernels_fused.h"
@@ -451,6 +450,7 @@ struct AttnCoreP {   // what of a ChainAttn the function reads
     it_gptr<const float> q_norm, k_norm;
     it_gptr<const float2> rope;
     it_gptr<uint16_t> k_slab, v_slab;
+    it_gptr<const int> n_pos;
     it_gptr<const uint8_t> o_q, o_s;   // the out-projection
     float eps_head, scale;
     int n_rot;
@@ -460,16 +460,14 @@ struct AttnCoreR {
     int ok;      // 0: one of this thread's waits gave up
 };
 // (the arguments one by one, so that they travel in registers: a struct by value goes through the stack)
-// (n_pos: the positions in the context, or where they stand)
-template <class N>
 __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_norm, it_gptr<const float> k_norm, it_gptr<const float2> rope,
-                                                         it_gptr<uint16_t> k_slab, it_gptr<uint16_t> v_slab, N n_pos_in,
+                                                         it_gptr<uint16_t> k_slab, it_gptr<uint16_t> v_slab, it_gptr<const int> n_pos_p,
                                                          it_gptr<const uint8_t> o_q, it_gptr<const uint8_t> o_s, float eps_head, float scale,
                                                          int n_rot, it_gptr<u64> ll_g, unsigned e, it_gptr<unsigned> abort_g, int spin_limit, int tid,
                                                          int b) {
     u64* const ll = (u64*)ll_g;   // (polled through explicit global loads, stored to as global: see ll_put)
     unsigned* const abort_flag = (unsigned*)abort_g;
-    const AttnCoreP at{q_norm, k_norm, rope, k_slab, v_slab, o_q, o_s, eps_head, scale, n_rot};
+    const AttnCoreP at{q_norm, k_norm, rope, k_slab, v_slab, n_pos_p, o_q, o_s, eps_head, scale, n_rot};
     const Ctl ctl{abort_flag, spin_limit};
 #ifdef IT_CHAIN_STAMPS
     long long ac_prev = wall_clock64();
@@ -497,9 +495,7 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
     float* const ws = sm + 8;            // 8 waves x 4 dim groups x (4 sums + the weight)
     float* const Ot = ws + 8 * 4 * 5;    // [8 waves][8 heads][32 dims]: a wave's weighted sums on their way to its stores
     bool ok = true;
-    int n_pos;
-    if constexpr (std::is_same_v<N, int>) n_pos = n_pos_in;
-    else n_pos = *n_pos_in;
+    const int n_pos = *at.n_pos;
     const int kpb = max(1, (n_pos + AS - 1) / AS);
     {
         const int kvh = b & 1, split = b >> 1;
@@ -757,15 +753,6 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
     return AttnCoreR{dot, ok ? 1 : 0};
 }
 
-// four elements of the residual stream as the chain finds it: in memory, or (short chains, which are launched outside a
-// graph) the token's embedding row, with embed8's arithmetic
-template <int NL> IT_DEV float4 first_x(const ChainPT<NL>& p, int tid) {
-    if (NL != CHAIN_SHORT_LAYERS || !p.emb_q) return ((const float4*)p.x)[tid];
-    const uint32_t q = ((const uint32_t*)p.emb_q)[tid];
-    const float d = it_f16_to_f32(p.emb_s[tid >> 3]);
-    return make_float4(d * (float)(int8_t)q, d * (float)(int8_t)(q >> 8), d * (float)(int8_t)(q >> 16), d * (float)(int8_t)(q >> 24));
-}
-
 template <int SF, int RF, int NL>
 __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
     __shared__ __align__(16) int8_t xq[NU * FF + FF];   // the stage's quantized activation (largest: the down stage's)
@@ -787,12 +774,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
     const unsigned e0 = *(const volatile unsigned*)p.epoch;
     if (tid0 == 0) dead = 0;
     // lane 63 of a wave owns one row of the residual stream: row 8 * block + wave
-    float x_row = 0.0f;
-    if ((tid0 & 63) == 63) {
-        const int row = b0 * CW + (tid0 >> 6);
-        if (NL == CHAIN_SHORT_LAYERS && p.emb_q) x_row = it_f16_to_f32(p.emb_s[row >> 5]) * (float)(int8_t)p.emb_q[row];
-        else x_row = p.x[row];
-    }
+    float x_row = (tid0 & 63) == 63 ? p.x[b0 * CW + (tid0 >> 6)] : 0.0f;
     AW aw;
     if (p.layer[0].has_mixer == 1) fetch_a<RF>(p.layer[0].m, aw, b0, __builtin_amdgcn_readfirstlane(tid0 >> 6), tid0 & 63);
     if (p.layer[0].has_mixer == 3) fetch_tail(p.layer[0].a, aw, b0, __builtin_amdgcn_readfirstlane(tid0 >> 6), tid0 & 63);
@@ -888,7 +870,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 const float4 nw = ((const float4*)at.norm_w)[tid];
                 float4 v;
                 bool ok = true;
-                if (l == 0) v = first_x(p, tid);
+                if (l == 0) v = ((const float4*)p.x)[tid];
                 else ok = ll_wait_quad(p.ll + RX, tid, e, ctl, &v);
                 if (!ok) dead = 1;
                 CH_STAMP(16);
@@ -910,13 +892,8 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             // ---------------------------------------------------------------- attention over the context, merge, sigmoid gate
             // (a function of its own: its registers are allotted apart from the stages around it, which have none to spare)
             forget(aw);
-            auto core = [&](auto n_pos) __attribute__((always_inline)) {
-                return attn_core(at.q_norm, at.k_norm, at.rope, at.k_slab, at.v_slab, n_pos, m.o_q, m.o_s, at.eps_head, at.scale, at.n_rot,
-                                 (it_gptr<u64>)p.ll, e, (it_gptr<unsigned>)p.abort_flag, p.spin_limit, tid, b);
-            };
-            AttnCoreR r;
-            if constexpr (NL == CHAIN_SHORT_LAYERS) r = core(p.n_pos ? p.n_pos : (int)*at.n_pos);
-            else r = core(at.n_pos);
+            const AttnCoreR r = attn_core(at.q_norm, at.k_norm, at.rope, at.k_slab, at.v_slab, at.n_pos, m.o_q, m.o_s, at.eps_head, at.scale, at.n_rot,
+                                          (it_gptr<u64>)p.ll, e, (it_gptr<unsigned>)p.abort_flag, p.spin_limit, tid, b);
             CH_STAMP(18);
             fetch_d();
             if (!r.ok) dead = 1;
@@ -941,7 +918,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             {
                 float4 v;
                 bool ok = true;
-                if (l == 0) v = first_x(p, tid);
+                if (l == 0) v = ((const float4*)p.x)[tid];
                 else ok = ll_wait_quad(p.ll + RX, tid, e, ctl, &v);
                 if (!ok) dead = 1;
                 if (!norm_quant(v, nw, m.eps_norm, xq, xs, red, &dead, tid, xf)) break;
@@ -1152,7 +1129,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             float4 v;
             bool ok = true;
             if (mixer) ok = ll_wait_quad(p.ll + RC, tid, e, ctl, &v);
-            else if (l == 0) v = first_x(p, tid);
+            else if (l == 0) v = ((const float4*)p.x)[tid];
             else ok = ll_wait_quad(p.ll + RX, tid, e, ctl, &v);
             if (!ok) dead = 1;
             if (!norm_quant(v, nw, f.eps, xq, xs, red, &dead, tid, xf)) break;

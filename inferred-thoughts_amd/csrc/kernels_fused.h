@@ -215,12 +215,6 @@ template <int NL> struct ChainPT {
     it_gptr<unsigned> abort_flag;        // uncached device word: set when a bounded wait gave up (the results are then void)
     it_gptr<unsigned long long> tally;   // expert read tally (optional)
     int spin_limit;              // polls a wait may take before it gives up
-    // A chain that opens its pass may take from its arguments what a kernel in front of it would have put in place (a launch's
-    // 4 us, and as much of host time, per token): the token's row of a Q8_0 embedding table instead of x (emb_q null: x as it
-    // stands), and the positions in the context (0: as the layers' n_pos words say).
-    int n_pos;
-    it_gptr<const uint8_t> emb_q;
-    it_gptr<const uint16_t> emb_s;
     ChainLayer layer[NL];   // (last: host code copies and clears the n_layers entries in use, not all 30 KB)
 };
 typedef ChainPT<CHAIN_MAX_LAYERS> ChainP;
