@@ -227,8 +227,6 @@ void it_hip::finish_pass() {
                 graph->attn_slots = fused_attn_slots;
                 graph->elided = fused_elided;
                 graph->has_chain = chain_launches > 0;
-                graph->launches = std::move(fused_runs);
-                graph->direct = graph->launches.size() <= 4 && chain_layers <= 4;
                 graph->valid = true;
                 stable_passes = 1;
             } else if (g) {
@@ -270,15 +268,6 @@ void it_hip::finish_pass() {
 }
 
 void it_hip::launch(Graph& g) {
-    // Up to four launches with small argument blocks go out one by one, 7 us a token sooner on two layers (70.6 against 77.7 us
-    // back to back).  A chain of more than four layers has a 30 KB block, which the graph holds and a launch copies (48
-    // layers: 1.419 ms a token so, 1.407 as a graph), and long lists cost the host more than the graph does.
-    if (g.direct) {
-        for (auto& f : g.launches) f(stream);
-        check(hipGetLastError(), "kernel launch");
-        graph_launches++;
-        return;
-    }
     check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
     graph_launches++;
 }

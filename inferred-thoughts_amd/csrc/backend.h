@@ -251,8 +251,6 @@ struct it_hip {
         std::vector<uint64_t> signature;  // hash of each seam call's static arguments
         bool valid = false;
         uint64_t born = 0, replays = 0;
-        std::vector<std::function<void(hipStream_t)>> launches;   // what the graph holds
-        bool direct = false;         // launched one by one (launch)
         // replay_pass: the caller's tag of this kind of pass, a pass it recorded (position, position scalars) and, once a
         // second pass has shown which scalars follow the position, what a pass leaves behind (the mirrors that are current)
         const void* tag = nullptr;
@@ -318,7 +316,6 @@ struct it_hip {
     bool fuse_enabled = true;
     unsigned* route_counter = nullptr;  // device word used by the fused router (zero between launches)
     uint64_t fused_launches = 0;  // launches in the captured graph after fusion
-    std::vector<std::function<void(hipStream_t)>> fused_runs;   // those launches
     void run_fused(std::vector<OpRec>& ops);
     std::vector<std::array<int, 4>> fused_attn_slots;  // filled by run_fused for the pass being captured
     // ---- layer chains (k_chain.hip): runs of decode layers as one persistent kernel each

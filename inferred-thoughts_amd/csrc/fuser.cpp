@@ -1440,18 +1440,18 @@ void it_hip::run_fused(std::vector<OpRec>& ops) {
         }
     }
     if (fuse_enabled && !expert_cold_entries) build_chains(pl, expert_tally);
-    fused_runs.clear();
+    uint64_t n = 0;
     for (size_t i = 0; i < ops.size(); i++) {
         for (auto& l : pl.at[i]) {
             Span sp(this, l.fam, l.bytes);
             l.fn(stream);
-            fused_runs.push_back(l.fn);
+            n++;
         }
         if (!pl.consumed[i]) {
             Span sp(this, FAM_OTHER, 0);
             ops[i].run(stream);
-            fused_runs.push_back(ops[i].run);
+            n++;
         }
     }
-    fused_launches = fused_runs.size();
+    fused_launches = n;
 }
