@@ -2538,6 +2538,21 @@ int64_t it_hip_clock_pick(uint8_t* heat, const uint8_t* leased, uint64_t n, uint
 // ------------------------------------------------------------------ extensions
 }  // extern "C"
 
+namespace {
+// The device's address of a host buffer that lies in one page-locked allocation from end to end, or null.  Asked at every
+// read (0.2 us): the caller may have freed the buffer since, and been given pageable memory at its address.
+float* locked_view(float* buf, size_t bytes) {
+    hipPointerAttribute_t at;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    const bool whole = ((uintptr_t)buf & 15) == 0 && hipPointerGetAttributes(&at, buf) == hipSuccess && at.type == hipMemoryTypeHost && at.devicePointer &&
+                       ((uintptr_t)at.devicePointer & 15) == 0 && hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)at.devicePointer) == hipSuccess &&
+                       (uintptr_t)at.devicePointer + bytes <= (uintptr_t)base + size;
+    (void)hipGetLastError();
+    return whole ? (float*)at.devicePointer : nullptr;
+}
+}  // namespace
+
 // A read by the host: a kernel behind the pass writes the floats, the chains' abort word and then a sequence number into
 // page-locked memory, and the host watches that number.  Against a copy, a stream synchronisation and a second copy for the
 // abort word (32 KB: 45 us after the pass's last kernel) the host has the values a few microseconds after it.
@@ -2555,12 +2570,8 @@ bool it_hip::fetch(Act& a, float* buf, size_t n) {
         fill_zero(home.arrived, 4, stream);
         home.cells = p;
     }
-    if (a.host_locked < 0) {
-        hipPointerAttribute_t at;
-        a.host_locked = hipPointerGetAttributes(&at, buf) == hipSuccess && at.type == hipMemoryTypeHost && (((uintptr_t)buf) & 15) == 0;
-        (void)hipGetLastError();
-    }
-    float* to = a.host_locked ? buf : home.stage;
+    float* const direct = locked_view(buf, n * sizeof(float));
+    float* const to = direct ? direct : home.stage;
     const unsigned seq = ++home.seq;
     itk::fetch(a.dev, to, (int64_t)n, chain_ran ? chain.abort_flag : nullptr, home.cells + 16, home.arrived, home.cells, seq, stream);
     if (!check(hipGetLastError(), "download activation")) return true;
@@ -2579,7 +2590,7 @@ bool it_hip::fetch(Act& a, float* buf, size_t n) {
         fail("download activation: the device did not report the end of the pass");
         return true;
     }
-    if (!a.host_locked) memcpy(buf, to, n * sizeof(float));
+    if (!direct) memcpy(buf, to, n * sizeof(float));
     if (chain_ran) {
         chain_ran = false;
         if (home.cells[16]) chain_gave_up();

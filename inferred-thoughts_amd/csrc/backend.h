@@ -78,7 +78,6 @@ struct it_hip {
         int s_row = 0;
         bool s_valid = false;
         void stale() { q_valid = s_valid = false; }
-        int host_locked = -1;  // the host buffer is page-locked (fetch): not asked yet, no, yes
     };
     struct Home {
         unsigned* cells = nullptr;     // page-locked: [0] sequence number, [16] abort word

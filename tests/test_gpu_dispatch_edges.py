@@ -60,6 +60,32 @@ def test_copies_home_by_size(hip, n):
         hip.release(a)
 
 
+@pytest.mark.parametrize("at,n", [(0, 4096), (4, 4092), (1, 4095), (0, 5), (4080, 16)])
+def test_copies_home_into_page_locked_memory(hip, at, n):
+    """Aligned ranges of a page-locked allocation, up to its end, are written by the device itself, others through the
+    backend's own; the same addresses in turn with pageable ones, on one backend."""
+    import ctypes as C
+    fresh(hip)
+    rt = C.CDLL("libamdhip64.so")
+    p = C.c_void_p()
+    assert rt.hipHostMalloc(C.byref(p), C.c_size_t(4096 * 4), 0) == 0
+    try:
+        locked = np.frombuffer((C.c_float * 4096).from_address(p.value), np.float32)
+        locked[:] = -1.0
+        a, x = locked[at:at + n], rng(n).standard_normal(n).astype(np.float32)
+        for k in range(3):
+            pageable = x.copy()
+            a[:] = x
+            for buf in (a, pageable):
+                hip.host_wrote(buf); hip.scale(buf, 2.0 + k); hip.host_needs(buf)
+                assert np.array_equal(buf, np.float32(2.0 + k) * x)
+                hip.release(buf)
+        assert (locked[:at] == -1.0).all() and (locked[at + n:] == -1.0).all()
+        hip.raise_if_error()
+    finally:
+        rt.hipHostFree(p)
+
+
 @pytest.mark.parametrize("n_in,n_out,n", [(512, 70, 63), (512, 70, 64), (512, 68, 65), (256, 36, 200)])
 def test_exact_dense_nvfp4_batches(exact, orc, n_in, n_out, n):
     import inferred_hip as ih
