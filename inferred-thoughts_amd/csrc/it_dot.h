@@ -72,9 +72,9 @@ IT_DEV h8v fp4x8_to_f16x8(uint32_t w, h2 scale) {
 typedef __attribute__((address_space(3))) void* lptr;
 // 16 bytes a lane from memory to LDS, one lane's behind the other's from `to` on (the same in every lane).  Written out because
 // the compiler's own form makes every later read of LDS wait for all such loads; here they are waited for by count, in front
-// of the barrier of the stage that reads them.
+// of the barrier of the stage that reads them.  (The LDS address goes in as M0 itself, so that the compiler knows what it holds.)
 IT_DEV void to_lds(const void* from, uint32_t to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(to), "v"(from) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "{m0}"(to), "v"(from) : "memory");
 }
 
 // operands of the f16 expert tile kernels (k_gemm_f16.hip, k_gemm_f16s.hip)
