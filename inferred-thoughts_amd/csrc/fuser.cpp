@@ -1378,7 +1378,7 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
         if (id(k) == OP_SCALE && h[k].p[0] == u.p[5] && h[k].i[0] == u.i[2] * u.i[3]) su = h[k++].f[0];
         if (id(k) == OP_SCALE && h[k].p[0] == a.p[5] && h[k].i[0] == a.i[2] * a.i[3]) sg = h[k++].f[0];
         if (id(k) == OP_EW && h[k].i[0] == 0 && h[k].p[0] == a.p[5] && h[k].p[1] == u.p[5] && h[k].i[1] == a.i[2] * a.i[3] && a.p[5] != u.p[5] &&
-            u.p[6] == a.p[6] && u.i[0] == a.i[0] && u.i[1] == a.i[1] && u.i[2] == a.i[2] && u.i[3] == a.i[3] && !used_later(h, k + 1, next, u.p[5])) {
+            u.p[6] == a.p[6] && u.i[0] == a.i[0] && u.i[1] == a.i[1] && u.i[2] == a.i[2] && u.i[3] == a.i[3]) {
             auto view = [](const OpRec& m) {
                 ExpertsView v{};
                 v.q = m.p[0]; v.scales = m.p[1]; v.fmt = (int)m.i[0]; v.n_in = (int)m.i[1]; v.n_out = (int)m.i[2]; v.n_expert = 1;
@@ -1389,12 +1389,9 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
             x.h = (uint16_t*)a.p[6]; x.l = (uint16_t*)a.p[7]; x.scale = (float*)a.p[8];
             const int nt = (int)a.i[3];
             Span sp(this, FAM_MATMUL, span_of(k + 1 - i));
-            const bool done = a.i[4] == 1 ? experts_gemm_f16s(vg, &vu, nullptr, nt, 1, 0, x, (float*)a.p[5], nullptr, 0, false, {}, sg, su, stream)
-                                          : experts_gemm_f16(vg, &vu, nullptr, nt, 1, 0, x, (float*)a.p[5], nullptr, 0, false, {}, sg, su, stream);
-            if (done) {
-                mark_elided({u.p[5]});
-                return k + 1 - i;
-            }
+            const bool done = a.i[4] == 1 ? experts_gemm_f16s(vg, &vu, nullptr, nt, 1, 0, x, (float*)a.p[5], nullptr, 0, false, {}, sg, su, stream, (float*)u.p[5])
+                                          : experts_gemm_f16(vg, &vu, nullptr, nt, 1, 0, x, (float*)a.p[5], nullptr, 0, false, {}, sg, su, stream, (float*)u.p[5]);
+            if (done) return k + 1 - i;
         }
     }
     if (a.id == OP_MATMUL && a.scaled && id(i + 1) == OP_SCALE && h[i + 1].p[0] == a.p[5] && h[i + 1].i[0] == a.i[2] * a.i[3]) {

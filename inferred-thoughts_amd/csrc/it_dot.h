@@ -86,6 +86,7 @@ struct ExpertsF16P {
     const uint16_t *xh, *xl;
     const float* rscale;
     float* out;
+    float* up_out;               // gate / up pair: the up product too (null: only silu(gate) * up)
     int n_in, n_out, x_mode, n_used;
     const int32_t* n_tiles;
     const int4* tiles;           // null: one matrix, tile t holds the pairs from t * (pairs a tile) on, in order

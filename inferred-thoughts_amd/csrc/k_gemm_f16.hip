@@ -317,13 +317,15 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
             if (GLU) {
                 const int row = rbase[0] + 8 * i4 + 4 * kg;
                 if (row >= p.n_out) continue;
-                float o[4];
+                float o[4], u[4];
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float g = acc[0][tt][4 * i4 + i] * rsc * e2a, u = acc[1][tt][4 * i4 + i] * rsc * e2b;
-                    o[i] = fx_silu(g) * u;
+                    const float g = acc[0][tt][4 * i4 + i] * rsc * e2a;
+                    u[i] = acc[1][tt][4 * i4 + i] * rsc * e2b;
+                    o[i] = fx_silu(g) * u[i];
                 }
                 *(float4*)(p.out + pair * p.n_out + row) = make_float4(o[0], o[1], o[2], o[3]);
+                if (p.up_out) *(float4*)(p.up_out + pair * p.n_out + row) = make_float4(u[0], u[1], u[2], u[3]);
             } else {
 #pragma unroll
                 for (int z = 0; z < 2; z++) {
@@ -394,8 +396,8 @@ bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks,
 
 bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
                       int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
-                      const TileCount& count, float scale_a, float scale_b, hipStream_t s) {
-    if (!x.h || !experts_f16_takes(w, up, n_picks, out)) return false;
+                      const TileCount& count, float scale_a, float scale_b, hipStream_t s, float* up_out) {
+    if (!x.h || !experts_f16_takes(w, up, n_picks, out) || (reinterpret_cast<uintptr_t>(up_out) & 15)) return false;
     if (ids && (!work || work_ints < experts_f16_work_ints(n_picks, w.n_expert))) return false;
     if (n_used < 1) n_used = 1;
     const size_t lds = (size_t)4 * FPAIRS * FBS * sizeof(uint16_t) + (size_t)2 * 256 * (FWS + 16);
@@ -425,6 +427,7 @@ bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t
     p.scale_b = scale_b;
     p.count = count;
     p.out = out;
+    p.up_out = up_out;
     p.n_in = w.n_in;
     p.n_out = w.n_out;
     p.x_mode = x_mode;

@@ -166,6 +166,8 @@ __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
             const float u4[4] = {up.x, up.y, up.z, up.w};
 #pragma unroll
             for (int i = 0; i < 4; i++) o[i] = fx_silu(acc[g][i] * rsc * e2a) * (u4[i] * rsc * e2b);
+            if (p.up_out)
+                *(float4*)(p.up_out + (int64_t)pair * p.n_out + row) = make_float4(u4[0] * rsc * e2b, u4[1] * rsc * e2b, u4[2] * rsc * e2b, u4[3] * rsc * e2b);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++) o[i] = acc[g][i] * rsc * e2a;
@@ -313,6 +315,10 @@ __global__ __launch_bounds__(512, 4) void experts_f16k_k(ExpertsF16P p, int batc
                 else o[q] = sum[0][q] * rsc * e2a;
             }
             *(float4*)(p.out + (int64_t)pair * p.n_out + row) = make_float4(o[0], o[1], o[2], o[3]);
+            if (GLU && p.up_out) {
+                const float* u = sum[NM - 1];
+                *(float4*)(p.up_out + (int64_t)pair * p.n_out + row) = make_float4(u[0] * rsc * e2b, u[1] * rsc * e2b, u[2] * rsc * e2b, u[3] * rsc * e2b);
+            }
         }
     }
 }
@@ -332,8 +338,8 @@ bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks
 
 bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
                        int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
-                       const TileCount& count, float scale_a, float scale_b, hipStream_t s) {
-    if (!x.h || !experts_f16s_takes(w, up, n_picks, out)) return false;
+                       const TileCount& count, float scale_a, float scale_b, hipStream_t s, float* up_out) {
+    if (!x.h || !experts_f16s_takes(w, up, n_picks, out) || (reinterpret_cast<uintptr_t>(up_out) & 15)) return false;
     if (ids && (!work || work_ints < experts_group_work_ints(n_picks, w.n_expert))) return false;
     if (n_used < 1) n_used = 1;
     // the layout of the int8 tile kernel's grouping (tiles of 16 pairs): either may reuse the other's
@@ -363,6 +369,7 @@ bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_
     p.scale_b = scale_b;
     p.count = count;
     p.out = out;
+    p.up_out = up_out;
     p.n_in = w.n_in;
     p.n_out = w.n_out;
     p.x_mode = x_mode;

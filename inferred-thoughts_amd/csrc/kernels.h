@@ -140,14 +140,14 @@ struct TileCount {
 bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const float* out);
 bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
                       int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
-                      const TileCount& count, float scale_a, float scale_b, hipStream_t s);
+                      const TileCount& count, float scale_a, float scale_b, hipStream_t s, float* up_out = nullptr);
 // NVFP4 experts with few pairs per expert in fast mode (k_gemm_f16s.hip): tiles of 16 pairs on MFMA 16x16x32 f16, no LDS;
 // the grouping has the layout of experts_gemm's (tiles of 16 pairs).  ids as for experts_gemm_f16; scale_a, scale_b: factors
 // of the two products.
 bool experts_f16s_takes(const ExpertsView& w, const ExpertsView* up, int n_picks, const float* out);
 bool experts_gemm_f16s(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
                        int x_mode, const SplitOut& x, float* out, int32_t* work, size_t work_ints, bool grouped,
-                       const TileCount& count, float scale_a, float scale_b, hipStream_t s);
+                       const TileCount& count, float scale_a, float scale_b, hipStream_t s, float* up_out = nullptr);
 // Small batches in fast mode (k_moe_rows.hip): pairs sorted by expert in tiles of 8 or 16, every weight row of a tile's
 // expert streamed once and multiplied with all its pairs by integer dots.  ids null: one dense matrix (strides
 // ignored), tile t = tokens 8 t .. 8 t + 7.  False: nothing launched (shape, alignment or scratch do not fit).

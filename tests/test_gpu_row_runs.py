@@ -61,6 +61,11 @@ def run(pair, n, bufs, script, outs, tol=1e-5, at_most=None, other_first=False):
     return got
 
 
+def q8_0_weights_of(r, n_out, n_in):
+    from oracle import binding as ob
+    return q8_0_weights(ob.Oracle(threads=2), r, n_out, n_in, std=0.05)
+
+
 def f32(r, k, s=1.0):
     return (r.standard_normal(k) * s).astype(np.float32)
 
@@ -215,3 +220,25 @@ def test_the_nvfp4_shared_expert(pair, n, nd, ff):
         be.matmul(ih.weights(wd, ih.NVFP4, 256, nd), b["h"], b["out"])
         be.scale(b["out"], 0.5)
     run(pair, n, b, script, ["gate", "out"], at_most=5)
+
+
+@pytest.mark.parametrize("n,nd,ff,scaled", [(40, 512, 64, True), (131, 768, 68, False), (200, 1024, 128, True), (1030, 512, 96, True)])
+def test_the_nvfp4_shared_experts_up_product_stays_readable(pair, n, nd, ff, scaled):
+    """The gate and up products in one launch leave the up product where an op or the host finds it: behind the gated product
+    (with the row lengths of either 16-wide kernel and of the 128-wide one)."""
+    import inferred_hip as ih
+    r = rng(8)
+    wg, wu, wd = nvfp4_weights(r, ff, nd), nvfp4_weights(r, ff, nd), q8_0_weights_of(r, 64, 64)
+    z = lambda k: np.zeros(k, np.float32)  # noqa: E731
+    b = dict(x=f32(r, n * nd, 0.2), gate=z(n * ff), up=z(n * ff), rows=z(n * ff), h=f32(r, n * 64), out=z(n * 64))
+
+    def script(be, b):
+        be.matmul(ih.weights(wg, ih.NVFP4, nd, ff), b["x"], b["gate"])
+        be.matmul(ih.weights(wu, ih.NVFP4, nd, ff), b["x"], b["up"])
+        if scaled:
+            be.scale(b["up"], 0.25)
+            be.scale(b["gate"], 0.03)
+        be.silu_mul(b["gate"], b["up"])
+        be.matmul(ih.weights(wd, ih.Q8_0, 64, 64), b["h"], b["out"])
+        be.gather_chunks(b["up"], ff, ff, 0, b["rows"])
+    run(pair, n, b, script, ["gate", "up", "rows"], at_most=6, other_first=True)
