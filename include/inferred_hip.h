@@ -382,7 +382,11 @@ void it_engine_state_sizes(const it_engine*, uint64_t out[2]);
 uint64_t it_engine_checkpoint(it_engine*, float* conv_out, float* ssm_out);
 int it_engine_restore(it_engine*, uint64_t pos, const float* conv_in, const float* ssm_in);
 int it_engine_rewind(it_engine*, uint64_t len);
-/* one forward pass at the current position; logits (n_vocab) may be NULL. 0 = ok */
+/* one forward pass at the current position; logits (n_vocab) may be NULL. 0 = ok.
+ * A pass without logits is issued and not waited for: it returns the errors that are known by then (a refused argument, an
+ * allocation, an earlier pass's), and one that the device reports later comes out of the next call that waits (a pass with
+ * logits, generate, it_hip_take_error), whose results and those since the failed pass are then void.  The same goes for
+ * prefill without logits and decode_greedy without ids. */
 int it_engine_forward(it_engine*, const uint32_t* tokens, uint64_t n, float* logits);
 /* chunked prefill; logits of the last token (may be NULL) */
 int it_engine_prefill(it_engine*, const uint32_t* tokens, uint64_t n, float* logits);

@@ -2344,6 +2344,7 @@ void it_hip_read_state(it_hip* be, float* host, uint64_t len) {
     size_t bytes = len * 4 < it->second.bytes ? len * 4 : it->second.bytes;
     if (!be->check(hipMemcpyAsync(host, it->second.dev, bytes, hipMemcpyDeviceToHost, be->stream), "download state")) return;
     be->check(hipStreamSynchronize(be->stream), "download state");
+    be->chain_check();
     be->d2h++;
     be->d2h_bytes += bytes;
 }
@@ -2355,6 +2356,7 @@ void it_hip_read_kv(it_hip* be, uint16_t* slab, uint64_t len) {
     size_t bytes = len * 2 < it->second.bytes ? len * 2 : it->second.bytes;
     if (!be->check(hipMemcpyAsync(slab, it->second.dev, bytes, hipMemcpyDeviceToHost, be->stream), "download kv")) return;
     be->check(hipStreamSynchronize(be->stream), "download kv");
+    be->chain_check();
     be->d2h++;
     be->d2h_bytes += bytes;
 }

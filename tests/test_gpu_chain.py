@@ -335,6 +335,35 @@ def test_a_wait_that_gives_up_is_an_error_not_a_hang():
     assert err is None, err
 
 
+def test_an_error_of_a_pass_without_logits_comes_out_of_the_next_call_that_waits(tmp_path):
+    """The engine does not wait for a pass whose logits stay on the device; an error that such a pass meets there (a chain's
+    wait, bounded to one poll) is returned by the next pass whose logits come home, and the one after it runs."""
+    import inferred_hip as ih
+    path = str(tmp_path / "short.gguf")
+    ih.synth_write_gguf(path, ih.big_config(n_layer=2, full_attention_interval=2, n_vocab=256, n_threads=8))
+    os.environ["INFERRED_HIP_CHAIN_SPINS"] = "1"
+    try:
+        be = ih.Hip(exact=False)
+    finally:
+        del os.environ["INFERRED_HIP_CHAIN_SPINS"]
+    m = ih.Model(path)
+    e = ih.Engine(m, be, 64)
+    try:
+        for i in range(4):     # two op by op, one recorded, one replayed
+            e.forward([i], want_logits=False)
+        with pytest.raises(RuntimeError, match="layer chain"):
+            e.forward([4])
+        assert be.take_error() is None and not be.chain_stats()["enabled"]
+        e.reset()
+        e.prefill([5, 6, 7], want_logits=False)
+        assert np.isfinite(e.forward([8])).all()
+    finally:
+        e.close(); m.close()
+        err = be.take_error()
+        be.close()
+    assert err is None, err
+
+
 @pytest.mark.parametrize("pos0", [5800, 40, 12000, 8189])
 def test_the_attention_mixer_inside_a_chain_against_the_oracle(pos0):
     """One attention layer whose FFN adds nothing (second scales of zero on every down product), so that the pass's
