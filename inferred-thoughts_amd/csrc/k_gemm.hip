@@ -147,10 +147,11 @@ __global__ __launch_bounds__(GT) void q8_gemm_k(const int8_t* __restrict__ wq, c
 // dozen to some hundred tokens every slab waits out most of a trip to memory.  Here a stage is asked for as soon as its
 // buffer has been read and costs no register, no store and one barrier for 256 k.  Such a load writes its lanes' 16 bytes
 // side by side, so a row's sixteen pieces are permuted by the row's number instead of being padded apart: sixteen rows' reads
-// meet every bank once.  The arithmetic is the same, product by product, in the same order.
-// Bound from some 500 tokens on by LDS reads and the twelve vector operations per product of the matrix cores together (about
-// half of each one's rate; with the scales' products moved to the matrix cores as outer products, eight operations, the time
-// does not change), below by the stages' latency.  8192 x 2048 over 64 / 201 / 512 / 5,700 tokens: 18.1 -> 11.2, 33.0 -> 27.5, 55.7 -> 50.8, 618 -> 528 us; 4096 x 2048:
+// of a piece start in different banks.  The arithmetic is the same, product by product, in the same order.
+// Bound from some 500 tokens on by the twelve vector operations per product of the matrix cores (5,700 tokens: vector ALU busy
+// 71 %, matrix cores 16 to 18 %, two waves a SIMD; LDS reads still meet in the banks, 3 to 4 conflict cycles for each
+// four-cycle unit of LDS activity, but 2 to 5 % of the wave cycles wait on them; with the scales' products moved to the matrix
+// cores as outer products, eight operations, the time does not change), below by the stages' latency.  8192 x 2048 over 64 / 201 / 512 / 5,700 tokens: 18.1 -> 11.2, 33.0 -> 27.5, 55.7 -> 50.8, 618 -> 528 us; 4096 x 2048:
 // 16.0 -> 9.3, 24.9 -> 15.4, 33.7 -> 28.3, 296 -> 272; 2048 x 4096: 28.5 -> 15.8, 32.4 -> 18.7, 41.2 -> 27.4, 290 -> 276.
 // Not kept: three or four stages (0 to 50 % slower everywhere: fewer blocks fit a CU); the f16 matrix cores with the
 // activations as an f16 pair and no scale per token, 128 x 256 tiles (8192 x 2048 over 5,700: 437 us with three stages, 46 % of

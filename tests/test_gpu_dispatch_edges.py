@@ -1,5 +1,5 @@
 """Where the dispatch changes kernels: the NVFP4 tiles' token and pair counts, copies to the host by size, bit-exact paths
-that take a short cut and fall back, and the short layer chain (own start, output matrix as its last stage) by vocabulary."""
+that take a short cut and fall back, and a chain of two layers against its stages by vocabulary."""
 import numpy as np
 import pytest
 
@@ -136,8 +136,10 @@ def test_exact_mean_square_at_a_rounding_tie(exact, orc, n, nd):
 
 @pytest.mark.parametrize("n_vocab", [8195, 16384, 16385])
 def test_short_chain_by_vocabulary(tmp_path, n_vocab):
-    """Decode steps of a two-layer model whose output matrix is (up to 16,384 rows) the chain's last stage, against the same
-    steps on a backend that launches every stage by itself; turn by turn, so that the later ones replay."""
+    """Decode steps of a two-layer model, its layers as one chain, against the same steps on a backend that launches every
+    stage by itself; turn by turn, so that the later ones replay.  The stages' sums are in another order, which moves Q8_0
+    steps of 1/127 of a block and now and then exchanges an expert: fast and exact mode differ by 5e-3 to 1.4e-2 of the logits'
+    2-norm on such models, so 2e-2 bounds two orders of sums, where a lost layer or a stale row gives about 1."""
     import inferred_hip as ih
     path = str(tmp_path / "short.gguf")
     ih.synth_write_gguf(path, ih.big_config(n_layer=2, full_attention_interval=2, n_vocab=n_vocab))
@@ -154,6 +156,6 @@ def test_short_chain_by_vocabulary(tmp_path, n_vocab):
         assert np.array_equal(turns[1], turns[2])
         got.append(turns[2])
         e.close(); m.close(); be.close()
-    scale = np.sqrt((got[1] ** 2).mean())
-    print(n_vocab, np.abs(got[0] - got[1]).max() / scale, flush=True)
-    assert np.abs(got[0] - got[1]).max() <= 0.1 * scale
+    err = np.linalg.norm(got[0] - got[1]) / np.linalg.norm(got[1])
+    print(n_vocab, err, flush=True)
+    assert err <= 2e-2, err
