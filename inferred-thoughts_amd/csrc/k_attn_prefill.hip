@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void attend_prefill_k(AttnArgs a, float* __res
     auto tile = [&](auto next, auto half, int kt, v16f (&sc)[2], v16f (&sn)[2]) __attribute__((always_inline)) {
         constexpr bool NEXT = decltype(next)::value;
         constexpr int B = decltype(half)::value;
-        __builtin_amdgcn_s_waitcnt(0x0f70);         // tile kt's V and tile kt + 1's K have landed (vmcnt 0)
+        __builtin_amdgcn_s_waitcnt(0x0070);         // tile kt's V and tile kt + 1's K have landed (vmcnt 0), and this wave has what it read (lgkmcnt 0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (NEXT) {                                 // (every wave is past tile kt's K and tile kt - 1's V)

@@ -208,7 +208,7 @@ __global__ __launch_bounds__(256) void q8_tile_k(const int8_t* __restrict__ wq, 
     ask(0, 0);
     for (int s = 0; s < n_stage; s++) {
         const int buf = s & 1;
-        __builtin_amdgcn_s_waitcnt(0x0f70);      // stage s has landed (vmcnt 0)
+        __builtin_amdgcn_s_waitcnt(0x0070);      // stage s has landed (vmcnt 0), and this wave has what it read of the last one (lgkmcnt 0)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         if (s + 1 < n_stage) ask(s + 1, buf ^ 1);      // (every wave has read that buffer)
