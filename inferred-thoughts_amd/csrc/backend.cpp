@@ -79,13 +79,14 @@ void it_hip::dyn_rotate() {
     dyn_host = dyn_hosts[dyn_cur];
     dyn_count = 0;
 }
-// What a recorded pass reads that its launches do not carry: host copies, positions, the token's embedding row.
+// What a recorded pass reads that its launches do not carry: positions, the token's embedding row, and host copies, which may
+// be newer values of the row's buffer.
 void it_hip::issue_inputs() {
-    for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
-    precopies.clear();
     dyn_upload();
     if (pre_embed.x) (void)itk::poke(nullptr, dyn_host, 0, &pre_embed.table, pre_embed.token, pre_embed.x, stream);
     pre_embed.x = nullptr;
+    for (auto& c : precopies) check(hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, stream), "upload activation");
+    precopies.clear();
 }
 void it_hip::dyn_upload() {
     if (!dyn_count) return;
@@ -2658,12 +2659,14 @@ int it_hip_embed_rows(it_hip* be, const it_weights* table, const uint32_t* ids, 
     if (!be->weights_view(table, "embed_rows", &w)) return 0;
     float* dx = be->act_out(x, x_len);
     if (!dx) return 0;
-    if (n == 1 && be->mode != it_hip::Mode::Eager) {
-        // a recorded pass: the row is made by the small kernel that carries the pass's positions
+    if (n == 1 && be->mode != it_hip::Mode::Eager && be->pending.empty() && !be->pre_embed.x) {
+        // a recorded pass: the row is made by the small kernel that carries the pass's positions, in front of the pass's ops
         be->pre_embed = {w, (int)ids[0], dx};
         be->pass_embed = be->pre_embed;
         return 1;
     }
+    // a second row, or one behind ops that may have to do with the buffer's last values: made where it stands
+    be->need_eager("an embedding row behind other ops of a pass", false);
     be->launches++;
     if (!be->held.empty()) be->release_held();
     it_hip::Span sp(be, it_hip::FAM_OTHER, x_len * 5);

@@ -72,3 +72,45 @@ def test_passes_of_two_kinds_in_turn_keep_their_graphs(tiny_gguf):
         be.raise_if_error()
     finally:
         eng.close(); m.close(); be.close()
+
+
+ROWS = {   # what a single-token pass makes of rows of the table: the ops, and the result from the rows
+    "two_rows": (lambda be, e, b: (e(b["x"], 0), e(b["y"], 1), be.add_assign(b["x"], b["y"])), lambda r, v: r[0] + r[1]),
+    "one_after_the_other": (lambda be, e, b: (e(b["y"], 0), be.add_assign(b["x"], b["y"]), e(b["y"], 1), be.add_assign(b["x"], b["y"])),
+                            lambda r, v: (v + r[0]) + r[1]),
+    "behind_the_buffers_last_values": (lambda be, e, b: (be.scale(b["x"], 2.0), e(b["x"], 0), be.scale(b["x"], 4.0)), lambda r, v: 4 * r[0]),
+    "newer_host_values": (lambda be, e, b: (e(b["x"], 0), b["x"].__setitem__(slice(None), b["v"]), be.host_wrote(b["x"]), be.scale(b["x"], 4.0)),
+                          lambda r, v: 4 * v),
+}
+
+
+@pytest.mark.parametrize("what", sorted(ROWS))
+def test_rows_in_the_order_of_the_passes_ops(what):
+    """A recorded pass makes its one embedding row in front of its ops; a second row, and one whose buffer other ops or the
+    host have to do with, keep their place."""
+    r = np.random.default_rng(1)
+    raw, rows = table(ih.Q8_0, 50, 64, r)
+    w = ih.weights(raw, ih.Q8_0, 64, 50)
+    be = ih.Hip()
+    ops, want = ROWS[what]
+    try:
+        b = dict(x=np.zeros(64, np.float32), y=np.zeros(64, np.float32), v=np.zeros(64, np.float32))
+        for i in range(6):    # op by op, recorded, replayed
+            ids = r.integers(0, 50, 2).astype(np.uint32)
+            v = r.standard_normal(64).astype(np.float32)
+            b["x"][:] = v
+            b["v"][:] = v + 1
+            be.begin_pass(1)
+            be.host_wrote(b["x"])
+
+            def embed(x, k):
+                one = ids[k:k + 1].copy()
+                assert be.L.it_hip_embed_rows(be.h, ih.C.addressof(w), one.ctypes.data, 1, x.ctypes.data, x.size) == 1
+            ops(be, embed, b)
+            be.end_pass()
+            be.host_needs(b["x"])
+            be.raise_if_error()
+            at = v + 1 if what == "newer_host_values" else v
+            assert np.array_equal(b["x"], want(rows[ids], at).astype(np.float32)), (what, i)
+    finally:
+        be.close()
