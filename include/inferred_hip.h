@@ -288,8 +288,9 @@ int it_hip_embed_rows(it_hip*, const it_weights* table, const uint32_t* ids, uin
  * kind of pass), inside the pass, between begin_pass and the first op.  replay_pass then issues a whole pass of that tag at
  * `pos` (*id: its token, embedded as by it_hip_embed_rows; id NULL: the arg-max, as by it_hip_embed_argmax at ring_index) from
  * what earlier passes of the tag recorded, in place of begin_pass, the ops and end_pass.  Returns 0, with nothing done, while
- * it cannot: the tag is new, buffers moved, graphs are off, or at `pos` one of the pass's ops would refuse its position (a
- * cache row or a context outside its slab).  The caller then issues the pass as usual.
+ * it cannot: the tag is new, buffers moved, graphs are off, the tag's passes take values from the host beside the token, or
+ * at `pos` one of the pass's ops would refuse its position (a cache row or a context outside its slab).  The caller then
+ * issues the pass as usual.
  * Of the ops' checks only those of the positions are made again.  In particular the host bytes of the weights are not
  * looked at (every op compares a sample of them with what is resident): a caller that maps another model where the last one
  * was calls it_hip_drop_mirrors first, as for any pass, or takes another tag. */

@@ -275,9 +275,16 @@ void it_hip::launch(Graph& g) {
 
 // After a recorded pass was launched: what a later one of the same tag needs to be launched without being recorded again.
 // The scalars of two passes at different positions tell which follow the position (they move with it, one for one) and
-// which are fixed; anything else keeps the tag's passes recorded.
+// which are fixed; anything else keeps the tag's passes recorded, as does a pass that takes values from the host beside its
+// token: they come anew with every pass.
 void it_hip::learn(Graph& g) {
-    if (!pass_tag || (g.known && g.epoch == res_epoch)) return;
+    if (!pass_tag) return;
+    if (pass_uploads) {
+        g.known = false;
+        g.tag = nullptr;
+        return;
+    }
+    if (g.known && g.epoch == res_epoch) return;
     const bool second = g.tag == pass_tag && g.pos != pass_pos && g.dyn.size() == dyn_count && g.ring_slot == pass_ring_slot;
     g.known = second;
     if (second) {
@@ -398,6 +405,7 @@ float* it_hip::act_in(const float* host, size_t len) {
     if (!a->dev_current) {
         if (mode != Mode::Eager) {
             precopies.push_back(PreCopy{a->dev, host, len * sizeof(float)});
+            pass_uploads = true;
         } else {
             // ops held back run later than this copy: if one of them touches the buffer, it has to run first
             if (!held.empty() && held_touches(a->dev, a->cap * sizeof(float))) release_held();
@@ -2278,6 +2286,7 @@ void it_hip_begin_pass(it_hip* be, uint64_t n_tokens) {
     be->pre_embed.x = nullptr;
     be->pass_tag = nullptr;
     be->pass_embed.x = nullptr;
+    be->pass_uploads = false;
     be->pass_ring_slot = -1;
     be->dyn_rotate();
     be->replay_cursor = 0;

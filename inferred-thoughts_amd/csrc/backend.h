@@ -355,6 +355,7 @@ struct it_hip {
     bool small_ffn(const std::vector<OpRec>& held_ops, size_t end, const OpRec* next);   // the routed FFN of a short batch (held_ops[0 .. end)) as two launches
     bool small_ffn_enabled = true;           // INFERRED_HIP_NO_SMALL_FFN=1 issues it op by op (a measurement switch)
     std::vector<PreCopy> precopies;  // host -> device inputs of a graphed pass, issued before the graph
+    bool pass_uploads = false;       // the pass had some
     // the embedding row of a recorded single-token pass, made by the kernel that carries its positions (x: not yet issued)
     struct PreEmbed {
         itk::WView table;

@@ -77,3 +77,42 @@ def test_replayed_up_to_the_end_of_the_slab(rows, exact):
         for be in backends:
             be.take_error()
             be.close()
+
+
+@pytest.mark.parametrize("host_values", [False, True])
+def test_a_pass_that_takes_values_from_the_host_is_issued_every_time(host_values):
+    """x = a row of the table, then x += a vector: of the device (made by the pass before) or of the host (new in each pass)."""
+    import inferred_hip as ih
+    from oracle import binding as ob
+    r = rng(4)
+    orc = ob.Oracle(threads=2)
+    raw = q8_0_weights(orc, r, VOCAB, DIM, std=1.0)
+    tw = ih.weights(raw, ih.Q8_0, DIM, VOCAB)
+    blocks = raw.reshape(VOCAB, DIM // 32, 34)
+    rows = (blocks[..., :2].copy().view(np.float16).astype(np.float32) * blocks[..., 2:].view(np.int8).astype(np.float32)).reshape(VOCAB, DIM)
+    tag = np.zeros(1, np.uint8)
+    be = ih.Hip()
+    try:
+        x, v = np.zeros(DIM, np.float32), np.zeros(DIM, np.float32)
+        replayed = 0
+        for pos in range(10):
+            one = r.integers(0, VOCAB, 1).astype(np.uint32)
+            v[:] = r.standard_normal(DIM)
+            if be.L.it_hip_replay_pass(be.h, tag.ctypes.data, pos, one.ctypes.data, 0):
+                replayed += 1
+            else:
+                be.begin_pass(1)
+                be.L.it_hip_tag_pass(be.h, tag.ctypes.data, pos)
+                assert be.L.it_hip_embed_rows(be.h, C.addressof(tw), one.ctypes.data, 1, x.ctypes.data, x.size)
+                if host_values:
+                    be.host_wrote(v)
+                    be.add_assign(x, v)
+                else:
+                    be.add_assign(x, x)
+                be.end_pass()
+            be.host_needs(x)
+            be.raise_if_error()
+            assert np.array_equal(x, rows[one[0]] + (v if host_values else rows[one[0]])), pos
+        assert replayed == 0 if host_values else replayed >= 4, replayed
+    finally:
+        be.close()
