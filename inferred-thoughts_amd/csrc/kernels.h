@@ -283,6 +283,11 @@ struct TilePrepP {
     uint16_t *k_slab, *v_slab;
 };
 bool attend_tile_prep_ok(const AttnArgs& a, const TilePrepP& pr);
+// up to DECODE_MAX_Q queries on the f16 matrix cores (k_attn_decode.hip); part as above, n_split <= 256 ranges of it at most
+constexpr int DECODE_MAX_Q = 16, DECODE_CUS = 256;
+bool attend_decode_takes(int n_q, int head_dim, int group);
+bool attend_decode(const AttnArgs& a, const TilePrepP* prep, int n_split, float* part, float* out, const float* gate, int gate_stride,
+                   hipStream_t s);
 bool attend_split_gated_prep(const AttnArgs& a, const TilePrepP& pr, int n_split, float* scratch, float* out,
                              const float* gate, int gate_stride, hipStream_t s);
 // the same with the merge multiplying by sigmoid(gate[head * gate_stride + i]) (n_q == 1)

@@ -55,3 +55,50 @@ def test_a_row_does_not_depend_on_what_stands_behind_it(hip, orc, n_q, n_pos, hd
         got = attend(hip, kb, vb)
         assert close(got[:t + 1], want[:t + 1]), (t, np.abs(got[:t + 1] - want[:t + 1]).max())
         assert not np.isfinite(got[t + 1:, :, 3]).any()
+
+
+@pytest.mark.parametrize("hd,nh,nkv", [(64, 8, 2), (64, 4, 4), (128, 8, 1), (128, 32, 4), (256, 16, 2), (256, 4, 2)])
+# one query to two groups of eight; contexts around a wave's quarter (8), a slice (32), a stage (64, 128) and a round of ranges
+@pytest.mark.parametrize("n_q", [1, 2, 3, 4, 5, 8, 9, 16])
+def test_queries_and_contexts_around_the_tiles_edges(hip, orc, n_q, hd, nh, nkv):
+    sc = 1.0 / np.sqrt(np.float32(hd))
+    for n_pos in (n_q, 31, 32, 33, 64, 65, 127, 128, 129, 257, 1000, 8193, 16400):
+        if n_pos < n_q:
+            continue
+        r = rng(n_pos * 31 + n_q)
+        kv_dim = nkv * hd
+        q = r.standard_normal(n_q * nh * hd).astype(np.float32)
+        k, v = f16_bits(r.standard_normal(n_pos * kv_dim)), f16_bits(r.standard_normal(n_pos * kv_dim))
+        out, want = np.zeros(n_q * nh * hd, np.float32), np.zeros(n_q * nh * hd, np.float32)
+        orc.attend(q, k, v, kv_dim, n_pos, hd, nh, nkv, sc, want)
+        hip.drop_mirrors(); hip.begin_pass(n_q)
+        hip.attend(q, k, v, kv_dim, n_pos, hd, nh, nkv, sc, out)
+        hip.host_needs(out); hip.end_pass(); hip.raise_if_error()
+        # probabilities are f16: 2^-11 of the largest value a row's average can hold
+        assert np.abs(out - want).max() <= 1e-3, (n_q, n_pos, np.abs(out - want).max())
+
+
+@pytest.mark.parametrize("n_q,n_pos", [(1, 5), (1, 700), (2, 700), (4, 333), (7, 1500)])
+def test_operands_that_are_not_16_byte_aligned(n_q, n_pos):
+    import inferred_hip as ih
+    from util import Hiprt
+    hd, nh, nkv = 128, 16, 4
+    r = rng(n_pos)
+    kv = n_pos * nkv * hd
+    q = r.standard_normal(n_q * nh * hd).astype(np.float32)
+    k, v = f16_bits(r.standard_normal(kv)), f16_bits(r.standard_normal(kv))
+    rt = Hiprt()
+    try:
+        got = []
+        for shift in (0, 1):   # q one float further, K and V one half further
+            dq = rt.upload(np.concatenate([np.zeros(shift, np.float32), q]))
+            dk, dv = (rt.upload(np.concatenate([np.zeros(shift, np.uint16), x])) for x in (k, v))
+            dout = rt.filled(q.nbytes, 0xff)
+            rc, msg = ih.attend_noalloc(dq + 4 * shift, q.size, dk + 2 * shift, dv + 2 * shift, kv, nkv * hd, n_pos, hd, nh, nkv,
+                                        float(hd ** -0.5), dout, q.size, stream=0)
+            assert rc == 0, msg
+            got.append(rt.download(dout, np.zeros_like(q)))
+        assert np.isfinite(got[0]).all()
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    finally:
+        rt.free_all()
