@@ -68,7 +68,8 @@ __device__ __constant__ const uint64_t IT_EXP2F_TAB[32] = {
     0x3fef5818dcfba487ull, 0x3fef7c97337b9b5full, 0x3fefa4afa2a490daull, 0x3fefd0765b6e4540ull,
 };
 
-IT_DEV float it_expf(float x) {
+// (the table may be a copy in LDS: a lookup in constant memory is a trip to L2 on a short kernel's critical path)
+IT_DEV float it_expf_by(float x, const uint64_t* tab) {
     const double InvLn2N = 0x1.71547652b82fep+0 * 32.0;
     const double Shift = 0x1.8p52;
     const double C0 = 0x1.c6af84b912394p-5 / 32.0 / 32.0 / 32.0;
@@ -88,7 +89,7 @@ IT_DEV float it_expf(float x) {
     uint64_t ki = (uint64_t)__double_as_longlong(kd);
     kd -= Shift;
     double r = z - kd;
-    uint64_t t = IT_EXP2F_TAB[ki % 32];
+    uint64_t t = tab[ki % 32];
     t += ki << (52 - 5);
     double s = __longlong_as_double((long long)t);
     z = C0 * r + C1;
@@ -98,6 +99,7 @@ IT_DEV float it_expf(float x) {
     y = y * s;
     return (float)y;
 }
+IT_DEV float it_expf(float x) { return it_expf_by(x, IT_EXP2F_TAB); }
 
 __device__ __constant__ const double IT_LOGF_TAB[16][2] = {
     {0x1.661ec79f8f3bep+0, -0x1.57bf7808caadep-2}, {0x1.571ed4aaf883dp+0, -0x1.2bef0a7c06ddbp-2},
@@ -110,7 +112,7 @@ __device__ __constant__ const double IT_LOGF_TAB[16][2] = {
     {0x1.886e6037841edp-1, 0x1.1058bc8a07ee1p-2},  {0x1.767dcf5534862p-1, 0x1.4043057b6ee09p-2},
 };
 
-IT_DEV float it_logf(float x) {
+IT_DEV float it_logf_by(float x, const double (*tab)[2]) {
     const double A0 = -0x1.00ea348b88334p-2, A1 = 0x1.5575b0be00b6ap-2, A2 = -0x1.ffffef20a4123p-2;
     const double Ln2 = 0x1.62e42fefa39efp-1;
     uint32_t ix = __float_as_uint(x);
@@ -126,7 +128,7 @@ IT_DEV float it_logf(float x) {
     int i = (tmp >> (23 - 4)) % 16;
     int32_t k = (int32_t)tmp >> 23;
     uint32_t iz = ix - (tmp & (0x1ffu << 23));
-    double invc = IT_LOGF_TAB[i][0], logc = IT_LOGF_TAB[i][1];
+    double invc = tab[i][0], logc = tab[i][1];
     double z = (double)__uint_as_float(iz);
     double r = z * invc - 1.0;
     double y0 = logc + (double)k * Ln2;
@@ -136,6 +138,7 @@ IT_DEV float it_logf(float x) {
     y = y * r2 + (y0 + r);
     return (float)y;
 }
+IT_DEV float it_logf(float x) { return it_logf_by(x, IT_LOGF_TAB); }
 
 // silu and sigmoid exactly as the reference writes them
 // (/root/reference src/ops/naive.rs:250, :335).
@@ -148,3 +151,5 @@ IT_DEV float fx_sigmoid(float g) { return 1.0f / (1.0f + fx_expf(-g)); }
 IT_DEV float fx_silu(float g) { return g / (1.0f + fx_expf(-g)); }
 IT_DEV float it_sigmoid(float g) { return 1.0f / (1.0f + it_expf(-g)); }
 IT_DEV float it_silu(float g) { return g / (1.0f + it_expf(-g)); }
+IT_DEV float it_sigmoid_by(float g, const uint64_t* tab) { return 1.0f / (1.0f + it_expf_by(-g, tab)); }
+IT_DEV float it_silu_by(float g, const uint64_t* tab) { return g / (1.0f + it_expf_by(-g, tab)); }

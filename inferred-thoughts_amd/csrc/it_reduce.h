@@ -11,33 +11,16 @@ namespace itk {
 // differs from that sum by less than n * 2^-52 of it, and division and rounding to f32 are monotonic: where both ends of
 // that interval give the same f32, so does the serial sum, and only where they do not (n = 2,048: one row in 10^5) is it
 // formed, by one lane (2,048 dependent f64 additions: 20 us, the tree 1).  Exact mode therefore has the CPU's bits.
-IT_DEV bool mean_is_certain(double sum, int n, double div, float* mean) {
+// Division by a power of two is a product with its inverse, to the bit (an f64 division is some thirty dependent operations).
+IT_DEV double over(double sum, int div) {
+    if (!(div & (div - 1))) return sum * __builtin_bit_cast(double, (uint64_t)(1023 - __builtin_ctz(div)) << 52);
+    return sum / (double)div;
+}
+IT_DEV bool mean_is_certain(double sum, int n, int div, float* mean) {
     const double off = sum * ((double)(n + 16) * 0x1p-52);
-    *mean = (float)((sum - off) / div);
-    return *mean == (float)((sum + off) / div);
+    *mean = (float)over(sum - off, div);
+    return *mean == (float)over(sum + off, div);
 }
-template <int THREADS>
-__device__ float block_meansq(const float* buf, int n, double div, int exact, double* red) {
-    double part = 0.0;
-    for (int i = threadIdx.x; i < n; i += THREADS) part += (double)(buf[i] * buf[i]);
-    for (int off = 32; off > 0; off >>= 1) part += __shfl_down(part, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = part;
-    __syncthreads();
-    double sum = 0.0;
-    for (int w = 0; w < THREADS / 64; w++) sum += red[w];
-    if (!exact) return (float)(sum / div);
-    float mean;
-    if (mean_is_certain(sum, n, div, &mean)) return mean;   // (the same answer in every thread)
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        sum = 0.0;
-        for (int i = 0; i < n; i++) sum += (double)(buf[i] * buf[i]);
-        red[0] = sum;
-    }
-    __syncthreads();
-    return (float)(red[0] / div);
-}
-
 // ------------------------------------------------------------------ lane exchanges without LDS
 // DPP moves reach the lanes of a row of 16: neighbour (quad_perm 1,0,3,2), pair (quad_perm
 // 2,3,0,1), the mirrored half of 8 and the mirrored row of 16.  After the first two steps a
@@ -135,6 +118,28 @@ IT_DEV double wave_sum_f64_tail(double v) {
         v += __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
     }
     return v;
+}
+
+template <int THREADS>
+__device__ float block_meansq(const float* buf, int n, int div, int exact, double* red) {
+    double part = 0.0;
+    for (int i = threadIdx.x; i < n; i += THREADS) part += (double)(buf[i] * buf[i]);
+    part = wave_sum_f64_tail(part);
+    if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = part;
+    __syncthreads();
+    double sum = 0.0;
+    for (int w = 0; w < THREADS / 64; w++) sum += red[w];
+    if (!exact) return (float)over(sum, div);
+    float mean;
+    if (mean_is_certain(sum, n, div, &mean)) return mean;   // (the same answer in every thread)
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sum = 0.0;
+        for (int i = 0; i < n; i++) sum += (double)(buf[i] * buf[i]);
+        red[0] = sum;
+    }
+    __syncthreads();
+    return (float)over(red[0], div);
 }
 
 // Sum over the 8 lanes of an aligned group with data-parallel-primitive moves (no LDS crossbar):

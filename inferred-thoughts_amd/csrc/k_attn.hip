@@ -29,7 +29,9 @@ __global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __rest
                                                       const float* __restrict__ gate, int gate_stride, int lds_pos) {
     extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each)
     __shared__ float red[17];
+    __shared__ uint64_t etab[32];   // (a lookup in constant memory is a trip to L2)
     const int hd = a.head_dim, tid = threadIdx.x, nt = blockDim.x;
+    if (tid < 32) etab[tid] = IT_EXP2F_TAB[tid];
     const int n_pos_last = a.n_pos_dyn ? *a.n_pos_dyn : a.n_pos;
     const int t = blockIdx.x / a.n_head, h = blockIdx.x % a.n_head;
     const int group = a.n_head / a.n_head_kv;
@@ -80,10 +82,10 @@ __global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __rest
     __syncthreads();
     m = red[0];
     for (int w = 1; w < nt / 64; w++) m = fmaxf(m, red[w]);
-    for (int s = tid; s < n_pos; s += nt) score(s) = it_expf(score(s) - m);
+    for (int s = tid; s < n_pos; s += nt) score(s) = it_expf_by(score(s) - m, etab);
     __threadfence_block();
     __syncthreads();
-    if (tid == 0) {
+    if (tid < 64) {   // (every lane: reads of one address by all cost less than by one lane)
         float sum = fold_terms(near, n_lds);
 #pragma unroll 16
         for (int s = lds_pos; s < n_pos; s++) sum += far[s];

@@ -28,7 +28,7 @@ __global__ __launch_bounds__(THREADS) void rms_norm_k(const float* __restrict__ 
     float* o = out + (int64_t)blockIdx.x * nd;
     for (int i = threadIdx.x; i < nd; i += THREADS) lds[i] = row[i];
     __syncthreads();
-    float mean = block_meansq<THREADS>(lds, nd, (double)nd, exact, red);
+    float mean = block_meansq<THREADS>(lds, nd, nd, exact, red);
     float scale = 1.0f / sqrtf(mean + eps);
     for (int i = threadIdx.x; i < nd; i += THREADS) o[i] = lds[i] * scale * w[i];
 }
@@ -47,7 +47,7 @@ __global__ __launch_bounds__(THREADS) void rms_norm_q8_k(const float* __restrict
     float* o = out + (int64_t)blockIdx.x * nd;
     for (int i = threadIdx.x; i < nd / 4; i += THREADS) ((float4*)lds)[i] = ((const float4*)row)[i];
     __syncthreads();
-    float mean = block_meansq<THREADS>(lds, nd, (double)nd, exact, red);
+    float mean = block_meansq<THREADS>(lds, nd, nd, exact, red);
     float scale = 1.0f / sqrtf(mean + eps);
     const int64_t blk0 = (int64_t)blockIdx.x * (nd / 32);
     for (int i0 = 0; i0 < nd / 4; i0 += THREADS) {      // uniform trip count: the lane moves below need every lane
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(64) void head_norm_k(float* __restrict__ x, const f
     float* head = x + (int64_t)blockIdx.x * hd;
     for (int i = threadIdx.x; i < hd; i += 64) lds[i] = head[i];
     __syncthreads();
-    float scale, mean = block_meansq<64>(lds, hd, mode == 0 ? (double)hd : 1.0, exact, red);
+    float scale, mean = block_meansq<64>(lds, hd, mode == 0 ? hd : 1, exact, red);
     if (mode == 0) {
         scale = 1.0f / sqrtf(mean + eps);
         for (int i = threadIdx.x; i < hd; i += 64) head[i] = lds[i] * scale * w[i];

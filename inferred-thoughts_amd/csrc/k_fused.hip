@@ -51,6 +51,25 @@ __device__ void lds_quantize_q8_0(const float* xf, int n, float* xs, int8_t* xq)
     }
 }
 
+// The Q8_0 form of four values, eight neighbouring lanes a block (naive.rs:652-675): the quants and, in every lane, the f16 scale.
+IT_DEV void quantize_quad(float4 v, uint32_t* packed, float* scale) {
+    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+    amax = fmaxf(amax, dpp_xor1(amax));
+    amax = fmaxf(amax, dpp_xor2(amax));
+    amax = fmaxf(amax, dpp_half_mirror(amax));
+    const float d = amax / 127.0f;
+    const float id = d != 0.0f ? 1.0f / d : 0.0f;
+    const float r[4] = {roundf(v.x * id), roundf(v.y * id), roundf(v.z * id), roundf(v.w * id)};
+    uint32_t q = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float c = fminf(fmaxf(r[i], -128.0f), 127.0f);
+        q |= ((uint32_t)(((r[i] != r[i]) ? 0 : (int)c) & 0xff)) << (8 * i);
+    }
+    *packed = q;
+    *scale = it_f16_to_f32(it_f32_to_f16(d));
+}
+
 IT_DEV void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_wave_barrier();
@@ -60,6 +79,11 @@ IT_DEV void wave_lds_sync() {
 // Terms of `nrows` rows starting at `row0` of one matrix against the LDS activation.
 // Two phases so every HBM load of the group is in flight before the first dot: a lane
 // owns IPL (row, 32-element unit) items, loads them all, then computes.
+// row of item `it` where a row has U units, inv = 1 / U: items are below 2^20, so the product is never within its rounding of
+// a whole number (an integer division is some forty instructions, eight of them ahead of a wave's first loads)
+IT_DEV int row_of(int it, float inv) { return (int)(((float)it + 0.5f) * inv); }
+IT_DEV float inv_of(int n) { return __builtin_amdgcn_rcpf((float)n); }
+
 template <int IPL>
 struct RowRegs {
     uint4 wa[IPL], wb[IPL];
@@ -71,11 +95,13 @@ __device__ __forceinline__ void load_items(RowRegs<IPL>& rr, const uint8_t* wq, 
                                            int nrows, int lane) {
     const int U = n_in >> 5;
     const int items = nrows * U;
+    const float inv = inv_of(U);
 #pragma unroll
     for (int k = 0; k < IPL; k++) {
+        if (k * 64 >= items) break;
         int it = k * 64 + lane;
         if (it < items) {
-            int r = it / U, u = it - r * U;
+            int r = row_of(it, inv), u = it - r * U;
             int64_t row = row0 + r;
             if (FMT == W_Q8_0) {
                 const uint4* wp = (const uint4*)(wq + row * n_in + u * 32);
@@ -94,11 +120,13 @@ __device__ __forceinline__ void compute_items(const RowRegs<IPL>& rr, int n_in, 
                                               const float* xs, float* terms, int tstride, int lane) {
     const int U = n_in >> 5;
     const int items = nrows * U;
+    const float inv = inv_of(U);
 #pragma unroll
     for (int k = 0; k < IPL; k++) {
+        if (k * 64 >= items) break;
         int it = k * 64 + lane;
         if (it < items) {
-            int r = it / U, u = it - r * U;
+            int r = row_of(it, inv), u = it - r * U;
             const uint4* ap = (const uint4*)(xq + u * 32);
             uint4 a0 = ap[0], a1 = ap[1];
             float dx = xs[u];
@@ -143,7 +171,7 @@ __device__ void wave_row_terms(const uint8_t* wq, const uint8_t* ws, int n_in, i
 // Called by one wave; probs (LDS, n_expert floats) holds the logits on entry.  A lane keeps its NE probabilities (experts
 // lane + 64 i) in registers; a round is one reduction over the wave for the value and a ballot per register for the lowest id that has it.
 template <int NE>
-__device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane) {
+__device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane, const uint64_t* etab) {
     float v[NE];
     float m = -INFINITY;
 #pragma unroll
@@ -157,7 +185,7 @@ __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, 
 #pragma unroll
     for (int i = 0; i < NE; i++) {
         const int e = lane + 64 * i;
-        v[i] = e < n_expert ? it_expf(v[i] - m) : -1.0f;
+        v[i] = e < n_expert ? it_expf_by(v[i] - m, etab) : -1.0f;
         if (e < n_expert) {
             probs[e] = v[i];
             part += v[i];
@@ -166,7 +194,7 @@ __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, 
     wave_lds_sync();
     float sum;
     if (exact) {
-        sum = __shfl(lane == 0 ? fold_terms(probs, n_expert) : 0.0f, 0, 64);
+        sum = fold_terms(probs, n_expert);   // (every lane: the same reads)
     } else {
         for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
         sum = part;
@@ -197,7 +225,7 @@ __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, 
     }
     // sum in pick order, serial f32
     float s = 0.0f;
-    for (int r = 0; r < n_used; r++) s += __shfl(picked_p, r, 64);
+    for (int r = 0; r < n_used; r++) s += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, picked_p), r));
     float denom = fmaxf(s, 6.103515625e-5f);
     if (lane < n_used) {
         ids[lane] = picked_id;
@@ -206,10 +234,10 @@ __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, 
     wave_lds_sync();
 }
 constexpr int ROUTE_MAX_EXPERTS = 2048;
-__device__ void wave_route(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane) {
-    if (n_expert <= 64) wave_route_n<1>(probs, n_expert, n_used, exact, ids, weights, lane);
-    else if (n_expert <= 512) wave_route_n<8>(probs, n_expert, n_used, exact, ids, weights, lane);
-    else wave_route_n<32>(probs, n_expert, n_used, exact, ids, weights, lane);   // up to ROUTE_MAX_EXPERTS (match_ffn)
+__device__ void wave_route(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane, const uint64_t* etab) {
+    if (n_expert <= 64) wave_route_n<1>(probs, n_expert, n_used, exact, ids, weights, lane, etab);
+    else if (n_expert <= 512) wave_route_n<8>(probs, n_expert, n_used, exact, ids, weights, lane, etab);
+    else wave_route_n<32>(probs, n_expert, n_used, exact, ids, weights, lane, etab);   // up to ROUTE_MAX_EXPERTS (match_ffn)
 }
 
 constexpr int FG_THREADS = 512, FG_LDS_MAX = 128 * 1024;
@@ -227,9 +255,26 @@ IT_DEV void put_out(const FusedGemvP& p, const FusedMat& m, int j, float v) {
     if (p.route_counter) __hip_atomic_store(m.out + j, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else m.out[j] = v;
 }
+// what a row's epilogue reads, asked for long before: the conv window and taps (epi 1), the value it is added to (epi 2)
+struct Epi {
+    float p0, p1, p2, w0, w1, w2, w3;
+};
+IT_DEV Epi ask_epi(const FusedGemvP& p, const FusedMat& m, int row0, int nrows, int lane) {
+    Epi e{};
+    if (lane >= nrows) return e;
+    const int64_t j = row0 + lane;
+    if (m.epi == 2) {
+        e.p0 = m.out[j];
+    } else if (m.epi == 1) {
+        const float *past = p.conv_state + j * 3, *w = p.conv_w + j * 4;
+        e.p0 = past[0]; e.p1 = past[1]; e.p2 = past[2];
+        e.w0 = w[0]; e.w1 = w[1]; e.w2 = w[2]; e.w3 = w[3];
+    }
+    return e;
+}
 // fold each row's terms in order and apply the matrix's epilogue
 IT_DEV void finish_rows(const FusedGemvP& p, const FusedMat& m, int row0, int nrows, const float* terms, int tstride,
-                        int nb, int lane) {
+                        int nb, int lane, const Epi& e, const uint64_t* etab) {
     if (lane >= nrows) return;
     const int T = m.fmt == W_NVFP4 ? nb * 2 : nb;
     float acc = fold_terms(terms + lane * tstride, T);
@@ -237,136 +282,278 @@ IT_DEV void finish_rows(const FusedGemvP& p, const FusedMat& m, int row0, int nr
     if (m.epi == 0) {
         put_out(p, m, j, acc);
     } else if (m.epi == 2) {
-        m.out[j] += acc;
+        m.out[j] = e.p0 + acc;
     } else if (m.epi == 3) {
-        m.out[j] = it_silu(acc);
+        m.out[j] = it_silu_by(acc, etab);
     } else {
         // causal conv (kernel 4) + silu on channel j, state [channel][3] oldest first
         float* past = p.conv_state + (int64_t)j * 3;
-        const float* w = p.conv_w + (int64_t)j * 4;
-        float p0 = past[0], p1 = past[1], p2 = past[2];
         float sum = 0.0f;
-        sum += p0 * w[0];
-        sum += p1 * w[1];
-        sum += p2 * w[2];
-        sum += acc * w[3];
-        m.out[j] = it_silu(sum);
-        past[0] = p1;
-        past[1] = p2;
+        sum += e.p0 * e.w0;
+        sum += e.p1 * e.w1;
+        sum += e.p2 * e.w2;
+        sum += acc * e.w3;
+        m.out[j] = it_silu_by(sum, etab);
+        past[0] = e.p1;
+        past[1] = e.p2;
         past[2] = acc;
     }
 }
 
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));   // four floats, wherever they start
+IT_DEV float4 load4(const float* p) {
+    const f4u v = *(const f4u*)p;
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+IT_DEV void store4(float* p, float4 v) { *(f4u*)p = f4u{v.x, v.y, v.z, v.w}; }
+
+// Blocks 0 .. q_blocks - 1 take the quantized rows, the rest the unquantized ones, whose fold is a chain of n_in additions (eight
+// cycles each: 2,048 take 7.5 us) that nothing else should wait for.
+// Bound by the chain activation -> norm -> Q8_0 -> dots -> fold -> epilogue of dependent instructions between two launches.  So a
+// thread keeps its four values of the activation (and of norm weight and gate) in registers from the load to the quants, one
+// barrier for the norm's sum and one for the quants; what a row's epilogue reads is asked for ahead of it, the exponential's
+// table sits in LDS, and a wave's row, scalar, is found without integer divisions.  512 values, 1,552 rows: 6.4 -> 5.0 us;
+// 2,048 values, 12,288 Q8_0 and 64 F32 rows 28.6 -> 11.7 (the F32 rows' LDS left one quantized row a pass), 513 F32 rows and
+// the route 24.9 -> 24.5.
+template <int NQ>
 __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double red[FG_THREADS / 64 + 1];
     __shared__ float hscale[64];
+    __shared__ uint64_t etab[32];
+    constexpr int W = FG_THREADS / 64;
     const int n_in = p.n_in, nb = n_in >> 5;
     float* xf = (float*)smem;
     float* xs = xf + n_in;
     int8_t* xq = (int8_t*)(xs + ((nb + 3) & ~3));
     float* terms_all = (float*)(xq + n_in);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool quantized = (int)blockIdx.x < p.q_blocks;
 
-    // the first row group's weights start moving before the activation prologue runs
-    constexpr int W = FG_THREADS / 64;
+    // the activation first, then the first row group's weights: they move while the prologue runs
+    float4 xv[NQ], wv[NQ], gv[NQ];
+#pragma unroll
+    for (int j = 0; j < NQ; j++) {
+        const int i = 4 * (tid + FG_THREADS * j);
+        xv[j] = wv[j] = gv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (i < n_in) {
+            xv[j] = load4(p.x + i);
+            if (p.mode == 1) wv[j] = load4(p.norm_w + i);
+            if (p.mode >= 2) {
+                wv[j] = load4(p.norm_w + i % p.head_dim);
+                gv[j] = load4(p.gate + i);
+            }
+        }
+    }
+    if (tid < 32) etab[tid] = IT_EXP2F_TAB[tid];
     const int R = p.rows_per_wave;
     const int tstride = nb * 2 + 4;
-    float* terms = terms_all + (size_t)wave * p.terms_stride;
+    float* terms = terms_all + (size_t)wave * (quantized ? p.terms_stride : n_in);
     const int g0 = blockIdx.x * W + wave;
-    const bool has0 = g0 < p.total_groups;
+    const bool has0 = quantized && g0 < p.total_groups;
     const FusedMat& m0 = p.m[has0 ? mat_index(p, g0) : 0];
     const int row00 = has0 ? (g0 - m0.group0) * R : 0;
     const int nrows0 = has0 ? min(R, m0.n_out - row00) : 0;
     RowRegs<8> rr;
+    Epi epi{};
     if (has0) {
         if (m0.fmt == W_NVFP4) load_items<W_NVFP4, 8>(rr, m0.q, m0.s, n_in, row00, nrows0, lane);
         else load_items<W_Q8_0, 8>(rr, m0.q, m0.s, n_in, row00, nrows0, lane);
+        epi = ask_epi(p, m0, row00, nrows0, lane);
+    }
+    // unquantized rows: one a wave at a time, dealt out over the blocks first
+    const int f_blocks = gridDim.x - p.q_blocks;
+    auto frow = [&](int fr) __attribute__((always_inline)) {   // (matrix, row)
+        int k = p.n_mats;
+        while (fr >= p.m[k].n_out) fr -= p.m[k++].n_out;
+        return make_int2(k, fr);
+    };
+    constexpr int FW = 8;                            // of 256 floats each: what is asked for ahead of the prologue
+    float4 fw[FW];
+    const int fr0 = wave * f_blocks + (int)blockIdx.x - p.q_blocks;
+    if (!quantized && fr0 < p.total_frows) {
+        const int2 at = frow(fr0);
+        const float* row = (const float*)p.m[at.x].q + (int64_t)at.y * n_in;
+#pragma unroll
+        for (int c = 0; c < FW; c++)
+            if (c * 256 < n_in) fw[c] = *(const float4*)(row + c * 256 + lane * 4);
     }
 
-    for (int i = tid; i < n_in; i += FG_THREADS) xf[i] = p.x[i];
-    __syncthreads();
+    auto squares = [](float4 v) __attribute__((always_inline)) {
+        double s = (double)(v.x * v.x);
+        s += (double)(v.y * v.y);
+        s += (double)(v.z * v.z);
+        s += (double)(v.w * v.w);
+        return s;
+    };
     if (p.mode == 1) {
-        float mean = block_meansq<FG_THREADS>(xf, n_in, (double)n_in, p.exact, red);
-        float scale = 1.0f / sqrtf(mean + p.eps);
-        for (int i = tid; i < n_in; i += FG_THREADS) xf[i] = xf[i] * scale * p.norm_w[i];
+        double part = 0.0;
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            const int i = 4 * (tid + FG_THREADS * j);
+            part += squares(xv[j]);
+            if (i < n_in) *(float4*)(xf + i) = xv[j];      // for the serial sum, should it be needed
+        }
+        part = wave_sum_f64_tail(part);
+        if (lane == 63) red[wave] = part;
         __syncthreads();
+        double sum = 0.0;
+        for (int w = 0; w < W; w++) sum += red[w];
+        float mean = (float)over(sum, n_in);
+        if (p.exact && !mean_is_certain(sum, n_in, n_in, &mean)) {   // (the same answer in every thread)
+            __syncthreads();
+            if (tid == 0) {
+                sum = 0.0;
+                for (int i = 0; i < n_in; i++) sum += (double)(xf[i] * xf[i]);
+                red[0] = sum;
+            }
+            __syncthreads();
+            mean = (float)over(red[0], n_in);
+        }
+        const float scale = 1.0f / sqrtf(mean + p.eps);
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            xv[j].x = xv[j].x * scale * wv[j].x;
+            xv[j].y = xv[j].y * scale * wv[j].y;
+            xv[j].z = xv[j].z * scale * wv[j].z;
+            xv[j].w = xv[j].w * scale * wv[j].w;
+        }
     } else if (p.mode == 2 || p.mode == 3) {
-        const int hd = p.head_dim, nh = n_in / hd;  // nh <= 64 (checked on the host)
-        // 8 lanes per head; a head's walk starts at its own place, so that the heads of a wave read different banks
-        for (int h0 = 0; h0 < nh; h0 += FG_THREADS / 8) {
-            const int h = h0 + (tid >> 3), sub = tid & 7, steps = hd / 8;
-            double part = 0.0;
-            if (h < nh)
-                for (int k = 0; k < steps; k++) {
-                    const float v = xf[h * hd + sub + 8 * ((k + h) % steps)];
-                    part += (double)(v * v);
+        const int hd = p.head_dim, lph = hd / 4;     // lanes of a head
+        const bool by_lanes = lph == 8 || lph == 16 || lph == 32 || lph == 64;
+        if (!by_lanes) {
+            // 8 lanes per head; a head's walk starts at its own place, so that the heads of a wave read different banks
+#pragma unroll
+            for (int j = 0; j < NQ; j++) {
+                const int i = 4 * (tid + FG_THREADS * j);
+                if (i < n_in) *(float4*)(xf + i) = xv[j];
+            }
+            __syncthreads();
+            const int nh = n_in / hd;  // nh <= 64 (checked on the host)
+            for (int h0 = 0; h0 < nh; h0 += FG_THREADS / 8) {
+                const int h = h0 + (tid >> 3), sub = tid & 7, steps = hd / 8;
+                double part = 0.0;
+                if (h < nh)
+                    for (int k = 0; k < steps; k++) {
+                        const float v = xf[h * hd + sub + 8 * ((k + h) % steps)];
+                        part += (double)(v * v);
+                    }
+                part += dpp_f64(part, 0);
+                part += dpp_f64(part, 1);
+                part += dpp_f64(part, 2);
+                if (h < nh && sub == 0) {
+                    float mean;
+                    if (!p.exact) {
+                        mean = (float)over(part, hd);
+                    } else if (!mean_is_certain(part, hd, hd, &mean)) {
+                        part = 0.0;
+                        for (int i = 0; i < hd; i++) part += (double)(xf[h * hd + i] * xf[h * hd + i]);
+                        mean = (float)over(part, hd);
+                    }
+                    hscale[h] = 1.0f / sqrtf(mean + p.eps);
                 }
-            part += dpp_f64(part, 0);
-            part += dpp_f64(part, 1);
-            part += dpp_f64(part, 2);
-            if (h < nh && sub == 0) {
-                float mean;
-                if (!p.exact) {
-                    mean = (float)(part / (double)hd);
-                } else if (!mean_is_certain(part, hd, (double)hd, &mean)) {
-                    part = 0.0;
-                    for (int i = 0; i < hd; i++) part += (double)(xf[h * hd + i] * xf[h * hd + i]);
-                    mean = (float)(part / (double)hd);
-                }
-                hscale[h] = 1.0f / sqrtf(mean + p.eps);
             }
         }
-        __syncthreads();
-        for (int i = tid; i < n_in; i += FG_THREADS) {
-            float core = xf[i] * hscale[i / hd] * p.norm_w[i % hd];
-            xf[i] = (p.mode == 2 ? it_silu(p.gate[i]) : p.gate[i]) * core;
+        __syncthreads();                             // (the table, too)
+#pragma unroll
+        for (int j = 0; j < NQ; j++) {
+            float scale;
+            if (by_lanes) {
+                double sum = squares(xv[j]);
+                sum += dpp_f64(sum, 0);
+                sum += dpp_f64(sum, 1);
+                sum += dpp_f64(sum, 2);
+                if (lph >= 16) sum += dpp_f64(sum, 3);
+                if (lph >= 32) sum += __shfl_xor(sum, 16, 64);
+                if (lph >= 64) sum += __shfl_xor(sum, 32, 64);
+                float mean = (float)over(sum, hd);
+                if (p.exact && !mean_is_certain(sum, hd, hd, &mean)) {   // (the same answer in every lane of the head)
+                    sum = 0.0;
+                    for (int l = 0; l < lph; l++) {
+                        const int from = (lane & ~(lph - 1)) + l;
+                        const float a = __shfl(xv[j].x, from, 64), b = __shfl(xv[j].y, from, 64), c = __shfl(xv[j].z, from, 64), d = __shfl(xv[j].w, from, 64);
+                        sum += (double)(a * a);
+                        sum += (double)(b * b);
+                        sum += (double)(c * c);
+                        sum += (double)(d * d);
+                    }
+                    mean = (float)over(sum, hd);
+                }
+                scale = 1.0f / sqrtf(mean + p.eps);
+            } else {
+                scale = hscale[min(4 * (tid + FG_THREADS * j), n_in - 1) / hd];
+            }
+            auto gated = [&](float x, float w, float g) __attribute__((always_inline)) {
+                const float core = x * scale * w;
+                return (p.mode == 2 ? it_silu_by(g, etab) : g) * core;
+            };
+            xv[j].x = gated(xv[j].x, wv[j].x, gv[j].x);
+            xv[j].y = gated(xv[j].y, wv[j].y, gv[j].y);
+            xv[j].z = gated(xv[j].z, wv[j].z, gv[j].z);
+            xv[j].w = gated(xv[j].w, wv[j].w, gv[j].w);
         }
-        __syncthreads();
     }
-    if (blockIdx.x == 0) {
-        if (p.x_copy)
-            for (int i = tid; i < n_in; i += FG_THREADS) p.x_copy[i] = xf[i];
-        if (p.x_copy2)
-            for (int i = tid; i < n_in; i += FG_THREADS) p.x_copy2[i] = xf[i];
+#pragma unroll
+    for (int j = 0; j < NQ; j++) {
+        const int i = 4 * (tid + FG_THREADS * j);
+        const bool live = i < n_in;
+        if (blockIdx.x == 0 && live) {
+            if (p.x_copy) store4(p.x_copy + i, xv[j]);
+            if (p.x_copy2) store4(p.x_copy2 + i, xv[j]);
+        }
+        if (quantized) {
+            uint32_t packed;
+            float d;
+            quantize_quad(xv[j], &packed, &d);
+            if (live) {
+                *(uint32_t*)(xq + i) = packed;
+                if ((tid & 7) == 0) xs[i >> 5] = d;
+            }
+        } else if (live) {
+            *(float4*)(xf + i) = xv[j];
+        }
     }
-    if (p.n_mats) {
-        lds_quantize_q8_0(xf, n_in, xs, xq);
-        __syncthreads();
-    }
+    __syncthreads();
 
     if (has0) {
         if (m0.fmt == W_NVFP4) compute_items<W_NVFP4, 8>(rr, n_in, nrows0, xq, xs, terms, tstride, lane);
         else compute_items<W_Q8_0, 8>(rr, n_in, nrows0, xq, xs, terms, tstride, lane);
         wave_lds_sync();
-        finish_rows(p, m0, row00, nrows0, terms, tstride, nb, lane);
+        finish_rows(p, m0, row00, nrows0, terms, tstride, nb, lane, epi, etab);
         wave_lds_sync();
     }
-    for (int g = g0 + gridDim.x * W; g < p.total_groups; g += gridDim.x * W) {
-        const FusedMat& m = p.m[mat_index(p, g)];
-        const int row0 = (g - m.group0) * R;
-        const int nrows = min(R, m.n_out - row0);
-        if (m.fmt == W_NVFP4) wave_row_terms<W_NVFP4>(m.q, m.s, n_in, row0, nrows, xq, xs, terms, tstride, lane);
-        else wave_row_terms<W_Q8_0>(m.q, m.s, n_in, row0, nrows, xq, xs, terms, tstride, lane);
-        wave_lds_sync();
-        finish_rows(p, m, row0, nrows, terms, tstride, nb, lane);
-        wave_lds_sync();
-    }
-    // Unquantized rows: the wave forms a row's products, one lane folds them in order (naive.rs:843-861).  Dealt out over
-    // the blocks first: the fold is a chain of n_in additions.
-    for (int fr = wave * gridDim.x + blockIdx.x; fr < p.total_frows; fr += W * gridDim.x) {
-        int k = p.n_mats, j = fr;
-        while (j >= p.m[k].n_out) j -= p.m[k++].n_out;
-        const FusedMat& m = p.m[k];
-        const float* row = (const float*)m.q + (int64_t)j * n_in;
-#pragma unroll 8
-        for (int i = lane * 4; i < n_in; i += 256) {
-            const float4 w = *(const float4*)(row + i), x = *(const float4*)(xf + i);
-            *(float4*)(terms + i) = make_float4(w.x * x.x, w.y * x.y, w.z * x.z, w.w * x.w);
+    if (quantized) {
+        for (int g = g0 + p.q_blocks * W; g < p.total_groups; g += p.q_blocks * W) {
+            const FusedMat& m = p.m[mat_index(p, g)];
+            const int row0 = (g - m.group0) * R;
+            const int nrows = min(R, m.n_out - row0);
+            const Epi e = ask_epi(p, m, row0, nrows, lane);
+            if (m.fmt == W_NVFP4) wave_row_terms<W_NVFP4>(m.q, m.s, n_in, row0, nrows, xq, xs, terms, tstride, lane);
+            else wave_row_terms<W_Q8_0>(m.q, m.s, n_in, row0, nrows, xq, xs, terms, tstride, lane);
+            wave_lds_sync();
+            finish_rows(p, m, row0, nrows, terms, tstride, nb, lane, e, etab);
+            wave_lds_sync();
         }
-        wave_lds_sync();
-        if (lane == 0) put_out(p, m, j, fold_terms(terms, n_in));
-        wave_lds_sync();
+    } else {
+        // the wave forms a row's products, one lane folds them in order (naive.rs:843-861)
+        for (int fr = fr0; fr < p.total_frows; fr += W * f_blocks) {
+            const int2 at = frow(fr);
+            const FusedMat& m = p.m[at.x];
+            const float* row = (const float*)m.q + (int64_t)at.y * n_in;
+            auto products = [&](int i, float4 w) __attribute__((always_inline)) {
+                const float4 x = *(const float4*)(xf + i);
+                *(float4*)(terms + i) = make_float4(w.x * x.x, w.y * x.y, w.z * x.z, w.w * x.w);
+            };
+#pragma unroll
+            for (int c = 0; c < FW; c++)
+                if (c * 256 < n_in) products(c * 256 + lane * 4, fr == fr0 ? fw[c] : *(const float4*)(row + c * 256 + lane * 4));
+#pragma unroll 8
+            for (int i = FW * 256 + lane * 4; i < n_in; i += 256) products(i, *(const float4*)(row + i));
+            wave_lds_sync();
+            const float sum = fold_terms(terms, n_in);   // (every lane: reads of one address by all cost less than by one lane)
+            if (lane == 0) put_out(p, m, at.y, sum);
+            wave_lds_sync();
+        }
     }
     if (p.route_counter) {
         // The block that finishes last turns the router logits (matrix 0's output) into the
@@ -389,7 +576,7 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
             if (wave == 0) {
                 __shared__ int rids[64];
                 __shared__ float rwts[64];
-                wave_route(probs, p.n_expert, p.n_used, p.exact, rids, rwts, lane);
+                wave_route(probs, p.n_expert, p.n_used, p.exact, rids, rwts, lane, etab);
                 if (lane < p.n_used) {
                     p.route_ids[lane] = rids[lane];
                     p.route_w[lane] = rwts[lane];
@@ -440,30 +627,35 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
                 R = r;
                 break;
             }
-    auto stride_for = [&](int r) { return std::max(r * (nb * 2 + 4), nf ? p.n_in : 0); };
-    auto lds_for = [&](int r) {
-        return (size_t)p.n_in * 4 + (size_t)((nb + 3) & ~3) * 4 + p.n_in + (size_t)W * stride_for(r) * 4;
-    };
-    while (R > 1 && lds_for(R) > 60 * 1024) R /= 2;
+    const size_t base = (size_t)p.n_in * 4 + (size_t)((nb + 3) & ~3) * 4 + p.n_in;
+    auto q_lds = [&](int r) { return base + (size_t)W * r * (nb * 2 + 4) * 4; };
+    while (R > 1 && q_lds(R) > 60 * 1024) R /= 2;
     p.rows_per_wave = R;
-    p.terms_stride = stride_for(R);
+    p.terms_stride = R * (nb * 2 + 4);
     int g = 0;
     for (int i = 0; i < nq; i++) {
         p.m[i].group0 = g;
         g += (p.m[i].n_out + R - 1) / R;
     }
     p.total_groups = g;
-    int blocks = std::max((g + W - 1) / W, p.total_frows);
     // one block per CU: every block pays the activation prologue, so more blocks than CUs
     // only repeats it (measured: 256 blocks 12 us, 772 blocks 22 us for norm + 12k rows of 2048)
-    if (blocks > 256) blocks = 256;
-    const size_t lds = lds_for(R);
-    if (lds > 64 * 1024) {
-        static const bool sized = hipFuncSetAttribute((const void*)fused_gemv_k, hipFuncAttributeMaxDynamicSharedMemorySize, FG_LDS_MAX) == hipSuccess;
-        if (!sized) (void)hipGetLastError();
-    }
-    hipLaunchKernelGGL(fused_gemv_k, dim3(blocks), dim3(FG_THREADS), lds, s, p);
+    p.q_blocks = std::min((g + W - 1) / W, 256);
+    // the unquantized rows on what CUs are left, or eight to a block
+    const int f_blocks = nf ? std::min(p.total_frows, std::max(256 - p.q_blocks, (p.total_frows + W - 1) / W)) : 0;
+    const int f_waves = nf ? std::min(W, (p.total_frows + f_blocks - 1) / f_blocks) : 0;
+    const int blocks = std::max(1, p.q_blocks + f_blocks);
+    const size_t lds = std::max(nq ? q_lds(R) : base, base + (size_t)f_waves * p.n_in * 4);
+    auto launch = [&](auto kernel) {
+        if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, FG_LDS_MAX) != hipSuccess) (void)hipGetLastError();
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(FG_THREADS), lds, s, p);
+    };
+    if (p.n_in <= 4 * FG_THREADS) launch(fused_gemv_k<1>);
+    else if (p.n_in <= 8 * FG_THREADS) launch(fused_gemv_k<2>);
+    else if (p.n_in <= 16 * FG_THREADS) launch(fused_gemv_k<4>);
+    else launch(fused_gemv_k<10>);   // (FG_LDS_MAX holds no more)
 }
+static_assert(FG_LDS_MAX / 7 <= 10 * 4 * FG_THREADS, "an activation that LDS holds fits the registers");
 // F32 rows beside (or in place of) quantized ones, in the kernel that keeps the CPU path's order
 bool fused_gemv_exact_takes(const FusedGemvP& p) {
     for (int i = 0; i < p.n_mats; i++) {
@@ -475,26 +667,6 @@ bool fused_gemv_exact_takes(const FusedGemvP& p) {
 }
 
 // ------------------------------------------------------------------ gdn rows
-// l2-normalised k (first half of kq) and q (second half) of key head `kh`, read from the
-// conv output [q | k | v] (naive.rs:254-273).
-template <int DK, int THREADS>
-__device__ void load_kq_l2(const float* conv, int key_dim, int kh, float eps, int exact, float* kq, double* red) {
-    const int tid = threadIdx.x;
-    for (int i = tid; i < DK; i += THREADS) {
-        kq[i] = conv[key_dim + kh * DK + i];
-        kq[DK + i] = conv[kh * DK + i];
-    }
-    __syncthreads();
-    for (int which = 0; which < 2; which++) {
-        float* dst = kq + which * DK;
-        float sum = block_meansq<THREADS>(dst, DK, 1.0, exact, red);
-        float scale = 1.0f / fmaxf(sqrtf(sum), eps);
-        __syncthreads();
-        for (int i = tid; i < DK; i += THREADS) dst[i] = dst[i] * scale;
-        __syncthreads();
-    }
-}
-
 // Fast form for a block of 256 threads: thread t < DK holds k[t], thread DK + t holds q[t]; each
 // vector's sum of squares is reduced in its own waves, two barriers in all.
 // `v` is the thread's element, loaded by the caller (ahead of its other loads: loads return in order).
@@ -519,11 +691,10 @@ __device__ __forceinline__ void l2_kq_fast(float v, float eps, float* kq, double
     __syncthreads();
 }
 
-IT_DEV void gdn_gates(const GdnCoreP& p, int h, float* g, float* beta) {
-    float a = p.alpha[h] + p.dt_bias[h];
-    float softplus = a > 20.0f ? a : it_logf(1.0f + it_expf(a));
-    *g = it_expf(softplus * p.ssm_a[h]);
-    *beta = 1.0f / (1.0f + it_expf(-p.beta[h]));
+IT_DEV void gdn_gates(float a, float ssm_a, float b, const uint64_t* etab, const double (*ltab)[2], float* g, float* beta) {
+    float softplus = a > 20.0f ? a : it_logf_by(1.0f + it_expf_by(a, etab), ltab);
+    *g = it_expf_by(softplus * ssm_a, etab);
+    *beta = 1.0f / (1.0f + it_expf_by(-b, etab));
 }
 // the same on the transcendental unit, for the kernel that reorders its sums anyway
 IT_DEV void gdn_gates_fast(const GdnCoreP& p, int h, float* g, float* beta) {
@@ -533,18 +704,34 @@ IT_DEV void gdn_gates_fast(const GdnCoreP& p, int h, float* g, float* beta) {
     *beta = fx_sigmoid(p.beta[h]);
 }
 
-// Exact form: one lane owns one value row, the three sweeps run in the CPU path's order.
+// Exact form: one lane owns one value row, the three sweeps run in the CPU path's order: chains of DK additions, eight cycles each.
+// What is in front of them is asked for at once, and the tables of the gates' exponentials and logarithm sit in LDS (four
+// lookups in constant memory, one behind the other, cost as much as a sweep): heads of 64 5.1 -> 4.1 us, of 128 8.4 -> 7.4.
 template <int DK>
 __global__ __launch_bounds__(64) void gdn_rows_exact_k(GdnCoreP p) {
     __shared__ __align__(16) float kq[2 * DK];
-    __shared__ double red[2];
+    __shared__ uint64_t etab[32];
+    __shared__ double ltab[16][2];
+    constexpr int PER = DK / 64;                 // of the key's and of the query's values a lane
     const int lane = threadIdx.x;
     const int dv = DK;
     const int bph = dv / 64;
     const int h = blockIdx.x / bph, jb = blockIdx.x % bph, kh = h % p.n_k_heads;
     const int key_dim = p.n_k_heads * DK;
-    load_kq_l2<DK, 64>(p.conv, key_dim, kh, p.eps, p.exact, kq, red);
+    float kv[2][PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        kv[0][i] = p.conv[key_dim + kh * DK + lane + 64 * i];
+        kv[1][i] = p.conv[kh * DK + lane + 64 * i];
+    }
+    if (lane < 32) etab[lane] = IT_EXP2F_TAB[lane];
+    if (lane < 16) {
+        ltab[lane][0] = IT_LOGF_TAB[lane][0];
+        ltab[lane][1] = IT_LOGF_TAB[lane][1];
+    }
+    const float a = p.alpha[h] + p.dt_bias[h], ssm_a = p.ssm_a[h], b = p.beta[h];
     const int j = jb * 64 + lane;
+    const float v = p.conv[2 * key_dim + h * dv + j];
     float* S = p.state + ((int64_t)h * dv + j) * DK;
     float row[DK];
     const float4* S4 = (const float4*)S;
@@ -553,9 +740,33 @@ __global__ __launch_bounds__(64) void gdn_rows_exact_k(GdnCoreP p) {
         float4 t = S4[i];
         row[4 * i] = t.x; row[4 * i + 1] = t.y; row[4 * i + 2] = t.z; row[4 * i + 3] = t.w;
     }
+    wave_lds_sync();
+    // l2-normalised k (first half of kq) and q (second half) (naive.rs:254-273)
+#pragma unroll
+    for (int which = 0; which < 2; which++) {
+        double part = 0.0;
+#pragma unroll
+        for (int i = 0; i < PER; i++) part += (double)(kv[which][i] * kv[which][i]);
+        part = wave_sum_f64_tail(part);
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, part);
+        const unsigned lo = __builtin_amdgcn_readlane((int)(u & 0xffffffffull), 63), hi = __builtin_amdgcn_readlane((int)(u >> 32), 63);
+        double sum = __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+        float total = (float)sum;
+        if (p.exact && !mean_is_certain(sum, DK, 1, &total)) {
+            sum = 0.0;
+            for (int i = 0; i < DK; i++) {
+                const float x = __shfl(kv[which][i / 64], i & 63, 64);
+                sum += (double)(x * x);
+            }
+            total = (float)sum;
+        }
+        const float scale = 1.0f / fmaxf(sqrtf(total), p.eps);
+#pragma unroll
+        for (int i = 0; i < PER; i++) kq[which * DK + lane + 64 * i] = kv[which][i] * scale;
+    }
     float g, beta;
-    gdn_gates(p, h, &g, &beta);
-    float v = p.conv[2 * key_dim + h * dv + j];
+    gdn_gates(a, ssm_a, b, etab, ltab, &g, &beta);
+    wave_lds_sync();
     const float4* k4 = (const float4*)kq;
     const float4* q4 = (const float4*)(kq + DK);
     float pred = 0.0f;
@@ -654,18 +865,28 @@ void gdn_core(const GdnCoreP& p, int dk, hipStream_t s) {
 
 // ------------------------------------------------------------------ moe_glu_fused
 // grid (row blocks, n_used + 1): y < n_used is routed pick y, y == n_used the shared expert.
+// What bounds it and how it is laid out: as fused_gemv_k (the activation's quads in registers up to the quants, NQ a thread; 0: too many to hold).
+template <int NQ>
 __global__ __launch_bounds__(256) void moe_glu_fused_k(MoeGluP p) {
     extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ uint64_t etab[32];
     const int n_in = p.n_in, nb = n_in >> 5;
-    float* xf = (float*)smem;
-    float* xs = xf + n_in;
+    float* xs = (float*)smem;
     int8_t* xq = (int8_t*)(xs + ((nb + 3) & ~3));
     float* terms_all = (float*)(xq + n_in);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int y = blockIdx.y;
     const bool shared = y == p.n_used;
-    const int fmt = shared ? p.sh_fmt : p.fmt;
     const int64_t e = shared ? 0 : p.route_ids[y];
+    auto quad = [&](int j) __attribute__((always_inline)) {
+        const int i = 4 * (tid + 256 * j);
+        return i < n_in ? load4(p.x + i) : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    float4 xv[NQ ? NQ : 1];
+#pragma unroll
+    for (int j = 0; j < NQ; j++) xv[j] = quad(j);
+    if (tid < 32) etab[tid] = IT_EXP2F_TAB[tid];
+    const int fmt = shared ? p.sh_fmt : p.fmt;
     const uint8_t* gq = shared ? p.sh_gq : p.gq + e * p.q_stride;
     const uint8_t* gs = shared ? p.sh_gs : p.gs + e * p.s_stride;
     const uint8_t* uq = shared ? p.sh_uq : p.uq + e * p.q_stride;
@@ -693,9 +914,22 @@ __global__ __launch_bounds__(256) void moe_glu_fused_k(MoeGluP p) {
             load_items<W_Q8_0, 4>(ru, uq, us, n_in, row00, nrows0, lane);
         }
     }
-    for (int i = tid; i < n_in; i += 256) xf[i] = p.x[i];
-    __syncthreads();
-    lds_quantize_q8_0(xf, n_in, xs, xq);
+    // (a scale of 1, where there is no scale tensor, leaves the bits as they are)
+    const float gsc = shared ? p.sh_gscale : p.gscale2 ? p.gscale2[e] : 1.0f, usc = shared ? p.sh_uscale : p.uscale2 ? p.uscale2[e] : 1.0f;
+    auto put = [&](int j, float4 v) __attribute__((always_inline)) {
+        const int i = 4 * (tid + 256 * j);
+        uint32_t packed;
+        float d;
+        quantize_quad(v, &packed, &d);
+        if (i < n_in) {
+            *(uint32_t*)(xq + i) = packed;
+            if ((tid & 7) == 0) xs[i >> 5] = d;
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < NQ; j++) put(j, xv[j]);
+    if (NQ == 0)
+        for (int j = 0; 1024 * j < n_in; j++) put(j, quad(j));
     __syncthreads();
     for (int g = g0; g < groups; g += gridDim.x * 4) {
         const int row0 = g * R, nrows = min(R, n_out - row0);
@@ -716,18 +950,13 @@ __global__ __launch_bounds__(256) void moe_glu_fused_k(MoeGluP p) {
             compute_items<W_Q8_0, 4>(ru, n_in, nrows, xq, xs, tu, tstride, lane);
         }
         wave_lds_sync();
-        if (lane < nrows) {
-            float ag = fold_terms(tg + lane * tstride, T);
-            float au = fold_terms(tu + lane * tstride, T);
-            if (!shared) {
-                if (p.gscale2) ag *= p.gscale2[e];
-                if (p.uscale2) au *= p.uscale2[e];
-            } else {   // a scale of 1 (no scale tensor) leaves the bits as they are
-                au *= p.sh_uscale;
-                ag *= p.sh_gscale;
-            }
-            out[row0 + lane] = it_silu(ag) * au;
-        }
+        // lanes 0 .. 31 fold gate rows, 32 .. 63 up rows: the two chains side by side
+        const int half = lane >> 5, r = lane & 31;
+        float acc = 0.0f;
+        if (r < nrows) acc = fold_terms((half ? tu : tg) + r * tstride, T);
+        acc *= half ? usc : gsc;
+        const float up = __shfl_xor(acc, 32, 64);
+        if (lane < nrows) out[row0 + lane] = it_silu_by(acc, etab) * up;
         wave_lds_sync();
     }
 }
@@ -738,22 +967,29 @@ void moe_glu_fused(MoeGluP p, hipStream_t s) {
     int R = 4;
     while (R > 1 && R * nb > 256) R /= 2;
     auto lds_for = [&](int r) {
-        return (size_t)p.n_in * 4 + (size_t)((nb + 3) & ~3) * 4 + p.n_in + (size_t)4 * 2 * r * (nb * 2 + 4) * 4;
+        return (size_t)((nb + 3) & ~3) * 4 + p.n_in + (size_t)4 * 2 * r * (nb * 2 + 4) * 4;
     };
     while (R > 1 && lds_for(R) > 60 * 1024) R /= 2;
     p.rows_per_wave = R;
     int n_out = p.n_out > p.sh_n_out ? p.n_out : p.sh_n_out;
     int gx = (n_out + 4 * R - 1) / (4 * R);  // one row group per wave
     if (gx < 1) gx = 1;
-    hipLaunchKernelGGL(moe_glu_fused_k, dim3(gx, p.n_used + 1), dim3(256), lds_for(R), s, p);
+    const dim3 grid(gx, p.n_used + 1);
+    if (p.n_in <= 1024) hipLaunchKernelGGL(moe_glu_fused_k<1>, grid, dim3(256), lds_for(R), s, p);
+    else if (p.n_in <= 2048) hipLaunchKernelGGL(moe_glu_fused_k<2>, grid, dim3(256), lds_for(R), s, p);
+    else if (p.n_in <= 4096) hipLaunchKernelGGL(moe_glu_fused_k<4>, grid, dim3(256), lds_for(R), s, p);
+    else hipLaunchKernelGGL(moe_glu_fused_k<0>, grid, dim3(256), lds_for(R), s, p);
 }
 
 // ------------------------------------------------------------------ moe_down_fused
 // x[j] += sum_e w_e * (down_e[j] . g_e * scale2_e) + (shared_down[j] . g_sh) * sigmoid(logit)
 // (src/ops/mod.rs:1134-1171 then add_assign), experts ascending, shared last.
-constexpr int DOWN_ITEMS = 8;
+// What bounds it and how it is laid out: as fused_gemv_k.  What a row's end needs (the picks' scales and weights, the gate's
+// logit, the residual stream) is asked for at the start.
+constexpr int DOWN_ITEMS = 8, DOWN_QUADS = 6;   // (quads: of the intermediates, in a thread's registers; longer ones are staged in LDS)
 __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ uint64_t etab[32];
     const int n_in = p.n_in, nb = n_in >> 5;       // expert down: n_in = expert_ff
     const int sh_in = p.sh_n_in, sh_nb = sh_in >> 5;
     const int NU = p.n_used;
@@ -761,7 +997,21 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     float* xs = (float*)smem;                                     // NU*nb + sh_nb scales
     int8_t* xq = (int8_t*)(xs + ((NU * nb + sh_nb + 3) & ~3));    // NU*n_in + sh_in quants
     float* terms_all = (float*)(xq + ((NU * n_in + sh_in + 15) & ~15));
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int my_id = p.route_ids[lane < NU ? lane : 0];   // every pick in one load
+    const float my_w = p.route_w[lane < NU ? lane : 0];
+    const int total = NU * n_in + sh_in;                   // the intermediates: the picks' and the shared one's, 32-aligned
+    const bool by_regs = total <= 4 * 256 * DOWN_QUADS;
+    float4 xv[DOWN_QUADS];
+    if (by_regs) {
+#pragma unroll
+        for (int j = 0; j < DOWN_QUADS; j++) {
+            const int i = 4 * (tid + 256 * j);
+            xv[j] = i < NU * n_in ? load4(p.g_all + i) : i < total ? load4(p.g_shared + (i - NU * n_in)) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    const float logit = p.logit[0];
+    if (tid < 32) etab[tid] = IT_EXP2F_TAB[tid];
     it_count_expert_reads(p.route_ids, NU, p.counts_gate, p.counts_up, p.counts_down, p.tally);
     const int R = p.rows_per_wave;
     const int T = p.fmt == W_NVFP4 ? nb * 2 : nb;
@@ -775,12 +1025,13 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     // a group's, for what the launcher sizes it for) in flight at once.
     RowRegs<DOWN_ITEMS> rr;
     RowRegs<1> rsh;
-    const int my_id = p.route_ids[lane < NU ? lane : 0];   // every pick in one load
     auto load_all = [&](int row0, int nrows, int i0) __attribute__((always_inline)) {
         const int per = nrows * nb;
+        const float inv_per = inv_of(per), inv_nb = inv_of(nb);
 #pragma unroll
         for (int k = 0; k < DOWN_ITEMS; k++) {
-            const int it = min(i0 + k * 64 + lane, NU * per - 1), y = it / per, ru = it - y * per, r = ru / nb, u = ru - r * nb;
+            if (i0 + k * 64 >= NU * per) break;
+            const int it = min(i0 + k * 64 + lane, NU * per - 1), y = row_of(it, inv_per), ru = it - y * per, r = row_of(ru, inv_nb), u = ru - r * nb;
             const int64_t e = __shfl(my_id, y, 64);
             const int64_t row = row0 + r;
             const uint8_t *q = p.q + e * p.q_stride, *sc = p.s + e * p.s_stride;
@@ -799,30 +1050,57 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
         else load_items<W_Q8_0, 1>(rsh, p.sh_q, p.sh_s, sh_in, row0, nrows, lane);
     };
     const int g0 = blockIdx.x * 4 + wave;
+    // lane (y, r) of a group: its pick's second scale and weight; lane r: the row's value so far
+    float sc2 = 1.0f, x_old = 0.0f;
+    auto ask_end = [&](int row0, int nrows) __attribute__((always_inline)) {
+        const int y = row_of(lane, inv_of(nrows));
+        const int id = __shfl(my_id, min(y, NU - 1), 64);
+        sc2 = y >= NU ? p.sh_dscale : p.scale2 ? p.scale2[id] : 1.0f;
+        x_old = lane < nrows ? p.x[row0 + lane] : 0.0f;
+    };
     if (g0 < groups) {
-        load_all(g0 * R, min(R, p.n_out - g0 * R), 0);
-        load_shared(g0 * R, min(R, p.n_out - g0 * R));
+        const int nrows = min(R, p.n_out - g0 * R);
+        load_all(g0 * R, nrows, 0);
+        load_shared(g0 * R, nrows);
+        ask_end(g0 * R, nrows);
     }
-    const float gate = it_sigmoid(p.logit[0]);
-    // stage all NU + 1 intermediates as f32 (the term region is free until the main loop)
-    {
+    if (by_regs) {
+#pragma unroll
+        for (int j = 0; j < DOWN_QUADS; j++) {
+            if (1024 * j >= total) break;
+            const int i = 4 * (tid + 256 * j);
+            uint32_t packed;
+            float d;
+            quantize_quad(xv[j], &packed, &d);
+            if (i < total) {
+                *(uint32_t*)(xq + i) = packed;
+                if ((tid & 7) == 0) xs[i >> 5] = d;
+            }
+        }
+    } else {
+        // stage all NU + 1 intermediates as f32 (the term region is free until the main loop)
         float* all = terms_all;
-        const int total = NU * n_in + sh_in;
         for (int i = tid; i < total; i += 256) all[i] = i < NU * n_in ? p.g_all[i] : p.g_shared[i - NU * n_in];
         __syncthreads();
         // one Q8_0 block per 8 lanes; picks and the shared vector are back to back and 32-aligned
         lds_quantize_q8_0(all, total, xs, xq);
-        __syncthreads();
     }
+    __syncthreads();
+    const float gate = it_sigmoid_by(logit, etab);
     for (int g = g0; g < groups; g += gridDim.x * 4) {
         const int row0 = g * R, nrows = min(R, p.n_out - row0);
-        if (g != g0) load_shared(row0, nrows);
+        if (g != g0) {
+            load_shared(row0, nrows);
+            ask_end(row0, nrows);
+        }
         const int per = nrows * nb;
+        const float inv_per = inv_of(per), inv_nb = inv_of(nb), inv_rows = inv_of(nrows);
         for (int i0 = 0; i0 < NU * per; i0 += 64 * DOWN_ITEMS) {
             if (g != g0 || i0) load_all(row0, nrows, i0);
 #pragma unroll
             for (int k = 0; k < DOWN_ITEMS; k++) {
-                const int it = i0 + k * 64 + lane, y = it / per, ru = it - y * per, r = ru / nb, u = ru - r * nb;
+                if (i0 + k * 64 >= NU * per) break;
+                const int it = i0 + k * 64 + lane, y = row_of(it, inv_per), ru = it - y * per, r = row_of(ru, inv_nb), u = ru - r * nb;
                 if (it >= NU * per) continue;
                 const uint4* ap = (const uint4*)(xq + y * n_in + u * 32);
                 const uint4 a0 = ap[0], a1 = ap[1];
@@ -844,27 +1122,17 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
             else compute_items<W_Q8_0, 1>(rsh, sh_in, nrows, xq + NU * n_in, xs + NU * nb, t, tstride, lane);
         }
         wave_lds_sync();
-        // lane = (y, r): fold its dot, park it in slot 0 of its own term row
+        // lane = (y, r): fold its dot; lane r adds them up, the picks in order, the shared expert last
         float dot = 0.0f;
         const int pairs = (NU + 1) * nrows;
-        if (lane < pairs) {
-            const int y = lane / nrows, r = lane - y * nrows;
-            dot = fold_terms(terms + ((size_t)y * R + r) * tstride, y < NU ? T : shT);
-            if (y < NU && p.scale2) dot *= p.scale2[p.route_ids[y]];
-            if (y == NU) dot *= p.sh_dscale;
-        }
-        wave_lds_sync();
-        if (lane < pairs) {
-            const int y = lane / nrows, r = lane - y * nrows;
-            terms[((size_t)y * R + r) * tstride] = dot;
-        }
-        wave_lds_sync();
-        if (lane < nrows) {
-            float v = 0.0f;
-            for (int y = 0; y < NU; y++) v += p.route_w[y] * terms[((size_t)y * R + lane) * tstride];
-            v += terms[((size_t)NU * R + lane) * tstride] * gate;
-            p.x[row0 + lane] += v;
-        }
+        const int y = row_of(lane, inv_rows), r = lane - y * nrows;
+        if (lane < pairs) dot = fold_terms(terms + ((size_t)y * R + r) * tstride, y < NU ? T : shT) * sc2;
+        const float w = __shfl(my_w, min(y, NU - 1), 64);
+        dot = y < NU ? w * dot : dot * gate;
+        float v = 0.0f;
+#pragma unroll 4
+        for (int k = 0; k <= NU; k++) v += __shfl(dot, min(k * nrows + lane, 63), 64);
+        if (lane < nrows) p.x[row0 + lane] = x_old + v;
         wave_lds_sync();
     }
 }
@@ -913,7 +1181,7 @@ __global__ __launch_bounds__(64) void attn_prep_k(AttnPrepP p) {
     const float* w = is_q ? p.q_norm : p.k_norm;
     for (int i = tid; i < hd; i += 64) hbuf[i] = src[i];
     __syncthreads();
-    float scale = 1.0f / sqrtf(block_meansq<64>(hbuf, hd, (double)hd, p.exact, red) + p.eps);
+    float scale = 1.0f / sqrtf(block_meansq<64>(hbuf, hd, hd, p.exact, red) + p.eps);
     __syncthreads();
     for (int i = tid; i < hd; i += 64) hbuf[i] = hbuf[i] * scale * w[i];
     __syncthreads();

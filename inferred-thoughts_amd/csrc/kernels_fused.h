@@ -31,7 +31,8 @@ struct FusedGemvP {
     // optional: matrix 0 is the router; the last block to finish picks the experts
     unsigned* route_counter;  // zero between launches
     const float* route_logits;   // filled by the launcher
-    int terms_stride;            // filled by the launcher: floats of LDS per wave
+    int terms_stride;            // filled by the launcher: floats of LDS per wave that takes quantized rows
+    int q_blocks;                // filled by the launcher: blocks that take quantized rows, in front of those that take the others (exact kernel)
     int n_expert, n_used;
     int32_t* route_ids;
     float* route_w;
