@@ -77,6 +77,13 @@ IT_DEV void to_lds(const void* from, uint32_t to) {
     asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "{m0}"(to), "v"(from) : "memory");
 }
 
+// The same from base + off (base: the same in every lane, in scalar registers).  A scalar register that a vector instruction has
+// written (a v_readlane of the compiler's) may be read by a memory instruction five wait states later; inside a statement the
+// compiler does not see that there is one.
+IT_DEV void to_lds_at(const void* base, uint32_t off, uint32_t to) {
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(to), "v"(off), "s"(base) : "memory");
+}
+
 // operands of the f16 expert tile kernels (k_gemm_f16.hip, k_gemm_f16s.hip)
 struct ExpertsF16P {
     const uint8_t *q, *s, *q2, *s2;

@@ -72,11 +72,6 @@ IT_DEV int here(int v) {
     asm volatile("" : "+v"(v));
     return v;
 }
-// 16 bytes a lane from base + off to LDS, one lane's behind the other's from `to` on (base, to: the same in every lane)
-IT_DEV void to_lds_at(const void* base, uint32_t off, uint32_t to) {
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "{m0}"(to), "v"(off), "s"(base) : "memory");
-}
-
 // NL loads of a wave, 1,024 bytes each: rows row0 .. of a slice (row0: a multiple of 8, the same in every lane), which are keys
 // key0 + row of one KV head, to `to` of LDS (whose array starts at `lds`, address `at`).  `left` of them are there: loads without a row
 // of their own are left out (ZERO: zeros instead), in the last one the rows behind are the last one again.
