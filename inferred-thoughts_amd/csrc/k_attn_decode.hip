@@ -549,7 +549,8 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int d = kb + 8 * (i >> 2) + 4 * g + (i & 3) - pos_lo;
-                    if (d >= 0 && d < n_block - 1) own_p[pw][d][c] = __builtin_bit_cast(uint16_t, pf[i >> 3][i & 7]);
+                    const _Float16 p = pf[i >> 3][i & 7];      // (a bit_cast of a vector's element itself reads the first one)
+                    if (d >= 0 && d < n_block - 1) own_p[pw][d][c] = __builtin_bit_cast(uint16_t, p);
                 }
             }
             const int vk = here(v_key);

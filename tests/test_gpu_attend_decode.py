@@ -57,6 +57,37 @@ def test_a_row_does_not_depend_on_what_stands_behind_it(hip, orc, n_q, n_pos, hd
         assert not np.isfinite(got[t + 1:, :, 3]).any()
 
 
+@pytest.mark.parametrize("hd,nh,nkv", [(64, 8, 2), (128, 8, 1), (256, 4, 4)])
+@pytest.mark.parametrize("n_pos", [9, 40, 70, 71, 1039])
+def test_an_infinite_value_counts_with_its_own_keys_weight(hip, orc, n_pos, hd, nh, nkv):
+    # two queries; the last key, which only the second sees, holds an infinity.  Scores of 0 and, in turn, of the last key or of
+    # all the others 200 lower, a weight of zero in f32 too: 0 x inf is not a number, any other weight's product an infinity
+    r = rng(n_pos + hd)
+    kv_dim = nkv * hd
+    q = np.zeros((2, nh, hd), np.float32)
+    q[..., 0] = 1.0
+    v = r.standard_normal((n_pos, kv_dim)).astype(np.float16)
+    v[-1, 3::hd] = np.inf
+    for last, others in ((0.0, 0.0), (0.0, -200.0), (-200.0, 0.0)):
+        k = np.zeros((n_pos, kv_dim), np.float16)
+        k[:, ::hd] = others
+        k[-1, ::hd] = last
+        rows = []
+        for be in (hip, orc):
+            out = np.zeros(q.size, np.float32)
+            if be is hip:
+                hip.drop_mirrors(); hip.begin_pass(2)
+            be.attend(q.reshape(-1), f16_bits(k).reshape(-1), f16_bits(v).reshape(-1), kv_dim, n_pos, hd, nh, nkv, np.float32(1.0), out)
+            if be is hip:
+                hip.host_needs(out); hip.end_pass(); hip.raise_if_error()
+            rows.append(out.reshape(2, nh, hd))
+        got, want = rows
+        assert np.isfinite(want[0]).all() and np.isfinite(got[0]).all(), (last, others)
+        assert np.array_equal(np.isnan(got[1]), np.isnan(want[1])), (last, others)
+        assert np.array_equal(np.isposinf(got[1]), np.isposinf(want[1])), (last, others)
+        assert close(np.nan_to_num(got, posinf=0), np.nan_to_num(want, posinf=0))
+
+
 @pytest.mark.parametrize("hd,nh,nkv", [(64, 8, 2), (64, 4, 4), (128, 8, 1), (128, 32, 4), (256, 16, 2), (256, 4, 2)])
 # one query to two groups of eight; contexts around a wave's quarter (8), a slice (32), a stage (64, 128) and a round of ranges
 @pytest.mark.parametrize("n_q", [1, 2, 3, 4, 5, 8, 9, 16])
