@@ -10,6 +10,7 @@
 // MFMA operand layout (16x16x32, i8): lane l supplies 8 consecutive k of row (l % 16) at
 // k = 8 * (l / 16) for both A (weight rows) and B (tokens); it receives D for token l % 16
 // and weight rows 4 * (l / 16) + {0,1,2,3}.
+#include <algorithm>
 #include <type_traits>
 
 #include "it_device.h"
@@ -148,24 +149,20 @@ __global__ __launch_bounds__(GT) void q8_gemm_k(const int8_t* __restrict__ wq, c
 // buffer has been read and costs no register, no store and one barrier for 256 k.  Such a load writes its lanes' 16 bytes
 // side by side, so a row's sixteen pieces are permuted by the row's number instead of being padded apart: sixteen rows' reads
 // of a piece start in different banks.  The arithmetic is the same, product by product, in the same order.
-// Bound from some 500 tokens on by the twelve vector operations per product of the matrix cores (5,700 tokens: vector ALU busy
-// 71 %, matrix cores 16 to 18 %, two waves a SIMD; LDS reads still meet in the banks, 3 to 4 conflict cycles for each
-// four-cycle unit of LDS activity, but 2 to 5 % of the wave cycles wait on them; with the scales' products moved to the matrix
-// cores as outer products, eight operations, the time does not change), below by the stages' latency.  8192 x 2048 over 64 / 201 / 512 / 5,700 tokens: 18.1 -> 11.2, 33.0 -> 27.5, 55.7 -> 50.8, 618 -> 528 us; 4096 x 2048:
-// 16.0 -> 9.3, 24.9 -> 15.4, 33.7 -> 28.3, 296 -> 272; 2048 x 4096: 28.5 -> 15.8, 32.4 -> 18.7, 41.2 -> 27.4, 290 -> 276.
-// Not kept: three or four stages (0 to 50 % slower everywhere: fewer blocks fit a CU); the f16 matrix cores with the
-// activations as an f16 pair and no scale per token, 128 x 256 tiles (8192 x 2048 over 5,700: 437 us with three stages, 46 % of
-// the rate the matrix cores sustain, but 20 % behind on everything smaller).
+// For the few-token end, where it is bound by the stages' latency (from some 500 tokens on by the twelve vector operations per
+// product, for which there is the kernel below).  8192 x 2048 over 64 tokens: 18.1 -> 11.2 us; 4096 x 2048 over 64 / 201: 16.0 -> 9.3,
+// 24.9 -> 15.4; 2048 x 4096 over 64 / 201 / 512: 28.5 -> 15.8, 32.4 -> 18.7, 41.2 -> 27.4.  Three or four stages: 0 to 50 % slower everywhere, fewer
+// blocks fit a CU.  The f16 matrix cores with the activations as an f16 pair and no scale per token, 128 x 256 tiles: 437 us for 8192 x 2048 over
+// 5,700, and 20 % behind on everything smaller.
 typedef _Float16 hv8 __attribute__((ext_vector_type(8)));
 
-template <int NT> constexpr int tile_stage_bytes() { return 64 * 256 + NT * 16 * 256 + 1024 + (NT > 2 ? 2048 : 1024); }
+template <int NT> constexpr int tile_stage_bytes() { return 64 * 256 + NT * 16 * 256 + 1024 + 1024; }
 
 template <int NT, bool FMA>
 __global__ __launch_bounds__(256) void q8_tile_k(const int8_t* __restrict__ wq, const uint16_t* __restrict__ ws,
                                                  const int8_t* __restrict__ xq, const float* __restrict__ xs,
                                                  float* __restrict__ out, int n_in, int n_out, int n_tok, float out_scale) {
     constexpr int STAGE = tile_stage_bytes<NT>(), X_AT = 64 * 256, WS_AT = X_AT + NT * 16 * 256, XS_AT = WS_AT + 1024;
-    constexpr int XS = NT > 2 ? 2 : 1;                  // waves that bring token scales
     extern __shared__ __align__(1024) uint8_t tlds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -187,9 +184,9 @@ __global__ __launch_bounds__(256) void q8_tile_k(const int8_t* __restrict__ wq, 
         const int row = (wave * NT + i) * 4 + (lane >> 4);
         xp[i] = xq + (int64_t)min(tok0 + row, n_tok - 1) * n_in + (((lane & 15) ^ (row & 15)) << 4);
     }
-    const bool has_scales = wave <= XS;
+    const bool has_scales = wave < 2;
     const uint8_t* sp = wave == 0 ? (const uint8_t*)(ws + (int64_t)min(row0 + lane, n_out - 1) * nb)
-                                  : (const uint8_t*)(xs + (int64_t)min(tok0 + min((wave - 1) * 32 + (lane >> 1), NT * 16 - 1), n_tok - 1) * nb + 4 * (lane & 1));
+                                  : (const uint8_t*)(xs + (int64_t)min(tok0 + min(lane >> 1, NT * 16 - 1), n_tok - 1) * nb + 4 * (lane & 1));
     const int s_step = wave == 0 ? 16 : 32;
     auto ask = [&](int s, int buf) __attribute__((always_inline)) {
         const uint32_t d = at + buf * STAGE;
@@ -261,6 +258,184 @@ __global__ __launch_bounds__(256) void q8_tile_k(const int8_t* __restrict__ wq, 
     }
 }
 
+// ------------------------------------------------------------------ ... and enough of them: 32 x 32 products, 128 rows a block
+// A block owns 128 weight rows x 32 TT tokens; each of its four waves takes 32 rows against all the tokens by MFMA 32x32x32, so a
+// block of 32 k of two tiles is one instruction with a lane's sixteen results behind it.  Lane l supplies 16 k, of its half
+// l / 32, of row (or token) l % 32 and receives D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32], i = 0..15: a token's scale serves a lane's
+// sixteen products, and a row's is read from LDS as f32 with three others.  (Above, two of a lane's twelve operations and half of
+// its LDS reads went into operands that served four products.)  A stage is 128 k and there are two; what of the next one a wave
+// brings is asked for between the products of this one, a request a product.
+// Bound by the three vector operations (convert, scale, add) of every product: 8192 x 2048 over 5,700 tokens 379 us, of which 282
+// remain without loads and stores, 236 without the matrix cores too.  The product of a tile is therefore started before the last
+// tile's is scaled (the compiler alone waited for each), and the outputs go through LDS to be stored 512 bytes a token (32 before: 411).
+// Before, with the 64 x 64 blocks of the kernel above, 563; 4096 x 2048: 270 -> 171; 2048 x 4096: 277 -> 182; 8192 x 2048 over 512:
+// 50 -> 35.  The arithmetic is the same, product by product, in the same order.
+typedef int v16i __attribute__((ext_vector_type(16)));
+constexpr int WIDE_ROWS = 128, WIDE_K = 128;
+template <int TT> constexpr int wide_stage_bytes() { return (WIDE_ROWS + 32 * TT) * (WIDE_K + 16); }
+
+template <int TT, bool FMA>
+__global__ __launch_bounds__(256, 2) void q8_wide_k(const int8_t* __restrict__ wq, const uint16_t* __restrict__ ws,
+                                                    const int8_t* __restrict__ xq, const float* __restrict__ xs,
+                                                    float* __restrict__ out, int n_in, int n_out, int n_tok, float out_scale) {
+    constexpr int STAGE = wide_stage_bytes<TT>(), X_AT = WIDE_ROWS * WIDE_K, WS_AT = X_AT + 32 * TT * WIDE_K, XS_AT = WS_AT + WIDE_ROWS * 16;
+    extern __shared__ __align__(1024) uint8_t tlds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c32 = lane & 31, half = lane >> 5, turn = (c32 >> 1) & 7;
+    const int row0 = blockIdx.x * WIDE_ROWS, tok0 = blockIdx.y * 32 * TT;
+    const int nb = n_in >> 5, n_stage = n_in / WIDE_K;
+    const uint32_t at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)tlds);
+    const int8_t* const wbase = wq + (int64_t)row0 * n_in;
+    const int8_t* const xbase = xq + (int64_t)tok0 * n_in;
+
+    // what this lane fetches every stage: a piece of four weight rows and of TT token rows, and four scales of a row
+    uint32_t wo[4], xo[TT];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int row = (wave * 4 + i) * 8 + (lane >> 3);
+        wo[i] = (uint32_t)min(row, n_out - 1 - row0) * n_in + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    }
+#pragma unroll
+    for (int i = 0; i < TT; i++) {
+        const int row = (wave * TT + i) * 8 + (lane >> 3);
+        xo[i] = (uint32_t)min(row, n_tok - 1 - tok0) * n_in + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    }
+    const bool of_w = wave < 2;       // which scales: of the 128 rows, or of the tokens
+    const int s_row = of_w ? tid : min(tid - 128, 32 * TT - 1);
+    const uint8_t* const sp = of_w ? (const uint8_t*)(ws + (int64_t)min(row0 + s_row, n_out - 1) * nb) : (const uint8_t*)(xs + (int64_t)min(tok0 + s_row, n_tok - 1) * nb);
+    auto ask = [&](int s, int buf, int i) __attribute__((always_inline)) {
+        const uint32_t d = at + buf * STAGE;
+        if (i < 4) to_lds_at(wbase + s * WIDE_K, wo[i & 3], d + (wave * 4 + i) * 1024);
+        else to_lds_at(xbase + s * WIDE_K, xo[(i - 4) % TT], d + X_AT + (wave * TT + i - 4) * 1024);
+    };
+    float4 sc;
+    auto load_scales = [&](int s) __attribute__((always_inline)) {
+        if (of_w) {
+            typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
+            const hv4 v = *(const hv4*)(sp + s * 8);
+            sc = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+        } else {
+            sc = *(const float4*)(sp + s * 16);
+        }
+    };
+    auto put_scales = [&](int buf) __attribute__((always_inline)) {
+        float* const d = (float*)(tlds + buf * STAGE + (of_w ? WS_AT : XS_AT)) + s_row;
+        const int step = of_w ? WIDE_ROWS : 32 * TT;
+        if (of_w || tid - 128 < 32 * TT) {
+            d[0] = sc.x;
+            d[step] = sc.y;
+            d[2 * step] = sc.z;
+            d[3 * step] = sc.w;
+        }
+    };
+    float acc[TT][16];
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[tt][i] = 0.0f;
+
+#pragma unroll
+    for (int i = 0; i < 4 + TT; i++) ask(0, 0, i);
+    load_scales(0);
+    auto stage = [&](int s, auto more_of) __attribute__((always_inline)) {
+        constexpr bool more = decltype(more_of)::value;
+        const int buf = s & 1;
+        put_scales(buf);                          // (the other buffer's are still read)
+        __builtin_amdgcn_s_waitcnt(0x0070);      // stage s has landed, and this wave's scales
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (more) load_scales(s + 1);
+        const uint8_t* const d = tlds + buf * STAGE;
+        // unit u: block u / TT of the stage, token tile u % TT.  Its product is started before the one before it is scaled and added, its
+        // operands are read one unit earlier.
+        constexpr int UNITS = 4 * TT;
+        v4i a[2], bv[2];
+        float x[2], w[2][16];
+        v16i c[2];
+        auto read = [&](int u) __attribute__((always_inline)) {
+            const int b = u / TT, tt = u % TT, piece = ((2 * b + half) ^ turn) << 4;
+            if (tt == 0) a[b & 1] = *(const v4i*)(d + (wave * 32 + c32) * WIDE_K + piece);
+            bv[u & 1] = *(const v4i*)(d + X_AT + (tt * 32 + c32) * WIDE_K + piece);
+        };
+        auto read_scales = [&](int u) __attribute__((always_inline)) {
+            const int b = u / TT, tt = u % TT;
+            if (tt == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float4 v = *(const float4*)(d + WS_AT + 4 * (b * WIDE_ROWS + wave * 32 + 8 * i + 4 * half));
+                    w[b & 1][4 * i] = v.x, w[b & 1][4 * i + 1] = v.y, w[b & 1][4 * i + 2] = v.z, w[b & 1][4 * i + 3] = v.w;
+                }
+            }
+            x[u & 1] = *(const float*)(d + XS_AT + 4 * (b * 32 * TT + tt * 32 + c32));
+        };
+        auto start = [&](int u) __attribute__((always_inline)) {
+            v16i z;
+#pragma unroll
+            for (int i = 0; i < 16; i++) z[i] = 0;
+            c[u & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[(u / TT) & 1], bv[u & 1], z, 0, 0, 0);
+        };
+        read(0);
+        read_scales(0);
+        start(0);
+        read(1);
+        read_scales(1);
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (u + 1 < UNITS) start(u + 1);
+            if (u + 2 < UNITS) read(u + 2);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int tt = u % TT;
+                if (FMA) acc[tt][i] = fmaf((float)c[u & 1][i], w[(u / TT) & 1][i] * x[u & 1], acc[tt][i]);
+                else acc[tt][i] += (float)c[u & 1][i] * (w[(u / TT) & 1][i] * x[u & 1]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 16; i++) asm volatile("" : "+v"(acc[u % TT][i]));      // (done here: kept for later they fill the registers)
+            constexpr int PER = (4 + TT + UNITS - 1) / UNITS;
+            if (more) {
+#pragma unroll
+                for (int k = 0; k < PER; k++)
+                    if (u * PER + k < 4 + TT) ask(s + 1, buf ^ 1, u * PER + k);
+            }
+            if (u + 2 < UNITS) read_scales(u + 2);
+        }
+    };
+    for (int s = 0; s + 1 < n_stage; s++) stage(s, std::true_type{});
+    stage(n_stage - 1, std::false_type{});
+    // through LDS, so that a token's 128 outputs are stored side by side
+    constexpr int OSTR = WIDE_ROWS + 4;
+    static_assert(32 * TT * OSTR * 4 <= 2 * STAGE);
+    float* const o_lds = (float*)tlds;
+    __syncthreads();
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; i4++) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = out_scale != 1.0f ? acc[tt][4 * i4 + i] * out_scale : acc[tt][4 * i4 + i];
+            *(float4*)(o_lds + (tt * 32 + c32) * OSTR + wave * 32 + 8 * i4 + 4 * half) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+    __syncthreads();
+    const int j = row0 + 4 * (tid & 31);
+    for (int tt = tid >> 5; tt < 32 * TT && tok0 + tt < n_tok; tt += 8) {
+        const float4 v = *(const float4*)(o_lds + tt * OSTR + 4 * (tid & 31));
+        float* const o = out + (int64_t)(tok0 + tt) * n_out + j;
+        if (j + 3 < n_out && !(n_out & 3)) {
+            *(float4*)o = v;
+        } else {
+            const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (j + i < n_out) o[i] = f[i];
+        }
+    }
+}
+
 }  // namespace
 
 bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, int n_tok, float* out, float out_scale,
@@ -280,26 +455,42 @@ bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, 
     } while (0)
     const bool slabs = w.n_in % 256 == 0 && !((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(act_scales) | reinterpret_cast<uintptr_t>(out)) & 15);
     if (slabs) {
-        // 16 tokens a block up to 640 of the smallest blocks (2.5 a CU), 32 above, 64 from 32,768 on (8192 rows over 5,700 tokens:
-        // 528 us with 64, 617 with 32; 4096 rows: 290, 272)
-        const int64_t units = (int64_t)gx * tiles;
-        auto launch = [&](auto nt, auto fm) {
-            constexpr int NT = decltype(nt)::value;
-            constexpr bool F = decltype(fm)::value;
-            constexpr size_t lds = 2 * tile_stage_bytes<NT>();
-            static const bool ok = hipFuncSetAttribute((const void*)q8_tile_k<NT, F>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess;
-            if (!ok) {
+        auto launch = [&](auto kernel, int rows, int toks, size_t lds) {
+            if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
                 (void)hipGetLastError();
                 return false;
             }
-            hipLaunchKernelGGL((q8_tile_k<NT, F>), dim3(gx, (tiles + NT - 1) / NT), dim3(256), lds, s, wq, ws, act_quants, act_scales, out, w.n_in,
-                               w.n_out, n_tok, out_scale);
+            hipLaunchKernelGGL(kernel, dim3((w.n_out + rows - 1) / rows, (n_tok + toks - 1) / toks), dim3(256), lds, s, wq, ws, act_quants, act_scales,
+                               out, w.n_in, w.n_out, n_tok, out_scale);
             return true;
         };
-        auto by_mode = [&](auto nt) { return fma ? launch(nt, std::true_type{}) : launch(nt, std::false_type{}); };
+        auto tile = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            return launch(fma ? q8_tile_k<NT, true> : q8_tile_k<NT, false>, 64, 16 * NT, 2 * tile_stage_bytes<NT>());
+        };
+        auto wide = [&](auto tt) {
+            constexpr int TT = decltype(tt)::value;
+            return launch(fma ? q8_wide_k<TT, true> : q8_wide_k<TT, false>, WIDE_ROWS, 32 * TT, 2 * wide_stage_bytes<TT>());
+        };
         using std::integral_constant;
-        if (units <= 640 ? by_mode(integral_constant<int, 1>{}) : units <= 32768 ? by_mode(integral_constant<int, 2>{}) : by_mode(integral_constant<int, 4>{}))
-            return true;
+        // 64 rows x 16 tokens a block up to 640 of them (2.5 a CU).  Above, the shape that takes least by the blocks a CU gets, b, from
+        // what rows of 2,048 measure (in us; a block alone on its CU is quicker): 64 x 32 2.5 + 6.2 b; 128 x 32, three a CU at a time,
+        // 19, 24 and 31; 128 x 64 25 and 37 for two; 128 x 128 38 and 66.  (4096 x 2048 over 300 / 400 / 512 / 1,100 / 5,700 tokens: 64 x 32 20.3, 26.2,
+        // 28.2, 54.0, 273; 128 x 32 20.9, 21.6, 23.1, 47.2, 209; 128 x 64 25.1, 26.1, 26.5, 53.6, 195; 128 x 128 38.8, 39.5, 39.1, 51.4, 171.)
+        const int64_t units = (int64_t)gx * tiles;
+        if (units <= 640) {
+            if (tile(integral_constant<int, 1>{})) return true;
+        } else {
+            const int64_t gw = (w.n_out + WIDE_ROWS - 1) / WIDE_ROWS;
+            auto per_cu = [&](int64_t rows, int toks) { return (rows * ((n_tok + toks - 1) / toks) + 255) / 256; };
+            const int64_t b1 = per_cu(gw, 32), b2 = per_cu(gw, 64), b4 = per_cu(gw, 128);
+            const int64_t cost[4] = {25 + 62 * per_cu(gx, 32), 306 * (b1 / 3) + (b1 % 3 == 2 ? 240 : b1 % 3 * 190), 369 * (b2 / 2) + b2 % 2 * 250,
+                                     656 * (b4 / 2) + b4 % 2 * 380};
+            const int64_t* const best = std::min_element(cost, cost + 4);
+            if (best == cost ? tile(integral_constant<int, 2>{}) : best == cost + 1 ? wide(integral_constant<int, 1>{})
+                             : best == cost + 2 ? wide(integral_constant<int, 2>{}) : wide(integral_constant<int, 4>{}))
+                return true;
+        }
     }
     // 64 tokens per block at most: four blocks fit a CU (38 KB of LDS, 98 VGPRs) and hide each other's LDS and
     // barrier waits; 128 tokens per block (two blocks per CU) measured 20 % slower despite reading the weights half as often
