@@ -100,6 +100,31 @@ void it_hip::dyn_upload() {
     if (hipEventRecord(dyn_evt[dyn_cur], stream) == hipSuccess) dyn_evt_used[dyn_cur] = true;
 }
 
+namespace {
+// The launches of a recorded pass in their order, if they are a single row of kernels and no more than FEW; else none.
+std::vector<hipKernelNodeParams> few_launches(hipGraph_t g) {
+    constexpr size_t FEW = 8;
+    std::vector<hipKernelNodeParams> out;
+    size_t n = 0, n_root = 1;
+    hipGraphNode_t node = nullptr;
+    if (hipGraphGetNodes(g, nullptr, &n) != hipSuccess || n == 0 || n > FEW || hipGraphGetRootNodes(g, &node, &n_root) != hipSuccess || n_root != 1) return {};
+    while (node) {
+        hipGraphNodeType type;
+        hipKernelNodeParams k{};
+        if (hipGraphNodeGetType(node, &type) != hipSuccess || type != hipGraphNodeTypeKernel || hipGraphKernelNodeGetParams(node, &k) != hipSuccess ||
+            !k.func || !k.kernelParams || k.extra)
+            return {};
+        out.push_back(k);
+        size_t n_next = 0;
+        if (hipGraphNodeGetDependentNodes(node, nullptr, &n_next) != hipSuccess || n_next > 1) return {};
+        hipGraphNode_t next = nullptr;
+        if (n_next && hipGraphNodeGetDependentNodes(node, &next, &n_next) != hipSuccess) return {};
+        node = next;
+    }
+    return out.size() == n ? out : std::vector<hipKernelNodeParams>{};
+}
+}  // namespace
+
 void it_hip::drop_one(Graph& g) {
     if (g.valid && !g.replays) graph_unused++;
     if (g.exec) (void)hipGraphExecDestroy(g.exec);
@@ -214,8 +239,9 @@ void it_hip::finish_pass() {
         graph = nullptr;
         if (e == hipSuccess && g) {
             hipGraphExec_t ex = nullptr;
-            e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
-            if (e == hipSuccess && ex) {
+            auto few = few_launches(g);
+            if (few.empty()) e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
+            if (e == hipSuccess && (ex || !few.empty())) {
                 // a free slot, else the oldest graph's
                 graph = &graphs[0];
                 for (Graph& c : graphs)
@@ -224,6 +250,7 @@ void it_hip::finish_pass() {
                 graph->born = ++graph_captures;
                 graph->graph = g;
                 graph->exec = ex;
+                graph->few = std::move(few);
                 graph->signature = pass_signature;
                 graph->attn_slots = fused_attn_slots;
                 graph->elided = fused_elided;
@@ -268,8 +295,14 @@ void it_hip::finish_pass() {
     pending.clear();
 }
 
+// A recorded pass goes out as one graph, or, where it is a handful of kernels (the chained layers, the head), as those launches:
+// they follow on the kernel before them and are followed without the 5 and 8 us that the device puts around a graph (a token
+// through two chained layers and the head, read by the host: 96 us as a graph, 89 so; a pass of 27 launches of 5 us each is 8 %
+// slower one by one, the host not being ahead of the device).
 void it_hip::launch(Graph& g) {
-    check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
+    if (g.few.empty()) check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
+    for (const hipKernelNodeParams& k : g.few)
+        if (!check(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, stream), "kernel launch")) break;
     graph_launches++;
 }
 

@@ -273,6 +273,7 @@ struct it_hip {
         std::vector<std::array<int, 4>> attn_slots;
         std::vector<const void*> elided;   // device buffers whose ops the graph's fused kernels skip
         bool has_chain = false;
+        std::vector<hipKernelNodeParams> few;   // the launches of a graph of no more than a handful, in order (owned by its nodes)
     };
     // One graph for each kind of single-token pass (fed by the host, fed by the arg-max, ...): a request that takes its
     // prompt's last token one way and goes on the other replays both.  `graph`: the one this pass replays or has recorded.
