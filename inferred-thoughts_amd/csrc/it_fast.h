@@ -125,58 +125,84 @@ IT_DEV double quad_sumsq(float4 v) {
 // value is the weights' denominator, the same in every thread.
 // n_expert <= 4 * THREADS, n_used <= 16.
 //
-// Selection is two-level, with every LDS loop of fixed length so its reads pipeline.  (a) Each
-// thread ranks its values among the 64 * K of its wave: only wave ranks < n_used can be in the
-// global top n_used, and they go to cand[wave][rank].  (b) The NW * 16 candidate slots are
-// ranked against each other.//
+// Selection.  A key is one of the n_used largest only if fewer than n_used of the block's half waves hold a larger one: that
+// leaves some fifteen of 512 keys, which are put side by side and ranked against one another.  (Ranking every key among the 64 of
+// its wave and then each wave's best against one another is 96 dependent compare-and-count pairs a thread, 17 cycles each: 1.4 us
+// of a decode layer's 28 where this takes 0.77.)
 // Probabilities are non-negative, so their bit patterns order like the values; a pick is
 // compared as the 64-bit key (probability bits, ~id): larger key = earlier pick, keys are
-// unique, and an empty slot is key 0.
+// unique, and key 0 is no key.
+template <int THREADS, int PER_THREAD> struct TopLds {
+    unsigned n;                                                       // candidates
+    __attribute__((aligned(16))) unsigned best[THREADS / 32];        // largest value of each half wave
+    __attribute__((aligned(16))) unsigned long long cand[PER_THREAD * THREADS];
+};
 template <int THREADS> struct RouteLds {
     float redf[2 * (THREADS / 64)];
-    __attribute__((aligned(16))) unsigned long long keys[4 * THREADS];
-    __attribute__((aligned(16))) unsigned long long cand[(THREADS / 64) * 16];
+    TopLds<THREADS, 4> top;
 };
 
 IT_DEV unsigned long long route_key(float p, int e) {
     return ((unsigned long long)__float_as_uint(p) << 32) | (unsigned long long)(~(unsigned)e);
 }
 
-// ranks this thread's key among the 64 keys of its wave and files the top n_used (n_expert <= THREADS)
-IT_DEV void wave_rank_one(const unsigned long long* wave_keys, unsigned long long key, int n_used,
-                          unsigned long long* cand) {
-    int rank = 0;
-    const ulonglong2* p2 = (const ulonglong2*)wave_keys;
-#pragma unroll
-    for (int j2 = 0; j2 < 32; j2++) {
-        const ulonglong2 q = p2[j2];
-        rank += q.x > key ? 1 : 0;
-        rank += q.y > key ? 1 : 0;
-    }
-    if (key != 0ull && rank < n_used) cand[rank] = key;
+template <int CTRL, int ROWS> IT_DEV unsigned dpp_umax(unsigned v) {
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false));
 }
-
-// the same with up to four keys per thread (n_expert > THREADS): kept out of line and rolled,
-// so the common kernel does not carry its registers
-template <int THREADS>
-__device__ __attribute__((noinline)) void wave_rank_many(const unsigned long long* keys, unsigned long long key0,
-                                                         unsigned long long key1, unsigned long long key2,
-                                                         unsigned long long key3, int K, int n_used,
-                                                         unsigned long long* cand) {
-    const unsigned long long key[4] = {key0, key1, key2, key3};
-    int rank[4] = {0, 0, 0, 0};
-    for (int k2 = 0; k2 < K; k2++) {
-        const unsigned long long* wk = keys + k2 * THREADS + (threadIdx.x & ~63);
-#pragma unroll 1
-        for (int j = 0; j < 64; j++) {
-            const unsigned long long q = wk[j];
+// the half waves' largest values; a barrier of the block follows, then top_pick.  (Every thread calls both.)
+template <int THREADS, int PER_THREAD>
+IT_DEV void top_begin(TopLds<THREADS, PER_THREAD>& sh, unsigned largest) {
+    largest = dpp_umax<0xB1, 0xf>(largest);        // lane ^ 1
+    largest = dpp_umax<0x4E, 0xf>(largest);        // lane ^ 2
+    largest = dpp_umax<0x141, 0xf>(largest);       // mirrored in 8
+    largest = dpp_umax<0x140, 0xf>(largest);       // in 16
+    largest = dpp_umax<0x142, 0xa>(largest);       // lane 15 of rows 0 and 2 into rows 1 and 3
+    if ((threadIdx.x & 31) == 16) sh.best[threadIdx.x >> 5] = largest;
+    if (threadIdx.x == 0) sh.n = 0;
+}
+// put(rank, key) for the n_used largest of the block's keys (key[k], k < K; 0: none); holds a barrier, and one follows before what
+// put writes is read
+template <int THREADS, int PER_THREAD, int N, class Put>
+IT_DEV void top_pick(TopLds<THREADS, PER_THREAD>& sh, const unsigned long long (&key)[N], int K, int n_used, Put put) {
+    static_assert(N <= PER_THREAD);
+    const int tid = threadIdx.x, lane = tid & 63;
+    unsigned best[THREADS / 32];
 #pragma unroll
-            for (int k = 0; k < 4; k++) rank[k] += q > key[k] ? 1 : 0;
-        }
+    for (int i = 0; i < THREADS / 128; i++) {
+        const uint4 q = ((const uint4*)sh.best)[i];
+        best[4 * i] = q.x, best[4 * i + 1] = q.y, best[4 * i + 2] = q.z, best[4 * i + 3] = q.w;
     }
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-        if (k < K && key[k] != 0ull && rank[k] < n_used) cand[rank[k]] = key[k];
+    for (int k = 0; k < N; k++) {
+        if (k >= K) break;
+        const unsigned mine = (unsigned)(key[k] >> 32);
+        int above0 = 0, above1 = 0;
+#pragma unroll
+        for (int i = 0; i < THREADS / 32; i += 2) {
+            above0 += best[i] > mine ? 1 : 0;
+            above1 += best[i + 1] > mine ? 1 : 0;
+        }
+        const bool in = key[k] != 0ull && above0 + above1 < n_used;
+        const unsigned long long all = __ballot(in);
+        if (all == 0ull) continue;
+        unsigned at = 0;
+        if (lane == 0) at = __hip_atomic_fetch_add(&sh.n, (unsigned)__popcll(all), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        at = __builtin_amdgcn_readfirstlane(at) + __builtin_amdgcn_mbcnt_hi((unsigned)(all >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)all, 0));
+        if (in) sh.cand[at] = key[k];
+    }
+    __syncthreads();
+    // eight threads a candidate
+    const int n = (int)sh.n, part = tid & 7;
+    for (int c0 = 0; c0 < n; c0 += THREADS / 8) {
+        const int c = c0 + (tid >> 3);
+        const unsigned long long me = c < n ? sh.cand[c] : ~0ull;
+        int rank = 0;
+        for (int j = part; j < n; j += 8) rank += sh.cand[j] > me ? 1 : 0;
+        rank += __builtin_amdgcn_update_dpp(0, rank, 0xB1, 0xf, 0xf, true);
+        rank += __builtin_amdgcn_update_dpp(0, rank, 0x4E, 0xf, 0xf, true);
+        rank += __builtin_amdgcn_update_dpp(0, rank, 0x141, 0xf, 0xf, true);
+        if (part == 0 && c < n && rank < n_used) put(rank, me);
+    }
 }
 
 // this thread's logits (up to four experts, THREADS apart): fetched ahead of the activation prologue so that the
@@ -199,7 +225,6 @@ __device__ __forceinline__ float block_route(const float l[4], int n_expert, int
     float m = -INFINITY;
 #pragma unroll
     for (int k = 0; k < 4; k++) m = fmaxf(m, l[k]);
-    if (tid < NW * 16) sh.cand[tid] = 0ull;  // slots a wave does not fill stay empty
     if (tid < 16) wts[tid] = 0.0f;
     m = group_max_tail<64>(m);
     if (lane == 63) sh.redf[wave] = m;
@@ -222,35 +247,20 @@ __device__ __forceinline__ float block_route(const float l[4], int n_expert, int
 #pragma unroll
     for (int i = 0; i < NW; i++) sum += sh.redf[NW + i];
     unsigned long long key[4];
+    unsigned largest = 0;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int e = tid + k * THREADS;
         v[k] = v[k] / sum;
         key[k] = (k < K && e < n_expert) ? route_key(v[k], e) : 0ull;
-        if (k < K) sh.keys[e] = key[k];
+        largest = max(largest, (unsigned)(key[k] >> 32));
     }
+    top_begin(sh.top, largest);
     __syncthreads();
-    if (K == 1) wave_rank_one(sh.keys + (tid & ~63), key[0], n_used, sh.cand + wave * 16);
-    else wave_rank_many<THREADS>(sh.keys, key[0], key[1], key[2], key[3], K, n_used, sh.cand + wave * 16);
-    __syncthreads();
-    {
-        // four threads per candidate slot, a quarter of the slots each
-        const int c = tid >> 2, part = tid & 3;
-        const unsigned long long me = sh.cand[c];
-        int cnt = 0;
-#pragma unroll
-        for (int c2 = 0; c2 < NW * 2; c2++) {
-            const ulonglong2 q = ((const ulonglong2*)sh.cand)[c2 * 4 + part];  // the four threads of a slot read neighbouring 16-byte pieces: no bank is hit twice
-            cnt += q.x > me ? 1 : 0;
-            cnt += q.y > me ? 1 : 0;
-        }
-        cnt += __shfl_xor(cnt, 1, 64);
-        cnt += __shfl_xor(cnt, 2, 64);
-        if (part == 0 && me != 0ull && cnt < n_used) {
-            ids[cnt] = (int)~(unsigned)(me & 0xffffffffull);
-            wts[cnt] = __uint_as_float((unsigned)(me >> 32));
-        }
-    }
+    top_pick(sh.top, key, K, n_used, [&](int rank, unsigned long long pick) {
+        ids[rank] = (int)~(unsigned)(pick & 0xffffffffull);
+        wts[rank] = __uint_as_float((unsigned)(pick >> 32));
+    });
     __syncthreads();
     float s = 0.0f;
 #pragma unroll

@@ -768,7 +768,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
     __shared__ float coef[16];
     __shared__ int dead;
     __shared__ float fpart[2 * CW];   // partial dots of rows shared by the waves (RF)
-    float* const xf = RF ? (float*)route_sh.keys : nullptr;   // the normed f32 vector of stages A and D (the route's keys come later)
+    float* const xf = RF ? (float*)route_sh.top.cand : nullptr;   // the normed f32 vector of stages A and D (the route's candidates come later)
     const int tid0 = threadIdx.x, b0 = blockIdx.x;
     const Ctl ctl{p.abort_flag, p.spin_limit};
     const unsigned e0 = *(const volatile unsigned*)p.epoch;
@@ -1186,9 +1186,8 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             uint32_t w0 = 0;
             bool ok = ll_wait1(p.ll + RD + tid, e, ctl, &w0);
             const float my_logit = __uint_as_float(w0);
-            const u64 my_key = ((u64)logit_order(my_logit) << 32) | (u64)(~(unsigned)tid);   // larger = earlier pick, unique
-            route_sh.keys[tid] = my_key;
-            if (tid < (CT / 64) * 16) route_sh.cand[tid] = 0ull;
+            const u64 my_key[1] = {((u64)logit_order(my_logit) << 32) | (u64)(~(unsigned)tid)};   // larger = earlier pick, unique
+            top_begin(route_sh.top, (unsigned)(my_key[0] >> 32));
             if (tid == 0) {
                 ok = ok && ll_wait1(p.ll + RD + NE, e, ctl, &w0);
                 sm[34] = __uint_as_float(w0);
@@ -1198,26 +1197,10 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             if (dead) break;
             CH_STAMP(8);
             CH_WSTAMP(0);
-            // (a) a key's rank among the 64 of its wave: only wave ranks below 10 can be among the 10 of the block
-            wave_rank_one(route_sh.keys + (tid & ~63), my_key, NU, route_sh.cand + wave * 16);
-            __syncthreads();
-            {   // (b) the 128 candidate slots against each other: four threads a slot, a quarter of the slots each
-                const int c = tid >> 2, part = tid & 3;
-                const u64 me = route_sh.cand[c];
-                int cnt = 0;
-#pragma unroll
-                for (int c2 = 0; c2 < (CT / 64) * 2; c2++) {
-                    const ulonglong2 q = ((const ulonglong2*)route_sh.cand)[c2 * 4 + part];
-                    cnt += q.x > me ? 1 : 0;
-                    cnt += q.y > me ? 1 : 0;
-                }
-                cnt += __shfl_xor(cnt, 1, 64);
-                cnt += __shfl_xor(cnt, 2, 64);
-                if (part == 0 && me != 0ull && cnt < NU) {
-                    ids[cnt] = (int)~(unsigned)(me & 0xffffffffull);
-                    wts[cnt] = logit_of_order((uint32_t)(me >> 32));   // the pick's logit; its probability follows below
-                }
-            }
+            top_pick(route_sh.top, my_key, 1, NU, [&](int rank, u64 pick) {
+                ids[rank] = (int)~(unsigned)(pick & 0xffffffffull);
+                wts[rank] = logit_of_order((uint32_t)(pick >> 32));   // the pick's logit; its probability follows below
+            });
             __syncthreads();
             CH_STAMP(9);
             CH_WSTAMP(1);
