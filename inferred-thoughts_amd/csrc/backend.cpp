@@ -1341,7 +1341,6 @@ it_hip::~it_hip() {
     if (argmax_out) (void)hipFree(argmax_out);
     if (argmax_host) (void)hipHostFree(argmax_host);
     if (home.cells) (void)hipHostFree(home.cells);
-    if (home.arrived) (void)hipFree(home.arrived);
     if (home.stage) (void)hipHostFree(home.stage);
     for (auto& st : id_stage) {
         if (st.host) (void)hipHostFree(st.host);
@@ -2598,31 +2597,36 @@ float* locked_view(float* buf, size_t bytes) {
 }
 }  // namespace
 
-// A read by the host: a kernel behind the pass writes the floats, the chains' abort word and then a sequence number into
-// page-locked memory, and the host watches that number.  Against a copy, a stream synchronisation and a second copy for the
+// A read by the host: the blocks of a kernel behind the pass write the floats and then, each, the chains' abort word and a sequence
+// number into page-locked memory, and the host watches those numbers.  Against a copy, a stream synchronisation and a second copy for the
 // abort word (32 KB: 45 us after the pass's last kernel) the host has the values a few microseconds after it.
 bool it_hip::fetch(Act& a, float* buf, size_t n) {
     constexpr size_t MAX = 1 << 18;   // floats
     if (!n || n > MAX) return false;
     if (!home.cells) {
-        unsigned* p = nullptr;
-        if (hipHostMalloc((void**)&p, 256, hipHostMallocDefault) != hipSuccess || hipMalloc((void**)&home.arrived, 4) != hipSuccess ||
+        unsigned long long* p = nullptr;
+        if (hipHostMalloc((void**)&p, itk::FETCH_CELLS * 8, hipHostMallocDefault) != hipSuccess ||
             hipHostMalloc((void**)&home.stage, MAX * 4, hipHostMallocDefault) != hipSuccess) {
             (void)hipGetLastError();
+            if (p) (void)hipHostFree(p);
             return false;
         }
-        memset(p, 0, 256);
-        fill_zero(home.arrived, 4, stream);
+        memset(p, 0, itk::FETCH_CELLS * 8);
         home.cells = p;
     }
     float* const direct = locked_view(buf, n * sizeof(float));
     float* const to = direct ? direct : home.stage;
     const unsigned seq = ++home.seq;
-    itk::fetch(a.dev, to, (int64_t)n, chain_ran ? chain.abort_flag : nullptr, home.cells + 16, home.arrived, home.cells, seq, stream);
+    const int cells = itk::fetch(a.dev, to, (int64_t)n, chain_ran ? chain.abort_flag : nullptr, home.cells, seq, stream);
     if (!check(hipGetLastError(), "download activation")) return true;
-    volatile unsigned* flag = home.cells;
+    const volatile unsigned long long* const cell = home.cells;
+    int there = 0;
+    auto arrived = [&] {
+        while (there < cells && (unsigned)cell[there] == seq) there++;
+        return there == cells;
+    };
     const uint64_t t0 = now_us();
-    for (uint64_t i = 1; *flag != seq; i++) {
+    for (uint64_t i = 1; !arrived(); i++) {
         __builtin_ia32_pause();
         // a long wait (a prompt's passes): let the runtime do the waiting, and report a fault if there is one
         if ((i & 1023) == 0 && now_us() - t0 > 2000) {
@@ -2631,14 +2635,14 @@ bool it_hip::fetch(Act& a, float* buf, size_t n) {
         }
     }
     std::atomic_thread_fence(std::memory_order_acquire);
-    if (*flag != seq) {
+    if (!arrived()) {
         fail("download activation: the device did not report the end of the pass");
         return true;
     }
     if (!direct) memcpy(buf, to, n * sizeof(float));
     if (chain_ran) {
         chain_ran = false;
-        if (home.cells[16]) chain_gave_up();
+        if (cell[0] >> 32) chain_gave_up();
     }
     return true;
 }

@@ -80,9 +80,8 @@ struct it_hip {
         void stale() { q_valid = s_valid = false; }
     };
     struct Home {
-        unsigned* cells = nullptr;     // page-locked: [0] sequence number, [16] abort word
-        unsigned* arrived = nullptr;   // device: blocks of a fetch that are done
-        float* stage = nullptr;        // page-locked, for host buffers that are not
+        unsigned long long* cells = nullptr;   // page-locked: a block's abort word and sequence number
+        float* stage = nullptr;                // page-locked, for host buffers that are not
         unsigned seq = 0;
     };
     Home home;

@@ -346,21 +346,19 @@ __global__ __launch_bounds__(256) void zero_spans_k(ZeroSpans z) {
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) ((uint4*)sp.p)[i] = make_uint4(0u, 0u, 0u, 0u);
     if (blockIdx.x == 0 && threadIdx.x < (sp.words & 3)) sp.p[quads * 4 + threadIdx.x] = 0u;
 }
-// Floats into page-locked host memory, then (with everything of every block there) the abort word and the sequence number
-// that the host waits for.  `arrived` is zero between launches.
+// Floats into page-locked host memory; a block whose share is there says so in a cell of its own, {abort word, sequence number}, and
+// the host waits for every cell.  Bound by the trips to host memory: one for the floats, whose end the fence waits for, and the
+// cell's.  (One counter of the blocks and one flag put two more trips and an atomic behind them: 4.7 us for 8,192 floats, now 3.8, and the host sees the cells before the kernel has ended.)
 __global__ __launch_bounds__(256) void fetch_k(const float* __restrict__ src, float* __restrict__ dst, int64_t n, const unsigned* abort_word,
-                                               unsigned* abort_to, unsigned* arrived, unsigned* flag, unsigned seq) {
+                                               unsigned long long* cells, unsigned seq) {
+    const unsigned given_up = abort_word && threadIdx.x == 0 ? *(const volatile unsigned*)abort_word : 0u;
     const int64_t quads = n / 4;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += (int64_t)gridDim.x * 256) ((float4*)dst)[i] = ((const float4*)src)[i];
     if (blockIdx.x == 0 && threadIdx.x < (n & 3)) dst[quads * 4 + threadIdx.x] = src[quads * 4 + threadIdx.x];
     __threadfence_system();
     __syncthreads();
-    if (threadIdx.x == 0 && atomicAdd(arrived, 1u) == gridDim.x - 1) {
-        *arrived = 0u;
-        if (abort_word) *(volatile unsigned*)abort_to = *(const volatile unsigned*)abort_word;
-        __threadfence_system();
-        __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    if (threadIdx.x == 0)
+        __hip_atomic_store(cells + blockIdx.x, (unsigned long long)given_up << 32 | seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 __global__ void fill_zero_k(uint32_t* p, int64_t n_words) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n_words;
@@ -464,10 +462,10 @@ void kv_write(uint16_t* slab, int64_t offset, const int* offset_dyn, int64_t off
               int64_t n, hipStream_t s) {
     EW_LAUNCH(kv_write_k, n, slab, offset, offset_dyn, offset_mul, src, n);
 }
-void fetch(const float* src, float* dst, int64_t n, const unsigned* abort_word, unsigned* abort_to, unsigned* arrived, unsigned* flag, unsigned seq,
-           hipStream_t s) {
-    hipLaunchKernelGGL(fetch_k, dim3((unsigned)std::min<int64_t>((n + 2047) / 2048, 64)), dim3(256), 0, s, src, dst, n, abort_word, abort_to, arrived,
-                       flag, seq);
+int fetch(const float* src, float* dst, int64_t n, const unsigned* abort_word, unsigned long long* cells, unsigned seq, hipStream_t s) {
+    const int blocks = (int)std::min<int64_t>((n + 1023) / 1024, FETCH_CELLS);
+    hipLaunchKernelGGL(fetch_k, dim3(blocks), dim3(256), 0, s, src, dst, n, abort_word, cells, seq);
+    return blocks;
 }
 void zero_spans(const ZeroSpan* spans, int n, hipStream_t s) {
     for (int at = 0; at < n; at += ZERO_SPANS) {

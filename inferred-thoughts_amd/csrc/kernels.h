@@ -223,10 +223,10 @@ struct ZeroSpan {
     int64_t words;
 };
 void zero_spans(const ZeroSpan* spans, int n, hipStream_t s);
-// n floats to page-locked host memory (16-byte aligned), *abort_word (may be null) to *abort_to, then `seq` to *flag, all
-// visible to the host in that order; *arrived is zero before and after
-void fetch(const float* src, float* dst, int64_t n, const unsigned* abort_word, unsigned* abort_to, unsigned* arrived, unsigned* flag, unsigned seq,
-           hipStream_t s);
+// n floats to page-locked host memory (16-byte aligned); the first `result` cells (page-locked too) then hold *abort_word (0: none)
+// in their upper and `seq` in their lower half, each once its share of the floats is visible to the host
+constexpr int FETCH_CELLS = 64;
+int fetch(const float* src, float* dst, int64_t n, const unsigned* abort_word, unsigned long long* cells, unsigned seq, hipStream_t s);
 // n <= POKE_MAX host ints to device memory, and (x non-null) the dequantized row `tok` of an embedding table to x, as one
 // small kernel whose argument block carries them (the host array may be reused as soon as the call returns); false: too
 // many, nothing was launched.
