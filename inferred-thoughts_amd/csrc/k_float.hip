@@ -2,6 +2,8 @@
 //
 // Exact mode: the CPU path's serial f32 fold over the row (/root/reference src/ops/naive.rs:843-861).  Fast mode: the
 // same products summed by the f32 matrix instruction, whose inputs, products and sums are f32 as well.
+#include <cstdint>
+
 #include "it_device.h"
 #include "kernels.h"
 #include "it_dot.h"
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(256) void float_gemv_fast_k(FloatMats m, const floa
 // in wave order.  Per 16 k a lane loads one float4 of its row and one of its token for each 16-wide tile and issues four
 // v_mfma_f32_16x16x4_f32 per pair of tiles, instruction j taking element j of both (k = 4 (lane / 16) + j: the same k on
 // both sides, in whatever order).  Operands come straight from L2: no LDS, no barrier in the loop.  513 x 2,048 F32 rows
-// (router + gate logit): 10 us for 23 tokens (9 blocks of a 64 x 64 tile on the vector ALU: 100 us), 146 us for 5,700 (369).
+// (router + gate logit): 9 us for 23 tokens (9 blocks of a 64 x 64 tile on the vector ALU: 100 us), 152 us for 5,700 (369).
 // (Asking for two or four steps at a time, twice buffered, is 10 to 60 % slower: not the latency of a step bounds it but the
 // rate at which loads of sixteen rows' 64 bytes are served.)
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -273,13 +275,27 @@ void run(const FloatMats& m, const float* x, int n_in, int n_tok, float out_scal
     } else if (!exact && vec && n_tok == 1) {
         hipLaunchKernelGGL(float_gemv_fast_k<FMT>, dim3((rows + 3) / 4), dim3(256), 0, s, m, x, n_in, out_scale);
     } else if (!exact && vec && n_in % 16 == 0) {
-        // the largest tile (fewest operand bytes per product) that still gives every SIMD a wave
-        auto waves = [&](int rt, int tt, int kw) {
-            return (int64_t)((rows + 16 * rt - 1) / (16 * rt)) * ((n_tok + 16 * tt - 1) / (16 * tt)) * kw;
-        };
-        if (waves(2, 4, 4) >= 1024) launch_mfma<FMT, 2, 4, 4>(m, x, n_in, n_tok, out_scale, s);
-        else if (waves(2, 2, 4) >= 1024) launch_mfma<FMT, 2, 2, 4>(m, x, n_in, n_tok, out_scale, s);
-        else launch_mfma<FMT, 1, 1, 8>(m, x, n_in, n_tok, out_scale, s);
+        // A CU is served operands at 30 GB/s whatever it holds: the tile that leaves the busiest of 256 CUs the fewest rows to read, its
+        // blocks' times the rows and tokens of a tile (0.28 to 0.30 us each at 2,048 k with eight waves, 0.30 to 0.34 with four).  513 x
+        // 2,048 over 201 / 333 / 512 / 1,024 / 5,700 tokens, the largest tile of 16 x 16, 32 x 32 and 32 x 64 that gives every SIMD a wave:
+        // 17.6, 25.8, 33.1, 48.9, 163 us; so 14.1, 19.1, 28.2, 34.0, 152.
+        struct Tile { int rt, tt; };
+        constexpr Tile tile[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {3, 3}, {3, 4}};
+        int best = 0;
+        int64_t least = INT64_MAX;
+        for (int i = 0; i < 6; i++) {
+            const int r = 16 * tile[i].rt, t = 16 * tile[i].tt;
+            const int64_t blocks = (int64_t)((rows + r - 1) / r) * ((n_tok + t - 1) / t), cost = (blocks + 255) / 256 * (r + t);
+            if (cost < least) least = cost, best = i;
+        }
+        switch (best) {
+            case 0: launch_mfma<FMT, 1, 1, 8>(m, x, n_in, n_tok, out_scale, s); break;
+            case 1: launch_mfma<FMT, 1, 2, 8>(m, x, n_in, n_tok, out_scale, s); break;
+            case 2: launch_mfma<FMT, 2, 2, 8>(m, x, n_in, n_tok, out_scale, s); break;
+            case 3: launch_mfma<FMT, 2, 4, 8>(m, x, n_in, n_tok, out_scale, s); break;
+            case 4: launch_mfma<FMT, 3, 3, 4>(m, x, n_in, n_tok, out_scale, s); break;
+            default: launch_mfma<FMT, 3, 4, 4>(m, x, n_in, n_tok, out_scale, s); break;
+        }
     } else {
         const int64_t total = (int64_t)rows * n_tok;
         hipLaunchKernelGGL(float_any_k<FMT>, dim3((unsigned)((total + 127) / 128)), dim3(128), 0, s, m, x, n_in, n_tok, out_scale);
