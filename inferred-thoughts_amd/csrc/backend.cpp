@@ -2003,15 +2003,16 @@ static bool expert_tiles_pay(uint64_t picks, uint64_t n_expert) { return picks >
 // Fast mode between the per-pair GEMVs and the wide matrix-core tiles, measured on the 512-expert top-10 FFN (hidden
 // 2048, inter 512).  NVFP4 runs 16-pair tiles on the f16 matrix cores (k_gemm_f16s.hip): level with the per-pair kernels at
 // 40 pairs (four tokens: 307 against 314 us for two layers' whole pass), ahead behind (40 tokens: 574 against 699, 63: 664
-// against 893; up to 32 tokens the FFN is two launches of its own, fuser.cpp), up to 48 pairs per expert (2,048 tokens: 961
-// against 1,017 us for the whole FFN; 4,096 tokens: 1,571 against 1,447), where the 128-pair tiles take over.  What that kernel
+// against 893; up to 32 tokens the FFN is two launches of its own, fuser.cpp), up to 36 pairs per expert, where the 128-pair tiles
+// take over (a prompt's pass through two layers, 1,600 / 1,800 / 2,000 / 2,300 tokens: 2,037, 2,222, 2,366, 2,751 us on the 16-pair tiles,
+// 2,126, 2,222, 2,312, 2,630 on the wide ones).  What that kernel
 // does not take (Q8_0, odd shapes) streams each expert's rows once for all its pairs (k_moe_rows.hip) from 1.25 pairs per
 // expert on, until the int8 tiles pay.
 static bool expert_grouping_pays(const it_hip* be, uint64_t picks, uint64_t n_expert) {
     return !be->exact && picks >= 32 && 4 * picks >= 5 * n_expert;
 }
 static bool expert_skinny_pay(const it_hip* be, uint64_t picks, uint64_t n_expert) {
-    return !be->exact && picks >= 32 && picks < 48 * n_expert;
+    return !be->exact && picks >= 32 && picks < 36 * n_expert;
 }
 static bool expert_rows_pay(const it_hip* be, uint64_t picks, uint64_t n_expert) {
     return expert_grouping_pays(be, picks, n_expert) && !expert_tiles_pay(picks, n_expert);
