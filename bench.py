@@ -14,6 +14,7 @@ timed on this box's host cores on a bounded sample of the same model.
 import argparse
 import json
 import os
+import re
 import sys
 import time
 from pathlib import Path
@@ -50,6 +51,35 @@ def family_profile():
     return out
 
 
+def short(n):
+    """A kernel's name without its namespaces and arguments."""
+    n = n.replace("itk::(anonymous namespace)::", "").replace("itk::", "").replace("void ", "")
+    return re.sub(r"\(.*", "", n)
+
+
+# the kernels of a fast-mode decode graph by how their names begin, and the family that their launches are filed under.  What only
+# a prompt's passes launch has none: a counter run holds the prompt too.
+DECODE_FAMILIES = {
+    "layer_chain_k": "layer_chain (a run of layers, persistent)",
+    "fused_gemv_fast_k": "fused_gemv (norm + quantize + dense GEMVs)",
+    "moe_glu_fast_k": "moe_glu (expert gate+up)",
+    "moe_down_fast_k": "matmul_experts (expert down)",
+    "gdn_rows_fast_k": "gdn_rows (l2 norm + delta rule)",
+    "attend_one_k": "attend",
+    "attend_few_k": "attend",
+    "attend_split_k": "attend",
+    "attend_merge": "attend",
+    "argmax": "other",
+}
+
+
+def decode_family(name, grid):
+    n = short(name)
+    if n.startswith("fused_gemv_fast_k") and grid >= 400000:
+        return "lm_head (norm + GEMV)"
+    return next((f for begin, f in DECODE_FAMILIES.items() if n.startswith(begin)), None)
+
+
 def summarize_profile(root_dir):
     """The text kept under profiles/ for the decode graph, from three rocprofv3 runs of `bench.py --decode-only` whose
     output directories sit under `root_dir`: trace/ (--kernel-trace), pmc_FETCH_SIZE/ and pmc_WRITE_SIZE/ (--pmc, with
@@ -59,35 +89,12 @@ def summarize_profile(root_dir):
     import collections
     import csv
     import glob
-    import re
     steps = 48
-
-    def short(n):
-        n = n.replace("itk::(anonymous namespace)::", "").replace("itk::", "").replace("void ", "")
-        return re.sub(r"\(.*", "", n)
 
     def grid_of(r):
         if "Grid_Size" in r:
             return int(r["Grid_Size"])
         return int(r["Grid_Size_X"]) * int(r.get("Grid_Size_Y", 1) or 1) * int(r.get("Grid_Size_Z", 1) or 1)
-
-    def family(name, grid):
-        n = short(name)
-        if n.startswith("layer_chain_k"):
-            return "layer_chain (a run of layers, persistent)"
-        if n.startswith("fused_gemv_fast_k"):
-            return "lm_head (norm + GEMV)" if grid >= 400000 else "fused_gemv (norm + quantize + dense GEMVs)"
-        if n.startswith("moe_glu_fast_k"):
-            return "moe_glu (expert gate+up)"
-        if n.startswith("moe_down_fast_k"):
-            return "matmul_experts (expert down)"
-        if n.startswith("gdn_rows_fast_k"):
-            return "gdn_rows (l2 norm + delta rule)"
-        if n.startswith("attend_decode_k") or n.startswith("attend_merge"):
-            return "attend"
-        if n.startswith("argmax"):
-            return "other"
-        return None
 
     trace = glob.glob(f"{root_dir}/trace/**/*kernel_trace.csv", recursive=True)[0]
     rows = []
@@ -96,7 +103,7 @@ def summarize_profile(root_dir):
             rows.append((int(r["Start_Timestamp"]), int(r["End_Timestamp"]), r["Kernel_Name"], grid_of(r)))
     rows.sort()
     # whole tokens: from just after one output-head launch to the next; the last `steps` of them
-    heads = [i for i, r in enumerate(rows) if family(r[2], r[3]) == "lm_head (norm + GEMV)"]
+    heads = [i for i, r in enumerate(rows) if decode_family(r[2], r[3]) == "lm_head (norm + GEMV)"]
     tail = rows[heads[-steps - 1] + 1:heads[-1] + 1]
     nodes = len(tail) // steps
     fam = collections.defaultdict(lambda: [0, 0.0])
@@ -104,8 +111,8 @@ def summarize_profile(root_dir):
     gaps = 0.0
     for i, (s0, e0, n, g) in enumerate(tail):
         d = (e0 - s0) / 1e3
-        fam[family(n, g)][0] += 1
-        fam[family(n, g)][1] += d
+        fam[decode_family(n, g)][0] += 1
+        fam[decode_family(n, g)][1] += d
         k = kern[(short(n), g)]
         k[0] += 1
         k[1] += d
@@ -129,7 +136,7 @@ def summarize_profile(root_dir):
                 continue
             if r["Kernel_Name"].startswith("__amd_rocclr_copyBuffer") and float(r["Counter_Value"]) > 50000:
                 copies.append(float(r["Counter_Value"]))
-            k = family(r["Kernel_Name"], grid_of(r))
+            k = decode_family(r["Kernel_Name"], grid_of(r))
             if k:
                 acc[k][0] += 1
                 acc[k][1] += float(r["Counter_Value"])

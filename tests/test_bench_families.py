@@ -1,0 +1,35 @@
+"""bench.py's view of the kernels: every attention kernel of the decode graph is filed under its family, and no entry of the
+table names a kernel that is gone."""
+import re
+from pathlib import Path
+
+import pytest
+
+import bench
+
+CSRC = Path(__file__).resolve().parent.parent / "inferred-thoughts_amd" / "csrc"
+
+
+def kernels(pattern):
+    """names of the kernels that the sources matching `pattern` define"""
+    return {n for f in CSRC.glob(pattern) for n in re.findall(r"__global__[^;{]*?\bvoid\s+(\w+)\s*\(", f.read_text())}
+
+
+def test_attention_kernels_have_their_family():
+    names = (kernels("k_attn.hip") | kernels("k_attn_decode.hip")) - {"attend_exact_k"}     # (exact mode has no such profile)
+    assert len(names) >= 5, names
+    for n in names:
+        assert bench.decode_family(f"void itk::(anonymous namespace)::{n}<256, 8, true>(itk::AttnArgs, int)", 65536) == "attend", n
+
+
+@pytest.mark.parametrize("begin", sorted(bench.DECODE_FAMILIES))
+def test_every_entry_names_a_kernel(begin):
+    assert any(n.startswith(begin) for n in kernels("*.hip"))
+
+
+def test_the_output_head_is_told_from_the_other_products():
+    name = "void itk::(anonymous namespace)::fused_gemv_fast_k<8, 2, 64, false, false>(itk::FusedGemvP)"
+    assert bench.decode_family(name, 524288).startswith("lm_head")
+    assert bench.decode_family(name, 131072).startswith("fused_gemv")
+    for n in kernels("k_attn_prefill.hip") | {"moe_group_k"}:                               # the prompt's
+        assert bench.decode_family(f"void itk::(anonymous namespace)::{n}<256, 8>(itk::AttnArgs)", 1024) is None, n
