@@ -80,6 +80,16 @@ def decode_family(name, grid):
     return next((f for begin, f in DECODE_FAMILIES.items() if n.startswith(begin)), None)
 
 
+def prefill_instructions(n_tokens, exact):
+    """What matrix instruction the kernels of each family issue in a pass of n_tokens, and the measured ceiling that its rate is
+    held against: one of as many multiply-accumulates a cycle."""
+    # Q8_0 products: 32x32x32 (k_gemm.hip, q8_wide_k), which does as many a cycle as 16x16x64; short batches take 16x16x32
+    dense = ("int8_32x32x32", "int8_16x16x64") if n_tokens >= 512 else ("int8_16x16x32", "int8_16x16x32")
+    experts = ("int8_16x16x32", "int8_16x16x32") if exact else ("f16_32x32x16", "f16_32x32x16")
+    return {"matmul (dense": dense, "moe_glu": experts, "matmul_experts": experts, "delta_rule": ("f32_16x16x4", "f32_16x16x4"),
+            "attend": ("f16_32x32x16", "f16_32x32x16")}
+
+
 def summarize_profile(root_dir):
     """The text kept under profiles/ for the decode graph, from three rocprofv3 runs of `bench.py --decode-only` whose
     output directories sit under `root_dir`: trace/ (--kernel-trace), pmc_FETCH_SIZE/ and pmc_WRITE_SIZE/ (--pmc, with
@@ -424,11 +434,7 @@ def main():
     F16_PEAK = 2500.0
     # this card's own ceilings: back-to-back MFMA instructions with no memory in the loop, in TOP/s (TFLOP/s)
     ceilings = {kind: round(be.mfma_ceiling(kind) / 1e12, 1) for kind in ih.Hip.MFMA_KINDS}
-    # the instruction each family issues
-    family_inst = {"matmul (dense": "int8_16x16x32", "moe_glu": "f16_32x32x16", "matmul_experts": "f16_32x32x16",
-                   "delta_rule": "f32_16x16x4", "attend": "f16_32x32x16"}
-    if args.exact:
-        family_inst.update({"moe_glu": "int8_16x16x32", "matmul_experts": "int8_16x16x32"})
+    family_inst = prefill_instructions(args.prompt, args.exact)
     prefill_kernels = {}
     for r in sorted(prows, key=lambda r: -r["ms"]):
         k = {"launches": r["launches"], "ms": round(r["ms"], 2)}
@@ -464,9 +470,9 @@ def main():
             flops = 2 * pairs * model.n_head * model.head_dim * 3 * n_attn_layers
             k.update(unit="f16 MFMA", tflops=round(flops / sec / 1e12, 1), mfma_frac=round(flops / sec / 1e12 / F16_PEAK, 4))
         rate = k.get("tflops", k.get("tops"))
-        inst = next((v for f, v in family_inst.items() if name.startswith(f)), None)
+        inst, ceiling = next((v for f, v in family_inst.items() if name.startswith(f)), (None, None))
         if rate is not None and inst is not None:
-            k.update(instruction=inst, measured_ceiling=ceilings[inst], frac_of_measured=round(rate / ceilings[inst], 4))
+            k.update(instruction=inst, measured_ceiling=ceilings[ceiling], frac_of_measured=round(rate / ceilings[ceiling], 4))
         prefill_kernels[name] = k
 
     # algorithmic bytes of one decode token (weights once + GDN state r+w + KV read)

@@ -33,3 +33,16 @@ def test_the_output_head_is_told_from_the_other_products():
     assert bench.decode_family(name, 131072).startswith("fused_gemv")
     for n in kernels("k_attn_prefill.hip") | {"moe_group_k"}:                               # the prompt's
         assert bench.decode_family(f"void itk::(anonymous namespace)::{n}<256, 8>(itk::AttnArgs)", 1024) is None, n
+
+
+@pytest.mark.parametrize("n_tokens,exact", [(100, False), (5700, False), (5700, True)])
+def test_a_familys_rate_is_held_against_an_instruction_of_the_same_rate(n_tokens, exact):
+    """The ceiling's instruction does as many multiply-accumulates a cycle as the one that the kernels issue."""
+    per_cycle = {"int8_32x32x32": 1024, "int8_16x16x64": 1024, "int8_16x16x32": 512, "f16_32x32x16": 512, "f16_16x16x32": 512,
+                 "f32_16x16x4": 32}
+    import inferred_hip as ih
+    for family, (issued, ceiling) in bench.prefill_instructions(n_tokens, exact).items():
+        assert ceiling in ih.Hip.MFMA_KINDS
+        assert per_cycle[issued] == per_cycle[ceiling], family
+    wide = bench.prefill_instructions(n_tokens, exact)["matmul (dense"][0] == "int8_32x32x32"
+    assert wide == (n_tokens >= 512)       # (most dense rows of a pass of 512 tokens go through k_gemm.hip's 32x32x32 products)
