@@ -26,6 +26,7 @@
 
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_launch.h"
 #include "it_reduce.h"
 #include "kernels.h"
 
@@ -668,13 +669,6 @@ __global__ __launch_bounds__(256) void attend_merge_wide_k(const float* __restri
     }
 }
 
-template <typename Kernel>
-bool lds_of(Kernel kernel, int bytes) {
-    if (bytes <= 64 * 1024 || hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) == hipSuccess) return true;
-    (void)hipGetLastError();
-    return false;
-}
-
 template <int HD, int G>
 bool launch(const AttnArgs& a, const TilePrepP* prep, int n_split, float* part, float* out, const float* gate, int gate_stride, hipStream_t s) {
     const int direct = !((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v)) & 15) && a.kv_dim < (1 << 20);   // (offsets of 24 bits)
@@ -689,16 +683,13 @@ bool launch(const AttnArgs& a, const TilePrepP* prep, int n_split, float* part, 
     const Result res{part, n_split == 1 ? out : nullptr, gate, gate_stride, n_split, kpb};
     const dim3 grid(a.n_head_kv, n_split, groups), block(256);
     if (a.n_q > 1) {
-        static const bool ok = lds_of(attend_few_k<HD, G>, few_lds<HD>());
-        if (!ok) return false;
+        if (!lds_allowed<&attend_few_k<HD, G>>(few_lds<HD>())) return false;
         hipLaunchKernelGGL((attend_few_k<HD, G>), grid, dim3(256 * few_waves<HD>()), few_lds<HD>(), s, a, direct, res);
     } else if (prep) {
-        static const bool ok = lds_of(attend_one_k<HD, G, true>, one_lds<HD>());
-        if (!ok) return false;
+        if (!lds_allowed<&attend_one_k<HD, G, true>>(one_lds<HD>())) return false;
         hipLaunchKernelGGL((attend_one_k<HD, G, true>), grid, block, one_lds<HD>(), s, a, *prep, direct, res);
     } else {
-        static const bool ok = lds_of(attend_one_k<HD, G, false>, one_lds<HD>());
-        if (!ok) return false;
+        if (!lds_allowed<&attend_one_k<HD, G, false>>(one_lds<HD>())) return false;
         hipLaunchKernelGGL((attend_one_k<HD, G, false>), grid, block, one_lds<HD>(), s, a, TilePrepP{}, direct, res);
     }
     if (n_split == 1) return true;

@@ -26,6 +26,7 @@
 // for A and for B; it receives D for column l % 32 and rows 8 * (i / 4) + 4 * (l / 32) + i % 4.
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_launch.h"
 #include "kernels.h"
 
 #include <algorithm>
@@ -334,15 +335,7 @@ template <int HD, int G>
 bool launch_prefill(const AttnArgs& a, int n_split, float* part, float* out, hipStream_t s) {
     constexpr int QT = 128 / G;
     const size_t lds = (size_t)4 * KT * HD * sizeof(uint16_t);   // two tiles of K, two of V
-    static bool sized = false;
-    if (!sized) {
-        if (lds > 64 * 1024 &&
-            hipFuncSetAttribute((const void*)attend_prefill_k<HD, G>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        sized = true;
-    }
+    if (!lds_allowed<&attend_prefill_k<HD, G>>(lds)) return false;
     hipLaunchKernelGGL((attend_prefill_k<HD, G>), dim3((a.n_q + QT - 1) / QT, a.n_head_kv, n_split), dim3(256), lds, s, a, out,
                        n_split > 1 ? part : nullptr);
     if (n_split > 1) {

@@ -46,6 +46,7 @@
 #include <cstring>
 #define IT_CHAIN_DEVICE_POINTERS
 #include "it_fast.h"
+#include "it_launch.h"
 #include "kernels_fused.h"
 
 namespace itk {
@@ -1500,22 +1501,25 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
 
 }  // namespace
 
+// (with the LDS an attention mixer's stages take: every instance is launched with it when a layer is one)
+template <int SF, int RF, int NL>
+static bool instance_fits() {
+    int occ = 0;
+    return lds_allowed<&layer_chain_k<SF, RF, NL>>(ATTN_LDS) &&
+           hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, (const void*)layer_chain_k<SF, RF, NL>, CT, ATTN_LDS) == hipSuccess && occ >= 1;
+}
+
 bool layer_chain_fits() {
-    static const bool fits = [] {
-        int dev = 0, cus = 0, occ = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return false;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < NB) return false;
-        const void* fns[8] = {(const void*)layer_chain_k<W_Q8_0, 0, CHAIN_MAX_LAYERS>,    (const void*)layer_chain_k<W_NVFP4, 0, CHAIN_MAX_LAYERS>,
-                              (const void*)layer_chain_k<W_Q8_0, 1, CHAIN_MAX_LAYERS>,    (const void*)layer_chain_k<W_NVFP4, 1, CHAIN_MAX_LAYERS>,
-                              (const void*)layer_chain_k<W_Q8_0, 0, CHAIN_SHORT_LAYERS>,  (const void*)layer_chain_k<W_NVFP4, 0, CHAIN_SHORT_LAYERS>,
-                              (const void*)layer_chain_k<W_Q8_0, 1, CHAIN_SHORT_LAYERS>,  (const void*)layer_chain_k<W_NVFP4, 1, CHAIN_SHORT_LAYERS>};
-        // (with the LDS an attention mixer's stages take: every instance is launched with it when a layer is one)
-        for (const void* fn : fns)
-            if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, ATTN_LDS) != hipSuccess ||
-                hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, CT, ATTN_LDS) != hipSuccess || occ < 1)
-                return false;
-        return true;
-    }();
+    static std::atomic<int> known[64];   // of each device: 0 not asked, 1 yes, -1 no
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+    if (const int k = known[dev].load(std::memory_order_acquire)) return k > 0;
+    const bool fits = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus >= NB &&
+                      instance_fits<W_Q8_0, 0, CHAIN_MAX_LAYERS>() && instance_fits<W_NVFP4, 0, CHAIN_MAX_LAYERS>() &&
+                      instance_fits<W_Q8_0, 1, CHAIN_MAX_LAYERS>() && instance_fits<W_NVFP4, 1, CHAIN_MAX_LAYERS>() &&
+                      instance_fits<W_Q8_0, 0, CHAIN_SHORT_LAYERS>() && instance_fits<W_NVFP4, 0, CHAIN_SHORT_LAYERS>() &&
+                      instance_fits<W_Q8_0, 1, CHAIN_SHORT_LAYERS>() && instance_fits<W_NVFP4, 1, CHAIN_SHORT_LAYERS>();
+    known[dev].store(fits ? 1 : -1, std::memory_order_release);
     return fits;
 }
 

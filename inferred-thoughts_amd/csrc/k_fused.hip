@@ -16,6 +16,7 @@
 #include <algorithm>
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_launch.h"
 #include "it_reduce.h"
 #include "kernels.h"
 #include "kernels_fused.h"
@@ -647,13 +648,13 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
     const int blocks = std::max(1, p.q_blocks + f_blocks);
     const size_t lds = std::max(nq ? q_lds(R) : base, base + (size_t)f_waves * p.n_in * 4);
     auto launch = [&](auto kernel) {
-        if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, FG_LDS_MAX) != hipSuccess) (void)hipGetLastError();
-        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(FG_THREADS), lds, s, p);
+        if (lds > 64 * 1024) (void)lds_allowed<decltype(kernel)::value>(FG_LDS_MAX);   // (refused: the launch reports it)
+        hipLaunchKernelGGL(decltype(kernel)::value, dim3(blocks), dim3(FG_THREADS), lds, s, p);
     };
-    if (p.n_in <= 4 * FG_THREADS) launch(fused_gemv_k<1>);
-    else if (p.n_in <= 8 * FG_THREADS) launch(fused_gemv_k<2>);
-    else if (p.n_in <= 16 * FG_THREADS) launch(fused_gemv_k<4>);
-    else launch(fused_gemv_k<10>);   // (FG_LDS_MAX holds no more)
+    if (p.n_in <= 4 * FG_THREADS) launch(KernelIs<&fused_gemv_k<1>>{});
+    else if (p.n_in <= 8 * FG_THREADS) launch(KernelIs<&fused_gemv_k<2>>{});
+    else if (p.n_in <= 16 * FG_THREADS) launch(KernelIs<&fused_gemv_k<4>>{});
+    else launch(KernelIs<&fused_gemv_k<10>>{});   // (FG_LDS_MAX holds no more)
 }
 static_assert(FG_LDS_MAX / 7 <= 10 * 4 * FG_THREADS, "an activation that LDS holds fits the registers");
 // F32 rows beside (or in place of) quantized ones, in the kernel that keeps the CPU path's order

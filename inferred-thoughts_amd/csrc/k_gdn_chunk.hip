@@ -14,6 +14,7 @@
 //
 // The sums are not in the CPU path's order: fast mode only; results agree to ~1e-5.
 #include "it_device.h"
+#include "it_launch.h"
 #include "kernels.h"
 
 // Phase stamps for tuning: a build with -DIT_STAMPS records the 100 MHz wall clock of one block's
@@ -415,15 +416,7 @@ static bool launch_chunked(const DeltaArgs& d, float* state, float* out, float* 
     constexpr int LS = DK + 4;
     const size_t prep_lds = (2 * GC * LS + 2 * GC) * sizeof(float);
     const size_t scan_lds = (2 * GC * LS + 2 * GC * TS + DVS * LS + GC * DVS + 2 * GC * US + 4 * GC) * sizeof(float);
-    static bool sized = false;
-    if (!sized) {
-        if (hipFuncSetAttribute((const void*)gdn_chunk_prep_k<DK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)prep_lds) != hipSuccess ||
-            hipFuncSetAttribute((const void*)gdn_chunk_scan_k<DK>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds) != hipSuccess) {
-            (void)hipGetLastError();
-            return false;
-        }
-        sized = true;
-    }
+    if (!lds_allowed<&gdn_chunk_prep_k<DK>>(prep_lds) || !lds_allowed<&gdn_chunk_scan_k<DK>>(scan_lds)) return false;
     const int n_chunks = (d.n_tokens + GC - 1) / GC;
     hipLaunchKernelGGL(gdn_chunk_prep_k<DK>, dim3(n_chunks, d.n_v_heads), dim3(256), prep_lds, s, d, work, q_scale);
     const int items = d.n_v_heads * (d.head_v_dim / DVS);

@@ -15,6 +15,7 @@
 
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_launch.h"
 #include "kernels.h"
 
 namespace itk {
@@ -456,21 +457,20 @@ bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, 
     const bool slabs = w.n_in % 256 == 0 && !((reinterpret_cast<uintptr_t>(ws) | reinterpret_cast<uintptr_t>(act_scales) | reinterpret_cast<uintptr_t>(out)) & 15);
     if (slabs) {
         auto launch = [&](auto kernel, int rows, int toks, size_t lds) {
-            if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
-                (void)hipGetLastError();
-                return false;
-            }
-            hipLaunchKernelGGL(kernel, dim3((w.n_out + rows - 1) / rows, (n_tok + toks - 1) / toks), dim3(256), lds, s, wq, ws, act_quants, act_scales,
+            if (!lds_allowed<decltype(kernel)::value>(lds)) return false;
+            hipLaunchKernelGGL(decltype(kernel)::value, dim3((w.n_out + rows - 1) / rows, (n_tok + toks - 1) / toks), dim3(256), lds, s, wq, ws, act_quants, act_scales,
                                out, w.n_in, w.n_out, n_tok, out_scale);
             return true;
         };
         auto tile = [&](auto nt) {
             constexpr int NT = decltype(nt)::value;
-            return launch(fma ? q8_tile_k<NT, true> : q8_tile_k<NT, false>, 64, 16 * NT, 2 * tile_stage_bytes<NT>());
+            constexpr size_t lds = 2 * tile_stage_bytes<NT>();
+            return fma ? launch(KernelIs<&q8_tile_k<NT, true>>{}, 64, 16 * NT, lds) : launch(KernelIs<&q8_tile_k<NT, false>>{}, 64, 16 * NT, lds);
         };
         auto wide = [&](auto tt) {
             constexpr int TT = decltype(tt)::value;
-            return launch(fma ? q8_wide_k<TT, true> : q8_wide_k<TT, false>, WIDE_ROWS, 32 * TT, 2 * wide_stage_bytes<TT>());
+            constexpr size_t lds = 2 * wide_stage_bytes<TT>();
+            return fma ? launch(KernelIs<&q8_wide_k<TT, true>>{}, WIDE_ROWS, 32 * TT, lds) : launch(KernelIs<&q8_wide_k<TT, false>>{}, WIDE_ROWS, 32 * TT, lds);
         };
         using std::integral_constant;
         // 64 rows x 16 tokens a block up to 640 of them (2.5 a CU).  Above, the shape that takes least by the blocks a CU gets, b, from

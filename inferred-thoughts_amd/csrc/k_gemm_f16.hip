@@ -24,6 +24,7 @@
 // rows 8 * (i / 4) + 4 * (l / 32) + i % 4, i = 0..15.
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_launch.h"
 #include "kernels.h"
 
 // Phase stamps for tuning: a build with -DIT_STAMPS records the 100 MHz wall clock of one block's first
@@ -385,15 +386,8 @@ bool experts_f16_takes(const ExpertsView& w, const ExpertsView* up, int n_picks,
     if (up && (up->fmt != w.fmt || up->n_in != w.n_in || up->n_out != w.n_out || (reinterpret_cast<uintptr_t>(up->q) & 15) ||
                (reinterpret_cast<uintptr_t>(up->scales) & 15) || up->q_stride != w.q_stride || up->s_stride != w.s_stride))
         return false;
-    static int sized = 0;   // 0 unknown, 1 yes, -1 the LDS size was refused
-    if (!sized) {
-        const size_t lds = (size_t)4 * FPAIRS * FBS * sizeof(uint16_t) + (size_t)2 * 256 * (FWS + 16);
-        sized = hipFuncSetAttribute((const void*)experts_f16_k<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess &&
-                        hipFuncSetAttribute((const void*)experts_f16_k<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) == hipSuccess
-                    ? 1 : -1;
-        if (sized < 0) (void)hipGetLastError();
-    }
-    return sized > 0;
+    const size_t lds = (size_t)4 * FPAIRS * FBS * sizeof(uint16_t) + (size_t)2 * 256 * (FWS + 16);
+    return lds_allowed<&experts_f16_k<true>>(lds) && lds_allowed<&experts_f16_k<false>>(lds);
 }
 
 bool experts_gemm_f16(const ExpertsView& w, const ExpertsView* up, const int32_t* ids, int n_picks, int n_used,
