@@ -103,7 +103,7 @@ void it_hip::dyn_upload() {
 namespace {
 // The launches of a recorded pass in their order, if they are a single row of kernels and no more than FEW; else none.
 std::vector<hipKernelNodeParams> few_launches(hipGraph_t g) {
-    constexpr size_t FEW = 8;
+    constexpr size_t FEW = 10;
     std::vector<hipKernelNodeParams> out;
     size_t n = 0, n_root = 1;
     hipGraphNode_t node = nullptr;
@@ -295,10 +295,11 @@ void it_hip::finish_pass() {
     pending.clear();
 }
 
-// A recorded pass goes out as one graph, or, where it is a handful of kernels (the chained layers, the head), as those launches:
-// they follow on the kernel before them and are followed without the 5 and 8 us that the device puts around a graph (a token
-// through two chained layers and the head, read by the host: 96 us as a graph, 89 so; a pass of 27 launches of 5 us each is 8 %
-// slower one by one, the host not being ahead of the device).
+// A recorded pass goes out as one graph, or, where it is a handful of kernels (the chained layers, the head; one layer's stages), as
+// those launches: they follow on the kernel before them and are followed without the 5 and 8 us that the device puts around a graph.
+// Host-read and device-fed tokens, as a graph and one by one, us: 2 launches 58.5 and 52.3, 4 launches 51.5 and 44.5, 7 94 and 88, 9
+// 45.5 and 41.5, 10 54.8 and 51.9.  With more the host is no longer ahead of the device: 13 76 and 80, 15 71.5 and 72, 19 103 and
+// 120, 28 136 and 141.
 void it_hip::launch(Graph& g) {
     if (g.few.empty()) check(hipGraphLaunch(g.exec, stream), "hipGraphLaunch");
     for (const hipKernelNodeParams& k : g.few)

@@ -8,7 +8,7 @@ from util import rng
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n_ops", [1, 2, 7, 8, 9, 10, 40])
+@pytest.mark.parametrize("n_ops", [1, 2, 7, 8, 9, 10, 11, 40])
 def test_replays_of_short_and_long_passes(n_ops):
     import inferred_hip as ih
     be = ih.Hip(exact=True)
