@@ -399,7 +399,7 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
     constexpr int SLICE = SL * HD * 2, STAGE = 2 * SLICE, Q_AT = 2 * STAGE;
     static_assert(G <= 8, "");
     extern __shared__ __align__(1024) uint8_t lds[];
-    __shared__ uint16_t own_p[4][FEW - 1][32];   // probabilities of the keys that not every query of the block sees
+    __shared__ float own_s[4][FEW - 1][32];      // scores (log2) of the keys that not every query of the block sees
     __shared__ int own_odd[2][4 * H];                // whether a wave has found an infinity or a NaN among such keys' values (of a slice)
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pw = w & 3, half = w >> 2;                                   // the wave's pair of queries, its share of the dims
@@ -469,7 +469,8 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
         else wait_loads<0>();
         zero_behind<HD>(V + w * NL * 1024, left - RW * w, RW, lane);
         // A masked key's probability is 0, and the matrix cores multiply it: from the values of keys that only the block's later
-        // queries see, infinities and NaN are taken out here and added at the end, to those queries.
+        // queries see, infinities and NaN are taken out here and added at the end, to those queries, with the f32 weight under the
+        // last maximum (such keys lie in up to two slices, the maximum may move between them, and an f16 weight is 0 from 17 nats on).
         const int own = max(0, pos_lo - kb);                               // the slice's first such key
         if (own < SL) {
             bool bad = false;
@@ -550,8 +551,7 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
                     const int d = kb + 8 * (i >> 2) + 4 * g + (i & 3) - pos_lo;
-                    const _Float16 p = pf[i >> 3][i & 7];      // (a bit_cast of a vector's element itself reads the first one)
-                    if (d >= 0 && d < n_block - 1) own_p[pw][d][c] = __builtin_bit_cast(uint16_t, p);
+                    if (d >= 0 && d < n_block - 1) own_s[pw][d][c] = sc[i];
                 }
             }
             const int vk = here(v_key);
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
         for (int d = 0; d < tq; d++) {           // (query tq sees pos_lo + tq keys)
             if (pos_lo + d < k0 || pos_lo + d >= k1) continue;
             const uint16_t* const v = vh + (int64_t)(pos_lo + d) * a.kv_dim + 32 * half * ND + 4 * g;
-            const float p = it_f16_to_f32(own_p[pw][d][c]);
+            const float p = __builtin_amdgcn_exp2f(own_s[pw][d][c] - m);
 #pragma unroll
             for (int dt = 0; dt < ND; dt++)
 #pragma unroll

@@ -88,6 +88,39 @@ def test_an_infinite_value_counts_with_its_own_keys_weight(hip, orc, n_pos, hd, 
         assert close(np.nan_to_num(got, posinf=0), np.nan_to_num(want, posinf=0))
 
 
+@pytest.mark.parametrize("hd,nh,nkv", [(64, 8, 2), (128, 8, 1), (256, 4, 4)])
+# eight queries, whose seven later keys stand in one slice of 32 keys or on both sides of an edge, in one range and in several
+@pytest.mark.parametrize("n_pos", [35, 38, 40, 67, 131, 1031])
+def test_infinite_values_of_later_keys_count_with_their_last_weight(hip, orc, n_pos, hd, nh, nkv):
+    # One of the keys that only later queries see holds infinities, and scores 40 or 200 below or above a key before or behind it: a
+    # weight of 4e-18 is one in f32 (and no f16), one of 1e-87 is not.  A key behind it raises the maximum after it was seen.
+    r = rng(n_pos * 7 + hd)
+    n_q, kv_dim = 8, nkv * hd
+    q = np.zeros((n_q, nh, hd), np.float32)
+    q[..., 0] = 1.0
+    values = r.standard_normal((n_pos, kv_dim)).astype(np.float16)
+    first = n_pos - n_q + 1                                    # the first key that not every query sees
+    for bad in range(first, n_pos):
+        for high in sorted({first, bad - 1, bad, n_pos - 1}):      # the key whose score is above all others'
+            for gap in (40.0, 200.0):
+                k, v = np.full((n_pos, kv_dim), 0, np.float16), values.copy()
+                k[high, ::hd] = gap
+                v[bad, 3::hd], v[bad, 5::hd] = np.inf, -np.inf
+                rows = []
+                for be in (hip, orc):
+                    out = np.zeros(q.size, np.float32)
+                    if be is hip:
+                        hip.drop_mirrors(); hip.begin_pass(n_q)
+                    be.attend(q.reshape(-1), f16_bits(k).reshape(-1), f16_bits(v).reshape(-1), kv_dim, n_pos, hd, nh, nkv, np.float32(1.0), out)
+                    if be is hip:
+                        hip.host_needs(out); hip.end_pass(); hip.raise_if_error()
+                    rows.append(out.reshape(n_q, nh, hd))
+                got, want = rows
+                for kind in (np.isnan, np.isposinf, np.isneginf):
+                    assert np.array_equal(kind(got), kind(want)), (kind.__name__, bad - first, high - first, gap)
+                assert close(np.nan_to_num(got, posinf=0, neginf=0), np.nan_to_num(want, posinf=0, neginf=0)), (bad - first, high - first, gap)
+
+
 @pytest.mark.parametrize("hd,nh,nkv", [(64, 8, 2), (64, 4, 4), (128, 8, 1), (128, 32, 4), (256, 16, 2), (256, 4, 2)])
 # one query to two groups of eight; contexts around a wave's quarter (8), a slice (32), a stage (64, 128) and a round of ranges
 @pytest.mark.parametrize("n_q", [1, 2, 3, 4, 5, 8, 9, 16])
