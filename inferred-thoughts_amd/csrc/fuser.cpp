@@ -158,7 +158,7 @@ bool match_gdn(Plan& pl, size_t i, int exact) {
     a.m[3] = mat_of(mb, 0);
     a.conv_state = (float*)conv.p[0];
     a.conv_w = (const float*)conv.p[2];
-    if ((float_fmt(ma.i[0]) || float_fmt(mb.i[0])) && !(exact ? fused_gemv_exact_takes(a) : fused_gemv_fast_takes(a))) return false;
+    if (!fused_gemv_takes(a)) return false;
 
     GdnCoreP c{};
     c.conv = (const float*)cv;
@@ -188,6 +188,7 @@ bool match_gdn(Plan& pl, size_t i, int exact) {
     b.exact = exact;
     b.n_mats = 1;
     b.m[0] = mat_of(mo, 2, (float*)rms.p[0]);
+    if (!fused_gemv_takes(b)) return false;
 
     pl.take(i, 18);
     {
@@ -239,6 +240,7 @@ bool match_norm_matmuls(Plan& pl, size_t i, int exact) {
     a.exact = exact;
     a.n_mats = (int)n;
     for (size_t j = 0; j < n; j++) a.m[j] = mat_of(o[m0 + j], 0);
+    if (!fused_gemv_takes(a)) return false;
     pl.take(i, m0 + n - i);
     pl.add(i, it_hip::FAM_FUSED_GEMV, gemv_bytes(a), [=](hipStream_t s) { fused_gemv(a, s); });
     return true;
@@ -257,6 +259,7 @@ bool match_matmul_residual(Plan& pl, size_t i, int exact) {
     b.exact = exact;
     b.n_mats = 1;
     b.m[0] = mat_of(m, 2, (float*)add.p[0]);
+    if (!fused_gemv_takes(b)) return false;
     pl.take(i, 3);
     pl.add(i, it_hip::FAM_FUSED_GEMV, gemv_bytes(b), [=](hipStream_t s) { fused_gemv(b, s); });
     return true;
@@ -279,6 +282,7 @@ bool match_final(Plan& pl, size_t i, int exact) {
     a.exact = exact;
     a.n_mats = 1;
     a.m[0] = mat_of(m, 0);
+    if (!fused_gemv_takes(a)) return false;
     pl.take(i, 4);
     pl.add(i, it_hip::FAM_LM_HEAD, gemv_bytes(a), [=](hipStream_t s) { fused_gemv(a, s); });
     return true;
@@ -373,6 +377,7 @@ bool match_attn(Plan& pl, size_t i, int exact) {
     b.exact = exact;
     b.n_mats = 1;
     b.m[0] = mat_of(mo, 2, (float*)rms.p[0]);
+    if (!fused_gemv_takes(a) || !fused_gemv_takes(b)) return false;
 
     pl.take(i, 18);
     pl.be->fused_attn_slots.push_back(slots);
@@ -530,7 +535,7 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
     a.n_used = (int)nu;
     a.route_ids = (int32_t*)rt.p[1];
     a.route_w = (float*)rt.p[2];
-    if ((float_fmt(mr.i[0]) || float_fmt(ml.i[0])) && !(exact ? fused_gemv_exact_takes(a) : fused_gemv_fast_takes(a))) return false;
+    if (!fused_gemv_takes(a)) return false;
 
     MoeGluP g{};
     g.x = (const float*)x;

@@ -241,7 +241,7 @@ __device__ void wave_route(float* probs, int n_expert, int n_used, int exact, in
     else wave_route_n<32>(probs, n_expert, n_used, exact, ids, weights, lane, etab);   // up to ROUTE_MAX_EXPERTS (match_ffn)
 }
 
-constexpr int FG_THREADS = 512, FG_LDS_MAX = 128 * 1024;
+constexpr int FG_THREADS = 512, FG_LDS_MAX = 128 * 1024, FG_MAX_IN = 8 * 64 * 32;
 
 IT_DEV int mat_index(const FusedGemvP& p, int g) {
     int mi = 0;
@@ -588,6 +588,10 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
     }
 }
 
+// LDS of a block: the activation (f32, scales, quants) and the terms of r rows a wave
+static size_t fg_base(int n_in) { return (size_t)n_in * 4 + (size_t)((n_in / 32 + 3) & ~3) * 4 + n_in; }
+static size_t fg_lds(int n_in, int r) { return fg_base(n_in) + (size_t)(FG_THREADS / 64) * r * (n_in / 32 * 2 + 4) * 4; }
+
 void fused_gemv(FusedGemvP p, hipStream_t s) {
     if (fused_gemv_fast(p, s)) return;
     constexpr int W = FG_THREADS / 64;
@@ -628,9 +632,7 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
                 R = r;
                 break;
             }
-    const size_t base = (size_t)p.n_in * 4 + (size_t)((nb + 3) & ~3) * 4 + p.n_in;
-    auto q_lds = [&](int r) { return base + (size_t)W * r * (nb * 2 + 4) * 4; };
-    while (R > 1 && q_lds(R) > 60 * 1024) R /= 2;
+    while (R > 1 && fg_lds(p.n_in, R) > 60 * 1024) R /= 2;
     p.rows_per_wave = R;
     p.terms_stride = R * (nb * 2 + 4);
     int g = 0;
@@ -646,7 +648,7 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
     const int f_blocks = nf ? std::min(p.total_frows, std::max(256 - p.q_blocks, (p.total_frows + W - 1) / W)) : 0;
     const int f_waves = nf ? std::min(W, (p.total_frows + f_blocks - 1) / f_blocks) : 0;
     const int blocks = std::max(1, p.q_blocks + f_blocks);
-    const size_t lds = std::max(nq ? q_lds(R) : base, base + (size_t)f_waves * p.n_in * 4);
+    const size_t lds = std::max(nq ? fg_lds(p.n_in, R) : fg_base(p.n_in), fg_base(p.n_in) + (size_t)f_waves * p.n_in * 4);
     auto launch = [&](auto kernel) {
         if (lds > 64 * 1024) (void)lds_allowed<decltype(kernel)::value>(FG_LDS_MAX);   // (refused: the launch reports it)
         hipLaunchKernelGGL(decltype(kernel)::value, dim3(blocks), dim3(FG_THREADS), lds, s, p);
@@ -654,17 +656,23 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
     if (p.n_in <= 4 * FG_THREADS) launch(KernelIs<&fused_gemv_k<1>>{});
     else if (p.n_in <= 8 * FG_THREADS) launch(KernelIs<&fused_gemv_k<2>>{});
     else if (p.n_in <= 16 * FG_THREADS) launch(KernelIs<&fused_gemv_k<4>>{});
-    else launch(KernelIs<&fused_gemv_k<10>>{});   // (FG_LDS_MAX holds no more)
+    else launch(KernelIs<&fused_gemv_k<8>>{});   // (fused_gemv_takes admits no more)
 }
-static_assert(FG_LDS_MAX / 7 <= 10 * 4 * FG_THREADS, "an activation that LDS holds fits the registers");
 // F32 rows beside (or in place of) quantized ones, in the kernel that keeps the CPU path's order
-bool fused_gemv_exact_takes(const FusedGemvP& p) {
+static bool fused_gemv_exact_takes(const FusedGemvP& p) {
     for (int i = 0; i < p.n_mats; i++) {
         if (p.m[i].fmt == W_Q8_0 || p.m[i].fmt == W_NVFP4) continue;
         if (p.m[i].fmt != W_F32 || p.m[i].epi != 0 || (reinterpret_cast<uintptr_t>(p.m[i].q) & 15)) return false;
     }
-    const int nb = p.n_in / 32;
-    return p.n_in % 256 == 0 && (size_t)p.n_in * 5 + (size_t)((nb + 3) & ~3) * 4 + (size_t)(FG_THREADS / 64) * std::max(p.n_in, 2 * nb + 4) * 4 <= FG_LDS_MAX;
+    return p.n_in % 256 == 0 && p.n_in <= FG_MAX_IN && std::max(fg_lds(p.n_in, 1), fg_base(p.n_in) + (size_t)(FG_THREADS / 64) * p.n_in * 4) <= FG_LDS_MAX;
+}
+// (A wave takes a row's 32-value units at once, eight a lane, and a thread holds its quads of the activation: rows of more than
+// 16,384 values are left to the ops one by one.)
+bool fused_gemv_takes(const FusedGemvP& p) {
+    bool floats = false;
+    for (int i = 0; i < p.n_mats; i++) floats |= p.m[i].fmt != W_Q8_0 && p.m[i].fmt != W_NVFP4;
+    if (floats) return p.exact ? fused_gemv_exact_takes(p) : fused_gemv_fast_takes(p);
+    return p.n_in <= FG_MAX_IN;
 }
 
 // ------------------------------------------------------------------ gdn rows

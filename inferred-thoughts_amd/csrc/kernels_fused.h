@@ -38,9 +38,10 @@ struct FusedGemvP {
     float* route_w;
 };
 void fused_gemv(FusedGemvP p, hipStream_t s);
-// whether the fast (exact) kernel takes p with unquantized matrices in it (formats, shapes, alignment)
+// whether fused_gemv may be launched with p: how long the activation is and, with unquantized matrices in it, formats, shapes, alignment
+bool fused_gemv_takes(const FusedGemvP& p);
+// whether the fast kernel takes p
 bool fused_gemv_fast_takes(const FusedGemvP& p);
-bool fused_gemv_exact_takes(const FusedGemvP& p);
 
 struct GdnCoreP {
     const float* conv;  // [q | k | v] after conv + silu
