@@ -570,8 +570,6 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
         g.route_w_out = (float*)rt.p[2];
     }
 
-    if (exact && sff > 2048) return false;   // a row of the shared down product is one pass of a wave
-
     MoeDownP d{};
     d.g_all = (const float*)g_all;
     d.g_shared = (const float*)e_gate;
@@ -600,6 +598,7 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
         d.counts_down = (uint32_t*)ex.p[7];
         d.tally = tally;
     }
+    if (!moe_fused_takes(g, d)) return false;
 
     pl.take(i, n_ops);
     const uint64_t glu_b = 2 * rows_bytes(g.fmt, (uint64_t)nu * ff, nd) + 2 * rows_bytes(g.sh_fmt, sff, nd) + (uint64_t)nd * 4 +

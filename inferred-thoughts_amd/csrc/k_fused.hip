@@ -1146,26 +1146,33 @@ __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     }
 }
 
+// LDS of a block: the picks' and the shared intermediate's scales and quants, and the terms of r rows a wave (f32 staging shares their place)
+static size_t down_lds(const MoeDownP& p, int r) {
+    const int nb = p.n_in / 32, sh_nb = p.sh_n_in / 32;
+    const int T = std::max(p.fmt == W_NVFP4 ? nb * 2 : nb, p.sh_fmt == W_NVFP4 ? sh_nb * 2 : sh_nb);
+    const size_t total = (size_t)p.n_used * p.n_in + p.sh_n_in;
+    return (size_t)((p.n_used * nb + sh_nb + 3) & ~3) * 4 + ((total + 15) & ~(size_t)15) + std::max((size_t)4 * (p.n_used + 1) * r * (T + 4) * 4, total * 4);
+}
+
 void moe_down_fused(MoeDownP p, hipStream_t s) {
     if (!p.exact && moe_down_fast(p, s)) return;
     const int nb = p.n_in / 32, sh_nb = p.sh_n_in / 32;
-    const int T = (p.fmt == W_NVFP4 ? nb * 2 : nb), shT = (p.sh_fmt == W_NVFP4 ? sh_nb * 2 : sh_nb);
-    const int Tmax = T > shT ? T : shT;
     // a row group per wave over the whole chip (256 blocks of four waves), and what the kernel's registers hold
     int R = 4;
     while (R > 1 && ((p.n_used + 1) * R > 64 || R * sh_nb > 64 || p.n_used * R * nb > 64 * DOWN_ITEMS || (p.n_out + R - 1) / R < 1024)) R /= 2;
-    auto lds_for = [&](int r) {
-        size_t terms = (size_t)4 * (p.n_used + 1) * r * (Tmax + 4) * 4;
-        size_t stage = (size_t)(p.n_used * p.n_in + p.sh_n_in) * 4;  // f32 staging shares the term region
-        return (size_t)((p.n_used * nb + sh_nb + 3) & ~3) * 4 + (size_t)((p.n_used * p.n_in + p.sh_n_in + 15) & ~15) +
-               (terms > stage ? terms : stage);
-    };
-    while (R > 1 && lds_for(R) > 60 * 1024) R /= 2;
+    while (R > 1 && down_lds(p, R) > 60 * 1024) R /= 2;
     p.rows_per_wave = R;
     int groups = (p.n_out + R - 1) / R;
     int blocks = (groups + 3) / 4;
     if (blocks > 512) blocks = 512;
-    hipLaunchKernelGGL(moe_down_fused_k, dim3(blocks), dim3(256), lds_for(R), s, p);
+    hipLaunchKernelGGL(moe_down_fused_k, dim3(blocks), dim3(256), down_lds(p, R), s, p);
+}
+
+// The kernels that keep the CPU path's order take 256 units of a gate / up row and 64 of the shared down row at once, and LDS that
+// need not be asked for.  In fast mode the picks are made by the fast gate / up kernel, so there is no other.
+bool moe_fused_takes(const MoeGluP& g, const MoeDownP& d) {
+    if (g.exact ? g.n_in > 4 * 64 * 32 : !moe_glu_fast(g, nullptr, true)) return false;
+    return (!d.exact && moe_down_fast(d, nullptr, true)) || (d.sh_n_in <= 64 * 32 && down_lds(d, 1) <= 63 * 1024);
 }
 
 // ------------------------------------------------------------------ attention prep

@@ -122,6 +122,8 @@ bool fused_gemv_fast(FusedGemvP p, hipStream_t s);
 // (dry_run: only say whether the shape is taken)
 bool moe_glu_fast(MoeGluP p, hipStream_t s, bool dry_run = false);
 bool moe_down_fast(MoeDownP p, hipStream_t s, bool dry_run = false);
+// whether moe_glu_fused and moe_down_fused may be launched as a pair
+bool moe_fused_takes(const MoeGluP& g, const MoeDownP& d);
 
 // ------------------------------------------------------------------ layer chain (k_chain.hip, fast mode)
 // A run of decode layers as ONE persistent kernel, one block per compute unit: the six dependent launches of a
