@@ -995,7 +995,7 @@ void moe_glu_fused(MoeGluP p, hipStream_t s) {
 // (src/ops/mod.rs:1134-1171 then add_assign), experts ascending, shared last.
 // What bounds it and how it is laid out: as fused_gemv_k.  What a row's end needs (the picks' scales and weights, the gate's
 // logit, the residual stream) is asked for at the start.
-constexpr int DOWN_ITEMS = 8, DOWN_QUADS = 6;   // (quads: of the intermediates, in a thread's registers; longer ones are staged in LDS)
+constexpr int DOWN_LDS_MAX = 159 * 1024, DOWN_ITEMS = 8, DOWN_QUADS = 6;   // (quads: of the intermediates, in a thread's registers; longer ones are staged in LDS)
 __global__ __launch_bounds__(256) void moe_down_fused_k(MoeDownP p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ uint64_t etab[32];
@@ -1165,14 +1165,15 @@ void moe_down_fused(MoeDownP p, hipStream_t s) {
     int groups = (p.n_out + R - 1) / R;
     int blocks = (groups + 3) / 4;
     if (blocks > 512) blocks = 512;
+    (void)lds_allowed<&moe_down_fused_k>(DOWN_LDS_MAX);   // (refused: the launch reports it)
     hipLaunchKernelGGL(moe_down_fused_k, dim3(blocks), dim3(256), down_lds(p, R), s, p);
 }
 
-// The kernels that keep the CPU path's order take 256 units of a gate / up row and 64 of the shared down row at once, and LDS that
-// need not be asked for.  In fast mode the picks are made by the fast gate / up kernel, so there is no other.
+// The kernels that keep the CPU path's order take 256 units of a gate / up row and 64 of the shared down row at once, and
+// intermediates that fit LDS.  In fast mode the picks are made by the fast gate / up kernel, so there is no other.
 bool moe_fused_takes(const MoeGluP& g, const MoeDownP& d) {
     if (g.exact ? g.n_in > 4 * 64 * 32 : !moe_glu_fast(g, nullptr, true)) return false;
-    return (!d.exact && moe_down_fast(d, nullptr, true)) || (d.sh_n_in <= 64 * 32 && down_lds(d, 1) <= 63 * 1024);
+    return (!d.exact && moe_down_fast(d, nullptr, true)) || (d.sh_n_in <= 64 * 32 && down_lds(d, 1) <= DOWN_LDS_MAX);
 }
 
 // ------------------------------------------------------------------ attention prep

@@ -19,7 +19,8 @@ NE = 16
     (True, 512, 256, 2048, 4, True),
     (True, 512, 256, 2112, 4, False),
     (True, 512, 1024, 1024, 10, True),     # 11,264 intermediates: staged in LDS
-    (True, 512, 2048, 512, 8, False),      # 16,896: more LDS than a launch has unasked
+    (True, 512, 3840, 1024, 8, True),      # 31,744: all of it
+    (True, 512, 4096, 512, 8, False),
     (True, 8192, 64, 64, 4, True),         # a gate / up row is 256 units
     (True, 8224, 64, 64, 4, False),
 ])
