@@ -183,7 +183,7 @@ bool match_gdn(Plan& pl, size_t i, int exact) {
     b.gate = (const float*)z;
     b.eps = rh.f[0];
     b.n_in = (int)vdim;
-    b.mode = 3;
+    b.mode = 2;
     b.head_dim = (int)dv;
     b.exact = exact;
     b.n_mats = 1;
@@ -644,7 +644,7 @@ bool chain_mixer(const FusedGemvP& a, const GdnCoreP& c, const FusedGemvP& b, Ch
     else if (f32m(a.m[2], 32, 0) && f32m(a.m[3], 32, 0)) *rf = 1;
     else return false;
     if (c.n_k_heads != 16 || c.n_v_heads != 32 || c.exact) return false;
-    if (b.n_in != 4096 || b.mode != 3 || b.head_dim != 128 || b.n_mats != 1 || !q8(b.m[0], 2048, 2) || b.m[0].out != a.x) return false;
+    if (b.n_in != 4096 || b.mode != 2 || b.head_dim != 128 || b.n_mats != 1 || !q8(b.m[0], 2048, 2) || b.m[0].out != a.x) return false;
     if (c.conv != a.m[0].out || c.alpha != a.m[2].out || c.beta != a.m[3].out || b.gate != a.m[1].out || b.x != c.core) return false;
     for (int i = 0; i < 4; i++)
         if (!al16(a.m[i].q) || (!(*rf && i >= 2) && !al16(a.m[i].s))) return false;

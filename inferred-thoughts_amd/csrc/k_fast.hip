@@ -64,8 +64,8 @@ inline Geo geo_of(int fmt, int n_in) {
 
 // The activation of a fused GEMV, from global f32 to quantized LDS, held in registers in
 // between: thread t owns floats [4t, 4t+4) and [4(t+THREADS), ...).  n_in <= 8 * THREADS.
-//   mode 0: as is; 1: rms_norm(x, norm_w) (naive.rs:633-650); 2: per-head rms_norm gated by
-//   silu(gate) (head_dim / 4 a power of two <= 64, so a head sits inside one wave).
+//   mode 0: as is; 1: rms_norm(x, norm_w) (naive.rs:633-650); 2: per-head rms_norm times the gate, which
+//   its producer has put through silu (head_dim / 4 a power of two <= 64, so a head sits inside one wave).
 // Ends with a block barrier; xq / xs are then complete.
 template <int THREADS>
 __device__ __forceinline__ void stage_activation(const float* x, int n_in, int mode, const float* norm_w, const float* gate, int head_dim,
@@ -101,7 +101,7 @@ __device__ __forceinline__ void stage_activation(const float* x, int n_in, int m
             v[k].z = v[k].z * scale * w[k].z;
             v[k].w = v[k].w * scale * w[k].w;
         }
-    } else if (mode == 2 || mode == 3) {
+    } else if (mode == 2) {
         const int lh = head_dim >> 2;  // lanes per head
 #pragma unroll
         for (int k = 0; k < 2; k++) {
@@ -112,11 +112,10 @@ __device__ __forceinline__ void stage_activation(const float* x, int n_in, int m
                 const float hs = 1.0f / sqrtf((float)(part / (double)head_dim) + eps);
                 const float4 w = ((const float4*)norm_w)[qi & (lh - 1)];
                 const float4 g = ((const float4*)gate)[qi];
-                // mode 3: the producer already stored silu(gate)
-                v[k].x = (mode == 2 ? fx_silu(g.x) : g.x) * (v[k].x * hs * w.x);
-                v[k].y = (mode == 2 ? fx_silu(g.y) : g.y) * (v[k].y * hs * w.y);
-                v[k].z = (mode == 2 ? fx_silu(g.z) : g.z) * (v[k].z * hs * w.z);
-                v[k].w = (mode == 2 ? fx_silu(g.w) : g.w) * (v[k].w * hs * w.w);
+                v[k].x = g.x * (v[k].x * hs * w.x);
+                v[k].y = g.y * (v[k].y * hs * w.y);
+                v[k].z = g.z * (v[k].z * hs * w.z);
+                v[k].w = g.w * (v[k].w * hs * w.w);
             }
         }
     }
@@ -366,7 +365,7 @@ static bool fused_gemv_fast_prepare(FusedGemvP& p, Geo* geo, int* fmt_out, int* 
     if (!g.ok || p.n_in > FT * 8 || p.n_in % 32) return false;
     if (!aligned16(p.x) || !aligned16(p.x_copy) || !aligned16(p.x_copy2)) return false;
     if (p.mode == 1 && !aligned16(p.norm_w)) return false;
-    if (p.mode == 2 || p.mode == 3) {
+    if (p.mode == 2) {
         const int lh = p.head_dim / 4;
         if (p.head_dim % 4 || lh < 1 || lh > 64 || (lh & (lh - 1)) || p.n_in % p.head_dim) return false;
         if (!aligned16(p.norm_w) || !aligned16(p.gate)) return false;

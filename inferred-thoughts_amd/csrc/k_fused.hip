@@ -320,7 +320,6 @@ template <int NQ>
 __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ double red[FG_THREADS / 64 + 1];
-    __shared__ float hscale[64];
     __shared__ uint64_t etab[32];
     constexpr int W = FG_THREADS / 64;
     const int n_in = p.n_in, nb = n_in >> 5;
@@ -340,7 +339,7 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         if (i < n_in) {
             xv[j] = load4(p.x + i);
             if (p.mode == 1) wv[j] = load4(p.norm_w + i);
-            if (p.mode >= 2) {
+            if (p.mode == 2) {
                 wv[j] = load4(p.norm_w + i % p.head_dim);
                 gv[j] = load4(p.gate + i);
             }
@@ -419,79 +418,34 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
             xv[j].z = xv[j].z * scale * wv[j].z;
             xv[j].w = xv[j].w * scale * wv[j].w;
         }
-    } else if (p.mode == 2 || p.mode == 3) {
-        const int hd = p.head_dim, lph = hd / 4;     // lanes of a head
-        const bool by_lanes = lph == 8 || lph == 16 || lph == 32 || lph == 64;
-        if (!by_lanes) {
-            // 8 lanes per head; a head's walk starts at its own place, so that the heads of a wave read different banks
-#pragma unroll
-            for (int j = 0; j < NQ; j++) {
-                const int i = 4 * (tid + FG_THREADS * j);
-                if (i < n_in) *(float4*)(xf + i) = xv[j];
-            }
-            __syncthreads();
-            const int nh = n_in / hd;  // nh <= 64 (checked on the host)
-            for (int h0 = 0; h0 < nh; h0 += FG_THREADS / 8) {
-                const int h = h0 + (tid >> 3), sub = tid & 7, steps = hd / 8;
-                double part = 0.0;
-                if (h < nh)
-                    for (int k = 0; k < steps; k++) {
-                        const float v = xf[h * hd + sub + 8 * ((k + h) % steps)];
-                        part += (double)(v * v);
-                    }
-                part += dpp_f64(part, 0);
-                part += dpp_f64(part, 1);
-                part += dpp_f64(part, 2);
-                if (h < nh && sub == 0) {
-                    float mean;
-                    if (!p.exact) {
-                        mean = (float)over(part, hd);
-                    } else if (!mean_is_certain(part, hd, hd, &mean)) {
-                        part = 0.0;
-                        for (int i = 0; i < hd; i++) part += (double)(xf[h * hd + i] * xf[h * hd + i]);
-                        mean = (float)over(part, hd);
-                    }
-                    hscale[h] = 1.0f / sqrtf(mean + p.eps);
-                }
-            }
-        }
-        __syncthreads();                             // (the table, too)
+    } else if (p.mode == 2) {
+        const int hd = p.head_dim, lph = hd / 4;     // 16 or 32 lanes a head
 #pragma unroll
         for (int j = 0; j < NQ; j++) {
-            float scale;
-            if (by_lanes) {
-                double sum = squares(xv[j]);
-                sum += dpp_f64(sum, 0);
-                sum += dpp_f64(sum, 1);
-                sum += dpp_f64(sum, 2);
-                if (lph >= 16) sum += dpp_f64(sum, 3);
-                if (lph >= 32) sum += __shfl_xor(sum, 16, 64);
-                if (lph >= 64) sum += __shfl_xor(sum, 32, 64);
-                float mean = (float)over(sum, hd);
-                if (p.exact && !mean_is_certain(sum, hd, hd, &mean)) {   // (the same answer in every lane of the head)
-                    sum = 0.0;
-                    for (int l = 0; l < lph; l++) {
-                        const int from = (lane & ~(lph - 1)) + l;
-                        const float a = __shfl(xv[j].x, from, 64), b = __shfl(xv[j].y, from, 64), c = __shfl(xv[j].z, from, 64), d = __shfl(xv[j].w, from, 64);
-                        sum += (double)(a * a);
-                        sum += (double)(b * b);
-                        sum += (double)(c * c);
-                        sum += (double)(d * d);
-                    }
-                    mean = (float)over(sum, hd);
+            double sum = squares(xv[j]);
+            sum += dpp_f64(sum, 0);
+            sum += dpp_f64(sum, 1);
+            sum += dpp_f64(sum, 2);
+            sum += dpp_f64(sum, 3);
+            if (lph == 32) sum += __shfl_xor(sum, 16, 64);
+            float mean = (float)over(sum, hd);
+            if (p.exact && !mean_is_certain(sum, hd, hd, &mean)) {   // (the same answer in every lane of the head)
+                sum = 0.0;
+                for (int l = 0; l < lph; l++) {
+                    const int from = (lane & ~(lph - 1)) + l;
+                    const float a = __shfl(xv[j].x, from, 64), b = __shfl(xv[j].y, from, 64), c = __shfl(xv[j].z, from, 64), d = __shfl(xv[j].w, from, 64);
+                    sum += (double)(a * a);
+                    sum += (double)(b * b);
+                    sum += (double)(c * c);
+                    sum += (double)(d * d);
                 }
-                scale = 1.0f / sqrtf(mean + p.eps);
-            } else {
-                scale = hscale[min(4 * (tid + FG_THREADS * j), n_in - 1) / hd];
+                mean = (float)over(sum, hd);
             }
-            auto gated = [&](float x, float w, float g) __attribute__((always_inline)) {
-                const float core = x * scale * w;
-                return (p.mode == 2 ? it_silu_by(g, etab) : g) * core;
-            };
-            xv[j].x = gated(xv[j].x, wv[j].x, gv[j].x);
-            xv[j].y = gated(xv[j].y, wv[j].y, gv[j].y);
-            xv[j].z = gated(xv[j].z, wv[j].z, gv[j].z);
-            xv[j].w = gated(xv[j].w, wv[j].w, gv[j].w);
+            const float scale = 1.0f / sqrtf(mean + p.eps);
+            xv[j].x = gv[j].x * (xv[j].x * scale * wv[j].x);
+            xv[j].y = gv[j].y * (xv[j].y * scale * wv[j].y);
+            xv[j].z = gv[j].z * (xv[j].z * scale * wv[j].z);
+            xv[j].w = gv[j].w * (xv[j].w * scale * wv[j].w);
         }
     }
 #pragma unroll
@@ -669,6 +623,7 @@ static bool fused_gemv_exact_takes(const FusedGemvP& p) {
 // (A wave takes a row's 32-value units at once, eight a lane, and a thread holds its quads of the activation: rows of more than
 // 16,384 values are left to the ops one by one.)
 bool fused_gemv_takes(const FusedGemvP& p) {
+    if (p.mode == 2 && ((p.head_dim != 64 && p.head_dim != 128) || p.n_in % p.head_dim)) return false;   // (a head is a row of 16 lanes, or two)
     bool floats = false;
     for (int i = 0; i < p.n_mats; i++) floats |= p.m[i].fmt != W_Q8_0 && p.m[i].fmt != W_NVFP4;
     if (floats) return p.exact ? fused_gemv_exact_takes(p) : fused_gemv_fast_takes(p);
