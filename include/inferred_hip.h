@@ -317,6 +317,8 @@ void it_hip_drop_mirrors(it_hip*);
 uint64_t it_hip_launch_count(it_hip*);
 /* decode graphs: captures, replays, fallbacks to eager, kernel launches in the captured graph */
 void it_hip_graph_stats(it_hip*, uint64_t out[4]);
+/* of the replays, those that went out as separate launches (recorded passes of a handful of kernels) */
+uint64_t it_hip_launched_replays(it_hip*);
 /* layer chains (runs of decode layers as one persistent kernel, fast mode; no counterpart in the reference, whose
  * graph keeps one node per kernel: src/ops/cuda/mod.rs:600-647): chain launches in the last fused pass, layers they
  * cover, 1 while chains are enabled for this backend, the bound on a hand-off wait in polls */

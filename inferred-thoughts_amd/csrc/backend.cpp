@@ -305,6 +305,7 @@ void it_hip::launch(Graph& g) {
     for (const hipKernelNodeParams& k : g.few)
         if (!check(hipLaunchKernel(k.func, k.gridDim, k.blockDim, k.kernelParams, k.sharedMemBytes, stream), "kernel launch")) break;
     graph_launches++;
+    if (!g.few.empty()) launched_replays++;
 }
 
 // After a recorded pass was launched: what a later one of the same tag needs to be launched without being recorded again.
@@ -2817,6 +2818,8 @@ void it_hip_graph_stats(it_hip* be, uint64_t out[4]) {
     out[2] = be->graph_aborts;
     out[3] = be->fused_launches;
 }
+
+uint64_t it_hip_launched_replays(it_hip* be) { return be->launched_replays; }
 
 void it_hip_chain_stats(it_hip* be, uint64_t out[4]) {
     out[0] = be->chain_launches;   // persistent-kernel launches in the last fused pass

@@ -297,7 +297,7 @@ struct it_hip {
     std::vector<uint64_t> pass_signature, prev_signature;
     int stable_passes = 0;      // consecutive eager decode passes with the same op sequence
     size_t replay_cursor = 0;
-    uint64_t graph_launches = 0, graph_captures = 0, graph_aborts = 0;
+    uint64_t graph_launches = 0, launched_replays = 0, graph_captures = 0, graph_aborts = 0;
     // work of the pass being captured or replayed, kept so it can run eagerly if the graph path breaks
     // One seam op as the fuser sees it: an id, its device pointers and integer
     // arguments (meaning per op, see the OpId table in backend.cpp), and the launch.

@@ -97,7 +97,7 @@ it_hip_kv_write it_hip_host_wrote it_hip_host_needs it_hip_begin_pass it_hip_end
 it_hip_read_state it_hip_read_kv it_hip_device_report it_hip_reserve_activations it_hip_tier_counters
 it_hip_config_report it_hip_setup_cost it_hip_prefetch_hint it_hip_set_expert_budget
 it_hip_set_expert_host_budget it_hip_set_expert_slots it_hip_set_expert_pool it_hip_expert_stats
-it_hip_clock_pick it_hip_argmax it_hip_embed_argmax it_hip_embed_rows it_hip_tag_pass it_hip_replay_pass it_hip_read_tokens it_hip_sync it_hip_profile_begin it_hip_profile_end it_hip_release it_hip_drop_mirrors it_hip_launch_count it_hip_graph_stats it_hip_chain_stats it_hip_fetch_read_counts it_hip_zero_state it_hip_mfma_ceiling it_model_open
+it_hip_clock_pick it_hip_argmax it_hip_embed_argmax it_hip_embed_rows it_hip_tag_pass it_hip_replay_pass it_hip_read_tokens it_hip_sync it_hip_profile_begin it_hip_profile_end it_hip_release it_hip_drop_mirrors it_hip_launch_count it_hip_graph_stats it_hip_launched_replays it_hip_chain_stats it_hip_fetch_read_counts it_hip_zero_state it_hip_mfma_ceiling it_model_open
 it_model_close it_model_dims it_model_decode_weight_bytes it_model_token_macs it_engine_new it_engine_free it_engine_reset
 it_engine_set_trace it_engine_pos it_engine_state_sizes it_engine_checkpoint it_engine_restore it_engine_rewind it_engine_forward it_engine_prefill it_engine_generate
 it_engine_decode_greedy it_engine_last_error it_engine_ssm_state it_engine_conv_state it_engine_k_slab
@@ -210,6 +210,7 @@ def lib() -> C.CDLL:
         "it_hip_drop_mirrors": (None, [vp]),
         "it_hip_launch_count": (u64, [vp]),
         "it_hip_graph_stats": (None, [vp, vp]),
+        "it_hip_launched_replays": (u64, [vp]),
         "it_hip_chain_stats": (None, [vp, vp]),
         "it_hip_fetch_read_counts": (None, [vp, vp]),
         "it_model_open": (vp, [C.c_char_p, C.c_char_p, C.c_size_t]),
@@ -468,6 +469,10 @@ class Hip:
         v = (c_u64 * 4)()
         self.L.it_hip_graph_stats(self.h, v)
         return {"captures": int(v[0]), "replays": int(v[1]), "aborts": int(v[2]), "graph_kernels": int(v[3])}
+
+    def launched_replays(self) -> int:
+        """Of graph_stats()["replays"], those that went out as separate launches."""
+        return int(self.L.it_hip_launched_replays(self.h))
 
     def chain_stats(self):
         """Layer chains of the last fused pass: persistent-kernel launches, the layers they cover, enabled, wait bound."""

@@ -40,6 +40,7 @@ def test_replays_of_short_and_long_passes(n_ops):
             be.raise_if_error()
         stats = be.graph_stats()
         assert stats["captures"] >= 1 and stats["replays"] >= 3, stats
+        assert be.launched_replays() == (stats["replays"] if n_ops <= 10 else 0), stats
     finally:
         be.take_error()
         be.close()
