@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
 //
 // Bound by the stream of the touched experts' nibbles and the vector work of expanding them, which are about equal.  512 experts,
 // ten a token, gate / up of 512 x 2,048 and down: 201 tokens 127 and 66 us before, 123 and 69 now; 512 tokens 157 and 87, now 141
-// and 79.  Of the 141 the loads alone take 106, the work without the loads 103.
+// and 79 (in a prompt's pass).  Of the 141 the loads alone take 106, the work without the loads 103.
 constexpr int SK_RING = 3;
 // four scale codes, 0x7f (not a number: counts as zero) made zero; and the b-th of them as a factor for fp4x8_to_f16x8 (see e4m3_to_scale)
 IT_DEV uint32_t scale_codes(uint32_t c) {
@@ -234,14 +234,26 @@ __global__ __launch_bounds__(512, 4) void experts_f16k_k(ExpertsF16P p, int per_
     uint8_t* const mine = ring + wave * SK_WAVE_LDS;
     const uint32_t mine_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)mine);
     const uint32_t row_off = (uint32_t)(lane >> 3) * (n_in >> 1) + kw * 128 + (((lane & 7) ^ ((lane >> 4) & 7)) << 4);
-    // the block's share of all tiles' batches, an even one: a run of batches of one tile after the other
-    const int64_t all = (int64_t)n_tiles_of(p, SK_PAIRS) * per_tile;
-    const int unit1 = (int)(all * (blockIdx.x + 1) / gridDim.x);
-    int unit = (int)(all * blockIdx.x / gridDim.x);
+    // The block's share of all tiles' batches, an even one: a run of batches of one tile after the other.  From one and a half tiles a
+    // block on, whole tiles first, one of each gridDim.x: an expert's tiles, side by side in the list, go through its rows at the
+    // same time on blocks of one XCD and take them from each other's cache lines.  (One after the other in a block's run, they had its
+    // rows from memory each time: 512 experts, gate / up and down, 18 / 22 / 30 / 34 pairs an expert: 231 and 124, 272 and 152, 316 and
+    // 177, 361 and 191 us so, now 206 and 122, 229 and 132, 276 and 156, 302 and 171.  At 10 pairs, 1.07 tiles a block, the run: 151
+    // and 89 against 156 and 98.)
+    const int tiles = n_tiles_of(p, SK_PAIRS), blocks = gridDim.x, whole = 2 * tiles >= 3 * blocks ? tiles / blocks : 0;
+    const int place = blocks % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (blocks / 8) + (int)blockIdx.x / 8;
+    const int64_t rest = (int64_t)(tiles - whole * blocks) * per_tile;
+    const int unit1 = whole * blocks * per_tile + (int)(rest * (blockIdx.x + 1) / blocks);
+    int unit = whole * blocks * per_tile + (int)(rest * blockIdx.x / blocks), round = 0;
     bool first_batch = true;
-    while (unit < unit1) {
-    const int tile = unit / per_tile, b0 = unit - tile * per_tile, n_batches = min(per_tile - b0, unit1 - unit);
-    unit += n_batches;
+    while (round < whole || unit < unit1) {
+    int tile = round * blocks + place, b0 = 0, n_batches = per_tile;
+    if (round++ >= whole) {
+        tile = unit / per_tile;
+        b0 = unit - tile * per_tile;
+        n_batches = min(per_tile - b0, unit1 - unit);
+        unit += n_batches;
+    }
     const int4 td = tile_of(p, tile, SK_PAIRS);
     const int64_t e = td.x;
     const int cnt = td.z;

@@ -1,5 +1,5 @@
 """The 16-pair expert tiles whose blocks share all tiles' row batches evenly (k_gemm_f16s.hip, rows of 256, 512, 1,024 or 2,048),
-against the CPU oracle: a share that begins and ends inside a tile, several tiles in one share, fewer batches than blocks, row
+against the CPU oracle: a share that begins and ends inside a tile, several tiles in one share, whole tiles and a rest, fewer batches than blocks, row
 groups that do not fill the last batch, row sets without any row, tiles of one pair and full ones.
 
 Products of weights exact in f16 with activations split into f16 hi and lo: 2^-22 of a factor and the f32 order of at most 2,048
@@ -41,6 +41,8 @@ def worst(a, b, n_rows):
     (33, 33, 2, 16 * 33),   # an odd number of groups over a few dozen tiles
     (300, 96, 8, 256),      # more batches than blocks: shares of a few batches, cut anywhere
     (17, 3, 3, 2048),       # two tiles an expert, the second of one pair
+    (768, 16, 16, 16),      # one batch a tile, 768 tiles for 512 blocks: whole tiles and a rest
+    (2049, 128, 8, 16),     # 1,100: two rounds of whole tiles, of which an expert has several
 ])
 def test_shares_of_the_tiles(hip, orc, n_tok, n_expert, n_used, n_out, n_in):
     import inferred_hip as ih
