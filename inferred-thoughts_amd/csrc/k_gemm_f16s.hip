@@ -234,25 +234,30 @@ __global__ __launch_bounds__(512, 4) void experts_f16k_k(ExpertsF16P p, int per_
     uint8_t* const mine = ring + wave * SK_WAVE_LDS;
     const uint32_t mine_at = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(lptr)mine);
     const uint32_t row_off = (uint32_t)(lane >> 3) * (n_in >> 1) + kw * 128 + (((lane & 7) ^ ((lane >> 4) & 7)) << 4);
-    // The block's share of all tiles' batches, an even one: a run of batches of one tile after the other.  From one and a half tiles a
-    // block on, whole tiles first, one of each gridDim.x: an expert's tiles, side by side in the list, go through its rows at the
+    // The block's share of all tiles' batches, an even one: a run of batches of one tile after the other.  From one and a quarter tiles
+    // a block on, whole tiles as well, one of each gridDim.x: an expert's tiles, side by side in the list, go through its rows at the
     // same time on blocks of one XCD and take them from each other's cache lines.  (One after the other in a block's run, they had its
-    // rows from memory each time: 512 experts, gate / up and down, 18 / 22 / 30 / 34 pairs an expert: 231 and 124, 272 and 152, 316 and
-    // 177, 361 and 191 us so, now 206 and 122, 229 and 132, 276 and 156, 302 and 171.  At 10 pairs, 1.07 tiles a block, the run: 151
-    // and 89 against 156 and 98.)
-    const int tiles = n_tiles_of(p, SK_PAIRS), blocks = gridDim.x, whole = 2 * tiles >= 3 * blocks ? tiles / blocks : 0;
+    // rows from memory each time: 512 experts, gate / up and down, 16 / 20 / 28 / 36 pairs an expert: 197 and 112, 254 and 140, 299 and
+    // 167, 384 and 204 us so, now 181 and 107, 217 and 127, 252 and 143, 305 and 174.  At 8 and 10 pairs, 1.00 and 1.07 tiles a block,
+    // the run alone: 144 and 85, 149 and 90 against 147 and 94, 151 and 94.)
+    const int tiles = n_tiles_of(p, SK_PAIRS), blocks = gridDim.x, whole = 4 * tiles >= 5 * blocks ? tiles / blocks : 0;
     const int place = blocks % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (blocks / 8) + (int)blockIdx.x / 8;
     const int64_t rest = (int64_t)(tiles - whole * blocks) * per_tile;
     const int unit1 = whole * blocks * per_tile + (int)(rest * (blockIdx.x + 1) / blocks);
     int unit = whole * blocks * per_tile + (int)(rest * blockIdx.x / blocks), round = 0;
+    const int first_run = 2 * (int)blockIdx.x >= blocks ? 0 : whole;   // (half of the blocks begin with the run: a CU's two are at different places of their tiles)
     bool first_batch = true;
-    while (round < whole || unit < unit1) {
+    while (true) {
+    const bool run = round >= first_run && unit < unit1;
+    if (!run && round >= whole) break;
     int tile = round * blocks + place, b0 = 0, n_batches = per_tile;
-    if (round++ >= whole) {
+    if (run) {
         tile = unit / per_tile;
         b0 = unit - tile * per_tile;
         n_batches = min(per_tile - b0, unit1 - unit);
         unit += n_batches;
+    } else {
+        round++;
     }
     const int4 td = tile_of(p, tile, SK_PAIRS);
     const int64_t e = td.x;
