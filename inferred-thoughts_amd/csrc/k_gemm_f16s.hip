@@ -240,19 +240,26 @@ __global__ __launch_bounds__(512, 4) void experts_f16k_k(ExpertsF16P p, int per_
     // rows from memory each time: 512 experts, gate / up and down, 16 / 20 / 28 / 36 pairs an expert: 197 and 112, 254 and 140, 299 and
     // 167, 384 and 204 us so, now 181 and 107, 217 and 127, 252 and 143, 305 and 174.  At 8 and 10 pairs, 1.00 and 1.07 tiles a block,
     // the run alone: 144 and 85, 149 and 90 against 147 and 94, 151 and 94.)
-    const int tiles = n_tiles_of(p, SK_PAIRS), blocks = gridDim.x, whole = 4 * tiles >= 5 * blocks ? tiles / blocks : 0;
-    const int place = blocks % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (blocks / 8) + (int)blockIdx.x / 8;
-    const int64_t rest = (int64_t)(tiles - whole * blocks) * per_tile;
-    const int unit1 = whole * blocks * per_tile + (int)(rest * (blockIdx.x + 1) / blocks);
-    int unit = whole * blocks * per_tile + (int)(rest * blockIdx.x / blocks), round = 0;
-    const int first_run = 2 * (int)blockIdx.x >= blocks ? 0 : whole;   // (half of the blocks begin with the run: a CU's two are at different places of their tiles)
+    const unsigned tiles = n_tiles_of(p, SK_PAIRS), blocks = gridDim.x, b = blockIdx.x;
+    const int whole = 4 * tiles >= 5 * blocks ? tiles / blocks : 0;
+    const int place = blocks % 8 ? b : b % 8 * (blocks / 8) + b / 8;
+    const unsigned rest = (tiles - whole * blocks) * per_tile, each = rest / blocks, more = rest - each * blocks;
+    // The batches left over: one for each CU before a second one for any (blocks b and b + 256 of two a CU share one; spread over all
+    // 512 blocks they fell to both or to neither: gate / up and down of 128 experts of 256 x 512 at 10 pairs 27 and 22 us, now 25 and 21,
+    // of 64 of 512 x 2,048 at 16 pairs 46 and 36, now 42 and 33).
+    auto run_at = [&](unsigned i) {
+        const unsigned a = min(more, 256u), over = blocks == 512 ? (min(i, 256u) * a + (max(i, 256u) - 256u) * (more - a)) >> 8 : min(i, more);
+        return (int)(whole * blocks * per_tile + i * each + over);
+    };
+    int unit = run_at(b), round = 0;
+    const int unit1 = run_at(b + 1), first_run = 2 * b >= blocks ? 0 : whole;   // (half of the blocks begin with the run: a CU's two are at different places of their tiles)
     bool first_batch = true;
     while (true) {
     const bool run = round >= first_run && unit < unit1;
     if (!run && round >= whole) break;
     int tile = round * blocks + place, b0 = 0, n_batches = per_tile;
     if (run) {
-        tile = unit / per_tile;
+        tile = (unsigned)unit / (unsigned)per_tile;
         b0 = unit - tile * per_tile;
         n_batches = min(per_tile - b0, unit1 - unit);
         unit += n_batches;
