@@ -2005,16 +2005,20 @@ static bool expert_tiles_pay(uint64_t picks, uint64_t n_expert) { return picks >
 // Fast mode between the per-pair GEMVs and the wide matrix-core tiles, measured on the 512-expert top-10 FFN (hidden
 // 2048, inter 512).  NVFP4 runs 16-pair tiles on the f16 matrix cores (k_gemm_f16s.hip): level with the per-pair kernels at
 // 40 pairs (four tokens: 307 against 314 us for two layers' whole pass), ahead behind (40 tokens: 574 against 699, 63: 664
-// against 893; up to 32 tokens the FFN is two launches of its own, fuser.cpp), up to 36 pairs per expert, where the 128-pair tiles
-// take over (a prompt's pass through two layers, 1,600 / 1,800 / 2,000 / 2,300 tokens: 2,037, 2,222, 2,366, 2,751 us on the 16-pair tiles,
-// 2,126, 2,222, 2,312, 2,630 on the wide ones).  What that kernel
+// against 893; up to 32 tokens the FFN is two launches of its own, fuser.cpp), up to 36 or 48 pairs per expert, where the 128-pair tiles
+// take over.  Both products, us, on the 16-pair tiles and on the wide ones at 36 / 44 / 48 pairs: 512 experts of 512 x 2,048 479, 551, 590
+// and 565, 605, 615; 256 of these 284, 305, 332 and 298, 320, 320; 256 of 256 x 2,048 180, 200, 218 and 181, 191, 204; 512 of 256 x 1,024 209,
+// 235, 254 and 204, 220, 228 (up to 128 experts of 512 x 2,048 the wide ones are ahead from 20 pairs on: 88 against 103 at 36 for 64).  So
+// 48 for many experts of a million weights, and for few small ones, which leave the wide tiles' grid short of blocks (16 of 256 x 512
+// at 36 to 47 pairs 33 against 36, 8 of 1,024 x 2,048 66 against 69 at 36).  What that kernel
 // does not take (Q8_0, odd shapes) streams each expert's rows once for all its pairs (k_moe_rows.hip) from 1.25 pairs per
 // expert on, until the int8 tiles pay.
 static bool expert_grouping_pays(const it_hip* be, uint64_t picks, uint64_t n_expert) {
     return !be->exact && picks >= 32 && 4 * picks >= 5 * n_expert;
 }
-static bool expert_skinny_pay(const it_hip* be, uint64_t picks, uint64_t n_expert) {
-    return !be->exact && picks >= 32 && picks < 36 * n_expert;
+static bool expert_skinny_pay(const it_hip* be, uint64_t picks, const it_experts* w) {
+    const bool far = (w->n_expert > 128 && w->n_in * w->n_out >= 1 << 20) || w->n_expert * std::max(w->n_in, w->n_out) <= 16384;
+    return !be->exact && picks >= 32 && picks < (far ? 48 : 36) * w->n_expert;
 }
 static bool expert_rows_pay(const it_hip* be, uint64_t picks, uint64_t n_expert) {
     return expert_grouping_pays(be, picks, n_expert) && !expert_tiles_pay(picks, n_expert);
@@ -2048,7 +2052,7 @@ void it_hip_matmul_experts(it_hip* be, const it_experts* w, const it_route* rout
     if (!dout) return;
     int np = (int)picks, nu = (int)n_used, xm = x_mode_of(rows, picks);
     size_t work_ints = 0;
-    const bool skinny_pay = expert_skinny_pay(be, picks, w->n_expert) && v.fmt == itk::W_NVFP4;
+    const bool skinny_pay = expert_skinny_pay(be, picks, w) && v.fmt == itk::W_NVFP4;
     const bool rows_pay = !skinny_pay && expert_rows_pay(be, picks, w->n_expert);
     int32_t* work = skinny_pay || rows_pay || expert_tiles_pay(picks, w->n_expert) ? be->moe_work_for(picks, w->n_expert, &work_ints) : nullptr;
     const bool rows_shape = rows_pay && work && itk::expert_rows_takes(v, nullptr, aq);
@@ -2116,7 +2120,7 @@ void it_hip_moe_glu(it_hip* be, const it_experts* gate, const it_experts* up, co
     if (!dout) return;
     int np = (int)picks, nu = (int)n_used, xm = x_mode_of(rows, picks);
     size_t work_ints = 0;
-    const bool skinny_pay = expert_skinny_pay(be, picks, gate->n_expert) && g.fmt == itk::W_NVFP4;
+    const bool skinny_pay = expert_skinny_pay(be, picks, gate) && g.fmt == itk::W_NVFP4;
     const bool rows_pay = !skinny_pay && expert_rows_pay(be, picks, gate->n_expert);
     int32_t* work = skinny_pay || rows_pay || expert_tiles_pay(picks, gate->n_expert) ? be->moe_work_for(picks, gate->n_expert, &work_ints) : nullptr;
     const bool rows_shape = rows_pay && work && itk::expert_rows_takes(g, &u, aq);

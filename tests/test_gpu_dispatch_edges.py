@@ -39,7 +39,7 @@ def fresh(be, n=1):
     be.begin_pass(n)
 
 
-@pytest.mark.parametrize("n_tok,n_expert,n_used", [(7, 16, 4), (8, 16, 4), (191, 16, 4), (192, 16, 4), (33, 512, 1), (63, 512, 10)])
+@pytest.mark.parametrize("n_tok,n_expert,n_used", [(7, 16, 4), (8, 16, 4), (191, 16, 4), (192, 16, 4), (575, 64, 4), (576, 64, 4), (33, 512, 1), (63, 512, 10)])
 def test_expert_tiles_by_pairs(hip, orc, n_tok, n_expert, n_used):
     fast.test_moe_stage_fast_nvfp4(hip, orc, n_tok, n_expert, n_used, 512, 256)
 
