@@ -125,6 +125,7 @@ struct Result {
     const float* gate;
     int gate_stride, n_split;
     int kpb;                     // keys of a range, a multiple of 32 (0: by the context that the device knows)
+    int per;                     // queries of a block, of a few
 };
 // Contexts that stay one range (and need no merge where the host knows them).  One query: 64 KB of K and of V (heads of 256: 6.3 us
 // at 128 keys where a range every 64 keys and the merge take 8.2, 8.9 against 8.2 at 256; of 128: 5.7 against 7.2 at 256, 7.3
@@ -380,7 +381,7 @@ __global__ __launch_bounds__(256, one_blocks<HD>()) void attend_one_k(AttnArgs a
 }
 
 // ------------------------------------------------------------------ a few queries
-// Up to eight queries a block, a pair of them for each of four waves: 32 columns, so 32x32x16 products: lane l supplies 8 k
+// Up to eight queries a block, a pair of them for each of four waves (of two, where the launcher says four): 32 columns, so 32x32x16 products: lane l supplies 8 k
 // values of row (l % 32), k group l / 32, for A and for B, and receives D for column l % 32 and rows 8 * (i / 4) + 4 * (l / 32) + i % 4.
 // Heads of 256 take two waves a pair (H), which form the same scores and half of the sums each: one wave's sums, 128 registers a
 // lane, would stand alone on its SIMD with everything between two trips to LDS exposed.  The waves bring a slice together, two
@@ -399,16 +400,17 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
     constexpr int SLICE = SL * HD * 2, STAGE = 2 * SLICE, Q_AT = 2 * STAGE;
     static_assert(G <= 8, "");
     extern __shared__ __align__(1024) uint8_t lds[];
-    __shared__ float own_s[4][FEW - 1][32];      // scores (log2) of the keys that not every query of the block sees
+    __shared__ float own_s[4][FEW - 1][32];      // scores (log2) of the keys that not every one of eight queries sees
     __shared__ int own_odd[2][4 * H];                // whether a wave has found an infinity or a NaN among such keys' values (of a slice)
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int pw = w & 3, half = w >> 2;                                   // the wave's pair of queries, its share of the dims
     const int c = lane & 31, g = lane >> 5, z = c >> 4;
     const int kvh = blockIdx.x, h0 = kvh * G, split = blockIdx.y;
-    const int t0 = blockIdx.z * FEW, t = t0 + 2 * pw;  // the block's first query, this wave's
+    const int t0 = blockIdx.z * res.per, t = t0 + 2 * pw;  // the block's first query, this wave's
     const int n_pos_last = a.n_pos_dyn ? *a.n_pos_dyn : a.n_pos;
-    const int n_block = min(FEW, a.n_q - t0);                              // queries of the block
+    const int n_block = min(res.per, a.n_q - t0);                              // queries of the block
     const int pos_lo = n_pos_last - a.n_q + 1 + t0, pos_hi = pos_lo + n_block - 1;   // keys that its first and its last one see
+    const int ahead = t0 % FEW, own_lo = pos_lo - ahead;                   // keys that the first of its eight queries sees (of another block, of four)
     const int my_pos = pos_lo + 2 * pw + z;                                 // (columns without a query: more than there are)
     const bool works = 2 * pw < n_block;                                    // waves without queries bring their share only
     const int kpb = keys_of_range(pos_hi, res, FEW_RANGE);
@@ -471,7 +473,7 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
         // A masked key's probability is 0, and the matrix cores multiply it: from the values of keys that only the block's later
         // queries see, infinities and NaN are taken out here and added at the end, to those queries, with the f32 weight under the
         // last maximum (such keys lie in up to two slices, the maximum may move between them, and an f16 weight is 0 from 17 nats on).
-        const int own = max(0, pos_lo - kb);                               // the slice's first such key
+        const int own = max(0, own_lo - kb);                               // the slice's first such key
         if (own < SL) {
             bool bad = false;
 #pragma unroll 1
@@ -550,8 +552,8 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
                 odd_any = true;
 #pragma unroll
                 for (int i = 0; i < 16; i++) {
-                    const int d = kb + 8 * (i >> 2) + 4 * g + (i & 3) - pos_lo;
-                    if (d >= 0 && d < n_block - 1) own_s[pw][d][c] = sc[i];
+                    const int d = kb + 8 * (i >> 2) + 4 * g + (i & 3) - own_lo;
+                    if (d >= 0 && d < ahead + n_block - 1) own_s[pw][d][c] = sc[i];
                 }
             }
             const int vk = here(v_key);
@@ -593,9 +595,9 @@ __global__ __launch_bounds__(256 * few_waves<HD>(), few_blocks<HD>() * few_waves
     const int tq = 2 * pw + z, head = c & 7;
     if ((c & 8) || head >= G || tq >= n_block) return;
     if (odd_any) {
-        for (int d = 0; d < tq; d++) {           // (query tq sees pos_lo + tq keys)
-            if (pos_lo + d < k0 || pos_lo + d >= k1) continue;
-            const uint16_t* const v = vh + (int64_t)(pos_lo + d) * a.kv_dim + 32 * half * ND + 4 * g;
+        for (int d = 0; d < ahead + tq; d++) {   // (query tq sees pos_lo + tq keys)
+            if (own_lo + d < k0 || own_lo + d >= k1) continue;
+            const uint16_t* const v = vh + (int64_t)(own_lo + d) * a.kv_dim + 32 * half * ND + 4 * g;
             const float p = __builtin_amdgcn_exp2f(own_s[pw][d][c] - m);
 #pragma unroll
             for (int dt = 0; dt < ND; dt++)
@@ -672,7 +674,11 @@ __global__ __launch_bounds__(256) void attend_merge_wide_k(const float* __restri
 template <int HD, int G>
 bool launch(const AttnArgs& a, const TilePrepP* prep, int n_split, float* part, float* out, const float* gate, int gate_stride, hipStream_t s) {
     const int direct = !((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v)) & 15) && a.kv_dim < (1 << 20);   // (offsets of 24 bits)
-    const int groups = a.n_q > 1 ? (a.n_q + FEW - 1) / FEW : 1;
+    // Eight queries a block, which read the cache once; four while that leaves one block a CU at most, half of the waves idle but none
+    // waiting for another on its SIMD (16 heads of 256 on 2, eight queries at 48 / 512 / 1,024 / 2,048: 13.2, 16.2, 16.4, 17.5 us with
+    // eight, 11.1, 14.2, 14.9, 16.0 with four; on 4 at 2,048, 256 blocks of four, 16.3 and 15.4, at 5,431 20.2 and 23.2).
+    const int per = a.n_head_kv * n_split * ((a.n_q + 3) / 4) <= DECODE_CUS ? 4 : FEW;
+    const int groups = a.n_q > 1 ? (a.n_q + per - 1) / per : 1;
     // one round of blocks: more of them would leave more results to merge, and have no more bytes in flight
     n_split = std::max(1, std::min(n_split, DECODE_CUS * (a.n_q > 1 ? few_blocks<HD>() : one_blocks<HD>()) / (groups * a.n_head_kv)));
     int kpb = 0;
@@ -680,7 +686,7 @@ bool launch(const AttnArgs& a, const TilePrepP* prep, int n_split, float* part, 
         kpb = keys_over(a.n_pos, n_split, a.n_q > 1 ? FEW_RANGE : one_range<HD>());
         n_split = (a.n_pos + kpb - 1) / kpb;
     }
-    const Result res{part, n_split == 1 ? out : nullptr, gate, gate_stride, n_split, kpb};
+    const Result res{part, n_split == 1 ? out : nullptr, gate, gate_stride, n_split, kpb, per};
     const dim3 grid(a.n_head_kv, n_split, groups), block(256);
     if (a.n_q > 1) {
         if (!lds_allowed<&attend_few_k<HD, G>>(few_lds<HD>())) return false;
