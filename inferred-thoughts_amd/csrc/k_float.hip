@@ -282,17 +282,20 @@ void run(const FloatMats& m, const float* x, int n_in, int n_tok, float out_scal
         struct Tile { int rt, tt; };
         constexpr Tile tile[] = {{1, 1}, {1, 2}, {2, 2}, {2, 4}, {3, 3}, {3, 4}};
         int best = 0;
-        int64_t least = INT64_MAX;
+        int64_t least = INT64_MAX, best_blocks = 0;
         for (int i = 0; i < 6; i++) {
             const int r = 16 * tile[i].rt, t = 16 * tile[i].tt;
             const int64_t blocks = (int64_t)((rows + r - 1) / r) * ((n_tok + t - 1) / t), cost = (blocks + 255) / 256 * (r + t);
-            if (cost < least) least = cost, best = i;
+            if (cost < least) least = cost, best = i, best_blocks = blocks;
         }
         switch (best) {
             case 0: launch_mfma<FMT, 1, 1, 8>(m, x, n_in, n_tok, out_scale, s); break;
             case 1: launch_mfma<FMT, 1, 2, 8>(m, x, n_in, n_tok, out_scale, s); break;
             case 2: launch_mfma<FMT, 2, 2, 8>(m, x, n_in, n_tok, out_scale, s); break;
-            case 3: launch_mfma<FMT, 2, 4, 8>(m, x, n_in, n_tok, out_scale, s); break;
+            case 3:   // (with a second block on a CU four waves do: 129 x 2,048 over 5,700 tokens 64 and 59 us; alone 33 and 38)
+                if (best_blocks > 256) launch_mfma<FMT, 2, 4, 4>(m, x, n_in, n_tok, out_scale, s);
+                else launch_mfma<FMT, 2, 4, 8>(m, x, n_in, n_tok, out_scale, s);
+                break;
             case 4: launch_mfma<FMT, 3, 3, 4>(m, x, n_in, n_tok, out_scale, s); break;
             default: launch_mfma<FMT, 3, 4, 4>(m, x, n_in, n_tok, out_scale, s); break;
         }

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
     (512, 1, 64), (33, 31, 3),          # 16 x 16
     (512, 1, 201), (100, 3, 515),       # 16 x 32
     (513, 2, 333), (95, 64, 1001),      # 32 x 32
-    (512, 1, 512), (33, 30, 5701),      # 32 x 64
+    (512, 1, 512), (33, 30, 5701), (128, 1, 5700),   # 32 x 64, of eight waves and of four
     (512, 1, 1024), (47, 50, 2049),     # 48 x 48
     (512, 1, 3001), (145, 100, 4097),   # 48 x 64
 ])
