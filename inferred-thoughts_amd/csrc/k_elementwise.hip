@@ -349,6 +349,8 @@ __global__ __launch_bounds__(256) void zero_spans_k(ZeroSpans z) {
 // Floats into page-locked host memory; a block whose share is there says so in a cell of its own, {abort word, sequence number}, and
 // the host waits for every cell.  Bound by the trips to host memory: one for the floats, whose end the fence waits for, and the
 // cell's.  (One counter of the blocks and one flag put two more trips and an atomic behind them: 4.7 us for 8,192 floats, now 3.8, and the host sees the cells before the kernel has ended.)
+// The cell's store is a relaxed one: that the floats are there before it is due to every thread's fence, which waits for its own stores
+// to reach the system, and the barrier between the fences and the cell.
 __global__ __launch_bounds__(256) void fetch_k(const float* __restrict__ src, float* __restrict__ dst, int64_t n, const unsigned* abort_word,
                                                unsigned long long* cells, unsigned seq) {
     const unsigned given_up = abort_word && threadIdx.x == 0 ? *(const volatile unsigned*)abort_word : 0u;

@@ -3,7 +3,7 @@
 // The backend's it_hip_attend mirrors host buffers on the device and grows its split-K
 // scratch (the per-split partial sums, maxima and normalisers) with hipMalloc.  Code
 // under HIP graph capture, a tight serving loop or a harness that forbids allocation
-// cannot call it.  This entry point runs the same kernels (attend_decode_k or
+// cannot call it.  This entry point runs the same kernels (attend_one_k, attend_few_k or
 // attend_split_k, then the merge) on operands that are already device resident and keeps
 // the partials in a fixed array inside the code object, so it calls no hipMalloc,
 // hipFree or allocating library routine.

@@ -1,8 +1,8 @@
 """Expert matmuls of a small batch in fast mode against the CPU oracle, through the C ABI.
 
 From 1.25 pairs per expert on, fast mode sorts the (token, pick) pairs by expert.  NVFP4 experts then run tiles of 16
-pairs on the f16 matrix cores (k_gemm_f16s.hip: weights exact in f16, activations as an f16 hi + lo pair) up to 48 pairs
-per expert; Q8_0 experts, and shapes that kernel does not take, stream every touched expert's rows once and multiply by
+pairs on the f16 matrix cores (k_gemm_f16s.hip: weights exact in f16, activations as an f16 hi + lo pair) up to 36 or 48 pairs
+per expert (by the experts' number and size); Q8_0 experts, and shapes that kernel does not take, stream every touched expert's rows once and multiply by
 the integer dots of the CPU path (k_moe_rows.hip) until the int8 tiles pay.  Only the f32 summation order (and the 2^-22
 of the split) differs from the oracle, so the bound is 2e-5 of the row's largest output, fifty times tighter than the
 mode's 1e-3.  Covered: NVFP4 and Q8_0; the gate/up pair with silu and a single matrix; rows of 8 .. 128 units; experts
