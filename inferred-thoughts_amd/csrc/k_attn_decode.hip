@@ -17,10 +17,10 @@
 // What bounds it: short contexts the chain of trips to memory and LDS and the number of instructions a wave issues between
 // them (four cycles each), long ones memory.  So one query's waves share nothing but the query: each walks a quarter of the
 // range with its own slice of K and of V in LDS, asked for again as soon as it has been read, and the four results are added at
-// the end.  With the merge, 16 query heads of 256 on 2 KV heads: 8.3 us at 1,024 positions, 18.1 at 32,000 (3.6 TB/s); five
-// queries at 5,431: 15.7; on 4 KV heads at 31,000: 26.0 (4.9 TB/s); 32 heads of 128 on 4 at 30,000: 16.5.  (10.1, 22.7, 17.0, 37.2
-// and 23.8 with K and V through registers, V turned on its way into LDS, a tile of 64 keys a block at a time, every wave forming
-// the same scores.)
+// the end.  Calls one after another on the same operands, with the merge, 16 query heads of 256 on 2 KV heads: 8.3 us at 1,024
+// positions, 9.2 at 5,800, 15.6 at 32,000 (4.2 TB/s); five queries at 5,431: 15.0; on 4 KV heads at 31,000: 22.8 (5.6 TB/s); 32 heads of
+// 128 on 4 at 30,000: 14.8.  (9.9, 10.3, 21.2, 16.1, 32.7 and 21.5 with K and V through registers, V turned on its way into LDS, a tile
+// of 64 keys a block at a time, every wave forming the same scores.)
 #include <algorithm>
 #include <type_traits>
 
@@ -675,8 +675,9 @@ template <int HD, int G>
 bool launch(const AttnArgs& a, const TilePrepP* prep, int n_split, float* part, float* out, const float* gate, int gate_stride, hipStream_t s) {
     const int direct = !((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v)) & 15) && a.kv_dim < (1 << 20);   // (offsets of 24 bits)
     // Eight queries a block, which read the cache once; four while that leaves one block a CU at most, half of the waves idle but none
-    // waiting for another on its SIMD (16 heads of 256 on 2, eight queries at 48 / 512 / 1,024 / 2,048: 13.2, 16.2, 16.4, 17.5 us with
-    // eight, 11.1, 14.2, 14.9, 16.0 with four; on 4 at 2,048, 256 blocks of four, 16.3 and 15.4, at 5,431 20.2 and 23.2).
+    // waiting for another on its SIMD (16 heads of 256 on 2, eight queries at 48 / 512 / 1,024 / 2,048, each launch between two events:
+    // 13.2, 16.2, 16.4, 17.5 us with eight, 11.1, 14.2, 14.9, 16.0 with four; on 4 at 2,048, 256 blocks of four, 16.3 and 15.4, at 5,431
+    // 20.2 and 23.2).
     const int per = a.n_head_kv * n_split * ((a.n_q + 3) / 4) <= DECODE_CUS ? 4 : FEW;
     const int groups = a.n_q > 1 ? (a.n_q + per - 1) / per : 1;
     // one round of blocks: more of them would leave more results to merge, and have no more bytes in flight

@@ -197,8 +197,9 @@ __global__ __launch_bounds__(256) void experts_f16s_k(ExpertsF16P p, int gpw) {
 // finished by all eight waves (one wave at a time before).
 //
 // Bound by the stream of the touched experts' nibbles and the vector work of expanding them, which are about equal.  512 experts,
-// ten a token, gate / up of 512 x 2,048 and down: 201 tokens 127 and 66 us before, 123 and 69 now; 512 tokens 157 and 87, now 141
-// and 79 (in a prompt's pass).  Of the 141 the loads alone take 106, the work without the loads 103.
+// ten a token, gate / up of 512 x 2,048 and down, each launch between two events: 204 tokens 137 and 81 us before, 133 and 79 now; 512
+// tokens 169 and 98, now 150 and 89.  Of gate / up's 512 tokens, 141 us in a prompt's pass, the loads alone take 106, the work without the
+// loads 103.
 constexpr int SK_RING = 3;
 // four scale codes, 0x7f (not a number: counts as zero) made zero; and the b-th of them as a factor for fp4x8_to_f16x8 (see e4m3_to_scale)
 IT_DEV uint32_t scale_codes(uint32_t c) {
