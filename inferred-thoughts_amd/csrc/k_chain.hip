@@ -33,12 +33,16 @@
 // A chain holds up to 56 layers, a whole token of the model this is written for; their parameters travel in the
 // kernel's argument block.
 //
-// Three things place the loads and the polls (each measured with the stage stamps below):
+// Four things place the loads, the polls and the stores (the first three measured with the stage stamps below):
 //   * loads return in issue order per wave, so a poll or a publication waits for everything its wave has in flight:
 //     few-word inputs (stages B and F) are gathered by waves that issue their own rows only afterwards;
 //   * a compute unit pulls 25-30 GB/s whatever it asks for: rows are issued where the stage before leaves the pipe idle;
 //   * two waves share a SIMD's vector ALU, so instructions count double: NVFP4 rows go through the hardware's
-//     fp4 -> f16 conversion and v_dot2_f32_f16 (half the instructions of the permute + v_dot4 form, same bits).
+//     fp4 -> f16 conversion and v_dot2_f32_f16 (half the instructions of the permute + v_dot4 form, same bits);
+//   * a line that 256 blocks poll takes one store better than eight: the rows of a block are neighbours, and a stage's
+//     results meet in LDS and leave in one store of one wave where that costs no more than a barrier.  An all-gather of
+//     2,048 words by itself 2.01 -> 1.63 us with the LDS trip, of 4,096 words 2.15 -> 1.69, and 2.11 again when a lane's
+//     pairs of words are neighbours instead of a load's; 48 tokens of 48 layers 66.9 -> 63.5 ms.
 //
 // Every wait is bounded: a poll that runs out of tries sets the abort word, every other wait sees it and the
 // grid drains.  The grid must be resident at once (one block per compute unit), which the launcher checks.
@@ -295,7 +299,7 @@ IT_DEV void forget(AW& a) {
     a.ab = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 IT_DEV int a_row(int k, int b, int wave) {   // row k of the wave in its own matrix
-    return k < 4 ? b + NB * (wave + CW * k) : k < 6 ? b + NB * (wave + CW * (k - 4)) : b < NV ? b : b - NV;
+    return k < 4 ? 32 * b + 4 * wave + k : k < 6 ? 16 * b + 2 * wave + (k - 4) : b < NV ? b : b - NV;
 }
 // An unquantized (F32) row of 2,048 weights is summed in the order the per-stage kernels use (fused_gemv_fast_k's
 // frow_chunk / frow_tree), so that these sums come out the same, to the bit, either way: a chunk of 256 weights is one
@@ -313,7 +317,7 @@ IT_DEV void fetch_a(const M& m, AW& a, int b, int wave, int lane, int parts = 7)
 #pragma unroll
         for (int k = 0; k < 2; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.qkv_q, m.qkv_s, D, a_row(k, b, wave), lane, true);
         if (lane < 4) {
-            const int64_t row = b + NB * (wave + CW * lane);
+            const int64_t row = 32 * b + 4 * wave + lane;
             a.taps = *(const float4*)(m.conv_w + row * 4);
             a.past[0] = m.conv_state[row * 3];
             a.past[1] = m.conv_state[row * 3 + 1];
@@ -339,14 +343,14 @@ IT_DEV void fetch_a(const M& m, AW& a, int b, int wave, int lane, int parts = 7)
     }
 }
 
-// The tail stage's rows (the in-projection of the attention layer behind the chain): 36 a block, row r of the flat list
-// [wq 8192 | wk 512 | wv 512] on block r % 256; a wave takes four wq rows, waves 0..3 one more (wk: 0, 1; wv: 2, 3).
+// The tail stage's rows (the in-projection of the attention layer behind the chain): 36 a block, neighbours in
+// their matrices: a wave takes four wq rows, waves 0..3 one more (wk: 0, 1; wv: 2, 3).
 template <class T>   // ChainTail or ChainAttn: the same three matrices
 IT_DEV void fetch_tail(const T& t, AW& a, int b, int wave, int lane) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) load_row<W_Q8_0, 2, 64>(a.t[k], t.q_q, t.q_s, D, b + NB * (wave + CW * k), lane, true);
+    for (int k = 0; k < 4; k++) load_row<W_Q8_0, 2, 64>(a.t[k], t.q_q, t.q_s, D, 32 * b + 4 * wave + k, lane, true);
     const bool kk = wave < 2;
-    load_row<W_Q8_0, 2, 64>(a.t[4], kk ? t.k_q : t.v_q, kk ? t.k_s : t.v_s, D, b + NB * (wave & 1), lane, wave < 4);
+    load_row<W_Q8_0, 2, 64>(a.t[4], kk ? t.k_q : t.v_q, kk ? t.k_s : t.v_s, D, 2 * b + (wave & 1), lane, wave < 4);
 }
 
 // An NVFP4 chunk against the activation through gfx950's own conversions: v_cvt_scalef32_pk_f16_fp4 turns one byte (two
@@ -662,10 +666,10 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
                     for (int q = 0; q < 4; q++) *(float4*)(Ow + c32 * 32 + 8 * q + 4 * g2) = make_float4(o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]);
                 }
                 const int hd8 = lane >> 3, d4 = lane & 7;
-                const float4 ov = *(const float4*)(Ow + hd8 * 32 + 4 * d4);
-                u64* part = ll + RP + (int64_t)((kvh * AG + hd8) * AS + split) * PW + 32 * wave + 4 * d4;
-                ll_put2f(part, ov.x, ov.y, e);
-                ll_put2f(part + 2, ov.z, ov.w, e);
+                const float2 o0 = *(const float2*)(Ow + hd8 * 32 + 2 * d4), o1 = *(const float2*)(Ow + hd8 * 32 + 16 + 2 * d4);
+                u64* part = ll + RP + (int64_t)((kvh * AG + hd8) * AS + split) * PW + 32 * wave + 2 * d4;
+                ll_put2f(part, o0.x, o0.y, e);
+                ll_put2f(part + 16, o1.x, o1.y, e);
             }
             if (lane == 0) {   // wave = head for the softmax's sums
                 u64* part = ll + RP + (int64_t)((kvh * AG + wave) * AS + split) * PW;
@@ -768,6 +772,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
     __shared__ __align__(16) float wts[16];
     __shared__ float coef[16];
     __shared__ int dead;
+    __shared__ float pub[64];   // a stage's outputs on their way to the one store that publishes them
     __shared__ float fpart[2 * CW];   // partial dots of rows shared by the waves (RF)
     float* const xf = RF ? (float*)route_sh.top.cand : nullptr;   // the normed f32 vector of stages A and D (the route's candidates come later)
     const int tid0 = threadIdx.x, b0 = blockIdx.x;
@@ -809,19 +814,19 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
         const unsigned e = e0 + 1 + (unsigned)l;
         const bool mixer = L.has_mixer != 0;   // the FFN's input comes from a mixer stage of this kernel
 
-        // Stage D's rows.  Waves 0, 1: router rows b and NB + b; waves 2, 3: gate and up rows 2 b and 2 b + 1 of the
-        // shared expert; wave 4 of the last block: the shared expert's gate-logit row.  Issued at the head of the stage
+        // Stage D's rows.  Wave 0 (waves 0, 1 beside an NVFP4 shared expert, whose rows leave no registers for a second one):
+        // router rows 2 b and 2 b + 1; waves 2, 3: gate and up rows 2 b and 2 b + 1 of the shared expert; wave 4 of the last block: the shared expert's gate-logit row.  Issued at the head of the stage
         // before D (small loads issued at the head of a stage are back before its input is).
         WChunks<2> d0, d1;
         WChunks<1> n0, n1;
         const int sh_row = 2 * b + (wave - 2);
         float4 rf0, rf1, lf;   // RF: this wave's quarter of an unquantized router row (two float4 a lane), its eighth of the gate-logit row
         auto fetch_d = [&]() {
-            const bool r = wave < 2, sh = wave == 2 || wave == 3, lg = wave == 4 && b == NB - 1;
+            const bool r = SF == W_Q8_0 ? wave == 0 : wave < 2, sh = wave == 2 || wave == 3, lg = wave == 4 && b == NB - 1;
             if (RF) {
-                // unquantized router and gate-logit rows: row b in waves 0..3, row NB + b in waves 4..7, 512 floats a wave;
+                // unquantized router and gate-logit rows: row 2 b in waves 0..3, row 2 b + 1 in waves 4..7, 512 floats a wave;
                 // the gate-logit row in the last block, 256 floats a wave; the partial dots meet in LDS
-                const float4* row = (const float4*)((const float*)f.r_q + (int64_t)(b + NB * (wave >> 2)) * D) + (wave & 3) * 128;
+                const float4* row = (const float4*)((const float*)f.r_q + (int64_t)(2 * b + (wave >> 2)) * D) + (wave & 3) * 128;
                 rf0 = row[lane];
                 rf1 = row[64 + lane];
                 lf = b == NB - 1 ? ((const float4*)f.l_q)[wave * 64 + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -834,10 +839,10 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 }
             } else if (SF == W_Q8_0) {
                 load_row<W_Q8_0, 2, 64>(d0, r ? f.r_q : sh ? f.sg_q : f.l_q, r ? f.r_s : sh ? f.sg_s : f.l_s, D,
-                                      r ? b + NB * wave : sh ? sh_row : 0, lane, r || sh || lg);
-                load_row<W_Q8_0, 2, 64>(d1, f.su_q, f.su_s, D, sh_row, lane, sh);
+                                      r ? 2 * b : sh ? sh_row : 0, lane, r || sh || lg);
+                load_row<W_Q8_0, 2, 64>(d1, r ? f.r_q : f.su_q, r ? f.r_s : f.su_s, D, r ? 2 * b + 1 : sh_row, lane, r || sh);
             } else {
-                load_row<W_Q8_0, 2, 64>(d0, r ? f.r_q : f.l_q, r ? f.r_s : f.l_s, D, r ? b + NB * wave : 0, lane, r || lg);
+                load_row<W_Q8_0, 2, 64>(d0, r ? f.r_q : f.l_q, r ? f.r_s : f.l_s, D, r ? 2 * b + wave : 0, lane, r || lg);
                 load_row<W_NVFP4, 1, 64>(n0, f.sg_q, f.sg_s, D, sh_row, lane, sh);
                 load_row<W_NVFP4, 1, 64>(n1, f.su_q, f.su_s, D, sh_row, lane, sh);
             }
@@ -885,9 +890,9 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     const float r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 63));
                     mine = lane == k ? r : mine;
                 }
-                if (lane < 4) ll_putf(p.ll + RQ + b + NB * (wave + CW * lane), mine, e);
-                else if (lane == 4 && wave < 2) ll_putf(p.ll + RK + b + NB * wave, mine, e);
-                else if (lane == 4 && wave < 4) ll_putf(p.ll + RV + b + NB * (wave - 2), mine, e);
+                if (lane < 4) ll_putf(p.ll + RQ + 32 * b + 4 * wave + lane, mine, e);
+                else if (lane == 4 && wave < 2) ll_putf(p.ll + RK + 2 * b + wave, mine, e);
+                else if (lane == 4 && wave < 4) ll_putf(p.ll + RV + 2 * b + (wave - 2), mine, e);
             }
             CH_STAMP(17);
             // ---------------------------------------------------------------- attention over the context, merge, sigmoid gate
@@ -900,9 +905,10 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             if (!r.ok) dead = 1;
             if (lane == 63) {   // + residual
                 x_row += r.dot;
-                ll_putf(p.ll + RC + my_row, x_row, e);
+                pub[wave] = x_row;
             }
             __syncthreads();
+            if (tid < CW) ll_putf(p.ll + RC + b * CW + tid, pub[tid], e);
             if (dead) break;
         }
         if (L.has_mixer == 1) {
@@ -940,7 +946,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 }
                 if (lane < 4) {
                     // causal conv (kernel 4) + silu on channel `row`, state [channel][3] oldest first
-                    const int64_t row = b + NB * (wave + CW * lane);
+                    const int64_t row = 32 * b + 4 * wave + lane;
                     float sum = 0.0f;
                     sum += aw.past[0] * aw.taps.x;
                     sum += aw.past[1] * aw.taps.y;
@@ -952,7 +958,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     past[1] = aw.past[2];
                     past[2] = mine;
                 } else if (lane < 6) {
-                    ll_putf(p.ll + RA_Z + b + NB * (wave + CW * (lane - 4)), fx_silu(mine), e);
+                    ll_putf(p.ll + RA_Z + 16 * b + 2 * wave + (lane - 4), fx_silu(mine), e);
                 } else if (!RF && lane == 6 && wave == 0 && b < 2 * NV) {
                     ll_putf(p.ll + RA_AL + b, mine, e);
                 }
@@ -1071,22 +1077,24 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 *(float4*)S = make_float4(row[0], row[1], row[2], row[3]);
                 if (seg == 0) {
                     // silu(z) * (o * hs * w) with the head's scale hs applied by the reader, which sums the squares
-                    ll_putf(p.ll + RB + h * DK + j0 + j, sm[16 + j] * (o * head_w), e);
+                    pub[j] = sm[16 + j] * (o * head_w);
                     sm[40 + j] = o * o;
                 }
                 __syncthreads();
-                if (tid == 0) {
+                if (tid < 17) {
                     float s = 0.0f;
 #pragma unroll
                     for (int i = 0; i < 16; i++) s += sm[40 + i];
-                    ll_putf(p.ll + RB_SS + b, s, e);
+                    // element 4 q + i of the block: the quads' first pairs, then their second ones, so that a reader's load
+                    // of one pair a lane is contiguous
+                    ll_putf(tid < 16 ? p.ll + RB + (tid & 2) * (VDIM / 4) + 8 * b + 2 * (tid >> 2) + (tid & 1) : p.ll + RB_SS + b, tid < 16 ? pub[tid & 15] : s, e);
                 }
             }
             // ---------------------------------------------------------------- C: out-projection + residual
             CH_STAMP(3);
             if (!IT_CHAIN_D_AT) fetch_d();
             {
-                const u64* const a4[4] = {p.ll + RB + 4 * tid, p.ll + RB + 4 * tid + 2, p.ll + RB + 4 * (tid + CT), p.ll + RB + 4 * (tid + CT) + 2};
+                const u64* const a4[4] = {p.ll + RB + 2 * tid, p.ll + RB + VDIM / 2 + 2 * tid, p.ll + RB + 2 * (tid + CT), p.ll + RB + VDIM / 2 + 2 * (tid + CT)};
                 uint32_t o[8];
                 bool ok = ll_wait_pairs<4>(a4, e, ctl, o);
                 if (tid < NB / 2) {
@@ -1117,8 +1125,10 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 const float acc = reduce_lanes<64>(dot_chunks<W_Q8_0, 4>(wc, x));
                 if (lane == 63) {
                     x_row += acc;
-                    ll_putf(p.ll + RC + my_row, x_row, e);
+                    pub[wave] = x_row;
                 }
+                __syncthreads();
+                if (tid < CW) ll_putf(p.ll + RC + b * CW + tid, pub[tid], e);
             }
         }
 
@@ -1149,9 +1159,12 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     fpart[wave] = pr;
                     fpart[CW + wave] = pl;
                 }
-            } else if (wave < 2 || (wave == 4 && b == NB - 1)) {
+            } else if (SF == W_Q8_0 && wave == 0) {
+                const float a0 = reduce_lanes<64>(dot_chunks<W_Q8_0, 2>(d0, x)), a1 = reduce_lanes<64>(dot_chunks<W_Q8_0, 2>(d1, x));
+                if (lane == 63) ll_put2f(p.ll + RD + 2 * b, a0, a1, e);
+            } else if ((SF != W_Q8_0 && wave < 2) || (wave == 4 && b == NB - 1)) {
                 const float a = reduce_lanes<64>(dot_chunks<W_Q8_0, 2>(d0, x));
-                if (lane == 63) ll_putf(p.ll + RD + (wave < 2 ? b + NB * wave : NE), a, e);
+                if (lane == 63) ll_putf(p.ll + RD + (wave < 2 ? 2 * b + wave : NE), a, e);
             }
             if (wave == 2 || wave == 3) {
                 float ag, au;
@@ -1170,7 +1183,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             }
             if (RF) {
                 __syncthreads();
-                if (tid < 2) ll_putf(p.ll + RD + b + NB * tid, (fpart[4 * tid] + fpart[4 * tid + 1]) + (fpart[4 * tid + 2] + fpart[4 * tid + 3]), e);
+                if (tid < 2) ll_putf(p.ll + RD + 2 * b + tid, (fpart[4 * tid] + fpart[4 * tid + 1]) + (fpart[4 * tid + 2] + fpart[4 * tid + 3]), e);
                 if (tid == 64 && b == NB - 1) ll_putf(p.ll + RD + NE, f32_tree(fpart + CW), e);
             }
         }
@@ -1461,8 +1474,12 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             acc = reduce_lanes<64>(acc);
             if (lane == 63) {
                 x_row += acc;
-                ll_putf(p.ll + RX + my_row, x_row, e + 1);
-                p.x[my_row] = x_row;
+                pub[wave] = x_row;
+            }
+            __syncthreads();
+            if (tid < CW) {
+                ll_putf(p.ll + RX + b * CW + tid, pub[tid], e + 1);
+                p.x[b * CW + tid] = pub[tid];
             }
         }
         CH_STAMP(12);
@@ -1490,9 +1507,9 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     const float r = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc), 63));
                     mine = lane == k ? r : mine;
                 }
-                if (lane < 4) t.out_q[b + NB * (wave + CW * lane)] = mine;
-                else if (lane == 4 && wave < 2) t.out_k[b + NB * wave] = mine;
-                else if (lane == 4 && wave < 4) t.out_v[b + NB * (wave - 2)] = mine;
+                if (lane < 4) t.out_q[32 * b + 4 * wave + lane] = mine;
+                else if (lane == 4 && wave < 2) t.out_k[2 * b + wave] = mine;
+                else if (lane == 4 && wave < 4) t.out_v[2 * b + (wave - 2)] = mine;
             }
         }
     }
