@@ -195,9 +195,10 @@ IT_DEV bool ll_give_up(int& spins, const Ctl& c) {
 #ifndef IT_CHAIN_FIRST_SLEEP
 #define IT_CHAIN_FIRST_SLEEP 8
 #endif
+template <int SL = IT_CHAIN_FIRST_SLEEP>   // (0 behind another wait of the same stage: the words are there)
 IT_DEV bool ll_wait1(const u64* p, unsigned e, const Ctl& c, uint32_t* out) {
     int spins = 0;
-    if (IT_CHAIN_FIRST_SLEEP > 0) __builtin_amdgcn_s_sleep(IT_CHAIN_FIRST_SLEEP);
+    if (SL > 0) __builtin_amdgcn_s_sleep(SL);
     for (;;) {
         v2u w;
         asm volatile("global_load_dwordx2 %0, %1, off sc0 sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(w) : "v"(p) : "memory");
@@ -210,12 +211,12 @@ IT_DEV bool ll_wait1(const u64* p, unsigned e, const Ctl& c, uint32_t* out) {
 }
 // K pairs of words at a[k] (16-byte aligned); out[2k], out[2k+1] = their payloads.  A pair that is complete is
 // latched; its load is simply repeated while the others are still awaited.
-template <int K>
+template <int K, int SL = IT_CHAIN_FIRST_SLEEP>
 IT_DEV bool ll_wait_pairs(const u64* const (&a)[K], unsigned e, const Ctl& c, uint32_t (&out)[2 * K]) {
     static_assert(K == 1 || K == 2 || K == 4, "");
     int spins = 0;
     unsigned done = 0;
-    if (IT_CHAIN_FIRST_SLEEP > 0) __builtin_amdgcn_s_sleep(IT_CHAIN_FIRST_SLEEP);
+    if (SL > 0) __builtin_amdgcn_s_sleep(SL);
     for (;;) {
         v4u w[K];
         if constexpr (K == 4)
@@ -1100,7 +1101,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 if (tid < NB / 2) {
                     const u64* const a1[1] = {p.ll + RB_SS + 2 * tid};
                     uint32_t s2[2];
-                    ok = ok && ll_wait_pairs<1>(a1, e, ctl, s2);
+                    ok = ok && ll_wait_pairs<1, 0>(a1, e, ctl, s2);
                     ssq[2 * tid] = __uint_as_float(s2[0]);
                     ssq[2 * tid + 1] = __uint_as_float(s2[1]);
                 }
@@ -1203,7 +1204,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             const u64 my_key[1] = {((u64)logit_order(my_logit) << 32) | (u64)(~(unsigned)tid)};   // larger = earlier pick, unique
             top_begin(route_sh.top, (unsigned)(my_key[0] >> 32));
             if (tid == 0) {
-                ok = ok && ll_wait1(p.ll + RD + NE, e, ctl, &w0);
+                ok = ok && ll_wait1<0>(p.ll + RD + NE, e, ctl, &w0);
                 sm[34] = __uint_as_float(w0);
             }
             if (!ok) dead = 1;
@@ -1302,18 +1303,8 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 if (tid < 8) {
                     // Q8_0 of the block's 32 intermediates (naive.rs:652-675), published as four quants a word
                     const float4 v = *(const float4*)(inter + tid * 4);
-                    float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-                    amax = group_max<8>(amax);
-                    const float d = amax / 127.0f;
-                    const float id = d != 0.0f ? 1.0f / d : 0.0f;
-                    const float r[4] = {roundf(v.x * id), roundf(v.y * id), roundf(v.z * id), roundf(v.w * id)};
-                    uint32_t packed = 0;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float cl = fminf(fmaxf(r[i], -128.0f), 127.0f);
-                        const int q = (r[i] != r[i]) ? 0 : (int)cl;
-                        packed |= ((uint32_t)(q & 0xff)) << (8 * i);
-                    }
+                    float d;
+                    const uint32_t packed = quant_word(v, group_max<8>(quad_amax(v)), &d);
                     ll_put(p.ll + RE + b * 8 + tid, packed, e);
                     if (tid == 0) ll_putf(p.ll + RE_SC + b, it_f16_to_f32(it_f32_to_f16(d)), e);
                 }
