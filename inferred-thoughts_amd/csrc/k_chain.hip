@@ -16,8 +16,8 @@
 //      weight, with the block's share of the head's sum of squares beside it
 //   C  head-norm scale, quantization, rows of ssm_out, residual
 //   D  rms_norm + quantization; router rows, the shared expert's gate logit, its gate / up rows
-//   E  top-10 of the logits in every block (ranked on the logits; the softmax of the ten follows under the rows'
-//      flight); 160 blocks take one 32-element block of one pick's gate / up rows each and publish it quantized, the
+//   E  top-10 of the logits in every block (ranked on the logits; the softmax's sum follows under the rows' flight, the
+//      ten's weights beside the publication); 160 blocks take one 32-element block of one pick's gate / up rows each and publish it quantized, the
 //      other 96 touch those rows' lines for the blocks of their XCD; the down rows are issued behind the publication
 //   F  down rows of the ten picks and of the shared expert, combine, residual
 // An attention layer's mixer (src/model/qwen35.rs:1141-1223) is five stages of its own in front of its FFN's D, E, F:
@@ -38,7 +38,10 @@
 //     few-word inputs (stages B and F) are gathered by waves that issue their own rows only afterwards;
 //   * a compute unit pulls 25-30 GB/s whatever it asks for: rows are issued where the stage before leaves the pipe idle;
 //   * two waves share a SIMD's vector ALU, so instructions count double: NVFP4 rows go through the hardware's
-//     fp4 -> f16 conversion and v_dot2_f32_f16 (half the instructions of the permute + v_dot4 form, same bits);
+//     fp4 -> f16 conversion and v_dot2_f32_f16 (half the instructions of the permute + v_dot4 form, same bits), their
+//     activations lie in LDS as the f16 pairs that takes (quantized once a thread, not converted in every wave), a lane
+//     forms one head's scale for stage C and not two, and the picks' weights are formed in a wave with nothing else to do
+//     (eight layers of a token together 235.2 -> 224.9 us, 221.0 -> 219.0 with Q8_0 routers);
 //   * a line that 256 blocks poll takes one store better than eight: the rows of a block are neighbours, and a stage's
 //     results meet in LDS and leave in one store of one wave where that costs no more than a barrier.  An all-gather of
 //     2,048 words by itself 2.01 -> 1.63 us with the LDS trip, of 4,096 words 2.15 -> 1.69, and 2.11 again when a lane's
@@ -130,21 +133,12 @@ __device__ long long it_chain_wave_stamps[8][8];
     } while (0)
 #endif
 
-#ifndef IT_CHAIN_FP4_HW
-#define IT_CHAIN_FP4_HW 1         // NVFP4 rows of stages D and E through the hardware's fp4 / fp8 conversions (1) or through v_perm_b32 + v_dot4 (0)
-#endif
 // Where the prefetches sit (tuning switches; the defaults are what measured best).
-#ifndef IT_CHAIN_F_POLLERS
-#define IT_CHAIN_F_POLLERS 1     // stage F's input gathered by waves 4..7 alone (1) or by every thread (0)
-#endif
 #ifndef IT_CHAIN_B_POLLERS
 #define IT_CHAIN_B_POLLERS 1     // stage B's input gathered by waves 5..7 alone (1) or by the first 274 threads (0)
 #endif
 #ifndef IT_CHAIN_TOUCH
 #define IT_CHAIN_TOUCH 1          // stage E's rows touched by the blocks that have none of their own
-#endif
-#ifndef IT_CHAIN_FLOADS_EARLY
-#define IT_CHAIN_FLOADS_EARLY 0   // stage F's down rows: 1 ahead of stage E's barrier and publication, 0 behind them
 #endif
 #ifndef IT_CHAIN_WC_AT
 #define IT_CHAIN_WC_AT 0      // out-projection row: 0 at the head of stage B, 1 after stage A's input has arrived, 2 after stage A's dots, 3 after stage B's input has arrived
@@ -191,9 +185,10 @@ IT_DEV bool ll_give_up(int& spins, const Ctl& c) {
 // Polls.  A load and its wait are ONE asm statement: the compiler does not know that the destination of an asm
 // load is not ready, so nothing may be schedulable between the two.
 // a short sleep ahead of a wait's first poll: a poll issued the moment the wave arrives nearly always fails, and every
-// failed poll is traffic that the words it waits for queue behind
+// failed poll is traffic that the words it waits for queue behind (eight layers of a token with 0, 4, 8, 12, 16 times 64
+// cycles: 232.6, 227.9, 224.9, 223.1, 223.0 us)
 #ifndef IT_CHAIN_FIRST_SLEEP
-#define IT_CHAIN_FIRST_SLEEP 8
+#define IT_CHAIN_FIRST_SLEEP 12
 #endif
 template <int SL = IT_CHAIN_FIRST_SLEEP>   // (0 behind another wait of the same stage: the words are there)
 IT_DEV bool ll_wait1(const u64* p, unsigned e, const Ctl& c, uint32_t* out) {
@@ -361,29 +356,37 @@ IT_DEV void fetch_tail(const T& t, AW& a, int b, int wave, int lane) {
 // a multiple of 0.5 below 2^24, so the f32 accumulation is exact and the result is the integer path's, bit for bit.
 // The sub-block scales come from v_cvt_pk_f32_fp8 (OCP e4m3; the format's ue4m3 is half of that, and the e2m1 values
 // here are half of the integer path's doubled ones: the two factors of 2 cancel; code 0x7f is 0 as in it_ue4m3_to_f32).
-#if IT_CHAIN_FP4_HW
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float f2v __attribute__((ext_vector_type(2)));
 struct XN {
     uint32_t p[16];   // sub-block A: pairs (j, 8 + j) j = 0..7, then sub-block B
     float d;
 };
-IT_DEV uint32_t pair_h(uint32_t lo, uint32_t hi, int j) {
-    const h2v v = {(_Float16)(int)(int8_t)(lo >> (8 * j)), (_Float16)(int)(int8_t)(hi >> (8 * j))};
-    return __builtin_bit_cast(uint32_t, v);
-}
-IT_DEV void load_xn(XN& x, const int8_t* xq, const float* xs, int lane) {
-    XChunks<W_NVFP4, 1> t;
-    load_x<W_NVFP4, 1, 64>(t, xq, xs, lane);
+// In LDS such an activation is four planes, one of each quarter of a 32-element unit's sixteen pairs: unit u's quarter q is
+// 16 bytes at q * (16 * units) + 16 * u, so that the lanes of a load read neighbours.
+IT_DEV void load_xn(XN& x, const uint8_t* xh, int units, int u, float d) {
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        x.p[j] = pair_h(t.a[0].x, t.a[0].z, j);
-        x.p[4 + j] = pair_h(t.a[0].y, t.a[0].w, j);
-        x.p[8 + j] = pair_h(t.b[0].x, t.b[0].z, j);
-        x.p[12 + j] = pair_h(t.b[0].y, t.b[0].w, j);
+    for (int q = 0; q < 4; q++) {
+        const uint4 t = *(const uint4*)(xh + (q * units + u) * 16);
+        x.p[4 * q] = t.x;
+        x.p[4 * q + 1] = t.y;
+        x.p[4 * q + 2] = t.z;
+        x.p[4 * q + 3] = t.w;
     }
-    x.d = t.d[0];
+    x.d = d;
 }
+// four quants each of elements j .. j + 3 (lo) and 8 + j .. (hi) of a sub-block as f16 pairs, exact: a byte plus 128 in the
+// low bits of 1,024's f16, less 1,152
+IT_DEV uint4 quant_pairs(uint32_t lo, uint32_t hi) {
+    const uint32_t a = lo ^ 0x80808080u, b = hi ^ 0x80808080u;
+    auto pair = [&](uint32_t sel) {
+        const h2v v = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(b, a, sel) | 0x64006400u) - h2v{(_Float16)1152.0f, (_Float16)1152.0f};
+        return __builtin_bit_cast(uint32_t, v);
+    };
+    return make_uint4(pair(0x0c040c00u), pair(0x0c050c01u), pair(0x0c060c02u), pair(0x0c070c03u));
+}
+// the word of the lane two further on in its quad
+IT_DEV uint32_t word_ahead2(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xee, 0xf, 0xf, true); }   // quad_perm [2, 3, 2, 3]
 #define IT_FP4_STEP(acc, word, sel, pi) \
     acc = __builtin_amdgcn_fdot2(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, sel), __builtin_bit_cast(h2v, x.p[pi]), acc, false)
 IT_DEV float dot_xn(const WChunks<1>& t, const XN& x) {
@@ -401,11 +404,6 @@ IT_DEV float dot_xn(const WChunks<1>& t, const XN& x) {
     acc += (x.d * dB) * sb;
     return acc;
 }
-#else
-typedef XChunks<W_NVFP4, 1> XN;
-IT_DEV void load_xn(XN& x, const int8_t* xq, const float* xs, int lane) { load_x<W_NVFP4, 1, 64>(x, xq, xs, lane); }
-IT_DEV float dot_xn(const WChunks<1>& t, const XN& x) { return dot_chunks<W_NVFP4, 1>(t, x); }
-#endif
 
 // a float's bits as an unsigned that orders like the value (negative below positive), and back
 IT_DEV uint32_t logit_order(float v) {
@@ -416,7 +414,8 @@ IT_DEV float logit_of_order(uint32_t o) { return __uint_as_float((o & 0x80000000
 
 // rms_norm (naive.rs:633-650) of the 2,048 floats the block's threads hold as quads, then Q8_0 (naive.rs:652-675)
 // into xq / xs.  Two barriers; returns false after the first when the block has to stop.
-IT_DEV void norm_quant_finish(float4 v, float4 w, float eps, double sum, int8_t* xq, float* xs, int tid, float* xf = nullptr) {
+// xh: the quants as f16 pairs too (load_xn's planes)
+IT_DEV void norm_quant_finish(float4 v, float4 w, float eps, double sum, int8_t* xq, float* xs, int tid, float* xf = nullptr, uint8_t* xh = nullptr) {
     const float mean = (float)(sum / (double)D);
     const float scale = 1.0f / sqrtf(mean + eps);
     v.x = v.x * scale * w.x;
@@ -424,10 +423,18 @@ IT_DEV void norm_quant_finish(float4 v, float4 w, float eps, double sum, int8_t*
     v.z = v.z * scale * w.z;
     v.w = v.w * scale * w.w;
     if (xf) ((float4*)xf)[tid] = v;   // the normed vector itself, for rows of unquantized matrices
-    quant_quad(v, true, tid, xq, xs);
+    const float amax = group_max<8>(quad_amax(v));
+    float d;
+    const uint32_t word = quant_word(v, amax, &d);
+    *(uint32_t*)(xq + tid * 4) = word;
+    if ((tid & 7) == 0) xs[tid >> 3] = it_f16_to_f32(it_f32_to_f16(d));
+    if (xh) {
+        const uint32_t ahead = word_ahead2(word);
+        if (!(tid & 2)) *(uint4*)(xh + (((tid >> 1) & 2) + (tid & 1)) * (D / 2) + (tid >> 3) * 16) = quant_pairs(word, ahead);
+    }
     __syncthreads();
 }
-IT_DEV bool norm_quant(float4 v, float4 w, float eps, int8_t* xq, float* xs, double* red, const int* dead, int tid, float* xf = nullptr) {
+IT_DEV bool norm_quant(float4 v, float4 w, float eps, int8_t* xq, float* xs, double* red, const int* dead, int tid, float* xf = nullptr, uint8_t* xh = nullptr) {
     const double part = wave_sum_f64_tail(quad_sumsq(v));
     if ((tid & 63) == 63) red[tid >> 6] = part;
     __syncthreads();
@@ -435,7 +442,7 @@ IT_DEV bool norm_quant(float4 v, float4 w, float eps, int8_t* xq, float* xs, dou
     double sum = 0.0;
 #pragma unroll
     for (int i = 0; i < CW; i++) sum += red[i];
-    norm_quant_finish(v, w, eps, sum, xq, xs, tid, xf);
+    norm_quant_finish(v, w, eps, sum, xq, xs, tid, xf, xh);
     return true;
 }
 
@@ -761,21 +768,23 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
 
 template <int SF, int RF, int NL>
 __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
-    __shared__ __align__(16) int8_t xq[NU * FF + FF];   // the stage's quantized activation (largest: the down stage's)
+    __shared__ __align__(16) int8_t xq[VDIM];   // the stage's quantized activation (largest: the out-projection's)
     __shared__ __align__(16) float xs[(NU * FF + FF) / 32];
     __shared__ double red[CW];
     __shared__ __align__(16) float kq[2 * DK];
     __shared__ __align__(16) float ssq[NB];
     __shared__ float sm[64];
     __shared__ __align__(16) float inter[32];
-    __shared__ RouteLds<CT> route_sh;
+    __shared__ TopLds<CT, 4> top_sh;
     __shared__ int ids[16];
     __shared__ __align__(16) float wts[16];
     __shared__ float coef[16];
     __shared__ int dead;
+    __shared__ __align__(16) uint8_t xh[(NU + 1) * FF * 2];   // activations of NVFP4 rows as f16 pairs: stages D and E's, then the down stage's
+    __shared__ float redf[CW];
     __shared__ float pub[64];   // a stage's outputs on their way to the one store that publishes them
     __shared__ float fpart[2 * CW];   // partial dots of rows shared by the waves (RF)
-    float* const xf = RF ? (float*)route_sh.top.cand : nullptr;   // the normed f32 vector of stages A and D (the route's candidates come later)
+    float* const xf = RF ? (float*)top_sh.cand : nullptr;   // the normed f32 vector of stages A and D (the route's candidates come later)
     const int tid0 = threadIdx.x, b0 = blockIdx.x;
     const Ctl ctl{p.abort_flag, p.spin_limit};
     const unsigned e0 = *(const volatile unsigned*)p.epoch;
@@ -1109,13 +1118,23 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 __syncthreads();
                 if (dead) break;
                 CH_STAMP(4);
-#pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    const int qi = tid + k * CT, head = qi >> 5;
+                // A lane's quads tid and tid + 512 are of heads tid / 32 and 16 + tid / 32: of each 32 lanes the first 16 form the one
+                // head's scale, the others the other's, and the halves are exchanged.
+                float hsk[2];
+                {
+                    const int head = (tid >> 5) + (lane & 16);
                     const float4 s0 = *(const float4*)(ssq + head * 8), s1 = *(const float4*)(ssq + head * 8 + 4);
                     const double sum = (double)s0.x + (double)s0.y + (double)s0.z + (double)s0.w + (double)s1.x + (double)s1.y +
                                        (double)s1.z + (double)s1.w;
-                    const float hs = 1.0f / sqrtf((float)(sum / (double)DK) + m.eps_head);
+                    const unsigned mine = __float_as_uint(1.0f / sqrtf((float)(sum / (double)DK) + m.eps_head));
+                    const auto both = __builtin_amdgcn_permlane16_swap(mine, mine, false, false);
+                    hsk[0] = __uint_as_float(both[0]);
+                    hsk[1] = __uint_as_float(both[1]);
+                }
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int qi = tid + k * CT;
+                    const float hs = hsk[k];
                     const float4 v = make_float4(__uint_as_float(o[4 * k]) * hs, __uint_as_float(o[4 * k + 1]) * hs,
                                                  __uint_as_float(o[4 * k + 2]) * hs, __uint_as_float(o[4 * k + 3]) * hs);
                     quant_quad(v, true, qi, xq, xs);
@@ -1144,13 +1163,13 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             else if (l == 0) v = ((const float4*)p.x)[tid];
             else ok = ll_wait_quad(p.ll + RX, tid, e, ctl, &v);
             if (!ok) dead = 1;
-            if (!norm_quant(v, nw, f.eps, xq, xs, red, &dead, tid, xf)) break;
+            if (!norm_quant(v, nw, f.eps, xq, xs, red, &dead, tid, xf, xh)) break;
             if (l + 1 < p.n_layers && p.layer[l + 1].has_mixer == 1 && ((IT_CHAIN_A_AT >> 8) & 15))
                 fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane, (IT_CHAIN_A_AT >> 8) & 15);
             CH_STAMP(6);
             XChunks<W_Q8_0, 2> x;
             load_x<W_Q8_0, 2, 64>(x, xq, xs, lane);
-            load_xn(xn, xq, xs, lane);
+            load_xn(xn, xh, D / 32, lane, xs[lane]);
             if (RF) {
                 const float4 xa = ((const float4*)xf)[(wave & 3) * 128 + lane], xb = ((const float4*)xf)[(wave & 3) * 128 + 64 + lane];
                 const float pr = reduce_lanes<64>(f32_chunk(rf0, xa)) + reduce_lanes<64>(f32_chunk(rf1, xb));
@@ -1193,7 +1212,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
         CH_STAMP(7);
         CHAIN_RECOORD();
         WChunks<1> fd[3];
-        WChunks<1> fsh;   // the shared expert's down row: lanes 32..63 (Q8_0) or 32..47 (NVFP4) beside the last two picks
+        WChunks<1> fsh;   // the shared expert's Q8_0 down row: lanes 32..63 (an NVFP4 one is lanes 32..47 of fd[2], beside the last two picks)
         {
             // The route (softmax over the 512 logits, the 10 largest, src/ops/mod.rs:1191-1216), in the order that lets
             // the picks' rows start moving first: the picks are ranked on the logits themselves (the softmax keeps their
@@ -1202,7 +1221,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             bool ok = ll_wait1(p.ll + RD + tid, e, ctl, &w0);
             const float my_logit = __uint_as_float(w0);
             const u64 my_key[1] = {((u64)logit_order(my_logit) << 32) | (u64)(~(unsigned)tid)};   // larger = earlier pick, unique
-            top_begin(route_sh.top, (unsigned)(my_key[0] >> 32));
+            top_begin(top_sh, (unsigned)(my_key[0] >> 32));
             if (tid == 0) {
                 ok = ok && ll_wait1<0>(p.ll + RD + NE, e, ctl, &w0);
                 sm[34] = __uint_as_float(w0);
@@ -1212,14 +1231,14 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             if (dead) break;
             CH_STAMP(8);
             CH_WSTAMP(0);
-            top_pick(route_sh.top, my_key, 1, NU, [&](int rank, u64 pick) {
+            top_pick(top_sh, my_key, 1, NU, [&](int rank, u64 pick) {
                 ids[rank] = (int)~(unsigned)(pick & 0xffffffffull);
                 wts[rank] = logit_of_order((uint32_t)(pick >> 32));   // the pick's logit; its probability follows below
             });
             __syncthreads();
             CH_STAMP(9);
             CH_WSTAMP(1);
-            const float my_dscale = (tid < NU && f.dscale2) ? f.dscale2[ids[tid]] : 1.0f;   // issued ahead of the rows below
+            const float my_dscale = (wave == 3 && lane < NU && f.dscale2) ? f.dscale2[ids[lane]] : 1.0f;   // issued ahead of the rows below
             // Rows pulled towards the caches ahead of the loads that use them.  A wave's 16-byte-a-lane load asks for eight
             // 128-byte lines; one 4-byte load with every lane on a line of its own asks for 64, so a few such loads put a
             // whole stage's rows in flight at once, from compute units that have nothing else to fetch.
@@ -1245,6 +1264,12 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     }
                 }
             }
+            // the softmax's sum, exp(logit - largest logit) over the 512, by wave here, under the rows' flight, and over the waves
+            // in order behind the stage's barrier
+            auto softmax_part = [&]() {
+                const float part = group_sum_tail<64>(fx_expf(my_logit - wts[0]));
+                if (lane == 63) redf[wave] = part;
+            };
             // the picks' rows: this block's 32 gate and 32 up rows
             WChunks<1> tg[4], tu[4];
             float scg = 1.0f, scu = 1.0f;
@@ -1263,6 +1288,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 if (f.uscale2) scu = f.uscale2[ex];
                 CH_STAMP(13);
                 CH_WSTAMP(2);
+                softmax_part();
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     float ag = reduce_lanes<64>(dot_xn(tg[i], xn));
@@ -1274,27 +1300,12 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     }
                     if (i == 0) CH_WSTAMP(3);
                 }
+            } else {
+                softmax_part();
+                asm volatile("" ::"v"(touched));   // (here, where nothing else is in flight that the touches' return would be waited for behind)
             }
             CH_STAMP(14);
             CH_WSTAMP(4);
-#if IT_CHAIN_FLOADS_EARLY
-            // the down rows of this wave's output row, for stage F: issued behind the publication, they land while the intermediates travel
-            // (four picks a step over 16 lanes each, the shared row beside the last two picks)
-#pragma unroll
-            for (int s = 0; s < 3; s++) {
-                const int y = s * 4 + (lane >> 4);
-                const bool routed = y < NU;
-                const int64_t ex = routed ? ids[y] : 0;
-                load_row<W_NVFP4, 1, 16>(fd[s], f.ed_q + ex * f.d_q_stride, f.ed_s + ex * f.d_s_stride, FF, my_row, lane & 15, routed);
-            }
-            if (SF == W_Q8_0) load_row<W_Q8_0, 1, 32>(fsh, f.sd_q, f.sd_s, FF, my_row, lane & 31, lane >= 32);
-            else load_row<W_NVFP4, 1, 16>(fsh, f.sd_q, f.sd_s, FF, my_row, lane & 15, lane >= 32 && lane < 48);
-#endif
-            // the softmax's sum: exp(logit - largest logit) over the 512, by wave and then over the waves in order
-            {
-                const float part = group_sum_tail<64>(fx_expf(my_logit - wts[0]));
-                if (lane == 63) route_sh.redf[wave] = part;
-            }
             CH_STAMP(15);
             CH_WSTAMP(5);
             __syncthreads();
@@ -1305,35 +1316,35 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     const float4 v = *(const float4*)(inter + tid * 4);
                     float d;
                     const uint32_t packed = quant_word(v, group_max<8>(quad_amax(v)), &d);
-                    ll_put(p.ll + RE + b * 8 + tid, packed, e);
+                    // (a pair of words holds the quants of elements j .. and 8 + j .. of a sub-block, as stage F pairs them)
+                    ll_put(p.ll + RE + b * 8 + ((tid & 4) | ((tid & 1) << 1) | ((tid >> 1) & 1)), packed, e);
                     if (tid == 0) ll_putf(p.ll + RE_SC + b, it_f16_to_f32(it_f32_to_f16(d)), e);
                 }
             }
-#if !IT_CHAIN_FLOADS_EARLY
             // the down rows of this wave's output row, for stage F: issued behind the publication, they land while the intermediates travel
             // (four picks a step over 16 lanes each, the shared row beside the last two picks)
 #pragma unroll
             for (int s = 0; s < 3; s++) {
                 const int y = s * 4 + (lane >> 4);
-                const bool routed = y < NU;
+                const bool routed = y < NU, shared = SF == W_NVFP4 && y == NU;
                 const int64_t ex = routed ? ids[y] : 0;
-                load_row<W_NVFP4, 1, 16>(fd[s], f.ed_q + ex * f.d_q_stride, f.ed_s + ex * f.d_s_stride, FF, my_row, lane & 15, routed);
+                load_row<W_NVFP4, 1, 16>(fd[s], shared ? (const uint8_t*)f.sd_q : f.ed_q + ex * f.d_q_stride, shared ? (const uint8_t*)f.sd_s : f.ed_s + ex * f.d_s_stride,
+                                         FF, my_row, lane & 15, routed || shared);
             }
             if (SF == W_Q8_0) load_row<W_Q8_0, 1, 32>(fsh, f.sd_q, f.sd_s, FF, my_row, lane & 31, lane >= 32);
-            else load_row<W_NVFP4, 1, 16>(fsh, f.sd_q, f.sd_s, FF, my_row, lane & 15, lane >= 32 && lane < 48);
-#endif
-            // the picks' weights for stage F (probability over the sum of the ten, naive.rs:362-376), and what the seam
-            // shows of the route (block 0): lane r of the first wave has pick r
-            if (wave == 0) {
+            // The picks' weights for stage F (probability over the sum of the ten, naive.rs:362-376), and what the seam shows of the
+            // route (block 0), in a wave that neither publishes nor gathers: lane r has pick r.
+            if (wave == 3) {
                 float sum = 0.0f;
 #pragma unroll
-                for (int i = 0; i < CT / 64; i++) sum += route_sh.redf[i];
+                for (int i = 0; i < CW; i++) sum += redf[i];
                 const float prob = lane < NU ? fx_expf(wts[lane] - wts[0]) / sum : 0.0f;
                 float denom = 0.0f;
 #pragma unroll
                 for (int r = 0; r < 16; r++)
                     denom += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, prob), r));
                 denom = fmaxf(denom, 6.103515625e-5f);
+                if (lane == NU) coef[NU] = fx_sigmoid(sm[34]) * f.sh_dscale;   // the shared expert's
                 if (lane < NU) {
                     const int ex = ids[lane];
                     const float w = prob / denom;
@@ -1349,7 +1360,6 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 if (b == 0 && lane == 0 && p.tally)
                     atomicAdd(p.tally, (unsigned long long)((f.counts_gate ? 1 : 0) + (f.counts_up ? 1 : 0) + (f.counts_down ? 1 : 0)) * NU);
             }
-            asm volatile("" ::"v"(touched));
         }
         // the next layer's in-projection rows start moving now: one stage ahead of their use
         CH_STAMP(10);
@@ -1361,18 +1371,20 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             if (l + 1 < p.n_layers && p.layer[l + 1].has_mixer == 3) fetch_tail(p.layer[l + 1].a, aw, b, wave, lane);
             if (next_mixer && ((IT_CHAIN_A_AT >> 4) & 15)) fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane, (IT_CHAIN_A_AT >> 4) & 15);
         };
-        if (!IT_CHAIN_F_POLLERS || wave < 4) fetch_next();
+        if (wave < 4) fetch_next();
 
         // -------------------------------------------------------------------- F: down, combine, residual
         {
-            uint32_t* dst = (uint32_t*)xq;
-            // word i < 1,280 is quad i of the routed quants; the rest are the 160 block scales
-            auto place = [&](int i, uint32_t v) {
-                if (i < NU * FF / 4) dst[i] = v;
-                else xs[i - NU * FF / 4] = __uint_as_float(v);
+            // pair i < 640 of the routed quants: half a sub-block of unit i / 4; the other pairs are the 160 block scales
+            auto place = [&](int i, uint32_t v0, uint32_t v1) {
+                if (i < NU * FF / 8) {
+                    const int u = i >> 2;   // unit u % 16 of pick u / 16
+                    *(uint4*)(xh + (u >> 4) * (FF * 2) + ((i & 3) * 16 + (u & 15)) * 16) = quant_pairs(v0, v1);
+                } else {
+                    *(float2*)(xs + 2 * (i - NU * FF / 8)) = make_float2(__uint_as_float(v0), __uint_as_float(v1));
+                }
             };
             bool ok = true;
-#if IT_CHAIN_F_POLLERS
             // Waves 4..7 gather: the 720 pairs of words of the routed intermediates (quants, then scales) and, waves 4 and
             // 5, the shared ones as quads (whole waves: the quantization's lane exchange needs its eight neighbours).
             if (wave >= 4) {
@@ -1384,42 +1396,25 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                                           wave < 6 ? p.ll + RS + 4 * pt + 2 : p.ll + RE + 2 * (p3 >= 0 ? p3 : pt)};
                 uint32_t o[8];
                 ok = ll_wait_pairs<4>(a4, e, ctl, o);
-                place(2 * pt, o[0]);
-                place(2 * pt + 1, o[1]);
-                place(2 * (pt + 256), o[2]);
-                place(2 * (pt + 256) + 1, o[3]);
+                place(pt, o[0], o[1]);
+                place(pt + 256, o[2], o[3]);
                 if (wave < 6) {
                     const float4 v = make_float4(__uint_as_float(o[4]), __uint_as_float(o[5]), __uint_as_float(o[6]), __uint_as_float(o[7]));
-                    quant_quad(v, true, pt, xq + NU * FF, xs + EB);
-                } else {
-                    place(2 * p2, o[4]);
-                    place(2 * p2 + 1, o[5]);
-                    if (p3 >= 0) {
-                        place(2 * p3, o[6]);
-                        place(2 * p3 + 1, o[7]);
+                    if (SF == W_Q8_0) {
+                        quant_quad(v, true, pt, xq, xs + EB);
+                    } else {
+                        float d;
+                        const uint32_t word = quant_word(v, group_max<8>(quad_amax(v)), &d);
+                        if ((pt & 7) == 0) xs[EB + (pt >> 3)] = it_f16_to_f32(it_f32_to_f16(d));
+                        const uint32_t ahead = word_ahead2(word);
+                        if (!(pt & 2)) *(uint4*)(xh + NU * (FF * 2) + ((((pt >> 1) & 2) + (pt & 1)) * 16 + (pt >> 3)) * 16) = quant_pairs(word, ahead);
                     }
+                } else {
+                    place(p2, o[4], o[5]);
+                    if (p3 >= 0) place(p3, o[6], o[7]);
                 }
                 fetch_next();
             }
-#else
-            // 1,440 words of quantized routed intermediates (pairs tid and tid + 512), the shared ones as quads
-            const int pr1 = tid + CT;
-            const bool two = pr1 < (NU * FF / 4 + EB) / 2, sq = tid < FF / 4;
-            const u64* const a4[4] = {p.ll + RE + 2 * tid, two ? p.ll + RE + 2 * pr1 : p.ll + RE + 2 * tid,
-                                      sq ? p.ll + RS + 4 * tid : p.ll + RE + 2 * tid, sq ? p.ll + RS + 4 * tid + 2 : p.ll + RE + 2 * tid};
-            uint32_t o[8];
-            ok = ll_wait_pairs<4>(a4, e, ctl, o);
-            place(2 * tid, o[0]);
-            place(2 * tid + 1, o[1]);
-            if (two) {
-                place(2 * pr1, o[2]);
-                place(2 * pr1 + 1, o[3]);
-            }
-            if (tid < 2 * 64) {   // whole waves: the quantization's lane exchange needs its eight neighbours
-                const float4 v = make_float4(__uint_as_float(o[4]), __uint_as_float(o[5]), __uint_as_float(o[6]), __uint_as_float(o[7]));
-                quant_quad(v, true, tid, xq + NU * FF, xs + EB);
-            }
-#endif
             if (!ok) dead = 1;
             __syncthreads();
             if (dead) break;
@@ -1430,37 +1425,21 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
 #pragma unroll
             for (int s = 0; s < 3; s++) {
                 const int y = s * 4 + (lane >> 4);
-                if (y < NU) {
-                    const uint4 xa = *(const uint4*)(xq + y * FF + c * 32), xb = *(const uint4*)(xq + y * FF + c * 32 + 16);
-                    float tA, tB;
-                    unit_nvfp4(fd[s].w[0], fd[s].sc[0], xa, xb, xs[y * (FF / 32) + c], &tA, &tB);
-                    float t = 0.0f;
-                    t += tA;
-                    t += tB;
-                    acc += coef[y] * t;
+                if (y < NU + (SF == W_NVFP4 ? 1 : 0)) {
+                    XN x;
+                    load_xn(x, xh + y * (FF * 2), FF / 32, c, xs[y * (FF / 32) + c]);
+                    acc += coef[y] * dot_xn(fd[s], x);
                 }
             }
-            if (lane >= 32) {
-                const float gate = fx_sigmoid(sm[34]) * f.sh_dscale;
-                const WChunks<1>& ws = fsh;
-                if (SF == W_Q8_0) {
-                    const int c2 = lane - 32;
-                    const uint4 xa = *(const uint4*)(xq + NU * FF + c2 * 16);
-                    int s = 0;
-                    s = dot4(ws.w[0].x, xa.x, s);
-                    s = dot4(ws.w[0].y, xa.y, s);
-                    s = dot4(ws.w[0].z, xa.z, s);
-                    s = dot4(ws.w[0].w, xa.w, s);
-                    acc += gate * ((float)s * (it_f16_to_f32((uint16_t)ws.sc[0]) * xs[EB + (c2 >> 1)]));
-                } else if (lane < 48) {
-                    const uint4 xa = *(const uint4*)(xq + NU * FF + c * 32), xb = *(const uint4*)(xq + NU * FF + c * 32 + 16);
-                    float tA, tB;
-                    unit_nvfp4(ws.w[0], ws.sc[0], xa, xb, xs[EB + c], &tA, &tB);
-                    float t = 0.0f;
-                    t += tA;
-                    t += tB;
-                    acc += gate * t;
-                }
+            if (SF == W_Q8_0 && lane >= 32) {
+                const int c2 = lane - 32;
+                const uint4 xa = *(const uint4*)(xq + c2 * 16);
+                int s = 0;
+                s = dot4(fsh.w[0].x, xa.x, s);
+                s = dot4(fsh.w[0].y, xa.y, s);
+                s = dot4(fsh.w[0].z, xa.z, s);
+                s = dot4(fsh.w[0].w, xa.w, s);
+                acc += coef[NU] * ((float)s * (it_f16_to_f32((uint16_t)fsh.sc[0]) * xs[EB + (c2 >> 1)]));
             }
             acc = reduce_lanes<64>(acc);
             if (lane == 63) {
