@@ -457,6 +457,23 @@ IT_DEV bool norm_quant(float4 v, float4 w, float eps, int8_t* xq, float* xs, dou
 // values on the f16 matrix cores (layouts at the loop), softmax bookkeeping a wave per head; a range is a few dozen
 // keys at the contexts this path is measured at, longer ones walk tiles of 64 keys.
 // Merge.  Block b: 16 dims of query head b / 16; thread t: range t / 4, four of the 16 dims.
+// the value of lane ^ 4 (lanes 0..3 and 8..11 of a row of 16 take the one four further on, the others four back), of
+// lane ^ 8, and the sums with lane ^ 16 and ^ 32, without the trip through the LDS crossbar
+IT_DEV float lane_xor4(float v) {
+    const int x = __builtin_bit_cast(int, v), up = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false);   // row_shl:4
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, x, 0x114, 0xf, 0xa, false));               // row_shr:4
+}
+IT_DEV float lane_xor8(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));   // row_ror:8
+}
+IT_DEV float sum_xor16(float v) {
+    const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
+IT_DEV float sum_xor32(float v) {
+    const auto t = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(t[0]) + __uint_as_float(t[1]);
+}
 extern __shared__ __align__(16) uint8_t chain_dyn_lds[];   // ATTN_LDS bytes when a layer of the chain is an attention mixer
 typedef __attribute__((address_space(1))) uint16_t g_u16;
 struct AttnCoreP {   // what of a ChainAttn the function reads
@@ -687,6 +704,7 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
         }
     }
     AC_STAMP(3);   // partial results published
+    WChunks<4> wo;   // the out-projection's row of this wave
     {
         const int h = b >> 4, dc = b & 15;
         const int n_live = (n_pos + kpb - 1) / kpb;   // ranges that hold keys
@@ -696,7 +714,7 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
         // (the gate of this thread's dim, the head's second half of wq's output: published a stage ago; asked for ahead of
         // the ranges' results, whose wait hides the round trip)
         uint32_t gw = 0;
-        if (tid < 16 && !ll_wait1(ll + RQ + h * 2 * HD + HD + dc * 16 + tid, e, ctl, &gw)) ok = false;
+        if (tid < 16 && !ll_wait1<0>(ll + RQ + h * 2 * HD + HD + dc * 16 + tid, e, ctl, &gw)) ok = false;
         if (sp < n_live) {
             const u64* base = ll + RP + (int64_t)(h * AS + sp) * PW;
             const u64* const a4[4] = {base + dc * 16 + q4 * 4, base + dc * 16 + q4 * 4 + 2, base + HD, base + HD};
@@ -710,6 +728,8 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
             }
         }
         AC_STAMP(4);   // the ranges' results gathered
+        // (issued where the ranges' results are in: the polls of the gated output are a merge behind, those of the results would queue)
+        load_row<W_Q8_0, 4, 64>(wo, at.o_q, at.o_s, VDIM, b * CW + wave, lane, true);
         const float mx = group_max<64>(m_s);
         if (lane == 0) sm[wave] = mx;
         __syncthreads();
@@ -720,10 +740,10 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
         float vals[5] = {wgt * o_s.x, wgt * o_s.y, wgt * o_s.z, wgt * o_s.w, wgt * l_s};
 #pragma unroll
         for (int i = 0; i < 5; i++) {
-            vals[i] += __shfl_xor(vals[i], 4, 64);
-            vals[i] += __shfl_xor(vals[i], 8, 64);
-            vals[i] += __shfl_xor(vals[i], 16, 64);
-            vals[i] += __shfl_xor(vals[i], 32, 64);
+            vals[i] += lane_xor4(vals[i]);
+            vals[i] += lane_xor8(vals[i]);
+            vals[i] = sum_xor16(vals[i]);
+            vals[i] = sum_xor32(vals[i]);
         }
         if (lane < 4) {
 #pragma unroll
@@ -746,9 +766,6 @@ __attribute__((noinline)) __device__ AttnCoreR attn_core(it_gptr<const float> q_
     // place: the barriers of the merge are behind every read of it), this wave's row
     float dot;
     {
-        const int my_row = b * CW + wave;
-        WChunks<4> wo;
-        load_row<W_Q8_0, 4, 64>(wo, at.o_q, at.o_s, VDIM, my_row, lane, true);
         int8_t* const oq = (int8_t*)chain_dyn_lds;
         float* const os = (float*)(chain_dyn_lds + NH * HD);
         const u64* const a4[4] = {ll + RT + 4 * tid, ll + RT + 4 * tid + 2, ll + RT + 4 * (tid + CT), ll + RT + 4 * (tid + CT) + 2};
@@ -954,31 +971,29 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                     const float v = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, acc[k]), 63));
                     mine = lane == k ? v : mine;
                 }
-                if (lane < 4) {
-                    // causal conv (kernel 4) + silu on channel `row`, state [channel][3] oldest first
-                    const int64_t row = 32 * b + 4 * wave + lane;
-                    float sum = 0.0f;
-                    sum += aw.past[0] * aw.taps.x;
-                    sum += aw.past[1] * aw.taps.y;
-                    sum += aw.past[2] * aw.taps.z;
-                    sum += mine * aw.taps.w;
-                    ll_putf(p.ll + RA + row, fx_silu(sum), e);
-                    float* past = m.conv_state + row * 3;
-                    past[0] = aw.past[1];
-                    past[1] = aw.past[2];
-                    past[2] = mine;
-                } else if (lane < 6) {
-                    ll_putf(p.ll + RA_Z + 16 * b + 2 * wave + (lane - 4), fx_silu(mine), e);
-                } else if (!RF && lane == 6 && wave == 0 && b < 2 * NV) {
-                    ll_putf(p.ll + RA_AL + b, mine, e);
-                }
+                // causal conv (kernel 4) + silu on channel `row`, state [channel][3] oldest first; silu alone on the z rows
+                const int64_t row = 32 * b + 4 * wave + lane;
+                float sum = 0.0f;
+                sum += aw.past[0] * aw.taps.x;
+                sum += aw.past[1] * aw.taps.y;
+                sum += aw.past[2] * aw.taps.z;
+                sum += mine * aw.taps.w;
+                const float val = fx_silu(lane < 4 ? sum : mine);
+                if (lane < 6) ll_putf(p.ll + (lane < 4 ? RA + 32 * b + 4 * wave : RA_Z + 16 * b + 2 * wave - 4) + lane, val, e);
+                if (!RF && lane == 6 && wave == 0 && b < 2 * NV) ll_putf(p.ll + RA_AL + b, mine, e);
                 if (RF) {
                     // the unquantized alpha / beta row of blocks 0..63 against the normed f32 vector: every wave its 256 floats
                     const float4 xa = ((const float4*)xf)[wave * 64 + lane];
                     const float part = reduce_lanes<64>(f32_chunk(aw.ab, xa));
                     if (lane == 63) fpart[wave] = part;
-                    __syncthreads();
-                    if (tid == 0 && b < 2 * NV) ll_putf(p.ll + RA_AL + b, f32_tree(fpart), e);
+                }
+                if (RF) __syncthreads();
+                if (RF && tid == 0 && b < 2 * NV) ll_putf(p.ll + RA_AL + b, f32_tree(fpart), e);
+                if (lane < 4) {
+                    float* past = m.conv_state + row * 3;
+                    past[0] = aw.past[1];
+                    past[1] = aw.past[2];
+                    past[2] = mine;
                 }
             }
             // ---------------------------------------------------------------- B: delta rule
