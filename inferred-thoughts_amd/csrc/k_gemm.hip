@@ -262,24 +262,28 @@ __global__ __launch_bounds__(256) void q8_tile_k(const int8_t* __restrict__ wq, 
 // ------------------------------------------------------------------ ... and enough of them: 32 x 32 products, 128 rows a block
 // A block owns 128 weight rows x 32 TT tokens; each of its four waves takes 32 rows against all the tokens by MFMA 32x32x32, so a
 // block of 32 k of two tiles is one instruction with a lane's sixteen results behind it.  Lane l supplies 16 k, of its half
-// l / 32, of row (or token) l % 32 and receives D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32], i = 0..15: a token's scale serves a lane's
-// sixteen products, and a row's is read from LDS as f32 with three others.  (Above, two of a lane's twelve operations and half of
-// its LDS reads went into operands that served four products.)  A stage is 128 k and there are two; what of the next one a wave
-// brings is asked for between the products of this one, a request a product.
-// Bound by the three vector operations (convert, scale, add) of every product: 8192 x 2048 over 5,700 tokens 379 us, of which 282
-// remain without loads and stores, 236 without the matrix cores too.  The product of a tile is therefore started before the last
-// tile's is scaled (the compiler alone waited for each), and the outputs go through LDS to be stored 512 bytes a token (32 before: 411).
-// Before, with the 64 x 64 blocks of the kernel above, 563; 4096 x 2048: 270 -> 171; 2048 x 4096: 277 -> 182; 8192 x 2048 over 512:
-// 50 -> 35.  The arithmetic is the same, product by product, in the same order.
+// l / 32, of row (or token) l % 32 and receives D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32], i = 0..15.  The sixteen factors dw * dx are a
+// product of the matrix cores too: both are f16, so that a 32x32x16_f16 with the row's scale and the token's as its one k
+// gives the exact products in the same lanes (operands: one 8-byte read a row and a token a stage, a mask a product).  A
+// stage is 128 k and there are two; what of the next one a wave brings is asked for between the products of this one, a request a
+// product.
+// Bound by the two vector operations (convert, multiply-add; three in exact mode) of every product and the matrix cores' two
+// instructions, which two waves of a SIMD overlap in part: 8192 x 2048 over 5,700 tokens 293 us, of which 271 remain without
+// loads and 250 without the factors' product (312 with the factors on the vector ALU); 4096 x 2048: 163 -> 153; 2048 x 4096: 176 -> 160;
+// 8192 x 2048 over 512 and 1,500: 37.5 -> 36, 94 -> 87.  The product of a tile is started before the last tile's is scaled (the
+// compiler alone waited for each), and the outputs go through LDS to be stored 512 bytes a token.  Where in a unit the factors'
+// product stands, and two or four requests a product, made no difference.  The arithmetic is the CPU path's, product by
+// product, in the same order.
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 constexpr int WIDE_ROWS = 128, WIDE_K = 128;
-template <int TT> constexpr int wide_stage_bytes() { return (WIDE_ROWS + 32 * TT) * (WIDE_K + 16); }
+template <int TT> constexpr int wide_stage_bytes() { return (WIDE_ROWS + 32 * TT) * (WIDE_K + 8); }
 
 template <int TT, bool FMA>
 __global__ __launch_bounds__(256, 2) void q8_wide_k(const int8_t* __restrict__ wq, const uint16_t* __restrict__ ws,
                                                     const int8_t* __restrict__ xq, const float* __restrict__ xs,
                                                     float* __restrict__ out, int n_in, int n_out, int n_tok, float out_scale) {
-    constexpr int STAGE = wide_stage_bytes<TT>(), X_AT = WIDE_ROWS * WIDE_K, WS_AT = X_AT + 32 * TT * WIDE_K, XS_AT = WS_AT + WIDE_ROWS * 16;
+    constexpr int STAGE = wide_stage_bytes<TT>(), X_AT = WIDE_ROWS * WIDE_K, WS_AT = X_AT + 32 * TT * WIDE_K, XS_AT = WS_AT + WIDE_ROWS * 8;
     extern __shared__ __align__(1024) uint8_t tlds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -310,26 +314,20 @@ __global__ __launch_bounds__(256, 2) void q8_wide_k(const int8_t* __restrict__ w
         if (i < 4) to_lds_at(wbase + s * WIDE_K, wo[i & 3], d + (wave * 4 + i) * 1024);
         else to_lds_at(xbase + s * WIDE_K, xo[(i - 4) % TT], d + X_AT + (wave * TT + i - 4) * 1024);
     };
-    float4 sc;
+    uint2 sc;                                     // four blocks' scales, f16
     auto load_scales = [&](int s) __attribute__((always_inline)) {
         if (of_w) {
-            typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
-            const hv4 v = *(const hv4*)(sp + s * 8);
-            sc = make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+            sc = *(const uint2*)(sp + s * 8);
         } else {
-            sc = *(const float4*)(sp + s * 16);
+            typedef _Float16 hv4 __attribute__((ext_vector_type(4)));
+            const float4 v = *(const float4*)(sp + s * 16);       // (f16 values)
+            sc = __builtin_bit_cast(uint2, hv4{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w});
         }
     };
     auto put_scales = [&](int buf) __attribute__((always_inline)) {
-        float* const d = (float*)(tlds + buf * STAGE + (of_w ? WS_AT : XS_AT)) + s_row;
-        const int step = of_w ? WIDE_ROWS : 32 * TT;
-        if (of_w || tid - 128 < 32 * TT) {
-            d[0] = sc.x;
-            d[step] = sc.y;
-            d[2 * step] = sc.z;
-            d[3 * step] = sc.w;
-        }
+        if (of_w || tid - 128 < 32 * TT) *(uint2*)(tlds + buf * STAGE + (of_w ? WS_AT : XS_AT) + 8 * s_row) = sc;
     };
+    const uint32_t lo16 = half ? 0u : 0xffffu, hi16 = half ? 0u : 0xffff0000u;   // lanes of the first half supply k 0 .. 7
     float acc[TT][16];
 #pragma unroll
     for (int tt = 0; tt < TT; tt++)
@@ -352,35 +350,35 @@ __global__ __launch_bounds__(256, 2) void q8_wide_k(const int8_t* __restrict__ w
         // operands are read one unit earlier.
         constexpr int UNITS = 4 * TT;
         v4i a[2], bv[2];
-        float x[2], w[2][16];
         v16i c[2];
+        v16f sp2[2];                              // the scales' products
+        // Block b's scale alone, as k = b of an f16 operand: of this lane's row, or of its token.
+        uint2 ws4, xs4[TT];
+        auto one_scale = [&](uint2 v, int b) __attribute__((always_inline)) {
+            const uint32_t e = (b & 2 ? v.y : v.x) & (b & 1 ? hi16 : lo16);
+            return __builtin_bit_cast(hv8, b & 2 ? make_uint4(0, e, 0, 0) : make_uint4(e, 0, 0, 0));
+        };
         auto read = [&](int u) __attribute__((always_inline)) {
             const int b = u / TT, tt = u % TT, piece = ((2 * b + half) ^ turn) << 4;
             if (tt == 0) a[b & 1] = *(const v4i*)(d + (wave * 32 + c32) * WIDE_K + piece);
             bv[u & 1] = *(const v4i*)(d + X_AT + (tt * 32 + c32) * WIDE_K + piece);
-        };
-        auto read_scales = [&](int u) __attribute__((always_inline)) {
-            const int b = u / TT, tt = u % TT;
-            if (tt == 0) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float4 v = *(const float4*)(d + WS_AT + 4 * (b * WIDE_ROWS + wave * 32 + 8 * i + 4 * half));
-                    w[b & 1][4 * i] = v.x, w[b & 1][4 * i + 1] = v.y, w[b & 1][4 * i + 2] = v.z, w[b & 1][4 * i + 3] = v.w;
-                }
-            }
-            x[u & 1] = *(const float*)(d + XS_AT + 4 * (b * 32 * TT + tt * 32 + c32));
         };
         auto start = [&](int u) __attribute__((always_inline)) {
             v16i z;
 #pragma unroll
             for (int i = 0; i < 16; i++) z[i] = 0;
             c[u & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[(u / TT) & 1], bv[u & 1], z, 0, 0, 0);
+            v16f zf;
+#pragma unroll
+            for (int i = 0; i < 16; i++) zf[i] = 0.0f;
+            sp2[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(one_scale(ws4, u / TT), one_scale(xs4[u % TT], u / TT), zf, 0, 0, 0);
         };
+        ws4 = *(const uint2*)(d + WS_AT + 8 * (wave * 32 + c32));
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++) xs4[tt] = *(const uint2*)(d + XS_AT + 8 * (tt * 32 + c32));
         read(0);
-        read_scales(0);
         start(0);
         read(1);
-        read_scales(1);
 #pragma unroll
         for (int u = 0; u < UNITS; u++) {
             __builtin_amdgcn_sched_barrier(0);
@@ -390,8 +388,8 @@ __global__ __launch_bounds__(256, 2) void q8_wide_k(const int8_t* __restrict__ w
 #pragma unroll
             for (int i = 0; i < 16; i++) {
                 const int tt = u % TT;
-                if (FMA) acc[tt][i] = fmaf((float)c[u & 1][i], w[(u / TT) & 1][i] * x[u & 1], acc[tt][i]);
-                else acc[tt][i] += (float)c[u & 1][i] * (w[(u / TT) & 1][i] * x[u & 1]);
+                if (FMA) acc[tt][i] = fmaf((float)c[u & 1][i], sp2[u & 1][i], acc[tt][i]);
+                else acc[tt][i] += (float)c[u & 1][i] * sp2[u & 1][i];
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -402,7 +400,6 @@ __global__ __launch_bounds__(256, 2) void q8_wide_k(const int8_t* __restrict__ w
                 for (int k = 0; k < PER; k++)
                     if (u * PER + k < 4 + TT) ask(s + 1, buf ^ 1, u * PER + k);
             }
-            if (u + 2 < UNITS) read_scales(u + 2);
         }
     };
     for (int s = 0; s + 1 < n_stage; s++) stage(s, std::true_type{});
