@@ -309,6 +309,13 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
 
     const float e2a = p.scale2 ? p.scale2[e] : p.scale_a;
     const float e2b = GLU ? (p.scale2_up ? p.scale2_up[e] : p.scale_b) : e2a;
+    // The down product's results go through LDS (every read of the slabs is in front of the last barrier), so that a pair's 256 leave
+    // side by side, past the caches that they would fill twice over: 32 of a store's 64 lanes in rows of their own took 113 of 453
+    // us of 5,700 tokens' products over 512 experts, ten a token; 417 so (3,000 tokens 290 -> 271).  Two, four or eight row
+    // blocks of a tile in one pipeline, each one's results stored under the next one's products: 443, 466, 529.
+    constexpr int OSTR = 256 + 4;
+    static_assert(FPAIRS * OSTR * 4 <= 4 * FPAIRS * FBS * 2 + 2 * 256 * (FWS + 16), "");
+    float* const O = (float*)Bh;
 #pragma unroll
     for (int tt = 0; tt < T; tt++) {
         const int slot = 32 * (T * th + tt) + r;
@@ -332,13 +339,20 @@ __device__ __forceinline__ void experts_f16_body(const ExpertsF16P& p, const int
             } else {
 #pragma unroll
                 for (int z = 0; z < 2; z++) {
-                    const int row = rbase[z] + 8 * i4 + 4 * kg;
-                    if (row >= p.n_out) continue;
-                    *(float4*)(p.out + pair * p.n_out + row) =
+                    *(float4*)(O + slot * OSTR + 64 * wave + 32 * z + 8 * i4 + 4 * kg) =
                         make_float4(acc[z][tt][4 * i4] * rsc * e2a, acc[z][tt][4 * i4 + 1] * rsc * e2a,
                                     acc[z][tt][4 * i4 + 2] * rsc * e2a, acc[z][tt][4 * i4 + 3] * rsc * e2a);
                 }
             }
+        }
+    }
+    if (!GLU) {
+        __syncthreads();
+        const int row = row_block * 256 + 4 * lane;
+        if (row < p.n_out) {
+            typedef float fv4 __attribute__((ext_vector_type(4)));
+            for (int slot = wave8; slot < cnt; slot += 8)
+                __builtin_nontemporal_store(*(const fv4*)(O + slot * OSTR + 4 * lane), (fv4*)(p.out + (int64_t)pair_s[slot] * p.n_out + row));
         }
     }
 }
