@@ -349,62 +349,6 @@ IT_DEV void fetch_tail(const T& t, AW& a, int b, int wave, int lane) {
     load_row<W_Q8_0, 2, 64>(a.t[4], kk ? t.k_q : t.v_q, kk ? t.k_s : t.v_s, D, 2 * b + (wave & 1), lane, wave < 4);
 }
 
-// An NVFP4 chunk against the activation through gfx950's own conversions: v_cvt_scalef32_pk_f16_fp4 turns one byte (two
-// e2m1 nibbles) into two f16 and v_dot2_f32_f16 multiplies them with two f16 activations, 2 instructions for 2 elements
-// where nibbles -> int8 through v_perm_b32 + v_dot4 takes 7 for 4.  The activations are the Q8_0 quants as f16 (exact),
-// paired as the nibbles of a byte are (element j with element 8 + j of a 16-element sub-block); every product and sum is
-// a multiple of 0.5 below 2^24, so the f32 accumulation is exact and the result is the integer path's, bit for bit.
-// The sub-block scales come from v_cvt_pk_f32_fp8 (OCP e4m3; the format's ue4m3 is half of that, and the e2m1 values
-// here are half of the integer path's doubled ones: the two factors of 2 cancel; code 0x7f is 0 as in it_ue4m3_to_f32).
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef float f2v __attribute__((ext_vector_type(2)));
-struct XN {
-    uint32_t p[16];   // sub-block A: pairs (j, 8 + j) j = 0..7, then sub-block B
-    float d;
-};
-// In LDS such an activation is four planes, one of each quarter of a 32-element unit's sixteen pairs: unit u's quarter q is
-// 16 bytes at q * (16 * units) + 16 * u, so that the lanes of a load read neighbours.
-IT_DEV void load_xn(XN& x, const uint8_t* xh, int units, int u, float d) {
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        const uint4 t = *(const uint4*)(xh + (q * units + u) * 16);
-        x.p[4 * q] = t.x;
-        x.p[4 * q + 1] = t.y;
-        x.p[4 * q + 2] = t.z;
-        x.p[4 * q + 3] = t.w;
-    }
-    x.d = d;
-}
-// four quants each of elements j .. j + 3 (lo) and 8 + j .. (hi) of a sub-block as f16 pairs, exact: a byte plus 128 in the
-// low bits of 1,024's f16, less 1,152
-IT_DEV uint4 quant_pairs(uint32_t lo, uint32_t hi) {
-    const uint32_t a = lo ^ 0x80808080u, b = hi ^ 0x80808080u;
-    auto pair = [&](uint32_t sel) {
-        const h2v v = __builtin_bit_cast(h2v, __builtin_amdgcn_perm(b, a, sel) | 0x64006400u) - h2v{(_Float16)1152.0f, (_Float16)1152.0f};
-        return __builtin_bit_cast(uint32_t, v);
-    };
-    return make_uint4(pair(0x0c040c00u), pair(0x0c050c01u), pair(0x0c060c02u), pair(0x0c070c03u));
-}
-// the word of the lane two further on in its quad
-IT_DEV uint32_t word_ahead2(uint32_t v) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xee, 0xf, 0xf, true); }   // quad_perm [2, 3, 2, 3]
-#define IT_FP4_STEP(acc, word, sel, pi) \
-    acc = __builtin_amdgcn_fdot2(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(word, 1.0f, sel), __builtin_bit_cast(h2v, x.p[pi]), acc, false)
-IT_DEV float dot_xn(const WChunks<1>& t, const XN& x) {
-    const uint4 w = t.w[0];
-    float sa = 0.0f, sb = 0.0f;
-    IT_FP4_STEP(sa, w.x, 0, 0); IT_FP4_STEP(sa, w.x, 1, 1); IT_FP4_STEP(sa, w.x, 2, 2); IT_FP4_STEP(sa, w.x, 3, 3);
-    IT_FP4_STEP(sa, w.y, 0, 4); IT_FP4_STEP(sa, w.y, 1, 5); IT_FP4_STEP(sa, w.y, 2, 6); IT_FP4_STEP(sa, w.y, 3, 7);
-    IT_FP4_STEP(sb, w.z, 0, 8); IT_FP4_STEP(sb, w.z, 1, 9); IT_FP4_STEP(sb, w.z, 2, 10); IT_FP4_STEP(sb, w.z, 3, 11);
-    IT_FP4_STEP(sb, w.w, 0, 12); IT_FP4_STEP(sb, w.w, 1, 13); IT_FP4_STEP(sb, w.w, 2, 14); IT_FP4_STEP(sb, w.w, 3, 15);
-    const uint32_t sc = t.sc[0] & 0x7f7fu;
-    const f2v s2 = __builtin_amdgcn_cvt_pk_f32_fp8((int)sc, false);
-    const float dA = (sc & 0x7fu) == 0x7fu ? 0.0f : s2.x, dB = (sc >> 8) == 0x7fu ? 0.0f : s2.y;
-    float acc = 0.0f;
-    acc += (x.d * dA) * sa;
-    acc += (x.d * dB) * sb;
-    return acc;
-}
-
 // a float's bits as an unsigned that orders like the value (negative below positive), and back
 IT_DEV uint32_t logit_order(float v) {
     const uint32_t u = __float_as_uint(v);

@@ -471,29 +471,52 @@ struct GluGeo {
     int s_cpl, s_l, s_groups, s_rg;
 };
 
-template <int FMT, int CPL, int L>
-IT_DEV void glu_job(const uint8_t* gq, const uint8_t* gs, const uint8_t* uq, const uint8_t* us, int n_in, int n_out,
-                    int row0, float sg, float su, const int8_t* xq, const float* xs, float* out, int lane,
-                    WChunks<CPL>* tg, WChunks<CPL>* tu, bool loaded) {
-    constexpr int P = 64 / L;
-    constexpr int RB = CPL >= 2 ? 1 : 2;
-    const int sub = lane % L, rsub = lane / L;
-    if (!loaded) {
+// the rows of a group: RB steps of P gate and up rows
+template <int FMT, int CPL, int L> struct GluRows {
+    static constexpr int P = 64 / L, RB = CPL >= 2 ? 1 : 2;
+    WChunks<CPL> g[RB], u[RB];
+    IT_DEV void load(const uint8_t* gq, const uint8_t* gs, const uint8_t* uq, const uint8_t* us, int n_in, int n_out, int row0, int lane) {
 #pragma unroll
         for (int r = 0; r < RB; r++) {
-            const int row = row0 + r * P + rsub;
-            load_w<FMT, CPL, L>(tg[r], gq, gs, n_in, row, sub, row < n_out);
-            load_w<FMT, CPL, L>(tu[r], uq, us, n_in, row, sub, row < n_out);
+            const int row = row0 + r * P + lane / L;
+            load_w<FMT, CPL, L>(g[r], gq, gs, n_in, row, lane % L, row < n_out);
+            load_w<FMT, CPL, L>(u[r], uq, us, n_in, row, lane % L, row < n_out);
         }
     }
+};
+// the lane's part of the activation, in the form that the format's dots take
+template <int FMT, int CPL, int L> struct GluAct {
     XChunks<FMT, CPL> x;
-    load_x<FMT, CPL, L>(x, xq, xs, sub);
+    IT_DEV void load(const int8_t* xq, const float* xs, int lane) { load_x<FMT, CPL, L>(x, xq, xs, lane % L); }
+    IT_DEV float dot(const WChunks<CPL>& t) const { return dot_chunks<FMT, CPL>(t, x); }
+};
+// f16 pairs for the hardware's conversion: half the instructions of a row, same bits, formed once a wave.  (A short batch's
+// launches are bound by what its waves issue as much as by their rows: prompts of 23 and 32 tokens through two layers 714 -> 672
+// and 790 -> 743 us with this and the same in moe_down_fast_k.  The next job's rows asked for ahead of a job's dots cost the third
+// block of a CU and 150 us; several steps of rows a block behind one quantization, in moe_down_fast_k, its fourth for nothing.)
+template <int CPL, int L> struct GluAct<W_NVFP4, CPL, L> {
+    XN x[CPL];
+    IT_DEV void load(const int8_t* xq, const float* xs, int lane) {
+        XChunks<W_NVFP4, CPL> t;
+        load_x<W_NVFP4, CPL, L>(t, xq, xs, lane % L);
 #pragma unroll
-    for (int r = 0; r < RB; r++) {
-        float ag = reduce_lanes<L>(dot_chunks<FMT, CPL>(tg[r], x));
-        float au = reduce_lanes<L>(dot_chunks<FMT, CPL>(tu[r], x));
-        const int row = row0 + r * P + rsub;
-        if (sub == L - 1 && row < n_out) {
+        for (int k = 0; k < CPL; k++) make_xn(x[k], t.a[k], t.b[k], t.d[k]);
+    }
+    IT_DEV float dot(const WChunks<CPL>& t) const {
+        float acc = 0.0f;
+#pragma unroll
+        for (int k = 0; k < CPL; k++) acc = dot_xn_add(acc, t.w[k], t.sc[k], x[k]);
+        return acc;
+    }
+};
+template <int FMT, int CPL, int L>
+IT_DEV void glu_finish(const GluRows<FMT, CPL, L>& t, const GluAct<FMT, CPL, L>& x, int n_out, int row0, float sg, float su, float* out, int lane) {
+#pragma unroll
+    for (int r = 0; r < t.RB; r++) {
+        float ag = reduce_lanes<L>(x.dot(t.g[r]));
+        float au = reduce_lanes<L>(x.dot(t.u[r]));
+        const int row = row0 + r * t.P + lane / L;
+        if (lane % L == L - 1 && row < n_out) {
             ag *= sg;
             au *= su;
             out[row] = fx_silu(ag) * au;
@@ -501,8 +524,9 @@ IT_DEV void glu_job(const uint8_t* gq, const uint8_t* gs, const uint8_t* uq, con
     }
 }
 
+// (three blocks a CU or more; what a wave with shared rows only holds is kept out of the routed loop's registers)
 template <int EF, int ECPL, int EL, int SF, int SCPL, int SL>
-__global__ __launch_bounds__(FT) void moe_glu_fast_k(MoeGluP p, GluGeo gg) {
+__global__ __launch_bounds__(FT, 6) void moe_glu_fast_k(MoeGluP p, GluGeo gg) {
     {   // a short batch: grid row t is token t
         const int64_t t = blockIdx.y;
         p.x += t * p.n_in;
@@ -533,18 +557,11 @@ __global__ __launch_bounds__(FT) void moe_glu_fast_k(MoeGluP p, GluGeo gg) {
     int g = blockIdx.x + wave * gridDim.x;
 
     // a wave whose first job is a shared-expert group knows its rows before the router has run
-    WChunks<SCPL> sg[2], su[2];
-    const bool pre = g >= routed_groups && g < total;
-    if (pre) {
-        constexpr int P = 64 / SL, RB = SCPL >= 2 ? 1 : 2;
-        const int row0 = (g - routed_groups) * gg.s_rg;
-#pragma unroll
-        for (int r = 0; r < RB; r++) {
-            const int row = row0 + r * P + lane / SL;
-            load_w<SF, SCPL, SL>(sg[r], p.sh_gq, p.sh_gs, n_in, row, lane % SL, row < p.sh_n_out);
-            load_w<SF, SCPL, SL>(su[r], p.sh_uq, p.sh_us, n_in, row, lane % SL, row < p.sh_n_out);
-        }
-    }
+    GluRows<SF, SCPL, SL> sh;
+    auto load_shared = [&](GluRows<SF, SCPL, SL>& to, int job) {
+        to.load(p.sh_gq, p.sh_gs, p.sh_uq, p.sh_us, n_in, p.sh_n_out, (job - routed_groups) * gg.s_rg, lane);
+    };
+    if (g >= routed_groups && g < total) load_shared(sh, g);
 
     float logit[4];
     if (p.logits) route_fetch<FT>(p.logits, p.n_expert, logit);
@@ -559,22 +576,36 @@ __global__ __launch_bounds__(FT) void moe_glu_fast_k(MoeGluP p, GluGeo gg) {
         if (tid < p.n_used) ids[tid] = p.route_ids[tid];
         __syncthreads();
     }
-    bool loaded = pre;
-    for (; g < total; g += gstride) {
-        if (g < routed_groups) {
-            const int y = g / gg.e_groups, row0 = (g - y * gg.e_groups) * gg.e_rg;
-            const int64_t e = ids[y];
-            const float scg = p.gscale2 ? p.gscale2[e] : 1.0f, scu = p.uscale2 ? p.uscale2[e] : 1.0f;
-            WChunks<ECPL> tg[2], tu[2];
-            glu_job<EF, ECPL, EL>(p.gq + e * p.q_stride, p.gs + e * p.s_stride, p.uq + e * p.q_stride,
-                                  p.us + e * p.s_stride, n_in, p.n_out, row0, scg, scu, xq, xs,
-                                  p.out + (int64_t)y * p.n_out, lane, tg, tu, false);
-        } else {
-            const int row0 = (g - routed_groups) * gg.s_rg;
-            glu_job<SF, SCPL, SL>(p.sh_gq, p.sh_gs, p.sh_uq, p.sh_us, n_in, p.sh_n_out, row0, p.sh_gscale, p.sh_uscale, xq, xs,
-                                  p.sh_out, lane, sg, su, loaded);
+    // shared-expert groups from g on, the first one's rows loaded
+    auto shared_jobs = [&](GluRows<SF, SCPL, SL>& rows) {
+        GluAct<SF, SCPL, SL> x;
+        for (;;) {
+            x.load(xq, xs, lane);
+            glu_finish<SF, SCPL, SL>(rows, x, p.sh_n_out, (g - routed_groups) * gg.s_rg, p.sh_gscale, p.sh_uscale, p.sh_out, lane);
+            g += gstride;
+            if (g >= total) return;
+            load_shared(rows, g);
         }
-        loaded = false;
+    };
+    if (g >= routed_groups) {
+        if (g < total) shared_jobs(sh);
+        return;
+    }
+    GluAct<EF, ECPL, EL> x;
+    if (EF == W_NVFP4) x.load(xq, xs, lane);
+    for (; g < routed_groups; g += gstride) {
+        const int y = g / gg.e_groups, row0 = (g - y * gg.e_groups) * gg.e_rg;
+        const int64_t e = ids[y];
+        const float scg = p.gscale2 ? p.gscale2[e] : 1.0f, scu = p.uscale2 ? p.uscale2[e] : 1.0f;
+        GluRows<EF, ECPL, EL> rows;
+        rows.load(p.gq + e * p.q_stride, p.gs + e * p.s_stride, p.uq + e * p.q_stride, p.us + e * p.s_stride, n_in, p.n_out, row0, lane);
+        if (EF != W_NVFP4) x.load(xq, xs, lane);   // (behind the rows: held through the loop it would cost a resident block)
+        glu_finish<EF, ECPL, EL>(rows, x, p.n_out, row0, scg, scu, p.out + (int64_t)y * p.n_out, lane);
+    }
+    if (g < total) {
+        GluRows<SF, SCPL, SL> rows;
+        load_shared(rows, g);
+        shared_jobs(rows);
     }
 }
 
@@ -668,7 +699,10 @@ __global__ __launch_bounds__(DT) void moe_down_fast_k(MoeDownP p) {
     const int n_in = p.n_in, sh_in = p.sh_n_in, NU = p.n_used;
     const int total = NU * n_in + sh_in;  // floats staged: picks back to back, then the shared vector
     int8_t* xq = (int8_t*)smem;
-    float* xs = (float*)(smem + ((total + 15) & ~15));
+    // (an NVFP4 matrix's activation as f16 pairs in load_xn's planes, 2 bytes a value; a Q8_0 one's as quants)
+    constexpr bool EH = EF == W_NVFP4, SH = SF == W_NVFP4;
+    uint8_t* const sq = smem + (EH ? 2 : 1) * NU * n_in;                                      // the shared vector's
+    float* xs = (float*)(smem + (((EH ? 2 : 1) * NU * n_in + (SH ? 2 : 1) * sh_in + 15) & ~15));
     __shared__ float coef[MAXU];
     __shared__ float partial[DW / 4][3][64];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -708,7 +742,23 @@ __global__ __launch_bounds__(DT) void moe_down_fast_k(MoeDownP p) {
     IT_STAMP(1);
 
 #pragma unroll
-    for (int k = 0; k < QR; k++) quant_quad(v[k], k * DT + tid < nq, k * DT + tid, xq, xs);
+    for (int k = 0; k < QR; k++) {
+        const int qi = k * DT + tid;
+        float d;
+        const uint32_t word = quant_word(v[k], group_max<8>(quad_amax(v[k])), &d);
+        const uint32_t ahead = word_ahead2(word);
+        if (qi >= nq) continue;
+        const bool shared = qi >= nq_routed;
+        const int q = shared ? qi - nq_routed : qi;
+        if ((qi & 7) == 0) xs[qi >> 3] = it_f16_to_f32(it_f32_to_f16(d));
+        if (shared ? SH : EH) {
+            // (the routed rows' units are a power of two, the lanes of one)
+            const int units = shared ? sh_in >> 5 : L, y = shared ? 0 : (q >> 3) / L, u = (q >> 3) - y * units;
+            if (!(q & 2)) *(uint4*)((shared ? sq : smem + y * n_in * 2) + ((((q >> 1) & 2) + (q & 1)) * units + u) * 16) = quant_pairs(word, ahead);
+        } else {
+            *(uint32_t*)((shared ? (int8_t*)sq : xq) + 4 * q) = word;
+        }
+    }
     IT_STAMP(2);
     __syncthreads();
     IT_STAMP(3);
@@ -718,15 +768,34 @@ __global__ __launch_bounds__(DT) void moe_down_fast_k(MoeDownP p) {
     for (int k = 0; k < QUARTU; k++) {
         const int y = 4 * k + quarter;
         if (y < NU) {
-            XChunks<EF, ECPL> x;
-            load_x<EF, ECPL, L>(x, xq + y * n_in, xs + y * (n_in >> 5), sub);
-            acc += coef[y] * dot_chunks<EF, ECPL>(t[k], x);
+            if (EH) {
+                XN x;
+                load_xn(x, smem + y * n_in * 2, L, sub, xs[y * L + sub]);
+                acc += coef[y] * dot_xn_add(0.0f, t[k].w[0], t[k].sc[0], x);
+                asm volatile("" ::: "memory");   // (one pick's activation at a time: all four would take the registers of a resident block)
+            } else {
+                XChunks<EF, ECPL> x;
+                load_x<EF, ECPL, L>(x, xq + y * n_in, xs + y * (n_in >> 5), sub);
+                acc += coef[y] * dot_chunks<EF, ECPL>(t[k], x);
+            }
         }
     }
     if (quarter == 3) {
-        XChunks<SF, SCPL> x;
-        load_x<SF, SCPL, L>(x, xq + NU * n_in, xs + NU * (n_in >> 5), sub);
-        acc += gate * dot_chunks<SF, SCPL>(tsh, x);
+        if (SH) {
+            float a = 0.0f;
+#pragma unroll
+            for (int k = 0; k < SCPL; k++) {
+                XN x;
+                load_xn(x, sq, sh_in >> 5, k * L + sub, xs[NU * (n_in >> 5) + k * L + sub]);
+                a = dot_xn_add(a, tsh.w[k], tsh.sc[k], x);
+                asm volatile("" ::: "memory");
+            }
+            acc += gate * a;
+        } else {
+            XChunks<SF, SCPL> x;
+            load_x<SF, SCPL, L>(x, (const int8_t*)sq, xs + NU * (n_in >> 5), sub);
+            acc += gate * dot_chunks<SF, SCPL>(tsh, x);
+        }
     }
     IT_STAMP(4);
     acc = reduce_lanes<L>(acc);
@@ -758,7 +827,7 @@ bool moe_down_fast(MoeDownP p, hipStream_t s, bool dry_run) {
         p.s_stride % 2)
         return false;
     const int total = p.n_used * p.n_in + p.sh_n_in;
-    const size_t lds = (size_t)((total + 15) & ~15) + (size_t)(total / 32) * 4;
+    const size_t lds = (((size_t)(p.fmt == W_NVFP4 ? 2 : 1) * p.n_used * p.n_in + (size_t)(p.sh_fmt == W_NVFP4 ? 2 : 1) * p.sh_n_in + 15) & ~(size_t)15) + (size_t)(total / 32) * 4;
     if (lds > 60 * 1024 || total > 3 * DT * 4) return false;
     const int P = 64 / L;
     const int blocks = (p.n_out + (DW / 4) * P - 1) / ((DW / 4) * P);
