@@ -1659,7 +1659,25 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     rec.id = OP_MATMUL; rec.p[0] = v.q; rec.p[1] = v.scales; rec.p[2] = dx; rec.p[3] = as; rec.p[4] = aq; rec.p[5] = dout;
     rec.p[6] = sp.h; rec.p[7] = sp.l; rec.p[8] = sp.scale;
     rec.i[0] = v.fmt; rec.i[1] = v.n_in; rec.i[2] = v.n_out; rec.i[3] = nt; rec.i[4] = tiles;
+    // The output matrix on a batch pass's last row takes the single-token product whether its norm comes in the same launch (fuser.cpp)
+    // or, where a buffer had to grow in between, has been made already: the sums are the same either way.
+    const bool last_row = !exact && n == 1 && be->in_pass && be->pass_tokens > 1 && be->fuse_enabled && (v.fmt == W_Q8_0 || v.fmt == W_NVFP4);
     auto run = [=](hipStream_t s, float scale_by) {
+        if (last_row && scale_by == 1.0f) {
+            FusedGemvP a{};
+            a.x = dx;
+            a.n_in = v.n_in;
+            a.n_mats = 1;
+            a.m[0].q = (const uint8_t*)v.q;
+            a.m[0].s = (const uint8_t*)v.scales;
+            a.m[0].out = dout;
+            a.m[0].n_out = v.n_out;
+            a.m[0].fmt = v.fmt;
+            if (fused_gemv_takes(a)) {
+                fused_gemv(a, s);
+                return;
+            }
+        }
         if (tiles == 1 && experts_gemm_f16s(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
         if (tiles == 2 && experts_gemm_f16(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
         if (int8_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;

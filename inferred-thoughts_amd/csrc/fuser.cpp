@@ -265,11 +265,9 @@ bool match_matmul_residual(Plan& pl, size_t i, int exact) {
     return true;
 }
 
-// last-row gather + final norm + LM head
-bool match_final(Plan& pl, size_t i, int exact) {
-    auto& o = pl.ops;
-    if (!pl.ids(i, {OP_GATHER, OP_RMS, OP_QUANT, OP_MATMUL})) return false;
-    const Op &g = o[i], &rms = o[i + 1], &q = o[i + 2], &m = o[i + 3];
+// last-row gather + final norm + LM head: whether the four ops are that, and as one product
+bool final_head(const Op& g, const Op& rms, const Op& q, const Op& m, int exact, FusedGemvP* out) {
+    if (g.id != OP_GATHER || rms.id != OP_RMS || q.id != OP_QUANT || m.id != OP_MATMUL) return false;
     if (g.i[3] != g.i[0] || rms.p[0] != g.p[1] || rms.i[0] != 1 || rms.i[1] != g.i[0]) return false;
     if (q.p[0] != rms.p[2] || q.i[0] != rms.i[1] || !mm_reads(m, rms.p[2], q)) return false;
     FusedGemvP a{};
@@ -282,7 +280,13 @@ bool match_final(Plan& pl, size_t i, int exact) {
     a.exact = exact;
     a.n_mats = 1;
     a.m[0] = mat_of(m, 0);
-    if (!fused_gemv_takes(a)) return false;
+    *out = a;
+    return fused_gemv_takes(a);
+}
+bool match_final(Plan& pl, size_t i, int exact) {
+    auto& o = pl.ops;
+    FusedGemvP a{};
+    if (!pl.ids(i, {OP_GATHER, OP_RMS, OP_QUANT, OP_MATMUL}) || !final_head(o[i], o[i + 1], o[i + 2], o[i + 3], exact, &a)) return false;
     pl.take(i, 4);
     pl.add(i, it_hip::FAM_LM_HEAD, gemv_bytes(a), [=](hipStream_t s) { fused_gemv(a, s); });
     return true;
@@ -962,6 +966,8 @@ bool references(const Op& op, const void* a, const void* b) {
 //                                                          not written: nothing else in the loop reads them)
 //   RMS_HEADS core, EW silu_mul(z, core), QUANT z        -> gated_norm_silu_q8 (core is left unnormed)
 //   MATMUL, SCALE of its result                          -> the product with the factor in its epilogue
+//   GATHER of the last row, RMS, QUANT, MATMUL of one token -> the single-token product with its own norm (the row's copy
+//                                                          is not written): 23 us in four launches, 8 in one
 //   MATMUL gate, MATMUL up, [SCALE up,] [SCALE gate,] EW silu_mul(gate, up), both NVFP4   -> one gate / up product
 // and the routed FFN of a short batch (2..32 tokens; src/model/qwen35.rs:1630-1700), whose products are held back too:
 //   SOFTMAX, ROUTE, [QUANT x], GLU, QUANT g, EXPERTS, MATMUL shared gate, MATMUL shared up, [SCALE]*, EW silu_mul,
@@ -1025,6 +1031,11 @@ bool it_hip::hold(const OpRec& r) {
     }
     if (held.size() < HELD_MAX) {
         if (small_ffn_enabled && !expert_cold_entries && small_ffn_next(held, r)) return true;
+        if (r.id == OP_MATMUL && r.i[3] == 1 && held.size() >= 3) {   // the output matrix on the last row: with its gather, norm and quantization
+            const OpRec* const h = &held[held.size() - 3];
+            FusedGemvP head{};
+            if (final_head(h[0], h[1], h[2], r, 0, &head)) return true;
+        }
         if (r.id == OP_MATMUL && r.i[4]) {   // a dense matrix on the expert tiles: the shared expert's
             // (behind ops that are not its own it would keep the device waiting for them)
             for (const OpRec& h : held)
@@ -1373,6 +1384,17 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
         p.q_eps = nq.f[0]; p.k_eps = nk.f[0];
         Span sp(this, FAM_ATTN_PREP, span_of(8));
         return attn_rows(p, (int)hd, stream) ? 8 : 0;
+    }
+    // ---- the output matrix on the pass's last row
+    if (a.id == OP_GATHER && i + 4 <= n) {
+        FusedGemvP head{};
+        if (final_head(a, h[i + 1], h[i + 2], h[i + 3], 0, &head) && !used_later(h, i + 4, next, a.p[1]) && !used_later(h, i + 4, next, h[i + 2].p[1])) {
+            Span sp(this, FAM_LM_HEAD, gemv_bytes(head));
+            fused_gemv(head, stream);
+            mark_elided({a.p[1]});
+            if (Act* f = act_by_dev(h[i + 1].p[2])) f->stale();   // (its quants are not made)
+            return 4;
+        }
     }
     // ---- dense products held back
     if (a.id == OP_MATMUL && a.i[4] && id(i + 1) == OP_MATMUL && h[i + 1].i[4] == a.i[4]) {
