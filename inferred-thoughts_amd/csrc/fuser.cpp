@@ -439,7 +439,8 @@ bool match_attn(Plan& pl, size_t i, int exact) {
     return true;
 }
 
-// routed FFN: 17 to 20 ops -> fused_gemv (norm + router + shared gate logit) + moe_glu_fused + moe_down_fused
+// routed FFN: 17 to 20 ops -> fused_gemv (norm + router + shared gate logit) + moe_glu_fused + moe_down_fused, the first two as one
+// launch where moe_route_glu takes them
 bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long long* tally) {
     // With a quantized router the activation is quantized before the router matmul; with an unquantized one
     // (F32 in real files) the first reader of the quantized form is the expert gate/up product, after the route.
@@ -609,13 +610,14 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
                            (uint64_t)(nu * ff + sff) * 4;
     const uint64_t down_b = rows_bytes(d.fmt, (uint64_t)nu * nd, ff) + rows_bytes(d.sh_fmt, nd, sff) +
                             (uint64_t)(nu * ff + sff) * 4 + (uint64_t)nd * 8;
-    {
+    const bool one = moe_route_glu(a, &g);
+    if (!one) {
         auto& la = pl.add(i, it_hip::FAM_FUSED_GEMV, gemv_bytes(a), [=](hipStream_t s) { fused_gemv(a, s); });
         la.stage = Plan::ST_ROUTER;
         la.gv = a;
     }
     {
-        auto& lg = pl.add(i, it_hip::FAM_MOE_GLU, glu_b, [=](hipStream_t s) { moe_glu_fused(g, s); });
+        auto& lg = pl.add(i, it_hip::FAM_MOE_GLU, glu_b + (one ? gemv_bytes(a) : 0), [=](hipStream_t s) { moe_glu_fused(g, s); });
         lg.stage = Plan::ST_GLU;
         lg.mg = g;
     }

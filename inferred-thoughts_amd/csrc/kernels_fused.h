@@ -75,8 +75,16 @@ struct MoeGluP {
     // fast mode, a short batch: token t of n_tok is grid row t, every per-token operand above (x, logits, the picks, out,
     // sh_out) t vectors further on.  0 or 1: one token.
     int n_tok;
+    // exact mode, a router of few rows (norm_w given): every block forms the norm, the logits and the picks itself, `x` is the
+    // residual stream, and block (0, 0) leaves what the router's launch would have
+    const float* norm_w;
+    float eps;
+    const uint8_t *rt_q, *rt_s, *sg_q, *sg_s;   // Q8_0 router, [n_expert][n_in], and shared gate, [n_in]
+    float *normed, *normed2, *logits_out, *sg_out;
 };
 void moe_glu_fused(MoeGluP p, hipStream_t s);
+// the two launches as one: g with what `a` (norm, router, shared gate) does, false: not of that form
+bool moe_route_glu(const FusedGemvP& a, MoeGluP* g);
 
 struct MoeDownP {
     const float* g_all;     // [n_used][n_in]
