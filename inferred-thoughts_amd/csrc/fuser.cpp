@@ -293,8 +293,8 @@ bool match_final(Plan& pl, size_t i, int exact) {
 }
 
 
-// attention mixer: 18 ops -> fused_gemv (norm + wq/wk/wv) + attn_prep + split-K attend with the
-// gate folded into its merge + fused_gemv (wo += x)
+// attention mixer: 18 ops -> fused_gemv (norm + wq/wk/wv) + attend with the gate, the new position's norms, rotation and cache
+// write in it (attn_prep in front where the split kernels do not take those) + fused_gemv (wo += x)
 bool match_attn(Plan& pl, size_t i, int exact) {
     if (!pl.ids(i, {OP_RMS, OP_QUANT, OP_MATMUL, OP_GATHER, OP_GATHER, OP_MATMUL, OP_MATMUL, OP_RMS_HEADS, OP_RMS_HEADS,
                     OP_ROPE, OP_ROPE, OP_KVWRITE, OP_KVWRITE, OP_ATTEND, OP_EW, OP_QUANT, OP_MATMUL, OP_EW}))
@@ -382,6 +382,7 @@ bool match_attn(Plan& pl, size_t i, int exact) {
     b.n_mats = 1;
     b.m[0] = mat_of(mo, 2, (float*)rms.p[0]);
     if (!fused_gemv_takes(a) || !fused_gemv_takes(b)) return false;
+    if (at.i[6] && hd > 4096) return false;   // (attend_exact's LDS: three heads' rows and the scores)
 
     pl.take(i, 18);
     pl.be->fused_attn_slots.push_back(slots);
@@ -423,10 +424,10 @@ bool match_attn(Plan& pl, size_t i, int exact) {
                 be->fail("attend: the split-K kernels could not be launched");
         });
     } else {
-        pl.add(i, it_hip::FAM_ATTN_PREP, (uint64_t)(2 * hd * nh + 2 * kvd) * 4 + kvd * 4, [=](hipStream_t s) { attn_prep(pp, s); });
         AttnArgs ax = aa;
         ax.n_pos = (int)at.i[9];   // what the scratch rows are sized for
-        pl.add(i, it_hip::FAM_ATTEND, kv_bytes, [=](hipStream_t s) { attend_exact(ax, scratch, attn_out, s, gate, gate_stride); });
+        pl.add(i, it_hip::FAM_ATTEND, kv_bytes + (uint64_t)(2 * hd * nh + 2 * kvd) * 4,
+               [=](hipStream_t s) { attend_exact(ax, scratch, attn_out, s, gate, gate_stride, &pp); });
     }
     Plan::Launch& l_out = pl.add(i, it_hip::FAM_FUSED_GEMV, gemv_bytes(b), [=](hipStream_t s) { fused_gemv(b, s); });
     if (three) {   // the form whose in- and out-projection a layer chain may take over

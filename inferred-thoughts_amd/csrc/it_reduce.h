@@ -49,6 +49,13 @@ IT_DEV double dpp_f64(double v, int which) {
     return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
 }
 
+// what a wave's lanes have written to LDS is there for all of them
+IT_DEV void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // sum (or max) over aligned groups of L lanes, L a power of two up to 64; every lane gets the result
 template <int L> IT_DEV float group_sum(float v) {
     if (L >= 2) v += dpp_xor1(v);

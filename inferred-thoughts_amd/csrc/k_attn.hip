@@ -16,6 +16,7 @@
 #include "it_dot.h"
 #include "it_reduce.h"
 #include "kernels.h"
+#include "kernels_fused.h"
 
 namespace itk {
 
@@ -24,10 +25,67 @@ namespace itk {
 // order is a chain: a position's dot in its thread, the weights' sum in one lane, a dim's weighted sum in its thread, each
 // with its loads several steps ahead.  333 positions, 16 heads of 256: 28 us (115 with every read waited for
 // and the weight divided anew for every dim).
+// PREP (one query): the block forms its query head and the new position's key and value from the projections, a wave each, and
+// keeps those in LDS; the first head of a KV head leaves them in the slabs, which no block reads at that position.  As a launch
+// in front (attn_prep) that took 4.6 us, 2.5 of them its start and the projections' trip.  A token of four layers of 512 values,
+// 117.4 -> 115.4 us.
 constexpr int EXACT_LDS = 4096;
-__global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __restrict__ scratch, float* __restrict__ out,
+// head_norm and rotation of one head of `hd` values by one wave, in place in LDS, as attn_prep_k.  The first 256 values' weights
+// and rotations are asked for with the values (a trip to L2 each otherwise).
+IT_DEV void wave_norm_rope(float* h, const float* __restrict__ src, const float* __restrict__ w, int hd, const AttnPrepP& p, int pos, int lane) {
+    constexpr int AHEAD = 4;
+    const int half = p.n_rot / 2;
+    const float2* const rope = p.rope + (int64_t)pos * half;
+    float x[AHEAD], wx[AHEAD];
+    float2 cs[AHEAD / 2];
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+        const int i = lane + 64 * k;
+        x[k] = i < hd ? src[i] : 0.0f;
+        wx[k] = i < hd ? w[i] : 0.0f;
+        if (k < AHEAD / 2) cs[k] = i < half ? rope[i] : make_float2(1.0f, 0.0f);
+    }
+    double part = 0.0;
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+        if (lane + 64 * k < hd) h[lane + 64 * k] = x[k];
+        part += (double)(x[k] * x[k]);
+    }
+    for (int i = lane + 64 * AHEAD; i < hd; i += 64) {
+        const float v = src[i];
+        h[i] = v;
+        part += (double)(v * v);
+    }
+    const double sum = __shfl(wave_sum_f64_tail(part), 63, 64);
+    wave_lds_sync();
+    float mean;
+    if (!mean_is_certain(sum, hd, hd, &mean)) {   // (the same answer in every lane)
+        double serial = 0.0;
+        for (int i = 0; i < hd; i++) serial += (double)(h[i] * h[i]);
+        mean = (float)over(serial, hd);
+    }
+    const float scale = 1.0f / sqrtf(mean + p.eps);
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+        if (lane + 64 * k < hd) h[lane + 64 * k] = x[k] * scale * wx[k];
+    for (int i = lane + 64 * AHEAD; i < hd; i += 64) h[i] = h[i] * scale * w[i];
+    wave_lds_sync();
+    auto turn = [&](int i, float2 r) __attribute__((always_inline)) {
+        const float x0 = h[i], x1 = h[i + half];
+        h[i] = x0 * r.x - x1 * r.y;
+        h[i + half] = x0 * r.y + x1 * r.x;
+    };
+#pragma unroll
+    for (int k = 0; k < AHEAD / 2; k++)
+        if (lane + 64 * k < half) turn(lane + 64 * k, cs[k]);
+    for (int i = lane + 32 * AHEAD; i < half; i += 64) turn(i, rope[i]);
+    wave_lds_sync();
+}
+template <bool PREP>
+__global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, AttnPrepP pr, float* __restrict__ scratch, float* __restrict__ out,
                                                       const float* __restrict__ gate, int gate_stride, int lds_pos) {
-    extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each)
+    extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each), then PREP's key and value
     __shared__ float red[17];
     __shared__ uint64_t etab[32];   // (a lookup in constant memory is a trip to L2)
     const int hd = a.head_dim, tid = threadIdx.x, nt = blockDim.x;
@@ -42,10 +100,41 @@ __global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __rest
     float* near = qs + ((hd + 3) & ~3);
     float* far = scratch + (int64_t)blockIdx.x * n_pos_last;
     auto score = [&](int s) -> float& { return s < lds_pos ? near[s] : far[s]; };
-    for (int i = tid; i < hd; i += nt) qs[i] = q[i];
+    const int n_slab = PREP ? n_pos - 1 : n_pos;   // positions read from the slabs
+    float* const fresh = near + lds_pos;           // the new position's key, then its value
+    if constexpr (PREP) {
+        const int wave = tid >> 6, lane = tid & 63, pos = n_pos - 1;
+        const bool leaves = h % group == 0;
+        if (wave == 0) {
+            wave_norm_rope(qs, pr.qg + (int64_t)h * 2 * hd, pr.q_norm, hd, pr, pos, lane);
+            for (int i = lane; i < hd; i += 64) pr.q[(int64_t)h * hd + i] = qs[i];
+        } else if (wave == 1) {
+            wave_norm_rope(fresh, pr.k + off, pr.k_norm, hd, pr, pos, lane);
+            for (int i = lane; i < hd; i += 64) {
+                const uint16_t v = it_f32_to_f16(fresh[i]);
+                fresh[i] = it_f16_to_f32(v);
+                if (leaves) pr.k_slab[(int64_t)pos * a.kv_dim + off + i] = v;
+            }
+        } else if (wave == 2) {
+            for (int i = lane; i < hd; i += 64) {
+                const uint16_t v = it_f32_to_f16(pr.v[off + i]);
+                fresh[hd + i] = it_f16_to_f32(v);
+                if (leaves) pr.v_slab[(int64_t)pos * a.kv_dim + off + i] = v;
+            }
+        }
+    } else {
+        for (int i = tid; i < hd; i += nt) qs[i] = q[i];
+    }
     __syncthreads();
     float m = -INFINITY;
-    for (int s = tid; s < n_pos; s += nt) {
+    if (PREP && tid == nt - 1) {                   // (of the wave with the fewest positions of its own)
+        float dot = 0.0f;
+#pragma unroll 8
+        for (int i = 0; i < hd; i++) dot += qs[i] * fresh[i];
+        m = dot * a.scale;
+        score(n_slab) = m;
+    }
+    for (int s = tid; s < n_slab; s += nt) {
         const uint16_t* key = a.k + (int64_t)s * a.kv_dim + off;
         float dot = 0.0f;
         auto add8 = [&](int i, uint4 kk) {
@@ -100,42 +189,46 @@ __global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __rest
         const uint16_t* v = a.v + off + i;
         float acc = 0.0f;
         int s = 0;
+        const int n_near = min(n_slab, lds_pos);
         constexpr int AHEAD = 32;   // positions whose values are on their way while as many are added
         uint16_t x0[AHEAD], x1[AHEAD];
         auto ask = [&](uint16_t (&x)[AHEAD], int from) __attribute__((always_inline)) {
 #pragma unroll
-            for (int c = 0; c < AHEAD; c++) x[c] = v[(int64_t)min(from + c, n_pos - 1) * a.kv_dim];
+            for (int c = 0; c < AHEAD; c++) x[c] = v[(int64_t)min(from + c, n_slab - 1) * a.kv_dim];
         };
         auto add = [&](const uint16_t (&x)[AHEAD], int from) __attribute__((always_inline)) {
 #pragma unroll
             for (int c = 0; c < AHEAD; c++) acc += near[from + c] * it_f16_to_f32(x[c]);
         };
-        if (n_lds >= AHEAD) ask(x0, 0);
-        for (; s + 2 * AHEAD <= n_lds; s += 2 * AHEAD) {
+        if (n_near >= AHEAD) ask(x0, 0);
+        for (; s + 2 * AHEAD <= n_near; s += 2 * AHEAD) {
             ask(x1, s + AHEAD);
             add(x0, s);
             ask(x0, s + 2 * AHEAD);
             add(x1, s + AHEAD);
         }
-        if (s + AHEAD <= n_lds) {
+        if (s + AHEAD <= n_near) {
             add(x0, s);
             s += AHEAD;
         }
-        for (; s < n_lds; s++) acc += near[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
+        for (; s < n_near; s++) acc += near[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
 #pragma unroll 8
-        for (s = lds_pos; s < n_pos; s++) acc += far[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
+        for (s = lds_pos; s < n_slab; s++) acc += far[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
+        if (PREP) acc += score(n_slab) * fresh[hd + i];
         if (gate) acc *= it_sigmoid(gate[(int64_t)h * gate_stride + i]);   // (n_q == 1: sigmoid_mul of the gated block)
         out[((int64_t)t * a.n_head + h) * hd + i] = acc;
     }
 }
 
-void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate, int gate_stride) {
+void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate, int gate_stride, const AttnPrepP* prep) {
     if (a.n_q <= 0) return;
     const int lds_pos = std::min((a.n_pos + 3) & ~3, EXACT_LDS);
     // few blocks: a thread per position while the score phase has that many; many: blocks that share a CU
     const int threads = a.n_q * a.n_head < 512 && a.n_pos > 256 ? 1024 : 256;
-    hipLaunchKernelGGL(attend_exact_k, dim3(a.n_q * a.n_head), dim3(threads), ((size_t)((a.head_dim + 3) & ~3) + lds_pos) * sizeof(float), s, a,
-                       scratch, out, gate, gate_stride, lds_pos);
+    const size_t lds = ((size_t)((a.head_dim + 3) & ~3) + lds_pos + (prep ? 2 * a.head_dim : 0)) * sizeof(float);
+    const dim3 grid(a.n_q * a.n_head), block(threads);
+    if (prep) hipLaunchKernelGGL(attend_exact_k<true>, grid, block, lds, s, a, *prep, scratch, out, gate, gate_stride, lds_pos);
+    else hipLaunchKernelGGL(attend_exact_k<false>, grid, block, lds, s, a, AttnPrepP{}, scratch, out, gate, gate_stride, lds_pos);
 }
 
 // ------------------------------------------------------------------ split-K

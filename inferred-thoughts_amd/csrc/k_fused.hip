@@ -71,12 +71,6 @@ IT_DEV void quantize_quad(float4 v, uint32_t* packed, float* scale) {
     *scale = it_f16_to_f32(it_f32_to_f16(d));
 }
 
-IT_DEV void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // Terms of `nrows` rows starting at `row0` of one matrix against the LDS activation.
 // Two phases so every HBM load of the group is in flight before the first dot: a lane
 // owns IPL (row, 32-element unit) items, loads them all, then computes.

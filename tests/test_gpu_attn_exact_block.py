@@ -1,0 +1,74 @@
+"""A single-token attention block of exact mode, recorded and replayed with the new position's norms, rotation and cache rows formed
+by the attention kernel itself, against the CPU oracle bit for bit: contexts across its loops' edges, the scores' place in LDS, one
+to eight query heads a KV head."""
+import numpy as np
+import pytest
+
+from test_gpu_fused_fast import Both, bufs
+from util import f16_bits, rng
+
+pytestmark = pytest.mark.gpu
+ND, EPS, THETA, PASSES = 256, 1e-6, 1e7, 9
+
+
+@pytest.mark.parametrize("nh,nkv,hd,n_rot,n_ctx,pos0", [
+    (8, 1, 64, 32, 512, 0),          # the first positions: nothing in the slabs
+    (8, 1, 64, 64, 512, 29),         # 32 positions, a whole step of the weighted sum
+    (4, 2, 256, 64, 300, 61),
+    (6, 2, 96, 48, 256, 247),        # 256 threads, up to the last position of the slab
+    (2, 2, 128, 128, 1200, 1020),    # 1,024 threads; the last has a position of its own beside the new one
+    (4, 4, 8, 4, 4200, 4093),        # scores past LDS
+    (2, 1, 320, 272, 64, 31),        # more values and rotations than a wave asks for ahead
+])
+def test_block(nh, nkv, hd, n_rot, n_ctx, pos0):
+    import inferred_hip as ih
+    from oracle import binding as ob
+    hip = ih.Hip(exact=True)
+    pair = Both(hip, ob.Oracle(threads=8))
+    orc = pair.orc
+    qd, kd = nh * hd, nkv * hd
+    r = rng(hd + pos0)
+    wq, wk, wv, wo = pair.q8(r, 2 * qd, ND, 2.0), pair.q8(r, kd, ND, 2.0), pair.q8(r, kd, ND, 2.0), pair.q8(r, ND, qd, 8.0)
+    norm_w, qn, kn = [(0.5 + r.random(n)).astype(np.float32) for n in (ND, hd, hd)]
+    B = bufs(x=ND, normed=ND, qg=2 * qd, q=qd, g=qd, k=kd, v=kd, attn=qd, mixed=ND)
+    k0, v0 = f16_bits(r.standard_normal(n_ctx * kd)), f16_bits(r.standard_normal(n_ctx * kd))
+    k0[pos0 * kd:] = 0
+    v0[pos0 * kd:] = 0
+    slabs = [dict(k=k0.copy(), v=v0.copy()) for _ in range(2)]
+    sc = float(1.0 / np.sqrt(np.float32(hd)))
+
+    def block(ops, i, b, s, pos):
+        W = lambda t: t[i]
+        ops.rms_norm(b["x"], norm_w, EPS, b["normed"])
+        ops.matmul(W(wq), b["normed"], b["qg"])
+        ops.gather_chunks(b["qg"], hd, 2 * hd, 0, b["q"]); ops.gather_chunks(b["qg"], hd, 2 * hd, hd, b["g"])
+        ops.matmul(W(wk), b["normed"], b["k"]); ops.matmul(W(wv), b["normed"], b["v"])
+        ops.rms_norm_heads(b["q"], qn, hd, EPS); ops.rms_norm_heads(b["k"], kn, hd, EPS)
+        ops.rope_neox(b["q"], pos, hd, n_rot, nh, THETA); ops.rope_neox(b["k"], pos, hd, n_rot, nkv, THETA)
+        ops.kv_write(s["k"], pos * kd, b["k"]); ops.kv_write(s["v"], pos * kd, b["v"])
+        ops.attend(b["q"], s["k"], s["v"], kd, pos + 1, hd, nh, nkv, sc, b["attn"])
+        ops.sigmoid_mul(b["attn"], b["g"])
+        ops.matmul(W(wo), b["attn"], b["mixed"])
+        ops.add_assign(b["x"], b["mixed"])
+
+    try:
+        for p in range(PASSES):              # two op by op, one recorded (again, where the scratch has grown), the rest replayed
+            pos = pos0 + p
+            x0 = rng(500 + p).standard_normal(ND).astype(np.float32)
+            for b in B:
+                b["x"][:] = x0
+            hip.begin_pass(1); hip.host_wrote(B[0]["x"]); block(hip, 0, B[0], slabs[0], pos); hip.end_pass()
+            for name in ("x", "attn", "q"):
+                hip.host_needs(B[0][name])
+            hip.read_kv(slabs[0]["k"]); hip.read_kv(slabs[0]["v"])
+            hip.raise_if_error()
+            block(orc, 1, B[1], slabs[1], pos)
+            for name in ("x", "attn", "q"):
+                assert np.array_equal(B[0][name].view(np.uint32), B[1][name].view(np.uint32)), (p, name)
+            for t in "kv":
+                assert np.array_equal(slabs[0][t], slabs[1][t]), (p, t)
+        g = hip.graph_stats()
+        assert g["captures"] == 1 and g["replays"] >= 1 and g["graph_kernels"] == 3, g
+    finally:
+        hip.take_error()
+        hip.close()
