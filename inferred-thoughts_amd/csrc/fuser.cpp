@@ -503,7 +503,7 @@ bool match_ffn(Plan& pl, size_t i, int exact, unsigned* counter, unsigned long l
     if (sm.p[0] != router || sm.i[0] != 1 || sm.i[1] != ne) return false;
     if (rt.p[0] != router || rt.i[0] != 1 || rt.i[1] != ne) return false;
     int64_t nu = rt.i[2];
-    if (nu > 16 || ne > nd || ne > 2048 || !counter) return false;   // (ROUTE_MAX_EXPERTS)
+    if (nu > 16 || ne > nd || ne > 2048 || !counter) return false;   // (what a block ranks: four experts a thread, 16 picks)
     if (glu.p[6] != rt.p[1] || glu.p[7] != q1.p[1] || glu.p[8] != q1.p[2] || glu.i[1] != nd || glu.i[3] != nu ||
         glu.i[4] != nu || !quantized_fmt(glu.i[0]))
         return false;

@@ -314,8 +314,11 @@ __device__ __forceinline__ void route_fetch(const float* logits, int n_expert, f
     }
 }
 
-template <int THREADS>
-__device__ __forceinline__ float block_route(const float l[4], int n_expert, int n_used, RouteLds<THREADS>& sh, int* ids, float* wts) {
+// EXACT: the CPU path's exponentials (etab: their table, in LDS) and its sum in the order of the experts (terms: n_expert floats of
+// LDS, 16-byte aligned), a chain of eight cycles an expert in one wave.
+template <int THREADS, bool EXACT = false>
+__device__ __forceinline__ float block_route(const float l[4], int n_expert, int n_used, RouteLds<THREADS>& sh, int* ids, float* wts,
+                                             const uint64_t* etab = nullptr, float* terms = nullptr) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr int NW = THREADS / 64;
     const int K = (n_expert + THREADS - 1) / THREADS;  // experts per thread that can be live
@@ -334,21 +337,34 @@ __device__ __forceinline__ float block_route(const float l[4], int n_expert, int
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int e = tid + k * THREADS;
-        v[k] = (k < K && e < n_expert) ? fx_expf(l[k] - m) : 0.0f;
-        part += v[k];
+        if constexpr (EXACT) {
+            if (k >= K) break;
+            v[k] = it_expf_by(l[k] - m, etab);
+            if (e < n_expert) terms[e] = v[k];
+        } else {
+            v[k] = (k < K && e < n_expert) ? fx_expf(l[k] - m) : 0.0f;
+            part += v[k];
+        }
     }
-    part = group_sum_tail<64>(part);
-    if (lane == 63) sh.redf[NW + wave] = part;
-    __syncthreads();
     float sum = 0.0f;
+    if constexpr (EXACT) {
+        __syncthreads();
+        if (wave == 0) sh.redf[NW] = fold_terms(terms, n_expert);   // (every lane: the same reads)
+        __syncthreads();
+        sum = sh.redf[NW];
+    } else {
+        part = group_sum_tail<64>(part);
+        if (lane == 63) sh.redf[NW + wave] = part;
+        __syncthreads();
 #pragma unroll
-    for (int i = 0; i < NW; i++) sum += sh.redf[NW + i];
+        for (int i = 0; i < NW; i++) sum += sh.redf[NW + i];
+    }
     unsigned long long key[4];
     unsigned largest = 0;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int e = tid + k * THREADS;
-        v[k] = v[k] / sum;
+        if (!EXACT || k < K) v[k] = v[k] / sum;
         key[k] = (k < K && e < n_expert) ? route_key(v[k], e) : 0ull;
         largest = max(largest, (unsigned)(key[k] >> 32));
     }

@@ -16,6 +16,7 @@
 #include <algorithm>
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_fast.h"
 #include "it_launch.h"
 #include "it_reduce.h"
 #include "kernels.h"
@@ -161,62 +162,31 @@ __device__ void wave_row_terms(const uint8_t* wq, const uint8_t* ws, int n_in, i
 // prologue modes: 0 = the activation as is; 1 = rms_norm(x, norm_w); 2 = per-head
 // rms_norm of x (weight norm_w[head_dim]) gated by silu(gate): silu(g) * ((x*scale)*w)
 // ------------------------------------------------------------------ router in one wave
-// softmax over all experts, then n_used rounds of arg-max with ties to the lower id, the
+// softmax over up to 64 experts, then n_used rounds of arg-max with ties to the lower id, the
 // picked probabilities summed in pick order (src/ops/mod.rs:1191-1216, naive.rs:362-376).
-// Called by one wave; probs (LDS, n_expert floats) holds the logits on entry.  A lane keeps its NE probabilities (experts
-// lane + 64 i) in registers; a round is one reduction over the wave for the value and a ballot per register for the lowest id that has it.
-template <int NE>
-__device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane, const uint64_t* etab) {
-    float v[NE];
-    float m = -INFINITY;
-#pragma unroll
-    for (int i = 0; i < NE; i++) {
-        const int e = lane + 64 * i;
-        v[i] = e < n_expert ? probs[e] : -INFINITY;
-        m = fmaxf(m, v[i]);
-    }
-    m = group_max<64>(m);
-    float part = 0.0f;
-#pragma unroll
-    for (int i = 0; i < NE; i++) {
-        const int e = lane + 64 * i;
-        v[i] = e < n_expert ? it_expf_by(v[i] - m, etab) : -1.0f;
-        if (e < n_expert) {
-            probs[e] = v[i];
-            part += v[i];
-        }
-    }
+// Called by one wave; probs (LDS, n_expert floats) holds the logits on entry.  Lane e keeps expert e's probability; a round is one
+// reduction over the wave for the value and a ballot for the lowest id that has it.
+__device__ void wave_route(float* probs, int n_expert, int n_used, int* ids, float* weights, int lane, const uint64_t* etab) {
+    const bool live = lane < n_expert;
+    float v = live ? probs[lane] : -INFINITY;
+    const float m = group_max<64>(v);
+    v = live ? it_expf_by(v - m, etab) : -1.0f;
+    if (live) probs[lane] = v;
     wave_lds_sync();
-    float sum;
-    if (exact) {
-        sum = fold_terms(probs, n_expert);   // (every lane: the same reads)
-    } else {
-        for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
-        sum = part;
-    }
-#pragma unroll
-    for (int i = 0; i < NE; i++)
-        if (lane + 64 * i < n_expert) v[i] = v[i] / sum;
+    const float sum = fold_terms(probs, n_expert);   // (every lane: the same reads)
+    if (live) v = v / sum;
     float picked_p = 0.0f;  // lane r keeps pick r's probability
     int picked_id = -1;
     for (int r = 0; r < n_used; r++) {
-        float best = v[0];
-#pragma unroll
-        for (int i = 1; i < NE; i++) best = fmaxf(best, v[i]);
-        best = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, group_max_tail<64>(best)), 63));
+        const float best = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, group_max_tail<64>(v)), 63));
         int id = best >= 0.0f ? -1 : r;   // (probabilities that are not numbers: some expert)
-#pragma unroll
-        for (int i = 0; i < NE; i++) {    // taken and absent experts hold -1
-            const unsigned long long has = __ballot(v[i] == best);
-            if (id < 0 && has) id = 64 * i + __builtin_ctzll(has);
-        }
+        const unsigned long long has = __ballot(v == best);   // taken and absent experts hold -1
+        if (id < 0 && has) id = __builtin_ctzll(has);
         if (lane == r) {
             picked_p = best;
             picked_id = id;
         }
-#pragma unroll
-        for (int i = 0; i < NE; i++)
-            if (lane + 64 * i == id) v[i] = -1.0f;
+        if (lane == id) v = -1.0f;
     }
     // sum in pick order, serial f32
     float s = 0.0f;
@@ -228,12 +198,9 @@ __device__ void wave_route_n(float* probs, int n_expert, int n_used, int exact, 
     }
     wave_lds_sync();
 }
-constexpr int ROUTE_MAX_EXPERTS = 2048, ROUTE_ITEMS = 4;
-__device__ void wave_route(float* probs, int n_expert, int n_used, int exact, int* ids, float* weights, int lane, const uint64_t* etab) {
-    if (n_expert <= 64) wave_route_n<1>(probs, n_expert, n_used, exact, ids, weights, lane, etab);
-    else if (n_expert <= 512) wave_route_n<8>(probs, n_expert, n_used, exact, ids, weights, lane, etab);
-    else wave_route_n<32>(probs, n_expert, n_used, exact, ids, weights, lane, etab);   // up to ROUTE_MAX_EXPERTS (match_ffn)
-}
+constexpr int ROUTE_ITEMS = 4;
+// LDS of the exponentials of a route by a whole block
+__host__ IT_DEV size_t route_terms(int n_expert) { return ((size_t)n_expert * 4 + 15) & ~(size_t)15; }
 
 constexpr int FG_THREADS = 512, FG_LDS_MAX = 128 * 1024, FG_MAX_IN = 8 * 64 * 32;
 
@@ -518,20 +485,24 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         }
         __syncthreads();
         if (is_last) {
-            float* probs = xf;  // n_expert <= n_in (checked on the host)
-            for (int i = tid; i < p.n_expert; i += FG_THREADS)
-                probs[i] = __hip_atomic_load(p.route_logits + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __syncthreads();
-            if (wave == 0) {
-                __shared__ int rids[64];
-                __shared__ float rwts[64];
-                wave_route(probs, p.n_expert, p.n_used, p.exact, rids, rwts, lane, etab);
-                if (lane < p.n_used) {
-                    p.route_ids[lane] = rids[lane];
-                    p.route_w[lane] = rwts[lane];
-                }
-                if (lane == 0) *p.route_counter = 0u;
+            // By the whole block: 512 experts took one wave 10.9 us (exponentials eight a lane, ten rounds of arg-max over
+            // eight registers), this 3.5.  (The activation and the terms are done with: their LDS holds the experts' exponentials and the
+            // pick's candidates.)
+            __shared__ int rids[16];
+            __shared__ __align__(16) float rwts[16];
+            auto& sh = *(fastk::RouteLds<FG_THREADS>*)(smem + route_terms(p.n_expert));
+            float l[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int e = tid + k * FG_THREADS;
+                l[k] = e < p.n_expert ? __hip_atomic_load(p.route_logits + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -INFINITY;
             }
+            const float denom = fastk::block_route<FG_THREADS, true>(l, p.n_expert, p.n_used, sh, rids, rwts, etab, (float*)smem);
+            if (tid < p.n_used) {
+                p.route_ids[tid] = rids[tid];
+                p.route_w[tid] = rwts[tid] / denom;
+            }
+            if (tid == 0) *p.route_counter = 0u;
         }
     }
 }
@@ -596,7 +567,8 @@ void fused_gemv(FusedGemvP p, hipStream_t s) {
     const int f_blocks = nf ? std::min(p.total_frows, std::max(256 - p.q_blocks, (p.total_frows + W - 1) / W)) : 0;
     const int f_waves = nf ? std::min(W, (p.total_frows + f_blocks - 1) / f_blocks) : 0;
     const int blocks = std::max(1, p.q_blocks + f_blocks);
-    const size_t lds = std::max(nq ? fg_lds(p.n_in, R) : fg_base(p.n_in), fg_base(p.n_in) + (size_t)f_waves * p.n_in * 4);
+    size_t lds = std::max(nq ? fg_lds(p.n_in, R) : fg_base(p.n_in), fg_base(p.n_in) + (size_t)f_waves * p.n_in * 4);
+    if (p.route_counter) lds = std::max(lds, route_terms(p.n_expert) + sizeof(fastk::RouteLds<FG_THREADS>));
     auto launch = [&](auto kernel) {
         if (lds > 64 * 1024) (void)lds_allowed<decltype(kernel)::value>(FG_LDS_MAX);   // (refused: the launch reports it)
         hipLaunchKernelGGL(decltype(kernel)::value, dim3(blocks), dim3(FG_THREADS), lds, s, p);
@@ -926,7 +898,7 @@ __global__ __launch_bounds__(256) void moe_glu_fused_k(MoeGluP p) {
                     if (first) *(lane < p.n_expert ? p.logits_out + lane : p.sg_out) = dot;
                 }
                 wave_lds_sync();
-                wave_route_n<1>(logits, p.n_expert, p.n_used, 1, ids, wts, lane, etab);
+                wave_route(logits, p.n_expert, p.n_used, ids, wts, lane, etab);
                 if (first && lane < p.n_used) {
                     p.route_ids_out[lane] = ids[lane];
                     p.route_w_out[lane] = wts[lane];

@@ -1,5 +1,5 @@
-"""Exact mode's routed FFN with few experts: the norm, the router and the shared gate formed by every block of the expert
-gate / up launch, on both sides of the sizes that takes, against the CPU oracle bit for bit."""
+"""Exact mode's routed FFN: with few experts the norm, the router and the shared gate formed by every block of the expert
+gate / up launch, on both sides of the sizes that takes, else the picks by a whole block, against the CPU oracle bit for bit."""
 import numpy as np
 import pytest
 
@@ -19,8 +19,11 @@ pytestmark = pytest.mark.gpu
     (992, 8, 1008 + 16, 32, 3, 2),  # 64 x 4 blocks: one a CU; threads without a quad
     (992, 8, 1024 + 32, 32, 3, 3),
     (1056, 8, 64, 64, 2, 3),        # more than a quad a thread
+    (544, 512, 32, 32, 10, 3),      # the picks by the router's last block, an expert a thread
+    (544, 513, 32, 32, 16, 3),      # and more
+    (1056, 1040, 32, 32, 10, 3),    # (the last pass: equal keys, all of them candidates)
 ])
-def test_few_experts(nd, ne, ff, sff, nu, kernels):
+def test_routed_block(nd, ne, ff, sff, nu, kernels):
     import inferred_hip as ih
     from oracle import binding as ob
     hip = ih.Hip(exact=True)
