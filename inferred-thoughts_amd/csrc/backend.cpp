@@ -1784,7 +1784,8 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
     const uint64_t n_pos_cap = (be->exact || !split_ok ? graphed : by_slab) ? slab_rows : a->n_pos;
     uint64_t bytes = a->n_pos * a->n_head_kv * a->head_dim * 4 + a->q_len * 8;
     if (be->exact || !split_ok) {
-        float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap));
+        // (one query: a row of scores for each 64 dims of a head, as attend_exact_one may leave)
+        float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap) * (n_q == 1 ? (a->head_dim + 63) / 64 : 1));
         if (!sc) return;
         const int* dyn = be->dyn_slot((int)a->n_pos, {(int)n_q, (int)std::min<uint64_t>(slab_rows, INT32_MAX)});
         AttnArgs args{dq, dk, dv, (int)n_q, (int)a->kv_dim, dyn ? (int)n_pos_cap : (int)a->n_pos, (int)a->head_dim,

@@ -382,7 +382,6 @@ bool match_attn(Plan& pl, size_t i, int exact) {
     b.n_mats = 1;
     b.m[0] = mat_of(mo, 2, (float*)rms.p[0]);
     if (!fused_gemv_takes(a) || !fused_gemv_takes(b)) return false;
-    if (at.i[6] && hd > 4096) return false;   // (attend_exact's LDS: three heads' rows and the scores)
 
     pl.take(i, 18);
     pl.be->fused_attn_slots.push_back(slots);
@@ -426,8 +425,14 @@ bool match_attn(Plan& pl, size_t i, int exact) {
     } else {
         AttnArgs ax = aa;
         ax.n_pos = (int)at.i[9];   // what the scratch rows are sized for
-        pl.add(i, it_hip::FAM_ATTEND, kv_bytes + (uint64_t)(2 * hd * nh + 2 * kvd) * 4,
-               [=](hipStream_t s) { attend_exact(ax, scratch, attn_out, s, gate, gate_stride, &pp); });
+        if (exact && attend_exact_one(ax, pp, scratch, attn_out, gate, gate_stride, nullptr, true)) {
+            pl.add(i, it_hip::FAM_ATTEND, kv_bytes + (uint64_t)(2 * hd * nh + 2 * kvd) * 4, [=](hipStream_t s) {
+                if (!attend_exact_one(ax, pp, scratch, attn_out, gate, gate_stride, s, false)) be->fail("attend: not launched");
+            });
+        } else {
+            pl.add(i, it_hip::FAM_ATTN_PREP, (uint64_t)(2 * hd * nh + 2 * kvd) * 4 + kvd * 4, [=](hipStream_t s) { attn_prep(pp, s); });
+            pl.add(i, it_hip::FAM_ATTEND, kv_bytes, [=](hipStream_t s) { attend_exact(ax, scratch, attn_out, s, gate, gate_stride); });
+        }
     }
     Plan::Launch& l_out = pl.add(i, it_hip::FAM_FUSED_GEMV, gemv_bytes(b), [=](hipStream_t s) { fused_gemv(b, s); });
     if (three) {   // the form whose in- and out-projection a layer chain may take over

@@ -14,6 +14,7 @@
 #include <algorithm>
 #include "it_device.h"
 #include "it_dot.h"
+#include "it_launch.h"
 #include "it_reduce.h"
 #include "kernels.h"
 #include "kernels_fused.h"
@@ -25,67 +26,10 @@ namespace itk {
 // order is a chain: a position's dot in its thread, the weights' sum in one lane, a dim's weighted sum in its thread, each
 // with its loads several steps ahead.  333 positions, 16 heads of 256: 28 us (115 with every read waited for
 // and the weight divided anew for every dim).
-// PREP (one query): the block forms its query head and the new position's key and value from the projections, a wave each, and
-// keeps those in LDS; the first head of a KV head leaves them in the slabs, which no block reads at that position.  As a launch
-// in front (attn_prep) that took 4.6 us, 2.5 of them its start and the projections' trip.  A token of four layers of 512 values,
-// 117.4 -> 115.4 us.
 constexpr int EXACT_LDS = 4096;
-// head_norm and rotation of one head of `hd` values by one wave, in place in LDS, as attn_prep_k.  The first 256 values' weights
-// and rotations are asked for with the values (a trip to L2 each otherwise).
-IT_DEV void wave_norm_rope(float* h, const float* __restrict__ src, const float* __restrict__ w, int hd, const AttnPrepP& p, int pos, int lane) {
-    constexpr int AHEAD = 4;
-    const int half = p.n_rot / 2;
-    const float2* const rope = p.rope + (int64_t)pos * half;
-    float x[AHEAD], wx[AHEAD];
-    float2 cs[AHEAD / 2];
-#pragma unroll
-    for (int k = 0; k < AHEAD; k++) {
-        const int i = lane + 64 * k;
-        x[k] = i < hd ? src[i] : 0.0f;
-        wx[k] = i < hd ? w[i] : 0.0f;
-        if (k < AHEAD / 2) cs[k] = i < half ? rope[i] : make_float2(1.0f, 0.0f);
-    }
-    double part = 0.0;
-#pragma unroll
-    for (int k = 0; k < AHEAD; k++) {
-        if (lane + 64 * k < hd) h[lane + 64 * k] = x[k];
-        part += (double)(x[k] * x[k]);
-    }
-    for (int i = lane + 64 * AHEAD; i < hd; i += 64) {
-        const float v = src[i];
-        h[i] = v;
-        part += (double)(v * v);
-    }
-    const double sum = __shfl(wave_sum_f64_tail(part), 63, 64);
-    wave_lds_sync();
-    float mean;
-    if (!mean_is_certain(sum, hd, hd, &mean)) {   // (the same answer in every lane)
-        double serial = 0.0;
-        for (int i = 0; i < hd; i++) serial += (double)(h[i] * h[i]);
-        mean = (float)over(serial, hd);
-    }
-    const float scale = 1.0f / sqrtf(mean + p.eps);
-    wave_lds_sync();
-#pragma unroll
-    for (int k = 0; k < AHEAD; k++)
-        if (lane + 64 * k < hd) h[lane + 64 * k] = x[k] * scale * wx[k];
-    for (int i = lane + 64 * AHEAD; i < hd; i += 64) h[i] = h[i] * scale * w[i];
-    wave_lds_sync();
-    auto turn = [&](int i, float2 r) __attribute__((always_inline)) {
-        const float x0 = h[i], x1 = h[i + half];
-        h[i] = x0 * r.x - x1 * r.y;
-        h[i + half] = x0 * r.y + x1 * r.x;
-    };
-#pragma unroll
-    for (int k = 0; k < AHEAD / 2; k++)
-        if (lane + 64 * k < half) turn(lane + 64 * k, cs[k]);
-    for (int i = lane + 32 * AHEAD; i < half; i += 64) turn(i, rope[i]);
-    wave_lds_sync();
-}
-template <bool PREP>
-__global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, AttnPrepP pr, float* __restrict__ scratch, float* __restrict__ out,
+__global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, float* __restrict__ scratch, float* __restrict__ out,
                                                       const float* __restrict__ gate, int gate_stride, int lds_pos) {
-    extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each), then PREP's key and value
+    extern __shared__ __align__(16) float qs[];  // head_dim, then the first lds_pos scores (a multiple of 4 each)
     __shared__ float red[17];
     __shared__ uint64_t etab[32];   // (a lookup in constant memory is a trip to L2)
     const int hd = a.head_dim, tid = threadIdx.x, nt = blockDim.x;
@@ -100,41 +44,10 @@ __global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, AttnPrepP pr,
     float* near = qs + ((hd + 3) & ~3);
     float* far = scratch + (int64_t)blockIdx.x * n_pos_last;
     auto score = [&](int s) -> float& { return s < lds_pos ? near[s] : far[s]; };
-    const int n_slab = PREP ? n_pos - 1 : n_pos;   // positions read from the slabs
-    float* const fresh = near + lds_pos;           // the new position's key, then its value
-    if constexpr (PREP) {
-        const int wave = tid >> 6, lane = tid & 63, pos = n_pos - 1;
-        const bool leaves = h % group == 0;
-        if (wave == 0) {
-            wave_norm_rope(qs, pr.qg + (int64_t)h * 2 * hd, pr.q_norm, hd, pr, pos, lane);
-            for (int i = lane; i < hd; i += 64) pr.q[(int64_t)h * hd + i] = qs[i];
-        } else if (wave == 1) {
-            wave_norm_rope(fresh, pr.k + off, pr.k_norm, hd, pr, pos, lane);
-            for (int i = lane; i < hd; i += 64) {
-                const uint16_t v = it_f32_to_f16(fresh[i]);
-                fresh[i] = it_f16_to_f32(v);
-                if (leaves) pr.k_slab[(int64_t)pos * a.kv_dim + off + i] = v;
-            }
-        } else if (wave == 2) {
-            for (int i = lane; i < hd; i += 64) {
-                const uint16_t v = it_f32_to_f16(pr.v[off + i]);
-                fresh[hd + i] = it_f16_to_f32(v);
-                if (leaves) pr.v_slab[(int64_t)pos * a.kv_dim + off + i] = v;
-            }
-        }
-    } else {
-        for (int i = tid; i < hd; i += nt) qs[i] = q[i];
-    }
+    for (int i = tid; i < hd; i += nt) qs[i] = q[i];
     __syncthreads();
     float m = -INFINITY;
-    if (PREP && tid == nt - 1) {                   // (of the wave with the fewest positions of its own)
-        float dot = 0.0f;
-#pragma unroll 8
-        for (int i = 0; i < hd; i++) dot += qs[i] * fresh[i];
-        m = dot * a.scale;
-        score(n_slab) = m;
-    }
-    for (int s = tid; s < n_slab; s += nt) {
+    for (int s = tid; s < n_pos; s += nt) {
         const uint16_t* key = a.k + (int64_t)s * a.kv_dim + off;
         float dot = 0.0f;
         auto add8 = [&](int i, uint4 kk) {
@@ -189,46 +102,347 @@ __global__ __launch_bounds__(1024) void attend_exact_k(AttnArgs a, AttnPrepP pr,
         const uint16_t* v = a.v + off + i;
         float acc = 0.0f;
         int s = 0;
-        const int n_near = min(n_slab, lds_pos);
         constexpr int AHEAD = 32;   // positions whose values are on their way while as many are added
         uint16_t x0[AHEAD], x1[AHEAD];
         auto ask = [&](uint16_t (&x)[AHEAD], int from) __attribute__((always_inline)) {
 #pragma unroll
-            for (int c = 0; c < AHEAD; c++) x[c] = v[(int64_t)min(from + c, n_slab - 1) * a.kv_dim];
+            for (int c = 0; c < AHEAD; c++) x[c] = v[(int64_t)min(from + c, n_pos - 1) * a.kv_dim];
         };
         auto add = [&](const uint16_t (&x)[AHEAD], int from) __attribute__((always_inline)) {
 #pragma unroll
             for (int c = 0; c < AHEAD; c++) acc += near[from + c] * it_f16_to_f32(x[c]);
         };
-        if (n_near >= AHEAD) ask(x0, 0);
-        for (; s + 2 * AHEAD <= n_near; s += 2 * AHEAD) {
+        if (n_lds >= AHEAD) ask(x0, 0);
+        for (; s + 2 * AHEAD <= n_lds; s += 2 * AHEAD) {
             ask(x1, s + AHEAD);
             add(x0, s);
             ask(x0, s + 2 * AHEAD);
             add(x1, s + AHEAD);
         }
-        if (s + AHEAD <= n_near) {
+        if (s + AHEAD <= n_lds) {
             add(x0, s);
             s += AHEAD;
         }
-        for (; s < n_near; s++) acc += near[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
+        for (; s < n_lds; s++) acc += near[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
 #pragma unroll 8
-        for (s = lds_pos; s < n_slab; s++) acc += far[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
-        if (PREP) acc += score(n_slab) * fresh[hd + i];
+        for (s = lds_pos; s < n_pos; s++) acc += far[s] * it_f16_to_f32(v[(int64_t)s * a.kv_dim]);
         if (gate) acc *= it_sigmoid(gate[(int64_t)h * gate_stride + i]);   // (n_q == 1: sigmoid_mul of the gated block)
         out[((int64_t)t * a.n_head + h) * hd + i] = acc;
     }
 }
 
-void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate, int gate_stride, const AttnPrepP* prep) {
+void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate, int gate_stride) {
     if (a.n_q <= 0) return;
     const int lds_pos = std::min((a.n_pos + 3) & ~3, EXACT_LDS);
     // few blocks: a thread per position while the score phase has that many; many: blocks that share a CU
     const int threads = a.n_q * a.n_head < 512 && a.n_pos > 256 ? 1024 : 256;
-    const size_t lds = ((size_t)((a.head_dim + 3) & ~3) + lds_pos + (prep ? 2 * a.head_dim : 0)) * sizeof(float);
-    const dim3 grid(a.n_q * a.n_head), block(threads);
-    if (prep) hipLaunchKernelGGL(attend_exact_k<true>, grid, block, lds, s, a, *prep, scratch, out, gate, gate_stride, lds_pos);
-    else hipLaunchKernelGGL(attend_exact_k<false>, grid, block, lds, s, a, AttnPrepP{}, scratch, out, gate, gate_stride, lds_pos);
+    hipLaunchKernelGGL(attend_exact_k, dim3(a.n_q * a.n_head), dim3(threads), ((size_t)((a.head_dim + 3) & ~3) + lds_pos) * sizeof(float), s, a,
+                       scratch, out, gate, gate_stride, lds_pos);
+}
+
+// ------------------------------------------------------------------ exact, one query
+// A recorded token's: a block per head and 64 dims of its result forms the query and the new position's key and value from the
+// projections, a wave each, and keeps the new rows in LDS; the first block of a KV head leaves them in the slabs, which no block reads
+// at that position.  (A launch in front took 4.6 us for that, 2.5 of them its start and the projections' trip.)
+// The chains are attend_exact_k's; what bounded them there were 16-byte reads of rows a KV stride apart, a line a lane, values two
+// bytes at a time, and what one CU is served (174 KB of keys in 3 us, as much of values in 6).  So a wave brings 64 keys' rows 64 dims
+// at a time, whole lines, through a piece of LDS of its own (rows 144 bytes apart: no bank conflicts), the next piece in registers
+// meanwhile; a block brings its 64 dims of 512 values while the weights are formed, all threads form the products, and one wave adds
+// them up.  340 positions, 16 heads of 256: 27.3 -> 15.1 us (22.5 with all dims in a block); a token of four layers of 512 values,
+// 33 to 290 positions, 8 heads of 64: 115.7 -> 112.0 us.
+constexpr int ONE_DIMS = 64, ONE_T = 512, ONE_ROW = 144, ONE_V = 8;      // threads; bytes of a key's piece in LDS; 16-byte pieces of values a thread brings
+constexpr int ONE_VALUES = ONE_T * ONE_V * 16, ONE_STAGE = 2 * ONE_VALUES;   // (as f32 products)
+static_assert(ONE_T * ONE_ROW <= ONE_STAGE, "the keys' pieces lie where the values go later");
+// head_norm and rotation of one head of `hd` values by one wave, in place in LDS, as attn_prep_k.  The first 256 values' weights
+// and rotations are asked for with the values (a trip to L2 each otherwise).
+IT_DEV void wave_norm_rope(float* h, const float* __restrict__ src, const float* __restrict__ w, int hd, const AttnPrepP& p, int pos, int lane) {
+    constexpr int AHEAD = 4;
+    const int half = p.n_rot / 2;
+    const float2* const rope = p.rope + (int64_t)pos * half;
+    float x[AHEAD], wx[AHEAD];
+    float2 cs[AHEAD / 2];
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+        const int i = lane + 64 * k;
+        x[k] = i < hd ? src[i] : 0.0f;
+        wx[k] = i < hd ? w[i] : 0.0f;
+        if (k < AHEAD / 2) cs[k] = i < half ? rope[i] : make_float2(1.0f, 0.0f);
+    }
+    double part = 0.0;
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++) {
+        if (lane + 64 * k < hd) h[lane + 64 * k] = x[k];
+        part += (double)(x[k] * x[k]);
+    }
+    for (int i = lane + 64 * AHEAD; i < hd; i += 64) {
+        const float v = src[i];
+        h[i] = v;
+        part += (double)(v * v);
+    }
+    const double sum = __shfl(wave_sum_f64_tail(part), 63, 64);
+    wave_lds_sync();
+    float mean;
+    if (!mean_is_certain(sum, hd, hd, &mean)) {   // (the same answer in every lane)
+        double serial = 0.0;
+        for (int i = 0; i < hd; i++) serial += (double)(h[i] * h[i]);
+        mean = (float)over(serial, hd);
+    }
+    const float scale = 1.0f / sqrtf(mean + p.eps);
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < AHEAD; k++)
+        if (lane + 64 * k < hd) h[lane + 64 * k] = x[k] * scale * wx[k];
+    for (int i = lane + 64 * AHEAD; i < hd; i += 64) h[i] = h[i] * scale * w[i];
+    wave_lds_sync();
+    auto turn = [&](int i, float2 r) __attribute__((always_inline)) {
+        const float x0 = h[i], x1 = h[i + half];
+        h[i] = x0 * r.x - x1 * r.y;
+        h[i + half] = x0 * r.y + x1 * r.x;
+    };
+#pragma unroll
+    for (int k = 0; k < AHEAD / 2; k++)
+        if (lane + 64 * k < half) turn(lane + 64 * k, cs[k]);
+    for (int i = lane + 32 * AHEAD; i < half; i += 64) turn(i, rope[i]);
+    wave_lds_sync();
+}
+// a lane's value, in a scalar register; and its product with a half of `h`, rounded once as a product of f32 is (what is added to
+// nothing is never -0: a sum that starts at 0 cannot tell the sign of a zero)
+IT_DEV float lane_value(float v, int lane) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane)); }
+template <bool HIGH, bool SCALAR>   // SCALAR: `s` is the same in every lane
+IT_DEV float times_half(float s, uint32_t h) {
+    float r;
+    if constexpr (SCALAR) {
+        if constexpr (HIGH) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "s"(s), "v"(h));
+        else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(r) : "s"(s), "v"(h));
+    } else {
+        if constexpr (HIGH) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(r) : "v"(s), "v"(h));
+        else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(r) : "v"(s), "v"(h));
+    }
+    return r;
+}
+template <int HD>
+__global__ __launch_bounds__(ONE_T) void attend_exact_one_k(AttnArgs a, AttnPrepP pr, float* __restrict__ scratch, float* __restrict__ out,
+                                                            const float* __restrict__ gate, int gate_stride, int lds_pos) {
+    extern __shared__ __align__(16) uint8_t one_smem[];   // ONE_STAGE bytes, then the query, the new key and value, and lds_pos scores
+    __shared__ float red[ONE_T / 64 + 1];
+    __shared__ uint64_t etab[32];
+    constexpr int hd = HD, NP = HD / 64;             // pieces of a key
+    constexpr int pv = ONE_DIMS / 8, rows = ONE_VALUES / 2 / ONE_DIMS;   // 16-byte pieces of a row of values, rows brought at a time
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint8_t* const lds = one_smem;
+    float* const qs = (float*)(lds + ONE_STAGE);
+    float* const fresh = qs + hd;                    // key, value
+    float* const near = fresh + 2 * hd;
+    const int n_pos = *a.n_pos_dyn, pos = n_pos - 1, n_lds = min(n_pos, lds_pos);   // positions 0 .. pos - 1 are read from the slabs
+    const int h = blockIdx.x, group = a.n_head / a.n_head_kv, off = h / group * hd, d0 = ONE_DIMS * blockIdx.y;   // the block's dims of the result
+    float* const far = scratch + (int64_t)(blockIdx.y * gridDim.x + h) * n_pos;
+    // (LDS and memory by separate instructions: through a pointer to either, a read waits for all that is on its way)
+    auto put = [&](int s, float v) __attribute__((always_inline)) {
+        if (s < lds_pos) near[s] = v;
+        asm volatile("");
+        if (s >= lds_pos) far[s] = v;
+    };
+    if (tid < 32) etab[tid] = IT_EXP2F_TAB[tid];
+
+    // ---- scores: step `it` of a wave is piece it % NP of positions 64 wave + 512 (it / NP) ..
+    const int steps = pos > 64 * wave ? (pos - 64 * wave + ONE_T - 1) / ONE_T * NP : 0;
+    uint8_t* const piece = lds + wave * 64 * ONE_ROW;
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));   // (arrays of uint4 were left in memory)
+    u4 kk[8] = {};
+    auto ask_k = [&](int base, int p) __attribute__((always_inline)) {
+        const uint16_t* const from = a.k + off + 64 * p + 8 * (lane & 7);
+#pragma unroll
+        for (int j = 0; j < 8; j++) kk[j] = *(const u4*)(from + (int64_t)min(base + 8 * j + (lane >> 3), pos - 1) * a.kv_dim);
+    };
+    if (steps) ask_k(64 * wave, 0);
+    {
+        const bool first = d0 == 0, leaves = first && h % group == 0;
+        if (wave == 0) {
+            wave_norm_rope(qs, pr.qg + (int64_t)h * 2 * hd, pr.q_norm, hd, pr, pos, lane);
+            if (first)
+                for (int i = lane; i < hd; i += 64) pr.q[(int64_t)h * hd + i] = qs[i];
+        } else if (wave == 1) {
+            wave_norm_rope(fresh, pr.k + off, pr.k_norm, hd, pr, pos, lane);
+            for (int i = lane; i < hd; i += 64) {
+                const uint16_t v = it_f32_to_f16(fresh[i]);
+                fresh[i] = it_f16_to_f32(v);
+                if (leaves) pr.k_slab[(int64_t)pos * a.kv_dim + off + i] = v;
+            }
+        } else if (wave == 2) {
+            for (int i = lane; i < hd; i += 64) {
+                const uint16_t v = it_f32_to_f16(pr.v[off + i]);
+                fresh[hd + i] = it_f16_to_f32(v);
+                if (leaves) pr.v_slab[(int64_t)pos * a.kv_dim + off + i] = v;
+            }
+        }
+    }
+    __syncthreads();
+    float m = -INFINITY;
+    if (tid == ONE_T - 1) {                          // (of the wave with the fewest positions of its own)
+        float dot = 0.0f;
+#pragma unroll 8
+        for (int i = 0; i < hd; i++) dot += qs[i] * fresh[i];
+        m = dot * a.scale;
+        put(pos, m);
+    }
+    // products are formed eight ahead of their addition, and the scalar they take two ahead of them (each waits some eight cycles
+    // for the one before it; the zeros in front add nothing)
+    float dot = 0.0f, due[8] = {};
+    for (int it = 0, base = 64 * wave, p = 0; it < steps; it++) {
+#pragma unroll
+        for (int j = 0; j < 8; j++) *(u4*)(piece + (8 * j + (lane >> 3)) * ONE_ROW + 16 * (lane & 7)) = kk[j];
+        wave_lds_sync();
+        const float q = qs[64 * p + lane];
+        const int s = base + lane;
+        const bool whole = ++p == NP;
+        if (whole) {
+            p = 0;
+            base += ONE_T;
+        }
+        if (it + 1 < steps) ask_k(base, p);
+        const uint8_t* const row = piece + lane * ONE_ROW;
+        u4 x[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) x[j] = *(const u4*)(row + 16 * j);
+        float s0 = lane_value(q, 0), s1 = lane_value(q, 1);
+#pragma unroll
+        for (int e = 0; e < 64; e++) {
+            const float s2 = lane_value(q, min(e + 2, 63));
+            dot += due[e % 8];
+            const uint32_t pair = x[e / 8][e / 2 % 4];
+            due[e % 8] = e & 1 ? times_half<true, true>(s0, pair) : times_half<false, true>(s0, pair);
+            s0 = s1;
+            s1 = s2;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        wave_lds_sync();
+        if (whole) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                dot += due[e];
+                due[e] = 0.0f;
+            }
+            const float v = dot * a.scale;
+            dot = 0.0f;
+            if (s < pos) {
+                put(s, v);
+                m = fmaxf(m, v);
+            }
+        }
+    }
+    // ---- the first values, while the weights are formed
+    u4 vv[ONE_V] = {};
+    auto ask_v = [&](int row0) __attribute__((always_inline)) {
+        const uint16_t* const from = a.v + off + d0 + 8 * (tid % pv);
+#pragma unroll
+        for (int j = 0; j < ONE_V; j++) {
+            if (row0 + ONE_T / pv * j >= pos) break;
+            vv[j] = *(const u4*)(from + (int64_t)min(row0 + tid / pv + ONE_T / pv * j, pos - 1) * a.kv_dim);
+        }
+    };
+    if (pos) ask_v(0);
+    m = group_max<64>(m);
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int w = 1; w < ONE_T / 64; w++) m = fmaxf(m, red[w]);
+    for (int s = tid; s < n_lds; s += ONE_T) near[s] = it_expf_by(near[s] - m, etab);
+    for (int s = lds_pos + tid; s < n_pos; s += ONE_T) far[s] = it_expf_by(far[s] - m, etab);
+    __threadfence_block();
+    __syncthreads();
+    if (wave == 0) {   // (every lane: reads of one address by all cost less than by one lane)
+        float sum = fold_terms(near, n_lds);
+#pragma unroll 16
+        for (int s = lds_pos; s < n_pos; s++) sum += far[s];
+        red[ONE_T / 64] = sum;
+    }
+    __syncthreads();
+    const float sum = red[ONE_T / 64];
+    for (int s = tid; s < n_lds; s += ONE_T) near[s] = near[s] / sum;
+    for (int s = lds_pos + tid; s < n_pos; s += ONE_T) far[s] = far[s] / sum;
+    __threadfence_block();
+
+    // ---- the weighted sum: every thread forms the products of what it has brought, the first wave adds them up, a dim a lane.
+    // Products lie [dim][row]; which four rows lie where is turned by the dim, so that eight rows of eight dims (written at once) and
+    // four rows of sixteen dims (read at once) hit different banks.
+    float* const prod = (float*)lds;
+    auto turn = [](int d) __attribute__((always_inline)) { return 2 * (((d >> 3) ^ d) & 7) | ((d >> 3) & 1); };
+    float acc = 0.0f;
+    for (int row0 = 0; row0 < pos; row0 += rows) {
+        __syncthreads();                             // (the weights are there; the products before have been read)
+        float w[ONE_V];
+        static_assert(EXACT_LDS % rows == 0, "all of a piece's weights in LDS, or none");
+        if (row0 < lds_pos) {
+#pragma unroll
+            for (int j = 0; j < ONE_V; j++) w[j] = near[min(row0 + tid / pv + ONE_T / pv * j, pos)];
+        } else {
+#pragma unroll
+            for (int j = 0; j < ONE_V; j++) w[j] = far[min(row0 + tid / pv + ONE_T / pv * j, pos)];
+        }
+#pragma unroll
+        for (int j = 0; j < ONE_V; j++) {
+            const int r = tid / pv + ONE_T / pv * j, s = row0 + r;
+            if (row0 + ONE_T / pv * j >= pos) break;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const int d = 8 * (tid % pv) + e;
+                const uint32_t pair = vv[j][e / 2];
+                const float x = e & 1 ? times_half<true, false>(w[j], pair) : times_half<false, false>(w[j], pair);
+                prod[d * rows + 4 * ((r >> 2) ^ turn(d)) + (r & 3)] = s < pos ? x : 0.0f;   // (0 adds nothing)
+            }
+        }
+        if (row0 + rows < pos) ask_v(row0 + rows);
+        __syncthreads();
+        if (wave) continue;
+        constexpr int AHEAD = 8;                     // times four rows, on their way while as many are added
+        const float4* const p = (const float4*)(prod + lane * rows);
+        const int n4 = (min(rows, pos - row0) + 4 * AHEAD - 1) / (4 * AHEAD) * AHEAD, t = turn(lane);
+        float4 x0[AHEAD], x1[AHEAD];
+        auto get = [&](float4 (&x)[AHEAD], int r4) __attribute__((always_inline)) {
+#pragma unroll
+            for (int c = 0; c < AHEAD; c++) x[c] = p[min(r4 + c, rows / 4 - 1) ^ t];
+        };
+        auto add = [&](const float4 (&x)[AHEAD]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int c = 0; c < AHEAD; c++) {
+                acc += x[c].x;
+                acc += x[c].y;
+                acc += x[c].z;
+                acc += x[c].w;
+            }
+        };
+        get(x0, 0);
+        int r4 = 0;
+        for (; r4 + 2 * AHEAD <= n4; r4 += 2 * AHEAD) {
+            get(x1, r4 + AHEAD);
+            add(x0);
+            get(x0, r4 + 2 * AHEAD);
+            add(x1);
+        }
+        if (r4 < n4) add(x0);
+    }
+    if (!pos) __syncthreads();                       // (the new position's weight)
+    if (tid < ONE_DIMS) {
+        acc += (pos < lds_pos ? near[pos] : far[pos]) * fresh[hd + d0 + tid];
+        if (gate) acc *= it_sigmoid(gate[(int64_t)h * gate_stride + d0 + tid]);   // (sigmoid_mul of the gated block)
+        out[(int64_t)h * hd + d0 + tid] = acc;
+    }
+}
+
+template <int HD>
+static bool one_launch(const AttnArgs& a, const AttnPrepP& prep, float* scratch, float* out, const float* gate, int gate_stride, hipStream_t s, bool dry_run) {
+    auto lds = [](int lds_pos) { return ONE_STAGE + (size_t)(3 * HD + lds_pos) * sizeof(float); };
+    const int lds_pos = std::min((a.n_pos + 3) & ~3, EXACT_LDS);
+    if (!lds_allowed<&attend_exact_one_k<HD>>(lds(EXACT_LDS))) return false;
+    if (!dry_run) hipLaunchKernelGGL(attend_exact_one_k<HD>, dim3(a.n_head, HD / ONE_DIMS), dim3(ONE_T), lds(lds_pos), s, a, prep, scratch, out, gate, gate_stride, lds_pos);
+    return true;
+}
+bool attend_exact_one(const AttnArgs& a, const AttnPrepP& prep, float* scratch, float* out, const float* gate, int gate_stride, hipStream_t s, bool dry_run) {
+    if (a.n_q != 1 || !a.n_pos_dyn || a.kv_dim % 8 || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15)) return false;
+    if (a.head_dim == 64) return one_launch<64>(a, prep, scratch, out, gate, gate_stride, s, dry_run);
+    if (a.head_dim == 128) return one_launch<128>(a, prep, scratch, out, gate, gate_stride, s, dry_run);
+    return a.head_dim == 256 && one_launch<256>(a, prep, scratch, out, gate, gate_stride, s, dry_run);
 }
 
 // ------------------------------------------------------------------ split-K

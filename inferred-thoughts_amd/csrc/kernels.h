@@ -262,10 +262,10 @@ struct AttnArgs {
 };
 // exact: the oracle's order (scores, serial softmax sum, positions outermost).
 // scratch: n_q * n_head * n_pos floats.  gate (n_q == 1; may be null): out *= sigmoid(gate[head * gate_stride + i])
+void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate = nullptr, int gate_stride = 0);
+// attn_prep's work and the attention of its query in one launch (scratch as attend_exact's); false: not launched
 struct AttnPrepP;
-// prep: the projections that the query and the new position are formed from (n_q 1, attn_prep's work in the same launch)
-void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate = nullptr, int gate_stride = 0,
-                  const AttnPrepP* prep = nullptr);
+bool attend_exact_one(const AttnArgs& a, const AttnPrepP& prep, float* scratch, float* out, const float* gate, int gate_stride, hipStream_t s, bool dry_run);
 // split-K flash decoding; scratch: n_q*n_head*n_split*(head_dim+2) floats.
 int attend_split_count(int n_pos_max, int n_q, int head_dim, int group);
 bool attend_split(const AttnArgs& a, int n_split_max, float* scratch, float* out, hipStream_t s);  // false: not launched
