@@ -587,15 +587,31 @@ struct ExpertsGemmP {
     const int32_t* order;
 };
 
-constexpr int NSTR = 64 + 8;  // LDS row stride of an NVFP4 slab (64 nibble bytes + pad)
+// the block's results: pair m's rows j0 .. j0 + 3
+template <bool GLU>
+IT_DEV void put_pairs(const ExpertsGemmP& p, int64_t e, int cnt, const int* pair_s, int j0, int m, const float (&acc)[GLU ? 2 : 1][4]) {
+    if (m >= cnt) return;
+    const int64_t pair = pair_s[m];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int j = j0 + i;
+        if (j >= p.n_out) continue;
+        float a0 = acc[0][i];
+        if (p.scale2) a0 *= p.scale2[e];
+        if (GLU) {
+            float a1 = acc[GLU ? 1 : 0][i];
+            if (p.scale2_up) a1 *= p.scale2_up[e];
+            a0 = it_silu(a0) * a1;
+        }
+        p.out[pair * p.n_out + j] = a0;
+    }
+}
 
-template <int FMT, bool GLU>
+template <bool GLU>
 __global__ __launch_bounds__(GT) void experts_gemm_k(ExpertsGemmP p) {
     constexpr int NM = GLU ? 2 : 1;
-    constexpr int ASTR = FMT == W_Q8_0 ? LSTR : NSTR;
-    constexpr int SPR = FMT == W_Q8_0 ? 4 : 8;  // scales per row per slab
-    __shared__ __align__(16) int8_t As[2][NM][64 * ASTR];
-    __shared__ float Asc[2][NM][64 * SPR];
+    __shared__ __align__(16) int8_t As[2][NM][64 * LSTR];
+    __shared__ float Asc[2][NM][64 * 4];
     __shared__ __align__(16) int8_t Bs[2][16 * LSTR];
     __shared__ float Bsc[2][16 * 4];
     __shared__ int xrow_s[16], pair_s[16];
@@ -620,7 +636,7 @@ __global__ __launch_bounds__(GT) void experts_gemm_k(ExpertsGemmP p) {
     const uint8_t* ws[2] = {it_expert_at(p.s, p.s_tab, e, p.s_stride), GLU ? it_expert_at(p.s2, p.s2_tab, e, p.s_stride) : nullptr};
 
     uint4 ra[NM][2], rb;
-    float rsa[NM][2], rsb;
+    float rsa[NM], rsb;
     rb = make_uint4(0, 0, 0, 0);
     rsb = 0.0f;
 #pragma unroll
@@ -628,28 +644,18 @@ __global__ __launch_bounds__(GT) void experts_gemm_k(ExpertsGemmP p) {
 #pragma unroll
         for (int q = 0; q < 2; q++) {
             ra[mt][q] = rb;
-            rsa[mt][q] = 0.0f;
+            rsa[mt] = 0.0f;
         }
     auto fetch = [&](int s) {
 #pragma unroll
         for (int mt = 0; mt < NM; mt++) {
-            if (FMT == W_Q8_0) {
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int idx = tid + q * GT, row = idx >> 3, seg = idx & 7;
-                    ra[mt][q] = *(const uint4*)(wq[mt] + (int64_t)min(row0 + row, p.n_out - 1) * n_in + s * SLAB + seg * 16);
-                }
-                const int row = tid >> 2, bi = tid & 3;
-                rsa[mt][0] = it_f16_to_f32(((const uint16_t*)ws[mt])[(int64_t)min(row0 + row, p.n_out - 1) * nb + s * 4 + bi]);
-            } else {
-                const int row = tid >> 2, seg = tid & 3;
-                ra[mt][0] = *(const uint4*)(wq[mt] + (int64_t)min(row0 + row, p.n_out - 1) * (n_in >> 1) + s * 64 + seg * 16);
-#pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int idx = tid + q * GT, r2 = idx >> 3, k = idx & 7;
-                    rsa[mt][q] = it_ue4m3_to_f32(ws[mt][(int64_t)min(row0 + r2, p.n_out - 1) * (n_in >> 4) + s * 8 + k]);
-                }
+            for (int q = 0; q < 2; q++) {
+                const int idx = tid + q * GT, row = idx >> 3, seg = idx & 7;
+                ra[mt][q] = *(const uint4*)(wq[mt] + (int64_t)min(row0 + row, p.n_out - 1) * n_in + s * SLAB + seg * 16);
             }
+            const int row = tid >> 2, bi = tid & 3;
+            rsa[mt] = it_f16_to_f32(((const uint16_t*)ws[mt])[(int64_t)min(row0 + row, p.n_out - 1) * nb + s * 4 + bi]);
         }
         if (tid < 128) {
             const int pr = tid >> 3, seg = tid & 7;
@@ -660,19 +666,12 @@ __global__ __launch_bounds__(GT) void experts_gemm_k(ExpertsGemmP p) {
     auto stash = [&](int buf) {
 #pragma unroll
         for (int mt = 0; mt < NM; mt++) {
-            if (FMT == W_Q8_0) {
 #pragma unroll
-                for (int q = 0; q < 2; q++) {
-                    const int idx = tid + q * GT, row = idx >> 3, seg = idx & 7;
-                    *(uint4*)(As[buf][mt] + row * ASTR + seg * 16) = ra[mt][q];
-                }
-                Asc[buf][mt][tid] = rsa[mt][0];
-            } else {
-                const int row = tid >> 2, seg = tid & 3;
-                *(uint4*)(As[buf][mt] + row * ASTR + seg * 16) = ra[mt][0];
-#pragma unroll
-                for (int q = 0; q < 2; q++) Asc[buf][mt][tid + q * GT] = rsa[mt][q];
+            for (int q = 0; q < 2; q++) {
+                const int idx = tid + q * GT, row = idx >> 3, seg = idx & 7;
+                *(uint4*)(As[buf][mt] + row * LSTR + seg * 16) = ra[mt][q];
             }
+            Asc[buf][mt][tid] = rsa[mt];
         }
         if (tid < 128) *(uint4*)(Bs[buf] + (tid >> 3) * LSTR + (tid & 7) * 16) = rb;
         if (tid < 64) Bsc[buf][tid] = rsb;
@@ -697,52 +696,153 @@ __global__ __launch_bounds__(GT) void experts_gemm_k(ExpertsGemmP p) {
             const float dx = Bsc[buf][m * 4 + bi];
 #pragma unroll
             for (int mt = 0; mt < NM; mt++) {
-                if (FMT == W_Q8_0) {
-                    const long a = *(const long*)(As[buf][mt] + (wave * 16 + m) * ASTR + bi * 32 + g * 8);
-                    const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bv, z, 0, 0, 0);
+                const long a = *(const long*)(As[buf][mt] + (wave * 16 + m) * LSTR + bi * 32 + g * 8);
+                const v4i d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bv, z, 0, 0, 0);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float dw = Asc[buf][mt][(wave * 16 + 4 * g + i) * 4 + bi];
-                        acc[mt][i] += (float)d[i] * (dw * dx);
-                    }
-                } else {
-                    // lane (m, g): sub-block g / 2 of the chunk, its low (g even) or high nibbles
-                    const uint2 nb8 = *(const uint2*)(As[buf][mt] + (wave * 16 + m) * ASTR + bi * 16 + (g >> 1) * 8);
-                    const int sh = (g & 1) * 4;
-                    const uint32_t lo = fp4x4_to_i8x4((nb8.x >> sh) & 0x0f0f0f0fu), hi = fp4x4_to_i8x4((nb8.y >> sh) & 0x0f0f0f0fu);
-                    const long a = (long)(((unsigned long long)hi << 32) | lo);
-                    const long bA = g < 2 ? bv : 0l, bB = g < 2 ? 0l : bv;
-                    const v4i dA = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bA, z, 0, 0, 0);
-                    const v4i dB = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bB, z, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float sA = Asc[buf][mt][(wave * 16 + 4 * g + i) * 8 + 2 * bi];
-                        const float sB = Asc[buf][mt][(wave * 16 + 4 * g + i) * 8 + 2 * bi + 1];
-                        acc[mt][i] += (dx * sA) * (float)dA[i];
-                        acc[mt][i] += (dx * sB) * (float)dB[i];
-                    }
+                for (int i = 0; i < 4; i++) {
+                    const float dw = Asc[buf][mt][(wave * 16 + 4 * g + i) * 4 + bi];
+                    acc[mt][i] += (float)d[i] * (dw * dx);
                 }
             }
         }
         if (s + 1 < nslab) stash(buf ^ 1);
         __syncthreads();
     }
-    if (m < cnt) {
-        const int64_t pair = pair_s[m];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int j = row0 + wave * 16 + 4 * g + i;
-            if (j >= p.n_out) continue;
-            float a0 = acc[0][i];
-            if (p.scale2) a0 *= p.scale2[e];
-            if (GLU) {
-                float a1 = acc[NM - 1][i];
-                if (p.scale2_up) a1 *= p.scale2_up[e];
-                a0 = it_silu(a0) * a1;
-            }
-            p.out[pair * p.n_out + j] = a0;
-        }
+    put_pairs<GLU>(p, e, cnt, pair_s, row0 + wave * 16 + 4 * g, m, acc);
+}
+
+// NVFP4, the CPU path's bits: a sub-block's dot is a sum of whole numbers, and the f16 matrix instruction forms it exactly (doubled
+// e2m1 by quants: 16 products below 1,524, in f32); so is the product of the activation's f16 step and the weight's e4m3 scale, a
+// second instruction of which one term is not 0.  Left to the vector ALU are gfx950's own conversion of the nibbles, the product of the
+// two results and its addition, sub-blocks in order.  On the int8 instructions that were also the nibbles' expansion, the halves'
+// selection, the dots' conversion and the scales' product, 2.7 times the instructions, which bounded it: 333 tokens, ten of 512 experts
+// of 512 x 2,048: gate and up 356 -> 194 us; a request of 333 tokens and eight more on two layers 3.50 -> 3.08 ms.
+// A lane takes bytes 2 g and 2 g + 1 of each sub-block (k order: low and high nibble of the one, of the other), so a row of a slab lies in
+// LDS as four groups of eight sub-blocks' two bytes, 16 bytes a lane and slab; the quants, as f16, in the same order.
+constexpr int NROW = 64 + 16, NCOL = 256 + 16;   // LDS bytes of a row's nibbles, of a pair's quants: sixteen rows at once hit different banks
+template <bool GLU>
+__global__ __launch_bounds__(GT, 4) void experts_nvfp4_k(ExpertsGemmP p) {
+    typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+    typedef float v4f __attribute__((ext_vector_type(4)));
+    constexpr int NM = GLU ? 2 : 1;
+    __shared__ __align__(16) uint8_t As[2][NM][64 * NROW];
+    __shared__ __align__(16) uint32_t Asc[2][NM][64 * 4];   // eight f16 a row
+    __shared__ __align__(16) uint8_t Bs[2][16 * NCOL];
+    __shared__ __align__(16) uint32_t Bsc[2][16 * 4];       // an f16 each
+    __shared__ int xrow_s[16], pair_s[16];
+    const int tile = blockIdx.x;
+    if (tile >= *p.n_tiles) return;
+    const int4 td = p.tiles[tile];
+    const int64_t e = td.x;
+    const int cnt = td.z;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.y * 64;
+    const int n_in = p.n_in, nb = n_in >> 5;
+    const int nslab = n_in / SLAB;
+    if (tid < 16) {
+        const int pair = p.order[td.y + min(tid, cnt - 1)];
+        pair_s[tid] = pair;
+        xrow_s[tid] = p.x_mode == 0 ? pair : (p.x_mode == 1 ? pair / p.n_used : 0);
     }
+    __syncthreads();
+    const int row = tid >> 2, seg = tid & 3, pr = tid >> 3, sub = tid & 7;   // what a thread brings: of a row two sub-blocks, of a pair one
+    const int64_t wrow = min(row0 + row, p.n_out - 1);
+    const uint8_t *wq[NM], *ws[NM];
+    wq[0] = it_expert_at(p.q, p.q_tab, e, p.q_stride) + wrow * (n_in >> 1) + seg * 16;
+    ws[0] = it_expert_at(p.s, p.s_tab, e, p.s_stride) + wrow * (n_in >> 4) + seg * 2;
+    if (GLU) {
+        wq[NM - 1] = it_expert_at(p.q2, p.q2_tab, e, p.q_stride) + wrow * (n_in >> 1) + seg * 16;
+        ws[NM - 1] = it_expert_at(p.s2, p.s2_tab, e, p.s_stride) + wrow * (n_in >> 4) + seg * 2;
+    }
+    const int8_t* const xq = p.act_quants + (int64_t)xrow_s[pr & 15] * n_in + sub * 16;
+    const float* const xs = p.act_scales + (int64_t)xrow_s[row & 15] * nb + seg;
+
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    u4 ra[NM] = {}, rb = {};
+    uint32_t rsa[NM] = {};
+    float rsb = 0.0f;
+    auto fetch = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < NM; mt++) {
+            ra[mt] = *(const u4*)(wq[mt] + s * 64);
+            rsa[mt] = *(const uint16_t*)(ws[mt] + s * 8);
+        }
+        if (tid < 128) rb = *(const u4*)(xq + s * SLAB);
+        if (tid < 64) rsb = xs[s * 4];
+    };
+    auto stash = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int mt = 0; mt < NM; mt++) {
+            // sub-blocks 2 seg (words 0, 1) and 2 seg + 1 (words 2, 3): group q's bytes 2 q, 2 q + 1 of each
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *(uint32_t*)(As[buf][mt] + row * NROW + q * 16 + seg * 4) =
+                    __builtin_amdgcn_perm(ra[mt][2 + q / 2], ra[mt][q / 2], q & 1 ? 0x07060302u : 0x05040100u);
+            const _Float16 s0 = (_Float16)it_ue4m3_to_f32(rsa[mt] & 0xffu), s1 = (_Float16)it_ue4m3_to_f32(rsa[mt] >> 8);
+            Asc[buf][mt][row * 4 + seg] = __builtin_bit_cast(uint16_t, s0) | (uint32_t)__builtin_bit_cast(uint16_t, s1) << 16;
+        }
+        if (tid < 128) {
+            auto quant = [&](int i) __attribute__((always_inline)) { return (_Float16)(float)(int8_t)(rb[i >> 2] >> (8 * (i & 3))); };
+#pragma unroll
+            for (int q = 0; q < 4; q++)
+                *(h4*)(Bs[buf] + pr * NCOL + q * 64 + sub * 8) = h4{quant(2 * q), quant(2 * q + 8), quant(2 * q + 1), quant(2 * q + 9)};
+        }
+        if (tid < 64) Bsc[buf][tid] = __builtin_bit_cast(uint16_t, (_Float16)rsb);
+    };
+
+    float acc[NM][4];
+#pragma unroll
+    for (int mt = 0; mt < NM; mt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[mt][i] = 0.0f;
+    const v4f z = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    fetch(0);
+    stash(0);
+    __syncthreads();
+    for (int s = 0; s < nslab; s++) {
+        const int buf = s & 1;
+        if (s + 1 < nslab) fetch(s + 1);
+        // the pair's quants, and its step of chunk c in the k slot that holds the scale of the sub-block (slots 4 g ..: sub-blocks 4 g ..)
+        h4 bq[8];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const u4 x = *(const u4*)(Bs[buf] + m * NCOL + g * 64 + c * 16);
+            bq[2 * c] = __builtin_bit_cast(h4, (uint64_t)x[1] << 32 | x[0]);
+            bq[2 * c + 1] = __builtin_bit_cast(h4, (uint64_t)x[3] << 32 | x[2]);
+        }
+        u4 dx = *(const u4*)(Bsc[buf] + m * 4);
+#pragma unroll
+        for (int c = 0; c < 4; c++) dx[c] = g == c >> 1 ? dx[c] : 0u;
+#pragma unroll
+        for (int mt = 0; mt < NM; mt++) {
+            const u4 nib = *(const u4*)(As[buf][mt] + (wave * 16 + m) * NROW + g * 16);
+            const h4 sc = *(const h4*)(Asc[buf][mt] + (wave * 16 + m) * 4 + 2 * (g & 1));   // (g of 2 and 3: their slots' steps are 0)
+            v4f dot[2], by[2];                       // (a sub-block's two results are on their way while the last one's are added)
+#pragma unroll
+            for (int j = 0; j <= 8; j++) {
+                if (j < 8) {
+                    const h2 lo = j & 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib[j / 2], 2.0f, 2) : __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib[j / 2], 2.0f, 0);
+                    const h2 hi = j & 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib[j / 2], 2.0f, 3) : __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib[j / 2], 2.0f, 1);
+                    const uint64_t step = (uint64_t)dx[j / 2] << (16 * (j & 3));
+                    dot[j & 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(h4{lo[0], lo[1], hi[0], hi[1]}, bq[j], z, 0, 0, 0);
+                    by[j & 1] = __builtin_amdgcn_mfma_f32_16x16x16f16(sc, __builtin_bit_cast(h4, step), z, 0, 0, 0);
+                }
+                if (j > 0) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) acc[mt][i] += by[(j - 1) & 1][i] * dot[(j - 1) & 1][i];
+                    // (here, not behind all products, whose results would fill the registers)
+                    asm volatile("" : "+v"(acc[mt][0]), "+v"(acc[mt][1]), "+v"(acc[mt][2]), "+v"(acc[mt][3]));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (s + 1 < nslab) stash(buf ^ 1);
+        __syncthreads();
+    }
+    put_pairs<GLU>(p, e, cnt, pair_s, row0 + wave * 16 + 4 * g, m, acc);
 }
 
 }  // namespace
@@ -790,11 +890,11 @@ bool experts_gemm(const ExpertsView& w, const ExpertsView* up, const int32_t* id
     p.order = order;
     dim3 grid(max_tiles, (w.n_out + 63) / 64);
     if (w.fmt == W_Q8_0) {
-        if (up) hipLaunchKernelGGL((experts_gemm_k<W_Q8_0, true>), grid, dim3(GT), 0, s, p);
-        else hipLaunchKernelGGL((experts_gemm_k<W_Q8_0, false>), grid, dim3(GT), 0, s, p);
+        if (up) hipLaunchKernelGGL(experts_gemm_k<true>, grid, dim3(GT), 0, s, p);
+        else hipLaunchKernelGGL(experts_gemm_k<false>, grid, dim3(GT), 0, s, p);
     } else {
-        if (up) hipLaunchKernelGGL((experts_gemm_k<W_NVFP4, true>), grid, dim3(GT), 0, s, p);
-        else hipLaunchKernelGGL((experts_gemm_k<W_NVFP4, false>), grid, dim3(GT), 0, s, p);
+        if (up) hipLaunchKernelGGL(experts_nvfp4_k<true>, grid, dim3(GT), 0, s, p);
+        else hipLaunchKernelGGL(experts_nvfp4_k<false>, grid, dim3(GT), 0, s, p);
     }
     return true;
 }
