@@ -66,6 +66,7 @@ DECODE_FAMILIES = {
     "moe_down_fast_k": "matmul_experts (expert down)",
     "gdn_rows_fast_k": "gdn_rows (l2 norm + delta rule)",
     "attend_one_k": "attend",
+    "attend_exact_one_k": "attend",
     "attend_few_k": "attend",
     "attend_split_k": "attend",
     "attend_merge": "attend",
@@ -85,6 +86,7 @@ def prefill_instructions(n_tokens, exact):
     held against: one of as many multiply-accumulates a cycle."""
     # Q8_0 products: 32x32x32 (k_gemm.hip, q8_wide_k), which does as many a cycle as 16x16x64; short batches take 16x16x32
     dense = ("int8_32x32x32", "int8_16x16x64") if n_tokens >= 512 else ("int8_16x16x32", "int8_16x16x32")
+    # (exact mode: what Q8_0 experts issue; NVFP4 ones take two f16 16x16x16 for sixteen weights and are held against the same)
     experts = ("int8_16x16x32", "int8_16x16x32") if exact else ("f16_32x32x16", "f16_32x32x16")
     return {"matmul (dense": dense, "moe_glu": experts, "matmul_experts": experts, "delta_rule": ("f32_16x16x4", "f32_16x16x4"),
             "attend": ("f16_32x32x16", "f16_32x32x16")}
