@@ -8,14 +8,17 @@
 // correction and products are the lane's own; a sum over the row runs through the four in turn, each adding its quarter to
 // what the one before it hands over, so that every addition is the reference's, in its order.
 #include "it_device.h"
+#include "it_dot.h"
 #include "it_reduce.h"
 #include "kernels.h"
 
 namespace itk {
 
-// A block is one wave: 16 rows of one head (256 blocks for 32 heads of 128).  Tokens go in chunks of 16: a chunk's k, q
-// (scaled), v and gates are staged in LDS, the next chunk's loads in flight meanwhile.  Bound by the two chains of dk dependent
-// additions a token (128: 0.93 us a token; one lane per row, with every token's loads waited for, took 4.1 us).
+// A block is 16 rows of one head (256 blocks for 32 heads of 128).  Tokens go in chunks of 16: a chunk's k, q
+// (scaled), v and gates are staged in LDS, the next chunk's loads in flight meanwhile.  Bound by the instructions between a token's
+// state and the next one's, a chain of dk dependent additions among them (one lane per row, with every token's loads waited for, took
+// 4.1 us a token of 128).  The read-out's chain is not between them: a second wave adds its products up, through LDS, while the first
+// is at the next token, stages the chunks and stores (333 tokens, 32 heads of 128: 272 us in one wave, 248 so; the request with eight more tokens 3.08 -> 3.06 ms).
 constexpr int DX_TCH = 16, DX_ROWS = 16;
 IT_DEV float quad_lane(float v, int which) {   // lane `which` of each aligned group of four, to all of it
     const int u = __builtin_bit_cast(int, v);
@@ -38,12 +41,14 @@ IT_DEV float quad_chain(const float (&p)[SEG]) {
     return acc;
 }
 template <int DK>
-__global__ __launch_bounds__(64) void delta_rule_k(DeltaArgs d, float* __restrict__ state, float* __restrict__ out, float q_scale) {
+__global__ __launch_bounds__(128) void delta_rule_k(DeltaArgs d, float* __restrict__ state, float* __restrict__ out, float q_scale) {
     constexpr int SEG = DK / 4, SS = SEG + 4;             // + 4: the four quarters' 16-byte reads fall on different banks
     constexpr int L4 = DX_TCH * DK / 4 / 64;              // float4 of k (and of q) per lane and chunk
     __shared__ __align__(16) float kb[2][DX_TCH][4 * SS], qb[2][DX_TCH][4 * SS];
     __shared__ float vb[2][DX_TCH][DX_ROWS], gb[2][DX_TCH][2];
-    const int lane = threadIdx.x, r = lane >> 2, seg = lane & 3;
+    constexpr int PS = DX_ROWS * SS + 16;                 // (rows' and quarters' 16-byte accesses: other banks, written and read)
+    __shared__ __align__(16) float pb[2][4 * PS];         // a token's read-out products, quarter by quarter
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane >> 2, seg = lane & 3;
     const int dv = d.head_v_dim;
     const int bph = (dv + DX_ROWS - 1) / DX_ROWS;
     const int h = blockIdx.x / bph, jb = blockIdx.x % bph;
@@ -58,14 +63,15 @@ __global__ __launch_bounds__(64) void delta_rule_k(DeltaArgs d, float* __restric
         const float4 t = ((const float4*)S)[i];
         row[4 * i] = t.x; row[4 * i + 1] = t.y; row[4 * i + 2] = t.z; row[4 * i + 3] = t.w;
     }
-    float4 rk[L4], rq[L4];
-    float rv[DX_TCH * DX_ROWS / 64], ra = 0.0f, rb = 0.0f;
+    typedef float f4 __attribute__((ext_vector_type(4)));   // (arrays of float4 were left in memory)
+    f4 rk[L4] = {}, rq[L4] = {};
+    float rv[DX_TCH * DX_ROWS / 64] = {}, ra = 0.0f, rb = 0.0f;
     auto load = [&](int t0) __attribute__((always_inline)) {
 #pragma unroll
         for (int p = 0; p < L4; p++) {
             const int idx = p * 64 + lane, t = min(t0 + idx / (DK / 4), n - 1), c = idx % (DK / 4);
-            rk[p] = ((const float4*)(d.k + (int64_t)t * kper + kh * DK))[c];
-            rq[p] = ((const float4*)(d.q + (int64_t)t * kper + kh * DK))[c];
+            rk[p] = ((const f4*)(d.k + (int64_t)t * kper + kh * DK))[c];
+            rq[p] = ((const f4*)(d.q + (int64_t)t * kper + kh * DK))[c];
         }
 #pragma unroll
         for (int p = 0; p < DX_TCH * DX_ROWS / 64; p++) {
@@ -81,8 +87,8 @@ __global__ __launch_bounds__(64) void delta_rule_k(DeltaArgs d, float* __restric
         for (int p = 0; p < L4; p++) {
             const int idx = p * 64 + lane, t = idx / (DK / 4), i = 4 * (idx % (DK / 4));
             const int at = i / SEG * SS + i % SEG;
-            *(float4*)&kb[b][t][at] = rk[p];
-            *(float4*)&qb[b][t][at] = make_float4(rq[p].x * q_scale, rq[p].y * q_scale, rq[p].z * q_scale, rq[p].w * q_scale);
+            *(f4*)&kb[b][t][at] = rk[p];
+            *(f4*)&qb[b][t][at] = f4{rq[p].x * q_scale, rq[p].y * q_scale, rq[p].z * q_scale, rq[p].w * q_scale};
         }
 #pragma unroll
         for (int p = 0; p < DX_TCH * DX_ROWS / 64; p++) vb[b][(p * 64 + lane) / DX_ROWS][(p * 64 + lane) % DX_ROWS] = rv[p];
@@ -93,42 +99,73 @@ __global__ __launch_bounds__(64) void delta_rule_k(DeltaArgs d, float* __restric
             gb[b][lane][1] = beta;
         }
     };
-    load(0);
+    auto meet = [&]() __attribute__((always_inline)) {      // (what is on its way from memory is not waited for)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (wave) {
+        load(0);
+        stash(0);
+    }
+    meet();
+    // the first wave's next token: key, gates, value (asked for a token ahead: a trip to LDS between two tokens otherwise)
+    f4 kn[SEG / 4];
+    float gn = 0.0f, bn = 0.0f, vn = 0.0f;
+    auto ask = [&](int b, int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < SEG / 4; i++) kn[i] = *(const f4*)&kb[b][t][seg * SS + 4 * i];
+        gn = gb[b][t][0];
+        bn = gb[b][t][1];
+        vn = vb[b][t][r];
+    };
+    ask(0, 0);
     for (int t0 = 0, b = 0; t0 < n; t0 += DX_TCH, b ^= 1) {
-        stash(b);
-        __syncthreads();   // (one wave: an LDS wait)
-        if (t0 + DX_TCH < n) load(t0 + DX_TCH);
         const int live = min(DX_TCH, n - t0);
         for (int t = 0; t < live; t++) {
-            const float g = gb[b][t][0], beta = gb[b][t][1], v = vb[b][t][r];
-            const float4* k4 = (const float4*)&kb[b][t][seg * SS];
-            const float4* q4 = (const float4*)&qb[b][t][seg * SS];
-            float kk[SEG], p[SEG];
+            float* const mine = pb[t & 1];                  // (a chunk that another follows is even)
+            if (wave == 0) {
+                const float g = gn, beta = bn, v = vn;
+                const float4* q4 = (const float4*)&qb[b][t][seg * SS];
+                float kk[SEG], p[SEG];
+                f4 qx[SEG / 4];
 #pragma unroll
-            for (int i = 0; i < SEG / 4; i++) {
-                const float4 x = k4[i];
-                kk[4 * i] = x.x; kk[4 * i + 1] = x.y; kk[4 * i + 2] = x.z; kk[4 * i + 3] = x.w;
-            }
+                for (int i = 0; i < SEG / 4; i++) {
+                    kk[4 * i] = kn[i].x; kk[4 * i + 1] = kn[i].y; kk[4 * i + 2] = kn[i].z; kk[4 * i + 3] = kn[i].w;
+                    qx[i] = ((const f4*)q4)[i];
+                }
+                if (t + 1 < live) ask(b, t + 1);
+                else ask(b ^ 1, 0);                         // (the next chunk's is there; behind the last one it is not used)
 #pragma unroll
-            for (int i = 0; i < SEG; i++) {
-                row[i] *= g;
-                p[i] = row[i] * kk[i];
-            }
-            const float delta = beta * (v - quad_chain<SEG>(p));
+                for (int i = 0; i < SEG; i++) {
+                    row[i] *= g;
+                    p[i] = row[i] * kk[i];
+                }
+                const float delta = beta * (v - quad_chain<SEG>(p));
 #pragma unroll
-            for (int i = 0; i < SEG / 4; i++) {
-                const float4 x = q4[i];
-                const float qq[4] = {x.x, x.y, x.z, x.w};
+                for (int i = 0; i < SEG / 4; i++) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    row[4 * i + e] += kk[4 * i + e] * delta;
-                    p[4 * i + e] = row[4 * i + e] * qq[e];
+                    for (int e = 0; e < 4; e++) {
+                        row[4 * i + e] += kk[4 * i + e] * delta;
+                        p[4 * i + e] = row[4 * i + e] * qx[i][e];
+                    }
+                    *(float4*)&mine[seg * PS + r * SS + 4 * i] = make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]);
                 }
             }
-            const float o = quad_chain<SEG>(p);
-            if (seg == 0 && j < dv) out[(int64_t)(t0 + t) * vper + h * dv + j] = o;
+            meet();
+            if (wave) {
+                float o = 0.0f;
+#pragma unroll
+                for (int s = 0; s < 4; s++) o = fold_terms_from(o, mine + s * PS + (lane & 15) * SS, SEG);
+                if (lane < DX_ROWS && jb * DX_ROWS + lane < dv) out[(int64_t)(t0 + t) * vper + h * dv + jb * DX_ROWS + lane] = o;
+                if (t0 + DX_TCH < n) {                      // (a whole chunk)
+                    if (t == 0) load(t0 + DX_TCH);
+                    if (t == DX_TCH / 2) stash(b ^ 1);
+                }
+            }
         }
     }
+    if (wave) return;
     if (j < dv) {
 #pragma unroll
         for (int i = 0; i < SEG / 4; i++) ((float4*)S)[i] = make_float4(row[4 * i], row[4 * i + 1], row[4 * i + 2], row[4 * i + 3]);
@@ -260,9 +297,9 @@ void delta_rule(const DeltaArgs& d, float* state, float* out, int exact, float* 
     }
     int blocks = d.n_v_heads * ((d.head_v_dim + DX_ROWS - 1) / DX_ROWS);
     switch (d.head_k_dim) {
-        case 32: hipLaunchKernelGGL(delta_rule_k<32>, dim3(blocks), dim3(64), 0, s, d, state, out, q_scale); break;
-        case 64: hipLaunchKernelGGL(delta_rule_k<64>, dim3(blocks), dim3(64), 0, s, d, state, out, q_scale); break;
-        case 128: hipLaunchKernelGGL(delta_rule_k<128>, dim3(blocks), dim3(64), 0, s, d, state, out, q_scale); break;
+        case 32: hipLaunchKernelGGL(delta_rule_k<32>, dim3(blocks), dim3(128), 0, s, d, state, out, q_scale); break;
+        case 64: hipLaunchKernelGGL(delta_rule_k<64>, dim3(blocks), dim3(128), 0, s, d, state, out, q_scale); break;
+        case 128: hipLaunchKernelGGL(delta_rule_k<128>, dim3(blocks), dim3(128), 0, s, d, state, out, q_scale); break;
         default: break;  // the caller validates head_k_dim
     }
 }
