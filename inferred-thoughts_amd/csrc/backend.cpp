@@ -1253,9 +1253,18 @@ float* it_hip::scratch_f32(size_t floats) {
     }
     attn_scratch = nullptr;
     attn_scratch_cap = 0;
-    if (!check(hipMalloc((void**)&attn_scratch, floats * sizeof(float)), "hipMalloc(attention scratch)"))
-        return nullptr;
-    attn_scratch_cap = floats;
+    // With room to grow by an eighth, and 256 KB at least: a context that grows token by token, op by op, would move it at every one of
+    // them (a wait for the stream each time, and no two passes alike for a recording).
+    size_t step = 1 << 16;
+    while (step * 8 < floats) step *= 2;
+    size_t cap = (floats + step - 1) / step * step;
+    if (hipMalloc((void**)&attn_scratch, cap * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        attn_scratch = nullptr;
+        cap = floats;
+        if (!check(hipMalloc((void**)&attn_scratch, cap * sizeof(float)), "hipMalloc(attention scratch)")) return nullptr;
+    }
+    attn_scratch_cap = cap;
     return attn_scratch;
 }
 
