@@ -265,15 +265,19 @@ bool match_matmul_residual(Plan& pl, size_t i, int exact) {
     return true;
 }
 
-// last-row gather + final norm + LM head: whether the four ops are that, and as one product
+// last-row gather + final norm + LM head: whether the four ops are that, and as one product, which leaves the gathered row too
+// (where the norm does not replace it)
 bool final_head(const Op& g, const Op& rms, const Op& q, const Op& m, int exact, FusedGemvP* out) {
     if (g.id != OP_GATHER || rms.id != OP_RMS || q.id != OP_QUANT || m.id != OP_MATMUL) return false;
     if (g.i[3] != g.i[0] || rms.p[0] != g.p[1] || rms.i[0] != 1 || rms.i[1] != g.i[0]) return false;
     if (q.p[0] != rms.p[2] || q.i[0] != rms.i[1] || !mm_reads(m, rms.p[2], q)) return false;
+    // (what the launch writes is none of what it reads, nor the same twice)
+    if (g.p[1] == g.p[0] || rms.p[2] == g.p[0] || m.p[5] == g.p[0] || m.p[5] == g.p[1] || m.p[5] == rms.p[2]) return false;
     FusedGemvP a{};
     a.x = (const float*)g.p[0] + g.i[2];
     a.norm_w = (const float*)rms.p[1];
     a.x_copy = (float*)rms.p[2];
+    a.x_raw = g.p[1] == rms.p[2] ? nullptr : (float*)g.p[1];
     a.eps = rms.f[0];
     a.n_in = (int)rms.i[1];
     a.mode = 1;
@@ -974,8 +978,8 @@ bool references(const Op& op, const void* a, const void* b) {
 //                                                          not written: nothing else in the loop reads them)
 //   RMS_HEADS core, EW silu_mul(z, core), QUANT z        -> gated_norm_silu_q8 (core is left unnormed)
 //   MATMUL, SCALE of its result                          -> the product with the factor in its epilogue
-//   GATHER of the last row, RMS, QUANT, MATMUL of one token -> the single-token product with its own norm (the row's copy
-//                                                          is not written): 23 us in four launches, 8 in one
+//   GATHER of the last row, RMS, QUANT, MATMUL of one token -> the single-token product with its own norm: 23 us in four
+//                                                          launches, 8 in one
 //   MATMUL gate, MATMUL up, [SCALE up,] [SCALE gate,] EW silu_mul(gate, up), both NVFP4   -> one gate / up product
 // and the routed FFN of a short batch (2..32 tokens; src/model/qwen35.rs:1630-1700), whose products are held back too:
 //   SOFTMAX, ROUTE, [QUANT x], GLU, QUANT g, EXPERTS, MATMUL shared gate, MATMUL shared up, [SCALE]*, EW silu_mul,
@@ -1396,10 +1400,9 @@ size_t it_hip::fuse_at(const std::vector<OpRec>& h, size_t i, const OpRec* next)
     // ---- the output matrix on the pass's last row
     if (a.id == OP_GATHER && i + 4 <= n) {
         FusedGemvP head{};
-        if (final_head(a, h[i + 1], h[i + 2], h[i + 3], 0, &head) && !used_later(h, i + 4, next, a.p[1]) && !used_later(h, i + 4, next, h[i + 2].p[1])) {
+        if (final_head(a, h[i + 1], h[i + 2], h[i + 3], 0, &head) && !used_later(h, i + 4, next, h[i + 2].p[1])) {
             Span sp(this, FAM_LM_HEAD, gemv_bytes(head));
             fused_gemv(head, stream);
-            mark_elided({a.p[1]});
             if (Act* f = act_by_dev(h[i + 1].p[2])) f->stale();   // (its quants are not made)
             return 4;
         }

@@ -354,6 +354,7 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
             const int i = 4 * (tid + FG_THREADS * j);
             part += squares(xv[j]);
             if (i < n_in) *(float4*)(xf + i) = xv[j];      // for the serial sum, should it be needed
+            if (i < n_in && blockIdx.x == 0 && p.x_raw) store4(p.x_raw + i, xv[j]);
         }
         part = wave_sum_f64_tail(part);
         if (lane == 63) red[wave] = part;

@@ -19,6 +19,7 @@ struct FusedGemvP {
     const float* gate;    // mode 2: silu of the gate, [n_in]
     float* x_copy;        // optional: the activation after the prologue, f32, written by block 0
     float* x_copy2;       // optional second copy (a whole-row gather of it)
+    float* x_raw;         // mode 1, optional: the activation as it came (a gather of it that the norm reads), written by block 0
     float eps;
     int n_in, mode, head_dim, exact, n_mats, rows_per_wave, total_groups;
     FusedMat m[4];
