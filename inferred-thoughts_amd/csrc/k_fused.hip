@@ -588,8 +588,12 @@ static bool fused_gemv_exact_takes(const FusedGemvP& p) {
     return p.n_in % 256 == 0 && p.n_in <= FG_MAX_IN && std::max(fg_lds(p.n_in, 1), fg_base(p.n_in) + (size_t)(FG_THREADS / 64) * p.n_in * 4) <= FG_LDS_MAX;
 }
 // (A wave takes a row's 32-value units at once, eight a lane, and a thread holds its quads of the activation: rows of more than
-// 16,384 values are left to the ops one by one.)
+// 16,384 values are left to the ops one by one.  Every block reads the whole activation, at its own time: what block 0 leaves and
+// what the rows' waves write lies elsewhere.)
 bool fused_gemv_takes(const FusedGemvP& p) {
+    if (p.x_copy == p.x || p.x_copy2 == p.x || p.x_raw == p.x) return false;
+    for (int i = 0; i < p.n_mats; i++)
+        if (p.m[i].out == p.x || p.m[i].out == p.gate) return false;
     if (p.mode == 2 && ((p.head_dim != 64 && p.head_dim != 128) || p.n_in % p.head_dim)) return false;   // (a head is a row of 16 lanes, or two)
     bool floats = false;
     for (int i = 0; i < p.n_mats; i++) floats |= p.m[i].fmt != W_Q8_0 && p.m[i].fmt != W_NVFP4;

@@ -39,7 +39,8 @@ struct FusedGemvP {
     float* route_w;
 };
 void fused_gemv(FusedGemvP p, hipStream_t s);
-// whether fused_gemv may be launched with p: how long the activation is and, with unquantized matrices in it, formats, shapes, alignment
+// whether fused_gemv may be launched with p: how long the activation is, that nothing is written over what other blocks still read,
+// and, with unquantized matrices in it, formats, shapes, alignment
 bool fused_gemv_takes(const FusedGemvP& p);
 // whether the fast kernel takes p
 bool fused_gemv_fast_takes(const FusedGemvP& p);
