@@ -778,6 +778,13 @@ void ssm_conv(float* state, const float* x, const float* w, int kernel, int nc, 
 
 // ------------------------------------------------------------------ argmax
 // First strict maximum (ties to the lower index), /root/reference src/profile.rs:192-213.
+// What the serial scan makes of value `v` at index `i`: one that is not a number is never taken, and a first value that is not a
+// number stays.  (Candidates are numbers then, so that every order of merging them gives the same one.)
+IT_DEV bool argmax_counts(float* v, int64_t i) {
+    if (*v == *v) return true;
+    *v = INFINITY;
+    return i == 0;
+}
 __global__ __launch_bounds__(256) void argmax_part_k(const float* __restrict__ x, int64_t n,
                                                      int32_t* __restrict__ pidx, float* __restrict__ pval) {
     __shared__ float sv[256];
@@ -788,12 +795,10 @@ __global__ __launch_bounds__(256) void argmax_part_k(const float* __restrict__ x
     int bi = 0x7fffffff;
     for (int64_t i = lo + threadIdx.x; i < hi; i += 256) {
         float v = x[i];
-        if (v > bv || bi == 0x7fffffff) {
-            // strided scan visits ascending indices per thread, so strict > keeps the lowest
-            if (bi == 0x7fffffff || v > bv) {
-                bv = v;
-                bi = (int)i;
-            }
+        // strided scan visits ascending indices per thread, so strict > keeps the lowest
+        if (argmax_counts(&v, i) && (bi == 0x7fffffff || v > bv)) {
+            bv = v;
+            bi = (int)i;
         }
     }
     sv[threadIdx.x] = bv;
@@ -922,14 +927,15 @@ __global__ __launch_bounds__(1024) void argmax_embed_one_k(const float* __restri
         if (1024 * k >= n) break;
         v[k] = tid + 1024 * k < n ? logits[tid + 1024 * k] : -INFINITY;
     }
-    float bv = v[0];
-    int bi = tid < n ? tid : 0x7fffffff;     // (as the two launches: a thread's first value stands until one is larger)
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
 #pragma unroll
-    for (int k = 1; k < ARGMAX_ONE; k++) {
+    for (int k = 0; k < ARGMAX_ONE; k++) {
+        const int i = tid + 1024 * k;
         if (1024 * k >= n) break;
-        if (v[k] > bv) {
+        if (i < n && argmax_counts(&v[k], i) && (bi == 0x7fffffff || v[k] > bv)) {
             bv = v[k];
-            bi = tid + 1024 * k;
+            bi = i;
         }
     }
     argmax_of_wave(&bv, &bi);
