@@ -336,6 +336,7 @@ bool match_attn(Plan& pl, size_t i, int exact) {
     if (!pl.be->attn_positions_agree({slots})) return false;
     const void* attn = at.p[5];
     if (sg.i[0] != 1 || sg.p[0] != attn || sg.p[1] != gb || sg.i[1] != hd * nh) return false;
+    if (attn == qg) return false;   // (the gates are read beside it while the result is written)
     if (q2.p[0] != attn || q2.i[0] != hd * nh || !mm_reads(mo, attn, q2)) return false;
     if (add.i[0] != 2 || add.p[1] != mo.p[5] || add.p[0] != rms.p[0] || add.i[1] != mo.i[2]) return false;
 

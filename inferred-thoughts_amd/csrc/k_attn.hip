@@ -440,6 +440,8 @@ static bool one_launch(const AttnArgs& a, const AttnPrepP& prep, float* scratch,
 }
 bool attend_exact_one(const AttnArgs& a, const AttnPrepP& prep, float* scratch, float* out, const float* gate, int gate_stride, hipStream_t s, bool dry_run) {
     if (a.n_q != 1 || !a.n_pos_dyn || a.kv_dim % 8 || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15)) return false;
+    // a head's blocks read the projections, write their dims of the result and, one of them, the query, each at its own time
+    if (out == prep.q || out == prep.k || out == prep.v) return false;
     if (a.head_dim == 64) return one_launch<64>(a, prep, scratch, out, gate, gate_stride, s, dry_run);
     if (a.head_dim == 128) return one_launch<128>(a, prep, scratch, out, gate, gate_stride, s, dry_run);
     return a.head_dim == 256 && one_launch<256>(a, prep, scratch, out, gate, gate_stride, s, dry_run);

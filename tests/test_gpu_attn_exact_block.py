@@ -25,6 +25,17 @@ ND, EPS, THETA, PASSES = 256, 1e-6, 1e7, 9
     (2, 1, 320, 64, 64, 31, 4),
 ])
 def test_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels):
+    recorded_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels)
+
+
+@pytest.mark.parametrize("over,kernels", [("q", 4), ("k", 4), ("v", 4), ("qg", 0)])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 8, 64), (4, 4, 256)])
+def test_result_over_an_input(nh, nkv, hd, over, kernels):
+    """What one block reads another must not have written: the rows by themselves, or the ops one by one."""
+    recorded_block(nh, nkv, hd, 64, 300, 125, kernels, attn=over)
+
+
+def recorded_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels, attn="attn"):
     import inferred_hip as ih
     from oracle import binding as ob
     hip = ih.Hip(exact=True)
@@ -41,6 +52,8 @@ def test_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels):
     v0[pos0 * kd:] = 0
     slabs = [dict(k=k0.copy(), v=v0.copy()) for _ in range(2)]
     sc = float(1.0 / np.sqrt(np.float32(hd)))
+    res = lambda b: b[attn][:qd]   # noqa: E731
+    read = ("x",) if attn != "attn" else ("x", "attn", "q")
 
     def block(ops, i, b, s, pos):
         W = lambda t: t[i]
@@ -51,9 +64,9 @@ def test_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels):
         ops.rms_norm_heads(b["q"], qn, hd, EPS); ops.rms_norm_heads(b["k"], kn, hd, EPS)
         ops.rope_neox(b["q"], pos, hd, n_rot, nh, THETA); ops.rope_neox(b["k"], pos, hd, n_rot, nkv, THETA)
         ops.kv_write(s["k"], pos * kd, b["k"]); ops.kv_write(s["v"], pos * kd, b["v"])
-        ops.attend(b["q"], s["k"], s["v"], kd, pos + 1, hd, nh, nkv, sc, b["attn"])
-        ops.sigmoid_mul(b["attn"], b["g"])
-        ops.matmul(W(wo), b["attn"], b["mixed"])
+        ops.attend(b["q"], s["k"], s["v"], kd, pos + 1, hd, nh, nkv, sc, res(b))
+        ops.sigmoid_mul(res(b), b["g"])
+        ops.matmul(W(wo), res(b), b["mixed"])
         ops.add_assign(b["x"], b["mixed"])
 
     try:
@@ -63,17 +76,17 @@ def test_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels):
             for b in B:
                 b["x"][:] = x0
             hip.begin_pass(1); hip.host_wrote(B[0]["x"]); block(hip, 0, B[0], slabs[0], pos); hip.end_pass()
-            for name in ("x", "attn", "q"):
+            for name in read:
                 hip.host_needs(B[0][name])
             hip.read_kv(slabs[0]["k"]); hip.read_kv(slabs[0]["v"])
             hip.raise_if_error()
             block(orc, 1, B[1], slabs[1], pos)
-            for name in ("x", "attn", "q"):
+            for name in read:
                 assert np.array_equal(B[0][name].view(np.uint32), B[1][name].view(np.uint32)), (p, name)
             for t in "kv":
                 assert np.array_equal(slabs[0][t], slabs[1][t]), (p, t)
         g = hip.graph_stats()
-        assert g["captures"] == 1 and g["replays"] >= 1 and g["graph_kernels"] == kernels, g
+        assert g["captures"] == 1 and g["replays"] >= 1 and (not kernels or g["graph_kernels"] == kernels), g
     finally:
         hip.take_error()
         hip.close()
