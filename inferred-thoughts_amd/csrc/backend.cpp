@@ -1253,8 +1253,8 @@ float* it_hip::scratch_f32(size_t floats) {
     }
     attn_scratch = nullptr;
     attn_scratch_cap = 0;
-    // With room to grow by an eighth, and 256 KB at least: a context that grows token by token, op by op, would move it at every one of
-    // them (a wait for the stream each time, and no two passes alike for a recording).
+    // In steps of an eighth to a quarter of it, of 256 KB at least: a context that grows token by token, op by op, would move it at
+    // every one of them (a wait for the stream each time, and no two passes alike for a recording).
     size_t step = 1 << 16;
     while (step * 8 < floats) step *= 2;
     size_t cap = (floats + step - 1) / step * step;
@@ -1793,8 +1793,9 @@ void it_hip_attend(it_hip* be, const it_attn* a, float* out, uint64_t out_len) {
     const uint64_t n_pos_cap = (be->exact || !split_ok ? graphed : by_slab) ? slab_rows : a->n_pos;
     uint64_t bytes = a->n_pos * a->n_head_kv * a->head_dim * 4 + a->q_len * 8;
     if (be->exact || !split_ok) {
-        // (one query: a row of scores for each 64 dims of a head, as attend_exact_one may leave)
-        float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap) * (n_q == 1 ? (a->head_dim + 63) / 64 : 1));
+        // (a recorded token's attention may be attend_exact_one, the one form with more than a row of scores a head)
+        const size_t rows = be->exact && graphed && n_q == 1 ? (size_t)attend_exact_one_rows((int)a->head_dim) : 1;
+        float* sc = be->scratch_f32((size_t)(n_q * a->n_head * n_pos_cap) * rows);
         if (!sc) return;
         const int* dyn = be->dyn_slot((int)a->n_pos, {(int)n_q, (int)std::min<uint64_t>(slab_rows, INT32_MAX)});
         AttnArgs args{dq, dk, dv, (int)n_q, (int)a->kv_dim, dyn ? (int)n_pos_cap : (int)a->n_pos, (int)a->head_dim,

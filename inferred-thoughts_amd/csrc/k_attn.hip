@@ -438,6 +438,7 @@ static bool one_launch(const AttnArgs& a, const AttnPrepP& prep, float* scratch,
     if (!dry_run) hipLaunchKernelGGL(attend_exact_one_k<HD>, dim3(a.n_head, HD / ONE_DIMS), dim3(ONE_T), lds(lds_pos), s, a, prep, scratch, out, gate, gate_stride, lds_pos);
     return true;
 }
+int attend_exact_one_rows(int head_dim) { return head_dim == 64 || head_dim == 128 || head_dim == 256 ? head_dim / ONE_DIMS : 1; }
 bool attend_exact_one(const AttnArgs& a, const AttnPrepP& prep, float* scratch, float* out, const float* gate, int gate_stride, hipStream_t s, bool dry_run) {
     if (a.n_q != 1 || !a.n_pos_dyn || a.kv_dim % 8 || ((uintptr_t)a.k & 15) || ((uintptr_t)a.v & 15)) return false;
     // a head's blocks read the projections, write their dims of the result and, one of them, the query, each at its own time

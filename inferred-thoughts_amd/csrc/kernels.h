@@ -263,7 +263,9 @@ struct AttnArgs {
 // exact: the oracle's order (scores, serial softmax sum, positions outermost).
 // scratch: n_q * n_head * n_pos floats.  gate (n_q == 1; may be null): out *= sigmoid(gate[head * gate_stride + i])
 void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, const float* gate = nullptr, int gate_stride = 0);
-// attn_prep's work and the attention of its query in one launch (scratch as attend_exact's); false: not launched
+// attn_prep's work and the attention of its query in one launch; false: not launched.  scratch: attend_exact_one_rows(head_dim) *
+// n_head * n_pos floats (rows: 1 for heads that it does not take)
+int attend_exact_one_rows(int head_dim);
 struct AttnPrepP;
 bool attend_exact_one(const AttnArgs& a, const AttnPrepP& prep, float* scratch, float* out, const float* gate, int gate_stride, hipStream_t s, bool dry_run);
 // split-K flash decoding; scratch: n_q*n_head*n_split*(head_dim+2) floats.

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from test_gpu_fused_fast import Both, bufs
-from util import f16_bits, rng
+from util import Hiprt, f16_bits, rng
 
 pytestmark = pytest.mark.gpu
 ND, EPS, THETA, PASSES = 256, 1e-6, 1e7, 9
@@ -89,4 +89,25 @@ def recorded_block(nh, nkv, hd, n_rot, n_ctx, pos0, kernels, attn="attn"):
         assert g["captures"] == 1 and g["replays"] >= 1 and (not kernels or g["graph_kernels"] == kernels), g
     finally:
         hip.take_error()
+        hip.close()
+
+
+@pytest.mark.parametrize("exact,nh,hd", [(False, 64, 320), (True, 64, 256), (True, 128, 1024)])
+def test_scratch_of_an_unrecorded_call(exact, nh, hd):
+    """A row of scores a head: only the recorded form of exact mode leaves more.  (Measured as what the call takes from the device:
+    its mirrors and slabs, and 4 bytes a score and an eighth to a quarter more; 8 MB for what the allocator rounds up to.)"""
+    import inferred_hip as ih
+    n_pos, rt = 40000, Hiprt()
+    hip = ih.Hip(exact=exact)
+    try:
+        q, out = (np.zeros(nh * hd, np.float32) for _ in range(2))
+        k, v = (np.zeros(n_pos * hd, np.uint16) for _ in range(2))
+        hip.attend(q, k, v, hd, 8, hd, nh, 1, 1.0, out)           # mirrors and slabs
+        hip.sync()
+        before = rt.mem_free()
+        hip.attend(q, k, v, hd, n_pos, hd, nh, 1, 1.0, out)
+        hip.sync()
+        hip.raise_if_error()
+        assert before - rt.mem_free() <= nh * n_pos * 4 * 1.25 + (8 << 20)
+    finally:
         hip.close()
