@@ -1672,7 +1672,7 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
     // or, where a buffer had to grow in between, has been made already: the sums are the same either way.
     const bool last_row = !exact && n == 1 && be->in_pass && be->pass_tokens > 1 && be->fuse_enabled && (v.fmt == W_Q8_0 || v.fmt == W_NVFP4);
     auto run = [=](hipStream_t s, float scale_by) {
-        if (last_row && scale_by == 1.0f) {
+        if (last_row) {   // (one token: no factor)
             FusedGemvP a{};
             a.x = dx;
             a.n_in = v.n_in;

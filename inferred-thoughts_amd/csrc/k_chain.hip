@@ -133,23 +133,6 @@ __device__ long long it_chain_wave_stamps[8][8];
     } while (0)
 #endif
 
-// Where the prefetches sit (tuning switches; the defaults are what measured best).
-#ifndef IT_CHAIN_B_POLLERS
-#define IT_CHAIN_B_POLLERS 1     // stage B's input gathered by waves 5..7 alone (1) or by the first 274 threads (0)
-#endif
-#ifndef IT_CHAIN_TOUCH
-#define IT_CHAIN_TOUCH 1          // stage E's rows touched by the blocks that have none of their own
-#endif
-#ifndef IT_CHAIN_WC_AT
-#define IT_CHAIN_WC_AT 0      // out-projection row: 0 at the head of stage B, 1 after stage A's input has arrived, 2 after stage A's dots, 3 after stage B's input has arrived
-#endif
-#ifndef IT_CHAIN_D_AT
-#define IT_CHAIN_D_AT 1       // stage D's rows: 0 at the head of stage C, 1 after stage B's input has arrived
-#endif
-#ifndef IT_CHAIN_A_AT
-#define IT_CHAIN_A_AT 0x070   // next in-projection, a hex digit of fetch_a parts per site: after D's input | at the head of stage F | after F's input
-#endif
-
 struct Ctl {
     unsigned* abort_flag;
     int spin_limit;
@@ -170,11 +153,7 @@ IT_DEV void ll_put2f(u64* p, float v0, float v1, unsigned e) {
 }
 
 // true when the wait must stop: the tries are used up (this thread raises the abort word) or another wait gave up
-#ifndef IT_CHAIN_SLEEP
-#define IT_CHAIN_SLEEP 0
-#endif
 IT_DEV bool ll_give_up(int& spins, const Ctl& c) {
-    if (IT_CHAIN_SLEEP > 0) __builtin_amdgcn_s_sleep(IT_CHAIN_SLEEP);
     if (++spins > c.spin_limit) {
         *(volatile unsigned*)c.abort_flag = 1u;
         return true;
@@ -187,10 +166,8 @@ IT_DEV bool ll_give_up(int& spins, const Ctl& c) {
 // a short sleep ahead of a wait's first poll: a poll issued the moment the wave arrives nearly always fails, and every
 // failed poll is traffic that the words it waits for queue behind (eight layers of a token with 0, 4, 8, 12, 16 times 64
 // cycles: 232.6, 227.9, 224.9, 223.1, 223.0 us)
-#ifndef IT_CHAIN_FIRST_SLEEP
-#define IT_CHAIN_FIRST_SLEEP 12
-#endif
-template <int SL = IT_CHAIN_FIRST_SLEEP>   // (0 behind another wait of the same stage: the words are there)
+constexpr int FIRST_SLEEP = 12;
+template <int SL = FIRST_SLEEP>   // (0 behind another wait of the same stage: the words are there)
 IT_DEV bool ll_wait1(const u64* p, unsigned e, const Ctl& c, uint32_t* out) {
     int spins = 0;
     if (SL > 0) __builtin_amdgcn_s_sleep(SL);
@@ -206,7 +183,7 @@ IT_DEV bool ll_wait1(const u64* p, unsigned e, const Ctl& c, uint32_t* out) {
 }
 // K pairs of words at a[k] (16-byte aligned); out[2k], out[2k+1] = their payloads.  A pair that is complete is
 // latched; its load is simply repeated while the others are still awaited.
-template <int K, int SL = IT_CHAIN_FIRST_SLEEP>
+template <int K, int SL = FIRST_SLEEP>
 IT_DEV bool ll_wait_pairs(const u64* const (&a)[K], unsigned e, const Ctl& c, uint32_t (&out)[2 * K]) {
     static_assert(K == 1 || K == 2 || K == 4, "");
     int spins = 0;
@@ -302,40 +279,32 @@ IT_DEV int a_row(int k, int b, int wave) {   // row k of the wave in its own mat
 // multiply-add chain per lane from zero and a lane reduction, and the eight chunk sums are added as a balanced tree.
 IT_DEV float f32_chunk(const float4 w, const float4 xv) { return fmaf(w.x, xv.x, fmaf(w.y, xv.y, fmaf(w.z, xv.z, fmaf(w.w, xv.w, 0.0f)))); }
 IT_DEV float f32_tree(const float* pc) { return ((pc[0] + pc[1]) + (pc[2] + pc[3])) + ((pc[4] + pc[5]) + (pc[6] + pc[7])); }
-// `parts` picks what is fetched: bit 0 the first two wqkv rows and the conv windows, bit 1 the other two wqkv rows,
-// bit 2 the two wz rows and the alpha / beta row.  (A block's 105 KB can be issued in pieces at up to three sites of the
-// layer before, IT_CHAIN_A_AT: loads return in the order they were issued, and a poll behind a large fetch waits for
-// all of it.  All at the head of stage F measured best once that stage's input was gathered by waves that issue
-// theirs behind the gather.)
+// A block's 105 KB.  (Issued in pieces at up to three sites of the layer before: loads return in the order they were issued, and a
+// poll behind a large fetch waits for all of it.  All at the head of stage F measured best once that stage's input was gathered by
+// waves that issue theirs behind the gather.)
 template <int RF, class M>   // M: a ChainMixer, wherever it lives
-IT_DEV void fetch_a(const M& m, AW& a, int b, int wave, int lane, int parts = 7) {
-    if (parts & 1) {
+IT_DEV void fetch_a(const M& m, AW& a, int b, int wave, int lane) {
 #pragma unroll
-        for (int k = 0; k < 2; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.qkv_q, m.qkv_s, D, a_row(k, b, wave), lane, true);
-        if (lane < 4) {
-            const int64_t row = 32 * b + 4 * wave + lane;
-            a.taps = *(const float4*)(m.conv_w + row * 4);
-            a.past[0] = m.conv_state[row * 3];
-            a.past[1] = m.conv_state[row * 3 + 1];
-            a.past[2] = m.conv_state[row * 3 + 2];
-        }
+    for (int k = 0; k < 2; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.qkv_q, m.qkv_s, D, a_row(k, b, wave), lane, true);
+    if (lane < 4) {
+        const int64_t row = 32 * b + 4 * wave + lane;
+        a.taps = *(const float4*)(m.conv_w + row * 4);
+        a.past[0] = m.conv_state[row * 3];
+        a.past[1] = m.conv_state[row * 3 + 1];
+        a.past[2] = m.conv_state[row * 3 + 2];
     }
-    if (parts & 2) {
 #pragma unroll
-        for (int k = 2; k < 4; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.qkv_q, m.qkv_s, D, a_row(k, b, wave), lane, true);
-    }
-    if (parts & 4) {
+    for (int k = 2; k < 4; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.qkv_q, m.qkv_s, D, a_row(k, b, wave), lane, true);
 #pragma unroll
-        for (int k = 4; k < 6; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.z_q, m.z_s, D, a_row(k, b, wave), lane, true);
-        if (RF) {
-            // an F32 row of 2,048 floats is shared by the block's eight waves, 256 floats each (a row in one wave would
-            // be 32 registers a lane); the partial dots meet in LDS
-            a.ab = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (b < 2 * NV) a.ab = ((const float4*)((const float*)(b < NV ? m.a_q : m.b_q) + (int64_t)a_row(6, b, wave) * D))[wave * 64 + lane];
-        } else {
-            const bool extra = wave == 0 && b < 2 * NV;
-            load_row<W_Q8_0, 2, 64>(a.t[6], b < NV ? m.a_q : m.b_q, b < NV ? m.a_s : m.b_s, D, a_row(6, b, wave), lane, extra);
-        }
+    for (int k = 4; k < 6; k++) load_row<W_Q8_0, 2, 64>(a.t[k], m.z_q, m.z_s, D, a_row(k, b, wave), lane, true);
+    if (RF) {
+        // an F32 row of 2,048 floats is shared by the block's eight waves, 256 floats each (a row in one wave would
+        // be 32 registers a lane); the partial dots meet in LDS
+        a.ab = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (b < 2 * NV) a.ab = ((const float4*)((const float*)(b < NV ? m.a_q : m.b_q) + (int64_t)a_row(6, b, wave) * D))[wave * 64 + lane];
+    } else {
+        const bool extra = wave == 0 && b < 2 * NV;
+        load_row<W_Q8_0, 2, 64>(a.t[6], b < NV ? m.a_q : m.b_q, b < NV ? m.a_s : m.b_s, D, a_row(6, b, wave), lane, extra);
     }
 }
 
@@ -900,14 +869,12 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 else ok = ll_wait_quad(p.ll + RX, tid, e, ctl, &v);
                 if (!ok) dead = 1;
                 if (!norm_quant(v, nw, m.eps_norm, xq, xs, red, &dead, tid, xf)) break;
-                if (IT_CHAIN_WC_AT == 1) load_row<W_Q8_0, 4, 64>(wc, m.o_q, m.o_s, VDIM, my_row, lane, true);
                 CH_STAMP(0);
                 XChunks<W_Q8_0, 2> x;
                 load_x<W_Q8_0, 2, 64>(x, xq, xs, lane);
                 float acc[7];
 #pragma unroll
                 for (int k = 0; k < 7; k++) acc[k] = (RF && k == 6) ? 0.0f : reduce_lanes<64>(dot_chunks<W_Q8_0, 2>(aw.t[k], x));
-                if (IT_CHAIN_WC_AT == 2) load_row<W_Q8_0, 4, 64>(wc, m.o_q, m.o_s, VDIM, my_row, lane, true);
                 // row k's dot goes from lane 63 to lane k, which finishes the row
                 float mine = 0.0f;
 #pragma unroll
@@ -943,11 +910,9 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             // ---------------------------------------------------------------- B: delta rule
             CH_STAMP(1);
             // (the out-projection's row goes out first: small loads issued at the head of a stage are back before its input is)
-#if IT_CHAIN_B_POLLERS
             // Waves 5..7 gather the stage's 290 words and issue their out-projection row only afterwards; waves 0..4 issue
             // theirs now and poll nothing: a poll returns behind everything its own wave has in flight.
             if (wave < 5) load_row<W_Q8_0, 4, 64>(wc, m.o_q, m.o_s, VDIM, my_row, lane, true);
-            float k_scale, q_scale;
             {
                 bool ok = true;
                 if (wave >= 5) {
@@ -982,43 +947,9 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
                 __syncthreads();
                 if (dead) break;
                 CH_STAMP(2);
-                if (IT_CHAIN_D_AT) fetch_d();
-                k_scale = 1.0f / fmaxf(sqrtf((float)red[0]), m.eps_l2);
-                q_scale = 1.0f / fmaxf(sqrtf((float)red[1]), m.eps_l2);
-#else
-            if (!IT_CHAIN_WC_AT) load_row<W_Q8_0, 4, 64>(wc, m.o_q, m.o_s, VDIM, my_row, lane, true);
-            const float k_scale = 1.0f, q_scale = 1.0f;
-            {
-                uint32_t w0 = 0, w1 = 0;
-                bool ok = true;
-                if (tid < 2 * DK) {
-                    ok = ll_wait1(p.ll + (tid < DK ? RA + KDIM + kh * DK + tid : RA + kh * DK + (tid - DK)), e, ctl, &w0);
-                } else if (tid < 2 * DK + 16) {
-                    const int j = h * DK + j0 + (tid - 2 * DK);
-                    ok = ll_wait1(p.ll + RA + 2 * KDIM + j, e, ctl, &w0) && ll_wait1(p.ll + RA_Z + j, e, ctl, &w1);
-                    sm[tid - 2 * DK] = __uint_as_float(w0);
-                    sm[16 + tid - 2 * DK] = __uint_as_float(w1);
-                } else if (tid < 2 * DK + 18) {
-                    ok = ll_wait1(p.ll + (tid == 2 * DK + 16 ? RA_AL : RA_BE) + h, e, ctl, &w0);
-                    sm[32 + tid - (2 * DK + 16)] = __uint_as_float(w0);
-                }
-                if (!ok) dead = 1;
-                // l2 norm of k (threads 0..127) and q (128..255): each vector's sum of squares in its own two waves
-                const float kqv = tid < 2 * DK ? __uint_as_float(w0) : 0.0f;
-                const double part = wave_sum_f64_tail((double)(kqv * kqv));
-                if (lane == 63) red[wave] = part;
-                __syncthreads();
-                if (dead) break;
-                CH_STAMP(2);
-                if (IT_CHAIN_D_AT) fetch_d();
-                if (IT_CHAIN_WC_AT == 3) load_row<W_Q8_0, 4, 64>(wc, m.o_q, m.o_s, VDIM, my_row, lane, true);
-                if (tid < 2 * DK) {
-                    const int w2 = tid < DK ? 0 : 2;
-                    const double sum = red[w2] + red[w2 + 1];
-                    kq[tid] = kqv * (1.0f / fmaxf(sqrtf((float)sum), m.eps_l2));
-                }
-                __syncthreads();
-#endif
+                fetch_d();
+                const float k_scale = 1.0f / fmaxf(sqrtf((float)red[0]), m.eps_l2);
+                const float q_scale = 1.0f / fmaxf(sqrtf((float)red[1]), m.eps_l2);
                 const float a = sm[32] + dt_bias;
                 const float softplus = a > 20.0f ? a : fx_logf(1.0f + fx_expf(a));
                 const float g = fx_expf(softplus * ssm_a);
@@ -1061,7 +992,6 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             }
             // ---------------------------------------------------------------- C: out-projection + residual
             CH_STAMP(3);
-            if (!IT_CHAIN_D_AT) fetch_d();
             {
                 const u64* const a4[4] = {p.ll + RB + 2 * tid, p.ll + RB + VDIM / 2 + 2 * tid, p.ll + RB + 2 * (tid + CT), p.ll + RB + VDIM / 2 + 2 * (tid + CT)};
                 uint32_t o[8];
@@ -1123,8 +1053,6 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             else ok = ll_wait_quad(p.ll + RX, tid, e, ctl, &v);
             if (!ok) dead = 1;
             if (!norm_quant(v, nw, f.eps, xq, xs, red, &dead, tid, xf, xh)) break;
-            if (l + 1 < p.n_layers && p.layer[l + 1].has_mixer == 1 && ((IT_CHAIN_A_AT >> 8) & 15))
-                fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane, (IT_CHAIN_A_AT >> 8) & 15);
             CH_STAMP(6);
             XChunks<W_Q8_0, 2> x;
             load_x<W_Q8_0, 2, 64>(x, xq, xs, lane);
@@ -1204,23 +1132,21 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             // The blocks without routed rows (160..255) touch the gate / up rows of the 20 blocks that share their XCD
             // (blocks are dealt to the eight XCDs in turn, each XCD has its own L2): 9 loads a block served.
             uint32_t touched = 0;
-            if (IT_CHAIN_TOUCH) {
-                if (b >= EB) {
-                    const int x = b & 7;
-                    for (int wi = ((b - EB) >> 3) * CW + wave; wi < 20 * 9; wi += 12 * CW) {
-                        const int tb = x + 8 * (wi / 9), part = wi % 9;
-                        const int64_t ex = ids[tb >> 4];
-                        const int r0 = (tb & 15) * 32;
-                        const uint8_t* a;
-                        if (part < 8) {   // eight rows of 1,024 bytes: gate (parts 0..3) or up (4..7)
-                            const uint8_t* q = (part < 4 ? f.eg_q : f.eu_q) + ex * f.gu_q_stride;
-                            a = q + (int64_t)(r0 + (part & 3) * 8 + (lane >> 3)) * (D / 2) + (lane & 7) * 128;
-                        } else {          // the scales of the 32 gate rows (lanes 0..31) and of the 32 up rows
-                            const uint8_t* sc = (lane < 32 ? f.eg_s : f.eu_s) + ex * f.gu_s_stride;
-                            a = sc + (int64_t)(r0 + (lane & 31)) * (D / 16);
-                        }
-                        touched += *(const volatile uint32_t*)a;
+            if (b >= EB) {
+                const int x = b & 7;
+                for (int wi = ((b - EB) >> 3) * CW + wave; wi < 20 * 9; wi += 12 * CW) {
+                    const int tb = x + 8 * (wi / 9), part = wi % 9;
+                    const int64_t ex = ids[tb >> 4];
+                    const int r0 = (tb & 15) * 32;
+                    const uint8_t* a;
+                    if (part < 8) {   // eight rows of 1,024 bytes: gate (parts 0..3) or up (4..7)
+                        const uint8_t* q = (part < 4 ? f.eg_q : f.eu_q) + ex * f.gu_q_stride;
+                        a = q + (int64_t)(r0 + (part & 3) * 8 + (lane >> 3)) * (D / 2) + (lane & 7) * 128;
+                    } else {          // the scales of the 32 gate rows (lanes 0..31) and of the 32 up rows
+                        const uint8_t* sc = (lane < 32 ? f.eg_s : f.eu_s) + ex * f.gu_s_stride;
+                        a = sc + (int64_t)(r0 + (lane & 31)) * (D / 16);
                     }
+                    touched += *(const volatile uint32_t*)a;
                 }
             }
             // the softmax's sum, exp(logit - largest logit) over the 512, by wave here, under the rows' flight, and over the waves
@@ -1328,7 +1254,7 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
         auto fetch_next = [&]() {
             if (l + 1 == p.n_layers && p.has_tail) fetch_tail(p.tail, aw, b, wave, lane);
             if (l + 1 < p.n_layers && p.layer[l + 1].has_mixer == 3) fetch_tail(p.layer[l + 1].a, aw, b, wave, lane);
-            if (next_mixer && ((IT_CHAIN_A_AT >> 4) & 15)) fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane, (IT_CHAIN_A_AT >> 4) & 15);
+            if (next_mixer) fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane);
         };
         if (wave < 4) fetch_next();
 
@@ -1378,7 +1304,6 @@ __global__ __launch_bounds__(CT) void layer_chain_k(ChainPT<NL> p) {
             __syncthreads();
             if (dead) break;
             CH_STAMP(11);
-            if (next_mixer && (IT_CHAIN_A_AT & 15)) fetch_a<RF>(p.layer[l + 1].m, aw, b, wave, lane, IT_CHAIN_A_AT & 15);
             float acc = 0.0f;
             const int c = lane & 15;
 #pragma unroll
