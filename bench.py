@@ -86,8 +86,8 @@ def prefill_instructions(n_tokens, exact):
     held against: one of as many multiply-accumulates a cycle."""
     # Q8_0 products: 32x32x32 (k_gemm.hip, q8_wide_k), which does as many a cycle as 16x16x64; short batches take 16x16x32
     dense = ("int8_32x32x32", "int8_16x16x64") if n_tokens >= 512 else ("int8_16x16x32", "int8_16x16x32")
-    # (exact mode: what Q8_0 experts issue; NVFP4 ones take two f16 16x16x16 for sixteen weights and are held against the same)
-    experts = ("int8_16x16x32", "int8_16x16x32") if exact else ("f16_32x32x16", "f16_32x32x16")
+    # the model's NVFP4 experts
+    experts = ("f16_16x16x16", "f16_16x16x16") if exact else ("f16_32x32x16", "f16_32x32x16")
     return {"matmul (dense": dense, "moe_glu": experts, "matmul_experts": experts, "delta_rule": ("f32_16x16x4", "f32_16x16x4"),
             "attend": ("f16_32x32x16", "f16_32x32x16")}
 
@@ -452,12 +452,10 @@ def main():
         elif name.startswith("moe_glu") or name.startswith("matmul_experts"):
             m = glu_macs if name.startswith("moe_glu") else down_macs
             useful = 2 * m * args.prompt / sec / 1e12
-            if args.exact:
-                k.update(unit="int8 MFMA", tops=round(useful, 1), mfma_frac=round(useful / INT8_PEAK_TOPS, 4))
-            else:
-                # f16 matrix cores, every product issued twice (activation hi and lo halves)
-                k.update(unit="f16 MFMA", useful_tops=round(useful, 1), tflops=round(2 * useful, 1),
-                         mfma_frac=round(2 * useful / F16_PEAK, 4))
+            # f16 matrix cores, two instructions for every product (the activation's hi and lo halves; in exact mode a
+            # sub-block's dots and its scales' products)
+            k.update(unit="f16 MFMA", useful_tops=round(useful, 1), tflops=round(2 * useful, 1),
+                     mfma_frac=round(2 * useful / F16_PEAK, 4))
         elif name == "delta_rule" and not args.exact:
             # chunked form, per (64-token chunk, value head): K S^T, Q S^T and the state update (64 x dk x dv each),
             # T R and P U (lower triangles, 64 x 64 x dv / 2 each), K K^T and Q K^T (64 x 64 x dk / 2 each)

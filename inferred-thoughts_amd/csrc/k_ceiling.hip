@@ -12,11 +12,12 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
 constexpr int CHAINS = 8;       // independent accumulators per wave
 constexpr int CEIL_THREADS = 256;
 
-// KIND: 0 int8 16x16x64, 1 int8 16x16x32, 2 f16 32x32x16, 3 f16 16x16x32, 4 f32 16x16x4
+// KIND: 0 int8 16x16x64, 1 int8 16x16x32, 2 f16 32x32x16, 3 f16 16x16x32, 4 f32 16x16x4, 5 f16 16x16x16
 template <int KIND>
 __global__ __launch_bounds__(CEIL_THREADS) void mfma_ceiling_k(int iters, float* sink) {
     const int lane = threadIdx.x;
@@ -68,6 +69,17 @@ __global__ __launch_bounds__(CEIL_THREADS) void mfma_ceiling_k(int iters, float*
         }
 #pragma unroll
         for (int j = 0; j < CHAINS; ++j) total += c[j][0] + c[j][1] + c[j][2] + c[j][3];
+    } else if constexpr (KIND == 5) {
+        v4h a, b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { a[e] = (_Float16)(0.001f * (lane + e)); b[e] = (_Float16)(0.002f * (lane - e)); }
+        v4f c[CHAINS] = {};
+        for (int i = 0; i < iters; ++i) {
+#pragma unroll
+            for (int j = 0; j < CHAINS; ++j) c[j] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < CHAINS; ++j) total += c[j][0] + c[j][1] + c[j][2] + c[j][3];
     } else {
         float a = 0.001f * lane, b = 0.002f * (lane - 7);
         v4f c[CHAINS] = {};
@@ -83,12 +95,12 @@ __global__ __launch_bounds__(CEIL_THREADS) void mfma_ceiling_k(int iters, float*
 }
 
 // multiply-accumulates of one instruction of each kind
-constexpr double KIND_MACS[5] = {16. * 16 * 64, 16. * 16 * 32, 32. * 32 * 16, 16. * 16 * 32, 16. * 16 * 4};
+constexpr double KIND_MACS[6] = {16. * 16 * 64, 16. * 16 * 32, 32. * 32 * 16, 16. * 16 * 32, 16. * 16 * 4, 16. * 16 * 16};
 
 }  // namespace
 
 extern "C" int it_hip_mfma_ceiling(it_hip* be, int kind, int iters, double* ops_per_s) {
-    if (!be || kind < 0 || kind > 4 || iters < 1 || !ops_per_s) return 1;
+    if (!be || kind < 0 || kind > 5 || iters < 1 || !ops_per_s) return 1;
     hipStream_t s = be->stream;
     hipDeviceProp_t prop;
     int dev = 0;
@@ -106,7 +118,8 @@ extern "C" int it_hip_mfma_ceiling(it_hip* be, int kind, int iters, double* ops_
             case 1: mfma_ceiling_k<1><<<blocks, CEIL_THREADS, 0, s>>>(n, sink); break;
             case 2: mfma_ceiling_k<2><<<blocks, CEIL_THREADS, 0, s>>>(n, sink); break;
             case 3: mfma_ceiling_k<3><<<blocks, CEIL_THREADS, 0, s>>>(n, sink); break;
-            default: mfma_ceiling_k<4><<<blocks, CEIL_THREADS, 0, s>>>(n, sink); break;
+            case 4: mfma_ceiling_k<4><<<blocks, CEIL_THREADS, 0, s>>>(n, sink); break;
+            default: mfma_ceiling_k<5><<<blocks, CEIL_THREADS, 0, s>>>(n, sink); break;
         }
     };
     launch(iters / 8 + 1);  // code object load and clock ramp

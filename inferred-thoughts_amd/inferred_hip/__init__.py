@@ -486,7 +486,7 @@ class Hip:
         self.L.it_hip_fetch_read_counts(self.h, v)
         return int(v[0]), int(v[1])
 
-    MFMA_KINDS = {"int8_16x16x64": 0, "int8_16x16x32": 1, "f16_32x32x16": 2, "f16_16x16x32": 3, "f32_16x16x4": 4}
+    MFMA_KINDS = {"int8_16x16x64": 0, "int8_16x16x32": 1, "f16_32x32x16": 2, "f16_16x16x32": 3, "f32_16x16x4": 4, "f16_16x16x16": 5}
 
     def mfma_ceiling(self, kind: str, iters: int = 20000) -> float:
         """Measured operations per second of back-to-back MFMA instructions of one kind."""

@@ -39,10 +39,14 @@ def test_the_output_head_is_told_from_the_other_products():
 def test_a_familys_rate_is_held_against_an_instruction_of_the_same_rate(n_tokens, exact):
     """The ceiling's instruction does as many multiply-accumulates a cycle as the one that the kernels issue."""
     per_cycle = {"int8_32x32x32": 1024, "int8_16x16x64": 1024, "int8_16x16x32": 512, "f16_32x32x16": 512, "f16_16x16x32": 512,
-                 "f32_16x16x4": 32}
+                 "f16_16x16x16": 256, "f32_16x16x4": 32}
     import inferred_hip as ih
     for family, (issued, ceiling) in bench.prefill_instructions(n_tokens, exact).items():
         assert ceiling in ih.Hip.MFMA_KINDS
         assert per_cycle[issued] == per_cycle[ceiling], family
+    # (NVFP4 experts: k_gemm_f16.hip's 32x32x16 and, keeping the CPU path's bits, k_gemm.hip's experts_nvfp4_k)
+    issued = bench.prefill_instructions(n_tokens, exact)["moe_glu"][0]
+    source = (CSRC / "k_gemm.hip").read_text().split("void experts_nvfp4_k(")[1].split("\n}\n")[0] if exact else (CSRC / "k_gemm_f16.hip").read_text()
+    assert issued.replace("f16_", "mfma_f32_") in source
     wide = bench.prefill_instructions(n_tokens, exact)["matmul (dense"][0] == "int8_32x32x32"
     assert wide == (n_tokens >= 512)       # (most dense rows of a pass of 512 tokens go through k_gemm.hip's 32x32x32 products)
