@@ -778,13 +778,9 @@ void ssm_conv(float* state, const float* x, const float* w, int kernel, int nc, 
 
 // ------------------------------------------------------------------ argmax
 // First strict maximum (ties to the lower index), /root/reference src/profile.rs:192-213.
-// What the serial scan makes of value `v` at index `i`: one that is not a number is never taken, and a first value that is not a
-// number stays.  (Candidates are numbers then, so that every order of merging them gives the same one.)
-IT_DEV bool argmax_counts(float* v, int64_t i) {
-    if (*v == *v) return true;
-    *v = INFINITY;
-    return i == 0;
-}
+// As the serial scan takes them: a value that is not a number, or no larger than minus infinity, is no candidate (a thread without one
+// has index 0x7fffffff, and without any the first index wins), and a first value that is not a number stays.  Candidates are numbers
+// then, so that every order of merging them gives the same one.
 __global__ __launch_bounds__(256) void argmax_part_k(const float* __restrict__ x, int64_t n,
                                                      int32_t* __restrict__ pidx, float* __restrict__ pval) {
     __shared__ float sv[256];
@@ -793,10 +789,14 @@ __global__ __launch_bounds__(256) void argmax_part_k(const float* __restrict__ x
     int64_t lo = per * blockIdx.x, hi = lo + per < n ? lo + per : n;
     float bv = -INFINITY;
     int bi = 0x7fffffff;
+    if (lo == 0 && threadIdx.x == 0 && !(x[0] == x[0])) {
+        bv = INFINITY;
+        bi = 0;
+    }
     for (int64_t i = lo + threadIdx.x; i < hi; i += 256) {
         float v = x[i];
         // strided scan visits ascending indices per thread, so strict > keeps the lowest
-        if (argmax_counts(&v, i) && (bi == 0x7fffffff || v > bv)) {
+        if (v > bv) {
             bv = v;
             bi = (int)i;
         }
@@ -927,15 +927,15 @@ __global__ __launch_bounds__(1024) void argmax_embed_one_k(const float* __restri
         if (1024 * k >= n) break;
         v[k] = tid + 1024 * k < n ? logits[tid + 1024 * k] : -INFINITY;
     }
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
+    const bool stays = tid == 0 && !(v[0] == v[0]);
+    float bv = stays ? INFINITY : -INFINITY;
+    int bi = stays ? 0 : 0x7fffffff;
 #pragma unroll
     for (int k = 0; k < ARGMAX_ONE; k++) {
-        const int i = tid + 1024 * k;
         if (1024 * k >= n) break;
-        if (i < n && argmax_counts(&v[k], i) && (bi == 0x7fffffff || v[k] > bv)) {
+        if (v[k] > bv) {
             bv = v[k];
-            bi = i;
+            bi = tid + 1024 * k;
         }
     }
     argmax_of_wave(&bv, &bi);
