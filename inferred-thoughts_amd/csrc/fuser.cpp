@@ -280,7 +280,7 @@ bool final_head(const Op& g, const Op& rms, const Op& q, const Op& m, int exact,
     a.x_raw = g.p[1] == rms.p[2] ? nullptr : (float*)g.p[1];
     a.eps = rms.f[0];
     a.n_in = (int)rms.i[1];
-    a.mode = 1;
+    a.mode = a.x_raw ? 3 : 1;
     a.exact = exact;
     a.n_mats = 1;
     a.m[0] = mat_of(m, 0);

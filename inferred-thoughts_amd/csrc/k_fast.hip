@@ -64,12 +64,12 @@ inline Geo geo_of(int fmt, int n_in) {
 
 // The activation of a fused GEMV, from global f32 to quantized LDS, held in registers in
 // between: thread t owns floats [4t, 4t+4) and [4(t+THREADS), ...).  n_in <= 8 * THREADS.
-//   mode 0: as is; 1: rms_norm(x, norm_w) (naive.rs:633-650); 2: per-head rms_norm times the gate, which
+//   mode 0: as is; 1, 3: rms_norm(x, norm_w) (naive.rs:633-650); 2: per-head rms_norm times the gate, which
 //   its producer has put through silu (head_dim / 4 a power of two <= 64, so a head sits inside one wave).
 // Ends with a block barrier; xq / xs are then complete.
 template <int THREADS>
 __device__ __forceinline__ void stage_activation(const float* x, int n_in, int mode, const float* norm_w, const float* gate, int head_dim,
-                                 float eps, float* raw, float* copy1, float* copy2, int8_t* xq, float* xs, double* red,
+                                 float eps, float* copy1, float* copy2, int8_t* xq, float* xs, double* red,
                                  float* xf = nullptr) {
     const int tid = threadIdx.x;
     const int nq = n_in >> 2;
@@ -81,16 +81,11 @@ __device__ __forceinline__ void stage_activation(const float* x, int n_in, int m
         live[k] = qi < nq;
         v[k] = live[k] ? ((const float4*)x)[qi] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    if (mode == 1) {
+    if (mode & 1) {
         float4 w[2];
 #pragma unroll
         for (int k = 0; k < 2; k++)
             w[k] = live[k] ? ((const float4*)norm_w)[tid + k * THREADS] : make_float4(0.f, 0.f, 0.f, 0.f);
-        if (raw) {
-#pragma unroll
-            for (int k = 0; k < 2; k++)
-                if (live[k]) ((float4*)raw)[tid + k * THREADS] = v[k];
-        }
         double part = wave_sum_f64_tail(quad_sumsq(v[0]) + quad_sumsq(v[1]));
         if ((tid & 63) == 63) red[tid >> 6] = part;
         __syncthreads();
@@ -224,7 +219,7 @@ __global__ __launch_bounds__(FT) void fused_gemv_fast_k(FusedGemvP p) {
     }
 
     const bool first = blockIdx.x == 0;
-    stage_activation<FT>(p.x, n_in, p.mode, p.norm_w, p.gate, p.head_dim, p.eps, first ? p.x_raw : nullptr, first ? p.x_copy : nullptr,
+    stage_activation<FT>(p.x, n_in, p.mode, p.norm_w, p.gate, p.head_dim, p.eps, first ? p.x_copy : nullptr,
                          first ? p.x_copy2 : nullptr, xq, xs, red, FM ? xf : nullptr);
     XChunks<FMT, CPL> x;
     load_x<FMT, CPL, L>(x, xq, xs, sub);
@@ -272,6 +267,9 @@ __global__ __launch_bounds__(FT) void fused_gemv_fast_k(FusedGemvP p) {
             }
         }
     }
+
+    if (p.mode == 3 && blockIdx.x == gridDim.x - 1)   // (behind the rows: in the prologue it cost every launch, this one or not, 0.1 us)
+        for (int i = threadIdx.x; i < n_in / 4; i += FT) ((float4*)p.x_raw)[i] = ((const float4*)p.x)[i];
 
     // unquantized matrices (the router and ssm alpha / beta of real files are F32): one wave per row, the row sum
     // split over the lanes.  An F32 row of up to 2,048 weights is held in registers: all of its loads are in flight
@@ -369,7 +367,7 @@ static bool fused_gemv_fast_prepare(FusedGemvP& p, Geo* geo, int* fmt_out, int* 
     const Geo g = geo_of(fmt, p.n_in);
     if (!g.ok || p.n_in > FT * 8 || p.n_in % 32) return false;
     if (!aligned16(p.x) || !aligned16(p.x_copy) || !aligned16(p.x_copy2) || !aligned16(p.x_raw)) return false;
-    if (p.mode == 1 && !aligned16(p.norm_w)) return false;
+    if ((p.mode & 1) && !aligned16(p.norm_w)) return false;
     if (p.mode == 2) {
         const int lh = p.head_dim / 4;
         if (p.head_dim % 4 || lh < 1 || lh > 64 || (lh & (lh - 1)) || p.n_in % p.head_dim) return false;
@@ -570,7 +568,7 @@ __global__ __launch_bounds__(FT, 6) void moe_glu_fast_k(MoeGluP p, GluGeo gg) {
 
     float logit[4];
     if (p.logits) route_fetch<FT>(p.logits, p.n_expert, logit);
-    stage_activation<FT>(p.x, n_in, 0, nullptr, nullptr, 0, 0.0f, nullptr, nullptr, nullptr, xq, xs, red);
+    stage_activation<FT>(p.x, n_in, 0, nullptr, nullptr, 0, 0.0f, nullptr, nullptr, xq, xs, red);
     if (p.logits) {
         const float denom = block_route<FT>(logit, p.n_expert, p.n_used, route_sh, ids, wts);
         if (blockIdx.x == 0 && tid < p.n_used) {

@@ -159,7 +159,7 @@ __device__ void wave_row_terms(const uint8_t* wq, const uint8_t* ws, int n_in, i
 }
 
 // ------------------------------------------------------------------ fused_gemv
-// prologue modes: 0 = the activation as is; 1 = rms_norm(x, norm_w); 2 = per-head
+// prologue modes: 0 = the activation as is; 1 = rms_norm(x, norm_w); 3 = that, and x left in x_raw; 2 = per-head
 // rms_norm of x (weight norm_w[head_dim]) gated by silu(gate): silu(g) * ((x*scale)*w)
 // ------------------------------------------------------------------ router in one wave
 // softmax over up to 64 experts, then n_used rounds of arg-max with ties to the lower id, the
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         xv[j] = wv[j] = gv[j] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (i < n_in) {
             xv[j] = load4(p.x + i);
-            if (p.mode == 1) wv[j] = load4(p.norm_w + i);
+            if (p.mode & 1) wv[j] = load4(p.norm_w + i);
             if (p.mode == 2) {
                 wv[j] = load4(p.norm_w + i % p.head_dim);
                 gv[j] = load4(p.gate + i);
@@ -347,14 +347,13 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
         s += (double)(v.w * v.w);
         return s;
     };
-    if (p.mode == 1) {
+    if (p.mode & 1) {
         double part = 0.0;
 #pragma unroll
         for (int j = 0; j < NQ; j++) {
             const int i = 4 * (tid + FG_THREADS * j);
             part += squares(xv[j]);
             if (i < n_in) *(float4*)(xf + i) = xv[j];      // for the serial sum, should it be needed
-            if (i < n_in && blockIdx.x == 0 && p.x_raw) store4(p.x_raw + i, xv[j]);
         }
         part = wave_sum_f64_tail(part);
         if (lane == 63) red[wave] = part;
@@ -472,6 +471,8 @@ __global__ __launch_bounds__(FG_THREADS) void fused_gemv_k(FusedGemvP p) {
             wave_lds_sync();
         }
     }
+    if (p.mode == 3 && blockIdx.x == gridDim.x - 1)   // (behind everything: in the prologue it cost every launch, this one or not, 0.1 us)
+        for (int i = 4 * tid; i < n_in; i += 4 * FG_THREADS) store4(p.x_raw + i, load4(p.x + i));
     if (p.route_counter) {
         // The block that finishes last turns the router logits (matrix 0's output) into the
         // token's expert choice, so the next kernel starts with the ids in hand.
