@@ -750,9 +750,14 @@ __global__ __launch_bounds__(DT) void moe_down_fast_k(MoeDownP p) {
 
 #pragma unroll
     for (int k = 0; k < QR; k++) {
+        // (quads past the end, whose zeros would take quant_word's long way: whole waves of them stop here, the others take a block of
+        // ones.  32 tokens, four picks of 256 Q8_0 values, half a quad a thread: 11.4 -> 7.5 us; 64 NVFP4 experts of 512 x 2,048, eight
+        // picks, two and a quarter: 49.8, 58.6 before the short quants)
         const int qi = k * DT + tid;
+        if (qi - lane >= nq) break;
         float d;
-        const uint32_t word = quant_word(v[k], group_max<8>(quad_amax(v[k])), &d);
+        const float amax = group_max<8>(quad_amax(v[k]));
+        const uint32_t word = quant_word(v[k], qi < nq ? amax : 1.0f, &d);
         const uint32_t ahead = word_ahead2(word);
         if (qi >= nq) continue;
         const bool shared = qi >= nq_routed;
