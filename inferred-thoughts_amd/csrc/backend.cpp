@@ -1655,15 +1655,16 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
         if (tiles && !be->act_split(x, x_len, v.n_in, &sp)) return;
     }
     const bool rows_dense = !tiles && !exact && v.fmt == W_NVFP4 && n >= 128 && n <= 512 && itk::expert_rows_takes(ev, nullptr, aq);
-    // Exact mode: the int8 tiles of the expert products, which keep the GEMV's bits, from 64 tokens on (2,048 x 512 over 333
-    // tokens: 20 us, 47 as a GEMV per token)
-    bool int8_tiles = false;
+    // Exact mode: the expert products' 16-pair tiles, which keep the GEMV's bits, from 64 tokens on (us there, and as a GEMV per token:
+    // 2,048 rows of 512 over 32 / 64 / 333 tokens 8.0, 8.1, 10.5 and 8.9, 13, 47; 4,096 of 2,048 17, 20, 40 and 38, 66, 322; 512 of 2,048
+    // 16, 16, 17 and 10, 15, 51: the last are behind below 80)
+    bool exact_tiles = false;
     if (exact && v.fmt == W_NVFP4 && n >= 64) {
         zids = be->zero_ids_for(n);
         work = be->moe_work_for(n, 1, &work_ints);
-        int8_tiles = zids && work;
+        exact_tiles = zids && work;
     }
-    const it_hip::Grouping gr = int8_tiles ? be->grouping(nt, 1) : it_hip::Grouping{};   // (every token on the one expert)
+    const it_hip::Grouping gr = exact_tiles ? be->grouping(nt, 1) : it_hip::Grouping{};   // (every token on the one expert)
     it_hip::OpRec rec;
     rec.id = OP_MATMUL; rec.p[0] = v.q; rec.p[1] = v.scales; rec.p[2] = dx; rec.p[3] = as; rec.p[4] = aq; rec.p[5] = dout;
     rec.p[6] = sp.h; rec.p[7] = sp.l; rec.p[8] = sp.scale;
@@ -1689,7 +1690,7 @@ static void matmul_impl(it_hip* be, const it_weights* w, const float* x, uint64_
         }
         if (tiles == 1 && experts_gemm_f16s(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
         if (tiles == 2 && experts_gemm_f16(ev, nullptr, nullptr, nt, 1, 0, sp, dout, nullptr, 0, false, {}, scale_by, 1.0f, s)) return;
-        if (int8_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;
+        if (exact_tiles && experts_gemm(ev, nullptr, zids, nt, 1, 0, as, aq, dout, work, work_ints, gr.held(16), s) && gr.made(16)) return;
         if (rows_dense && expert_rows(ev, nullptr, nullptr, nt, 1, 0, as, aq, dout, scale_by, nullptr, 0, false, s)) return;
         matmul(v, dx, as, aq, nt, dout, scale_by, exact, s);
     };
@@ -2026,18 +2027,21 @@ static bool host_ids_in_range(it_hip* be, const it_route* r, uint64_t n_expert, 
     return true;
 }
 
-// Expert-sorted tiles read an expert's rows once for all of its pairs; the per-pair kernels read them once per
-// pair but stream them at several times the rate.  Measured on the 512-expert shape (pairs per expert 0.08 .. 5):
-// the tiles win from about 3.5 pairs per expert on (a batch of 128 tokens at top-10 still takes 653 us per pair
-// against 772 us tiled; at 256 tokens it is 1,180 against 848).
+// Expert-sorted 16-pair tiles (k_gemm.hip) read an expert's rows once for all of its pairs.  The line, 3.5 pairs per expert, is where they
+// meet fast mode's other Q8_0 form (k_moe_rows.hip): the whole FFN's launches over 256 experts of 512 x 2,048, eight a token, 80 / 96 / 128 / 179
+// tokens 266, 269, 280, 284 us as tiles, 248, 258, 292, 323 in the other form.  Exact mode's other form reads the rows once per pair and
+// meets the tiles earlier: the same experts over 16 / 32 / 64 / 128 / 256 tokens 158, 221, 337, 561, 1,017 us per pair, 186, 224, 269, 293, 302 tiled;
+// NVFP4 146, 209, 327, 520, 895 and 158, 204, 251, 273, 285; 512 NVFP4 ones, ten a token, 172, 245, 394, 653, 1,189 and 188, 247, 329, 390, 421:
+// level at about one pair per expert.
 static bool expert_tiles_pay(uint64_t picks, uint64_t n_expert) { return picks >= 32 && 2 * picks >= 7 * n_expert; }
 // Fast mode between the per-pair GEMVs and the wide matrix-core tiles, measured on the 512-expert top-10 FFN (hidden
 // 2048, inter 512).  NVFP4 runs 16-pair tiles on the f16 matrix cores (k_gemm_f16s.hip): level with the per-pair kernels at
 // 40 pairs (four tokens: 307 against 314 us for two layers' whole pass), ahead behind (40 tokens: 574 against 699, 63: 664
 // against 893; up to 32 tokens the FFN is two launches of its own, fuser.cpp), up to 36 or 48 pairs per expert, where the 128-pair tiles
-// take over.  Both products, us, on the 16-pair tiles and on the wide ones at 36 / 44 / 48 pairs: 512 experts of 512 x 2,048 479, 551, 590
-// and 565, 605, 615; 256 of these 284, 305, 332 and 298, 320, 320; 256 of 256 x 2,048 180, 200, 218 and 181, 191, 204; 512 of 256 x 1,024 209,
-// 235, 254 and 204, 220, 228 (up to 128 experts of 512 x 2,048 the wide ones are ahead from 20 pairs on: 88 against 103 at 36 for 64).  So
+// take over.  The whole FFN's launches, us, on the 16-pair tiles and on the wide ones at 36 / 44 / 48 pairs: 512 experts of 512 x 2,048 659, 752, 793
+// and 728, 787, 819; 256 of these 411, 454, 478 and 429, 452, 470 (up to 128 experts of 512 x 2,048 the wide ones are ahead from 20 pairs
+// on: 128 against 138 for 64, 153 against 170 at 36).  Both products alone, before the wide ones' results left through LDS (the down
+// product 8 % quicker for it): 256 of 256 x 2,048 180, 200, 218 and 181, 191, 204; 512 of 256 x 1,024 209, 235, 254 and 204, 220, 228.  So
 // 48 for many experts of a million weights, and for few small ones, which leave the wide tiles' grid short of blocks (16 of 256 x 512
 // at 36 to 47 pairs 33 against 36, 8 of 1,024 x 2,048 66 against 69 at 36).  What that kernel
 // does not take (Q8_0, odd shapes) streams each expert's rows once for all its pairs (k_moe_rows.hip) from 1.25 pairs per

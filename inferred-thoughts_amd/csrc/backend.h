@@ -98,7 +98,8 @@ struct it_hip {
     // The routed FFN of a short batch is held back to become two launches that read none of these forms (fuser.cpp), so its
     // expert products do not ask for one: a launch that turns out to need it makes it there, in room of the backend's own that
     // the next launch reads and nothing else.
-    static constexpr int SHORT_FFN_TOKENS = 32;   // (measured on the 512-expert top-10 layer: 176 against 232 us at 32, 271 against 298 at 48, behind from about 56 on)
+    static constexpr int SHORT_FFN_TOKENS = 32;   // (measured on the 512-expert top-10 layer: 141 against 195 us at 32, 169 against 184 at 40, level at 48, 234 against 206 at 56;
+    // 256 experts, top-8: 114 against 161, 138 against 148, 165 against 153 at 48)
     bool short_ffn(uint64_t n_tok) const {
         return mode == Mode::Eager && in_pass && pass_tokens > 1 && n_tok >= 2 && n_tok <= SHORT_FFN_TOKENS && !exact && fuse_enabled &&
                small_ffn_enabled && !expert_cold_entries;

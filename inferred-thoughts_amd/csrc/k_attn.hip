@@ -149,7 +149,9 @@ void attend_exact(const AttnArgs& a, float* scratch, float* out, hipStream_t s, 
 // at a time, whole lines, through a piece of LDS of its own (rows 144 bytes apart: no bank conflicts), the next piece in registers
 // meanwhile; a block brings its 64 dims of 512 values while the weights are formed, all threads form the products, and one wave adds
 // them up.  340 positions, 16 heads of 256: 27.3 -> 15.1 us (22.5 with all dims in a block); a token of four layers of 512 values,
-// 33 to 290 positions, 8 heads of 64: 115.7 -> 112.0 us.
+// 33 to 290 positions, 8 heads of 64: 115.7 -> 112.0 us.  Longer contexts, where a head's blocks repeat its scores and the weights lie in
+// memory from 4,096 on: an attention block with 16 heads of 256 over 2,000 / 4,000 / 8,000 / 32,000 positions 131, 237, 537, 2,373 us in the two
+// launches, 67, 105, 203, 804 so; 8 heads of 64 92, 157, 308, 1,720 and 54, 75, 144, 590.
 constexpr int ONE_DIMS = 64, ONE_T = 512, ONE_ROW = 144, ONE_V = 8;      // threads; bytes of a key's piece in LDS; 16-byte pieces of values a thread brings
 constexpr int ONE_VALUES = ONE_T * ONE_V * 16, ONE_STAGE = 2 * ONE_VALUES;   // (as f32 products)
 static_assert(ONE_T * ONE_ROW <= ONE_STAGE, "the keys' pieces lie where the values go later");

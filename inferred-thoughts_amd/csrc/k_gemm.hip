@@ -472,9 +472,11 @@ bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, 
         using std::integral_constant;
         // 64 rows x 16 tokens a block up to 640 of them (2.5 a CU).  Above, the shape that takes least by the blocks a CU gets, b, from
         // what rows of 2,048 measure (in us; a block alone on its CU is quicker): 64 x 32 2.5 + 6.2 b; 128 x 32, three a CU at a time,
-        // 19, 24 and 31; 128 x 64 25 and 37 for two; 128 x 128 38 and 66.  (4096 x 2048 over 300 / 400 / 512 / 1,100 / 5,700 tokens: 64 x 32 20.3, 26.2,
-        // 28.2, 54.0, 273; 128 x 32 20.9, 21.6, 23.1, 47.2, 209; 128 x 64 25.1, 26.1, 26.5, 53.6, 195; 128 x 128 38.8, 39.5, 39.1, 51.4, 171.)
-        // It serves other row lengths as it is: 1,024 to 8,192 rows of 512 to 8,192 over 100 to 2,500 tokens, 90 shapes, none more than 3 %
+        // 19, 24 and 31; 128 x 64 25 and 37 for two; 128 x 128 38 and 66: what they took with the scales' products on the vector ALU, 4 to 9 %
+        // more than now.  (4096 x 2048 over 300 / 400 / 512 / 1,100 / 1,500 / 5,700 tokens, now: 64 x 32 21.6, 27.8, 29.3, 54.1, 70.0, 239; 128 x 32
+        // 20.8, 21.9, 23.0, 46.3, 53.5, 200; 128 x 64 24.1, 25.2, 26.0, 43.1, 46.0, 162; 128 x 128 35.9, 36.7, 37.3, 51.4, 55.1, 161.  The third
+        // 128 x 64 block of a CU costs less than the sum says: at 1,100 and 1,500 tokens the shape taken, 128 x 32, is the second best.)
+        // It served other row lengths as it is: 1,024 to 8,192 rows of 512 to 8,192 over 100 to 2,500 tokens, 90 shapes, none more than 3 %
         // behind 16, 32 or 64 tokens a block by their number alone.
         const int64_t units = (int64_t)gx * tiles;
         if (units <= 640) {
@@ -513,13 +515,11 @@ bool q8_gemm(const WView& w, const float* act_scales, const int8_t* act_quants, 
 // The per-pair GEMV reads an expert's matrix once per pair.  Here the pairs are first sorted
 // into per-expert lists ("expert-sorted token lists": moe_group_k), the lists are cut into
 // tiles of up to 16 pairs, and one block multiplies 64 rows of that expert's matrix with the
-// tile's 16 activation rows on the int8 matrix cores, so a matrix is read once per tile.
-// Per pair and row the arithmetic is the GEMV's: per-block integer dots, scaled and added in
-// block order (Q8_0: (float)isum * (dw * dx); NVFP4: (dy * dA) * (float)sa then
-// (dy * dB) * (float)sb per 32-element chunk), then the expert's second scale, then silu-mul
-// for the gate/up pair.  An NVFP4 chunk holds two 16-element sub-blocks with their own
-// scales; each needs its own integer sum, so the chunk takes two MFMAs whose token operand is
-// zeroed outside the sub-block.
+// tile's 16 activation rows on the matrix cores (Q8_0 int8, NVFP4 f16), so a matrix is read
+// once per tile.  Per pair and row the arithmetic is the GEMV's: per-block integer dots, scaled
+// and added in block order (Q8_0: (float)isum * (dw * dx); NVFP4: (dy * dA) * (float)sa then
+// (dy * dB) * (float)sb per 32-element chunk of two sub-blocks), then the expert's second scale,
+// then silu-mul for the gate/up pair.
 namespace itk {
 namespace {
 
