@@ -366,7 +366,7 @@ static bool fused_gemv_fast_prepare(FusedGemvP& p, Geo* geo, int* fmt_out, int* 
         if (p.m[i].fmt != fmt) return false;
     const Geo g = geo_of(fmt, p.n_in);
     if (!g.ok || p.n_in > FT * 8 || p.n_in % 32) return false;
-    if (!aligned16(p.x) || !aligned16(p.x_copy) || !aligned16(p.x_copy2) || !aligned16(p.x_raw)) return false;
+    if (!aligned16(p.x) || !aligned16(p.x_copy) || !aligned16(p.x_copy2) || (p.mode == 3 && !aligned16(p.x_raw))) return false;
     if ((p.mode & 1) && !aligned16(p.norm_w)) return false;
     if (p.mode == 2) {
         const int lh = p.head_dim / 4;

@@ -592,9 +592,9 @@ static bool fused_gemv_exact_takes(const FusedGemvP& p) {
 // 16,384 values are left to the ops one by one.  Every block reads the whole activation, at its own time: what block 0 leaves and
 // what the rows' waves write lies elsewhere.)
 bool fused_gemv_takes(const FusedGemvP& p) {
-    if (p.x_copy == p.x || p.x_copy2 == p.x || p.x_raw == p.x) return false;
+    if (p.x_copy == p.x || p.x_copy2 == p.x || (p.mode == 3 && p.x_raw == p.x)) return false;
     for (int i = 0; i < p.n_mats; i++)
-        if (p.m[i].out == p.x || p.m[i].out == p.gate) return false;
+        if (p.m[i].out == p.x || p.m[i].out == p.gate) return false;   // (mode 3: or x_raw)
     if (p.mode == 2 && ((p.head_dim != 64 && p.head_dim != 128) || p.n_in % p.head_dim)) return false;   // (a head is a row of 16 lanes, or two)
     bool floats = false;
     for (int i = 0; i < p.n_mats; i++) floats |= p.m[i].fmt != W_Q8_0 && p.m[i].fmt != W_NVFP4;
